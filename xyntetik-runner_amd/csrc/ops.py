@@ -83,6 +83,7 @@ _PROTOS = {
     "xr_head_rmsnorm": [_p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _f, _i, _p],
     "xr_moe_table_route": [_p, _p, _p, _p, _i, _i, _i, _i, _f, _p],
     "xr_sample": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p],
+    "xr_sample_split": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p, C.c_longlong, _i, _p],
     "xr_layernorm": [_p, _p, _p, _p, _i, _i, _i, _f, _i, _p],
     "xr_layernorm_conv": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _f, _i, _p],
     "xr_causal_conv": [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
@@ -1667,16 +1668,24 @@ class Ops:
             raise KernelError("sample: logits must be float32 [rows, vocab]")
         W, V = logits.shape
         out = torch.empty((W,), dtype=torch.int32, device=logits.device)
-        # room for the greedy rows' first pass (32 ranges a row) when a row is long enough to need one
-        greedy_ws = torch.empty((W, 32, 2), dtype=torch.float32, device=logits.device) if V >= 8192 else None
-        self.lib.check(self.lib.xr_sample(
-            out.data_ptr(), logits.data_ptr(), W, V, logits.stride(0), temp.data_ptr(), _ptr(top_k),
-            _ptr(top_p), _ptr(min_p), _ptr(repeat_penalty), draw.data_ptr(), _ptr(recent), _ptr(n_recent),
-            recent.shape[1] if recent is not None else 0, _ptr(exempt),
-            exempt.numel() if exempt is not None else 0, _ptr(greedy_ws), _stream()))
+        # room for the first pass (32 ranges a row) when a row is long enough to need one
+        part = torch.empty((W, 32, 2), dtype=torch.float32, device=logits.device) if V >= 8192 else None
+        args = (out.data_ptr(), logits.data_ptr(), W, V, logits.stride(0), temp.data_ptr(), _ptr(top_k),
+                _ptr(top_p), _ptr(min_p), _ptr(repeat_penalty), draw.data_ptr(), _ptr(recent), _ptr(n_recent),
+                recent.shape[1] if recent is not None else 0, _ptr(exempt), exempt.numel() if exempt is not None else 0, _ptr(part))
+        if part is not None and top_k is not None:
+            # Sampled rows (a batch without any brings no options): a row's histogram is shared out so that up to 512
+            # workgroups of 1,024 threads work on them, two a compute unit; more than 8 shares a row cost more to add up
+            # again than they save.
+            splits = max(1, min(8, 512 // max(1, W)))
+            ws = torch.empty((W * splits * _SAMPLE_BIN_BYTES,), dtype=torch.uint8, device=logits.device)
+            self.lib.check(self.lib.xr_sample_split(*args, ws.data_ptr(), ws.numel(), splits, _stream()))
+        else:
+            self.lib.check(self.lib.xr_sample(*args, _stream()))
         return out
 
 
+_SAMPLE_BIN_BYTES = 2048 * 12       # a share of a row's histogram: mass and number of the candidates of every bin
 _LOCK = threading.Lock()
 _OPS: Optional[Ops] = None
 
