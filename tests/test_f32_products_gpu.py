@@ -1,0 +1,35 @@
+"""The 32-bit product on the matrix cores and for few rows, at the edges of their tiles, runs and groups, against 64 bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# rows: one, the ends of the few-row kernel's groups, either side of its limit, of a tile's 32, 64 and 128; columns: less than a
+# slice of 32, no multiple of it, either side of a run of 128; weight rows: few, no multiple of a tile, enough for the large tile
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 33, 64, 65, 130])
+@pytest.mark.parametrize("N,K", [(7, 4), (96, 64), (100, 124), (65, 132), (200, 260), (16448, 68)])
+def test_product(M, N, K):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    rng = np.random.default_rng(M * 1000 + N + K)
+    a, w, bias, c = rng.normal(size=(M, K + 8)), rng.normal(size=(N, K)), rng.normal(size=N), rng.normal(size=(M, N))
+    t = lambda x: torch.tensor(x, dtype=torch.float32, device=dev)
+    at = t(a)[:, 4:4 + K]                                  # rows that are part of wider ones
+    exact = lambda x: x.double().cpu().numpy()
+    want = exact(at) @ exact(t(w)).T
+    # every product and sum rounds to 2^-24 of what has been added up so far: within K 2^-24 of the sum of magnitudes
+    bound = (K + 4) * 2.0 ** -24 * (np.abs(exact(at)) @ np.abs(exact(t(w))).T + np.abs(bias) + np.abs(c))
+    got = ops.linear(at, t(w))
+    assert (np.abs(exact(got) - want) <= bound).all()
+    with_bias = ops.linear(at, t(w), bias=t(bias))
+    assert (np.abs(exact(with_bias) - (want + exact(t(bias)))) <= bound).all()
+    out = t(c)
+    ops.linear(at, t(w), out=out, accumulate=True)
+    assert (np.abs(exact(out) - (want + exact(t(c)))) <= bound).all()
+    # a row's result does not depend on the rows beside it, within a kernel's range of rows
+    few = ops.linear(at[: max(1, M // 2)], t(w))
+    if (M <= 16) == (few.shape[0] <= 16):
+        assert torch.equal(few, got[: few.shape[0]])
+    assert torch.equal(ops.linear(at, t(w), out_dtype=torch.bfloat16), got.bfloat16())

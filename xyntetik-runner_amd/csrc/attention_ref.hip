@@ -1,6 +1,7 @@
 // Attention over the paged cache with 32-bit arithmetic only: the attention of the
 // true 32-bit path, for prompt portions and decoded tokens alike, any head size up
-// to 256.  One wave per (token, query head).
+// to 256.  k_attention_ref: one wave per (token, query head), any type.  k_attention_f32: 32-bit operands on the
+// matrix cores, a workgroup per 32 rows of a request and key/value head (below); same options, same result up to rounding.
 //
 // For the token at position p of its request and query head h (key/value head
 // h / (H/Hk), contiguous groups): s_t = (q . K_t) * scale for t in [lo, p], causal by
@@ -96,6 +97,240 @@ __global__ __launch_bounds__(64) void k_attention_ref(
         const int d = lane + 64 * dd;
         if (d < Dv) st<T>(orow, d, acc[dd] / l * f);
     }
+}
+
+// The same for 32-bit operands with the two products on the matrix cores (v_mfma_f32_16x16x4_f32: 32-bit operands, products
+// and sums).  A workgroup of four waves takes 32 rows (token x head of the group, token major) of one request and key/value
+// head and walks the keys they see in tiles of 64: keys and values through LDS, wave w the scores of keys 16 w .. 16 w + 15,
+// a softmax row a wave at a time, then wave w every fourth 16 channels of the output.  An MFMA step takes one
+// column from each quarter of the wave; a lane reads the four columns of its quarter at once and feeds four steps.
+// Keys that no row of the workgroup sees are never read (their pages may be gone) and count as zeros.
+// One wave a (token, head) walked the keys lane by lane, every lane a row of its own: 401 tokens, 32 heads of 64 took
+// 900 us and now 89, a decoded token of a tiny model 12 and now 7.
+#define AF_ROWS 32
+#define AF_KEYS 64
+#define AF_MAX_D 128
+#define AF_LD_S (AF_KEYS + 4)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct AttnF32 {
+    float* out;
+    const float* q;
+    const float* kc;
+    const float* vc;
+    const int* positions;
+    const int* cu_q;
+    const int* block_table;
+    const float* slopes;
+    const float* sinks;
+    const float* gate;
+    int table_stride, H, Hk, D, Dv, page_shift, page_mask, page_size, window, chunk, keep, ld_gate, ld_out;
+    float scale, cap, out_scale;
+};
+
+static inline int af_ld(int d) { return ((d + 15) & ~15) + 4; }
+static inline size_t af_lds_bytes(int D, int Dv) {
+    return sizeof(float) * ((size_t)(AF_ROWS + AF_KEYS) * af_ld(D) + (size_t)((Dv + 15) & ~15) * AF_LD_S + AF_ROWS * AF_LD_S);
+}
+
+__global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
+    extern __shared__ __align__(16) float lds[];
+    __shared__ int row_pos[AF_ROWS], row_lo[AF_ROWS];
+    __shared__ float row_corr[AF_ROWS], row_l[AF_ROWS], row_m[AF_ROWS];
+    const int b = blockIdx.z, kvh = blockIdx.y, G = a.H / a.Hk;
+    const int t0 = a.cu_q[b], nq = a.cu_q[b + 1] - t0;
+    const int r0 = blockIdx.x * AF_ROWS;                // of the request's nq * G rows
+    const int n_rows = nq * G - r0 < AF_ROWS ? nq * G - r0 : AF_ROWS;
+    if (n_rows <= 0) return;
+    const int D16 = (a.D + 15) & ~15, Dv16 = (a.Dv + 15) & ~15, ldd = D16 + 4;
+    float* Q = lds;
+    float* Kt = Q + AF_ROWS * ldd;
+    float* Vt = Kt + AF_KEYS * ldd;
+    float* S = Vt + Dv16 * AF_LD_S;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int* bt = a.block_table + (size_t)b * a.table_stride;
+
+    if (tid < AF_ROWS) {
+        const int r = tid < n_rows ? tid : n_rows - 1;  // (rows past the end repeat the last; nothing of them is written)
+        const int pos = a.positions[t0 + (r0 + r) / G];
+        row_pos[tid] = pos;
+        row_lo[tid] = a.chunk > 0 ? pos - pos % a.chunk : (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
+        row_m[tid] = -INFINITY;
+        row_l[tid] = 0.f;
+    }
+    for (int i = tid; i < AF_ROWS * D16 / 4; i += 256) {
+        const int r = i / (D16 / 4), d = (i - r * (D16 / 4)) * 4;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r < n_rows && d < a.D)
+            v = *reinterpret_cast<const float4*>(a.q + ((size_t)(t0 + (r0 + r) / G) * a.H + kvh * G + (r0 + r) % G) * a.D + d);
+        *reinterpret_cast<float4*>(Q + r * ldd + d) = v;
+    }
+    __syncthreads();
+    // positions rise with the rows, and so do the first keys
+    const int lo_min = row_lo[0], lo_max = row_lo[AF_ROWS - 1], hi = row_pos[AF_ROWS - 1] + 1;
+    const int kept_max = a.keep < lo_max ? a.keep : lo_max;     // first keys that stay readable behind the window
+    f32x4 acc[2][AF_MAX_D / 64];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int c = 0; c < AF_MAX_D / 64; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int l16 = lane & 15, quad = lane >> 4;
+    const int tiles = n_rows > 16 ? 2 : 1;
+
+    for (int seg = kept_max > 0 ? 0 : 1; seg < 2; ++seg) {
+        const int from = seg ? lo_min : 0, to = seg ? hi : kept_max;
+        for (int k0 = from & ~(AF_KEYS - 1); k0 < to; k0 += AF_KEYS) {
+            __syncthreads();                            // the tile before has been read
+            for (int i = tid; i < AF_KEYS * D16 / 4; i += 256) {
+                const int j = i / (D16 / 4), d = (i - j * (D16 / 4)) * 4, key = k0 + j;
+                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (key >= from && key < to && d < a.D)
+                    v = *reinterpret_cast<const float4*>(a.kc + (((size_t)bt[key >> a.page_shift] * a.Hk + kvh) * a.page_size + (key & a.page_mask)) * a.D + d);
+                *reinterpret_cast<float4*>(Kt + j * ldd + d) = v;
+            }
+            for (int i = tid; i < Dv16 * (AF_KEYS / 4); i += 256) {     // four keys of a channel lie in one page, side by side
+                const int d = i / (AF_KEYS / 4), j = (i - d * (AF_KEYS / 4)) * 4, key = k0 + j;
+                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (d < a.Dv && key + 3 >= from && key < to) {
+                    v = *reinterpret_cast<const float4*>(a.vc + (((size_t)bt[key >> a.page_shift] * a.Hk + kvh) * a.Dv + d) * a.page_size + (key & a.page_mask));
+                    if (key < from) v.x = 0.f;
+                    if (key + 1 < from || key + 1 >= to) v.y = 0.f;
+                    if (key + 2 < from || key + 2 >= to) v.z = 0.f;
+                    if (key + 3 >= to) v.w = 0.f;
+                }
+                *reinterpret_cast<float4*>(Vt + d * AF_LD_S + j) = v;
+            }
+            __syncthreads();
+            {   // scores: a lane has key 16 wave + lane % 16 and rows 4 (lane / 16) + e of each 16
+                f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                const float* kp = Kt + (16 * wave + l16) * ldd + 4 * quad;
+                const float* qp = Q + l16 * ldd + 4 * quad;
+                for (int d = 0; d < D16; d += 16) {
+                    const float4 fk = *reinterpret_cast<const float4*>(kp + d);
+                    const float4 f0 = *reinterpret_cast<const float4*>(qp + d);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fk.x)[x], s[0], 0, 0, 0);
+                    if (tiles > 1) {
+                        const float4 f1 = *reinterpret_cast<const float4*>(qp + 16 * ldd + d);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fk.x)[x], s[1], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) S[(16 * i + 4 * quad + e) * AF_LD_S + 16 * wave + l16] = s[i][e];
+            }
+            __syncthreads();
+            // softmax: rows wave, wave + 4, ...; a lane has one key
+            const int key = k0 + lane;
+#pragma unroll
+            for (int x = 0; x < AF_ROWS / 4; ++x) {
+                const int r = wave + 4 * x;
+                if (r >= n_rows) { if (r < 16 * tiles) S[r * AF_LD_S + lane] = 0.f; continue; }
+                const int pos = row_pos[r], lo = row_lo[r];
+                const bool valid = key >= from && key < to && (seg ? key >= lo && key <= pos : key < a.keep && key < lo);
+                float v = -INFINITY;
+                if (valid) {
+                    v = S[r * AF_LD_S + lane] * a.scale;
+                    if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
+                    if (a.slopes) v -= a.slopes[kvh * G + (r0 + r) % G] * (float)(pos - key);
+                }
+                const float m = row_m[r];
+                const float mn = fmaxf(m, wave_max(v));
+                const float p = valid ? expf(v - mn) : 0.f;
+                const float sum = wave_sum(p);
+                S[r * AF_LD_S + lane] = p;
+                if (lane == 0) {
+                    const float corr = m == -INFINITY ? 0.f : expf(m - mn);
+                    row_corr[r] = corr;
+                    row_l[r] = row_l[r] * corr + sum;
+                    row_m[r] = mn;
+                }
+            }
+            __syncthreads();
+            float corr[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) corr[i][e] = row_corr[16 * i + 4 * quad + e];
+#pragma unroll
+            for (int c = 0; c < AF_MAX_D / 64; ++c) {
+                const int d0 = 16 * (wave + 4 * c);
+                if (d0 >= Dv16) continue;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][c][e] *= corr[i][e];
+                const float* vp = Vt + (d0 + l16) * AF_LD_S + 4 * quad;
+                const float* pp = S + l16 * AF_LD_S + 4 * quad;
+#pragma unroll
+                for (int k = 0; k < AF_KEYS; k += 16) {
+                    const float4 fv = *reinterpret_cast<const float4*>(vp + k);
+                    const float4 f0 = *reinterpret_cast<const float4*>(pp + k);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fv.x)[x], acc[0][c], 0, 0, 0);
+                    if (tiles > 1) {
+                        const float4 f1 = *reinterpret_cast<const float4*>(pp + 16 * AF_LD_S + k);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) acc[1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fv.x)[x], acc[1][c], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    // a lane has channel lane % 16 of its 16 and rows 4 (lane / 16) + e
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 16 * i + 4 * quad + e;
+            if (r >= n_rows) continue;
+            const int t = t0 + (r0 + r) / G, h = kvh * G + (r0 + r) % G;
+            float l = row_l[r], corr = 1.f;
+            if (a.sinks) {                              // one more entry of the denominator, with nothing to add to the output
+                const float sk = a.sinks[h], mn = fmaxf(row_m[r], sk);
+                corr = expf(row_m[r] - mn);
+                l = l * corr + expf(sk - mn);
+            }
+            const float f = a.gate ? a.out_scale / (1.0f + expf(-a.gate[(size_t)t * a.ld_gate + h])) : a.out_scale;
+#pragma unroll
+            for (int c = 0; c < AF_MAX_D / 64; ++c) {
+                const int d = 16 * (wave + 4 * c) + l16;
+                if (d < a.Dv) a.out[(size_t)t * a.ld_out + (size_t)h * a.Dv + d] = acc[i][c][e] * corr / l * f;
+            }
+        }
+}
+
+// 32-bit operands, `B` requests with up to `max_q` tokens in the step (rows [cu_q[b], cu_q[b + 1]) are request b's, at rising positions).
+extern "C" int xr_attention_f32(float* out, const float* q, const float* k_cache, const float* v_cache, const int* positions,
+                                const int* cu_q, const int* block_table, int table_stride, int B, int max_q, int H, int Hk, int D,
+                                int Dv, int page_size, float scale, int window, int chunk, int keep, const float* slopes,
+                                const float* sinks, float cap, const float* gate, int ld_gate, float out_scale, int ld_out,
+                                hipStream_t stream) {
+    XR_REQUIRE(ld_out >= H * Dv && (!gate || ld_gate >= H), "attention: output rows %d apart, gate rows %d apart for %d heads of %d", ld_out, ld_gate, H, Dv);
+    XR_REQUIRE(cap >= 0.f, "attention: soft cap %g of the scores is negative", (double)cap);
+    XR_REQUIRE(B >= 0 && max_q >= 0 && H > 0 && Hk > 0 && H % Hk == 0, "attention: bad sizes B=%d of up to %d tokens, %d heads over %d", B, max_q, H, Hk);
+    XR_REQUIRE(D > 0 && D <= AF_MAX_D && D % 4 == 0 && Dv > 0 && Dv <= AF_MAX_D, "attention: head size %d (a multiple of 4) or value size %d exceeds %d", D, Dv, AF_MAX_D);
+    XR_REQUIRE(((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0, "attention: operands are not 16-byte aligned");
+    const int shift = ilog2_exact(page_size);
+    XR_REQUIRE(shift >= 2, "attention: page size %d is no power of two of at least 4", page_size);
+    XR_REQUIRE(window >= 0 && chunk >= 0 && keep >= 0, "attention: window %d, chunk %d or kept keys %d are negative", window, chunk, keep);
+    XR_REQUIRE(B <= 65535 && Hk <= 65535, "attention: %d requests, %d key/value heads", B, Hk);
+    if (B == 0 || max_q == 0) return XR_OK;
+    AttnF32 a{out, q, k_cache, v_cache, positions, cu_q, block_table, slopes, sinks, gate, table_stride, H, Hk, D, Dv, shift,
+              page_size - 1, page_size, window, chunk, keep, ld_gate, ld_out, scale, cap, out_scale};
+    const size_t bytes = af_lds_bytes(D, Dv);
+    if (bytes > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+        XR_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+    }
+    dim3 grid((unsigned)(((long long)max_q * (H / Hk) + AF_ROWS - 1) / AF_ROWS), Hk, B);
+    k_attention_f32<<<grid, 256, bytes, stream>>>(a);
+    XR_CHECK_LAUNCH("attention_f32");
+    return XR_OK;
 }
 
 extern "C" int xr_attention_ref(void* out, const void* q, const void* k_cache, const void* v_cache,

@@ -1,13 +1,14 @@
-// Plain matrix product out[M,N] = a[M,K] * w[N,K]^T (+ bias) with 32-bit FMA only:
-// the matrix product of the true 32-bit path, and the yardstick of the MFMA kernels.
+// Matrix product out[M,N] = a[M,K] * w[N,K]^T (+ bias) in true 32 bits: the matrix product of the 32-bit
+// path, and (k_gemm_ref, FMA only, any types and alignment) the yardstick of the bfloat16 MFMA kernels.
 // Weights are [n_out][n_in] row-major as the reference keeps them
 // (src/model.c:193-205).  A row's result does not depend on the rows beside it, but the order
 // of its sum over k depends on how many rows the product has: with more than 16 rows the tile
-// kernel below sums in ascending order in two levels, with up to 16 the kernel further down
+// kernels (k_gemm_f32 on the matrix cores, k_gemm_ref where operands are not 16-byte aligned or not 32-bit)
+// sum in two levels, with up to 16 the kernel further down
 // (k_gemv_ref) gives every lane every 64th group of four columns and adds the lanes' sums in a
 // tree.  A token's 32-bit result therefore differs in its last bits between a step of 16 rows and
 // one of 17 (both stay within 1e-6 of the exact product at K = 14,336).
-// The tile kernel's two levels: runs of RBK * RB_FOLD = 128 columns are summed by FMA, and the runs'
+// The tile kernels' two levels: runs of RBK * RB_FOLD = 128 columns are summed one after another, and the runs'
 // sums are added up with a compensated (Kahan) sum.  One running 32-bit sum over the 14,336
 // columns of a wide feed-forward loses about 1e-5 of the result to rounding, which at such
 // widths is as much as a real fault may be; summed this way a product is about ten times closer
@@ -87,17 +88,162 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
     }
 }
 
+// The same sums on the matrix cores (v_mfma_f32_32x32x2_f32: 32-bit operands, products and sums), 16-byte loads.
+// A workgroup of four waves, two by two, makes a tile of BM x BN; slices of 32 columns go through registers into
+// LDS, two buffers, the next slice's loads behind the current one's products.  An MFMA step takes two columns, one
+// from each half of the wave; which two does not matter as long as both operands agree, so a lane reads four columns at once
+// (its half's) and feeds four steps with them.  Rows in LDS are 36 floats apart: the 16-byte reads of 32 rows meet no bank twice.
+// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 runs at 111 TFLOP/s, 401 x 128256 x 2048 at 84 (a
+// fifth of the last row of tiles' work is padding), 401 x 2048 x 8192 at 63 (224 tiles of 64 x 64 for 256 compute units); the FMA
+// kernel above reached 18 to 25.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+#define FBK 32
+#define F_STRIDE (FBK + 4)
+
+template <typename TO, bool ACC, int BM, int BN>
+__global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+                                                     const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
+    constexpr int TM = BM / 64, TN = BN / 64;           // 32 x 32 tiles a wave
+    constexpr int LA = BM / 32, LW = BN / 32;           // 16-byte loads a thread and slice (a row of a slice is 8 of them)
+    __shared__ __align__(16) float As[2][BM * F_STRIDE];
+    __shared__ __align__(16) float Ws[2][BN * F_STRIDE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+    const int lr = tid >> 3, lk = (tid & 7) * 4;        // this thread's row (of every 32) and columns of a slice
+    float4 ra[LA], rw[LW];
+    auto fetch = [&](int k0) {
+        const int k = k0 + lk;
+#pragma unroll
+        for (int e = 0; e < LA; ++e) {
+            const int m = m0 + lr + 32 * e;
+            ra[e] = m < M && k < K ? *reinterpret_cast<const float4*>(a + (size_t)m * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int e = 0; e < LW; ++e) {
+            const int n = n0 + lr + 32 * e;
+            rw[e] = n < N && k < K ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto keep = [&](int buf) {
+#pragma unroll
+        for (int e = 0; e < LA; ++e) *reinterpret_cast<float4*>(&As[buf][(lr + 32 * e) * F_STRIDE + lk]) = ra[e];
+#pragma unroll
+        for (int e = 0; e < LW; ++e) *reinterpret_cast<float4*>(&Ws[buf][(lr + 32 * e) * F_STRIDE + lk]) = rw[e];
+    };
+    f32x16 acc[TM][TN], tot[TM][TN], lost[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = tot[i][j][e] = lost[i][j][e] = 0.f;
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float y = acc[i][j][e] - lost[i][j][e];
+                    const float t = tot[i][j][e] + y;
+                    lost[i][j][e] = (t - tot[i][j][e]) - y;
+                    tot[i][j][e] = t;
+                    acc[i][j][e] = 0.f;
+                }
+    };
+    const int row = lane & 31, half = (lane >> 5) * 4;
+    fetch(0);
+    keep(0);
+    __syncthreads();
+    int slice = 0;
+    for (int k0 = 0; k0 < K; k0 += FBK, ++slice) {
+        const int buf = slice & 1;
+        if (k0 + FBK < K) fetch(k0 + FBK);
+#pragma unroll
+        for (int kk = 0; kk < FBK; kk += 8) {
+            float4 fa[TM], fw[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const float4*>(&As[buf][(wm + 32 * i + row) * F_STRIDE + kk + half]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const float4*>(&Ws[buf][(wn + 32 * j + row) * F_STRIDE + kk + half]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((&fa[i].x)[s], (&fw[j].x)[s], acc[i][j], 0, 0, 0);
+        }
+        if ((slice + 1) % (RBK * RB_FOLD / FBK) == 0) fold();
+        if (k0 + FBK < K) keep(buf ^ 1);
+        __syncthreads();
+    }
+    fold();
+    // a lane has column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a tile
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int n = n0 + wn + 32 * j + row;
+        if (n >= N) continue;
+        const float add = bias ? bias[n] : 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + wm + 32 * i + 8 * (e >> 2) + half + (e & 3);
+                if (m >= M) continue;
+                const size_t at = (size_t)m * ldo + n;
+                float v = tot[i][j][e];
+                if (bias) v += add;
+                if (ACC) v += ld<TO>(out, at);
+                st<TO>(out, at, v);
+            }
+    }
+}
+
+template <int BM, int BN>
+static void launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
+                            int out_dtype, int accumulate, hipStream_t stream) {
+    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    if (out_dtype == XR_BF16) k_gemm_f32<bf16_t, false, BM, BN><<<grid, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo);
+    else if (accumulate) k_gemm_f32<float, true, BM, BN><<<grid, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+    else k_gemm_f32<float, false, BM, BN><<<grid, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+}
+
 // Up to 16 rows of 32-bit operands (decoded tokens): the product is bound by how fast the weights
 // arrive, and the tile kernel above, 64 weight rows a workgroup, leaves most of the chip idle then
-// (a decode step of the Llama-3.1-8B shape took 136 ms).  Here a wave takes 8 weight rows: a lane
+// (a decode step of the Llama-3.1-8B shape took 136 ms).  Here a wave takes COLS weight rows: a lane
 // sums, for every row of `a` and each of them, the columns 4 l .. 4 l + 3 (mod 256) in ascending
 // order by FMA, and the lanes' sums are added in a fixed tree.  A row's result does not depend
 // on the rows beside it; it differs from the tile kernel's by the order of the sum only.
-template <int MT, typename TO, bool ACC>
+// All sums go through the tree at once: at the first step a lane hands half of its sums to the lane 32 further and
+// takes over the other half, and so on, until a lane holds the whole sum of one (row, weight row) or what is left of few sums
+// goes on as a plain tree.  The additions are those of a tree a sum, in the same order.  (Three rows through 64 x 64 weights:
+// 3.4 us with 2 weight rows a wave and one tree, 9.5 us with 8 weight rows and a tree of six steps for each of 32 sums.)
+template <int N>
+__device__ inline void tree_sums(float (&v)[N], int lane, int& mine) {
+    mine = 0;
+    int o = 32;
+#pragma unroll
+    for (int n = N; n > 1; n >>= 1) {
+        if (o > 0) {
+            const bool up = lane & o;
+            mine = 2 * mine + (up ? 1 : 0);
+#pragma unroll
+            for (int i = 0; i < n / 2; ++i) {
+                const float keep = up ? v[n / 2 + i] : v[i], give = up ? v[i] : v[n / 2 + i];
+                v[i] = keep + __shfl_xor(give, o, 64);
+            }
+            o >>= 1;
+        }
+    }
+    for (; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o, 64);
+}
+
+template <int MT, int COLS, typename TO, bool ACC>
 __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const float* __restrict__ a,
                                                    const float* __restrict__ w, const float* __restrict__ bias,
                                                    int M, int N, int K, int lda, int ldo) {
-    constexpr int COLS = 8;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n0 = (blockIdx.x * 4 + wave) * COLS;
     if (n0 >= N) return;
@@ -126,30 +272,42 @@ __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const fl
             }
         }
     }
+    // 64 sums at a time (a lane ends with one), or all of them where they are fewer
+    constexpr int ALL = COLS * MT, GROUP = ALL < 64 ? ALL : 64;
 #pragma unroll
-    for (int c = 0; c < COLS; ++c)
+    for (int g0 = 0; g0 < ALL; g0 += GROUP) {
+        float v[GROUP];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            float v = acc[c][m];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            const int n = n0 + c;
-            if (lane == 0 && m < M && n < N) {
-                if (bias) v += bias[n];
-                const size_t at = (size_t)m * ldo + n;
-                if (ACC) v += ld<TO>(out, at);
-                st<TO>(out, at, v);
-            }
+        for (int i = 0; i < GROUP; ++i) v[i] = acc[(g0 + i) / MT][(g0 + i) % MT];
+        int mine;
+        tree_sums<GROUP>(v, lane, mine);
+        const int n = n0 + (g0 + mine) / MT, m = (g0 + mine) % MT;
+        if ((lane & (64 / GROUP - 1)) == 0 && m < M && n < N) {
+            float s = v[0];
+            if (bias) s += bias[n];
+            const size_t at = (size_t)m * ldo + n;
+            if (ACC) s += ld<TO>(out, at);
+            st<TO>(out, at, s);
         }
+    }
 }
 
+template <int MT, int COLS>
+static void launch_gemv_cols(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
+                             int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
+    const unsigned blocks = (unsigned)((N + 4 * COLS - 1) / (4 * COLS));
+    if (out_dtype == XR_BF16) k_gemv_ref<MT, COLS, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo);
+    else if (accumulate) k_gemv_ref<MT, COLS, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+    else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+}
+
+// Weight rows a wave: 8 share the reads of `a`, but only where that still gives every compute unit two workgroups;
+// below that a wave takes 2 (a product of 2,048 weight rows: 256 workgroups instead of 64).
 template <int MT>
 static void launch_gemv_ref(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
                             int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
-    const unsigned blocks = (unsigned)((N + 31) / 32);
-    if (out_dtype == XR_BF16) k_gemv_ref<MT, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo);
-    else if (accumulate) k_gemv_ref<MT, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
-    else k_gemv_ref<MT, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+    if (N >= 2 * 256 * 32) launch_gemv_cols<MT, 8>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+    else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
 }
 
 // accumulate != 0: out (float) += product.
@@ -159,10 +317,19 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
     XR_REQUIRE(lda >= K && ldo >= N, "gemm: row strides lda=%d ldo=%d are shorter than K=%d N=%d", lda, ldo, K, N);
     XR_REQUIRE(!accumulate || out_dtype == XR_F32, "gemm: accumulation needs a 32-bit output");
     if (M == 0) return XR_OK;
-    if (M <= 16 && in_dtype == XR_F32 && (out_dtype == XR_F32 || out_dtype == XR_BF16) && K % 4 == 0 && lda % 4 == 0 &&
+    if (in_dtype == XR_F32 && (out_dtype == XR_F32 || out_dtype == XR_BF16) && K % 4 == 0 && lda % 4 == 0 &&
         ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0) {
         const float* af = (const float*)a;
         const float* wf = (const float*)w;
+        if (M > 16) {
+            // 128 x 64 tiles read three quarters of what 64 x 64 ones read from L2, but two of their workgroups fill a compute
+            // unit: they are taken where there are at least that many (128 x 128 tiles with their three sums a value spill)
+            const long long tiles = (long long)((M + 127) / 128) * ((N + 63) / 64);
+            if (tiles >= 512) launch_gemm_f32<128, 64>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            else launch_gemm_f32<64, 64>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            XR_CHECK_LAUNCH("gemm_f32");
+            return XR_OK;
+        }
         if (M == 1) launch_gemv_ref<1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
         else if (M <= 4) launch_gemv_ref<4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
         else if (M <= 8) launch_gemv_ref<8>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);

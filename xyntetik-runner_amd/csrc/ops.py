@@ -68,6 +68,7 @@ _PROTOS = {
     "xr_gemm_bf16": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p, _p, _p],
     "xr_pack_weight": [_p, _p, _i, _i, _p],
     "xr_rope_table": [_p, _p, _p, _i, _i, _f, _p],
+    "xr_attention_f32": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _p, _p, _f, _p, _i, _f, _i, _p],
     "xr_attention_ref": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _i, _p, _p, _f, _p, _i, _f, _i, _p],
     "xr_head_norm_rope_write": [_p, _p, _p, _i, _p, _p, _f, _i, _p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p],
     "xr_ssd_chunks": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
@@ -807,6 +808,14 @@ class Ops:
                 ctx.starts_dev.data_ptr(), block_table.data_ptr(), block_table.stride(0), _ptr(part_o), _ptr(part_ml), H, Hk, D, Dv, page_size,
                 float(scale), int(window or 0), int(chunk or 0), _ptr(slopes), None if extra else _ptr(sinks),
                 float(softcap), *gating, _stream()))
+            return out
+        if (q.dtype == torch.float32 and D % 4 == 0 and D <= 128 and Dv <= 128 and page_size >= 4
+                and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) & 15):
+            # 32-bit rows on the matrix cores: 32 rows of a request a workgroup (larger heads do not fit LDS)
+            self.lib.check(self.lib.xr_attention_f32(
+                out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr(), ctx.cu_q.data_ptr(),
+                block_table.data_ptr(), block_table.stride(0), len(ctx.q_lens), max(ctx.q_lens), H, Hk, D, Dv, page_size, float(scale),
+                int(window or 0), int(chunk or 0), int(keep_first), _ptr(slopes), _ptr(sinks), float(softcap), *gating, _stream()))
             return out
         self.lib.check(self.lib.xr_attention_ref(
             out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr(),
