@@ -492,12 +492,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
     // equal shares, and those of a share's missing column leave at once.)  (Measured on the 8B shape's prompt
     // step of 2,048 rows against m_fast 1: 29.4 -> 27.9 ms.  With 32 row tiles, in groups of 8 x 4
     // tiles an XCD, it lost: 8192 x 28672 x 4096 in 1,776 us against 1,456.)
+    // m_fast 3: the same with an eighth of the tiles an XCD, whole columns or not, where whole columns would give
+    // some XCDs a round of 32 workgroups more (252 tiles of 6 rows x 42 columns: 36 on two XCDs, 30 on the others;
+    // 1536 x 12288 x 4096 took 233 us and now 152).  Shares that begin within a column cost 1% elsewhere.
     int bm_v, bn_v;
     if (g.m_fast == 2) {
         const int l = tile_ >> 3;
         bm_v = l % tiles_m;
         bn_v = (l / tiles_m) * 8 + (tile_ & 7);
         if (bn_v >= tiles_n) return;
+    } else if (g.m_fast == 3) {
+        const int share = (tiles_m * tiles_n + 7) >> 3, t = (tile_ & 7) * share + (tile_ >> 3);
+        if (t >= tiles_m * tiles_n) return;
+        bm_v = t % tiles_m;
+        bn_v = t / tiles_m;
     } else {
         bm_v = g.m_fast ? tile_ % tiles_m : tile_ / tiles_n;
         bn_v = g.m_fast ? tile_ / tiles_m : tile_ % tiles_n;
@@ -1069,7 +1077,11 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     unsigned tiles_n = (unsigned)((g.col1 - g.col0 + n_out_tile - 1) / n_out_tile), tiles_m = (unsigned)((g.M + BM - 1) / BM);
     unsigned tiles = tiles_n * tiles_m;
     if (g.m_fast == 2 && (tiles_m > 8 || tiles_n < 8)) g.m_fast = 1;
-    if (g.m_fast == 2) tiles = 8 * tiles_m * ((tiles_n + 7) / 8);
+    if (g.m_fast == 2) {
+        const unsigned columns = tiles_m * ((tiles_n + 7) / 8), even = (tiles + 7) / 8;       // tiles of the XCD that has most
+        if ((columns + 31) / 32 > (even + 31) / 32) g.m_fast = 3;
+        tiles = 8 * (g.m_fast == 3 ? even : columns);
+    }
     if (g.splits < 1 || !g.partial || g.col0 > 0 || g.col1 < g.N) g.splits = 1;
     if (g.splits > 1) {
         int slices = (g.K + 63) / 64;
