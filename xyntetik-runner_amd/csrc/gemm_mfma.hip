@@ -1548,55 +1548,51 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         } else if (M <= 64) {
             variant = 31;
         } else {
-            // The tile that keeps the chip busiest: larger tiles do more products for a byte that
-            // L1 delivers (what bounds this kernel), but their count may fill the 256 compute
-            // units badly.  A tile's time is its area over its measured rate with the chip full
-            // (relative to 256x256); a launch takes as many of these as its tiles make rounds of
-            // 256.  When the last round of the best tile would leave most of the chip idle, the
+            // The tile and the number of K ranges that should take the least time.  Larger tiles do more products for
+            // a byte that L1 delivers, but their count may fill the 256 compute units badly: a launch takes as many
+            // rounds as its workgroups make of 256.  Where tiles are few, K is split among workgroups (one round of them), and
+            // a kernel adds the ranges up.  When the last round of the best tile would leave most of the chip idle, the
             // columns of the full rounds go to that tile and the rest to a second launch with a
-            // smaller one (3 rounds + 1 of half-size tiles instead of 4).  A tile shape whose tiles
-            // are too few for the chip competes with K split among workgroups (below).
-            // (The 256 compute units and the tiles' relative rates below are tuning measured on an
-            // MI355X with the 8B shape's products, not limits: elsewhere they cost speed only.)
-            // (rate: of the tile's products, relative to 256x256; fixed: seconds a round beside them.  At
-            // 2,048 rows a round of 256x256 tiles took 107 us with K = 4,096 and 191 with 7,168, one of
-            // 256x128 tiles 61 us with K = 4,096 and 194 with 14,336, one of 256x192 tiles 118.)
-            struct Cand { int variant, bm, bn; double rate, fixed; };
-            const double four = rope_direct ? 0.85 : 1.0;        // (the eight-wave kernels of these tiles, which a rotating product takes)
-            const Cand cands[4] = {{14, 256, 256, 1.0 * four, 0.0}, {26, 256, 192, 0.73, 8e-6}, {12, 256, 128, 1.0 * four, 8e-6},
-                                   {17, 128, 128, 0.63, 0.0}};
+            // smaller one (3 rounds + 1 of half-size tiles instead of 4).
+            // The model, in seconds (tuning measured on an MI355X, not limits: elsewhere it costs speed only): a round of
+            // tiles takes its products' time, bm bn K x 0.36e-12 / rate (97 us for 256x256 and K = 4,096 as measured), or that of its
+            // weights from memory at `bytes` a second, whichever is longer; `launch` once and `round` for every round (a product that
+            // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
+            // at 2.2 TB/s and costs a launch, and writes the norm that follows, if one was asked for: without
+            // ranges its kernel takes 19 us with what lies around it.  Fitted to 3,800 timed launches (the 8B and the 1B class's four
+            // products and Suripel's two, 72 to 2,048 rows, four tiles, 1 to 16 ranges): the tile chosen is 1.2% slower
+            // than the best of them on average, 6.6% with the model before it (which knew no memory time and too high a
+            // price for 128x128 tiles: down at 137 rows in 256x256 tiles and 16 ranges 45-53 us, in 256x128 and 6 ranges 39-45;
+            // a 4,096 to 6,144 product of 400 rows 47 us, in whole 128x128 tiles 32).
+            // (Rotating products: the eight-wave kernels, but 128x128 tiles with four waves: 600 rows of a 4,096 to 6,144 product 42 us
+            // against 53, 800 rows 72 against 98.)
+            struct Cand { int variant, bm, bn; double rate, launch, round, bytes; };
+            const Cand plain[4] = {{14, 256, 256, 1.0, 5.8e-6, 0.0, 5.0e12}, {26, 256, 192, 0.95, 3.7e-6, 0.0, 5.0e12},
+                                   {12, 256, 128, 0.95, 5.1e-6, 0.0, 4.1e12}, {17, 128, 128, 0.72, 3.9e-6, 0.0, 4.1e12}};
+            const Cand turning[4] = {{14, 256, 256, 0.95, 0.0, 8e-6, 5.0e12}, {26, 256, 192, 0.81, 0.0, 9e-6, 5.0e12},
+                                     {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {58, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
+            const Cand* cands = rope_direct ? turning : plain;
             auto width = [&](const Cand& c) { return sw ? c.bn / 2 : c.bn; };
             auto usable = [&](const Cand& c) { return !(sw && c.variant == 26); };
             auto count = [&](const Cand& c, int cols) { return ((M + c.bm - 1) / c.bm) * ((cols + width(c) - 1) / width(c)); };
-            // Times in seconds: a 256x256 tile's products over K columns take 65536 K x 0.4e-12 s at
-            // full rate (107 us at K = 4,096, as measured).  A launch whose tiles are too few for the
-            // chip (under 160) may split K so that its workgroups make one round; the kernel that then
-            // adds the ranges up moves (ranges x their width + 2 x N) x M x 4 bytes at about 4.5 TB/s
-            // and costs a launch, and it writes the norm that follows, if one was asked for, which
-            // saves that kernel (11 us at 2,048 x 4,096).  Measured against this model at 256 to 1,024
-            // rows (us, model / measured): down at 512 rows in 256x128 tiles and 4 ranges 79 / 74-79, in
-            // 128x128 and 2 ranges 90 / 94, in 256x256 and 8 ranges 80 / 79; q/k/v at 256 rows in 256x128
-            // and 5 ranges 28 / 32, in 128x128 and 2 ranges 31 / 36.
-            const double unit = 0.4e-12;
-            auto seconds = [&](const Cand& c, int cols) {
-                return (double)((count(c, cols) + 255) / 256) * ((double)c.bm * c.bn / c.rate * K * unit + c.fixed);
+            auto seconds = [&](const Cand& c, int cols, int ranges) {
+                const int groups = count(c, cols) * ranges, rounds = (groups + 255) / 256, rows = (M + c.bm - 1) / c.bm;
+                const double k = (K + ranges - 1) / ranges, products = (double)c.bm * c.bn * k * 0.36e-12 / c.rate;
+                const double weights = (double)(groups < 256 ? groups : 256) * c.bn * k * 2 / rows / c.bytes;
+                return rounds * ((products > weights ? products : weights) + c.round) + c.launch;
             };
-            auto adding = [&](int ranges) {
-                return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 4.5e12 + 3e-6 - (want_whole_norm ? 11e-6 : 0.0);
-            };
+            auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.2e12 + 4e-6; };
+            const double norm_alone = want_whole_norm ? 19e-6 : 0.0;
             int best = 0, best_splits = 1, second = -1, cols_first = N;
             double t_best = 1e30;
             for (int i = 0; i < 4; ++i) {
                 if (!usable(cands[i])) continue;
                 const int c = count(cands[i], N);
-                double t = seconds(cands[i], N);
-                int sp = 1;
-                if (c < 160 && workspace && !rope_direct) {
-                    const int s2 = pick_splits(c);
-                    const double ts = (double)cands[i].bm * cands[i].bn / cands[i].rate * ((K + s2 - 1) / s2) * unit + cands[i].fixed + adding(s2);
-                    if (s2 >= 2 && ts < t) { t = ts; sp = s2; }
+                for (int sp = 1; sp <= 16; ++sp) {
+                    if (sp > 1 && (rope_direct || !workspace || c * sp > 256 || K / sp < 256 || (size_t)sp * M * w_rows * 4 > workspace_bytes)) break;
+                    const double t = seconds(cands[i], N, sp) + (sp > 1 ? adding(sp) : norm_alone);
+                    if (t < t_best) { best = i; best_splits = sp; t_best = t; }
                 }
-                if (t < t_best) { best = i; best_splits = sp; t_best = t; }
             }
             for (int i = 0; i < 3; ++i) {
                 if (!usable(cands[i])) continue;
@@ -1605,8 +1601,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                 if (full < 1 || count(cands[i], N) % 256 == 0 || cols <= 0 || cols >= N) continue;
                 for (int j = i + 1; j < 4; ++j) {
                     if (!usable(cands[j]) || cols % width(cands[j])) continue;
-                    const double t = seconds(cands[i], cols) + seconds(cands[j], N - cols);
-                    if (t < 0.92 * t_best) { best = i; best_splits = 1; second = j; cols_first = cols; t_best = t; }   // (a second launch costs a little, too)
+                    const double t = seconds(cands[i], cols, 1) + seconds(cands[j], N - cols, 1) + norm_alone;
+                    if (t < 0.98 * t_best) { best = i; best_splits = 1; second = j; cols_first = cols; t_best = t; }   // (a second launch costs a little, too)
                 }
             }
             variant = cands[best].variant;
