@@ -22,7 +22,7 @@
 // each 50 us, so a row's histogram is shared out to up to 8 workgroups where the caller brings room for their
 // partial counts; the cuts are a chain of short steps that one workgroup a row walks.
 // Where every cut was a radix selection (22 passes over the row for top-p) 64 rows of 128,256 logits
-// took 1,150 us and one row 900.
+// took 1,150 us; now 57 in three kernels (6 + 17 + 34).
 #include "common.h"
 #include "no_alloc.h"
 
@@ -84,18 +84,31 @@ __device__ inline float key_z(u64 key) {
 }
 
 // f(value, index) for the candidates [lo, hi) of a row, `step` threads side by side; lo is a multiple of 4.
-// 16-byte loads where the row's address allows it: one load instruction for four candidates.
+// 16-byte loads where the row's address allows it, up to 8 of them on their way before the first value is looked at (one
+// after the other, a workgroup's pass over 128k logits is 31 trips to memory: k_sample for 64 rows 45 us, now 34).
 template <typename F>
-__device__ inline void for_row(const float* row, int lo, int hi, int tid, int step, F f) {
+__device__ __forceinline__ void for_row(const float* row, int lo, int hi, int tid, int step, F f) {
     int tail = lo;
     if (((uintptr_t)row & 15) == 0) {
+        constexpr int U = 8;
         tail = lo + ((hi - lo) & ~3);
-        for (int i = lo + 4 * tid; i < tail; i += 4 * step) {
-            const float4 v = *reinterpret_cast<const float4*>(row + i);
-            f(v.x, i);
-            f(v.y, i + 1);
-            f(v.z, i + 2);
-            f(v.w, i + 3);
+        for (int i0 = lo + 4 * tid; i0 < tail; i0 += 4 * step * U) {
+            float4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + 4 * step * u;
+                v[u] = *reinterpret_cast<const float4*>(row + (i < tail ? i : i0));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + 4 * step * u;
+                if (i < tail) {
+                    f(v[u].x, i);
+                    f(v[u].y, i + 1);
+                    f(v[u].z, i + 2);
+                    f(v[u].w, i + 3);
+                }
+            }
         }
     }
     for (int i = tail + tid; i < hi; i += step) f(row[i], i);
@@ -188,7 +201,7 @@ __device__ inline bool row_item(const RowView& rv, int i, u64& key, u64& mass) {
     return true;
 }
 
-__device__ u64 block_sum_u64(u64 v, u64* sh) {
+__device__ __forceinline__ u64 block_sum_u64(u64 v, u64* sh) {
     // sh has SM_THREADS / 64 entries
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -202,7 +215,7 @@ __device__ u64 block_sum_u64(u64 v, u64* sh) {
 }
 
 // Mass (by_mass) or number of the kept candidates.
-__device__ u64 kept_total(const RowView& rv, bool by_mass, u64* sh) {
+__device__ __forceinline__ u64 kept_total(const RowView& rv, bool by_mass, u64* sh) {
     u64 acc = 0;
     for (int i = threadIdx.x; i < rv.V; i += SM_THREADS) {
         u64 key, mass;
@@ -214,7 +227,7 @@ __device__ u64 kept_total(const RowView& rv, bool by_mass, u64* sh) {
 // Smallest key B among the kept candidates with F(B) > target, where F(B) is the mass
 // (by_mass) or the number of kept candidates with key <= B.  If no key reaches the
 // target the largest kept key is returned.
-__device__ u64 radix_select(const RowView& rv, bool by_mass, u64 target,
+__device__ __forceinline__ u64 radix_select(const RowView& rv, bool by_mass, u64 target,
                                            u64* hist, u64* sh2) {
     u64 prefix = 0, remaining = target;
     for (int shift = 48; shift >= 0; shift -= 8) {
@@ -284,8 +297,8 @@ __device__ inline void row_extent(const float* part, int r, float& mx, float& mn
 
 // Mass and (with `counts`) number of the candidates [lo, hi) by bin, added to `mass` and `count` in LDS.
 // (a candidate that is no number is in no bin)
-__device__ inline void fill_hist(const float* row, int lo, int hi, float temp, const Bins& bins, bool counts, u64* mass, unsigned* count) {
-    for_row(row, lo, hi, threadIdx.x, SM_THREADS, [&](float v, int) {
+__device__ __forceinline__ void fill_hist(const float* row, int lo, int hi, float temp, const Bins& bins, bool counts, u64* mass, unsigned* count) {
+    for_row(row, lo, hi, threadIdx.x, SM_THREADS, [&](float v, int) __attribute__((always_inline)) {
         const float z = v / temp;
         if (z != z) return;
         const int b = bins.of(z);
@@ -349,7 +362,7 @@ struct List {
 };
 
 // Gather and sort the bins [lo, hi]; false: more candidates than the list holds.
-__device__ bool gather(const float* row, int V, float temp, const Bins& bins, int lo, int hi, List& list, u64* sh) {
+__device__ __forceinline__ bool gather(const float* row, int V, float temp, const Bins& bins, int lo, int hi, List& list, u64* sh) {
     __syncthreads();
     if (threadIdx.x == 0) { list.n = 0; list.lo = lo; list.hi = hi; }
     __syncthreads();
@@ -358,7 +371,7 @@ __device__ bool gather(const float* row, int V, float temp, const Bins& bins, in
     const float above = hi == SM_BINS - 1 ? -INFINITY : bins.zmax - (float)(hi + 1) / bins.scale - slack;
     const float below = bins.zmax - (float)lo / bins.scale + slack;
     const float vlo = above * temp - 1e-6f * fabsf(above * temp), vhi = below * temp + 1e-6f * fabsf(below * temp);
-    for_row(row, 0, V, threadIdx.x, SM_THREADS, [&](float v, int i) {
+    for_row(row, 0, V, threadIdx.x, SM_THREADS, [&](float v, int i) __attribute__((always_inline)) {
         if (!(v >= vlo && v <= vhi)) return;
         const float z = v / temp;
         const int b = bins.of(z);
@@ -387,7 +400,7 @@ __device__ bool gather(const float* row, int V, float temp, const Bins& bins, in
 }
 
 // The list's sums of mass; a candidate with exp(z - z_max) < min_e or a key over `limit` counts nothing.
-__device__ void sum_list(List& list, float zmax, float min_e, u64 limit, u64* sh) {
+__device__ __forceinline__ void sum_list(List& list, float zmax, float min_e, u64 limit, u64* sh) {
     const int i = 2 * threadIdx.x;
     u64 m[2];
 #pragma unroll
@@ -407,7 +420,7 @@ __device__ void sum_list(List& list, float zmax, float min_e, u64 limit, u64* sh
 
 // The first index whose inclusive sum exceeds `target` (there is one), the same in all threads.
 template <typename T>
-__device__ int first_over(const T* sums, int n, T before, T target, int* sh1) {
+__device__ __forceinline__ int first_over(const T* sums, int n, T before, T target, int* sh1) {
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += SM_THREADS)
         if (before + sums[i] > target && (i == 0 || !(before + sums[i - 1] > target))) *sh1 = i;
@@ -416,7 +429,7 @@ __device__ int first_over(const T* sums, int n, T before, T target, int* sh1) {
 }
 
 // The pick where a cut's bin does not fit the list: every boundary by a radix selection over the row.
-__device__ int sample_by_radix(const SampleArgs& a, int r, const float* row, float temp, float zmax, u64* hist, u64* sh, u64* sh2) {
+__device__ __forceinline__ int sample_by_radix(const SampleArgs& a, int r, const float* row, float temp, float zmax, u64* hist, u64* sh, u64* sh2) {
     RowView rv;
     rv.row = row; rv.V = a.V; rv.temp = temp; rv.zmax = zmax;
     rv.limit = ~0ull; rv.min_e = 0.f;
@@ -437,7 +450,7 @@ __device__ int sample_by_radix(const SampleArgs& a, int r, const float* row, flo
 }
 
 // The pick of a sampled row, from its bins' inclusive sums; -1: a cut's bin does not fit the list.
-__device__ int sample_by_bins(const SampleArgs& a, int r, const float* row, float temp, const Bins& bins, const u64* mass,
+__device__ __forceinline__ int sample_by_bins(const SampleArgs& a, int r, const float* row, float temp, const Bins& bins, const u64* mass,
                               const unsigned* count, List& list, u64* sh, int* sh1) {
     bool have = false;          // (the same in all threads, as is every cut below)
     auto need = [&](int lo, int hi) {
@@ -568,11 +581,18 @@ __global__ __launch_bounds__(SM_THREADS) void k_sample(SampleArgs a) {
     u64 m0 = 0, m1 = 0;
     unsigned c0 = 0, c1 = 0;
     if (a.hist_mass) {
-        for (int s = 0; s < a.hist_splits; ++s) {
-            const size_t at = ((size_t)r * a.hist_splits + s) * SM_BINS + b0;
-            m0 += a.hist_mass[at];
-            m1 += a.hist_mass[at + 1];
-            if (counts) { c0 += a.hist_count[at]; c1 += a.hist_count[at + 1]; }
+        for (int s0 = 0; s0 < a.hist_splits; s0 += 8) {      // (eight shares' loads side by side)
+            ulonglong2 m[8];
+            uint2 c[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const size_t at = ((size_t)r * a.hist_splits + (s0 + u < a.hist_splits ? s0 + u : s0)) * SM_BINS + b0;
+                m[u] = *reinterpret_cast<const ulonglong2*>(a.hist_mass + at);
+                c[u] = counts ? *reinterpret_cast<const uint2*>(a.hist_count + at) : make_uint2(0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (s0 + u < a.hist_splits) { m0 += m[u].x; m1 += m[u].y; c0 += c[u].x; c1 += c[u].y; }
         }
     } else {
         mass[b0] = mass[b0 + 1] = 0;
@@ -640,7 +660,7 @@ extern "C" int xr_sample_split(int* out, float* logits, int W, int V, int ld, co
                                const int* exempt, int n_exempt, float* greedy_ws, void* hist_ws, long long hist_bytes,
                                int splits, hipStream_t stream) {
     XR_REQUIRE(greedy_ws && hist_ws && splits > 0 && splits <= 32, "sample_split: no work area or %d splits", splits);
-    XR_REQUIRE(((uintptr_t)hist_ws & 7) == 0 && hist_bytes >= (long long)W * splits * SM_BINS * 12, "sample_split: a work area of %lld bytes for %d rows in %d parts",
+    XR_REQUIRE(((uintptr_t)hist_ws & 15) == 0 && hist_bytes >= (long long)W * splits * SM_BINS * 12, "sample_split: a work area of %lld bytes for %d rows in %d parts",
                hist_bytes, W, splits);
     return sample_launch(out, logits, W, V, ld, temp, top_k, top_p, min_p, repeat_penalty, draw, recent, n_recent,
                          recent_cap, exempt, n_exempt, greedy_ws, (u64*)hist_ws, splits, stream);
