@@ -14,6 +14,7 @@
 // widths is as much as a real fault may be; summed this way a product is about ten times closer
 // to the exact one, so the 32-bit path can be held to the tolerance that small models are.
 #include "common.h"
+#include "async_copy.h"
 
 #define RBM 64
 #define RBN 64
@@ -88,48 +89,53 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
     }
 }
 
-// The same sums on the matrix cores (v_mfma_f32_32x32x2_f32: 32-bit operands, products and sums), 16-byte loads.
-// A workgroup of four waves, two by two, makes a tile of BM x BN; slices of 32 columns go through registers into
-// LDS, two buffers, the next slice's loads behind the current one's products.  An MFMA step takes two columns, one
-// from each half of the wave; which two does not matter as long as both operands agree, so a lane reads four columns at once
-// (its half's) and feeds four steps with them.  Rows in LDS are 36 floats apart: the 16-byte reads of 32 rows meet no bank twice.
-// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 runs at 111 TFLOP/s, 401 x 128256 x 2048 at 84 (a
-// fifth of the last row of tiles' work is padding), 401 x 2048 x 8192 at 63 (224 tiles of 64 x 64 for 256 compute units); the FMA
+// The same sums on the matrix cores (v_mfma_f32_32x32x2_f32: 32-bit operands, products and sums), 16-byte pieces copied
+// straight into LDS.  A workgroup of four waves, two by two, makes a tile of BM x BN from slices of 32 columns, STAGES - 1 of
+// them on their way while one is used: a slice's products take a wave 1,000 to 2,000 cycles, less than a trip to memory
+// (with the next slice alone ahead of the products, through registers, 401 x 2048 x 8192 took 213 us and 2048 x 16384 x 2048 1,237).
+// An MFMA step takes two columns, one from each half of the wave; which two does not matter as long as both operands agree,
+// so a lane reads four columns at once (its half's) and feeds four steps with them.  A row's eight pieces lie turned by
+// half its number, so that the reads of 16 rows meet no bank twice.  Workgroup i runs on XCD i % 8, and an XCD takes an
+// eighth of the tiles, row tiles first: a weight tile comes from memory for one XCD (401 x 128256 x 2048, 1 GB of weights, read
+// them four times with the column tiles first).
+// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 at 112 TFLOP/s, 401 x 128256 x 2048 at 100 (84 before),
+// 401 x 2048 x 8192 at 69 (63; 224 tiles for 256 compute units, one wave a SIMD, which waits out its own reads); the FMA
 // kernel above reached 18 to 25.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define FBK 32
-#define F_STRIDE (FBK + 4)
 
-template <typename TO, bool ACC, int BM, int BN>
+template <typename TO, bool ACC, int BM, int BN, int STAGES>
 __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
                                                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
     constexpr int TM = BM / 64, TN = BN / 64;           // 32 x 32 tiles a wave
-    constexpr int LA = BM / 32, LW = BN / 32;           // 16-byte loads a thread and slice (a row of a slice is 8 of them)
-    __shared__ __align__(16) float As[2][BM * F_STRIDE];
-    __shared__ __align__(16) float Ws[2][BN * F_STRIDE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    constexpr int ROWS = BM + BN, CH = FBK / 4;         // rows of a slice (activations, then weights), pieces of a row
+    constexpr int LOADS = ROWS * CH / 256;              // copies a lane and slice
+    static_assert(BM % 32 == 0 && LOADS * STAGES < 64, "whole copy instructions, and a count that fits the counter");
+    extern __shared__ __align__(16) float4 lds[];       // [STAGES][ROWS][CH]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN);
+    const int tile = (int)(blockIdx.x & 7) * ((tiles + 7) >> 3) + (int)(blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * BN;
     const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-    const int lr = tid >> 3, lk = (tid & 7) * 4;        // this thread's row (of every 32) and columns of a slice
-    float4 ra[LA], rw[LW];
-    auto fetch = [&](int k0) {
-        const int k = k0 + lk;
+    auto turn = [](int r) { return (r >> 1) & (CH - 1); };
+    // this lane's pieces of a slice: 8 rows a copy instruction
+    const float* src[LOADS];
+    int col[LOADS];
+    const float* zero_src = reinterpret_cast<const float*>(xr_zero_chunk);
 #pragma unroll
-        for (int e = 0; e < LA; ++e) {
-            const int m = m0 + lr + 32 * e;
-            ra[e] = m < M && k < K ? *reinterpret_cast<const float4*>(a + (size_t)m * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+    for (int i = 0; i < LOADS; ++i) {
+        const int r = (i * 4 + wave) * 8 + (lane >> 3);
+        col[i] = ((lane & (CH - 1)) ^ turn(r)) * 4;
+        const int m = m0 + r, n = n0 + r - BM;
+        src[i] = r < BM ? (m < M ? a + (size_t)m * lda + col[i] : nullptr) : (n < N ? w + (size_t)n * K + col[i] : nullptr);
+    }
+    const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * 64 * 16));
+    auto copy = [&](int slice) {                        // (pieces that do not exist are zeros)
+        const uint32_t dst = lds_wave + (uint32_t)(slice % STAGES * ROWS * CH * 16);
 #pragma unroll
-        for (int e = 0; e < LW; ++e) {
-            const int n = n0 + lr + 32 * e;
-            rw[e] = n < N && k < K ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
-    auto keep = [&](int buf) {
-#pragma unroll
-        for (int e = 0; e < LA; ++e) *reinterpret_cast<float4*>(&As[buf][(lr + 32 * e) * F_STRIDE + lk]) = ra[e];
-#pragma unroll
-        for (int e = 0; e < LW; ++e) *reinterpret_cast<float4*>(&Ws[buf][(lr + 32 * e) * F_STRIDE + lk]) = rw[e];
+        for (int i = 0; i < LOADS; ++i)
+            lds_dma16(src[i] && slice * FBK + col[i] < K ? src[i] + (size_t)slice * FBK : zero_src, dst + i * 256 * 16);
     };
     f32x16 acc[TM][TN], tot[TM][TN], lost[TM][TN];
 #pragma unroll
@@ -153,20 +159,23 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
                 }
     };
     const int row = lane & 31, half = (lane >> 5) * 4;
-    fetch(0);
-    keep(0);
-    __syncthreads();
-    int slice = 0;
-    for (int k0 = 0; k0 < K; k0 += FBK, ++slice) {
-        const int buf = slice & 1;
-        if (k0 + FBK < K) fetch(k0 + FBK);
+    const int n_slices = (K + FBK - 1) / FBK;
 #pragma unroll
-        for (int kk = 0; kk < FBK; kk += 8) {
+    for (int st = 0; st < STAGES - 1; ++st) copy(st);
+    for (int slice = 0; slice < n_slices; ++slice) {
+        wait_vmcnt<LOADS * (STAGES - 2)>();             // this wave's share of the slice has landed
+        __builtin_amdgcn_s_barrier();                   // every wave's has, and nobody reads the slice before any more
+        copy(slice + STAGES - 1);
+        const float4* As = lds + slice % STAGES * ROWS * CH;
+        const float4* Ws = As + BM * CH;
+#pragma unroll
+        for (int kk = 0; kk < CH; kk += 2) {
+            const int c = kk + (lane >> 5);
             float4 fa[TM], fw[TN];
 #pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const float4*>(&As[buf][(wm + 32 * i + row) * F_STRIDE + kk + half]);
+            for (int i = 0; i < TM; ++i) { const int r = wm + 32 * i + row; fa[i] = As[r * CH + (c ^ turn(r))]; }
 #pragma unroll
-            for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const float4*>(&Ws[buf][(wn + 32 * j + row) * F_STRIDE + kk + half]);
+            for (int j = 0; j < TN; ++j) { const int r = wn + 32 * j + row; fw[j] = Ws[r * CH + (c ^ turn(r))]; }
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -176,9 +185,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((&fa[i].x)[s], (&fw[j].x)[s], acc[i][j], 0, 0, 0);
         }
         if ((slice + 1) % (RBK * RB_FOLD / FBK) == 0) fold();
-        if (k0 + FBK < K) keep(buf ^ 1);
-        __syncthreads();
     }
+    wait_vmcnt<0>();                                    // the trailing copies of zeros
     fold();
     // a lane has column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a tile
 #pragma unroll
@@ -201,13 +209,25 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
     }
 }
 
-template <int BM, int BN>
-static void launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
-                            int out_dtype, int accumulate, hipStream_t stream) {
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    if (out_dtype == XR_BF16) k_gemm_f32<bf16_t, false, BM, BN><<<grid, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo);
-    else if (accumulate) k_gemm_f32<float, true, BM, BN><<<grid, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
-    else k_gemm_f32<float, false, BM, BN><<<grid, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+template <int BM, int BN, int STAGES>
+static int launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
+                           int out_dtype, int accumulate, hipStream_t stream) {
+    const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    XR_REQUIRE(tiles < (1ll << 28), "gemm: %lld tiles", tiles);
+    const unsigned blocks = 8 * (unsigned)((tiles + 7) / 8);
+    constexpr int smem = STAGES * (BM + BN) * FBK * 4;
+    auto run = [&](auto kernel, auto* to) {
+        if (smem > 65536) {
+            const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+            if (e != hipSuccess) (void)hipGetLastError();
+            XR_REQUIRE(e == hipSuccess, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+        }
+        kernel<<<blocks, 256, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
+        return XR_OK;
+    };
+    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, BM, BN, STAGES>, (bf16_t*)out);
+    if (accumulate) return run(k_gemm_f32<float, true, BM, BN, STAGES>, (float*)out);
+    return run(k_gemm_f32<float, false, BM, BN, STAGES>, (float*)out);
 }
 
 // Up to 16 rows of 32-bit operands (decoded tokens): the product is bound by how fast the weights
@@ -322,11 +342,12 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
         const float* af = (const float*)a;
         const float* wf = (const float*)w;
         if (M > 16) {
-            // 128 x 64 tiles read three quarters of what 64 x 64 ones read from L2, but two of their workgroups fill a compute
-            // unit: they are taken where there are at least that many (128 x 128 tiles with their three sums a value spill)
-            const long long tiles = (long long)((M + 127) / 128) * ((N + 63) / 64);
-            if (tiles >= 512) launch_gemm_f32<128, 64>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
-            else launch_gemm_f32<64, 64>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            // 64 x 128 tiles read three quarters of what 64 x 64 ones read from L2, but two of their workgroups fill a compute
+            // unit: they are taken where there are at least that many (larger tiles with their three sums a value spill)
+            const long long tiles = (long long)((M + 63) / 64) * ((N + 127) / 128);
+            const int rc = tiles >= 512 ? launch_gemm_f32<64, 128, 3>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                                        : launch_gemm_f32<64, 64, 4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            if (rc != XR_OK) return rc;
             XR_CHECK_LAUNCH("gemm_f32");
             return XR_OK;
         }
