@@ -1337,7 +1337,8 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
     // arrive, and two slices, one of them in use, left a compute unit 32 KB on its way: the down
     // product at 128 rows 46 -> 37 us, gate+up 72 -> 57, q/k/v at 512 rows 65 -> 45)
     // (the written order also where the weights' arrival bounds the kernel: little, 1-2%)
-    if ((variant == 17 && !g.rope.cs) || variant == 58) {
+    // (here also where the product rotates its result: 600 rows of a 4,096 to 6,144 product 42 us against 53)
+    if (variant == 17 || variant == 58) {
         const int rc = launch_tile_async<128, 128, 2, 2, 4, 2, 64>(g, stream);
         if (rc != XR_NOT_TAKEN) return rc;
     }
@@ -1570,7 +1571,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             const Cand plain[4] = {{14, 256, 256, 1.0, 5.8e-6, 0.0, 5.0e12}, {26, 256, 192, 0.95, 3.7e-6, 0.0, 5.0e12},
                                    {12, 256, 128, 0.95, 5.1e-6, 0.0, 4.1e12}, {17, 128, 128, 0.72, 3.9e-6, 0.0, 4.1e12}};
             const Cand turning[4] = {{14, 256, 256, 0.95, 0.0, 8e-6, 5.0e12}, {26, 256, 192, 0.81, 0.0, 9e-6, 5.0e12},
-                                     {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {58, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
+                                     {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {17, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
             const Cand* cands = rope_direct ? turning : plain;
             auto width = [&](const Cand& c) { return sw ? c.bn / 2 : c.bn; };
             auto usable = [&](const Cand& c) { return !(sw && c.variant == 26); };
