@@ -98,21 +98,22 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
 // half its number, so that the reads of 16 rows meet no bank twice.  Workgroup i runs on XCD i % 8, and an XCD takes an
 // eighth of the tiles, row tiles first: a weight tile comes from memory for one XCD (401 x 128256 x 2048, 1 GB of weights, read
 // them four times with the column tiles first).
-// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 at 112 TFLOP/s, 401 x 128256 x 2048 at 100 (84 before),
-// 401 x 2048 x 8192 at 69 (63; 224 tiles for 256 compute units, one wave a SIMD, which waits out its own reads); the FMA
-// kernel above reached 18 to 25.
+// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 at 112 to 119 TFLOP/s, 401 x 128256 x 2048 at 100 to 105
+// (84 before), 401 x 2048 x 8192 at 79 (63; 224 tiles for 256 compute units); the FMA kernel above reached 18 to 25.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define FBK 32
 
-template <typename TO, bool ACC, int BM, int BN, int STAGES>
-__global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+// KG 2 (few tiles): two sets of four waves make the same tile, each from every second slice, and add their sums up at the end:
+// two waves a SIMD, one of which works while the other waits for its reads.
+template <typename TO, bool ACC, int BM, int BN, int STAGES, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
                                                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
     constexpr int TM = BM / 64, TN = BN / 64;           // 32 x 32 tiles a wave
     constexpr int ROWS = BM + BN, CH = FBK / 4;         // rows of a slice (activations, then weights), pieces of a row
-    constexpr int LOADS = ROWS * CH / 256;              // copies a lane and slice
+    constexpr int LOADS = ROWS * CH / 256;              // copies a lane and stage (KG slices)
     static_assert(BM % 32 == 0 && LOADS * STAGES < 64, "whole copy instructions, and a count that fits the counter");
-    extern __shared__ __align__(16) float4 lds[];       // [STAGES][ROWS][CH]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    extern __shared__ __align__(16) float4 lds[];       // [STAGES][KG][ROWS][CH]
+    const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3, set = wave8 >> 2;
     const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN);
     const int tile = (int)(blockIdx.x & 7) * ((tiles + 7) >> 3) + (int)(blockIdx.x >> 3);
     if (tile >= tiles) return;
@@ -125,17 +126,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
     const float* zero_src = reinterpret_cast<const float*>(xr_zero_chunk);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-        const int r = (i * 4 + wave) * 8 + (lane >> 3);
-        col[i] = ((lane & (CH - 1)) ^ turn(r)) * 4;
+        const int all = (i * 4 * KG + wave8) * 8 + (lane >> 3), r = all % ROWS;
+        col[i] = ((lane & (CH - 1)) ^ turn(r)) * 4 + all / ROWS * FBK;
         const int m = m0 + r, n = n0 + r - BM;
         src[i] = r < BM ? (m < M ? a + (size_t)m * lda + col[i] : nullptr) : (n < N ? w + (size_t)n * K + col[i] : nullptr);
     }
-    const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * 64 * 16));
-    auto copy = [&](int slice) {                        // (pieces that do not exist are zeros)
-        const uint32_t dst = lds_wave + (uint32_t)(slice % STAGES * ROWS * CH * 16);
+    const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave8 * 64 * 16));
+    auto copy = [&](int stage) {                        // (pieces that do not exist are zeros)
+        const uint32_t dst = lds_wave + (uint32_t)(stage % STAGES * KG * ROWS * CH * 16);
 #pragma unroll
         for (int i = 0; i < LOADS; ++i)
-            lds_dma16(src[i] && slice * FBK + col[i] < K ? src[i] + (size_t)slice * FBK : zero_src, dst + i * 256 * 16);
+            lds_dma16(src[i] && stage * KG * FBK + col[i] < K ? src[i] + (size_t)stage * KG * FBK : zero_src, dst + i * KG * 256 * 16);
     };
     f32x16 acc[TM][TN], tot[TM][TN], lost[TM][TN];
 #pragma unroll
@@ -159,14 +160,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
                 }
     };
     const int row = lane & 31, half = (lane >> 5) * 4;
-    const int n_slices = (K + FBK - 1) / FBK;
+    const int n_stages = (K + KG * FBK - 1) / (KG * FBK);
 #pragma unroll
     for (int st = 0; st < STAGES - 1; ++st) copy(st);
-    for (int slice = 0; slice < n_slices; ++slice) {
-        wait_vmcnt<LOADS * (STAGES - 2)>();             // this wave's share of the slice has landed
-        __builtin_amdgcn_s_barrier();                   // every wave's has, and nobody reads the slice before any more
-        copy(slice + STAGES - 1);
-        const float4* As = lds + slice % STAGES * ROWS * CH;
+    for (int stage = 0; stage < n_stages; ++stage) {
+        wait_vmcnt<LOADS * (STAGES - 2)>();             // this wave's share of the stage has landed
+        __builtin_amdgcn_s_barrier();                   // every wave's has, and nobody reads the stage before any more
+        copy(stage + STAGES - 1);
+        const float4* As = lds + (stage % STAGES * KG + set) * ROWS * CH;
         const float4* Ws = As + BM * CH;
 #pragma unroll
         for (int kk = 0; kk < CH; kk += 2) {
@@ -184,10 +185,30 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
                     for (int j = 0; j < TN; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((&fa[i].x)[s], (&fw[j].x)[s], acc[i][j], 0, 0, 0);
         }
-        if ((slice + 1) % (RBK * RB_FOLD / FBK) == 0) fold();
+        if ((stage + 1) % (RBK * RB_FOLD / FBK) == 0) fold();
     }
     wait_vmcnt<0>();                                    // the trailing copies of zeros
     fold();
+    if constexpr (KG == 2) {                            // the second set's sums are one more run of the first's
+        __syncthreads();
+        float* other = reinterpret_cast<float*>(lds) + wave * TM * TN * 1024 + lane;
+        if (set == 1)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) other[((i * TN + j) * 16 + e) * 64] = tot[i][j][e] - lost[i][j][e];
+        __syncthreads();
+        if (set == 1) return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = other[((i * TN + j) * 16 + e) * 64];
+        fold();
+    }
     // a lane has column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a tile
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -209,25 +230,25 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(TO* __restrict__ out, const
     }
 }
 
-template <int BM, int BN, int STAGES>
+template <int BM, int BN, int STAGES, int KG>
 static int launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
                            int out_dtype, int accumulate, hipStream_t stream) {
     const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     XR_REQUIRE(tiles < (1ll << 28), "gemm: %lld tiles", tiles);
     const unsigned blocks = 8 * (unsigned)((tiles + 7) / 8);
-    constexpr int smem = STAGES * (BM + BN) * FBK * 4;
+    constexpr int smem = STAGES * KG * (BM + BN) * FBK * 4;
     auto run = [&](auto kernel, auto* to) {
         if (smem > 65536) {
             const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
             if (e != hipSuccess) (void)hipGetLastError();
             XR_REQUIRE(e == hipSuccess, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
         }
-        kernel<<<blocks, 256, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
+        kernel<<<blocks, 256 * KG, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
         return XR_OK;
     };
-    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, BM, BN, STAGES>, (bf16_t*)out);
-    if (accumulate) return run(k_gemm_f32<float, true, BM, BN, STAGES>, (float*)out);
-    return run(k_gemm_f32<float, false, BM, BN, STAGES>, (float*)out);
+    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, BM, BN, STAGES, KG>, (bf16_t*)out);
+    if (accumulate) return run(k_gemm_f32<float, true, BM, BN, STAGES, KG>, (float*)out);
+    return run(k_gemm_f32<float, false, BM, BN, STAGES, KG>, (float*)out);
 }
 
 // Up to 16 rows of 32-bit operands (decoded tokens): the product is bound by how fast the weights
@@ -345,8 +366,11 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
             // 64 x 128 tiles read three quarters of what 64 x 64 ones read from L2, but two of their workgroups fill a compute
             // unit: they are taken where there are at least that many (larger tiles with their three sums a value spill)
             const long long tiles = (long long)((M + 63) / 64) * ((N + 127) / 128);
-            const int rc = tiles >= 512 ? launch_gemm_f32<64, 128, 3>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                                        : launch_gemm_f32<64, 64, 4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            // (with no more 64 x 64 tiles than compute units, eight waves a tile: 401 x 2048 x 8192 195 us with four, 171 with eight)
+            const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
+            const int rc = tiles >= 512 ? launch_gemm_f32<64, 128, 3, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                         : small > 256  ? launch_gemm_f32<64, 64, 4, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                                        : launch_gemm_f32<64, 64, 3, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
             if (rc != XR_OK) return rc;
             XR_CHECK_LAUNCH("gemm_f32");
             return XR_OK;
