@@ -103,6 +103,7 @@ _PROTOS = {
     "xr_moe_experts": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _p, _i, _p, _p, _p, _i, _i, _p],
     "xr_delta_prepare": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f, _f, _p],
     "xr_linear_recurrence": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i, _f, _f, _p],
+    "xr_recurrence_chunks": [_p] * 11 + [C.c_longlong] + [_i] * 12 + [_f, _f, _p],
     "xr_qkv_store": [_p, _p, _p, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_pool_blocks": [_p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_attention_pool_partial": [_p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _p],
@@ -1514,6 +1515,22 @@ class Ops:
         elif decay is None or decay.dtype != torch.float32 or decay.numel() != H:
             raise KernelError(f"linear_recurrence: retention needs float32 decay [{H}]")
         out = torch.empty((T, H * Dv), dtype=torch.float32, device=q.device)
+        act = 1 if activation else 0
+        if (kind in ("retention", "delta") and ctx.max_q_len >= self.CHUNKS_FROM and 32 < D <= 128 and D % 16 == 0 and Dv % 16 == 0
+                and q.stride(0) % 4 == 0 and not (q.data_ptr() | k.data_ptr() | v.data_ptr() | state.data_ptr()) & 15):
+            # A long portion in chunks of 64 rows on the matrix cores.  From 96 rows on: 32 heads of 128 x 128 take the delta
+            # rule 23 us so and 22 token by token at 64 rows, 28 and 31 at 96, 239 and 590 at 2,048; retention (16 heads)
+            # 22 and 17, 20 and 24, 149 and 275.
+            delta = 1 if kind == "delta" else 0
+            floats = (T // 64 + ctx.B + 1) * H * ((1 + delta) * 64 * 64 + 3 * 64)       # (as the library counts them)
+            if floats <= self.CHUNKS_SCRATCH:
+                scratch = torch.empty((floats,), dtype=torch.float32, device=q.device)
+                self.lib.check(self.lib.xr_recurrence_chunks(
+                    out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(beta), _ptr(gate), _ptr(decay), state.data_ptr(),
+                    ctx.cu_q.data_ptr(), ctx.slots.data_ptr(), scratch.data_ptr(), floats, T, ctx.B, ctx.max_q_len, H, G, D, Dv,
+                    q.stride(0), gate.stride(0) if delta else 0, beta.stride(0) if delta else 0, delta, act, float(q_scale),
+                    float(k_scale), _stream()))
+                return out
         # Retention and wkv over long portions run in chunks side by side (the state before a chunk enters the
         # chunk's last state through the chunk's decays alone: one number a head, or their product channel by
         # channel; a chunk's sum from zero and that add up); the delta rule's chain cannot be cut.
@@ -1532,7 +1549,7 @@ class Ops:
                                                      ctx.slots.data_ptr(), ctx.B, H, G, D, Dv, q.stride(0),
                                                      gate.stride(0) if gate is not None else 0,
                                                      beta.stride(0) if beta is not None else 0, RECURRENCES[kind],
-                                                     chunk_len, n_chunks, _ptr(scratch), _ptr(prod), 1 if activation else 0,
+                                                     chunk_len, n_chunks, _ptr(scratch), _ptr(prod), act,
                                                      float(q_scale), float(k_scale), _stream()))
         return out
 
@@ -1589,6 +1606,8 @@ class Ops:
                 shared["ssd_plan"] = plan
         return plan[:3]
 
+    CHUNKS_FROM = 96                 # the longest portion of a step from which retention and the delta rule run in chunks on the matrix cores
+    CHUNKS_SCRATCH = 1 << 27         # floats that the chunks' matrices may take (steps of some 30,000 rows with 32 heads)
     RETENTION_CHUNK = 256            # rows a chunk; a multiple of the kernel's 16 staged tokens
     RETENTION_CHUNKED_FROM = 1024    # the longest portion of a step from which chunks pay
 
