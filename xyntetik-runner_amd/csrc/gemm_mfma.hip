@@ -1568,8 +1568,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // (Rotating products: the eight-wave kernels, but 128x128 tiles with four waves: 600 rows of a 4,096 to 6,144 product 42 us
             // against 53, 800 rows 72 against 98.)
             struct Cand { int variant, bm, bn; double rate, launch, round, bytes; };
-            const Cand plain[4] = {{14, 256, 256, 1.0, 5.8e-6, 0.0, 5.0e12}, {26, 256, 192, 0.95, 3.7e-6, 0.0, 5.0e12},
-                                   {12, 256, 128, 0.95, 5.1e-6, 0.0, 4.1e12}, {17, 128, 128, 0.72, 3.9e-6, 0.0, 4.1e12}};
+            const Cand plain[4] = {{14, 256, 256, 1.0, 5.8e-6, 0.0, 5.0e12}, {26, 256, 192, 0.86, 3.7e-6, 0.0, 5.0e12},
+                                   {12, 256, 128, 0.92, 5.1e-6, 0.0, 4.1e12}, {17, 128, 128, 0.71, 3.9e-6, 0.0, 4.1e12}};
             const Cand turning[4] = {{14, 256, 256, 0.95, 0.0, 8e-6, 5.0e12}, {26, 256, 192, 0.81, 0.0, 9e-6, 5.0e12},
                                      {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {17, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
             const Cand* cands = rope_direct ? turning : plain;
