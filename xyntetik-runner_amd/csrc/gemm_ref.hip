@@ -7,7 +7,8 @@
 // sum in two levels, with up to 16 the kernel further down
 // (k_gemv_ref) gives every lane every 64th group of four columns and adds the lanes' sums in a
 // tree.  A token's 32-bit result therefore differs in its last bits between a step of 16 rows and
-// one of 17 (both stay within 1e-6 of the exact product at K = 14,336).
+// one of 17 (both stay within 1e-6 of the exact product at K = 14,336), and between steps of so many rows that
+// k_gemm_f32 takes another number of waves for a tile (a run is then 128 columns of every second slice of 32).
 // The tile kernels' two levels: runs of RBK * RB_FOLD = 128 columns are summed one after another, and the runs'
 // sums are added up with a compensated (Kahan) sum.  One running 32-bit sum over the 14,336
 // columns of a wide feed-forward loses about 1e-5 of the result to rounding, which at such
