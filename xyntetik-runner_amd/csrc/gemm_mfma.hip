@@ -1560,16 +1560,16 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // weights from memory at `bytes` a second, whichever is longer; `launch` once and `round` for every round (a product that
             // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
             // at 2.2 TB/s and costs a launch, and writes the norm that follows, if one was asked for: without
-            // ranges its kernel takes 19 us with what lies around it.  Fitted to 3,800 timed launches (the 8B and the 1B class's four
-            // products and Suripel's two, 72 to 2,048 rows, four tiles, 1 to 16 ranges): the tile chosen is 1.2% slower
-            // than the best of them on average, 6.6% with the model before it (which knew no memory time and too high a
+            // ranges its kernel takes 12.5 us.  Fitted to 5,500 timed launches (the products of the 8B, the 7B and the 1B class's
+            // layers and Suripel's two, 66 to 2,048 rows, four tiles, 1 to 16 ranges): the tile and ranges chosen are 1.5% slower
+            // than the best of them on average (1.8% up to 300 rows), 6.6% with the model before it (which knew no memory time and too high a
             // price for 128x128 tiles: down at 137 rows in 256x256 tiles and 16 ranges 45-53 us, in 256x128 and 6 ranges 39-45;
             // a 4,096 to 6,144 product of 400 rows 47 us, in whole 128x128 tiles 32).
             // (Rotating products: the eight-wave kernels, but 128x128 tiles with four waves: 600 rows of a 4,096 to 6,144 product 42 us
             // against 53, 800 rows 72 against 98.)
             struct Cand { int variant, bm, bn; double rate, launch, round, bytes; };
-            const Cand plain[4] = {{14, 256, 256, 1.0, 5.8e-6, 0.0, 5.0e12}, {26, 256, 192, 0.86, 3.7e-6, 0.0, 5.0e12},
-                                   {12, 256, 128, 0.92, 5.1e-6, 0.0, 4.1e12}, {17, 128, 128, 0.71, 3.9e-6, 0.0, 4.1e12}};
+            const Cand plain[4] = {{14, 256, 256, 1.0, 4.3e-6, 0.0, 6.0e12}, {26, 256, 192, 0.85, 3.7e-6, 0.0, 3.9e12},
+                                   {12, 256, 128, 0.89, 3.7e-6, 0.0, 3.6e12}, {17, 128, 128, 0.71, 3.9e-6, 0.0, 5.6e12}};
             const Cand turning[4] = {{14, 256, 256, 0.95, 0.0, 8e-6, 5.0e12}, {26, 256, 192, 0.81, 0.0, 9e-6, 5.0e12},
                                      {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {17, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
             const Cand* cands = rope_direct ? turning : plain;
@@ -1583,10 +1583,20 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                 return rounds * ((products > weights ? products : weights) + c.round) + c.launch;
             };
             auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.2e12 + 4e-6; };
-            const double norm_alone = want_whole_norm ? 19e-6 : 0.0;
+            const double norm_alone = want_whole_norm ? 12.5e-6 : 0.0;
             int best = 0, best_splits = 1, second = -1, cols_first = N;
             double t_best = 1e30;
-            for (int i = 0; i < 4; ++i) {
+            // Up to 128 rows are one row of 128x128 tiles: K in as many ranges as make one round of workgroups, or whole from 160
+            // tiles on.  (Timed alone, five or six ranges of 32 tiles are 2-5% faster than eight; among a layer's other kernels the
+            // prompt of 70 to 128 tokens is 2-3% slower with them: 1,286 us against 1,267, 1,378 against 1,336, 1,441 against 1,407.)
+            const bool one_row = M <= 128 && !rope_direct && count(cands[3], N) <= 256;
+            if (one_row) {
+                const int c = count(cands[3], N);
+                best = 3;
+                best_splits = c < 160 ? pick_splits(c) : 1;
+                t_best = 0.0;
+            }
+            for (int i = 0; i < 4 && !one_row; ++i) {
                 if (!usable(cands[i])) continue;
                 const int c = count(cands[i], N);
                 for (int sp = 1; sp <= 16; ++sp) {
@@ -1595,7 +1605,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                     if (t < t_best) { best = i; best_splits = sp; t_best = t; }
                 }
             }
-            for (int i = 0; i < 3; ++i) {
+            for (int i = 0; i < 3 && !one_row; ++i) {
                 if (!usable(cands[i])) continue;
                 const int tm = (M + cands[i].bm - 1) / cands[i].bm, full = count(cands[i], N) / 256;
                 const int cols = full * 256 / tm * width(cands[i]);          // the columns of the full rounds
