@@ -623,6 +623,13 @@ def test_projection_with_rotation_and_cache_write_of_a_product_split_over_k(ops,
     check_projection_with_rotation_and_cache_write(ops, dt, 4, 2, 64, 64, False, 64, starts, q_lens, True, 1024)
 
 
+@pytest.mark.parametrize("H,Hk,E,rows", [(72, 64, 4096, 300), (96, 96, 1024, 511)])
+def test_projection_with_rotation_and_cache_write_of_a_wide_product(ops, H, Hk, E, rows):
+    """Up to 511 rows and so many columns that two launches would suit the tiles (a full round of workgroups and the rest): the
+    kernel that rotates and caches takes the sums of all columns, so there is one."""
+    check_projection_with_rotation_and_cache_write(ops, "bfloat16", H, Hk, 128, 128, False, 64, [0], [rows], False, E)
+
+
 @pytest.mark.parametrize("variant", [51, 55, 114, 112])
 @pytest.mark.parametrize("H,Hk,D,rot,inter", [(4, 2, 64, 64, False), (3, 1, 48, 32, False), (2, 1, 80, 80, True), (5, 1, 128, 128, False)])
 def test_projection_with_rotation_in_the_tile_kernels_by_name(ops, variant, H, Hk, D, rot, inter):

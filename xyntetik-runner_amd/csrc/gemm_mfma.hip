@@ -1559,7 +1559,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // tiles takes its products' time, bm bn K x 0.36e-12 / rate (97 us for 256x256 and K = 4,096 as measured), or that of its
             // weights from memory at `bytes` a second, whichever is longer; `launch` once and `round` for every round (a product that
             // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
-            // at 2.2 TB/s and costs a launch, and writes the norm that follows, if one was asked for: without
+            // at 2.2 TB/s and costs a launch (a rotating product of up to 511 rows pays for that kernel whole, too: counted as free, it
+            // sent 300 rows of a 3,072 to 5,120 product into one range, 35 us, where two take 29), and writes the norm that follows, if one was asked for: without
             // ranges its kernel takes 12.5 us.  Fitted to 5,500 timed launches (the products of the 8B, the 7B and the 1B class's
             // layers and Suripel's two, 66 to 2,048 rows, four tiles, 1 to 16 ranges): the tile and ranges chosen are 1.5% slower
             // than the best of them on average (1.8% up to 300 rows), 6.6% with the model before it (which knew no memory time and too high a
@@ -1601,11 +1602,12 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                 const int c = count(cands[i], N);
                 for (int sp = 1; sp <= 16; ++sp) {
                     if (sp > 1 && (rope_direct || !workspace || c * sp > 256 || K / sp < 256 || (size_t)sp * M * w_rows * 4 > workspace_bytes)) break;
-                    const double t = seconds(cands[i], N, sp) + (sp > 1 ? adding(sp) : norm_alone);
+                    const double t = seconds(cands[i], N, sp) + (sp > 1 || g.raw ? adding(sp) : norm_alone);
                     if (t < t_best) { best = i; best_splits = sp; t_best = t; }
                 }
             }
-            for (int i = 0; i < 3 && !one_row; ++i) {
+            // (one launch where the epilogue is a kernel of its own: that kernel takes the raw sums of all columns)
+            for (int i = 0; i < 3 && !one_row && !g.raw; ++i) {
                 if (!usable(cands[i])) continue;
                 const int tm = (M + cands[i].bm - 1) / cands[i].bm, full = count(cands[i], N) / 256;
                 const int cols = full * 256 / tm * width(cands[i]);          // the columns of the full rounds
