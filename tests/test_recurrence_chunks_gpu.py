@@ -45,8 +45,10 @@ PORTIONS = [[(0, 64), (64, 65), (129, 1), (130, 200)], [(0, 63), (63, 1), (64, 2
 
 
 def both(ops, monkeypatch, *args, **kw):
-    """(in chunks however short the portions are, token by token)"""
+    """(in chunks from portions of ``shortest`` rows on, token by token)"""
+    shortest = kw.pop("shortest", 1)
     monkeypatch.setattr(type(ops), "CHUNKS_FROM", 1)
+    monkeypatch.setattr(type(ops), "chunked_rows", lambda self, kind, q_lens, H, Dv: shortest if max(q_lens) >= shortest else None)
     chunks = run(ops, *args, **kw)
     monkeypatch.setattr(type(ops), "CHUNKS_FROM", 1 << 30)
     plain = run(ops, *args, **kw)
@@ -75,6 +77,29 @@ def test_delta_rule_in_chunks(monkeypatch, H, G, D, Dv):
     # a row is a sum of some D products with a state that up to 330 updates rounded, 2^-24 each: 5e-6 of the largest value
     assert error(chunks, want) < 5e-6, (error(chunks, want), error(plain, want))
     assert error(chunks, want) < 2 * error(plain, want) + 2e-7, (error(chunks, want), error(plain, want))
+
+
+@pytest.mark.parametrize("kind", ["delta", "retention"])
+@pytest.mark.parametrize("shortest", [2, 64, 65, 200])
+def test_long_portions_in_chunks_beside_short_ones_token_by_token(monkeypatch, kind, shortest):
+    """One step's requests go both ways, each once: the portions of ``shortest`` rows and more in chunks, the others token by token,
+    in whatever order they come."""
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    H, D, Dv = 4, 64, 32
+    rng = np.random.default_rng(shortest)
+    lens = [sum(n for _, n in p) for p in PORTIONS]
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    qs, ks = ([f32(S.unit(rng.normal(size=(n, H, D)))) for n in lens] for _ in range(2))
+    vs = [f32(rng.normal(size=(n, H, Dv))) for n in lens]
+    if kind == "delta":
+        extra = ([f32(S.sigmoid(rng.normal(size=(n, H)))) for n in lens], [f32(np.exp(-rng.exponential(0.1, size=(n, H)))) for n in lens])
+        want = [S.gated_delta_rule(q, k, v, b, g) for q, k, v, b, g in zip(qs, ks, vs, *extra)]
+    else:
+        extra = f32(np.array([0.97, 1.0, 0.5, 0.9]))
+        want = [S.retention(q, k, v, extra) for q, k, v in zip(qs, ks, vs)]
+    mixed, plain = both(ops, monkeypatch, kind, qs, ks, vs, extra, H, H, D, Dv, PORTIONS, [2, 0, 4, 1], 5, shortest=shortest)
+    assert error(mixed, want) < 5e-6, (error(mixed, want), error(plain, want))
 
 
 @pytest.mark.parametrize("H,D,Dv", [(2, 48, 16), (3, 64, 32), (1, 80, 48), (2, 128, 128)])

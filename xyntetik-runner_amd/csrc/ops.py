@@ -11,7 +11,7 @@ from __future__ import annotations
 import ctypes as C
 import threading
 from dataclasses import dataclass
-from typing import Dict, Optional
+from typing import Dict, Optional, Sequence
 
 import torch
 
@@ -102,8 +102,8 @@ _PROTOS = {
     "xr_heads_gemm_bf16": [_p, _p, _p, _i, _i, _i, _i, _i, C.c_longlong, _i, C.c_longlong, _i, _p],
     "xr_moe_experts": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _p, _i, _p, _p, _p, _i, _i, _p],
     "xr_delta_prepare": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f, _f, _p],
-    "xr_linear_recurrence": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i, _f, _f, _p],
-    "xr_recurrence_chunks": [_p] * 11 + [C.c_longlong] + [_i] * 12 + [_f, _f, _p],
+    "xr_linear_recurrence": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i, _f, _f, _p, _p],
+    "xr_recurrence_chunks": [_p] * 12 + [C.c_longlong] + [_i] * 12 + [_f, _f, _p],
     "xr_qkv_store": [_p, _p, _p, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_pool_blocks": [_p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_attention_pool_partial": [_p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _p],
@@ -1516,26 +1516,26 @@ class Ops:
             raise KernelError(f"linear_recurrence: retention needs float32 decay [{H}]")
         out = torch.empty((T, H * Dv), dtype=torch.float32, device=q.device)
         act = 1 if activation else 0
-        if (kind in ("retention", "delta") and ctx.max_q_len >= self.CHUNKS_FROM and 32 < D <= 128 and D % 16 == 0 and Dv % 16 == 0
-                and q.stride(0) % 4 == 0 and not (q.data_ptr() | k.data_ptr() | v.data_ptr() | state.data_ptr()) & 15):
-            # A long portion in chunks of 64 rows on the matrix cores.  From 96 rows on: 32 heads of 128 x 128 take the delta
-            # rule 23 us so and 22 token by token at 64 rows, 28 and 31 at 96, 239 and 590 at 2,048; retention (16 heads)
-            # 22 and 17, 20 and 24, 149 and 275.
+        rest = None
+        plan = self._chunk_plan(kind, ctx, H, D, Dv)
+        if (plan is not None and q.stride(0) % 4 == 0
+                and not (q.data_ptr() | k.data_ptr() | v.data_ptr() | state.data_ptr()) & 15):
+            # Long portions in chunks of 64 rows on the matrix cores, the step's other requests token by token.
+            portions, n_long, places, longest, rest = plan
             delta = 1 if kind == "delta" else 0
-            floats = (T // 64 + ctx.B + 1) * H * ((1 + delta) * 64 * 64 + 3 * 64)       # (as the library counts them)
-            if floats <= self.CHUNKS_SCRATCH:
-                scratch = torch.empty((floats,), dtype=torch.float32, device=q.device)
-                self.lib.check(self.lib.xr_recurrence_chunks(
-                    out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(beta), _ptr(gate), _ptr(decay), state.data_ptr(),
-                    ctx.cu_q.data_ptr(), ctx.slots.data_ptr(), scratch.data_ptr(), floats, T, ctx.B, ctx.max_q_len, H, G, D, Dv,
-                    q.stride(0), gate.stride(0) if delta else 0, beta.stride(0) if delta else 0, delta, act, float(q_scale),
-                    float(k_scale), _stream()))
+            scratch = torch.empty((places * self._chunk_floats(kind, H),), dtype=torch.float32, device=q.device)
+            self.lib.check(self.lib.xr_recurrence_chunks(
+                out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(beta), _ptr(gate), _ptr(decay), state.data_ptr(),
+                ctx.cu_q.data_ptr(), ctx.slots.data_ptr(), portions.data_ptr(), scratch.data_ptr(), scratch.numel(), places, n_long,
+                longest, H, G, D, Dv, q.stride(0), gate.stride(0) if delta else 0, beta.stride(0) if delta else 0, delta, act,
+                float(q_scale), float(k_scale), _stream()))
+            if rest.numel() == 0:
                 return out
         # Retention and wkv over long portions run in chunks side by side (the state before a chunk enters the
         # chunk's last state through the chunk's decays alone: one number a head, or their product channel by
         # channel; a chunk's sum from zero and that add up); the delta rule's chain cannot be cut.
         chunk_len, n_chunks, scratch, prod = 0, 0, None, None
-        if kind in ("retention", "wkv", "gla", "ssd") and ctx.max_q_len >= self.RETENTION_CHUNKED_FROM:
+        if rest is None and kind in ("retention", "wkv", "gla", "ssd") and ctx.max_q_len >= self.RETENTION_CHUNKED_FROM:
             n = -(-ctx.max_q_len // self.RETENTION_CHUNK)
             if ctx.B * n <= 4096:
                 chunk_len, n_chunks = self.RETENTION_CHUNK, n
@@ -1546,12 +1546,80 @@ class Ops:
                     prod = torch.empty((ctx.B * n, H), dtype=torch.float32, device=q.device)
         self.lib.check(self.lib.xr_linear_recurrence(out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(beta),
                                                      _ptr(gate), _ptr(decay), state.data_ptr(), ctx.cu_q.data_ptr(),
-                                                     ctx.slots.data_ptr(), ctx.B, H, G, D, Dv, q.stride(0),
+                                                     ctx.slots.data_ptr(), ctx.B if rest is None else rest.numel(), H, G, D, Dv, q.stride(0),
                                                      gate.stride(0) if gate is not None else 0,
                                                      beta.stride(0) if beta is not None else 0, RECURRENCES[kind],
                                                      chunk_len, n_chunks, _ptr(scratch), _ptr(prod), act,
-                                                     float(q_scale), float(k_scale), _stream()))
+                                                     float(q_scale), float(k_scale), _ptr(rest), _stream()))
         return out
+
+    # Retention and the delta rule in chunks on the matrix cores.  What a step takes either way, in microseconds, with w = H Dv / 4096
+    # (1 where the workgroups of one request, 16 columns each, are as many as compute units):
+    #   token by token: 4, and the longest chain, rows x `chain`, with 0.4 w a request beside it, or what fills the chip, w x (all
+    #   rows x `bulk` and 0.65 a request, whose state is read and written)
+    #   in chunks: 12, and `run` a chunk and 2.3 a request, the longest chain or all of them x w, and `mats` w a chunk
+    # Fitted to heads of 128 x 128, 16 and 32 of them, one portion of 96 to 2,048 rows alone and beside 1 to 63 decoded tokens, and 4
+    # to 20 portions of 95 to 512 rows.  With 32 heads the delta rule takes 28 us in chunks and 31 token by token for a portion of 96
+    # rows alone, 231 and 592 for 2,048; with 63 decoded tokens beside it 128 rows take 76 and 67 (and 667 where the decoded tokens
+    # were chunks, too), 400 rows 104 and 144, 2,048 rows 291 and 626; 20 portions of 100 rows 331 and 222.
+    CHUNK_COSTS = {"delta": (0.289, 0.115, 5.3, 1.85), "retention": (0.23, 0.09, 3.7, 0.97)}       # chain, bulk, run, mats
+    CHUNKS_FROM = 96                 # shorter portions never run in chunks
+    CHUNKS_SCRATCH = 1 << 27         # floats that the chunks' matrices may take (steps of some 30,000 rows with 32 heads)
+
+    @staticmethod
+    def _chunk_floats(kind: str, H: int) -> int:
+        """Scratch of a chunk, as the library counts it: one or two 64 x 64 matrices and three vectors a head."""
+        return H * ((2 if kind == "delta" else 1) * 64 * 64 + 3 * 64)
+
+    def chunked_rows(self, kind: str, q_lens: Sequence[int], H: int, Dv: int) -> Optional[int]:
+        """The shortest portion of a step that runs in chunks of 64 rows (None: none does): the division that takes the least time."""
+        chain, bulk, run, mats = self.CHUNK_COSTS[kind]
+        w = H * Dv / 4096
+        lens = sorted(q_lens, reverse=True)
+        rows, all_runs, places, longest = sum(lens), 0.0, 0, 0.0
+
+        def tokens(i: int, rows: int) -> float:            # the requests from the i-th longest on
+            requests = len(lens) - i
+            return 4.0 + max(chain * lens[i] + 0.4 * w * requests, w * (bulk * rows + 0.65 * requests)) if requests else 0.0
+
+        best, shortest = tokens(0, rows) if lens else 0.0, None
+        for i, n in enumerate(lens):
+            if n < self.CHUNKS_FROM:
+                break
+            chunks = -(-n // 64)
+            rows, places, all_runs, longest = rows - n, places + chunks, all_runs + run * chunks + 2.3, max(longest, run * chunks + 2.3)
+            if i + 1 < len(lens) and lens[i + 1] == n:
+                continue
+            t = 12.0 + max(longest, w * all_runs) + mats * w * places + tokens(i + 1, rows)
+            if t < best and places * self._chunk_floats(kind, H) <= self.CHUNKS_SCRATCH:
+                best, shortest = t, n
+        return shortest
+
+    def _chunk_plan(self, kind: str, ctx, H: int, D: int, Dv: int):
+        """(portions that run in chunks ``[n, 2]``: request, first chunk; n; chunks; longest portion; the other requests), or None:
+        none runs so.  Made once a step."""
+        if (kind not in self.CHUNK_COSTS or ctx.max_q_len < self.CHUNKS_FROM or not 32 < D <= 128 or D % 16 or Dv % 16):
+            return None
+        shared = getattr(ctx, "shared", None)
+        key = ("recurrence_chunks", kind, H, Dv)
+        if shared is not None and key in shared:
+            return shared[key][0]
+        plan, host = None, None
+        shortest = self.chunked_rows(kind, ctx.q_lens, H, Dv)
+        if shortest is not None:
+            portions, rest, places = [], [], 0
+            for b, n in enumerate(ctx.q_lens):
+                if n >= shortest:
+                    portions += [b, places]
+                    places += -(-n // 64)
+                else:
+                    rest.append(b)
+            host = torch.tensor(portions + rest, dtype=torch.int32).pin_memory()
+            dev = host.to(ctx.device, non_blocking=True)
+            plan = (dev[:len(portions)], len(portions) // 2, places, ctx.max_q_len, dev[len(portions):])
+        if shared is not None:
+            shared[key] = (plan, host)             # (the pinned copy lives as long as the plan)
+        return plan
 
     SSD_CHUNKED_FROM = 64            # the longest portion of a step from which a state space runs in chunks on the matrix cores
 
@@ -1606,8 +1674,6 @@ class Ops:
                 shared["ssd_plan"] = plan
         return plan[:3]
 
-    CHUNKS_FROM = 96                 # the longest portion of a step from which retention and the delta rule run in chunks on the matrix cores
-    CHUNKS_SCRATCH = 1 << 27         # floats that the chunks' matrices may take (steps of some 30,000 rows with 32 heads)
     RETENTION_CHUNK = 256            # rows a chunk; a multiple of the kernel's 16 staged tokens
     RETENTION_CHUNKED_FROM = 1024    # the longest portion of a step from which chunks pay
 

@@ -41,12 +41,10 @@ struct ChunkArgs {
     float* vecs;                // [places, H, RC_VEC]
     const int* cu_q;
     const int* slots;
+    const int* reqs;            // the portions that run so: (request, place of its first chunk) of each
     int H, G, Dv, ld, ld_g, ld_b, act;
     float q_scale, k_scale;
 };
-
-// The first place of request b's chunks: requests take at most ceil(n / 64) of the places from cu_q[b] / 64 + b on.
-__device__ inline int chunk_place(const int* cu_q, int b) { return cu_q[b] / RC_L + b; }
 
 __device__ inline float rc_act(float x, int act, float scale) { return (act ? x / (1.0f + expf(-x)) : x) * scale; }
 __device__ inline float4 rc_act4(float4 x, int act, float scale) {
@@ -85,11 +83,11 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
     __shared__ double L[RC_L];
     __shared__ float beta[RC_L];
     __shared__ __align__(16) float tmp[4][16 * 20];     // a wave's 16 x 16, by column
-    const int b = blockIdx.z, h = blockIdx.y, chunk = blockIdx.x;
+    const int b = a.reqs[2 * blockIdx.z], h = blockIdx.y, chunk = blockIdx.x;
     const int row_b = a.cu_q[b], n = a.cu_q[b + 1] - row_b;
     if (chunk * RC_L >= n) return;
     const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L < RC_L ? n - chunk * RC_L : RC_L;
-    const size_t place = (size_t)(chunk_place(a.cu_q, b) + chunk) * a.H + h;
+    const size_t place = (size_t)(a.reqs[2 * blockIdx.z + 1] + chunk) * a.H + h;
     float* mats = a.mats + place * (DELTA ? 2 : 1) * RC_L * RC_L;
     const int kvh = h / (a.H / a.G);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
@@ -200,14 +198,14 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
     __shared__ float vec[RC_VEC];
     // Workgroup i runs on XCD i % 8: the column workgroups of a head, which read the same rows and matrices, go to one XCD
     // (where the heads come in eights), so that its L2 serves all but the first of them.
-    const int shares = a.Dv / RC_C, id = blockIdx.x, b = blockIdx.y;
+    const int shares = a.Dv / RC_C, id = blockIdx.x, b = a.reqs[2 * blockIdx.y];
     const bool eights = a.H % 8 == 0;
     const int h = eights ? (id >> 3) / shares * 8 + (id & 7) : id / shares, c0 = (eights ? (id >> 3) % shares : id % shares) * RC_C;
     const int row_b = a.cu_q[b], n = a.cu_q[b + 1] - row_b;
     if (n <= 0) return;
     const int kvh = h / (a.H / a.G);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
-    const int place0 = chunk_place(a.cu_q, b);
+    const int place0 = a.reqs[2 * blockIdx.y + 1];
     float* st = a.state + (((size_t)a.slots[b] * a.H + h) * J * a.Dv + c0) * 16;
     for (int i = tid; i < J * RC_C * 4; i += 256) {
         const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
@@ -324,29 +322,27 @@ static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t strea
     return XR_OK;
 }
 
-// Floats of scratch for `T` rows of `B` requests.
-static long long chunks_scratch(int T, int B, int H, int delta) {
-    return (long long)(T / RC_L + B + 1) * H * ((delta ? 2 : 1) * RC_L * RC_L + RC_VEC);
-}
+// `n_reqs` portions of up to `max_q` rows: reqs [n_reqs][2] are the request and the place of its first chunk; they take `places` chunks
+// of 64 rows together, one after another.
 
 extern "C" int xr_recurrence_chunks(float* out, const float* q, const float* k, const float* v, const float* beta, const float* gate,
-                                    const float* decay, float* state, const int* cu_q, const int* slots, float* scratch, long long scratch_floats,
-                                    int T, int B, int max_q, int H, int G, int D, int Dv, int ld, int ld_g, int ld_b, int delta, int act,
+                                    const float* decay, float* state, const int* cu_q, const int* slots, const int* reqs, float* scratch,
+                                    long long scratch_floats, int places, int n_reqs, int max_q, int H, int G, int D, int Dv, int ld, int ld_g, int ld_b, int delta, int act,
                                     float q_scale, float k_scale, hipStream_t stream) {
-    XR_REQUIRE(T >= 0 && B >= 0 && max_q >= 0 && H > 0 && G > 0 && H % G == 0, "recurrence in chunks: %d heads over %d key heads", H, G);
+    XR_REQUIRE(places >= 0 && n_reqs >= 0 && max_q >= 0 && H > 0 && G > 0 && H % G == 0, "recurrence in chunks: %d heads over %d key heads", H, G);
     XR_REQUIRE(D % 16 == 0 && D > 32 && D <= 128 && Dv > 0 && Dv % RC_C == 0, "recurrence in chunks: key size %d (48 to 128), value size %d: in steps of 16", D, Dv);
-    XR_REQUIRE(out && q && k && v && state && cu_q && slots && scratch, "recurrence in chunks: a pointer is missing");
+    XR_REQUIRE(out && q && k && v && state && cu_q && slots && reqs && scratch, "recurrence in chunks: a pointer is missing");
     XR_REQUIRE(delta ? (beta && gate && ld_b >= H && ld_g >= H) : decay != nullptr, "recurrence in chunks: the gates are missing");
     XR_REQUIRE(ld % 4 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)state | (uintptr_t)scratch) & 15) == 0,
                "recurrence in chunks: rows that are not 16-byte aligned (%d apart)", ld);
     XR_REQUIRE(act == 0 || act == 1, "recurrence in chunks: activation %d of q, k and v (0: none, 1: SiLU)", act);
-    XR_REQUIRE(B <= 65535 && H <= 65535, "recurrence in chunks: %d requests, %d heads", B, H);
-    XR_REQUIRE(scratch_floats >= chunks_scratch(T, B, H, delta), "recurrence in chunks: a scratch of %lld floats", scratch_floats);
-    if (B == 0 || max_q == 0) return XR_OK;
-    const long long places = T / RC_L + B + 1;
-    ChunkArgs a{out, q, k, v, beta, gate, decay, state, scratch, scratch + places * H * (delta ? 2 : 1) * RC_L * RC_L, cu_q, slots,
+    XR_REQUIRE(n_reqs <= 65535 && H <= 65535, "recurrence in chunks: %d requests, %d heads", n_reqs, H);
+    const long long mats = (long long)places * H * (delta ? 2 : 1) * RC_L * RC_L;
+    XR_REQUIRE(scratch_floats >= mats + (long long)places * H * RC_VEC, "recurrence in chunks: a scratch of %lld floats for %d chunks", scratch_floats, places);
+    if (n_reqs == 0 || max_q == 0) return XR_OK;
+    ChunkArgs a{out, q, k, v, beta, gate, decay, state, scratch, scratch + mats, cu_q, slots, reqs,
                 H, G, Dv, ld, ld_g, ld_b, act, q_scale, k_scale};
-#define RC(DD) case DD: return delta ? launch_chunks<DD, true>(a, B, max_q, stream) : launch_chunks<DD, false>(a, B, max_q, stream)
+#define RC(DD) case DD: return delta ? launch_chunks<DD, true>(a, n_reqs, max_q, stream) : launch_chunks<DD, false>(a, n_reqs, max_q, stream)
     switch (D) { RC(48); RC(64); RC(80); RC(96); RC(112); RC(128); }
 #undef RC
     return XR_BAD_ARG;

@@ -68,6 +68,7 @@ struct RecArgs {
     // request, chunk and head, prod [request x chunk][head].)
     float* prod;
     float q_scale, k_scale;  // factors on the queries and on the keys as they are fetched (behind the activation, if there is one)
+    const int* reqs;         // the requests to run (one a place of the grid), or null: all of the step's.  Not with pass 1 and 2.
 };
 
 // the value of lane (l ^ 1), (l ^ 2) of a quad, or of the lane 4 / 8 further round a row of 16
@@ -101,6 +102,7 @@ __global__ __launch_bounds__(256) void k_recurrence(RecArgs a) {
     const int pass = !CHAIN ? a.pass : 0;
     int b = blockIdx.z, chunk = 0;
     if (pass) { chunk = b % a.n_chunks; b /= a.n_chunks; }
+    else if (a.reqs) b = a.reqs[b];
     int row0 = a.cu_q[b], n = a.cu_q[b + 1] - row0;
     if (pass) {
         if (chunk * a.chunk_len >= n || (pass == 2 && chunk == 0)) return;
@@ -426,7 +428,8 @@ extern "C" int xr_linear_recurrence(float* out, const float* q, const float* k, 
                                     const float* gate, const float* decay, float* state, const int* cu_q,
                                     const int* slots, int B, int H, int G, int D, int Dv, int ld, int ld_g, int ld_b, int mode,
                                     int chunk_len, int n_chunks, float* scratch, float* prod, int act, float q_scale, float k_scale,
-                                    hipStream_t stream) {
+                                    const int* reqs, hipStream_t stream) {
+    // (with `reqs`, B is their number)
     XR_REQUIRE(B >= 0 && H > 0 && G > 0 && H % G == 0, "recurrence: %d heads over %d key heads", H, G);
     XR_REQUIRE(D > 0 && D <= 256 && Dv > 0, "recurrence: key size %d (1 to 256), value size %d", D, Dv);
     XR_REQUIRE(mode >= XR_REC_RETENTION && mode <= XR_REC_SSD, "recurrence: mode %d", mode);
@@ -446,9 +449,10 @@ extern "C" int xr_linear_recurrence(float* out, const float* q, const float* k, 
     XR_REQUIRE(!chunks || (!chain && n_chunks > 1 && scratch && chunk_len % REC_TOKENS == 0),
                "recurrence: chunks are for retention and wkv, with room for their states");
     XR_REQUIRE(!chunks || mode == XR_REC_RETENTION || prod, "recurrence: channel decays in chunks need room for the chunks' decay products");
+    XR_REQUIRE(!chunks || !reqs, "recurrence: chunks are for all of a step's requests");
     XR_REQUIRE(!chunks || (long long)B * n_chunks <= 65535, "recurrence: %d requests of %d chunks", B, n_chunks);
     RecArgs a{out, q, k, v, beta, gate, decay, state, cu_q, slots, H, G, D, Dv, ld, ld_g, ld_b, chunks ? 1 : 0, chunk_len, n_chunks, scratch, act, prod,
-              q_scale, k_scale};
+              q_scale, k_scale, reqs};
     const int R = rec_lanes(D), cols = 256 / R, per = (D + R - 1) / R;
     dim3 grid((Dv + cols - 1) / cols, H, chunks ? B * n_chunks : B);
 #define REC(M)                                                                          \
