@@ -118,3 +118,12 @@ def test_retention_in_chunks(monkeypatch, H, D, Dv, activation):
     chunks, plain = both(ops, monkeypatch, "retention", qs, ks, vs, decay, H, H, D, Dv, PORTIONS, [2, 0, 4, 1], 5, activation=activation, k_scale=0.25)
     assert error(chunks, want) < 5e-6, (error(chunks, want), error(plain, want))
     assert error(chunks, want) < 2 * error(plain, want) + 2e-7, (error(chunks, want), error(plain, want))
+
+
+def test_which_steps_read_rows_again():
+    """Where retention applies its activation to the rows before the recurrence instead of in it."""
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    again = lambda kind, D, *q_lens: ops.recurrence_reads_rows_again(kind, step_ctx([0] * len(q_lens), list(q_lens), list(range(len(q_lens)))), 32, D, 128)
+    assert again("retention", 128, 1, 200, 1) and again("retention", 128, 1023) and again("retention", 256, 1024)
+    assert not again("retention", 128, 95) and not again("retention", 128, *[100] * 20) and not again("retention", 256, 1023)

@@ -1595,6 +1595,12 @@ class Ops:
                 best, shortest = t, n
         return shortest
 
+    def recurrence_reads_rows_again(self, kind: str, ctx, H: int, D: int, Dv: int) -> bool:
+        """Whether ``linear_recurrence`` fetches a row of this step more than once a head (a portion in chunks, of either kind): an
+        activation is then cheaper applied to the rows before."""
+        return ((kind in ("retention", "wkv", "gla", "ssd") and ctx.max_q_len >= self.RETENTION_CHUNKED_FROM)
+                or self._chunk_plan(kind, ctx, H, D, Dv) is not None)
+
     def _chunk_plan(self, kind: str, ctx, H: int, D: int, Dv: int):
         """(portions that run in chunks ``[n, 2]``: request, first chunk; n; chunks; longest portion; the other requests), or None:
         none runs so.  Made once a step."""
