@@ -104,7 +104,8 @@ __global__ __launch_bounds__(64) void k_attention_ref(
 // head and walks the keys they see in tiles of 64: keys and values through LDS, wave w the scores of keys 16 w .. 16 w + 15,
 // a softmax row a wave at a time, then wave w every fourth 16 channels of the output.  An MFMA step takes one
 // column from each quarter of the wave; a lane reads the four columns of its quarter at once and feeds four steps.
-// Keys that no row of the workgroup sees are never read (their pages may be gone) and count as zeros.
+// Keys that no row of the workgroup sees are never read (their pages may be gone) and count as zeros.  A tile whose values are not
+// all finite is added key by key, so that such a value shows in the rows that see it and in no other.
 // One wave a (token, head) walked the keys lane by lane, every lane a row of its own: 401 tokens, 32 heads of 64 took
 // 900 us and now 89, a decoded token of a tiny model 12 and now 7.
 #define AF_ROWS 32
@@ -137,6 +138,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
     extern __shared__ __align__(16) float lds[];
     __shared__ int row_pos[AF_ROWS], row_lo[AF_ROWS];
     __shared__ float row_corr[AF_ROWS], row_l[AF_ROWS], row_m[AF_ROWS];
+    __shared__ int odd_tile;                            // the last tile of keys with a value that is not finite
     const int b = blockIdx.z, kvh = blockIdx.y, G = a.H / a.Hk;
     const int t0 = a.cu_q[b], nq = a.cu_q[b + 1] - t0;
     const int r0 = blockIdx.x * AF_ROWS;                // of the request's nq * G rows
@@ -157,6 +159,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
         row_lo[tid] = a.chunk > 0 ? pos - pos % a.chunk : (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
         row_m[tid] = -INFINITY;
         row_l[tid] = 0.f;
+        if (tid == 0) odd_tile = -1;
     }
     for (int i = tid; i < AF_ROWS * D16 / 4; i += 256) {
         const int r = i / (D16 / 4), d = (i - r * (D16 / 4)) * 4;
@@ -197,6 +200,8 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
                     if (key + 1 < from || key + 1 >= to) v.y = 0.f;
                     if (key + 2 < from || key + 2 >= to) v.z = 0.f;
                     if (key + 3 >= to) v.w = 0.f;
+                    const float n = 0.f * v.x + 0.f * v.y + 0.f * v.z + 0.f * v.w;      // (0, or no number where one of them is not finite)
+                    if (n != n) odd_tile = 2 * k0 + seg;
                 }
                 *reinterpret_cast<float4*>(Vt + d * AF_LD_S + j) = v;
             }
@@ -262,6 +267,18 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[i][c][e] *= corr[i][e];
+                if (odd_tile == 2 * k0 + seg) {         // 0 times it is no 0: a row adds the keys that it sees, one by one
+                    for (int i = 0; i < tiles; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int r = 16 * i + 4 * quad + e, lo = row_lo[r], last = seg ? row_pos[r] : min(a.keep, lo) - 1;
+                            float sum = 0.f;
+                            for (int j = 0; j < AF_KEYS; ++j)
+                                if (k0 + j >= (seg ? lo : 0) && k0 + j <= last) sum = fmaf(S[r * AF_LD_S + j], Vt[(d0 + l16) * AF_LD_S + j], sum);
+                            if (i) acc[1][c][e] += sum; else acc[0][c][e] += sum;
+                        }
+                    continue;
+                }
                 const float* vp = Vt + (d0 + l16) * AF_LD_S + 4 * quad;
                 const float* pp = S + l16 * AF_LD_S + 4 * quad;
 #pragma unroll
