@@ -52,3 +52,41 @@ def test_attention_in_32_bits(H, Hk, D, Dv, mask):
             t += 1
     # 32-bit sums over up to 95 keys of weights that sum to one: a few 2^-24 times sqrt(95), scores within 1e-5 of theirs
     same(got.cpu().numpy().reshape(want.shape), want, 2e-5, str(mask))
+
+
+@pytest.mark.parametrize("kind,where", [(k, w) for k in ("delta", "retention") for w in ("q", "k", "v", "decay", "negative decay", "big")]
+                         + [("delta", "beta")])
+@pytest.mark.parametrize("D,Dv", [(48, 16), (128, 32)])
+def test_recurrences_in_chunks(monkeypatch, kind, where, D, Dv):
+    """Rows before one with an infinity or a NaN, in the middle of a chunk, are as they are without it; the rows behind it and the
+    state are what the recurrence makes of it token by token.  A negative decay is one like another."""
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    from test_recurrence_chunks_gpu import PORTIONS, both
+    ops = load_ops()
+    H = 2
+    rng = np.random.default_rng(D)
+    lens = [sum(n for _, n in p) for p in PORTIONS]
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    unit = lambda x: x / np.linalg.norm(x, axis=-1, keepdims=True)
+    qs, ks = ([f32(unit(rng.normal(size=(n, H, D)))) for n in lens] for _ in range(2))
+    vs = [f32(rng.normal(size=(n, H, Dv))) for n in lens]
+    beta, gate = ([f32(x + 0.5 * rng.uniform(size=(n, H))) for n in lens] for x in (0.25, 0.5))
+    decay = f32(np.array([0.97, 0.9]))
+    bad = {"q": qs, "k": ks, "v": vs, "beta": beta}.get(where)
+    if bad is not None:
+        bad[0][137].flat[1], bad[0][299].flat[0], bad[1][20].flat[-1] = np.inf, np.nan, -np.inf
+        bad[2][127].flat[0], bad[3][0].flat[0] = np.nan, np.inf
+    elif where == "decay":
+        gate[0][137, 1] = gate[2][128, 0] = decay[1] = np.nan
+    elif where == "negative decay":
+        gate[0][[137, 138, 190], 1], gate[1][64, 0], decay[1] = -0.5, -1.0, -0.9
+    else:                               # sums that pass the largest number on the way
+        vs[0][130:140, 1, 2], ks[0][130:140, 1] = 3e38, ks[0][130, 1]
+    extra = (beta, gate) if kind == "delta" else decay
+    chunks, plain = both(ops, monkeypatch, kind, qs, ks, vs, extra, H, H, D, Dv, PORTIONS, [2, 0, 4, 1], 5)
+    for b, (got, want) in enumerate(zip(chunks, plain)):
+        if where != "big":
+            same(got, want, 2e-5, f"request {b}")
+        else:                           # (where a sum overflows depends on its order: the rows before, and the other columns)
+            same(got[:130], want[:130], 2e-5, f"request {b}")
+            same(np.delete(got, 2, axis=2), np.delete(want, 2, axis=2), 2e-5, f"request {b}")

@@ -15,7 +15,8 @@
 // the delta rule the inverse T of the unit lower triangular I + beta_i exp(L_i - L_j) (k_i . k_j), so that
 // U = T (beta (V - exp(L) K S0)) is a product.  k_chunk_run then walks a request's chunks, a workgroup per head and 16
 // columns of the state (columns never meet), the state in LDS: three to five small products a chunk.  Rows past a portion's
-// end are zeros with beta 0 and no decay.  L is formed and subtracted in 64 bits; a decay of nothing counts as exp(-100).
+// end are zeros with beta 0 and no decay.  L is formed and subtracted in 64 bits; a decay of nothing counts as exp(-100).  A portion
+// that comes to something not finite, or has a negative decay, runs again token by token, a workgroup its 16 columns.
 // Bound by the chain of chunks, a chunk (5.7 us of the delta rule, 4.4 of retention) by five barriers, the trips to LDS between
 // them and, a third of it, its products.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 184 us and k_chunk_mats 59 for the
 // delta rule, 142 and 31 for retention; token by token (k_recurrence) 634, and retention in two passes over chunks of 256
@@ -108,8 +109,8 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
         float bt = 0.f;
         if (tid < rows) {
             const float g = DELTA ? a.gate[(size_t)(row0 + tid) * a.ld_g + h] : a.decay[h];
-            s = g > 0.f ? log((double)g) : -100.0;
-            s = s > -100.0 ? s : -100.0;
+            s = g == 0.f ? -100.0 : log((double)g);     // (no number for a negative decay: such a portion runs token by token)
+            s = s < -100.0 ? -100.0 : s;
             if (DELTA) bt = a.beta[(size_t)(row0 + tid) * a.ld_b + h];
         }
 #pragma unroll
@@ -196,6 +197,7 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
     __shared__ __align__(16) float U[RC_C][RC_LDM], W[RC_C][RC_LDM];     // by column: u_i; (delta) the right side; u_i exp(L_63 - L_i)
     __shared__ float V[RC_L][RC_C + 1];
     __shared__ float vec[RC_VEC];
+    __shared__ int odd;                                 // something came out that is not finite
     // Workgroup i runs on XCD i % 8: the column workgroups of a head, which read the same rows and matrices, go to one XCD
     // (where the heads come in eights), so that its L2 serves all but the first of them.
     const int shares = a.Dv / RC_C, id = blockIdx.x, b = a.reqs[2 * blockIdx.y];
@@ -236,10 +238,7 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
         if (r >= rows) rv = make_float4(0.f, 0.f, 0.f, 0.f);
         if (tid < RC_VEC) rvec = a.vecs[place * RC_VEC + tid];
     };
-    fetch(0);
-    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
-        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
-        __syncthreads();                                // the chunk before has been read, the state is written
+    auto stage = [&]() {                                // the fetched chunk to LDS
 #pragma unroll
         for (int e = 0; e < NQ; ++e) {
             const int i = tid + e * 256, r = i / (D / 4), c = i % (D / 4) * 4;
@@ -257,6 +256,14 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
             V[r][c] = x.x; V[r][c + 1] = x.y; V[r][c + 2] = x.z; V[r][c + 3] = x.w;
         }
         if (tid < RC_VEC) vec[tid] = rvec;
+    };
+    if (tid == 0) odd = 0;
+    float none = 0.f;                                   // 0, or no number once a read-out was not finite
+    fetch(0);
+    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
+        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
+        __syncthreads();                                // the chunk before has been read, the state is written
+        stage();
         __syncthreads();
         if ((chunk + 1) * RC_L < n) fetch(chunk + 1);
         const int i0 = 16 * wave + 4 * quad;            // this lane's rows of a product whose rows are the chunk's
@@ -285,6 +292,7 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (i0 + e < rows) a.out[((size_t)(row0 + i0 + e) * a.H + h) * a.Dv + c0 + l16] = o[e];
+        none += 0.f * o[0] + 0.f * o[1] + 0.f * o[2] + 0.f * o[3];
         const float all = vec[RC_L - 1];                // exp(L_63)
         for (int j = wave; j < J; j += 4) {             // 16 rows of the state: its own decayed, and K^T W
             float4 s0 = rc_ld4(&S[j][l16][4 * quad]);
@@ -299,9 +307,55 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
     }
     __syncthreads();
     for (int i = tid; i < J * RC_C * 4; i += 256) {
-        const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
-        rc_st4(st + ((size_t)j * a.Dv + c) * 16 + r, rc_ld4(&S[j][c][r]));
+        const float4 x = rc_ld4(&S[i / (RC_C * 4)][i / 4 % RC_C][i % 4 * 4]);
+        none += 0.f * x.x + 0.f * x.y + 0.f * x.z + 0.f * x.w;
     }
+    if (none != none) odd = 1;
+    __syncthreads();
+    if (!odd) {
+        for (int i = tid; i < J * RC_C * 4; i += 256) {
+            const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
+            rc_st4(st + ((size_t)j * a.Dv + c) * 16 + r, rc_ld4(&S[j][c][r]));
+        }
+        return;
+    }
+    // Not finite somewhere (a state that once is stays so): the portion again from its first state, token by token.  0 times an
+    // infinity or a NaN is no 0, so that above it shows in rows before its own, too; and a negative decay has no logarithm.
+    const int c = tid >> 4, r = tid & 15;               // 16 lanes a column, rows r, r + 16, ..
+    float s[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) s[j] = st[((size_t)j * a.Dv + c) * 16 + r];
+    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
+        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L < RC_L ? n - chunk * RC_L : RC_L;
+        fetch(chunk);
+        __syncthreads();
+        stage();
+        __syncthreads();
+        for (int i = 0; i < rows; ++i) {
+            const float g = DELTA ? a.gate[(size_t)(row0 + i) * a.ld_g + h] : a.decay[h];
+            const float* k = K + i * LD + r;
+            const float* q = Q + i * LD + r;
+            float u = V[i][c], o = 0.f;
+            if (DELTA) {
+                float d = 0.f;
+#pragma unroll
+                for (int j = 0; j < J; ++j) d = fmaf(s[j], k[16 * j], d);
+#pragma unroll
+                for (int m = 8; m > 0; m >>= 1) d += __shfl_xor(d, m, 64);
+                u = vec[2 * RC_L + i] * (u - g * d);
+            }
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                s[j] = fmaf(g, s[j], k[16 * j] * u);
+                o = fmaf(s[j], q[16 * j], o);
+            }
+#pragma unroll
+            for (int m = 8; m > 0; m >>= 1) o += __shfl_xor(o, m, 64);
+            if (r == 0) a.out[((size_t)(row0 + i) * a.H + h) * a.Dv + c0 + c] = o;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) st[((size_t)j * a.Dv + c) * 16 + r] = s[j];
 }
 
 template <int D, bool DELTA>
