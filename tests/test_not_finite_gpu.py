@@ -90,3 +90,30 @@ def test_recurrences_in_chunks(monkeypatch, kind, where, D, Dv):
         else:                           # (where a sum overflows depends on its order: the rows before, and the other columns)
             same(got[:130], want[:130], 2e-5, f"request {b}")
             same(np.delete(got, 2, axis=2), np.delete(want, 2, axis=2), 2e-5, f"request {b}")
+
+
+# rows for the few-row kernel, for tiles of two sets of waves, of one, and 64 x 128 of them; a row stride that is no multiple of four
+# (the kernel without matrix cores); one run of columns, several, and a rest
+@pytest.mark.parametrize("M,N,aligned", [(5, 96, True), (17, 100, True), (130, 16448, True), (260, 16448, True), (40, 100, False)])
+@pytest.mark.parametrize("K", [64, 128, 200, 384])
+def test_products_in_32_bits(M, N, aligned, K):
+    """A product or a sum past the largest number is infinite, whichever columns it comes from, a NaN stays one, and no other
+    row or column is touched."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    rng = np.random.default_rng(K + M)
+    a, w = (rng.normal(size=s).astype(np.float32) for s in ((M, K), (N, K)))
+    a[1, 3], w[:, 3] = 3e38, 2.0 + np.abs(w[:, 3])                       # a product, in the first run
+    a[2, K - 1], w[:, K - 1] = -3e38, 2.0 + np.abs(w[:, K - 1])          # and the last column, to the other side
+    a[3, [5, 40]], w[:, [5, 40]] = 2e38, 1.0                             # a sum of two, from the two sets' slices of 32
+    a[4, K // 2] = np.nan
+    w[7, K // 2 + 1] = np.inf
+    row = torch.zeros((M, K + (8 if aligned else 5)), device=DEV)
+    row[:, 4:4 + K] = torch.tensor(a)
+    got = ops.linear(row[:, 4:4 + K], torch.tensor(w, device=DEV)).cpu().numpy()
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = (a.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
+    same(np.delete(got, [1, 2, 3], axis=0), np.delete(want, [1, 2, 3], axis=0), 2e-5)
+    for r, sign in ((1, 1), (2, -1), (3, 1)):
+        assert (np.delete(got[r], 7) == sign * np.inf).all(), f"row {r}"

@@ -22,6 +22,16 @@
 #define RBK 16
 #define RB_FOLD 8
 
+// A run's sum into the sum of the runs, by Kahan's compensated addition.  What is lost is at most half a unit of the last place,
+// 1e31: the bounds only act where the sum is infinite, whose next compensation would make it NaN (2048 x 16384 x 2048 takes 1,161
+// us without them, 1,170 with).
+__device__ inline void fold_run(float& acc, float& tot, float& lost) {
+    const float y = acc - lost, t = tot + y;
+    lost = __builtin_amdgcn_fmed3f((t - tot) - y, -1e32f, 1e32f);
+    tot = t;
+    acc = 0.f;
+}
+
 template <typename TI, typename TO, bool ACC>
 __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI* __restrict__ a,
                                                    const TI* __restrict__ w, const float* __restrict__ bias,
@@ -35,15 +45,12 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = tot[i][j] = lost[i][j] = 0.f;
-#define FOLD_RUN()                                                   \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i)                    \
-        _Pragma("unroll") for (int j = 0; j < 4; ++j) {              \
-            const float y = acc[i][j] - lost[i][j];                  \
-            const float t = tot[i][j] + y;                           \
-            lost[i][j] = (t - tot[i][j]) - y;                        \
-            tot[i][j] = t;                                           \
-            acc[i][j] = 0.f;                                         \
-        }
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fold_run(acc[i][j], tot[i][j], lost[i][j]);
+    };
 
     int slice = 0;
     for (int k0 = 0; k0 < K; k0 += RBK, ++slice) {
@@ -69,10 +76,9 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
                 for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
         }
         __syncthreads();
-        if (slice % RB_FOLD == RB_FOLD - 1) { FOLD_RUN() }
+        if (slice % RB_FOLD == RB_FOLD - 1) fold();
     }
-    FOLD_RUN()
-#undef FOLD_RUN
+    fold();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         int gm = m0 + ty * 4 + i;
@@ -153,11 +159,9 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, 
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const float y = acc[i][j][e] - lost[i][j][e];
-                    const float t = tot[i][j][e] + y;
-                    lost[i][j][e] = (t - tot[i][j][e]) - y;
-                    tot[i][j][e] = t;
-                    acc[i][j][e] = 0.f;
+                    float x = acc[i][j][e], t = tot[i][j][e], l = lost[i][j][e];
+                    fold_run(x, t, l);
+                    acc[i][j][e] = x; tot[i][j][e] = t; lost[i][j][e] = l;
                 }
     };
     const int row = lane & 31, half = (lane >> 5) * 4;
