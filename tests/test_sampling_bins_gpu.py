@@ -75,6 +75,42 @@ def test_pick_by_bins(V):
     assert plain == [pick(r, o[0], o[1], 0, 1.0, 0.0) for r, o in zip(rows, opts)]
 
 
+@pytest.mark.parametrize("V", [8195, 128256])
+def test_pick_where_candidates_are_ruled_out_or_have_no_mass(V):
+    """Rows whose allowed candidates are flat, few or one beside -inf, and rows so steep that a top-k cut falls among candidates whose
+    mass is nothing."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    rng = np.random.default_rng(V + 1)
+    rows, opts = [], []
+    for kind in ("flat", "few", "one", "two", "steep", "steeper"):
+        for top_k, top_p, min_p in ((0, 1.0, 0.0), (1, 1.0, 0.0), (3, 1.0, 0.0), (40, 1.0, 0.0), (40, 0.95, 0.05), (200, 0.9, 0.0),
+                                    (3000, 1.0, 0.0), (0, 0.95, 0.0), (0, 1.0, 0.05), (0, 1.0, 1.0)):
+            row = np.full(V, -np.inf, dtype=np.float32)
+            if kind == "flat":
+                allowed = rng.random(V) < 0.67
+                row[allowed] = rng.standard_normal(int(allowed.sum())).astype(np.float32) * 0.05
+            elif kind.startswith("steep"):      # the second best 8 and 30 below the best; everything but some forty past the span
+                row[:] = rng.standard_normal(V) * 0.5 - 40.0
+                row[rng.choice(V, 40, replace=False)] = rng.standard_normal(40) if kind == "steep" else -22.0
+                row[V // 2] = 8.0
+            else:
+                n = {"few": 20, "one": 1, "two": 2}[kind]
+                row[rng.choice(V, n, replace=False)] = rng.standard_normal(n)
+            rows.append(row)
+            draw = float(rng.integers(0, 1 << 24)) / (1 << 24)
+            opts.append((float(rng.choice([0.3, 0.8, 1.3])), draw, top_k, float(np.float32(top_p)), float(np.float32(min_p))))
+    f = lambda i: torch.tensor([o[i] for o in opts], dtype=torch.float32, device=dev)
+    top_k = torch.tensor([o[2] for o in opts], dtype=torch.int32, device=dev)
+    logits = torch.tensor(np.stack(rows), device=dev)
+    want = [pick(r, *o) for r, o in zip(rows, opts)]
+    got = ops.sample(logits, f(0), f(1), top_k=top_k, top_p=f(3), min_p=f(4)).cpu().tolist()
+    assert [(i, g) for i, g in enumerate(got) if g != want[i]] == [(i, w) for i, w in enumerate(want) if w != got[i]], opts
+    plain = ops.sample(logits, f(0), f(1)).cpu().tolist()
+    assert plain == [pick(r, o[0], o[1], 0, 1.0, 0.0) for r, o in zip(rows, opts)]
+
+
 def test_penalty_of_a_window_with_repeats():
     """Each occurrence of a token counts, whichever workgroup holds the token; exempt ones are left alone."""
     import torch
