@@ -6,9 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 # rows: one, the ends of the few-row kernel's groups, either side of its limit, of a tile's 32, 64 and 128; columns: less than a
-# slice of 32, no multiple of it, either side of a run of 128; weight rows: few, no multiple of a tile, enough for the large tile
-@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 33, 64, 65, 130])
-@pytest.mark.parametrize("N,K", [(7, 4), (96, 64), (100, 124), (65, 132), (200, 260), (16448, 68)])
+# slice of 32, no multiple of it, either side of a run of 128; weight rows: few, no multiple of a tile, and so many that 200 rows make
+# 516 tiles of 64 x 128 (512 are taken in such tiles, fewer in 64 x 64)
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 33, 64, 65, 130, 200])
+@pytest.mark.parametrize("N,K", [(7, 4), (96, 64), (100, 124), (65, 132), (200, 260), (16448, 68), (16450, 132)])
 def test_product(M, N, K):
     import torch
     from xyntetik_runner_amd.csrc.ops import load_ops

@@ -4,6 +4,8 @@
 //   retention:   S <- g S + k v^T;                                  o = S^T q
 //   delta rule:  S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
 //
+// (The chunked form of the delta rule, with its triangular inverse: S. Yang, B. Wang, Y. Zhang, Y. Shen, Y. Kim, "Parallelizing Linear
+// Transformers with the Delta Rule over Sequence Length", 2024; with decays: S. Yang, J. Kautz, A. Hatamizadeh, "Gated Delta Networks", 2024.)
 // A chunk begins with the state S0.  With L_i the sum of log g up to row i of the chunk (inclusive):
 //
 //   u_i = v_i                                                                            (retention)
@@ -83,7 +85,6 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
     float* T = A + RC_L * RC_LDM;                       // (delta) its inverse
     __shared__ double L[RC_L];
     __shared__ float beta[RC_L];
-    __shared__ __align__(16) float tmp[4][16 * 20];     // a wave's 16 x 16, by column
     const int b = a.reqs[2 * blockIdx.z], h = blockIdx.y, chunk = blockIdx.x;
     const int row_b = a.cu_q[b], n = a.cu_q[b + 1] - row_b;
     if (chunk * RC_L >= n) return;
@@ -169,10 +170,9 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
                 s = rc_mfma4(rc_ld4(A + (16 * i + l16) * RC_LDM + 16 * m + 4 * quad),
                              make_float4(tp[0], tp[RC_LDM], tp[2 * RC_LDM], tp[3 * RC_LDM]), s);
             }
-            rc_st4(&tmp[wave][l16 * 20 + 4 * quad], make_float4(s[0], s[1], s[2], s[3]));
-            __builtin_amdgcn_wave_barrier();            // (one wave's own area, served in order)
+            // (a result's layout, a lane four rows of a column, is an operand's)
             rc_f32x4 t = {0.f, 0.f, 0.f, 0.f};
-            t = rc_mfma4(rc_ld4(T + (16 * i + l16) * RC_LDM + 16 * i + 4 * quad), rc_ld4(&tmp[wave][l16 * 20 + 4 * quad]), t);
+            t = rc_mfma4(rc_ld4(T + (16 * i + l16) * RC_LDM + 16 * i + 4 * quad), make_float4(s[0], s[1], s[2], s[3]), t);
 #pragma unroll
             for (int e = 0; e < 4; ++e) T[(16 * i + 4 * quad + e) * RC_LDM + 16 * j + l16] = -t[e];
         }

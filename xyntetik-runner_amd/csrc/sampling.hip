@@ -367,7 +367,7 @@ struct List {
 };
 
 // Gather and sort the bins [lo, hi]; false: more candidates than the list holds.
-__device__ __forceinline__ bool gather(const float* row, int V, float temp, const Bins& bins, int lo, int hi, List& list, u64* sh) {
+__device__ __forceinline__ bool gather(const float* row, int V, float temp, const Bins& bins, int lo, int hi, List& list) {
     __syncthreads();
     if (threadIdx.x == 0) { list.n = 0; list.lo = lo; list.hi = hi; }
     __syncthreads();
@@ -460,7 +460,7 @@ __device__ __forceinline__ int sample_by_bins(const SampleArgs& a, int r, const 
     bool have = false;          // (the same in all threads, as is every cut below)
     auto need = [&](int lo, int hi) {
         if (have && list.lo <= lo && hi <= list.hi) return true;
-        have = gather(row, a.V, temp, bins, lo, hi, list, sh);
+        have = gather(row, a.V, temp, bins, lo, hi, list);
         if (have) sum_list(list, bins.zmax, 0.f, ~0ull, sh);
         return have;
     };
@@ -500,7 +500,7 @@ __device__ __forceinline__ int sample_by_bins(const SampleArgs& a, int r, const 
             edge = SM_BINS;
         } else {
             const int to = last < past ? last : past;
-            have = gather(row, a.V, temp, bins, edge, to, list, sh);
+            have = gather(row, a.V, temp, bins, edge, to, list);
             if (!have) return -1;
             sum_list(list, bins.zmax, min_e, limit, sh);
             kept = before() + (list.n > 0 ? list.sum[list.n - 1] : 0ull);
