@@ -34,3 +34,21 @@ def test_product(M, N, K):
     if (M <= 16) == (few.shape[0] <= 16):
         assert torch.equal(few, got[: few.shape[0]])
     assert torch.equal(ops.linear(at, t(w), out_dtype=torch.bfloat16), got.bfloat16())
+
+
+# the rows at which a few-row kernel ends, and weight rows and columns on either side of the lines between 2, 4 and 8 weight rows a wave
+@pytest.mark.parametrize("M", [1, 3, 8, 16])
+@pytest.mark.parametrize("N,K", [(4095, 256), (4097, 256), (6145, 260), (8191, 4096), (8193, 4096), (16383, 512), (16385, 512), (16385, 4096)])
+def test_weight_rows_a_wave(M, N, K):
+    """How many weight rows a wave takes changes no bit: the sums are those of narrow products, two weight rows a wave."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w = (torch.randn(s, generator=g, device=dev) for s in ((M, K), (N, K)))
+    narrow = torch.cat([ops.linear(a, w[i:i + 2048]) for i in range(0, N, 2048)], dim=1)
+    assert torch.equal(ops.linear(a, w), narrow)
+    # and the sums themselves: K products and additions of 2^-24 each
+    want, size = (a.double() @ w.double().T), (a.double().abs() @ w.double().abs().T)
+    assert ((narrow.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size).all()

@@ -264,8 +264,8 @@ static int launch_gemm_f32(void* out, const float* a, const float* w, const floa
 // on the rows beside it; it differs from the tile kernel's by the order of the sum only.
 // All sums go through the tree at once: at the first step a lane hands half of its sums to the lane 32 further and
 // takes over the other half, and so on, until a lane holds the whole sum of one (row, weight row) or what is left of few sums
-// goes on as a plain tree.  The additions are those of a tree a sum, in the same order.  (Three rows through 64 x 64 weights:
-// 3.4 us with 2 weight rows a wave and one tree, 9.5 us with 8 weight rows and a tree of six steps for each of 32 sums.)
+// goes on as a plain tree.  The additions are those of a tree a sum, in the same order.  (2048 x 2048, 16 rows: 13 us with 2 weight
+// rows a wave and one tree, 46 us with 8 weight rows and a tree of six steps for each of 128 sums.)
 template <int N>
 __device__ inline void tree_sums(float (&v)[N], int lane, int& mine) {
     mine = 0;
@@ -277,8 +277,10 @@ __device__ inline void tree_sums(float (&v)[N], int lane, int& mine) {
             mine = 2 * mine + (up ? 1 : 0);
 #pragma unroll
             for (int i = 0; i < n / 2; ++i) {
-                const float keep = up ? v[n / 2 + i] : v[i], give = up ? v[i] : v[n / 2 + i];
-                v[i] = keep + __shfl_xor(give, o, 64);
+                // (both values first: a choice between two elements in place is an index that is not known, which
+                // costs a choice among all elements: 32 sums took 2,000 selects and 4 us)
+                const float low = v[i], high = v[n / 2 + i];
+                v[i] = (up ? high : low) + __shfl_xor(up ? low : high, o, 64);
             }
             o >>= 1;
         }
@@ -347,12 +349,22 @@ static void launch_gemv_cols(void* out, const float* a, const float* w, const fl
     else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
 }
 
-// Weight rows a wave: 8 share the reads of `a`, but only where that still gives every compute unit two workgroups;
-// below that a wave takes 2 (a product of 2,048 weight rows: 256 workgroups instead of 64).
+// Weight rows a wave: more share the reads of `a` and cost fewer sums, fewer spread over more compute units.  One row: 2.  More
+// rows: 2 for as long as weight rows are few, then 4, and 8 where K is long enough to keep them busy (or rows are 16).  Times in us
+// with 2, 4 and 8, weights from memory: 4096 x 4096, 8 rows 19, 22, 29; 8192 x 2048, 16 rows 32, 22, 28; 14336 x 4096, 16 rows 105, 76, 61;
+// 16384 x 2048, 3 rows 27, 27, 35; 28672 x 4096, 8 rows 132, 102, 101.
+template <int MT>
+static int gemv_cols(int N, int K) {
+    if (MT == 1 || N < (MT == 4 ? 16384 : MT == 8 ? 6144 : 4096)) return 2;
+    return (K >= 4096 && N >= 8192) || (MT == 16 && N >= 16384) ? 8 : 4;
+}
+
 template <int MT>
 static void launch_gemv_ref(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
                             int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
-    if (N >= 2 * 256 * 32) launch_gemv_cols<MT, 8>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+    const int cols = gemv_cols<MT>(N, K);
+    if (cols == 8) launch_gemv_cols<MT, 8>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+    else if (cols == 4) launch_gemv_cols<MT, 4>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
     else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
 }
 
