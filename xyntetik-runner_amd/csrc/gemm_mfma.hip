@@ -70,7 +70,8 @@ struct GemmArgs {
     int epi;
     int act;           // the gate's activation (XR_ACT_*), with EPI_GATED; with EPI_STORE what the results pass (XR_POST_*)
     float act_param;   // and its number, for a gate that takes one
-    int m_fast;        // tile order of the asynchronous kernel: 1 = consecutive workgroups share a weight tile, 2 = by XCD
+    int m_fast;        // tile order of the asynchronous kernel: 1 = consecutive workgroups share a weight tile, 2 = whole columns by XCD,
+                       // 3 = an eighth of the tiles (and K ranges) an XCD
     int splits;        // > 1: K is cut into this many ranges, each workgroup writes raw sums to `partial`
     int k_per_split;   // columns per range (a multiple of 64)
     float* partial;    // [splits][M][rows of w]
@@ -483,9 +484,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
     constexpr int BN_OUT_S = BN / 2;
     const int bn_out = g.epi == EPI_GATED ? BN_OUT_S : BN;
     const int tiles_n = (g.col1 - g.col0 + bn_out - 1) / bn_out;
-    const int tile_ = __builtin_amdgcn_readfirstlane(item / g.splits), split_ = __builtin_amdgcn_readfirstlane(item % g.splits);
     // (the divisions are done in vector registers; their results go back to scalar ones)
-    // m_fast 2 (at most 8 row tiles): workgroup i runs on XCD i % 8, and each XCD takes every 8th
+    // m_fast 2 (at most 8 row tiles, K whole): workgroup i runs on XCD i % 8, and each XCD takes every 8th
     // column tile with all its row tiles, row tiles first, so a weight tile is fetched from memory by
     // one XCD alone, and the XCD's 32 workgroups of a moment share 4 weight tiles and the activation
     // tiles in its L2.  (Where the column tiles are no multiple of 8 the launch has workgroups for 8
@@ -494,22 +494,31 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
     // tiles an XCD, it lost: 8192 x 28672 x 4096 in 1,776 us against 1,456.)
     // m_fast 3: the same with an eighth of the tiles an XCD, whole columns or not, where whole columns would give
     // some XCDs a round of 32 workgroups more (252 tiles of 6 rows x 42 columns: 36 on two XCDs, 30 on the others;
-    // 1536 x 12288 x 4096 took 233 us and now 152).  Shares that begin within a column cost 1% elsewhere.
-    int bm_v, bn_v;
-    if (g.m_fast == 2) {
-        const int l = tile_ >> 3;
+    // 1536 x 12288 x 4096 took 233 us and now 152; shares that begin within a column cost 1% elsewhere), where row tiles are
+    // 9 to 16 (1100 x 3584 x 18944 in 128 x 128 tiles 218 us with m_fast 1 and 160; all such launches measured: 9% less in the middle),
+    // and where K is split and row tiles are 2 to 16: an XCD has an eighth of all ranges' tiles, one range after another, so that its workgroups
+    // read few ranges.  (With the ranges of a tile side by side instead, three of them put all three on every XCD: 1000 x 3584 x 18944 in
+    // 256 x 192 tiles 255 us, now 155; 500 x 2560 x 9728 in 128 x 128 tiles 58 and 46; two or four ranges are as before.
+    // One row of tiles reads its weights once in any order.)
+    int bm_v, bn_v, split_v = 0;
+    if (g.m_fast == 3) {
+        const int tiles = tiles_m * tiles_n, share = (tiles * g.splits + 7) >> 3, p = (item & 7) * share + (item >> 3);
+        if (p >= tiles * g.splits) return;
+        split_v = p / tiles;
+        bm_v = (p - split_v * tiles) % tiles_m;
+        bn_v = (p - split_v * tiles) / tiles_m;
+    } else if (g.m_fast == 2) {
+        const int l = item >> 3;
         bm_v = l % tiles_m;
-        bn_v = (l / tiles_m) * 8 + (tile_ & 7);
+        bn_v = (l / tiles_m) * 8 + (item & 7);
         if (bn_v >= tiles_n) return;
-    } else if (g.m_fast == 3) {
-        const int share = (tiles_m * tiles_n + 7) >> 3, t = (tile_ & 7) * share + (tile_ >> 3);
-        if (t >= tiles_m * tiles_n) return;
-        bm_v = t % tiles_m;
-        bn_v = t / tiles_m;
     } else {
-        bm_v = g.m_fast ? tile_ % tiles_m : tile_ / tiles_n;
-        bn_v = g.m_fast ? tile_ / tiles_m : tile_ % tiles_n;
+        const int tile = item / g.splits;
+        split_v = item - tile * g.splits;
+        bm_v = g.m_fast ? tile % tiles_m : tile / tiles_n;
+        bn_v = g.m_fast ? tile / tiles_m : tile % tiles_n;
     }
+    const int split_ = __builtin_amdgcn_readfirstlane(split_v);
     const int bm_ = __builtin_amdgcn_readfirstlane(bm_v);
     const int bx = __builtin_amdgcn_readfirstlane(g.col0 / bn_out + bn_v);
     const int k_begin = split_ * g.k_per_split;
@@ -1076,12 +1085,6 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     }
     unsigned tiles_n = (unsigned)((g.col1 - g.col0 + n_out_tile - 1) / n_out_tile), tiles_m = (unsigned)((g.M + BM - 1) / BM);
     unsigned tiles = tiles_n * tiles_m;
-    if (g.m_fast == 2 && (tiles_m > 8 || tiles_n < 8)) g.m_fast = 1;
-    if (g.m_fast == 2) {
-        const unsigned columns = tiles_m * ((tiles_n + 7) / 8), even = (tiles + 7) / 8;       // tiles of the XCD that has most
-        if ((columns + 31) / 32 > (even + 31) / 32) g.m_fast = 3;
-        tiles = 8 * (g.m_fast == 3 ? even : columns);
-    }
     if (g.splits < 1 || !g.partial || g.col0 > 0 || g.col1 < g.N) g.splits = 1;
     if (g.splits > 1) {
         int slices = (g.K + 63) / 64;
@@ -1090,6 +1093,18 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
         g.splits = (slices + per - 1) / per;            // no empty range
     }
     if (g.splits == 1) g.k_per_split = ((g.K + 63) / 64) * 64;
+    unsigned groups = tiles * g.splits;
+    if (g.m_fast == 2) {
+        const unsigned columns = tiles_m * ((tiles_n + 7) / 8), even = (groups + 7) / 8;      // workgroups of the XCD that has most
+        if (g.splits > 1 ? tiles_m > 1 && tiles_m <= 16 : tiles_n >= 8 && tiles_m <= 16 && (tiles_m > 8 || (columns + 31) / 32 > (even + 31) / 32)) {
+            g.m_fast = 3;
+            groups = 8 * even;
+        } else if (g.splits > 1 || tiles_m > 8 || tiles_n < 8) {
+            g.m_fast = 1;
+        } else {
+            groups = 8 * columns;
+        }
+    }
     if (PIPE == 2) {
         // the loop with its instructions in a written order: whole slices only, at least ST of them
         // in every K range, and every lane's piece within 4 GB of the tile's first
@@ -1111,7 +1126,7 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
         const void* base = raw_out ? (const void*)g.partial : (const void*)g.out;
         g.vec_out = g.N % 4 == 0 && ld % 4 == 0 && ((uintptr_t)base % 16) == 0 && (!raw_out || ((size_t)g.M * ld) % 4 == 0);
     }
-    k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK><<<tiles * g.splits, 64 * WM_ * WN_, smem, stream>>>(g);
+    k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK><<<groups, 64 * WM_ * WN_, smem, stream>>>(g);
     XR_CHECK_LAUNCH("gemm_tile_async");
     if (g.norm_whole) {
         k_gemm_finish_norm<<<(unsigned)g.M, 1024, 0, stream>>>(g);
