@@ -1557,12 +1557,12 @@ class Ops:
     # (1 where the workgroups of one request, 16 columns each, are as many as compute units):
     #   token by token: 4, and the longest chain, rows x `chain`, with 0.4 w a request beside it, or what fills the chip, w x (all
     #   rows x `bulk` and 0.65 a request, whose state is read and written)
-    #   in chunks: 12, and `run` a chunk and 2.3 a request, the longest chain or all of them x w, and `mats` w a chunk
+    #   in chunks: 15, and `run` a chunk and 2.3 a request, the longest chain or all of them x w, and `mats` w a chunk
     # Fitted to heads of 128 x 128, 16 and 32 of them, one portion of 96 to 2,048 rows alone and beside 1 to 63 decoded tokens, and 4
-    # to 20 portions of 95 to 512 rows.  With 32 heads the delta rule takes 28 us in chunks and 31 token by token for a portion of 96
-    # rows alone, 231 and 592 for 2,048; with 63 decoded tokens beside it 128 rows take 76 and 67 (and 667 where the decoded tokens
-    # were chunks, too), 400 rows 104 and 144, 2,048 rows 291 and 626; 20 portions of 100 rows 331 and 222.
-    CHUNK_COSTS = {"delta": (0.289, 0.115, 5.3, 1.85), "retention": (0.23, 0.09, 3.7, 0.97)}       # chain, bulk, run, mats
+    # to 20 portions of 95 to 512 rows.  With 32 heads the delta rule takes 31 us token by token for a portion of 96 rows alone and
+    # a little more in chunks, 592 and 256 for 2,048; with 63 decoded tokens beside it 128 rows take 67 and 80 (and 667 where the
+    # decoded tokens were chunks, too), 400 rows 144 and 110, 2,048 rows 626 and 305; 20 portions of 100 rows 222 and more than 331.
+    CHUNK_COSTS = {"delta": (0.289, 0.115, 5.3, 2.3), "retention": (0.23, 0.09, 3.45, 1.17)}       # chain, bulk, run, mats
     CHUNKS_FROM = 96                 # shorter portions never run in chunks
     CHUNKS_SCRATCH = 1 << 27         # floats that the chunks' matrices may take (steps of some 30,000 rows with 32 heads)
 
@@ -1590,7 +1590,7 @@ class Ops:
             rows, places, all_runs, longest = rows - n, places + chunks, all_runs + run * chunks + 2.3, max(longest, run * chunks + 2.3)
             if i + 1 < len(lens) and lens[i + 1] == n:
                 continue
-            t = 12.0 + max(longest, w * all_runs) + mats * w * places + tokens(i + 1, rows)
+            t = 15.0 + max(longest, w * all_runs) + mats * w * places + tokens(i + 1, rows)
             if t < best and places * self._chunk_floats(kind, H) <= self.CHUNKS_SCRATCH:
                 best, shortest = t, n
         return shortest

@@ -1,5 +1,5 @@
 // Retention and the gated delta rule over long portions, in chunks of 64 rows on the matrix cores with 32-bit operands,
-// products and sums (v_mfma_f32_16x16x4_f32).  The recurrences and the state are those of recurrent_kernels.hip:
+// products and sums (v_mfma_f32_16x16x4_f32; q . k in 64 bits, v_mfma_f64_16x16x4_f64).  The recurrences and the state are those of recurrent_kernels.hip:
 //
 //   retention:   S <- g S + k v^T;                                  o = S^T q
 //   delta rule:  S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
@@ -19,13 +19,14 @@
 // columns of the state (columns never meet), the state in LDS: three to five small products a chunk.  Rows past a portion's
 // end are zeros with beta 0 and no decay.  L is formed and subtracted in 64 bits; a decay of nothing counts as exp(-100).  A portion
 // that comes to something not finite, or has a negative decay, runs again token by token, a workgroup its 16 columns.
-// Bound by the chain of chunks, a chunk (5.7 us of the delta rule, 4.4 of retention) by five barriers, the trips to LDS between
-// them and, a third of it, its products.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 184 us and k_chunk_mats 59 for the
-// delta rule, 142 and 31 for retention; token by token (k_recurrence) 634, and retention in two passes over chunks of 256
-// side by side 520.
+// Bound by the chain of chunks, a chunk (5.7 us of the delta rule, 4.1 of retention) by five barriers, the trips to LDS between
+// them and, a third of it, its products.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 182 us and k_chunk_mats 74 for the
+// delta rule, 130 and 34 for retention (k_chunk_mats 57 and 24 with q . k in 32 bits); token by token (k_recurrence) 634, and
+// retention in two passes over chunks of 256 side by side 520.
 #include "common.h"
 
 typedef float rc_f32x4 __attribute__((ext_vector_type(4)));
+typedef double rc_f64x4 __attribute__((ext_vector_type(4)));
 #define RC_L 64                 // rows of a chunk
 #define RC_LDM (RC_L + 4)       // LDS floats between rows of a 64 x 64 matrix
 #define RC_C 16                 // columns of the state a workgroup takes
@@ -63,16 +64,24 @@ __device__ inline rc_f32x4 rc_mfma4(float4 a, float4 b, rc_f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
 }
 
-// 16 rows (a lane's at `rows`) times 16 columns of the state: two chains of products side by side, every operand read before them
+// The same in 64 bits (of a result a lane has the rows lane / 16 + 4 e of column lane % 16)
+__device__ inline rc_f64x4 rc_mfma4(float4 a, float4 b, rc_f64x4 c) {
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.x, (double)b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.y, (double)b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.z, (double)b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.w, (double)b.w, c, 0, 0, 0);
+}
+
+// 16 rows (a lane's at `rows`) times 16 columns of the state: four chains of products side by side, every operand read before them
 template <int J>
 __device__ inline rc_f32x4 times_state(const float* rows, const float* state) {
     float4 x[J], y[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) { x[j] = rc_ld4(rows + 16 * j); y[j] = rc_ld4(state + j * RC_C * 20); }
-    rc_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    rc_f32x4 s[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int j = 0; j < J; ++j) s[j & 1] = rc_mfma4(x[j], y[j], s[j & 1]);
-    return s[0] + s[1];
+    for (int j = 0; j < J; ++j) s[j & 3] = rc_mfma4(x[j], y[j], s[j & 3]);
+    return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 template <int D, bool DELTA>
@@ -129,19 +138,26 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
     }
     __syncthreads();
     for (int ct = 0; ct <= wave; ++ct) {                // rows 16 wave .., columns 16 ct ..
-        rc_f32x4 s = {0.f, 0.f, 0.f, 0.f}, t = s;
+        // q . k in 64 bits, k . k in four chains of 32: with one chain of 128 sums each the errors of the results were twice those
+        // of the recurrence token by token, and with these they are as large or smaller (retention's half)
+        rc_f64x4 s = {0.0, 0.0, 0.0, 0.0};
+        rc_f32x4 t[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
         for (int d = 0; d < D; d += 16) {
             const float4 fb = rc_ld4(K + (16 * ct + l16) * LD + d + 4 * quad);
             s = rc_mfma4(rc_ld4(Q + (16 * wave + l16) * LD + d + 4 * quad), fb, s);
-            if (DELTA) t = rc_mfma4(rc_ld4(K + (16 * wave + l16) * LD + d + 4 * quad), fb, t);
+            if (DELTA) t[d / 16 & 3] = rc_mfma4(rc_ld4(K + (16 * wave + l16) * LD + d + 4 * quad), fb, t[d / 16 & 3]);
         }
+        const rc_f32x4 kk = (t[0] + t[1]) + (t[2] + t[3]);
         const int j = 16 * ct + l16;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int i = 16 * wave + 4 * quad + e;
-            const float f = j <= i ? expf((float)(L[i] - L[j])) : 0.f;
-            mats[i * RC_L + j] = j <= i ? s[e] * f : 0.f;
-            if (DELTA) A[i * RC_LDM + j] = j < i ? beta[i] * f * t[e] : 0.f;
+            const int i = 16 * wave + 4 * e + quad;
+            mats[i * RC_L + j] = j <= i ? (float)(s[e] * expf((float)(L[i] - L[j]))) : 0.f;
+            if (DELTA) {
+                const int r = 16 * wave + 4 * quad + e;
+                A[r * RC_LDM + j] = j < r ? beta[r] * expf((float)(L[r] - L[j])) * kk[e] : 0.f;
+            }
         }
     }
     if (!DELTA) return;
@@ -288,21 +304,26 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] *= vec[i0 + e];
         __syncthreads();                                // U and W are there, and the state of the chunk's start is read
-        for (int m = 0; m <= wave; ++m) o = rc_mfma4(rc_ld4(P + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&U[l16][16 * m + 4 * quad]), o);
+        rc_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int m = 0; m < RC_L / 16; ++m)
+            if (m <= wave) p[m & 1] = rc_mfma4(rc_ld4(P + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&U[l16][16 * m + 4 * quad]), p[m & 1]);
+        o += p[0] + p[1];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (i0 + e < rows) a.out[((size_t)(row0 + i0 + e) * a.H + h) * a.Dv + c0 + l16] = o[e];
         none += 0.f * o[0] + 0.f * o[1] + 0.f * o[2] + 0.f * o[3];
         const float all = vec[RC_L - 1];                // exp(L_63)
         for (int j = wave; j < J; j += 4) {             // 16 rows of the state: its own decayed, and K^T W
-            float4 s0 = rc_ld4(&S[j][l16][4 * quad]);
-            rc_f32x4 s = {s0.x * all, s0.y * all, s0.z * all, s0.w * all};
+            const float4 s0 = rc_ld4(&S[j][l16][4 * quad]);
+            rc_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int m = 0; m < RC_L / 16; ++m) {
                 const float* kp = K + (16 * m + 4 * quad) * LD + 16 * j + l16;
-                s = rc_mfma4(make_float4(kp[0], kp[LD], kp[2 * LD], kp[3 * LD]), rc_ld4(&W[l16][16 * m + 4 * quad]), s);
+                s[m & 1] = rc_mfma4(make_float4(kp[0], kp[LD], kp[2 * LD], kp[3 * LD]), rc_ld4(&W[l16][16 * m + 4 * quad]), s[m & 1]);
             }
-            rc_st4(&S[j][l16][4 * quad], make_float4(s[0], s[1], s[2], s[3]));
+            const rc_f32x4 t = s[0] + s[1];
+            rc_st4(&S[j][l16][4 * quad], make_float4(fmaf(s0.x, all, t[0]), fmaf(s0.y, all, t[1]), fmaf(s0.z, all, t[2]), fmaf(s0.w, all, t[3])));
         }
     }
     __syncthreads();
