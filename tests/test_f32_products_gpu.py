@@ -52,3 +52,22 @@ def test_weight_rows_a_wave(M, N, K):
     # and the sums themselves: K products and additions of 2^-24 each
     want, size = (a.double() @ w.double().T), (a.double().abs() @ w.double().abs().T)
     assert ((narrow.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size).all()
+
+
+# tiles of one set of waves (more than 256 of 64 x 64) and of two, each from every second slice
+@pytest.mark.parametrize("M,N,K,many", [(17, 1000, 4096, False), (17, 2048, 14336, False), (130, 1024, 8192, False), (401, 4096, 8192, True)])
+def test_sums_of_one_sign_are_as_close_with_two_sets_of_waves(M, N, K, many):
+    """Positive numbers, whose sums only grow: compensated sums of runs, however many waves share the columns.  The same rows and
+    columns among so many that one set of waves makes each tile are the yardstick."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    assert (-(-M // 64) * -(-N // 64) > 256) == many
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w = (torch.rand(s, generator=g, device=dev) for s in ((M, K), (N, K)))
+    want = a.double() @ w.double().T
+    off = lambda got: ((got.double() - want).norm() / want.norm()).item()
+    rows = a.repeat(-(-257 * 64 // (-(-N // 64) * M)) + 1, 1)             # (each row's sum is its own: the first M of them)
+    assert -(-rows.shape[0] // 64) * -(-N // 64) > 256
+    assert off(ops.linear(a, w)) <= 1.02 * off(ops.linear(rows, w)[:M])   # (millions of roundings: their 2-norms agree to 1%)
