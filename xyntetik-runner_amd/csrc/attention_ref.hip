@@ -340,7 +340,8 @@ extern "C" int xr_attention_f32(float* out, const float* q, const float* k_cache
               page_size - 1, page_size, window, chunk, keep, ld_gate, ld_out, scale, cap, out_scale};
     const size_t bytes = af_lds_bytes(D, Dv);
     if (bytes > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        // (the largest there is, whatever this call needs: smaller heads of another thread would take it back)
+        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)af_lds_bytes(AF_MAX_D, AF_MAX_D));
         if (e != hipSuccess) (void)hipGetLastError();
         XR_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
     }
