@@ -1576,9 +1576,10 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
             // at 2.2 TB/s and costs a launch (a rotating product of up to 511 rows pays for that kernel whole, too: counted as free, it
             // sent 300 rows of a 3,072 to 5,120 product into one range, 35 us, where two take 29), and writes the norm that follows, if one was asked for: without
-            // ranges its kernel takes 12.5 us.  Fitted to 5,500 timed launches (the products of the 8B, the 7B and the 1B class's
+            // ranges that kernel counts 12.5 us, a number of the fit and above its own time (10.8 us at 2,048 rows of 4,096, 5.2 at 137).  Fitted to 5,500 timed launches (the products of the 8B, the 7B and the 1B class's
             // layers and Suripel's two, 66 to 2,048 rows, four tiles, 1 to 16 ranges): the tile and ranges chosen are 1.5% slower
-            // than the best of them on average (1.8% up to 300 rows), 6.6% with the model before it (which knew no memory time and too high a
+            // than the best of them on average (1.8% up to 300 rows; 2.9% over 294 products of seven other sets of sizes and today's order of
+            // the tiles), 6.6% with the model before it (which knew no memory time and too high a
             // price for 128x128 tiles: down at 137 rows in 256x256 tiles and 16 ranges 45-53 us, in 256x128 and 6 ranges 39-45;
             // a 4,096 to 6,144 product of 400 rows 47 us, in whole 128x128 tiles 32).
             // (Rotating products: the eight-wave kernels, but 128x128 tiles with four waves: 600 rows of a 4,096 to 6,144 product 42 us
