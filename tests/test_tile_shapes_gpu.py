@@ -1,0 +1,68 @@
+"""The tiles of 128, 160 and 192 rows: edges of tiles, every epilogue, rotation, and the choice among tiles and pairs of launches."""
+import pytest
+
+from test_kernels_gpu import check_projection_with_rotation_and_cache_write, ops, rel      # noqa: F401  (ops is the fixture)
+
+pytestmark = pytest.mark.gpu
+TILES = {16: (128, 256), 27: (192, 192), 28: (192, 128), 29: (160, 256)}
+
+
+@pytest.mark.parametrize("variant", sorted(TILES))
+@pytest.mark.parametrize("dm,dn,K", [(0, 0, 192), (1, 4, 256), (-1, -4, 1024), (None, 20, 4160)])
+def test_tiles_by_name(ops, variant, dm, dn, K):     # noqa: F811
+    """One row and column more or less than whole tiles, and fewer rows than a tile; the fewest slices of K that the loop takes."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import KernelError
+    bm, bn = TILES[variant]
+    M, N = (5 if dm is None else 2 * bm + dm), 3 * bn + dn
+    dev = torch.device("cuda:0")
+    torch.manual_seed(variant * 10 + K)
+    a = (torch.randn(M, K, device=dev) * 0.5).bfloat16()
+    w = (torch.randn(N, K, device=dev) * 0.1).bfloat16()
+    b = torch.randn(N, device=dev) * 0.1
+    plain = a.double() @ w.double().T
+    for wt in (w, ops.pack_weight(w)):
+        got = ops.linear(a, wt, bias=b, out_dtype=torch.float32, variant=variant)
+        assert rel(got, plain + b.double()) < 1e-5                                       # 32-bit sums
+        for order in (1000, 2000):                                                       # the other orders of workgroups
+            assert torch.equal(got, ops.linear(a, wt, bias=b, out_dtype=torch.float32, variant=order + variant))
+        assert rel(ops.linear(a, wt, bias=b, variant=variant), plain + b.double()) < 6e-3     # rounded once to bfloat16
+    base = torch.randn(M, N, device=dev)
+    out = base.clone()
+    ops.linear(a, w, out=out, accumulate=True, variant=variant)
+    assert rel(out, base.double() + plain) < 1e-5
+    w2 = (torch.randn(2 * N, K, device=dev) * 0.1).bfloat16()
+    if variant == 27:       # an odd number of 32-column tiles a wave: gate and up do not meet
+        with pytest.raises(KernelError, match="pair"):
+            ops.linear_swiglu(a, w2, variant=variant)
+    else:
+        r = a.double() @ w2.double().T
+        want = r[:, :N] / (1 + torch.exp(-r[:, :N])) * r[:, N:]
+        for wt in (w2, ops.pack_weight(w2, gated=True)):
+            assert rel(ops.linear_swiglu(a, wt, variant=variant), want) < 6e-3
+    for bad in (72, 128):   # no whole slices, and fewer than three
+        with pytest.raises(KernelError, match="four-wave"):
+            ops.linear(a[:, :bad].contiguous(), w[:, :bad].contiguous(), variant=variant)
+
+
+@pytest.mark.parametrize("variant", sorted(TILES))
+@pytest.mark.parametrize("H,Hk,D,rot,inter", [(4, 2, 64, 64, False), (3, 1, 48, 32, False), (2, 1, 80, 80, True), (5, 1, 128, 128, False)])
+def test_rotation_in_the_tiles_by_name(ops, variant, H, Hk, D, rot, inter):      # noqa: F811
+    check_projection_with_rotation_and_cache_write(ops, "bfloat16", H, Hk, D, rot, inter, 16, [5, 0], [530, 70], True, 256, variant=variant)
+
+
+@pytest.mark.parametrize("M", [137, 192, 193, 300, 321, 640, 1300, 1524])
+@pytest.mark.parametrize("N,K", [(4096, 512), (12288, 256), (11008, 328)])
+def test_the_chosen_tiles(ops, M, N, K):      # noqa: F811
+    """What the library chooses for sizes at which the new tiles, K ranges and two launches come in; K 328 is no whole slices, so
+    that only the loops that look at columns take it."""
+    import torch
+    dev = torch.device("cuda:0")
+    torch.manual_seed(M + N + K)
+    a = (torch.randn(M, K, device=dev) * 0.5).bfloat16()
+    w = (torch.randn(N, K, device=dev) * 0.1).bfloat16()
+    want = a.double() @ w.double().T
+    assert rel(ops.linear(a, ops.pack_weight(w), out_dtype=torch.float32), want) < 1e-5
+    half = N // 2 // 32 * 32
+    gate, up = want[:, :half], want[:, half:2 * half]
+    assert rel(ops.linear_swiglu(a, ops.pack_weight(w[:2 * half].contiguous(), gated=True)), gate / (1 + torch.exp(-gate)) * up) < 6e-3

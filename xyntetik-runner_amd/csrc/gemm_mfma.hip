@@ -1059,6 +1059,21 @@ __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
 // (what a launcher answers when its kernel does not take the product and another one must)
 #define XR_NOT_TAKEN -1000
 
+// Whether the loop with its instructions in a written order takes a product in `splits` K ranges of `k_per_split` columns: whole
+// slices only, at least `stages` of them in every range, and every lane's piece within 4 GB of the tile's first.
+static bool takes_written_order(const GemmArgs& g, int splits, int k_per_split, int bm, int bn, int stages, int bk) {
+    const int last = g.K - (splits - 1) * k_per_split;
+    const size_t span = (size_t)(g.epi == EPI_GATED ? g.N + bn : bn) + 16;
+    return g.K % bk == 0 && last >= stages * bk && k_per_split >= stages * bk && (size_t)bm * g.lda * 2 < (1ull << 32) &&
+           span * (size_t)(((g.K + 31) / 32) * 32) * 2 < (1ull << 32);
+}
+// K in `splits` ranges of whole 64-column slices: the columns of a range, and how many ranges that leaves (none of them empty)
+static int range_columns(int K, int& splits) {
+    const int slices = (K + 63) / 64, per = (slices + splits - 1) / splits;
+    splits = (slices + per - 1) / per;
+    return per * 64;
+}
+
 template <int BM, int BN, int WM_, int WN_, int ST, int PIPE = 0, int BK = 64>
 static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     if (g.epi == EPI_GATED && (BN / WN_ / 32) % 2) {
@@ -1086,13 +1101,7 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     unsigned tiles_n = (unsigned)((g.col1 - g.col0 + n_out_tile - 1) / n_out_tile), tiles_m = (unsigned)((g.M + BM - 1) / BM);
     unsigned tiles = tiles_n * tiles_m;
     if (g.splits < 1 || !g.partial || g.col0 > 0 || g.col1 < g.N) g.splits = 1;
-    if (g.splits > 1) {
-        int slices = (g.K + 63) / 64;
-        int per = (slices + g.splits - 1) / g.splits;
-        g.k_per_split = per * 64;
-        g.splits = (slices + per - 1) / per;            // no empty range
-    }
-    if (g.splits == 1) g.k_per_split = ((g.K + 63) / 64) * 64;
+    g.k_per_split = range_columns(g.K, g.splits);
     unsigned groups = tiles * g.splits;
     if (g.m_fast == 2) {
         const unsigned columns = tiles_m * ((tiles_n + 7) / 8), even = (groups + 7) / 8;      // workgroups of the XCD that has most
@@ -1105,16 +1114,7 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
             groups = 8 * columns;
         }
     }
-    if (PIPE == 2) {
-        // the loop with its instructions in a written order: whole slices only, at least ST of them
-        // in every K range, and every lane's piece within 4 GB of the tile's first
-        const int last = g.K - (g.splits - 1) * g.k_per_split;
-        const size_t span = (size_t)(g.epi == EPI_GATED ? g.N + BN : BN) + 16;
-        if (g.K % BK || last < ST * BK || g.k_per_split < ST * BK || (size_t)BM * g.lda * 2 >= (1ull << 32) ||
-            span * (size_t)(((g.K + 31) / 32) * 32) * 2 >= (1ull << 32)) {
-            return XR_NOT_TAKEN;
-        }
-    }
+    if (PIPE == 2 && !takes_written_order(g, g.splits, g.k_per_split, BM, BN, ST, BK)) return XR_NOT_TAKEN;
     if (g.raw && (!g.partial || g.col0 > 0 || g.col1 < g.N)) {
         xr_set_error("gemm: no room for the raw sums of a product whose epilogue is a kernel of its own");
         return XR_BAD_ARG;
@@ -1358,7 +1358,19 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
         if (rc != XR_NOT_TAKEN) return rc;
     }
     if (variant == 17 || variant == 117) return launch_tile_async<128, 128, 2, 2, 4, false>(g, stream);
-    if (variant == 51 || variant == 55 || variant == 58) {
+    // Tiles of 128, 160 and 192 rows, four waves and the written order only: between them and the three above a launch's workgroups
+    // come closer to whole rounds of 256, and 129 to 192 rows pay for 192 instead of 256.  (192x128 and 192x192 with three slices in
+    // flight; a fourth, all 160 KB of LDS, gains nothing.  160x256: waves side by side, each all 160 rows of 64 columns.)  Measured
+    // against the best of 256x256, 256x192, 256x128 and 128x128, us: gate+up of the 8B shape at 137 rows 61.8 -> 57.1 (192x128), at
+    // 300 104.9 -> 73.3 and at 640 168.8 -> 141.1 (160x256); 12,288 x 4,096 at 1,524 rows 163.5 -> 131.7 and 6,144 x 4,096 at 1,300
+    // 89.2 -> 61.8 (192x192); gate+up of the 7B class at 640 rows 151.3 -> 121.3 (128x256).
+    int rc = XR_NOT_TAKEN;
+    if (variant == 16) rc = launch_tile_async<128, 256, 2, 2, 3, 2, 64>(g, stream);
+    if (variant == 27) rc = launch_tile_async<192, 192, 2, 2, 3, 2, 64>(g, stream);
+    if (variant == 28) rc = launch_tile_async<192, 128, 2, 2, 3, 2, 64>(g, stream);
+    if (variant == 29) rc = launch_tile_async<160, 256, 1, 4, 3, 2, 64>(g, stream);
+    if (rc != XR_NOT_TAKEN) return rc;
+    if (variant == 51 || variant == 55 || variant == 58 || variant == 16 || (variant >= 27 && variant <= 29)) {
         xr_set_error("gemm: the four-wave kernel does not take K %d in %d ranges, lda %d, or a rotation", g.K, g.splits, g.lda);
         return XR_BAD_ARG;
     }
@@ -1571,65 +1583,79 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // columns of the full rounds go to that tile and the rest to a second launch with a
             // smaller one (3 rounds + 1 of half-size tiles instead of 4).
             // The model, in seconds (tuning measured on an MI355X, not limits: elsewhere it costs speed only): a round of
-            // tiles takes its products' time, bm bn K x 0.36e-12 / rate (97 us for 256x256 and K = 4,096 as measured), or that of its
-            // weights from memory at `bytes` a second, whichever is longer; `launch` once and `round` for every round (a product that
+            // tiles takes its products' time, bm bn K x 0.36e-12 / rate (89 us for 256x256 and K = 4,096 as measured), or that of its
+            // weights from memory at `bytes` a second, whichever is longer; a last round that fills the chip by a share f does its products
+            // in 0.8 + 0.2 f of that (fewer tiles meet at L2, and the clock falls less); `launch` once and `round` for every round (a product that
             // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
             // at 2.2 TB/s and costs a launch (a rotating product of up to 511 rows pays for that kernel whole, too: counted as free, it
             // sent 300 rows of a 3,072 to 5,120 product into one range, 35 us, where two take 29), and writes the norm that follows, if one was asked for: without
-            // ranges that kernel counts 12.5 us, a number of the fit and above its own time (10.8 us at 2,048 rows of 4,096, 5.2 at 137).  Fitted to 5,500 timed launches (the products of the 8B, the 7B and the 1B class's
-            // layers and Suripel's two, 66 to 2,048 rows, four tiles, 1 to 16 ranges): the tile and ranges chosen are 1.5% slower
-            // than the best of them on average (1.8% up to 300 rows; 2.9% over 294 products of seven other sets of sizes and today's order of
-            // the tiles), 6.6% with the model before it (which knew no memory time and too high a
-            // price for 128x128 tiles: down at 137 rows in 256x256 tiles and 16 ranges 45-53 us, in 256x128 and 6 ranges 39-45;
-            // a 4,096 to 6,144 product of 400 rows 47 us, in whole 128x128 tiles 32).
-            // (Rotating products: the eight-wave kernels, but 128x128 tiles with four waves: 600 rows of a 4,096 to 6,144 product 42 us
-            // against 53, 800 rows 72 against 98.)
-            struct Cand { int variant, bm, bn; double rate, launch, round, bytes; };
-            const Cand plain[4] = {{14, 256, 256, 1.0, 4.3e-6, 0.0, 6.0e12}, {26, 256, 192, 0.85, 3.7e-6, 0.0, 3.9e12},
-                                   {12, 256, 128, 0.89, 3.7e-6, 0.0, 3.6e12}, {17, 128, 128, 0.71, 3.9e-6, 0.0, 5.6e12}};
-            const Cand turning[4] = {{14, 256, 256, 0.95, 0.0, 8e-6, 5.0e12}, {26, 256, 192, 0.81, 0.0, 9e-6, 5.0e12},
-                                     {12, 256, 128, 0.91, 0.0, 9e-6, 4.1e12}, {17, 128, 128, 0.76, 0.0, 9e-6, 4.1e12}};
+            // ranges that kernel counts 12.5 us, a number of the fit and above its own time (10.8 us at 2,048 rows of 4,096, 5.2 at 137).  Fitted to 7,700 timed
+            // launches (the products of the 8B, the 7B and the 1B class's layers and Suripel's two widths, 96 to 2,048 rows, fourteen tiles,
+            // 1 to 16 ranges): the tile and ranges chosen are 2.1% slower on average than the best of all fourteen (8% in the worst tenth); the best choice
+            // among 256x256, 256x192, 256x128 and 128x128 alone is 6.5% (18%).  Of the tiles that were left out none brings 0.2% on average:
+            // 192x256, 256x192 and 128x192 with four waves, 320x192, 320x128, 96x256, and a fifth or sixth slice in flight.
+            // (Rotating products: the eight-wave kernels, but for 128x128 and the tiles that have four waves only: 600 rows of a 4,096 to 6,144 product 42 us
+            // against 53, 800 rows 72 against 98; 1,300 rows in 192x192 tiles 78 against 94.  Fitted to 33 products of three shapes, 520 to 2,048 rows.)
+            struct Cand { int variant, bm, bn, stages; double rate, launch, round, bytes; };
+            constexpr int N_CANDS = 7;
+            const Cand plain[N_CANDS] = {{14, 256, 256, 0, 1.094, 2.3e-6, 0.0, 4.6e12}, {27, 192, 192, 3, 1.056, 3.7e-6, 0.0, 5.1e12},
+                                         {12, 256, 128, 0, 0.995, 3.6e-6, 0.0, 4.2e12}, {29, 160, 256, 3, 1.006, 3.8e-6, 0.0, 5.3e12},
+                                         {16, 128, 256, 3, 0.886, 3.4e-6, 0.0, 5.8e12}, {28, 192, 128, 3, 0.827, 2.8e-6, 0.0, 4.6e12},
+                                         {17, 128, 128, 0, 0.690, 2.9e-6, 0.0, 5.5e12}};
+            const Cand turning[N_CANDS] = {{14, 256, 256, 0, 0.804, 0.0, 0.0, 5.0e12}, {26, 256, 192, 0, 0.892, 0.0, 20e-6, 5.0e12},
+                                           {12, 256, 128, 0, 0.939, 0.0, 14.5e-6, 5.0e12}, {27, 192, 192, 3, 0.923, 0.0, 20e-6, 5.0e12},
+                                           {16, 128, 256, 3, 0.925, 0.0, 20e-6, 5.0e12}, {28, 192, 128, 3, 1.061, 0.0, 20e-6, 5.0e12},
+                                           {17, 128, 128, 0, 0.849, 0.0, 12.6e-6, 5.0e12}};
             const Cand* cands = rope_direct ? turning : plain;
             auto width = [&](const Cand& c) { return sw ? c.bn / 2 : c.bn; };
-            auto usable = [&](const Cand& c) { return !(sw && c.variant == 26); };
+            // (256x192 and 192x192 tiles do not pair gate and up columns; the tiles with the written order only need whole slices)
+            auto usable = [&](const Cand& c, int ranges) {
+                if (sw && c.bn == 192) return false;
+                if (!c.stages) return true;
+                int r = ranges;
+                const int columns = range_columns(K, r);
+                return takes_written_order(g, r, columns, c.bm, c.bn, c.stages, 64);
+            };
             auto count = [&](const Cand& c, int cols) { return ((M + c.bm - 1) / c.bm) * ((cols + width(c) - 1) / width(c)); };
             auto seconds = [&](const Cand& c, int cols, int ranges) {
                 const int groups = count(c, cols) * ranges, rounds = (groups + 255) / 256, rows = (M + c.bm - 1) / c.bm;
                 const double k = (K + ranges - 1) / ranges, products = (double)c.bm * c.bn * k * 0.36e-12 / c.rate;
-                const double weights = (double)(groups < 256 ? groups : 256) * c.bn * k * 2 / rows / c.bytes;
-                return rounds * ((products > weights ? products : weights) + c.round) + c.launch;
+                const double last = (groups - (rounds - 1) * 256) / 256.0, weights = 256.0 * c.bn * k * 2 / rows / c.bytes;
+                const double products_last = products * (0.8 + 0.2 * last), weights_last = weights * last;
+                return (rounds - 1) * (products > weights ? products : weights) + (products_last > weights_last ? products_last : weights_last) +
+                       rounds * c.round + c.launch;
             };
-            auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.2e12 + 4e-6; };
+            auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.2e12 + 3e-6; };
             const double norm_alone = want_whole_norm ? 12.5e-6 : 0.0;
             int best = 0, best_splits = 1, second = -1, cols_first = N;
             double t_best = 1e30;
             // Up to 128 rows are one row of 128x128 tiles: K in as many ranges as make one round of workgroups, or whole from 160
             // tiles on.  (Timed alone, five or six ranges of 32 tiles are 2-5% faster than eight; among a layer's other kernels the
             // prompt of 70 to 128 tokens is 2-3% slower with them: 1,286 us against 1,267, 1,378 against 1,336, 1,441 against 1,407.)
-            const bool one_row = M <= 128 && !rope_direct && count(cands[3], N) <= 256;
+            const bool one_row = M <= 128 && !rope_direct && count(cands[N_CANDS - 1], N) <= 256;
             if (one_row) {
-                const int c = count(cands[3], N);
-                best = 3;
+                const int c = count(cands[N_CANDS - 1], N);
+                best = N_CANDS - 1;
                 best_splits = c < 160 ? pick_splits(c) : 1;
                 t_best = 0.0;
             }
-            for (int i = 0; i < 4 && !one_row; ++i) {
-                if (!usable(cands[i])) continue;
+            for (int i = 0; i < N_CANDS && !one_row; ++i) {
                 const int c = count(cands[i], N);
                 for (int sp = 1; sp <= 16; ++sp) {
                     if (sp > 1 && (rope_direct || !workspace || c * sp > 256 || K / sp < 256 || (size_t)sp * M * w_rows * 4 > workspace_bytes)) break;
+                    if (!usable(cands[i], sp)) continue;
                     const double t = seconds(cands[i], N, sp) + (sp > 1 || g.raw ? adding(sp) : norm_alone);
                     if (t < t_best) { best = i; best_splits = sp; t_best = t; }
                 }
             }
             // (one launch where the epilogue is a kernel of its own: that kernel takes the raw sums of all columns)
-            for (int i = 0; i < 3 && !one_row && !g.raw; ++i) {
-                if (!usable(cands[i])) continue;
+            for (int i = 0; i < N_CANDS && !one_row && !g.raw; ++i) {
+                if (!usable(cands[i], 1)) continue;
                 const int tm = (M + cands[i].bm - 1) / cands[i].bm, full = count(cands[i], N) / 256;
                 const int cols = full * 256 / tm * width(cands[i]);          // the columns of the full rounds
                 if (full < 1 || count(cands[i], N) % 256 == 0 || cols <= 0 || cols >= N) continue;
-                for (int j = i + 1; j < 4; ++j) {
-                    if (!usable(cands[j]) || cols % width(cands[j])) continue;
+                for (int j = 0; j < N_CANDS; ++j) {
+                    if (j == i || !usable(cands[j], 1) || cols % width(cands[j])) continue;
                     const double t = seconds(cands[i], cols, 1) + seconds(cands[j], N - cols, 1) + norm_alone;
                     if (t < 0.98 * t_best) { best = i; best_splits = 1; second = j; cols_first = cols; t_best = t; }   // (a second launch costs a little, too)
                 }
