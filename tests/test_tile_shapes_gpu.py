@@ -66,3 +66,22 @@ def test_the_chosen_tiles(ops, M, N, K):      # noqa: F811
     half = N // 2 // 32 * 32
     gate, up = want[:, :half], want[:, half:2 * half]
     assert rel(ops.linear_swiglu(a, ops.pack_weight(w[:2 * half].contiguous(), gated=True)), gate / (1 + torch.exp(-gate)) * up) < 6e-3
+
+
+# rows of one row of tiles; column tiles enough for workgroups to begin at every slice of K and go round (K 256: as many slices as the
+# loop has in flight), a K range each with streaming copies (17 rows) and without (64 rows)
+@pytest.mark.parametrize("variant,M,N,K", [(0, 17, 5128, 256), (0, 64, 5128, 320), (58, 128, 5128, 256), (28, 192, 5128, 192), (55, 256, 5128, 192),
+                                           (0, 64, 20480, 4096), (0, 17, 2048, 8192), (0, 64, 2048, 8192), (0, 128, 21504, 1024)])
+def test_one_row_of_tiles(ops, variant, M, N, K):      # noqa: F811
+    import torch
+    dev = torch.device("cuda:0")
+    torch.manual_seed(M + N + K)
+    a = (torch.randn(M, K, device=dev) * 0.5).bfloat16()
+    w = (torch.randn(N, K, device=dev) * 0.1).bfloat16()
+    want = a.double() @ w.double().T
+    for wt in (w, ops.pack_weight(w)):
+        assert rel(ops.linear(a, wt, out_dtype=torch.float32, variant=variant), want) < 1e-5
+    half = N // 2 // 32 * 32
+    w2 = w[:2 * half].contiguous()
+    for wt in (w2, ops.pack_weight(w2, gated=True)):
+        assert rel(ops.linear_swiglu(a, wt, variant=variant), want[:, :half] / (1 + torch.exp(-want[:, :half])) * want[:, half:2 * half]) < 6e-3

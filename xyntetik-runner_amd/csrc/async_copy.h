@@ -24,6 +24,11 @@ __device__ inline void lds_dma16_base(const void* base, uint32_t byte_offset, ui
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :: "v"(byte_offset), "s"(base), "s"(lds_byte_addr) : "memory");
 }
+// the same for what is read once (a stream that must not push out what others read again)
+__device__ inline void lds_dma16_base_stream(const void* base, uint32_t byte_offset, uint32_t lds_byte_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                 :: "v"(byte_offset), "s"(base), "s"(lds_byte_addr) : "memory");
+}
 template <int N> __device__ inline void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "the counter holds 6 bits");
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");

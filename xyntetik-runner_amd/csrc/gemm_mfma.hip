@@ -460,7 +460,13 @@ template <int LOADS> __device__ inline void wait_slices(int slices) {
     else wait_vmcnt<LOADS * 3>();
 }
 
-template <int BM, int BN, int WARPS_M, int WARPS_N, int STAGES, int PIPE = 0, int BK = 64>
+// ONCE (written order only): the launch has one row of tiles, so every weight is read by one workgroup alone.  Its copies of weights
+// are marked as streaming, and a workgroup begins its K range item / 8 slices in and goes round to what it left out: the 16-row groups of
+// packed weights lie K x 32 bytes apart, and with K a power of two workgroups in step with each other ask the same few channels of
+// memory at a time.  (Copies alone, 224 tiles of 128 weight rows of 4,096 columns: 41.5 us; streaming 38.2, both 36.0; one start for each
+// of 8 neighbours, or one of its own for every workgroup, is no faster than none.  Gate+up of the 8B shape at 64 rows 49.2 us -> 38.9,
+// at 137 57.1 -> 54.3.)
+template <int BM, int BN, int WARPS_M, int WARPS_N, int STAGES, int PIPE = 0, int BK = 64, bool ONCE = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uint4* lds) {
     constexpr int WAVES = WARPS_M * WARPS_N;
     constexpr int CH = BK / 8, RPL = 64 / CH;           // chunks of a row; rows that one load instruction covers
@@ -631,13 +637,30 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
                                     : (uint32_t)((n - n_base) * g.K + c * 8) * 2u;
             }
         }
-        const bf16_t* a_nxt = g.a + (size_t)m0 * g.lda + k_begin;
-        const bf16_t* w_nxt = g.w_packed ? g.w + (size_t)(n_base >> 4) * kblocks * 512 + (size_t)k_begin * 16
-                                         : g.w + (size_t)n_base * g.K + k_begin;
+        int next = 0;                                             // the slice that the next copies bring, counted from k_begin
+        if constexpr (ONCE) next = __builtin_amdgcn_readfirstlane((item >> 3) % nk);
         const int w_step = g.w_packed ? BK * 16 : BK;
+        const bf16_t* a_nxt = g.a + (size_t)m0 * g.lda + k_begin + next * BK;
+        const bf16_t* w_nxt = (g.w_packed ? g.w + (size_t)(n_base >> 4) * kblocks * 512 + (size_t)k_begin * 16
+                                          : g.w + (size_t)n_base * g.K + k_begin) + (size_t)next * w_step;
+        auto advance = [&]() {
+            a_nxt += BK;
+            w_nxt += w_step;
+            if constexpr (ONCE) {
+                if (++next == nk) {
+                    next = 0;
+                    a_nxt -= nk * BK;
+                    w_nxt -= (size_t)nk * w_step;
+                }
+            }
+        };
         bf16x8 af[2][TM], wf[2][TN];
 #define LONE_COPY(DI, DST)                                                                           \
-    lds_dma16_base((DI) < LA ? a_nxt : w_nxt, off[DI], lds_wave + (uint32_t)((DST) * BUF * 16 + (DI) * WAVES * 64 * 16));
+    {                                                                                                \
+        const uint32_t to_ = lds_wave + (uint32_t)((DST) * BUF * 16 + (DI) * WAVES * 64 * 16);       \
+        if (ONCE && (DI) >= LA) lds_dma16_base_stream(w_nxt, off[DI], to_);                          \
+        else lds_dma16_base((DI) < LA ? a_nxt : w_nxt, off[DI], to_);                                \
+    }
 // one k-step: the products of fragment set F; if RD, the reads of k-step RD_KS of the slice in
 // buffer RD_BUF into the other set; if PART >= 0, copies PART*DPK .. of the next slice into buffer DST
 #define LONE_KSTEP(F, RD, RD_BUF, RD_KS, PART, DST)                                                  \
@@ -666,7 +689,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
             }                                                                                        \
             __builtin_amdgcn_sched_barrier(0);                                                       \
         }                                                                                            \
-        if ((PART) == DSTEPS - 1) { a_nxt += BK; w_nxt += w_step; }                                                 \
+        if ((PART) == DSTEPS - 1) advance();                                                         \
     }
 // the last k-step of the slice in buffer SB, behind the barrier that frees this buffer and
 // certifies the next slice, and the other k-steps of the slice after it
@@ -684,8 +707,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
         for (int st = 0; st < STAGES; ++st) {
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) LONE_COPY(i, st)
-            a_nxt += BK;
-            w_nxt += w_step;
+            advance();
         }
         wait_vmcnt<LOADS * (STAGES - 1)>();              // slice 0 has landed
         __builtin_amdgcn_s_barrier();
@@ -938,10 +960,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
 // One workgroup a tile and K range.  (Workgroups that stay and take every 256th tile were measured
 // too, with the tiles assigned in turn or taken from a counter: no faster, and what the compiler then
 // keeps in registers from tile to tile it spills.)
-template <int BM, int BN, int WARPS_M, int WARPS_N, int STAGES, int PIPE = 0, int BK = 64>
+template <int BM, int BN, int WARPS_M, int WARPS_N, int STAGES, int PIPE = 0, int BK = 64, bool ONCE = false>
 __global__ __launch_bounds__(64 * WARPS_M * WARPS_N) void k_gemm_tile_async(GemmArgs g) {
     extern __shared__ uint4 lds[];
-    gemm_tile<BM, BN, WARPS_M, WARPS_N, STAGES, PIPE, BK>(g, (int)blockIdx.x, lds);
+    gemm_tile<BM, BN, WARPS_M, WARPS_N, STAGES, PIPE, BK, ONCE>(g, (int)blockIdx.x, lds);
 }
 
 // Sums the K ranges of a split product in a fixed order and applies the epilogue.
@@ -1074,7 +1096,11 @@ static int range_columns(int K, int& splits) {
     return per * 64;
 }
 
-template <int BM, int BN, int WM_, int WN_, int ST, int PIPE = 0, int BK = 64>
+// WITH_ONCE: there is a kernel for launches of one row of tiles, too (see ONCE at gemm_tile).  It serves where K is whole, and where
+// the sums of the K ranges are at most a fourteenth of the weights' bytes: the kernel that adds the ranges up reads those sums from the
+// caches, and beside weights that stream past it that is slower (streaming and in turn against plain: the down product of the 8B shape in 8
+// ranges at 24 rows 24.0 us and 26.3, at 64 27.6 and 28.0, at 128 35.3 and 34.2; the output product at 64 rows 15.6 and 14.3).
+template <int BM, int BN, int WM_, int WN_, int ST, int PIPE = 0, int BK = 64, bool WITH_ONCE = false>
 static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     if (g.epi == EPI_GATED && (BN / WN_ / 32) % 2) {
         xr_set_error("gemm: a %dx%d tile cannot pair gate and up columns", BM, BN);
@@ -1085,6 +1111,9 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        if (WITH_ONCE && e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK, WITH_ONCE>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) {
             (void)hipGetLastError();             // or the next launch's check would report this refusal
             xr_set_error("gemm: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
@@ -1126,7 +1155,10 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
         const void* base = raw_out ? (const void*)g.partial : (const void*)g.out;
         g.vec_out = g.N % 4 == 0 && ld % 4 == 0 && ((uintptr_t)base % 16) == 0 && (!raw_out || ((size_t)g.M * ld) % 4 == 0);
     }
-    k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK><<<groups, 64 * WM_ * WN_, smem, stream>>>(g);
+    if (WITH_ONCE && tiles_m == 1 && (g.splits == 1 || (size_t)g.splits * g.M * 28 <= (size_t)g.K))
+        k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK, WITH_ONCE><<<groups, 64 * WM_ * WN_, smem, stream>>>(g);
+    else
+        k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK><<<groups, 64 * WM_ * WN_, smem, stream>>>(g);
     XR_CHECK_LAUNCH("gemm_tile_async");
     if (g.norm_whole) {
         k_gemm_finish_norm<<<(unsigned)g.M, 1024, 0, stream>>>(g);
@@ -1337,7 +1369,7 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
     // the rotation is work for the vector units, where four waves with 16 tiles each took 128 us for the
     // q/k/v product of 2,048 rows against 115 in 256x192 tiles with eight.)
     if ((variant == 12 && !g.rope.cs) || variant == 55) {
-        const int rc = launch_tile_async<256, 128, 2, 2, 3, 2, 64>(g, stream);
+        const int rc = launch_tile_async<256, 128, 2, 2, 3, 2, 64, true>(g, stream);
         if (rc != XR_NOT_TAKEN) return rc;
     }
     if (variant == 12) return launch_tile_async<256, 128, 4, 2, 3, 1>(g, stream);
@@ -1354,7 +1386,7 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
     // (the written order also where the weights' arrival bounds the kernel: little, 1-2%)
     // (here also where the product rotates its result: 600 rows of a 4,096 to 6,144 product 42 us against 53)
     if (variant == 17 || variant == 58) {
-        const int rc = launch_tile_async<128, 128, 2, 2, 4, 2, 64>(g, stream);
+        const int rc = launch_tile_async<128, 128, 2, 2, 4, 2, 64, true>(g, stream);
         if (rc != XR_NOT_TAKEN) return rc;
     }
     if (variant == 17 || variant == 117) return launch_tile_async<128, 128, 2, 2, 4, false>(g, stream);
@@ -1367,7 +1399,7 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
     int rc = XR_NOT_TAKEN;
     if (variant == 16) rc = launch_tile_async<128, 256, 2, 2, 3, 2, 64>(g, stream);
     if (variant == 27) rc = launch_tile_async<192, 192, 2, 2, 3, 2, 64>(g, stream);
-    if (variant == 28) rc = launch_tile_async<192, 128, 2, 2, 3, 2, 64>(g, stream);
+    if (variant == 28) rc = launch_tile_async<192, 128, 2, 2, 3, 2, 64, true>(g, stream);
     if (variant == 29) rc = launch_tile_async<160, 256, 1, 4, 3, 2, 64>(g, stream);
     if (rc != XR_NOT_TAKEN) return rc;
     if (variant == 51 || variant == 55 || variant == 58 || variant == 16 || (variant >= 27 && variant <= 29)) {
@@ -1703,7 +1735,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         // the others as before; five, 256 weight rows a tile, or twice the K ranges for two
         // workgroups a compute unit gain nothing or lose)
         // (with the order of instructions written out where the product allows: decode at batch 64 7.43 -> 7.31 ms)
-        const int rc = launch_tile_async<64, 128, 2, 2, 4, 2, 64>(g, stream);
+        const int rc = launch_tile_async<64, 128, 2, 2, 4, 2, 64, true>(g, stream);
         return rc != XR_NOT_TAKEN ? rc : launch_tile_async<64, 128, 2, 2, 4>(g, stream);
     }
     return launch_tile_variant(variant, g, stream);
