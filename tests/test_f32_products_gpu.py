@@ -71,3 +71,29 @@ def test_sums_of_one_sign_are_as_close_with_two_sets_of_waves(M, N, K, many):
     rows = a.repeat(-(-257 * 64 // (-(-N // 64) * M)) + 1, 1)             # (each row's sum is its own: the first M of them)
     assert -(-rows.shape[0] // 64) * -(-N // 64) > 256
     assert off(ops.linear(a, w)) <= 1.02 * off(ops.linear(rows, w)[:M])   # (millions of roundings: their 2-norms agree to 1%)
+
+
+# rows and weight rows at the edges of tiles of 32 and 64 for which one, two and four sets of waves share the columns; columns that are whole
+# stages of one, two or four slices of 32, and that are not (516, 1028); fewer slices than a run (544)
+@pytest.mark.parametrize("M,N", [(17, 31), (32, 2048), (33, 2050), (64, 4097), (401, 3072), (300, 96), (130, 8200)])
+@pytest.mark.parametrize("K", [516, 544, 1024, 1028, 2080])
+def test_products_shared_by_sets_of_waves(M, N, K):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w, bias, c = (torch.randn(s, generator=g, device=dev) for s in ((M, K + 4), (N, K), (N,), (M, N)))
+    a = a[:, 4:]
+    want = a.double() @ w.double().T
+    # (each product and sum rounds to 2^-24 of what has been added up so far)
+    bound = (K + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs() + c.double().abs())
+    assert ((ops.linear(a, w).double() - want).abs() <= bound).all()
+    assert ((ops.linear(a, w, bias=bias).double() - want - bias.double()).abs() <= bound).all()
+    out = c.clone()
+    ops.linear(a, w, out=out, accumulate=True)
+    assert ((out.double() - want - c.double()).abs() <= bound).all()
+    a[0, K // 2] = float("inf")
+    got = ops.linear(a, w)
+    assert not torch.isfinite(got[0]).any() and not torch.isnan(got[0][w[:, K // 2] != 0]).any()      # (an infinite sum stays infinite)
+    assert ((got[1:].double() - want[1:]).abs() <= bound[1:]).all()

@@ -8,12 +8,14 @@
 // (k_gemv_ref) gives every lane every 64th group of four columns and adds the lanes' sums in a
 // tree.  A token's 32-bit result therefore differs in its last bits between a step of 16 rows and
 // one of 17 (both stay within 1e-6 of the exact product at K = 14,336), and between steps of so many rows that
-// k_gemm_f32 takes another number of waves for a tile (a run is then 128 columns of every second slice of 32).
+// k_gemm_f32 takes another number of waves for a tile (a run is then 128 columns of every second or fourth slice of 32).
 // The tile kernels' two levels: runs of RBK * RB_FOLD = 128 columns are summed one after another, and the runs'
 // sums are added up with a compensated (Kahan) sum.  One running 32-bit sum over the 14,336
 // columns of a wide feed-forward loses about 1e-5 of the result to rounding, which at such
 // widths is as much as a real fault may be; summed this way a product is about ten times closer
 // to the exact one, so the 32-bit path can be held to the tolerance that small models are.
+#include <type_traits>
+
 #include "common.h"
 #include "async_copy.h"
 
@@ -97,53 +99,77 @@ __global__ __launch_bounds__(256) void k_gemm_ref(TO* __restrict__ out, const TI
 }
 
 // The same sums on the matrix cores (v_mfma_f32_32x32x2_f32: 32-bit operands, products and sums), 16-byte pieces copied
-// straight into LDS.  A workgroup of four waves, two by two, makes a tile of BM x BN from slices of 32 columns, STAGES - 1 of
-// them on their way while one is used: a slice's products take a wave 1,000 to 2,000 cycles, less than a trip to memory
-// (with the next slice alone ahead of the products, through registers, 401 x 2048 x 8192 took 213 us and 2048 x 16384 x 2048 1,237).
+// straight into LDS.  A workgroup makes a tile of BM x BN from slices of 32 columns, STAGES - 1 of
+// them on their way while one is used (a slice's products take a wave 1,000 to 2,000 cycles).
 // An MFMA step takes two columns, one from each half of the wave; which two does not matter as long as both operands agree,
 // so a lane reads four columns at once (its half's) and feeds four steps with them.  A row's eight pieces lie turned by
 // half its number, so that the reads of 16 rows meet no bank twice.  Workgroup i runs on XCD i % 8, and an XCD takes an
 // eighth of the tiles, row tiles first: a weight tile comes from memory for one XCD (401 x 128256 x 2048, 1 GB of weights, read
 // them four times with the column tiles first).
-// Bound by the matrix cores' 32-bit rate (157 TFLOP/s): 2048 x 16384 x 2048 at 112 to 119 TFLOP/s, 401 x 128256 x 2048 at 100 to 105
-// (84 before), 401 x 2048 x 8192 at 79 (63; 224 tiles for 256 compute units); the FMA kernel above reached 18 to 25.
+// Bound by the matrix cores' 32-bit rate (157 TFLOP/s; 153 is what the card's library gets of it on 8192 x 8192 x 8192) and the sums of
+// runs: 2048 x 16384 x 2048 at 131 TFLOP/s, 401 x 128256 x 2048 at 126, 401 x 2048 x 8192 at 95 (416 rows of tiles, 3.25 tiles of
+// 32 x 32 a compute unit where four are the fullest one's); the FMA kernel above reached 18 to 25.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define FBK 32
 
-// KG 2 (few tiles): two sets of four waves make the same tile, each from every second slice, and add their sums up at the end:
-// two waves a SIMD, one of which works while the other waits for its reads.
-template <typename TO, bool ACC, int BM, int BN, int STAGES, int KG>
-__global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+// GM x GN waves make a tile, each its 32 x 32 tiles.  KG > 1 (few tiles): KG sets of so many waves make the same tile, each from every
+// KG-th slice, and add their sums up at the end.  The products of one wave do not overlap its own sums of runs, nor its waits for reads
+// and for the other waves, so what keeps the matrix cores busy is waves: two stages of 64 x 64 or 32 x 64 in LDS leave room for four and
+// more a SIMD.  (2048 x 16384 x 2048: three stages of 64 x 128, two waves a SIMD, 1,302 us; with a run's four stages unrolled, so that no
+// sums move between registers, 1,187; two stages of 64 x 64 and four waves 1,070.  Without the sums of runs 1,034, and they cannot go.)
+// WHOLE: K is whole stages.  A row that does not exist is then read from the last one that does (its results are not stored), so
+// that a copy is a base in scalar registers and a fixed offset a lane; else a lane's pieces beyond the matrices are zeros.
+template <typename TO, bool ACC, int GM, int GN, int BM, int BN, int STAGES, int KG, bool WHOLE>
+__global__ __launch_bounds__(64 * GM * GN * KG, 4) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
                                                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
-    constexpr int TM = BM / 64, TN = BN / 64;           // 32 x 32 tiles a wave
+    constexpr int WAVES = GM * GN;                      // of a set
+    constexpr int TM = BM / 32 / GM, TN = BN / 32 / GN; // 32 x 32 tiles a wave
     constexpr int ROWS = BM + BN, CH = FBK / 4;         // rows of a slice (activations, then weights), pieces of a row
-    constexpr int LOADS = ROWS * CH / 256;              // copies a lane and stage (KG slices)
-    static_assert(BM % 32 == 0 && LOADS * STAGES < 64, "whole copy instructions, and a count that fits the counter");
+    constexpr int LOADS = ROWS * CH / (64 * WAVES);     // copies a lane and stage (KG slices)
+    static_assert(ROWS * CH % (64 * WAVES) == 0 && BM % 32 == 0 && LOADS * STAGES < 64, "whole copy instructions, and a count that fits the counter");
     extern __shared__ __align__(16) float4 lds[];       // [STAGES][KG][ROWS][CH]
-    const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3, set = wave8 >> 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 % WAVES, set = wave8 / WAVES;
     const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN);
     const int tile = (int)(blockIdx.x & 7) * ((tiles + 7) >> 3) + (int)(blockIdx.x >> 3);
     if (tile >= tiles) return;
     const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * BN;
-    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+    const int wm = wave / GN * (BM / GM), wn = wave % GN * (BN / GN);
     auto turn = [](int r) { return (r >> 1) & (CH - 1); };
-    // this lane's pieces of a slice: 8 rows a copy instruction
+    const int n_stages = (K + KG * FBK - 1) / (KG * FBK);
+    // this lane's pieces of a slice: 8 rows a copy instruction, the first of a stage activations and weights by turns of ROWS / 8
     const float* src[LOADS];
     int col[LOADS];
+    uint32_t off[LOADS];
     const float* zero_src = reinterpret_cast<const float*>(xr_zero_chunk);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-        const int all = (i * 4 * KG + wave8) * 8 + (lane >> 3), r = all % ROWS;
+        const int all = (i * WAVES * KG + wave8) * 8 + (lane >> 3), r = all % ROWS;
         col[i] = ((lane & (CH - 1)) ^ turn(r)) * 4 + all / ROWS * FBK;
         const int m = m0 + r, n = n0 + r - BM;
-        src[i] = r < BM ? (m < M ? a + (size_t)m * lda + col[i] : nullptr) : (n < N ? w + (size_t)n * K + col[i] : nullptr);
+        if constexpr (WHOLE)
+            off[i] = r < BM ? (uint32_t)((m < M ? r : M - 1 - m0) * (size_t)lda + col[i]) * 4u : (uint32_t)((n < N ? r - BM : N - 1 - n0) * (size_t)K + col[i]) * 4u;
+        else
+            src[i] = r < BM ? (m < M ? a + (size_t)m * lda + col[i] : nullptr) : (n < N ? w + (size_t)n * K + col[i] : nullptr);
     }
+    const float* a_tile = a + (size_t)m0 * lda;
+    const float* w_tile = w + (size_t)n0 * K;
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave8 * 64 * 16));
-    auto copy = [&](int stage) {                        // (pieces that do not exist are zeros)
+    auto copy = [&](int stage) {
         const uint32_t dst = lds_wave + (uint32_t)(stage % STAGES * KG * ROWS * CH * 16);
+        if constexpr (WHOLE) {
+            const int s = stage < n_stages ? stage : n_stages - 1;       // (past the end the last stage once more: as many copies on their way)
+            const float* const a_now = a_tile + (size_t)s * KG * FBK;
+            const float* const w_now = w_tile + (size_t)s * KG * FBK;
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i)
-            lds_dma16(src[i] && stage * KG * FBK + col[i] < K ? src[i] + (size_t)stage * KG * FBK : zero_src, dst + i * KG * 256 * 16);
+            for (int i = 0; i < LOADS; ++i) {
+                const bool act = (i * WAVES * KG + wave8) * 8 % ROWS < BM;
+                lds_dma16_base(act ? a_now : w_now, off[i], dst + i * KG * WAVES * 64 * 16);
+            }
+        } else {                                                         // (pieces that do not exist are zeros)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                lds_dma16(src[i] && stage * KG * FBK + col[i] < K ? src[i] + (size_t)stage * KG * FBK : zero_src, dst + i * KG * WAVES * 64 * 16);
+        }
     };
     f32x16 acc[TM][TN], tot[TM][TN], lost[TM][TN];
 #pragma unroll
@@ -151,7 +177,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, 
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = tot[i][j][e] = lost[i][j][e] = 0.f;
+            for (int e = 0; e < 16; ++e) tot[i][j][e] = lost[i][j][e] = 0.f;
     auto fold = [&]() {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -161,68 +187,96 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, 
                 for (int e = 0; e < 16; ++e) {
                     float x = acc[i][j][e], t = tot[i][j][e], l = lost[i][j][e];
                     fold_run(x, t, l);
-                    acc[i][j][e] = x; tot[i][j][e] = t; lost[i][j][e] = l;
+                    tot[i][j][e] = t; lost[i][j][e] = l;
                 }
     };
     const int row = lane & 31, half = (lane >> 5) * 4;
-    const int n_stages = (K + KG * FBK - 1) / (KG * FBK);
 #pragma unroll
     for (int st = 0; st < STAGES - 1; ++st) copy(st);
-    for (int stage = 0; stage < n_stages; ++stage) {
-        wait_vmcnt<LOADS * (STAGES - 2)>();             // this wave's share of the stage has landed
-        __builtin_amdgcn_s_barrier();                   // every wave's has, and nobody reads the stage before any more
-        copy(stage + STAGES - 1);
-        const float4* As = lds + (stage % STAGES * KG + set) * ROWS * CH;
+    auto products = [&](const float4* As, auto first) {
         const float4* Ws = As + BM * CH;
+        // (the operands of the next four steps are read while these are multiplied, into a second set of registers: the compiler keeps
+        // one set, and a read then waits for the products before it and they for the read)
+        float4 fa[2][TM], fw[2][TN];
+        auto read = [&](int kk, int set_) {
+            const int c = kk + (lane >> 5);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) { const int r = wm + 32 * i + row; fa[set_][i] = As[r * CH + (c ^ turn(r))]; }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) { const int r = wn + 32 * j + row; fw[set_][j] = Ws[r * CH + (c ^ turn(r))]; }
+        };
+        read(0, 0);
 #pragma unroll
         for (int kk = 0; kk < CH; kk += 2) {
-            const int c = kk + (lane >> 5);
-            float4 fa[TM], fw[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) { const int r = wm + 32 * i + row; fa[i] = As[r * CH + (c ^ turn(r))]; }
-#pragma unroll
-            for (int j = 0; j < TN; ++j) { const int r = wn + 32 * j + row; fw[j] = Ws[r * CH + (c ^ turn(r))]; }
+            const int now = (kk >> 1) & 1;
+            if (kk + 2 < CH) read(kk + 2, now ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((&fa[i].x)[s], (&fw[j].x)[s], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < TN; ++j) {
+                        const bool begins = decltype(first)::value && kk == 0 && s == 0;
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32((&fa[now][i].x)[s], (&fw[now][j].x)[s], begins ? f32x16{} : acc[i][j], 0, 0, 0);
+                    }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if ((stage + 1) % (RBK * RB_FOLD / FBK) == 0) fold();
+    };
+    constexpr int RUN = RBK * RB_FOLD / FBK;            // stages of a run
+    for (int run = 0; run < n_stages; run += RUN) {
+#pragma unroll
+        for (int u = 0; u < RUN; ++u) {
+            const int stage = run + u;
+            if (u > 0 && stage >= n_stages) break;
+            wait_vmcnt<LOADS * (STAGES - 2)>();         // this wave's share of the stage has landed
+            __builtin_amdgcn_s_barrier();               // every wave's has, and nobody reads the stage before any more
+            copy(stage + STAGES - 1);
+            const float4* As = lds + (stage % STAGES * KG + set) * ROWS * CH;
+            if (u == 0) products(As, std::true_type{});
+            else products(As, std::false_type{});
+        }
+        fold();
     }
-    wait_vmcnt<0>();                                    // the trailing copies of zeros
-    fold();
-    if constexpr (KG == 2) {                            // the second set's sums, and what they lack
-        static_assert(2 * TM * TN * 4 * 1024 <= STAGES * KG * ROWS * FBK, "room for both");
+    wait_vmcnt<0>();                                    // the trailing copies
+    if constexpr (KG > 1) {                             // the other sets' sums, and what they lack
+        static_assert(2 * TM * TN * WAVES * (KG - 1) * 1024 <= STAGES * KG * ROWS * FBK, "room for all of them");
         __syncthreads();
-        float* other = reinterpret_cast<float*>(lds) + wave * 2 * TM * TN * 1024 + lane;
-        if (set == 1)
+        float* const theirs = reinterpret_cast<float*>(lds) + wave * 2 * TM * TN * 1024 + lane;
+        constexpr int SET = WAVES * 2 * TM * TN * 1024;
+        if (set > 0)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
-                        other[((i * TN + j) * 32 + e) * 64] = tot[i][j][e];
-                        other[((i * TN + j) * 32 + 16 + e) * 64] = lost[i][j][e];
+                        theirs[(set - 1) * SET + ((i * TN + j) * 32 + e) * 64] = tot[i][j][e];
+                        theirs[(set - 1) * SET + ((i * TN + j) * 32 + 16 + e) * 64] = lost[i][j][e];
                     }
         __syncthreads();
-        if (set == 1) return;
+        if (set > 0) return;
+        // The sets' sums one after another, what each addition loses (exactly: Knuth's two-sum), and what all of them lack,
+        // rounded once (an infinite sum's loss is no number: the bounds make it one, as in fold_run).  One more run of the
+        // first set instead rounds another's sum on the way: 17 x 2048 x 14336 of one sign 0.56 units of 2^-24 off, 0.42 so.
+#pragma unroll 1
+        for (int o = 0; o < KG - 1; ++o)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const float x = tot[i][j][e], y = theirs[o * SET + ((i * TN + j) * 32 + e) * 64], t = x + y, z = t - x;
+                        lost[i][j][e] -= ((x - (t - z)) + (y - z)) - theirs[o * SET + ((i * TN + j) * 32 + 16 + e) * 64];
+                        tot[i][j][e] = t;
+                    }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    // the two sums, what that addition loses (exactly: Knuth's two-sum), and what both lack, rounded once (an
-                    // infinite sum's loss is no number: the bounds make it one, as in fold_run).  One more run of the first
-                    // set instead rounds the second's sum on the way: 17 x 2048 x 14336 of one sign 0.56 units of 2^-24 off, 0.42 so.
-                    const float x = tot[i][j][e], y = other[((i * TN + j) * 32 + e) * 64], t = x + y, z = t - x;
-                    const float lacks = ((x - (t - z)) + (y - z)) - (lost[i][j][e] + other[((i * TN + j) * 32 + 16 + e) * 64]);
-                    tot[i][j][e] = t + __builtin_amdgcn_fmed3f(lacks, -1e32f, 1e32f);
-                }
+                for (int e = 0; e < 16; ++e) tot[i][j][e] += __builtin_amdgcn_fmed3f(-lost[i][j][e], -1e32f, 1e32f);
     }
     // a lane has column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a tile
 #pragma unroll
@@ -245,12 +299,13 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_f32(TO* __restrict__ out, 
     }
 }
 
-template <int BM, int BN, int STAGES, int KG>
+template <int GM, int GN, int BM, int BN, int STAGES, int KG>
 static int launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
                            int out_dtype, int accumulate, hipStream_t stream) {
     const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     XR_REQUIRE(tiles < (1ll << 28), "gemm: %lld tiles", tiles);
     const unsigned blocks = 8 * (unsigned)((tiles + 7) / 8);
+    const bool whole = K % (KG * FBK) == 0 && (size_t)BM * lda < (1u << 30) && (size_t)BN * K < (1u << 30);
     constexpr int smem = STAGES * KG * (BM + BN) * FBK * 4;
     auto run = [&](auto kernel, auto* to) {
         if (smem > 65536) {
@@ -258,12 +313,12 @@ static int launch_gemm_f32(void* out, const float* a, const float* w, const floa
             if (e != hipSuccess) (void)hipGetLastError();
             XR_REQUIRE(e == hipSuccess, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
         }
-        kernel<<<blocks, 256 * KG, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
+        kernel<<<blocks, 64 * GM * GN * KG, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
         return XR_OK;
     };
-    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, BM, BN, STAGES, KG>, (bf16_t*)out);
-    if (accumulate) return run(k_gemm_f32<float, true, BM, BN, STAGES, KG>, (float*)out);
-    return run(k_gemm_f32<float, false, BM, BN, STAGES, KG>, (float*)out);
+    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, GM, GN, BM, BN, STAGES, KG, false>, (bf16_t*)out);
+    if (accumulate) return whole ? run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, true>, (float*)out) : run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, false>, (float*)out);
+    return whole ? run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, true>, (float*)out) : run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, false>, (float*)out);
 }
 
 // Up to 16 rows of 32-bit operands (decoded tokens): the product is bound by how fast the weights
@@ -378,6 +433,15 @@ static void launch_gemv_ref(void* out, const float* a, const float* w, const flo
     else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
 }
 
+// microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves (all sets of them), as the model in xr_gemm_ref counts them
+static double f32_tile_us(int M, int N, int K, int bm, int bn, int waves, double rate) {
+    const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn), most = (double)(((long long)tiles + 255) / 256);
+    const double mean = tiles / 256 > 1.0 ? tiles / 256 : 1.0, simd = most * waves / 4.0;
+    const double products = (0.74 * most + 0.26 * mean) * (bm * bn / 1024) * K * 4.4e-3 * rate * (simd + 0.2125) / simd;
+    const double weights = (double)N * K * 4 / 5.5e6;
+    return products > weights ? products : weights;
+}
+
 // accumulate != 0: out (float) += product.
 extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float* bias, int M, int N, int K,
                            int lda, int ldo, int in_dtype, int out_dtype, int accumulate, hipStream_t stream) {
@@ -390,14 +454,22 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
         const float* af = (const float*)a;
         const float* wf = (const float*)w;
         if (M > 16) {
-            // 64 x 128 tiles read three quarters of what 64 x 64 ones read from L2, but two of their workgroups fill a compute
-            // unit: they are taken where there are at least that many (larger tiles with their three sums a value spill)
-            const long long tiles = (long long)((M + 63) / 64) * ((N + 127) / 128);
-            // (with no more 64 x 64 tiles than compute units, eight waves a tile: 401 x 2048 x 8192 195 us with four, 171 with eight)
-            const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
-            const int rc = tiles >= 512 ? launch_gemm_f32<64, 128, 3, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                         : small > 256  ? launch_gemm_f32<64, 64, 4, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                                        : launch_gemm_f32<64, 64, 3, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            // The tile that should take the least time: a compute unit's tiles (the fullest one's, and on average) do their products at
+            // a rate that grows with its waves (w of them a SIMD: w / (w + 0.21)).  Fitted to 1,000 timed launches (the products of the 1B and
+            // the 8B shape's layers, 17 to 2,048 rows, nine tiles): 2.6% above the best of the nine on average.  Left out: 64 x 64 with
+            // one or four sets, 32 x 64 with four, 32 x 128 with two (0.1 to 0.9% together), 32 x 32 with eight (its registers spill).
+            // 401 x 16384 x 2048 343 us -> 234, 401 x 2048 x 8192 187 -> 142, 401 x 3072 x 2048 93 -> 57, 64 x 2048 x 8192 163 -> 60,
+            // 2048 x 16384 x 2048 1,302 -> 1,051, 401 x 128256 x 2048 2,010 -> 1,665.
+            const double tile_us[4] = {f32_tile_us(M, N, K, 32, 128, 4, 0.914), f32_tile_us(M, N, K, 64, 64, 8, 0.898),
+                                       f32_tile_us(M, N, K, 32, 64, 4, 0.987), f32_tile_us(M, N, K, 32, 32, 4, 1.190)};
+            // (up to four runs of columns are no work for sets of waves: one set, and sums that are the same for any number of rows)
+            int best = 0;
+            for (int i = 1; i < 4 && K > 4 * RBK * RB_FOLD; ++i)
+                if (tile_us[i] < tile_us[best]) best = i;
+            const int rc = best == 0   ? launch_gemm_f32<1, 4, 32, 128, 2, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                           : best == 1 ? launch_gemm_f32<2, 2, 64, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                           : best == 2 ? launch_gemm_f32<1, 2, 32, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                                       : launch_gemm_f32<1, 1, 32, 32, 2, 4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
             if (rc != XR_OK) return rc;
             XR_CHECK_LAUNCH("gemm_f32");
             return XR_OK;
