@@ -58,13 +58,7 @@ class Sampler:
             for r, s in enumerate(states):
                 win[r, :] = s.recent
         dev = host.to(self.device, non_blocking=True)
-        temp, top_p, min_p, penalty, draw = dev[:nf].view(torch.float32).view(5, W).unbind(0)
         if all(greedy):
-            out = self.ops.sample(logits, temp, draw)
-        else:
-            top_k, n_recent = dev[nf:nf + 2 * W].view(2, W).unbind(0)
-            out = self.ops.sample(
-                logits, temp, draw, top_k=top_k, top_p=top_p, min_p=min_p, repeat_penalty=penalty,
-                recent=dev[nf + 2 * W:].view(W, RECENT_WINDOW) if need_window else None,
-                n_recent=n_recent if need_window else None, exempt=self.exempt)
-        return out
+            temp, _, _, _, draw = dev[:nf].view(torch.float32).view(5, W).unbind(0)
+            return self.ops.sample(logits, temp, draw)
+        return self.ops.sample_packed(logits, dev, RECENT_WINDOW if need_window else 0, exempt=self.exempt)
