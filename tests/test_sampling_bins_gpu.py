@@ -137,3 +137,25 @@ def test_penalty_of_a_window_with_repeats():
     ops.sample(logits, f32(np.ones(W)), f32(np.full(W, 0.5)), top_k=i32(np.zeros(W)), top_p=f32(np.ones(W)), min_p=f32(np.zeros(W)),
                repeat_penalty=f32(rp), recent=i32(recent), n_recent=i32(n), exempt=i32(exempt))
     assert np.array_equal(logits.cpu().numpy(), want)
+
+
+# candidates of the bin that a cut gathers: either side of what is sorted by counting (64, 128, 256 and 512 keys) and of one key alone
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 128, 129, 257, 511, 512, 513, 1000])
+def test_pick_within_a_bin_of_so_many(n):
+    """One candidate far above the others, which lie in a bin or two: n in the bin that is gathered, in any order of ids."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    rng = np.random.default_rng(n)
+    V, rows, opts = 8192, [], []
+    for i in range(12):
+        row = np.full(V, -np.inf, dtype=np.float32)
+        at = rng.permutation(V)[:n + 2]
+        row[at[0]], row[at[1]] = 0.5, -20.0                     # (the row's span: bins of 0.01)
+        row[at[2:]] = -0.004 - 0.004 * rng.random(n)            # (distances 0.504 to 0.508 of z: one bin)
+        rows.append(row)
+        opts.append((1.0, float(rng.integers(0, 1 << 24)) / (1 << 24), 0, float(np.float32(rng.choice([0.4, 0.7, 0.95, 1.0]))), 0.0))
+    f = lambda i: torch.tensor([o[i] for o in opts], dtype=torch.float32, device=dev)
+    top_k = torch.zeros((len(opts),), dtype=torch.int32, device=dev)
+    got = ops.sample(torch.tensor(np.stack(rows), device=dev), f(0), f(1), top_k=top_k, top_p=f(3), min_p=f(4)).cpu().tolist()
+    assert got == [pick(r, *o) for r, o in zip(rows, opts)]

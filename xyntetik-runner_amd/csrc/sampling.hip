@@ -22,7 +22,7 @@
 // each 50 us, so a row's histogram is shared out to up to 8 workgroups where the caller brings room for their
 // partial counts; the cuts are a chain of short steps that one workgroup a row walks.
 // Where every cut was a radix selection (22 passes over the row for top-p) 64 rows of 128,256 logits
-// took 1,150 us; now 57 in three kernels (6 + 17 + 34).
+// took 1,150 us; now 53 in three kernels (6 + 17 + 30; 34 with bins of some hundred candidates sorted by a network).
 #include "common.h"
 #include "no_alloc.h"
 
@@ -32,6 +32,7 @@
 #define SM_BINS 2048            // ranges of z a row's candidates are counted in
 #define SM_SPAN 28.f            // below z_max - 28 a candidate's mass is 0 (exp(-28) < 2^-40)
 #define SM_LIST 2048            // candidates of a cut's bin that are sorted in LDS
+#define SM_RANKED 512           // and up to so many by counting the keys below each
 #define ROW_SPLITS 32           // workgroups that look for a row's largest and smallest logit
 
 typedef unsigned long long u64;
@@ -392,6 +393,26 @@ __device__ __forceinline__ bool gather(const float* row, int V, float temp, cons
     __syncthreads();
     const int n = list.n;
     if (n > SM_LIST) return false;
+    if (n <= SM_RANKED) {
+        // few: every key's place is the number of keys below it (no two are equal), counted by as many threads as there are for a key,
+        // each over its share (a pair's step of the network below, with its barrier, costs 16 waves as much as 30 comparisons: 256 keys
+        // take it 36 steps)
+        unsigned* const place = reinterpret_cast<unsigned*>(list.sum);
+        int keys = 64;
+        while (keys < n) keys <<= 1;
+        const int t = threadIdx.x & (keys - 1), share = threadIdx.x / keys, shares = SM_THREADS / keys;
+        const int per = (n + shares - 1) / shares, from = share * per, to = from + per < n ? from + per : n;
+        const u64 key = list.key[t < n ? t : 0];
+        if (threadIdx.x < keys) place[threadIdx.x] = 0;
+        __syncthreads();
+        unsigned below_it = 0;
+        for (int j = from; j < to; ++j) below_it += list.key[j] < key ? 1u : 0u;
+        if (t < n) atomicAdd(&place[t], below_it);
+        __syncthreads();
+        if (share == 0 && t < n) list.key[place[t]] = key;
+        __syncthreads();
+        return true;
+    }
     int m = 2;
     while (m < n) m <<= 1;
     for (int i = n + threadIdx.x; i < m; i += SM_THREADS) list.key[i] = ~0ull;
