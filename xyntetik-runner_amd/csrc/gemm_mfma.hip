@@ -1603,7 +1603,13 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         return workspace ? s : 1;
     };
     if (variant == 0) {
-        if (M <= 16) {
+        // (9 to 16 rows of a product wide enough to fill the chip with tiles of 128 weight rows and K whole: the skinny kernel reads its
+        // rows from L2 for every 16 weight rows, as many bytes as the weights are.  21,504 x 4,096 at 16 rows 40 us, in tiles 30; 128,256 x
+        // 4,096 216 and 193.  Decode of 9 and 16 requests: Suripel of width 4,096 1,041 us -> 963 and 1,059 -> 980, the others' heads 1%.
+        // At 8 rows the two are even.)
+        const bool wide = M > 8 && !norm && !rope && w_packed && (N + (sw ? 63 : 127)) / (sw ? 64 : 128) >= 160 &&
+                          takes_written_order(g, 1, K, 64, 128, 4, 64);
+        if (M <= 16 && !wide) {
             variant = 1;
         } else if (M <= 64) {
             variant = 31;
