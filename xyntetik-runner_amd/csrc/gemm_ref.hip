@@ -353,14 +353,32 @@ __device__ inline void tree_sums(float (&v)[N], int lane, int& mine) {
     for (; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o, 64);
 }
 
-template <int MT, int COLS, typename TO, bool ACC>
+// NORM: the rows are an RMS norm's input, norm_w its weight: their columns are multiplied by the weight on the way, a wave adds up
+// its rows' squares beside its products and scales the sums by 1 / sqrt(mean + eps).  GATED: of the COLS weight rows half are gate rows and
+// half up rows (N of each, the up rows behind the gate rows), whose sums meet 32 lanes apart, and act(gate) * up is what is stored.
+// (Steps of a few rows on a small model are a chain of launches: with both a layer of the decode step has 6 kernels of 9; a step of
+// 3 requests on 2 layers of width 64 has 18 of 23, a replay of 17 such steps takes 2,284 us for 2,408.)
+struct GemvExtra {
+    const float* norm_w;
+    float inv_width, eps;
+    int act;
+    float act_param;
+};
+
+template <int MT, int COLS, typename TO, bool ACC, bool NORM = false, bool GATED = false>
 __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const float* __restrict__ a,
                                                    const float* __restrict__ w, const float* __restrict__ bias,
-                                                   int M, int N, int K, int lda, int ldo) {
+                                                   int M, int N, int K, int lda, int ldo, GemvExtra x) {
+    constexpr int OUT = GATED ? COLS / 2 : COLS;        // outputs of a wave
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0 = (blockIdx.x * 4 + wave) * COLS;
+    const int n0 = (blockIdx.x * 4 + wave) * OUT;
     if (n0 >= N) return;
-    float acc[COLS][MT];
+    // the c-th weight row, and the output it belongs to
+    auto out_of = [&](int c) { return n0 + (GATED ? c % OUT : c); };
+    auto row_of = [&](int c) { return out_of(c) + (GATED && c >= OUT ? N : 0); };
+    float acc[COLS][MT], sq[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) sq[m] = 0.f;
 #pragma unroll
     for (int c = 0; c < COLS; ++c)
 #pragma unroll
@@ -370,10 +388,17 @@ __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const fl
 #pragma unroll
         for (int m = 0; m < MT; ++m)
             av[m] = m < M ? *reinterpret_cast<const float4*>(a + (size_t)m * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (NORM) {
+            const float4 g = *reinterpret_cast<const float4*>(x.norm_w + k);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                sq[m] += av[m].x * av[m].x + av[m].y * av[m].y + av[m].z * av[m].z + av[m].w * av[m].w;
+                av[m] = make_float4(av[m].x * g.x, av[m].y * g.y, av[m].z * g.z, av[m].w * g.w);
+            }
+        }
 #pragma unroll
         for (int c = 0; c < COLS; ++c) {
-            const int n = n0 + c;
-            const float4 wv = n < N ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 wv = out_of(c) < N ? *reinterpret_cast<const float4*>(w + (size_t)row_of(c) * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
                 float t = acc[c][m];
@@ -385,8 +410,14 @@ __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const fl
             }
         }
     }
+    float scale[MT];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) scale[m] = 1.0f / sqrtf(wave_sum(sq[m]) * x.inv_width + x.eps);
+    }
     // 64 sums at a time (a lane ends with one), or all of them where they are fewer
     constexpr int ALL = COLS * MT, GROUP = ALL < 64 ? ALL : 64;
+    static_assert(!GATED || (ALL <= 64 && ALL >= 2), "a gate's sum and its up row's are half the sums apart: the tree's first step, 32 lanes");
 #pragma unroll
     for (int g0 = 0; g0 < ALL; g0 += GROUP) {
         float v[GROUP];
@@ -394,10 +425,20 @@ __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const fl
         for (int i = 0; i < GROUP; ++i) v[i] = acc[(g0 + i) / MT][(g0 + i) % MT];
         int mine;
         tree_sums<GROUP>(v, lane, mine);
-        const int n = n0 + (g0 + mine) / MT, m = (g0 + mine) % MT;
-        if ((lane & (64 / GROUP - 1)) == 0 && m < M && n < N) {
-            float s = v[0];
-            if (bias) s += bias[n];
+        const int c = (g0 + mine) / MT, n = out_of(c), m = (g0 + mine) % MT;
+        float s = v[0];
+        if constexpr (NORM) {
+            float f = scale[0];
+#pragma unroll
+            for (int i = 1; i < MT; ++i) f = m == i ? scale[i] : f;
+            s *= f;
+        }
+        if (bias && n < N) s += bias[row_of(c)];
+        if constexpr (GATED) {
+            const float up = __shfl_xor(s, 32, 64);
+            s = gate_value<false>(x.act, x.act_param, s, up);
+        }
+        if ((lane & (64 / GROUP - 1)) == 0 && m < M && n < N && !(GATED && c >= OUT)) {
             const size_t at = (size_t)m * ldo + n;
             if (ACC) s += ld<TO>(out, at);
             st<TO>(out, at, s);
@@ -409,9 +450,9 @@ template <int MT, int COLS>
 static void launch_gemv_cols(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
                              int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
     const unsigned blocks = (unsigned)((N + 4 * COLS - 1) / (4 * COLS));
-    if (out_dtype == XR_BF16) k_gemv_ref<MT, COLS, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo);
-    else if (accumulate) k_gemv_ref<MT, COLS, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
-    else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo);
+    if (out_dtype == XR_BF16) k_gemv_ref<MT, COLS, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
+    else if (accumulate) k_gemv_ref<MT, COLS, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
+    else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
 }
 
 // Weight rows a wave: more share the reads of `a` and cost fewer sums, fewer spread over more compute units.  One row: 2.  More
@@ -490,5 +531,39 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
     else { xr_set_error("gemm: bad dtypes in=%d out=%d", in_dtype, out_dtype); return XR_BAD_ARG; }
 #undef G
     XR_CHECK_LAUNCH("gemm_ref");
+    return XR_OK;
+}
+
+// Up to XR_GEMV_EXTRA_ROWS 32-bit rows through a product that norms its rows itself and / or gates its result: out [M, N] is
+// norm(a) w^T (+ bias), or with `gated` act(gate) * up of the 2 N weight rows (gate rows, then up rows).  norm_w: the RMS norm's weight [K], or
+// null (the rows are taken as they are).  `a` must not be what is written.
+#define XR_GEMV_EXTRA_ROWS 4
+extern "C" int xr_gemv_extra_rows() { return XR_GEMV_EXTRA_ROWS; }
+extern "C" int xr_gemv_extra(float* out, const float* a, const float* w, const float* bias, const float* norm_w, float eps, int gated, int act,
+                             float act_param, int M, int N, int K, int lda, int ldo, hipStream_t stream) {
+    XR_REQUIRE(M >= 0 && M <= XR_GEMV_EXTRA_ROWS && N > 0 && K > 0, "gemv: bad sizes M=%d (at most %d) N=%d K=%d", M, XR_GEMV_EXTRA_ROWS, N, K);
+    XR_REQUIRE(lda >= K && ldo >= N, "gemv: row strides lda=%d ldo=%d are shorter than K=%d N=%d", lda, ldo, K, N);
+    XR_REQUIRE(K % 4 == 0 && lda % 4 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)norm_w) % 16) == 0, "gemv: operands that are not 16-byte aligned rows of a multiple of 4");
+    XR_REQUIRE(norm_w || gated, "gemv: a plain product is xr_gemm_ref's");
+    XR_REQUIRE(!gated || (act >= 0 && act < XR_ACT_COUNT), "gemv: unknown activation code %d", act);
+    if (M == 0) return XR_OK;
+    const GemvExtra x{norm_w, 1.0f / (float)K, eps, act, act_param};
+    auto run = [&](auto rows) {
+        constexpr int MT = decltype(rows)::value;
+        // (two weight rows a wave, or two outputs: these are for few rows and small matrices; larger ones by the same lines as plain products)
+        const bool wide = gemv_cols<MT>(gated ? 2 * N : N, K) > 2;
+#define XV(COLS, NORM, GATED)                                                                                                   \
+    {                                                                                                                           \
+        constexpr int per = 4 * ((GATED) ? (COLS) / 2 : (COLS));                                                                \
+        k_gemv_ref<MT, COLS, float, false, NORM, GATED><<<(unsigned)((N + per - 1) / per), 256, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, x); \
+    }
+        if (gated && norm_w) { if (wide) XV(8, true, true) else XV(2, true, true) }
+        else if (gated) { if (wide) XV(8, false, true) else XV(2, false, true) }
+        else { if (wide) XV(4, true, false) else XV(2, true, false) }
+#undef XV
+    };
+    if (M == 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 4>{});
+    XR_CHECK_LAUNCH("gemv_extra");
     return XR_OK;
 }

@@ -64,6 +64,8 @@ _PROTOS = {
     "xr_fill_rows_many": [_p, _p, _i, _sz, _p, _i, _u32, _p],
     "xr_convert": [_p, _p, _sz, _i, _i, _p],
     "xr_stream_read": [_p, _sz, _p, _i, _p],
+    "xr_gemv_extra": [_p, _p, _p, _p, _p, _f, _i, _i, _f, _i, _i, _i, _i, _i, _p],
+    "xr_gemv_extra_rows": [],
     "xr_gemm_ref": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_gemm_bf16": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p, _p, _p],
     "xr_pack_weight": [_p, _p, _i, _i, _p],
@@ -178,6 +180,27 @@ class UnscaledRows:
         return self.data.device
 
 
+class UnnormedRows:
+    """A few 32-bit rows of the residual stream that a product norms itself: ``data [M, E]`` the rows as they are (not a copy),
+    ``weight [E]`` and ``eps`` the RMSNorm's.  ``Ops.linear`` and ``Ops.linear_gated`` take this in place of the normed rows, before
+    the stream is written again.  Made by ``Ops.linear_add_rmsnorm``."""
+
+    def __init__(self, data: torch.Tensor, weight: torch.Tensor, eps: float):
+        self.data, self.weight, self.eps = data, weight, eps
+
+    @property
+    def shape(self):
+        return self.data.shape
+
+    @property
+    def dtype(self):
+        return self.data.dtype
+
+    @property
+    def device(self):
+        return self.data.device
+
+
 class _GemmNorm(C.Structure):
     """XrGemmNorm of the library."""
     _fields_ = [("ss_in", _p), ("n_ss", _i), ("ss_inv_width", _f), ("ss_eps", _f), ("norm_w", _p),
@@ -239,6 +262,7 @@ class Ops:
         self.fuse_rope = True       # False: project_rope_kv_write always runs two kernels
         self.ROPE_TILE_ROWS = int(lib.dll.xr_rope_tile_rows())
         self.FINISH_ROWS = self.ROPE_TILE_ROWS - 1
+        self.EXTRA_ROWS = int(lib.dll.xr_gemv_extra_rows())      # 32-bit rows that a product may norm, and whose result it may gate
 
     # -- checks -----------------------------------------------------------------
     @staticmethod
@@ -409,6 +433,10 @@ class Ops:
         """
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w
+        if isinstance(a, UnnormedRows):
+            if out is None and activation is None and out_dtype in (None, torch.float32) and _then is None and self._extra_ok(a.data, w, bias):
+                return self._gemv_extra(a.data, w, bias, w.shape[0], norm=a)
+            a = self.rmsnorm(a.data, a.weight, a.eps, torch.float32)
         norm, a = self._norm_before(a, _then)
         self._dev(a, wt, bias, out)
         if a.dim() != 2 or len(w.shape) != 2 or a.shape[1] != w.shape[1]:
@@ -450,6 +478,22 @@ class Ops:
             self.act_rows_(out, activation)
         return out
 
+    def _extra_ok(self, a: torch.Tensor, w, bias: Optional[torch.Tensor]) -> bool:
+        """Whether a product of 32-bit rows may norm them or gate its result itself: few rows, 16-byte aligned."""
+        return (self.fold_norms and isinstance(w, torch.Tensor) and a.dtype == w.dtype == torch.float32 and a.dim() == w.dim() == 2
+                and 0 < a.shape[0] <= self.EXTRA_ROWS and a.shape[1] == w.shape[1] and a.shape[1] % 4 == 0 and a.stride(0) % 4 == 0
+                and a.stride(1) == 1 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous()
+                and (bias is None or (bias.dtype == torch.float32 and bias.numel() == w.shape[0] and bias.is_contiguous())))
+
+    def _gemv_extra(self, a: torch.Tensor, w: torch.Tensor, bias, N: int, norm: Optional["UnnormedRows"] = None, act: Optional[int] = None,
+                    param: float = 0.0) -> torch.Tensor:
+        self._dev(a, w, bias, norm.weight if norm is not None else None)
+        out = torch.empty((a.shape[0], N), dtype=torch.float32, device=a.device)
+        self.lib.check(self.lib.xr_gemv_extra(out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), _ptr(norm.weight) if norm is not None else None,
+                                              float(norm.eps) if norm is not None else 0.0, 0 if act is None else 1, act or 0, float(param),
+                                              a.shape[0], N, a.shape[1], a.stride(0), N, _stream()))
+        return out
+
     @staticmethod
     def _norm_before(a, then: Optional[_GemmNorm]):
         """(what the library needs to know about a norm folded into this product, the rows)"""
@@ -476,7 +520,7 @@ class Ops:
         the K ranges takes whole rows and writes the finished norm.  In every other case the norm's own
         kernel runs.  A tensor comes back in both."""
         wt = w.data if isinstance(w, PackedWeight) else w
-        rows = a.data if isinstance(a, UnscaledRows) else a
+        rows = a.data if isinstance(a, (UnscaledRows, UnnormedRows)) else a
         M, N = rows.shape[0], w.shape[0]
         fits = (self.fold_norms and out_dtype == torch.bfloat16 and norm_weight is not None
                 and N % 8 == 0 and norm_weight.numel() == N and norm_weight.is_contiguous()
@@ -503,6 +547,11 @@ class Ops:
                 return UnscaledRows(xg, sumsq[:then.ss_out_rows], eps)
             return normed(residual, norm_weight, eps, out_dtype)            # the library declined
         self.linear(a, w, bias=bias, out=residual, accumulate=True)
+        # (a few 32-bit rows: what reads the result norms them itself)
+        if (defer and not centred and self.fold_norms and out_dtype == torch.float32 and 0 < M <= self.EXTRA_ROWS and norm_weight is not None
+                and norm_weight.dtype == torch.float32 and norm_weight.numel() == N and norm_weight.is_contiguous()
+                and norm_weight.data_ptr() % 16 == 0 and residual.dtype == torch.float32 and residual.shape[1] == N):
+            return UnnormedRows(residual, norm_weight, eps)
         return normed(residual, norm_weight, eps, out_dtype)
 
     def post_norm(self, x: torch.Tensor, y: torch.Tensor, alpha: float, norm_weight: torch.Tensor, eps: float,
@@ -553,6 +602,11 @@ class Ops:
         act = activation_code(activation)
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w
+        rows = a.data if isinstance(a, UnnormedRows) else a
+        if not isinstance(a, UnscaledRows) and w.shape[0] % 2 == 0 and self._extra_ok(rows, w, bias):
+            return self._gemv_extra(rows, w, bias, w.shape[0] // 2, norm=a if isinstance(a, UnnormedRows) else None, act=act, param=param)
+        if isinstance(a, UnnormedRows):
+            a = self.rmsnorm(a.data, a.weight, a.eps, torch.float32)
         norm, a = self._norm_before(a, None)
         F = w.shape[0] // 2
         if w.shape[0] % 2:
@@ -701,7 +755,7 @@ class Ops:
         product and ``rope_kv_write`` run one after the other.  ``cs_table``: a callable that returns the
         step's ``rope_table`` (asked for only where the tile kernel rotates).  ``variant``: a tile kernel
         by number instead of the library's choice (tests; from 512 rows on)."""
-        rows = h.data if isinstance(h, UnscaledRows) else h
+        rows = h.data if isinstance(h, (UnscaledRows, UnnormedRows)) else h
         wt = w.data if isinstance(w, PackedWeight) else w
         T, Q, KV = rows.shape[0], H * D, Hk * D
         if w.shape[0] != Q + 2 * KV:

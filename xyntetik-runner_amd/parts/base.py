@@ -40,7 +40,8 @@ may override ``forward_add_norm(..., residual, norm, defer)``, which adds into t
 residual stream and returns ``norm`` of the result, so that its last product can do
 both (``Ops.linear_add_rmsnorm``).  With ``defer`` the result may be an
 ``UnscaledRows`` (the rows still lack the division by their root mean square, which
-the next product applies to its own result); a caller sets ``defer`` only if the part
+the next product applies to its own result) or an ``UnnormedRows`` (a few 32-bit rows of the
+stream itself, which the next product norms); a caller sets ``defer`` only if the part
 that reads the result has ``takes_unscaled_rows`` set, which says that it hands ``h``
 to ``Ops.linear`` or ``Ops.linear_gated`` and reads nothing else of it than its
 ``shape``, ``dtype`` and ``device``.  A block with ``chained`` set takes the result of
@@ -201,7 +202,7 @@ class Mixer(Part):
     def forward(self, ctx, cache, h: torch.Tensor) -> torch.Tensor:
         raise NotImplementedError
 
-    #: True if ``h`` may be an ``UnscaledRows`` (it only goes into ``Ops.linear``)
+    #: True if ``h`` may be an ``UnscaledRows`` or an ``UnnormedRows`` (it only goes into ``Ops.linear``)
     takes_unscaled_rows = False
 
     def forward_add(self, ctx, cache, h: torch.Tensor, residual: torch.Tensor) -> None:
@@ -269,7 +270,7 @@ class FeedForward(Part):
     def forward(self, ctx, h: torch.Tensor) -> torch.Tensor:
         raise NotImplementedError
 
-    #: True if ``h`` may be an ``UnscaledRows`` (it only goes into ``Ops.linear`` or ``Ops.linear_gated``)
+    #: True if ``h`` may be an ``UnscaledRows`` or an ``UnnormedRows`` (it only goes into ``Ops.linear`` or ``Ops.linear_gated``)
     takes_unscaled_rows = False
 
     def forward_add(self, ctx, h: torch.Tensor, residual: torch.Tensor) -> None:
