@@ -503,10 +503,14 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
             // 2048 x 16384 x 2048 1,302 -> 1,051, 401 x 128256 x 2048 2,010 -> 1,665.
             const double tile_us[4] = {f32_tile_us(M, N, K, 32, 128, 4, 0.914), f32_tile_us(M, N, K, 64, 64, 8, 0.898),
                                        f32_tile_us(M, N, K, 32, 64, 4, 0.987), f32_tile_us(M, N, K, 32, 32, 4, 1.190)};
-            // (up to four runs of columns are no work for sets of waves: one set, and sums that are the same for any number of rows)
-            int best = 0;
-            for (int i = 1; i < 4 && K > 4 * RBK * RB_FOLD; ++i)
-                if (tile_us[i] < tile_us[best]) best = i;
+            // Up to 256 tiles of 64 x 64 at least two sets of waves share the columns: shorter runs, and an error that is smaller by a third
+            // where a sum is no more than a few runs (positive numbers, K 64 to 516: 1.07e-7 with two sets, 1.43e-7 with one).  Up to four
+            // runs of columns are no work for more sets, and the number of sets then depends on the number of those tiles alone.
+            const bool few = (long long)((M + 63) / 64) * ((N + 63) / 64) <= 256;
+            const bool few_runs = K <= 4 * RBK * RB_FOLD;
+            int best = few ? 1 : 0;
+            for (int i = 1; i < 4; ++i)
+                if (tile_us[i] < tile_us[best] && !(few_runs && (!few || i == 3))) best = i;
             const int rc = best == 0   ? launch_gemm_f32<1, 4, 32, 128, 2, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
                            : best == 1 ? launch_gemm_f32<2, 2, 64, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
                            : best == 2 ? launch_gemm_f32<1, 2, 32, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
