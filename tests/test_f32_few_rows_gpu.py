@@ -52,3 +52,26 @@ def test_more_rows_are_normed_by_the_norms_kernel():
         got = ops.linear_add_rmsnorm(a, w, x, wn, 1e-5, torch.float32, defer=True)
         assert isinstance(got, UnnormedRows) == (M <= ops.EXTRA_ROWS)
         assert not isinstance(ops.linear_add_rmsnorm(a, w, x, wn, 1e-5, torch.float32), UnnormedRows)      # not asked for
+
+
+# one row and the most, and outputs with 2, 4 and 8 weight rows a wave
+@pytest.mark.parametrize("M", [1, 3, 4])
+@pytest.mark.parametrize("N,K", [(64, 176), (252, 260), (16388, 256), (8192, 4096), (16384, 4096)])
+def test_deferred_rows_stay_what_they_are_when_the_stream_is_written_again(M, N, K):
+    """What comes back is a copy: a part may add to the stream between two products of the rows it was given."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import UnnormedRows, load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w, x, bias, w2 = (torch.randn(s, generator=g, device=dev) for s in ((M, K), (N, K), (M, N + 4), (N,), (96, N)))
+    x, wn = x[:, 4:], torch.rand(N, generator=g, device=dev) + 0.5               # (a stream that is part of wider rows)
+    want = x.clone()
+    ops.linear(a, w, bias=bias, out=want, accumulate=True)
+    h = ops.linear_add_rmsnorm(a, w, x, wn, 1e-5, torch.float32, bias=bias, defer=True)
+    assert isinstance(h, UnnormedRows)
+    assert torch.equal(x, want) and torch.equal(h.data, want)                    # the bits that the plain sum leaves
+    first, gated = ops.linear(h, w2), ops.linear_gated(h, w2)
+    ops.linear(a, w, out=x, accumulate=True)
+    assert not torch.equal(x, want)
+    assert torch.equal(ops.linear(h, w2), first) and torch.equal(ops.linear_gated(h, w2), gated)

@@ -358,11 +358,14 @@ __device__ inline void tree_sums(float (&v)[N], int lane, int& mine) {
 // half up rows (N of each, the up rows behind the gate rows), whose sums meet 32 lanes apart, and act(gate) * up is what is stored.
 // (Steps of a few rows on a small model are a chain of launches: with both a layer of the decode step has 6 kernels of 9; a step of
 // 3 requests on 2 layers of width 64 has 18 of 23, a replay of 17 such steps takes 2,284 us for 2,408.)
+// ACC with `copy`: the sums that are stored also go there, rows of N numbers, for a product that norms them later, when the sums
+// themselves may have been added to again.
 struct GemvExtra {
     const float* norm_w;
     float inv_width, eps;
     int act;
     float act_param;
+    float* copy;
 };
 
 template <int MT, int COLS, typename TO, bool ACC, bool NORM = false, bool GATED = false>
@@ -442,17 +445,20 @@ __global__ __launch_bounds__(256) void k_gemv_ref(TO* __restrict__ out, const fl
             const size_t at = (size_t)m * ldo + n;
             if (ACC) s += ld<TO>(out, at);
             st<TO>(out, at, s);
+            if (ACC && x.copy) x.copy[(size_t)m * N + n] = s;
         }
     }
 }
 
 template <int MT, int COLS>
 static void launch_gemv_cols(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
-                             int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
+                             int lda, int ldo, int out_dtype, int accumulate, float* copy, hipStream_t stream) {
     const unsigned blocks = (unsigned)((N + 4 * COLS - 1) / (4 * COLS));
-    if (out_dtype == XR_BF16) k_gemv_ref<MT, COLS, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
-    else if (accumulate) k_gemv_ref<MT, COLS, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
-    else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, GemvExtra{});
+    GemvExtra x{};
+    x.copy = copy;
+    if (out_dtype == XR_BF16) k_gemv_ref<MT, COLS, bf16_t, false><<<blocks, 256, 0, stream>>>((bf16_t*)out, a, w, bias, M, N, K, lda, ldo, x);
+    else if (accumulate) k_gemv_ref<MT, COLS, float, true><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, x);
+    else k_gemv_ref<MT, COLS, float, false><<<blocks, 256, 0, stream>>>((float*)out, a, w, bias, M, N, K, lda, ldo, x);
 }
 
 // Weight rows a wave: more share the reads of `a` and cost fewer sums, fewer spread over more compute units.  One row: 2.  More
@@ -467,11 +473,11 @@ static int gemv_cols(int N, int K) {
 
 template <int MT>
 static void launch_gemv_ref(void* out, const float* a, const float* w, const float* bias, int M, int N, int K,
-                            int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream) {
+                            int lda, int ldo, int out_dtype, int accumulate, hipStream_t stream, float* copy = nullptr) {
     const int cols = gemv_cols<MT>(N, K);
-    if (cols == 8) launch_gemv_cols<MT, 8>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
-    else if (cols == 4) launch_gemv_cols<MT, 4>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
-    else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+    if (cols == 8) launch_gemv_cols<MT, 8>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, copy, stream);
+    else if (cols == 4) launch_gemv_cols<MT, 4>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, copy, stream);
+    else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, copy, stream);
 }
 
 // microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves (all sets of them), as the model in xr_gemm_ref counts them
@@ -551,7 +557,7 @@ extern "C" int xr_gemv_extra(float* out, const float* a, const float* w, const f
     XR_REQUIRE(norm_w || gated, "gemv: a plain product is xr_gemm_ref's");
     XR_REQUIRE(!gated || (act >= 0 && act < XR_ACT_COUNT), "gemv: unknown activation code %d", act);
     if (M == 0) return XR_OK;
-    const GemvExtra x{norm_w, 1.0f / (float)K, eps, act, act_param};
+    const GemvExtra x{norm_w, 1.0f / (float)K, eps, act, act_param, nullptr};
     auto run = [&](auto rows) {
         constexpr int MT = decltype(rows)::value;
         // (two weight rows a wave, or two outputs: these are for few rows and small matrices; larger ones by the same lines as plain products)
@@ -569,5 +575,19 @@ extern "C" int xr_gemv_extra(float* out, const float* a, const float* w, const f
     if (M == 1) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 4>{});
     XR_CHECK_LAUNCH("gemv_extra");
+    return XR_OK;
+}
+
+// Up to XR_GEMV_EXTRA_ROWS 32-bit rows: out [M, N] += a w^T (+ bias), as xr_gemm_ref adds them, and the new rows of `out` also to
+// `copy` [M, N], which a later product norms (so that `out` may be added to before it does).
+extern "C" int xr_gemv_add_copy(float* out, float* copy, const float* a, const float* w, const float* bias, int M, int N, int K, int lda,
+                                int ldo, hipStream_t stream) {
+    XR_REQUIRE(M >= 0 && M <= XR_GEMV_EXTRA_ROWS && N > 0 && K > 0, "gemv: bad sizes M=%d (at most %d) N=%d K=%d", M, XR_GEMV_EXTRA_ROWS, N, K);
+    XR_REQUIRE(lda >= K && ldo >= N, "gemv: row strides lda=%d ldo=%d are shorter than K=%d N=%d", lda, ldo, K, N);
+    XR_REQUIRE(K % 4 == 0 && lda % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) % 16) == 0, "gemv: operands that are not 16-byte aligned rows of a multiple of 4");
+    if (M == 0) return XR_OK;
+    if (M == 1) launch_gemv_ref<1>(out, a, w, bias, M, N, K, lda, ldo, XR_F32, 1, stream, copy);
+    else launch_gemv_ref<4>(out, a, w, bias, M, N, K, lda, ldo, XR_F32, 1, stream, copy);
+    XR_CHECK_LAUNCH("gemv_add_copy");
     return XR_OK;
 }

@@ -66,6 +66,7 @@ _PROTOS = {
     "xr_stream_read": [_p, _sz, _p, _i, _p],
     "xr_gemv_extra": [_p, _p, _p, _p, _p, _f, _i, _i, _f, _i, _i, _i, _i, _i, _p],
     "xr_gemv_extra_rows": [],
+    "xr_gemv_add_copy": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p],
     "xr_gemm_ref": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_gemm_bf16": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p, _p, _p],
     "xr_pack_weight": [_p, _p, _i, _i, _p],
@@ -181,9 +182,9 @@ class UnscaledRows:
 
 
 class UnnormedRows:
-    """A few 32-bit rows of the residual stream that a product norms itself: ``data [M, E]`` the rows as they are (not a copy),
-    ``weight [E]`` and ``eps`` the RMSNorm's.  ``Ops.linear`` and ``Ops.linear_gated`` take this in place of the normed rows, before
-    the stream is written again.  Made by ``Ops.linear_add_rmsnorm``."""
+    """A few 32-bit rows that a product norms itself: ``data [M, E]`` a copy of the residual stream's rows as they are, which stays
+    what it is when the stream is written again, ``weight [E]`` and ``eps`` the RMSNorm's.  ``Ops.linear`` and ``Ops.linear_gated``
+    take this in place of the normed rows.  Made by ``Ops.linear_add_rmsnorm``."""
 
     def __init__(self, data: torch.Tensor, weight: torch.Tensor, eps: float):
         self.data, self.weight, self.eps = data, weight, eps
@@ -517,8 +518,10 @@ class Ops:
         weighted rows and their partial sums of squares, and an ``UnscaledRows`` comes back, whose
         scale the next product applies.  With more rows, where the product is split over K (always
         from 17 to 64 rows, above that when its tiles are too few for the chip), the kernel that adds up
-        the K ranges takes whole rows and writes the finished norm.  In every other case the norm's own
-        kernel runs.  A tensor comes back in both."""
+        the K ranges takes whole rows and writes the finished norm.  For at most ``EXTRA_ROWS`` 32-bit
+        rows with ``defer`` an ``UnnormedRows`` comes back: a copy of the updated rows, which the next
+        product norms.  In every other case the norm's own kernel runs.  Except where one of the two is
+        named a tensor comes back."""
         wt = w.data if isinstance(w, PackedWeight) else w
         rows = a.data if isinstance(a, (UnscaledRows, UnnormedRows)) else a
         M, N = rows.shape[0], w.shape[0]
@@ -546,12 +549,17 @@ class Ops:
             if deferred:
                 return UnscaledRows(xg, sumsq[:then.ss_out_rows], eps)
             return normed(residual, norm_weight, eps, out_dtype)            # the library declined
-        self.linear(a, w, bias=bias, out=residual, accumulate=True)
-        # (a few 32-bit rows: what reads the result norms them itself)
-        if (defer and not centred and self.fold_norms and out_dtype == torch.float32 and 0 < M <= self.EXTRA_ROWS and norm_weight is not None
+        # (a few 32-bit rows: what reads the result norms them itself, from a copy that the product's kernel leaves beside the stream)
+        if (defer and not centred and out_dtype == torch.float32 and norm_weight is not None
                 and norm_weight.dtype == torch.float32 and norm_weight.numel() == N and norm_weight.is_contiguous()
-                and norm_weight.data_ptr() % 16 == 0 and residual.dtype == torch.float32 and residual.shape[1] == N):
-            return UnnormedRows(residual, norm_weight, eps)
+                and norm_weight.data_ptr() % 16 == 0 and residual.dtype == torch.float32 and tuple(residual.shape) == (M, N)
+                and residual.stride(1) == 1 and isinstance(a, torch.Tensor) and self._extra_ok(a, w, bias)):
+            self._dev(a, w, bias, residual, norm_weight)
+            copy = torch.empty((M, N), dtype=torch.float32, device=a.device)
+            self.lib.check(self.lib.xr_gemv_add_copy(residual.data_ptr(), copy.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N,
+                                                     a.shape[1], a.stride(0), residual.stride(0), _stream()))
+            return UnnormedRows(copy, norm_weight, eps)
+        self.linear(a, w, bias=bias, out=residual, accumulate=True)
         return normed(residual, norm_weight, eps, out_dtype)
 
     def post_norm(self, x: torch.Tensor, y: torch.Tensor, alpha: float, norm_weight: torch.Tensor, eps: float,

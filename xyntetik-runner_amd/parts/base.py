@@ -40,11 +40,11 @@ may override ``forward_add_norm(..., residual, norm, defer)``, which adds into t
 residual stream and returns ``norm`` of the result, so that its last product can do
 both (``Ops.linear_add_rmsnorm``).  With ``defer`` the result may be an
 ``UnscaledRows`` (the rows still lack the division by their root mean square, which
-the next product applies to its own result) or an ``UnnormedRows`` (a few 32-bit rows of the
-stream itself, which the next product norms); a caller sets ``defer`` only if the part
+the next product applies to its own result) or an ``UnnormedRows`` (a copy of a few 32-bit
+rows of the stream, which the next product norms); a caller sets ``defer`` only if the part
 that reads the result has ``takes_unscaled_rows`` set, which says that it hands ``h``
-to ``Ops.linear`` or ``Ops.linear_gated`` and reads nothing else of it than its
-``shape``, ``dtype`` and ``device``.  A block with ``chained`` set takes the result of
+to ``Ops.linear`` or ``Ops.linear_gated``, before or after it adds to the stream, and reads
+nothing else of it than its ``shape``, ``dtype`` and ``device``.  A block with ``chained`` set takes the result of
 its first norm from the block before it and makes the next block's
 (``entry_norm()``); every default does the plain thing.
 """
