@@ -435,7 +435,7 @@ class Ops:
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w
         if isinstance(a, UnnormedRows):
-            if out is None and activation is None and out_dtype in (None, torch.float32) and _then is None and self._extra_ok(a.data, w, bias):
+            if out is None and activation is None and out_dtype in (None, torch.float32) and _then is None and self._extra_ok(a, w, bias):
                 return self._gemv_extra(a.data, w, bias, w.shape[0], norm=a)
             a = self.rmsnorm(a.data, a.weight, a.eps, torch.float32)
         norm, a = self._norm_before(a, _then)
@@ -479,8 +479,13 @@ class Ops:
             self.act_rows_(out, activation)
         return out
 
-    def _extra_ok(self, a: torch.Tensor, w, bias: Optional[torch.Tensor]) -> bool:
-        """Whether a product of 32-bit rows may norm them or gate its result itself: few rows, 16-byte aligned."""
+    def _extra_ok(self, a, w, bias: Optional[torch.Tensor]) -> bool:
+        """Whether a product of 32-bit rows may norm them (``UnnormedRows``) or gate its result itself: few rows, 16-byte aligned, and of
+        a norm one 32-bit weight a column (the norm's own kernel takes, or refuses, any other)."""
+        if isinstance(a, UnnormedRows):
+            g, a = a.weight, a.data
+            if g is None or g.dtype != torch.float32 or g.numel() != a.shape[1] or not g.is_contiguous() or g.data_ptr() % 16:
+                return False
         return (self.fold_norms and isinstance(w, torch.Tensor) and a.dtype == w.dtype == torch.float32 and a.dim() == w.dim() == 2
                 and 0 < a.shape[0] <= self.EXTRA_ROWS and a.shape[1] == w.shape[1] and a.shape[1] % 4 == 0 and a.stride(0) % 4 == 0
                 and a.stride(1) == 1 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous()
@@ -611,7 +616,7 @@ class Ops:
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w
         rows = a.data if isinstance(a, UnnormedRows) else a
-        if not isinstance(a, UnscaledRows) and w.shape[0] % 2 == 0 and self._extra_ok(rows, w, bias):
+        if not isinstance(a, UnscaledRows) and w.shape[0] % 2 == 0 and self._extra_ok(a, w, bias):
             return self._gemv_extra(rows, w, bias, w.shape[0] // 2, norm=a if isinstance(a, UnnormedRows) else None, act=act, param=param)
         if isinstance(a, UnnormedRows):
             a = self.rmsnorm(a.data, a.weight, a.eps, torch.float32)
