@@ -139,8 +139,9 @@ def test_penalty_of_a_window_with_repeats():
     assert np.array_equal(logits.cpu().numpy(), want)
 
 
-# candidates of the bin that a cut gathers: either side of what is sorted by counting (64, 128, 256 and 512 keys) and of one key alone
-@pytest.mark.parametrize("n", [1, 2, 63, 65, 128, 129, 257, 511, 512, 513, 1000])
+# candidates of the bin that a cut gathers: either side of what is sorted by counting (5 to 256 keys, 64, 128 and 256 of them at a time),
+# and of the network's sizes
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 63, 64, 65, 128, 129, 256, 257, 511, 512, 513, 1000])
 def test_pick_within_a_bin_of_so_many(n):
     """One candidate far above the others, which lie in a bin or two: n in the bin that is gathered, in any order of ids."""
     import torch

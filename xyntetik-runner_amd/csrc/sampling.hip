@@ -32,7 +32,7 @@
 #define SM_BINS 2048            // ranges of z a row's candidates are counted in
 #define SM_SPAN 28.f            // below z_max - 28 a candidate's mass is 0 (exp(-28) < 2^-40)
 #define SM_LIST 2048            // candidates of a cut's bin that are sorted in LDS
-#define SM_RANKED 512           // and up to so many by counting the keys below each
+#define SM_RANKED 256           // and up to so many by counting the keys below each
 #define ROW_SPLITS 32           // workgroups that look for a row's largest and smallest logit
 
 typedef unsigned long long u64;
@@ -393,10 +393,11 @@ __device__ __forceinline__ bool gather(const float* row, int V, float temp, cons
     __syncthreads();
     const int n = list.n;
     if (n > SM_LIST) return false;
-    if (n <= SM_RANKED) {
+    if (n > 4 && n <= SM_RANKED) {
         // few: every key's place is the number of keys below it (no two are equal), counted by as many threads as there are for a key,
         // each over its share (a pair's step of the network below, with its barrier, costs 16 waves as much as 30 comparisons: 256 keys
-        // take it 36 steps)
+        // take it 36 steps).  A pick of one row of 8,192 logits in us, by the network and counted: 4 keys 18.0 and 18.0, 8 18.6 and 18.3, 64 21.3 and
+        // 19.5, 128 22.9 and 20.9, 256 24.5 and 23.7, but 1 17.3 and 17.6, 300 26.5 and 27.8, 511 26.8 and 33.0.
         unsigned* const place = reinterpret_cast<unsigned*>(list.sum);
         int keys = 64;
         while (keys < n) keys <<= 1;
