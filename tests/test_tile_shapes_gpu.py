@@ -52,10 +52,10 @@ def test_rotation_in_the_tiles_by_name(ops, variant, H, Hk, D, rot, inter):     
 
 
 @pytest.mark.parametrize("M", [137, 192, 193, 300, 321, 640, 1300, 1524])
-@pytest.mark.parametrize("N,K", [(4096, 512), (12288, 256), (11008, 328)])
+@pytest.mark.parametrize("N,K", [(4096, 512), (12288, 256), (11008, 328), (22016, 512), (2048, 1376), (1024, 4096)])
 def test_the_chosen_tiles(ops, M, N, K):      # noqa: F811
     """What the library chooses for sizes at which the new tiles, K ranges and two launches come in; K 328 is no whole slices, so
-    that only the loops that look at columns take it."""
+    that only the loops that look at columns take it, and nor is K 1376, which is split."""
     import torch
     dev = torch.device("cuda:0")
     torch.manual_seed(M + N + K)
@@ -66,6 +66,11 @@ def test_the_chosen_tiles(ops, M, N, K):      # noqa: F811
     half = N // 2 // 32 * 32
     gate, up = want[:, :half], want[:, half:2 * half]
     assert rel(ops.linear_swiglu(a, ops.pack_weight(w[:2 * half].contiguous(), gated=True)), gate / (1 + torch.exp(-gate)) * up) < 6e-3
+
+
+@pytest.mark.parametrize("H,Hk,D,E,q_lens", [(12, 12, 64, 768, [600, 1448]), (16, 4, 128, 1000, [530, 70]), (8, 2, 80, 640, [513]), (40, 4, 128, 256, [1300])])
+def test_rotation_in_the_chosen_tiles(ops, H, Hk, D, E, q_lens):      # noqa: F811
+    check_projection_with_rotation_and_cache_write(ops, "bfloat16", H, Hk, D, D, False, 16, [0] * len(q_lens), q_lens, False, E)
 
 
 # rows of one row of tiles (9 and 16 where tiles are wide products' way); column tiles enough for workgroups to begin at every slice of K and go round (K 256: as many slices as the

@@ -1621,63 +1621,73 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // columns of the full rounds go to that tile and the rest to a second launch with a
             // smaller one (3 rounds + 1 of half-size tiles instead of 4).
             // The model, in seconds (tuning measured on an MI355X, not limits: elsewhere it costs speed only): a round of
-            // tiles takes its products' time, bm bn K x 0.36e-12 / rate (89 us for 256x256 and K = 4,096 as measured), or that of its
+            // tiles takes its products' time, bm bn K x 0.36e-12 / rate (`else_rate` where the four-wave loop does not take the product: K no
+            // whole slices), or that of its
             // weights from memory at `bytes` a second, whichever is longer; a last round that fills the chip by a share f does its products
-            // in 0.8 + 0.2 f of that (fewer tiles meet at L2, and the clock falls less); `launch` once and `round` for every round (a product that
-            // rotates its result pays for that at every round's end).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
-            // at 2.2 TB/s and costs a launch (a rotating product of up to 511 rows pays for that kernel whole, too: counted as free, it
+            // in 1 - e + e f of that, e 0.082 and rotating 0.034 (fewer tiles meet at L2, and the clock falls less); `launch` once and `round` for every round:
+            // the tile's results leave, 2.6 times as long where they are 32-bit, or are rotated (512 rows of a 512 to 22,016 product are 172 tiles of
+            // 256x256, 28.9 us, or 230 of 256x192, 19.6; 2,048 rows of a rotating 768 to 2,304 one 108 tiles of 256x192 with eight waves, 28.3 us, or of
+            // 192x192 with four, 47.5).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
+            // at 2.2 TB/s, and ranges that fill more than 0.69 of the chip gain little (137 rows of a 4,096 to 6,144 product in 192x128 tiles: four ranges, 192
+            // workgroups, 25.5 us, five, 240, 29.7) (a rotating product of up to 511 rows pays for that kernel whole, too: counted as free, it
             // sent 300 rows of a 3,072 to 5,120 product into one range, 35 us, where two take 29), and writes the norm that follows, if one was asked for: without
-            // ranges that kernel counts 12.5 us, a number of the fit and above its own time (10.8 us at 2,048 rows of 4,096, 5.2 at 137).  Fitted to 7,700 timed
-            // launches (the products of the 8B, the 7B and the 1B class's layers and Suripel's two widths, 96 to 2,048 rows, fourteen tiles,
-            // 1 to 16 ranges): the tile and ranges chosen are 2.1% slower on average than the best of all fourteen (8% in the worst tenth); the best choice
-            // among 256x256, 256x192, 256x128 and 128x128 alone is 6.5% (18%).  Of the tiles that were left out none brings 0.2% on average:
+            // ranges that kernel counts 11.3 us and its bytes at 5 TB/s.  The numbers are those with which the choices are best, not each part's own time.
+            // Fitted to 55,000 timed launches of 61 products (768 to 50,264 weight rows, 320 to 28,672 columns, 129 to 4,096
+            // rows, 1 to 16 ranges; plain, gated, added up, added up and normed; weights from memory, and from the caches where they are small):
+            // the tile and ranges chosen are 0.9% slower on average than the best of all eight tiles (1.2% for products left out of a fit); with
+            // numbers fitted to fewer and wider products, without `round`, `else_rate` and 256x192 tiles, it was 3.0%, at worst 47%.  Rotating
+            // ones: 350 products of fifteen shapes, 512 to 4,096 rows, 0.1% (0.2%); fitted to three shapes it was 6.3%, at worst 73%.
+            // Of the tiles that were left out none brings 0.2% on average:
             // 192x256, 256x192 and 128x192 with four waves, 320x192, 320x128, 96x256, and a fifth or sixth slice in flight.
-            // (Rotating products: the eight-wave kernels, but for 128x128 and the tiles that have four waves only: 600 rows of a 4,096 to 6,144 product 42 us
-            // against 53, 800 rows 72 against 98; 1,300 rows in 192x192 tiles 78 against 94.  Fitted to 33 products of three shapes, 520 to 2,048 rows.)
-            struct Cand { int variant, bm, bn, stages; double rate, launch, round, bytes; };
-            constexpr int N_CANDS = 7;
-            const Cand plain[N_CANDS] = {{14, 256, 256, 0, 1.094, 2.3e-6, 0.0, 4.6e12}, {27, 192, 192, 3, 1.056, 3.7e-6, 0.0, 5.1e12},
-                                         {12, 256, 128, 0, 0.995, 3.6e-6, 0.0, 4.2e12}, {29, 160, 256, 3, 1.006, 3.8e-6, 0.0, 5.3e12},
-                                         {16, 128, 256, 3, 0.886, 3.4e-6, 0.0, 5.8e12}, {28, 192, 128, 3, 0.827, 2.8e-6, 0.0, 4.6e12},
-                                         {17, 128, 128, 0, 0.690, 2.9e-6, 0.0, 5.5e12}};
-            const Cand turning[N_CANDS] = {{14, 256, 256, 0, 0.804, 0.0, 0.0, 5.0e12}, {26, 256, 192, 0, 0.892, 0.0, 20e-6, 5.0e12},
-                                           {12, 256, 128, 0, 0.939, 0.0, 14.5e-6, 5.0e12}, {27, 192, 192, 3, 0.923, 0.0, 20e-6, 5.0e12},
-                                           {16, 128, 256, 3, 0.925, 0.0, 20e-6, 5.0e12}, {28, 192, 128, 3, 1.061, 0.0, 20e-6, 5.0e12},
-                                           {17, 128, 128, 0, 0.849, 0.0, 12.6e-6, 5.0e12}};
+            // (Rotating products in 256x256, 256x192 and 256x128 tiles: the eight-wave kernels.)
+            // stages: slices in flight of the tile's four-wave loop (0: it has none, or it is not used here); only: it has no other
+            struct Cand { int variant, bm, bn, stages; bool only; double rate, else_rate, launch, round, bytes; };
+            const Cand plain[] = {{14, 256, 256, 2, false, 1.103, 1.100, 4.08e-6, 6.54e-6, 3.75e12}, {26, 256, 192, 0, false, 0.904, 0.904, 6.59e-6, 2.07e-6, 2.93e12},
+                                  {27, 192, 192, 3, true, 1.048, 1.048, 6.25e-6, 3.40e-6, 2.75e12}, {12, 256, 128, 3, false, 0.953, 0.835, 4.07e-6, 3.37e-6, 5.82e12},
+                                  {29, 160, 256, 3, true, 1.103, 1.103, 4.48e-6, 4.32e-6, 10.10e12}, {16, 128, 256, 3, true, 0.924, 0.924, 5.22e-6, 3.17e-6, 11.30e12},
+                                  {28, 192, 128, 3, true, 0.862, 0.862, 1.64e-6, 4.30e-6, 8.12e12}, {17, 128, 128, 4, false, 0.623, 0.449, 2.96e-6, 2.32e-6, 8.13e12}};
+            const Cand turning[] = {{14, 256, 256, 0, false, 0.929, 0.929, 3.33e-6, 16.3e-6, 6.04e12}, {26, 256, 192, 0, false, 0.743, 0.743, 1.31e-6, 2.95e-6, 12.1e12},
+                                    {27, 192, 192, 3, true, 0.934, 0.934, 0.56e-6, 20.7e-6, 15.6e12},  {12, 256, 128, 0, false, 0.715, 0.715, 1.24e-6, 2.64e-6, 2.65e12},
+                                    {29, 160, 256, 3, true, 0.927, 0.927, 1.97e-6, 15.8e-6, 5.75e12},  {16, 128, 256, 3, true, 0.849, 0.849, 1.80e-6, 18.1e-6, 7.27e12},
+                                    {28, 192, 128, 3, true, 0.855, 0.855, 2.01e-6, 14.3e-6, 9.94e12},  {17, 128, 128, 0, false, 0.661, 0.661, 3.23e-6, 6.19e-6, 8.21e12}};
+            constexpr int n_cands = sizeof(plain) / sizeof(Cand);
+            static_assert(sizeof(turning) == sizeof(plain), "as many tiles");
             const Cand* cands = rope_direct ? turning : plain;
+            const double emptier = rope_direct ? 0.034 : 0.082;
             auto width = [&](const Cand& c) { return sw ? c.bn / 2 : c.bn; };
-            // (256x192 and 192x192 tiles do not pair gate and up columns; the tiles with the written order only need whole slices)
-            auto usable = [&](const Cand& c, int ranges) {
-                if (sw && c.bn == 192) return false;
-                if (!c.stages) return true;
+            auto written = [&](const Cand& c, int ranges) {
                 int r = ranges;
                 const int columns = range_columns(K, r);
                 return takes_written_order(g, r, columns, c.bm, c.bn, c.stages, 64);
             };
+            // (256x192 and 192x192 tiles do not pair gate and up columns)
+            auto usable = [&](const Cand& c, int ranges) { return !(sw && c.bn == 192) && (!c.only || written(c, ranges)); };
             auto count = [&](const Cand& c, int cols) { return ((M + c.bm - 1) / c.bm) * ((cols + width(c) - 1) / width(c)); };
             auto seconds = [&](const Cand& c, int cols, int ranges) {
                 const int groups = count(c, cols) * ranges, rounds = (groups + 255) / 256, rows = (M + c.bm - 1) / c.bm;
-                const double k = (K + ranges - 1) / ranges, products = (double)c.bm * c.bn * k * 0.36e-12 / c.rate;
+                const bool wide_sums = !rope_direct && (!g.out_bf16 || ranges > 1 || g.raw), loop = !c.stages || c.only || written(c, ranges);
+                const double k = (K + ranges - 1) / ranges, products = (double)c.bm * c.bn * k * 0.36e-12 / (loop ? c.rate : c.else_rate);
                 const double last = (groups - (rounds - 1) * 256) / 256.0, weights = 256.0 * c.bn * k * 2 / rows / c.bytes;
-                const double products_last = products * (0.8 + 0.2 * last), weights_last = weights * last;
-                return (rounds - 1) * (products > weights ? products : weights) + (products_last > weights_last ? products_last : weights_last) +
-                       rounds * c.round + c.launch;
+                const double products_last = products * (1.0 - emptier + emptier * last), weights_last = weights * last;
+                const double crowded = ranges > 1 && last > 0.691 ? 1.0 + 0.367 * (last - 0.691) : 1.0;
+                return (rounds - 1) * (products > weights ? products : weights) + crowded * (products_last > weights_last ? products_last : weights_last) +
+                       rounds * (wide_sums ? 2.60 * c.round : c.round) + c.launch;
             };
-            auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.2e12 + 3e-6; };
-            const double norm_alone = want_whole_norm ? 12.5e-6 : 0.0;
+            auto adding = [&](int ranges) { return ((double)ranges * w_rows + 2.0 * N) * M * 4 / 2.17e12 + 0.54e-6; };
+            const double norm_alone = want_whole_norm ? 11.3e-6 + (double)M * N * 6 / 4.95e12 : 0.0;
             int best = 0, best_splits = 1, second = -1, cols_first = N;
             double t_best = 1e30;
             // Up to 128 rows are one row of 128x128 tiles: K in as many ranges as make one round of workgroups, or whole from 160
             // tiles on.  (Timed alone, five or six ranges of 32 tiles are 2-5% faster than eight; among a layer's other kernels the
             // prompt of 70 to 128 tokens is 2-3% slower with them: 1,286 us against 1,267, 1,378 against 1,336, 1,441 against 1,407.)
-            const bool one_row = M <= 128 && !rope_direct && count(cands[N_CANDS - 1], N) <= 256;
+            const bool one_row = M <= 128 && !rope_direct && count(cands[n_cands - 1], N) <= 256;
             if (one_row) {
-                const int c = count(cands[N_CANDS - 1], N);
-                best = N_CANDS - 1;
+                const int c = count(cands[n_cands - 1], N);
+                best = n_cands - 1;
                 best_splits = c < 160 ? pick_splits(c) : 1;
                 t_best = 0.0;
             }
-            for (int i = 0; i < N_CANDS && !one_row; ++i) {
+            for (int i = 0; i < n_cands && !one_row; ++i) {
                 const int c = count(cands[i], N);
                 for (int sp = 1; sp <= 16; ++sp) {
                     if (sp > 1 && (rope_direct || !workspace || c * sp > 256 || K / sp < 256 || (size_t)sp * M * w_rows * 4 > workspace_bytes)) break;
@@ -1687,12 +1697,12 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                 }
             }
             // (one launch where the epilogue is a kernel of its own: that kernel takes the raw sums of all columns)
-            for (int i = 0; i < N_CANDS && !one_row && !g.raw; ++i) {
+            for (int i = 0; i < n_cands && !one_row && !g.raw; ++i) {
                 if (!usable(cands[i], 1)) continue;
                 const int tm = (M + cands[i].bm - 1) / cands[i].bm, full = count(cands[i], N) / 256;
                 const int cols = full * 256 / tm * width(cands[i]);          // the columns of the full rounds
                 if (full < 1 || count(cands[i], N) % 256 == 0 || cols <= 0 || cols >= N) continue;
-                for (int j = 0; j < N_CANDS; ++j) {
+                for (int j = 0; j < n_cands; ++j) {
                     if (j == i || !usable(cands[j], 1) || cols % width(cands[j])) continue;
                     const double t = seconds(cands[i], cols, 1) + seconds(cands[j], N - cols, 1) + norm_alone;
                     if (t < 0.98 * t_best) { best = i; best_splits = 1; second = j; cols_first = cols; t_best = t; }   // (a second launch costs a little, too)
