@@ -76,7 +76,7 @@ def test_rotation_in_the_chosen_tiles(ops, H, Hk, D, E, q_lens):      # noqa: F8
 # rows of one row of tiles (9 and 16 where tiles are wide products' way); column tiles enough for workgroups to begin at every slice of K and go round (K 256: as many slices as the
 # loop has in flight), a K range each with streaming copies (17 rows) and without (64 rows)
 @pytest.mark.parametrize("variant,M,N,K", [(0, 17, 5128, 256), (0, 64, 5128, 320), (58, 128, 5128, 256), (28, 192, 5128, 192), (55, 256, 5128, 192),
-                                           (0, 9, 21504, 256), (0, 16, 21504, 4096), (0, 64, 20480, 4096), (0, 17, 2048, 8192), (0, 64, 2048, 8192), (0, 128, 21504, 1024)])
+                                           (0, 9, 21504, 256), (0, 9, 32000, 4096), (0, 16, 21504, 4096), (0, 64, 20480, 4096), (0, 17, 2048, 8192), (0, 64, 2048, 8192), (0, 128, 21504, 1024)])
 def test_one_row_of_tiles(ops, variant, M, N, K):      # noqa: F811
     import torch
     dev = torch.device("cuda:0")

@@ -1603,12 +1603,23 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         return workspace ? s : 1;
     };
     if (variant == 0) {
-        // (9 to 16 rows of a product wide enough to fill the chip with tiles of 128 weight rows and K whole: the skinny kernel reads its
-        // rows from L2 for every 16 weight rows, as many bytes as the weights are.  21,504 x 4,096 at 16 rows 40 us, in tiles 30; 128,256 x
-        // 4,096 216 and 193.  Decode of 9 and 16 requests: Suripel of width 4,096 1,041 us -> 963 and 1,059 -> 980, the others' heads 1%.
-        // At 8 rows the two are even.)
-        const bool wide = M > 8 && !norm && !rope && w_packed && (N + (sw ? 63 : 127)) / (sw ? 64 : 128) >= 160 &&
-                          takes_written_order(g, 1, K, 64, 128, 4, 64);
+        // 9 to 16 rows of a product wide enough for tiles of 128 weight rows and K whole: the skinny kernel reads its
+        // rows from L2 for every 16 weight rows, as many bytes as the weights are, and takes longer for every row; tiles take as long for 9 as
+        // for 16, and a round more where they are just over 256.  The lesser of two models in us: tiles pay for the launch, for each further round,
+        // and K for the weights of a full round from memory, or for what a lone tile waits for its own; the skinny kernels (plain, plain from 65,536 weight rows
+        // on, gated) for the weights, or for their workgroups.  Fitted to 640 pairs (20,480 to 128,256 weight rows, K 256 to 8,192): 0.5% slower than
+        // the better one on average, never 4% slower than the skinny kernel; tiles wherever there are 160 were up to 43% slower (9 rows of 512 to
+        // 40,960 11.1 us, in tiles 15.9; 16 rows of 4,096 to 32,000 63.0 and 45.2; 9 of 512 to 22,016 8.3 and 9.7).
+        const int wide_tiles = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), wide_rounds = (wide_tiles + 255) / 256;
+        bool wide = M > 8 && M <= 16 && !norm && !rope && w_packed && wide_tiles >= 160 && takes_written_order(g, 1, K, 64, 128, 4, 64);
+        if (wide) {
+            const double last = 0.00925 * K * (wide_tiles - 256 * (wide_rounds - 1)) / 256, alone = 0.00526 * K, mb = 2e-6 * w_rows * K;
+            const double tiles_us = 6.95 + (2.72 + 0.00925 * K) * (wide_rounds - 1) + (last > alone ? last : alone);
+            const double groups_us = sw ? 6.5 + 4.0e-4 * w_rows : N >= 65536 ? 5.8 + 2.48e-4 * w_rows : 0.0;
+            const double bytes_us = sw ? 3.0 + mb / 6.25 : N >= 65536 ? 3.0 + mb / 6.08 : 5.86 + mb / 6.31 * (1.0 + 0.0373 * (M - 9));
+            const double by_row = sw ? 1.0 + 0.0138 * (M - 9) : N >= 65536 ? 1.0 + 0.0104 * (M - 9) : 1.0;
+            wide = tiles_us < 0.97 * by_row * (bytes_us > groups_us ? bytes_us : groups_us);
+        }
         if (M <= 16 && !wide) {
             variant = 1;
         } else if (M <= 64) {
