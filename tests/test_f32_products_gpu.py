@@ -97,3 +97,47 @@ def test_products_shared_by_sets_of_waves(M, N, K):
     got = ops.linear(a, w)
     assert not torch.isfinite(got[0]).any() and not torch.isnan(got[0][w[:, K // 2] != 0]).any()      # (an infinite sum stays infinite)
     assert ((got[1:].double() - want[1:]).abs() <= bound[1:]).all()
+
+
+# every tile by number (xr_f32_tile's: 32 x 128 with one set of waves, 64 x 64 and 32 x 64 with two, 32 x 32 with four, 64 x 64 in runs of 64
+# columns): rows and weight rows short of a tile, one past it and many; K that is whole stages of one, two and four slices, and that is not
+@pytest.mark.parametrize("tile", range(5))
+@pytest.mark.parametrize("M,N,K", [(17, 31, 516), (33, 129, 1024), (65, 2050, 2080), (130, 515, 1028), (401, 2050, 768), (64, 28675, 544)])
+def test_tiles_by_number(tile, M, N, K):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w, bias, c = (torch.randn(s, generator=g, device=dev) for s in ((M, K + 4), (N, K), (N,), (M, N)))
+    a = a[:, 4:]
+    want = a.double() @ w.double().T
+    # (each product and sum rounds to 2^-24 of what has been added up so far)
+    bound = (K + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs() + c.double().abs())
+    got = ops.linear(a, w, variant=40 + tile)
+    assert ((got.double() - want).abs() <= bound).all()
+    # a run of at most 128 columns is one sum, the runs' sums are compensated: a root mean square error of less than 4 units of 2^-24 of it
+    assert ((got.double() - want).norm() / want.norm()).item() < 4 * 2.0 ** -24
+    assert torch.equal(ops.linear(a, w, out_dtype=torch.bfloat16, variant=40 + tile), got.bfloat16())
+    assert ((ops.linear(a, w, bias=bias, variant=40 + tile).double() - want - bias.double()).abs() <= bound).all()
+    out = c.clone()
+    ops.linear(a, w, out=out, accumulate=True, variant=40 + tile)
+    assert ((out.double() - want - c.double()).abs() <= bound).all()
+    a[0, K // 2] = float("inf")
+    got = ops.linear(a, w, variant=40 + tile)
+    assert not torch.isfinite(got[0]).any() and not torch.isnan(got[0][w[:, K // 2] != 0]).any()      # (an infinite sum stays infinite)
+    assert ((got[1:].double() - want[1:]).abs() <= bound[1:]).all()
+
+
+# no branch of the choice is left without a product: wide heads of few rows, few runs of columns in many and in few tiles, and the four lines
+# between 512 and 1,024 columns
+@pytest.mark.parametrize("M,N,K,tile", [(17, 128256, 2048, 0), (1024, 8192, 260, 0), (401, 16384, 2048, 1), (401, 128256, 2048, 0), (300, 2048, 516, 4),
+                                        (33, 12288, 1024, 1), (401, 3072, 2048, 2), (64, 2048, 8192, 3), (20, 64, 64, 2), (64, 768, 768, 3), (401, 768, 768, 3), (401, 900, 768, 2),
+                                        (1024, 768, 768, 4), (128, 6144, 768, 4), (401, 2304, 768, 1)])
+def test_the_chosen_tile(M, N, K, tile):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    assert ops.lib.xr_f32_tile(M, N, K) == tile
+    a, w = torch.randn(M, K, device=dev), torch.randn(N, K, device=dev)
+    assert torch.equal(ops.linear(a, w), ops.linear(a, w, variant=40 + tile))

@@ -119,7 +119,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // sums move between registers, 1,187; two stages of 64 x 64 and four waves 1,070.  Without the sums of runs 1,034, and they cannot go.)
 // WHOLE: K is whole stages.  A row that does not exist is then read from the last one that does (its results are not stored), so
 // that a copy is a base in scalar registers and a fixed offset a lane; else a lane's pieces beyond the matrices are zeros.
-template <typename TO, bool ACC, int GM, int GN, int BM, int BN, int STAGES, int KG, bool WHOLE>
+// RUN: a run's stages.
+template <typename TO, bool ACC, int GM, int GN, int BM, int BN, int STAGES, int KG, bool WHOLE, int RUN = RBK * RB_FOLD / FBK>
 __global__ __launch_bounds__(64 * GM * GN * KG, 4) void k_gemm_f32(TO* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
                                                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
     constexpr int WAVES = GM * GN;                      // of a set
@@ -223,7 +224,6 @@ __global__ __launch_bounds__(64 * GM * GN * KG, 4) void k_gemm_f32(TO* __restric
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    constexpr int RUN = RBK * RB_FOLD / FBK;            // stages of a run
     for (int run = 0; run < n_stages; run += RUN) {
 #pragma unroll
         for (int u = 0; u < RUN; ++u) {
@@ -299,12 +299,13 @@ __global__ __launch_bounds__(64 * GM * GN * KG, 4) void k_gemm_f32(TO* __restric
     }
 }
 
-template <int GM, int GN, int BM, int BN, int STAGES, int KG>
+template <int GM, int GN, int BM, int BN, int STAGES, int KG, int RUN = RBK * RB_FOLD / FBK>
 static int launch_gemm_f32(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
                            int out_dtype, int accumulate, hipStream_t stream) {
     const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     XR_REQUIRE(tiles < (1ll << 28), "gemm: %lld tiles", tiles);
     const unsigned blocks = 8 * (unsigned)((tiles + 7) / 8);
+    // (32 x 32 tiles with 16-bit results are faster with their copies looked at: 33 x 768 x 768 13.4 us, 14.0 without)
     const bool whole = K % (KG * FBK) == 0 && (size_t)BM * lda < (1u << 30) && (size_t)BN * K < (1u << 30);
     constexpr int smem = STAGES * KG * (BM + BN) * FBK * 4;
     auto run = [&](auto kernel, auto* to) {
@@ -316,9 +317,9 @@ static int launch_gemm_f32(void* out, const float* a, const float* w, const floa
         kernel<<<blocks, 64 * GM * GN * KG, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
         return XR_OK;
     };
-    if (out_dtype == XR_BF16) return run(k_gemm_f32<bf16_t, false, GM, GN, BM, BN, STAGES, KG, false>, (bf16_t*)out);
-    if (accumulate) return whole ? run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, true>, (float*)out) : run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, false>, (float*)out);
-    return whole ? run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, true>, (float*)out) : run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, false>, (float*)out);
+    if (out_dtype == XR_BF16) return whole && KG < 4 ? run(k_gemm_f32<bf16_t, false, GM, GN, BM, BN, STAGES, KG, true, RUN>, (bf16_t*)out) : run(k_gemm_f32<bf16_t, false, GM, GN, BM, BN, STAGES, KG, false, RUN>, (bf16_t*)out);
+    if (accumulate) return whole ? run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, true, RUN>, (float*)out) : run(k_gemm_f32<float, true, GM, GN, BM, BN, STAGES, KG, false, RUN>, (float*)out);
+    return whole ? run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, true, RUN>, (float*)out) : run(k_gemm_f32<float, false, GM, GN, BM, BN, STAGES, KG, false, RUN>, (float*)out);
 }
 
 // Up to 16 rows of 32-bit operands (decoded tokens): the product is bound by how fast the weights
@@ -480,18 +481,54 @@ static void launch_gemv_ref(void* out, const float* a, const float* w, const flo
     else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, copy, stream);
 }
 
-// microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves (all sets of them), as the model in xr_gemm_ref counts them
-static double f32_tile_us(int M, int N, int K, int bm, int bn, int waves, double rate) {
+// microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves in `sets`, as the model in xr_gemm_ref counts them: `column`
+// ns for a column of 32 x 32 results, `ragged` times that where K is no whole stages, `tile` us for a tile's first stage and its sums' way out
+static double f32_tile_us(int M, int N, int K, int bm, int bn, int waves, int sets, double column, double ragged, double tile) {
     const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn), most = (double)(((long long)tiles + 255) / 256);
-    const double mean = tiles / 256 > 1.0 ? tiles / 256 : 1.0, simd = most * waves / 4.0;
-    const double products = (0.74 * most + 0.26 * mean) * (bm * bn / 1024) * K * 4.4e-3 * rate * (simd + 0.2125) / simd;
-    const double weights = (double)N * K * 4 / 5.5e6;
+    const double mean = tiles / 256 > 1.0 ? tiles / 256 : 1.0, simd = most * waves / 4.0, ns = K % (sets * FBK) == 0 ? column : column * ragged;
+    const double products = (0.722 * most + 0.278 * mean) * ((bm * bn / 1024) * (double)K * ns * 1e-3 + tile) * (simd + 0.501) / simd;
+    const double weights = (double)N * K * 4 / 5.0e6;
     return products > weights ? products : weights;
 }
 
-// accumulate != 0: out (float) += product.
+// Which tile makes a 32-bit product of more than 16 rows: 0 32 x 128 (one set of waves), 1 64 x 64 (two), 2 32 x 64 (two), 3 32 x 32 (four),
+// 4 64 x 64 (two) in runs of 64 columns.
+#define XR_F32_TILES 5
+static int f32_tile(int M, int N, int K) {
+    // The tile that should take the least time: a compute unit's tiles (the fullest one's, and on average) do their products at
+    // a rate that grows with its waves (w of them a SIMD: w / (w + 0.5)), less where K is no whole stages (what is copied is
+    // then looked at piece by piece), and each pays for its beginning and end.  Fitted to 2,400 timed launches (31 products, 64 to 128,256
+    // weight rows, K 64 to 14,336, 17 to 2,048 rows, weights from memory): 0.3% above the best of the four on average.  (Without a
+    // tile's own time, fitted to K from 2,048 on, 1.9%: 1024 x 768 x 768 ran in 768 tiles of 32 x 32, 29.2 us, where 64 x 64 ones take 20.5, and
+    // 33 x 12288 x 1024 34.2 for 25.0.)  Left out: 64 x 64 with
+    // one or four sets, 32 x 64 with four, 32 x 128 with two (0.1 to 0.9% together), 32 x 32 with eight (its registers spill).
+    // 401 x 16384 x 2048 343 us -> 234, 401 x 2048 x 8192 187 -> 142, 401 x 3072 x 2048 93 -> 57, 64 x 2048 x 8192 163 -> 60,
+    // 2048 x 16384 x 2048 1,302 -> 1,051, 401 x 128256 x 2048 2,010 -> 1,665.
+    const double tile_us[4] = {f32_tile_us(M, N, K, 32, 128, 4, 1, 3.84, 1.03, 1.80), f32_tile_us(M, N, K, 64, 64, 8, 2, 3.58, 1.07, 3.17),
+                               f32_tile_us(M, N, K, 32, 64, 4, 2, 4.07, 1.06, 1.76), f32_tile_us(M, N, K, 32, 32, 4, 4, 4.49, 1.17, 3.10)};
+    // Up to 256 tiles of 64 x 64 at least two sets of waves share the columns: shorter runs, and an error that is smaller by a third
+    // where a sum is no more than a few runs (positive numbers, K 64 to 516: 1.07e-7 with two sets, 1.43e-7 with one).  Up to four
+    // runs of columns are no work for more sets, and the number of sets then depends on the number of those tiles alone.
+    const bool few = (long long)((M + 63) / 64) * ((N + 63) / 64) <= 256;
+    const bool few_runs = K <= 4 * RBK * RB_FOLD;
+    int best = few ? 1 : 0;
+    for (int i = 1; i < 4; ++i)
+        if (tile_us[i] < tile_us[best] && !(few_runs && (!few || i == 3))) best = i;
+    // Between four runs of columns and eight, the runs of four sets are shorter than 128 columns (192 columns a set at K 768: 128 and 64), and
+    // their error is smaller than that of two sets.  They are kept up to 328 tiles of 32 x 32, where they are the fastest or nearly, and where a
+    // compute unit would have three of those tiles two sets run 64 x 64 ones in runs of 64 columns (1024 x 768 x 768, us and error against 64 bits:
+    // 32 x 32 28.9 and 1.88e-7, so 21.1 and 1.48e-7, in whole runs 20.2 and 2.06e-7).
+    if (few && !few_runs && K < 8 * RBK * RB_FOLD) {
+        const long long small = (long long)((M + 31) / 32) * ((N + 31) / 32);
+        best = small <= 328 ? 3 : small <= 512 ? 2 : small <= 768 ? 4 : 1;
+    }
+    return best;
+}
+extern "C" int xr_f32_tile(int M, int N, int K) { return f32_tile(M, N, K); }
+
+// accumulate != 0: out (float) += product.  variant: 40 + a number of f32_tile's names the tile (tests); any other, the library's choice.
 extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float* bias, int M, int N, int K,
-                           int lda, int ldo, int in_dtype, int out_dtype, int accumulate, hipStream_t stream) {
+                           int lda, int ldo, int in_dtype, int out_dtype, int accumulate, int variant, hipStream_t stream) {
     XR_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
     XR_REQUIRE(lda >= K && ldo >= N, "gemm: row strides lda=%d ldo=%d are shorter than K=%d N=%d", lda, ldo, K, N);
     XR_REQUIRE(!accumulate || out_dtype == XR_F32, "gemm: accumulation needs a 32-bit output");
@@ -501,26 +538,12 @@ extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float*
         const float* af = (const float*)a;
         const float* wf = (const float*)w;
         if (M > 16) {
-            // The tile that should take the least time: a compute unit's tiles (the fullest one's, and on average) do their products at
-            // a rate that grows with its waves (w of them a SIMD: w / (w + 0.21)).  Fitted to 1,000 timed launches (the products of the 1B and
-            // the 8B shape's layers, 17 to 2,048 rows, nine tiles): 2.6% above the best of the nine on average.  Left out: 64 x 64 with
-            // one or four sets, 32 x 64 with four, 32 x 128 with two (0.1 to 0.9% together), 32 x 32 with eight (its registers spill).
-            // 401 x 16384 x 2048 343 us -> 234, 401 x 2048 x 8192 187 -> 142, 401 x 3072 x 2048 93 -> 57, 64 x 2048 x 8192 163 -> 60,
-            // 2048 x 16384 x 2048 1,302 -> 1,051, 401 x 128256 x 2048 2,010 -> 1,665.
-            const double tile_us[4] = {f32_tile_us(M, N, K, 32, 128, 4, 0.914), f32_tile_us(M, N, K, 64, 64, 8, 0.898),
-                                       f32_tile_us(M, N, K, 32, 64, 4, 0.987), f32_tile_us(M, N, K, 32, 32, 4, 1.190)};
-            // Up to 256 tiles of 64 x 64 at least two sets of waves share the columns: shorter runs, and an error that is smaller by a third
-            // where a sum is no more than a few runs (positive numbers, K 64 to 516: 1.07e-7 with two sets, 1.43e-7 with one).  Up to four
-            // runs of columns are no work for more sets, and the number of sets then depends on the number of those tiles alone.
-            const bool few = (long long)((M + 63) / 64) * ((N + 63) / 64) <= 256;
-            const bool few_runs = K <= 4 * RBK * RB_FOLD;
-            int best = few ? 1 : 0;
-            for (int i = 1; i < 4; ++i)
-                if (tile_us[i] < tile_us[best] && !(few_runs && (!few || i == 3))) best = i;
-            const int rc = best == 0   ? launch_gemm_f32<1, 4, 32, 128, 2, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                           : best == 1 ? launch_gemm_f32<2, 2, 64, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                           : best == 2 ? launch_gemm_f32<1, 2, 32, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
-                                       : launch_gemm_f32<1, 1, 32, 32, 2, 4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
+            const int tile = variant >= 40 && variant < 40 + XR_F32_TILES ? variant - 40 : f32_tile(M, N, K);
+            const int rc = tile == 0   ? launch_gemm_f32<1, 4, 32, 128, 2, 1>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                           : tile == 1 ? launch_gemm_f32<2, 2, 64, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                           : tile == 2 ? launch_gemm_f32<1, 2, 32, 64, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                           : tile == 3 ? launch_gemm_f32<1, 1, 32, 32, 2, 4>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream)
+                                       : launch_gemm_f32<2, 2, 64, 64, 2, 2, 2>(out, af, wf, bias, M, N, K, lda, ldo, out_dtype, accumulate, stream);
             if (rc != XR_OK) return rc;
             XR_CHECK_LAUNCH("gemm_f32");
             return XR_OK;

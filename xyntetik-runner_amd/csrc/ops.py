@@ -67,7 +67,8 @@ _PROTOS = {
     "xr_gemv_extra": [_p, _p, _p, _p, _p, _f, _i, _i, _f, _i, _i, _i, _i, _i, _p],
     "xr_gemv_extra_rows": [],
     "xr_gemv_add_copy": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p],
-    "xr_gemm_ref": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
+    "xr_gemm_ref": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
+    "xr_f32_tile": [_i, _i, _i],
     "xr_gemm_bf16": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p, _p, _p],
     "xr_pack_weight": [_p, _p, _i, _i, _p],
     "xr_rope_table": [_p, _p, _p, _i, _i, _f, _p],
@@ -474,7 +475,7 @@ class Ops:
             return out.copy_(self.act_rows(self.linear(a, w, bias=bias, out_dtype=torch.float32), activation, out.dtype))
         self.lib.check(self.lib.xr_gemm_ref(out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K,
                                             a.stride(0), out.stride(0), dtype_code(a.dtype),
-                                            dtype_code(out.dtype), 1 if accumulate else 0, _stream()))
+                                            dtype_code(out.dtype), 1 if accumulate else 0, variant, _stream()))
         if activation is not None:
             self.act_rows_(out, activation)
         return out
