@@ -308,12 +308,8 @@ static int launch_gemm_f32(void* out, const float* a, const float* w, const floa
     // (32 x 32 tiles with 16-bit results are faster with their copies looked at: 33 x 768 x 768 13.4 us, 14.0 without)
     const bool whole = K % (KG * FBK) == 0 && (size_t)BM * lda < (1u << 30) && (size_t)BN * K < (1u << 30);
     constexpr int smem = STAGES * KG * (BM + BN) * FBK * 4;
+    static_assert(smem <= 65536, "more LDS has to be asked for");
     auto run = [&](auto kernel, auto* to) {
-        if (smem > 65536) {
-            const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-            if (e != hipSuccess) (void)hipGetLastError();
-            XR_REQUIRE(e == hipSuccess, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
-        }
         kernel<<<blocks, 64 * GM * GN * KG, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo);
         return XR_OK;
     };
