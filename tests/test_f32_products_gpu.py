@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 
 
 # rows: one, the ends of the few-row kernel's groups, either side of its limit, of a tile's 32, 64 and 128; columns: less than a
-# slice of 32, no multiple of it, either side of a run of 128; weight rows: few, no multiple of a tile, and so many that 200 rows make
-# 516 tiles of 64 x 128 (512 are taken in such tiles, fewer in 64 x 64)
+# slice of 32, no multiple of it, either side of a run of 128; weight rows: few, no multiple of a tile, and so many that there are
+# more than 256 tiles of 64 x 64 (one set of waves makes a tile then, two where there are fewer)
 @pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 33, 64, 65, 130, 200])
 @pytest.mark.parametrize("N,K", [(7, 4), (96, 64), (100, 124), (65, 132), (200, 260), (16448, 68), (16450, 132)])
 def test_product(M, N, K):
@@ -54,28 +54,30 @@ def test_weight_rows_a_wave(M, N, K):
     assert ((narrow.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size).all()
 
 
-# tiles of one set of waves (more than 256 of 64 x 64) and of two, each from every second slice
-@pytest.mark.parametrize("M,N,K,many", [(17, 1000, 4096, False), (17, 2048, 14336, False), (130, 1024, 8192, False), (401, 4096, 8192, True)])
-def test_sums_of_one_sign_are_as_close_with_two_sets_of_waves(M, N, K, many):
-    """Positive numbers, whose sums only grow: compensated sums of runs, however many waves share the columns.  The same rows and
-    columns among so many that one set of waves makes each tile are the yardstick."""
+# products that the library makes in tiles of two sets of waves and of four
+@pytest.mark.parametrize("M,N,K", [(17, 1000, 4096), (17, 2048, 14336), (130, 1024, 8192), (401, 4096, 8192)])
+def test_sums_of_one_sign_are_as_close_with_several_sets_of_waves(M, N, K):
+    """Positive numbers, whose sums only grow: compensated sums of runs, however many sets of waves share the columns.  The tile that
+    one set makes is the yardstick."""
     import torch
     from xyntetik_runner_amd.csrc.ops import load_ops
     ops, dev = load_ops(), torch.device("cuda:0")
-    assert (-(-M // 64) * -(-N // 64) > 256) == many
+    assert ops.lib.xr_f32_tile(M, N, K) in (1, 2, 3)
     g = torch.Generator(device=dev)
     g.manual_seed(M + N + K)
     a, w = (torch.rand(s, generator=g, device=dev) for s in ((M, K), (N, K)))
     want = a.double() @ w.double().T
     off = lambda got: ((got.double() - want).norm() / want.norm()).item()
-    rows = a.repeat(-(-257 * 64 // (-(-N // 64) * M)) + 1, 1)             # (each row's sum is its own: the first M of them)
-    assert -(-rows.shape[0] // 64) * -(-N // 64) > 256
-    assert off(ops.linear(a, w)) <= 1.02 * off(ops.linear(rows, w)[:M])   # (millions of roundings: their 2-norms agree to 1%)
+    one = off(ops.linear(a, w, variant=40))
+    assert one < 2.0 ** -24                               # (what is left is the rounding inside a run)
+    for tile in (1, 2, 3, 4):
+        assert off(ops.linear(a, w, variant=40 + tile)) <= 1.02 * one         # (millions of roundings: their 2-norms agree to 1%)
+    assert off(ops.linear(a, w)) <= 1.02 * one
 
 
-# rows and weight rows at the edges of tiles of 32 and 64 for which one, two and four sets of waves share the columns; columns that are whole
-# stages of one, two or four slices of 32, and that are not (516, 1028); fewer slices than a run (544)
-@pytest.mark.parametrize("M,N", [(17, 31), (32, 2048), (33, 2050), (64, 4097), (401, 3072), (300, 96), (130, 8200)])
+# rows and weight rows at the edges of tiles, in the tiles that the library chooses for them: 32 x 32 with four sets, 32 x 64 and 64 x 64 with two;
+# columns that are whole stages of one, two or four slices of 32, and that are not (516, 1028); fewer slices than a run (544)
+@pytest.mark.parametrize("M,N", [(17, 31), (32, 2048), (33, 2050), (64, 4097), (401, 3072), (401, 2050), (300, 96), (130, 8200)])
 @pytest.mark.parametrize("K", [516, 544, 1024, 1028, 2080])
 def test_products_shared_by_sets_of_waves(M, N, K):
     import torch
