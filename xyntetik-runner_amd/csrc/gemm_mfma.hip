@@ -1,14 +1,15 @@
 // bfloat16 matrix products on the gfx950 matrix cores, 32-bit accumulation:
 //   out[M,N] = a[M,K] * w[N,K]^T (+ bias)        (weights [n_out][n_in], row-major)
 // Two kernels share the epilogues:
-//   * k_gemm_tile_async: more than 16 rows (prompt portions, large batches).  A workgroup
+//   * k_gemm_tile_async: more than 16 rows (prompt portions, large batches), and 9 to 16 rows of
+//     packed weights so many that it is the faster one (the head of a model, a wide first product).  A workgroup
 //     computes a BM x BN tile; both operands are copied from memory straight into LDS in
 //     64-wide K slices (16-byte chunks, XOR-swizzled so that fragment reads do not collide),
 //     several slices ahead, and fed to v_mfma_f32_32x32x16_bf16.  With few tiles K is split
 //     over workgroups and k_gemm_finish adds the parts in a fixed order.  Three main loops:
 //     four waves with the order of their instructions written out (what serves, where K is
 //     whole slices), and two with eight waves for the rest.
-//   * k_gemm_skinny: M <= 16 (decoding).  The product is bound by reading the weights
+//   * k_gemm_skinny: the other products of up to 16 rows (decoding).  The product is bound by reading the weights
 //     once, so each wave streams 16 weight rows straight from memory into MFMA fragments
 //     (v_mfma_f32_16x16x32_bf16, weights as the A operand, tokens as the B operand) with
 //     many loads in flight, and the waves of a workgroup split K among themselves.

@@ -6,10 +6,11 @@
 // kernels (k_gemm_f32 on the matrix cores, k_gemm_ref where operands are not 16-byte aligned or not 32-bit)
 // sum in two levels, with up to 16 the kernel further down
 // (k_gemv_ref) gives every lane every 64th group of four columns and adds the lanes' sums in a
-// tree.  A token's 32-bit result therefore differs in its last bits between a step of 16 rows and
-// one of 17 (both stay within 1e-6 of the exact product at K = 14,336), and between steps of so many rows that
-// k_gemm_f32 takes another number of waves for a tile (a run is then 128 columns of every second or fourth slice of 32).
-// The tile kernels' two levels: runs of RBK * RB_FOLD = 128 columns are summed one after another, and the runs'
+// tree, and with up to 4 rows (xr_gemv_extra) norms them on the way, so that the norm's factor comes behind the sum instead of before
+// it.  A token's 32-bit result therefore differs in its last bits between steps of 4 rows and 5, of 16 rows and
+// 17 (all stay within 1e-6 of the exact product at K = 14,336), and between steps of so many rows that
+// k_gemm_f32 takes another number of waves for a tile (a run is then 128 columns of every second or fourth slice of 32, or 64 of every second).
+// The tile kernels' two levels: runs of RBK * RB_FOLD = 128 columns (64 in one tile, see f32_tile) are summed one after another, and the runs'
 // sums are added up with a compensated (Kahan) sum.  One running 32-bit sum over the 14,336
 // columns of a wide feed-forward loses about 1e-5 of the result to rounding, which at such
 // widths is as much as a real fault may be; summed this way a product is about ten times closer
@@ -477,7 +478,7 @@ static void launch_gemv_ref(void* out, const float* a, const float* w, const flo
     else launch_gemv_cols<MT, 2>(out, a, w, bias, M, N, K, lda, ldo, out_dtype, accumulate, copy, stream);
 }
 
-// microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves in `sets`, as the model in xr_gemm_ref counts them: `column`
+// microseconds of a 32-bit product in tiles of bm x bn made by `waves` waves in `sets`, as f32_tile counts them: `column`
 // ns for a column of 32 x 32 results, `ragged` times that where K is no whole stages, `tile` us for a tile's first stage and its sums' way out
 static double f32_tile_us(int M, int N, int K, int bm, int bn, int waves, int sets, double column, double ragged, double tile) {
     const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn), most = (double)(((long long)tiles + 255) / 256);

@@ -429,9 +429,9 @@ class Ops:
         """``a [M, K] @ w [N, K]^T (+ bias)``; with ``accumulate`` added into 32-bit ``out``; ``activation`` "relu2": the
         square of what is positive of it (in the kernels' epilogues).
 
-        bfloat16 operands run on the matrix cores (32-bit accumulation); float32 operands, and
-        shapes the MFMA kernels do not take, run the plain 32-bit FMA kernel.  ``w`` is a matrix
-        or a ``PackedWeight``.
+        bfloat16 operands run on the matrix cores (32-bit accumulation), float32 operands in 32 bits throughout (more than
+        16 aligned rows on the matrix cores, too), and what those kernels do not take runs the plain 32-bit FMA kernel.  ``w`` is a matrix
+        or a ``PackedWeight``.  ``variant``: a kernel by number instead of the library's choice (tests).
         """
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w
@@ -611,8 +611,10 @@ class Ops:
         """``act(a @ w[:F]^T) * (a @ w[F:]^T)`` for ``w [2F, K]`` = gate rows then up rows
         (a matrix, or a ``PackedWeight`` made with ``gated=True``); ``activation`` is one of
         ``GATE_ACTIVATIONS``, with its number ``param`` for one of ``SHAPED_GATES``.  The matrix-core kernels
-        apply the gate in their epilogue; where they do not serve (float32, sizes they do not take) the
-        product leaves both branches in 32 bits and ``gate_mul`` makes the value of them."""
+        apply the gate in their epilogue, and so does the product of up to ``EXTRA_ROWS`` float32 rows; elsewhere
+        (more float32 rows, sizes they do not take) the
+        product leaves both branches in 32 bits and ``gate_mul`` makes the value of them.  (bfloat16: up to 16 rows the gate is
+        made with ``expf`` and a division, in tiles, from 9 rows of wide weights on, with the hardware's 2^x and reciprocal.)"""
         act = activation_code(activation)
         packed = isinstance(w, PackedWeight)
         wt = w.data if packed else w

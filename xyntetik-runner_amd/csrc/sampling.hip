@@ -22,7 +22,7 @@
 // each 50 us, so a row's histogram is shared out to up to 8 workgroups where the caller brings room for their
 // partial counts; the cuts are a chain of short steps that one workgroup a row walks.
 // Where every cut was a radix selection (22 passes over the row for top-p) 64 rows of 128,256 logits
-// took 1,150 us; now 53 in three kernels (6 + 17 + 30; 34 with bins of some hundred candidates sorted by a network).
+// took 1,150 us; now 54 in three kernels (7 + 17 + 31; 34 with bins of 5 to 256 candidates sorted by a network).
 #include "common.h"
 #include "no_alloc.h"
 
