@@ -1608,7 +1608,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         // rows from L2 for every 16 weight rows, as many bytes as the weights are, and takes longer for every row; tiles take as long for 9 as
         // for 16, and a round more where they are just over 256.  The lesser of two models in us: tiles pay for the launch, for each further round,
         // and K for the weights of a full round from memory, or for what a lone tile waits for its own; the skinny kernels (plain, plain from 65,536 weight rows
-        // on, gated) for the weights, or for their workgroups.  Fitted to 640 pairs (20,480 to 128,256 weight rows, K 256 to 8,192): 0.3% slower than
+        // on, gated) for the weights, or for their workgroups.  Fitted to 680 pairs (20,480 to 128,256 weight rows, K 256 to 8,192): 0.3% slower than
         // the better one on average, at most 4.4% slower than the skinny kernel; tiles wherever there are 160 were up to 43% slower (9 rows of 512 to
         // 40,960 11.1 us, in tiles 15.9; 16 rows of 4,096 to 32,000 63.0 and 45.2; 9 of 512 to 22,016 8.3 and 9.7).
         const int wide_tiles = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), wide_rounds = (wide_tiles + 255) / 256;
