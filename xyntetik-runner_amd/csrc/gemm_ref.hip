@@ -1,5 +1,5 @@
 // Matrix product out[M,N] = a[M,K] * w[N,K]^T (+ bias) in true 32 bits: the matrix product of the 32-bit
-// path, and (k_gemm_ref, FMA only, any types and alignment) the yardstick of the bfloat16 MFMA kernels.
+// path (but for products of many rows or columns, which gemm_f32_parts.hip makes), and (k_gemm_ref, FMA only, any types and alignment) the yardstick of the bfloat16 MFMA kernels.
 // Weights are [n_out][n_in] row-major as the reference keeps them
 // (src/model.c:193-205).  A row's result does not depend on the rows beside it, but the order
 // of its sum over k depends on how many rows the product has: with more than 16 rows the tile
@@ -488,6 +488,14 @@ static double f32_tile_us(int M, int N, int K, int bm, int bn, int waves, int se
     return products > weights ? products : weights;
 }
 
+// that of tiles 0 to 3
+static void f32_tile_times(int M, int N, int K, double (&us)[4]) {
+    us[0] = f32_tile_us(M, N, K, 32, 128, 4, 1, 3.84, 1.03, 1.80);
+    us[1] = f32_tile_us(M, N, K, 64, 64, 8, 2, 3.58, 1.07, 3.17);
+    us[2] = f32_tile_us(M, N, K, 32, 64, 4, 2, 4.07, 1.06, 1.76);
+    us[3] = f32_tile_us(M, N, K, 32, 32, 4, 4, 4.49, 1.17, 3.10);
+}
+
 // Which tile makes a 32-bit product of more than 16 rows: 0 32 x 128 (one set of waves), 1 64 x 64 (two), 2 32 x 64 (two), 3 32 x 32 (four),
 // 4 64 x 64 (two) in runs of 64 columns.
 #define XR_F32_TILES 5
@@ -501,8 +509,8 @@ static int f32_tile(int M, int N, int K) {
     // one or four sets, 32 x 64 with four, 32 x 128 with two (0.1 to 0.9% together), 32 x 32 with eight (its registers spill).
     // 401 x 16384 x 2048 343 us -> 234, 401 x 2048 x 8192 187 -> 142, 401 x 3072 x 2048 93 -> 57, 64 x 2048 x 8192 163 -> 60,
     // 2048 x 16384 x 2048 1,302 -> 1,051, 401 x 128256 x 2048 2,010 -> 1,665.
-    const double tile_us[4] = {f32_tile_us(M, N, K, 32, 128, 4, 1, 3.84, 1.03, 1.80), f32_tile_us(M, N, K, 64, 64, 8, 2, 3.58, 1.07, 3.17),
-                               f32_tile_us(M, N, K, 32, 64, 4, 2, 4.07, 1.06, 1.76), f32_tile_us(M, N, K, 32, 32, 4, 4, 4.49, 1.17, 3.10)};
+    double tile_us[4];
+    f32_tile_times(M, N, K, tile_us);
     // Up to 256 tiles of 64 x 64 at least two sets of waves share the columns: shorter runs, and an error that is smaller by a third
     // where a sum is no more than a few runs (positive numbers, K 64 to 516: 1.07e-7 with two sets, 1.43e-7 with one).  Up to four
     // runs of columns are no work for more sets, and the number of sets then depends on the number of those tiles alone.
@@ -522,6 +530,14 @@ static int f32_tile(int M, int N, int K) {
     return best;
 }
 extern "C" int xr_f32_tile(int M, int N, int K) { return f32_tile(M, N, K); }
+// the time that the fastest tile takes by that model, for the choice between these kernels and gemm_f32_parts.hip's
+double xr_f32_tiles_us(int M, int N, int K) {
+    double tile_us[4], best;
+    f32_tile_times(M, N, K, tile_us);
+    best = tile_us[0];
+    for (int i = 1; i < 4; ++i) best = tile_us[i] < best ? tile_us[i] : best;
+    return best;
+}
 
 // accumulate != 0: out (float) += product.  variant: 40 + a number of f32_tile's names the tile (tests); any other, the library's choice.
 extern "C" int xr_gemm_ref(void* out, const void* a, const void* w, const float* bias, int M, int N, int K,

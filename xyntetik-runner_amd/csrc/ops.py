@@ -69,6 +69,9 @@ _PROTOS = {
     "xr_gemv_add_copy": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p],
     "xr_gemm_ref": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_f32_tile": [_i, _i, _i],
+    "xr_gemm_f32_parts": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p],
+    "xr_gemm_f32_parts_plan": [_i, _i, _i],
+    "xr_gemm_f32_parts_ranges": [_i],
     "xr_gemm_bf16": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p, _p, _p],
     "xr_pack_weight": [_p, _p, _i, _i, _p],
     "xr_rope_table": [_p, _p, _p, _i, _i, _f, _p],
@@ -154,6 +157,13 @@ class PackedWeight:
     @property
     def device(self):
         return self.data.device
+
+
+class F32Weight(torch.Tensor):
+    """A float32 weight matrix as it is, as one that a model keeps: its products of many rows may be made of bfloat16 parts
+    (``Ops.linear``).  Made by ``Ops.pack_weight``; what is computed from it is a plain tensor."""
+
+    __torch_function__ = torch._C._disabled_torch_function_impl
 
 
 class UnscaledRows:
@@ -410,7 +420,10 @@ class Ops:
     def pack_weight(self, w: torch.Tensor, gated: bool = False):
         """``w`` for use as the weight of ``linear`` (``gated``: of ``linear_gated``): packed for
         the MFMA kernels where they will serve it (bfloat16, a width that is a multiple of 8, for
-        gate and up rows a height that is a multiple of 32), else ``w`` itself."""
+        gate and up rows a height that is a multiple of 32), a float32 matrix wide enough for products
+        of parts as an ``F32Weight`` (the same memory), else ``w`` itself."""
+        if w.dtype == torch.float32 and w.dim() == 2 and w.shape[1] >= 512 and w.shape[1] % 64 == 0:
+            return w.as_subclass(F32Weight)
         if not (self.use_mfma and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] % 8 == 0):
             return w
         N, K = w.shape
@@ -430,7 +443,8 @@ class Ops:
         square of what is positive of it (in the kernels' epilogues).
 
         bfloat16 operands run on the matrix cores (32-bit accumulation), float32 operands in 32 bits throughout (more than
-        16 aligned rows on the matrix cores, too), and what those kernels do not take runs the plain 32-bit FMA kernel.  ``w`` is a matrix
+        16 aligned rows on the matrix cores, too: by its 32-bit instructions, or with an ``F32Weight``, where that is faster, by bfloat16 ones
+        from three exact parts of every number), and what those kernels do not take runs the plain 32-bit FMA kernel.  ``w`` is a matrix
         or a ``PackedWeight``.  ``variant``: a kernel by number instead of the library's choice (tests).
         """
         packed = isinstance(w, PackedWeight)
@@ -473,12 +487,29 @@ class Ops:
             raise KernelError("linear: a packed weight needs bfloat16 rows that are 16-byte aligned")
         if activation is not None and out.dtype != torch.float32:
             return out.copy_(self.act_rows(self.linear(a, w, bias=bias, out_dtype=torch.float32), activation, out.dtype))
-        self.lib.check(self.lib.xr_gemm_ref(out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K,
-                                            a.stride(0), out.stride(0), dtype_code(a.dtype),
-                                            dtype_code(out.dtype), 1 if accumulate else 0, variant, _stream()))
+        plan = self._parts_plan(a, w, out, variant)
+        if plan:
+            ranges = self.lib.xr_gemm_f32_parts_ranges(plan)
+            sums = torch.empty((ranges, M, N, 2), dtype=torch.float32, device=a.device) if ranges > 1 else None
+            self.lib.check(self.lib.xr_gemm_f32_parts(out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K,
+                                                      a.stride(0), out.stride(0), dtype_code(out.dtype), 1 if accumulate else 0, plan,
+                                                      _ptr(sums), _stream()))
+        else:
+            self.lib.check(self.lib.xr_gemm_ref(out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K,
+                                                a.stride(0), out.stride(0), dtype_code(a.dtype),
+                                                dtype_code(out.dtype), 1 if accumulate else 0, variant, _stream()))
         if activation is not None:
             self.act_rows_(out, activation)
         return out
+
+    def _parts_plan(self, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, variant: int) -> int:
+        """How the library makes a 32-bit product of bfloat16 parts on the matrix cores (``xr_gemm_f32_parts_plan``), or 0 where it does
+        not.  A ``variant`` of 60 + a plan asks for that plan, 40 to 44 for the 32-bit kernel's tiles."""
+        M, K = a.shape
+        if (not isinstance(w, F32Weight) or a.dtype != torch.float32 or M <= 16 or 40 <= variant <= 44 or K % 64 or a.stride(0) % 4
+                or a.data_ptr() % 16 or w.data_ptr() % 16 or out.dtype not in (torch.float32, torch.bfloat16)):
+            return 0
+        return variant - 60 if variant > 60 else self.lib.xr_gemm_f32_parts_plan(M, w.shape[0], K)
 
     def _extra_ok(self, a, w, bias: Optional[torch.Tensor]) -> bool:
         """Whether a product of 32-bit rows may norm them (``UnnormedRows``) or gate its result itself: few rows, 16-byte aligned, and of
