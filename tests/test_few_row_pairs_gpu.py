@@ -1,0 +1,58 @@
+"""Products of few rows and few weight rows, whose k-steps are taken in pairs by workgroups of 8 weight rows, at the edges of their sizes."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# weight rows: fewer than a workgroup's 8, no multiple of 8 or 16, the most; columns: whole pairs of 32, an odd step at the end, a last step of 8
+@pytest.mark.parametrize("N,K", [(7, 2048), (2048, 2048), (2041, 2080), (2024, 2056), (40, 14336), (1000, 4104), (2048, 10752)])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
+def test_product(M, N, K):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w, bias, c = (torch.randn(s, generator=g, device=dev) for s in ((M, K + 8), (N, K), (N,), (M, N)))
+    a, w = a.bfloat16()[:, 8:], (w * 0.1).bfloat16()
+    want = a.double() @ w.double().T
+    # exact products of bfloat16 numbers, at most K additions that round to 2^-24 of what has been added up so far
+    bound = (K + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs() + c.double().abs())
+    packed = ops.pack_weight(w)
+    got = ops.linear(a, packed, out_dtype=torch.float32)
+    assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(ops.linear(a, w, out_dtype=torch.float32), got)
+    assert torch.equal(ops.linear(a, packed, bias=bias, out_dtype=torch.float32), got + bias)
+    assert torch.equal(ops.linear(a, packed), got.bfloat16())
+    out = c.clone()
+    ops.linear(a, packed, out=out, accumulate=True)
+    assert torch.equal(out, c + got)
+    # a row's result does not depend on the rows beside it, on either side of 8 rows
+    assert torch.equal(ops.linear(a[:1], packed, out_dtype=torch.float32), got[:1])
+    many = torch.cat([a, a[:1].expand(16 - M, K)]) if M < 16 else a
+    assert torch.equal(ops.linear(many.contiguous(), packed, out_dtype=torch.float32)[:M], got)
+
+
+@pytest.mark.parametrize("N,F,K", [(2048, 512, 2048), (2040, 8192, 2080), (24, 128256 // 16, 4096)])
+@pytest.mark.parametrize("M", [1, 8, 9])
+def test_the_norm_behind_it(M, N, F, K):
+    """The product adds into a stream and leaves its weighted rows and the sums of their squares to the next product."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import UnscaledRows, load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a, w, x, nw, w2 = (torch.randn(s, generator=g, device=dev) for s in ((M, K), (N, K), (M, N), (N,), (F, N)))
+    a, w, w2 = a.bfloat16(), ops.pack_weight((w * 0.05).bfloat16()), ops.pack_weight((w2 * 0.05).bfloat16())
+    x = x * torch.linspace(0.1, 30, M, device=dev)[:, None]
+    want = x.clone()
+    ops.linear(a, w, out=want, accumulate=True)
+    h = ops.linear_add_rmsnorm(a, w, x, nw, 1e-5, torch.bfloat16, defer=True)
+    assert isinstance(h, UnscaledRows) and torch.equal(x, want) and torch.equal(h.data, (x * nw).bfloat16())
+    d = x.double()
+    # (sums of N squares, every one and every addition rounded to 2^-24)
+    assert ((h.sumsq[:, :M].double().sum(0) - (d * d).sum(1)).abs() <= (N + 2) * 2.0 ** -24 * (d * d).sum(1)).all()
+    scale = torch.rsqrt((d * d).mean(1, keepdim=True) + 1e-5)
+    rows, wt = h.data.double() * scale, ops.linear(torch.eye(N, device=dev).bfloat16(), w2, out_dtype=torch.float32).double() if N % 8 == 0 else None
+    got = ops.linear(h, w2, out_dtype=torch.float32).double()
+    assert ((got - rows @ wt).abs() <= (N + 8) * 2.0 ** -23 * (rows.abs() @ wt.abs())).all()

@@ -89,7 +89,7 @@ struct GemmArgs {
     int n_ss;
     float ss_inv_width, ss_eps;
     // After (with EPI_ACCUM): the updated output row times norm_w goes to xg [M][N], and
-    // the sums of squares of columns 16p .. 16p+15 of the updated rows go to ss_out[p][16].
+    // the sums of squares of columns 16p .. 16p+15 of the updated rows (8p .. 8p+7 from workgroups of pairs) go to ss_out[p][16].
     const void* norm_w;
     int norm_w_bf16;
     bf16_t* xg;
@@ -1180,27 +1180,36 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
 // L2) of U k-steps of 32 before it uses them; with N/(16*RT) workgroups of KSW waves this
 // keeps tens of kilobytes in flight on every compute unit.  The slices are summed through
 // LDS in a fixed order.
-template <int MT, int RT, int KSW, int U, bool SWIGLU, bool NT>
+// PAIRS: products with so few weight rows that workgroups of 16 leave half the chip idle.  Steps are taken in pairs, the even ones'
+// sum and the odd ones' apart.  1 (up to 8 rows): a workgroup owns 8 weight rows, and one instruction makes both steps of a pair: rows 0 to 7 of
+// its operands are the even step's, 8 to 15 the odd one's, and what rows of one and columns of the other make is not used.  2 (9 to
+// 16 rows): 16 weight rows, the two sums in registers of their own, so that a row's result is the same either way.
+template <int MT, int RT, int KSW, int U, bool SWIGLU, bool NT, int PAIRS = 0>
 __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
     constexpr int NWT = SWIGLU ? 2 : 1;  // weight fragments per row group (gate and up)
-    constexpr int MTOK = MT * 16, ROWS = RT * 16, THREADS = 64 * KSW;
-    extern __shared__ float red[];       // [KSW][NWT][ROWS][MTOK]
+    constexpr int MTOK = MT * 16, ROWS = PAIRS == 1 ? 8 : RT * 16, THREADS = 64 * KSW;
+    constexpr int SROWS = RT * 16;
+    static_assert(PAIRS == 0 || (MT == 1 && RT == 1 && !SWIGLU && (PAIRS == 1 || U % 2 == 0)), "pairs of k-steps: plain products of one group each way");
+    constexpr int STEP = PAIRS == 1 ? 64 : 32;                        // columns of one product
+    extern __shared__ float red[];       // [KSW][NWT][SROWS][MTOK]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
+    const int l16 = PAIRS == 1 ? lane & 7 : lane & 15, lq = lane >> 4;
+    const int odd = PAIRS == 1 ? (lane >> 3) & 1 : 0;                 // this lane's step of a pair
     const int n_base = blockIdx.x * ROWS;
-    const int steps_total = (g.K + 31) / 32;
-    const int steps_per = (steps_total + KSW - 1) / KSW;
-    const int kbeg = wave * steps_per * 32;
-    const int kend_ = kbeg + steps_per * 32;
+    constexpr int SHARE = PAIRS ? 64 : 32;                            // a wave's columns are whole pairs
+    const int shares = (g.K + SHARE - 1) / SHARE;
+    const int kbeg = wave * ((shares + KSW - 1) / KSW) * SHARE;
+    const int kend_ = kbeg + (shares + KSW - 1) / KSW * SHARE;
     const int kend = kend_ < g.K ? kend_ : g.K;
 
     // Row-major: the lane reads row l16 of its group at column 8 * lq of the k-step.  Packed:
     // the wave reads the k-step's block of its group, the lane its 16 bytes of it.
     const size_t kblocks = (size_t)((g.K + 31) / 32);
-    const int step_stride = g.w_packed ? 512 : 32;
-    const int lane_off = g.w_packed ? (l16 * 4 + lq) * 8 : lq * 8;
-    const int dead_off = g.w_packed ? (l16 * 4 + lq) * 8 : 0;      // where a lane whose column does not exist reads
+    const int step_stride = (g.w_packed ? 512 : 32) * (STEP / 32);
+    const int in_block = PAIRS == 1 ? (n_base & 8) + l16 : l16;    // the lane's row of its 16
+    const int lane_off = g.w_packed ? odd * 512 + (in_block * 4 + lq) * 8 : odd * 32 + lq * 8;
+    const int dead_off = g.w_packed ? (in_block * 4 + lq) * 8 : 0; // where a lane whose column does not exist reads
     const bf16_t* wp[NWT][RT];
     bool w_ok[RT];
 #pragma unroll
@@ -1226,9 +1235,10 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
         ap[i] = g.a + (size_t)(a_ok[i] ? tok : 0) * g.lda;
     }
 
-    f32x4 acc[NWT][RT][MT];
+    constexpr int NSUM = PAIRS == 2 ? 2 : NWT;
+    f32x4 acc[NSUM][RT][MT];
 #pragma unroll
-    for (int t = 0; t < NWT; ++t)
+    for (int t = 0; t < NSUM; ++t)
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -1237,7 +1247,7 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
     // the first SS_AHEAD partial sums of squares of a folded norm are copied to LDS meanwhile
     // (no registers are held for them; a wave's copy moves 16 partial rows)
     constexpr int SS_AHEAD = 256;
-    float* scale_s = red + KSW * NWT * ROWS * MTOK;       // [16 parts][16 rows]
+    float* scale_s = red + KSW * NWT * SROWS * MTOK;       // [16 parts][16 rows]
     float* ss_s = scale_s + 256;                          // [SS_AHEAD][16 rows]
     if (g.ss_in) {
         const int chunks = (g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD) * 4;      // pieces of 16 bytes
@@ -1250,14 +1260,14 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
     }
 
     const uint4 zero = make_uint4(0, 0, 0, 0);
-    for (int k0 = kbeg; k0 < kend; k0 += 32 * U) {
+    for (int k0 = kbeg; k0 < kend; k0 += STEP * U) {
         uint4 wreg[U][NWT][RT], areg[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = k0 + u * 32 + lq * 8;
+            const int k = k0 + u * STEP + odd * 32 + lq * 8;
             const bool k_ok = k < kend;
             const int ks = k_ok ? k : 0;             // a column that exists; the value is dropped
-            const size_t wo = k_ok ? (size_t)((k0 >> 5) + u) * step_stride + lane_off : (size_t)dead_off;
+            const size_t wo = k_ok ? (size_t)(k0 / STEP + u) * step_stride + lane_off : (size_t)dead_off;
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -1275,9 +1285,10 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
 #pragma unroll
                 for (int r = 0; r < RT; ++r)
 #pragma unroll
-                    for (int t = 0; t < NWT; ++t)
-                        acc[t][r][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), af,
-                                                                                acc[t][r][i], 0, 0, 0);
+                    for (int t = 0; t < NWT; ++t) {
+                        f32x4& sum = acc[PAIRS == 2 ? u & 1 : t][r][i];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), af, sum, 0, 0, 0);
+                    }
             }
     }
 
@@ -1290,7 +1301,8 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
             for (int i = 0; i < MT; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    red[((wave * NWT + t) * ROWS + r * 16 + lq * 4 + e) * MTOK + i * 16 + l16] = acc[t][r][i][e];
+                    red[((wave * NWT + t) * SROWS + r * 16 + lq * 4 + e) * MTOK + i * 16 + (lane & 15)] =
+                        PAIRS == 2 ? acc[0][r][i][e] + acc[NSUM - 1][r][i][e] : acc[t][r][i][e];
     // the rows' scales, from the partial sums the producer of `a` left: thread (part, tok) of the
     // first 256 sums every 16th partial, each thread of the last loop sums the 16 parts of its
     // row; the order is the same in every instance of this kernel, so a row's scale does not
@@ -1316,7 +1328,11 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
         for (int t = 0; t < NWT; ++t) {
             float s = 0.f;
 #pragma unroll
-            for (int k = 0; k < KSW; ++k) s += red[((k * NWT + t) * ROWS + col) * MTOK + tok];
+            for (int k = 0; k < KSW; ++k) {
+                float x = red[((k * NWT + t) * SROWS + col) * MTOK + tok];
+                if (PAIRS == 1) x += red[(k * SROWS + 8 + col) * MTOK + 8 + (tok & 7)];       // the odd steps' sum
+                s += x;
+            }
             v[t] = s;
         }
         if (g.ss_in) {
@@ -1349,10 +1365,11 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                 g.xg[(size_t)tok * g.N + nn] = f32_to_bf16(xn * nw);
             }
             float sq = xn * xn;
+            constexpr int PW = PAIRS ? 8 : 16;   // columns of a partial sum
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
-            const int part = blockIdx.x * RT + (col >> 4);
-            if ((col & 15) == 0 && tok < 16 && part * 16 < g.N) g.ss_out[part * 16 + tok] = sq;
+            for (int o = PW / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+            const int part = (n_base + col) / PW;
+            if (col % PW == 0 && tok < 16 && part * PW < g.N) g.ss_out[part * 16 + tok] = sq;
         } else if (ok) {
             store_out(g, tok, nn, v[0] + (g.bias ? g.bias[nn] : 0.f));
         }
@@ -1417,13 +1434,13 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
 // returns the number of workgroups, or an error (< 0)
 static inline int rc_of(int launched) { return launched < 0 ? launched : XR_OK; }
 
-template <int MT, int RT, int KSW, int U, bool SW, bool NT = false>
+template <int MT, int RT, int KSW, int U, bool SW, bool NT = false, int PAIRS = 0>
 static int launch_skinny(const GemmArgs& g, hipStream_t stream) {
     constexpr int NWT = SW ? 2 : 1;
     size_t smem = (size_t)KSW * NWT * RT * 16 * MT * 16 * 4 + 256 * 4 + 256 * 64;    // the sums of the waves, 256 partial scales, 256 rows of partial sums
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_skinny<MT, RT, KSW, U, SW, NT>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) {
             (void)hipGetLastError();             // or the next launch's check would report this refusal
@@ -1432,8 +1449,9 @@ static int launch_skinny(const GemmArgs& g, hipStream_t stream) {
         }
         attr_set = true;
     }
-    unsigned blocks = (unsigned)((g.N + 16 * RT - 1) / (16 * RT));
-    k_gemm_skinny<MT, RT, KSW, U, SW, NT><<<blocks, 64 * KSW, smem, stream>>>(g);
+    constexpr int rows = PAIRS == 1 ? 8 : 16 * RT;
+    unsigned blocks = (unsigned)((g.N + rows - 1) / rows);
+    k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS><<<blocks, 64 * KSW, smem, stream>>>(g);
     XR_CHECK_LAUNCH("gemm_skinny");
     return (int)blocks;
 }
@@ -1526,8 +1544,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                            "gemm: rows that become a norm: more than 16, 16-byte aligned, %d apart", norm->post_ld);
                 g.post_x = (float*)norm->post_x; g.post_ld = norm->post_ld; g.post_alpha = norm->post_alpha;
             }
-            XR_REQUIRE(M > 16 || (norm->ss_out && norm->ss_out_rows >= (N + 15) / 16),
-                       "gemm: room for %d partial sums of squares, %d needed", norm->ss_out ? norm->ss_out_rows : 0, (N + 15) / 16);
+            XR_REQUIRE(M > 16 || (norm->ss_out && norm->ss_out_rows >= (N + 7) / 8),
+                       "gemm: room for %d partial sums of squares, %d needed", norm->ss_out ? norm->ss_out_rows : 0, (N + 7) / 8);
             XR_REQUIRE(!norm->centred || M > 16, "gemm: a layer norm after a product of %d rows: from 17 rows on", M);
             g.norm_centred = norm->centred ? 1 : 0;
             g.norm_w = norm->norm_w; g.norm_w_bf16 = norm->norm_w_bf16; g.xg = (bf16_t*)norm->xg; g.ss_out = norm->ss_out;
@@ -1744,12 +1762,18 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // are read once, with loads marked as streaming: that alone gave 3-9% on every one of
             // them (the head of the 8B shape at one row: 1.05 GB in 149 us, 7.1 TB/s).
             int blocks;
+            // Up to 2,048 weight rows, 2,048 columns on: workgroups of 8 weight rows (one for every compute unit at 2,048).  us without and
+            // with at 1 and 8 rows: 2048 x 8192 11.3, 11.5 and 8.3, 9.2; 2048 x 10752 15.5, 15.1 and 10.8, 12.4; 2048 x 2048 4.7, 5.2 and 4.2, 4.7; 1024 x
+            // 4096 6.1, 7.0 and 4.8, 5.8.  Not so 3072 x 2048 (5.0, 5.4 and 5.1, 6.3), 2560 x 6912 (10.9, 11.2 and 11.4, 14.7) and 1024 x 1024 (3.6 and
+            // 3.7).  (Rotated results are made from 16 columns.)
+            const bool pairs = !sw && !rope && N <= 2048 && K >= 2048;
             if (sw) blocks = launch_skinny<1, 1, 8, 8, true, true>(g, stream);
+            else if (pairs) blocks = M <= 8 ? launch_skinny<1, 1, 8, 4, false, true, 1>(g, stream) : launch_skinny<1, 1, 8, 4, false, true, 2>(g, stream);
             else if (N >= 65536) blocks = M <= 8 ? launch_skinny<1, 1, 8, 8, false, true>(g, stream) : launch_skinny<1, 2, 4, 8, false, true>(g, stream);
             else if (N > 4096 && K <= 8192) blocks = K > 4096 ? launch_skinny<1, 1, 4, 8, false, true>(g, stream) : launch_skinny<1, 1, 4, 4, false, true>(g, stream);
             else blocks = launch_skinny<1, 1, 8, 4, false, true>(g, stream);
             if (blocks < 0) return blocks;
-            if (norm) norm->ss_out_rows = (N + 15) / 16;
+            if (norm) norm->ss_out_rows = pairs ? (N + 7) / 8 : (N + 15) / 16;
             return XR_OK;
         }
         if (M <= 32) return rc_of(sw ? launch_skinny<2, 1, 16, 8, true>(g, stream) : launch_skinny<2, 1, 16, 8, false>(g, stream));

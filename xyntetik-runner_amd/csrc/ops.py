@@ -575,7 +575,7 @@ class Ops:
             self._dev(norm_weight)
             then = _GemmNorm()
             xg = torch.empty((M, N), dtype=torch.bfloat16, device=rows.device)
-            parts = -(-N // 16)
+            parts = -(-N // 8)
             sumsq = torch.empty((parts, 16), dtype=torch.float32, device=rows.device) if deferred else None
             then.norm_w, then.norm_w_bf16 = norm_weight.data_ptr(), dtype_code(norm_weight.dtype)
             then.xg, then.ss_out, then.ss_out_rows = xg.data_ptr(), _ptr(sumsq), parts
