@@ -1,11 +1,15 @@
-"""Products of few rows and few weight rows, whose k-steps are taken in pairs by workgroups of 8 weight rows, at the edges of their sizes."""
+"""Products of few rows at the edges of their sizes: few weight rows, whose k-steps are taken in pairs by workgroups of 8 of them, and whole
+steps of K, whose loads are a ring."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-# weight rows: fewer than a workgroup's 8, no multiple of 8 or 16, the most; columns: whole pairs of 32, an odd step at the end, a last step of 8
-@pytest.mark.parametrize("N,K", [(7, 2048), (2048, 2048), (2041, 2080), (2024, 2056), (40, 14336), (1000, 4104), (2048, 10752)])
+# pairs: weight rows: fewer than a workgroup's 8, no multiple of 8 or 16, the most; columns: whole pairs of 32, an odd step at the end, a last step
+# of 8.  Rings: one step, fewer than waves, fewer than a ring, one past it, waves with different numbers of steps; fewer than 4,096 weight
+# rows, no multiple of 16, and more; 65,536 and more.  Batches (K no whole steps) beside them.
+@pytest.mark.parametrize("N,K", [(7, 2048), (2048, 2048), (2041, 2080), (2024, 2056), (40, 14336), (1000, 4104), (2048, 10752),
+                                 (40, 32), (3000, 288), (2060, 4128), (4100, 1056), (4112, 5152), (5000, 1064), (65552, 96)])
 @pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
 def test_product(M, N, K):
     import torch
@@ -27,6 +31,13 @@ def test_product(M, N, K):
     out = c.clone()
     ops.linear(a, packed, out=out, accumulate=True)
     assert torch.equal(out, c + got)
+    if N % 32 == 0 or N in (40, 4112, 3000):                    # and gated: the first rows' gate, the others' up rows
+        F = N // 32 * 16
+        gated = ops.linear_gated(a, ops.pack_weight(w[:2 * F].contiguous(), gated=True)).double()
+        x, y = want[:, :F], want[:, F:2 * F]
+        silu, room = x / (1 + torch.exp(-x)), bound[:, :F] + bound[:, F:2 * F]
+        # (the sums' errors through the gate, whose slope is at most 1.1, and a bfloat16 rounding of 2^-9)
+        assert ((gated - silu * y).abs() <= 1.1 * room * (1 + x.abs() + y.abs()) + 2.0 ** -8 * (silu * y).abs()).all()
     # a row's result does not depend on the rows beside it, on either side of 8 rows
     assert torch.equal(ops.linear(a[:1], packed, out_dtype=torch.float32), got[:1])
     many = torch.cat([a, a[:1].expand(16 - M, K)]) if M < 16 else a

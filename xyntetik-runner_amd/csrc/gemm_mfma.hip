@@ -1184,7 +1184,9 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
 // sum and the odd ones' apart.  1 (up to 8 rows): a workgroup owns 8 weight rows, and one instruction makes both steps of a pair: rows 0 to 7 of
 // its operands are the even step's, 8 to 15 the odd one's, and what rows of one and columns of the other make is not used.  2 (9 to
 // 16 rows): 16 weight rows, the two sums in registers of their own, so that a row's result is the same either way.
-template <int MT, int RT, int KSW, int U, bool SWIGLU, bool NT, int PAIRS = 0>
+// WHOLE: K is whole steps.  Batches of U steps wait out a trip to memory each, and spend some 70 instructions on their addresses and on dropping
+// what does not exist; here the loads are a ring, with addresses that cost two instructions a step, and nothing is dropped.
+template <int MT, int RT, int KSW, int U, bool SWIGLU, bool NT, int PAIRS = 0, bool WHOLE = false>
 __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
     constexpr int NWT = SWIGLU ? 2 : 1;  // weight fragments per row group (gate and up)
     constexpr int MTOK = MT * 16, ROWS = PAIRS == 1 ? 8 : RT * 16, THREADS = 64 * KSW;
@@ -1244,52 +1246,122 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[t][r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // the first SS_AHEAD partial sums of squares of a folded norm are copied to LDS meanwhile
-    // (no registers are held for them; a wave's copy moves 16 partial rows)
-    constexpr int SS_AHEAD = 256;
+    // The rows' scales, from the partial sums the producer of `a` left: thread (part, tok) of the first 256 sums every 16th partial (16 at a
+    // time on their way before the weights), each thread of the last loop sums the 16 parts of its row; the order is the same in every
+    // instance of this kernel, so a row's scale does not depend on the batch.
     float* scale_s = red + KSW * NWT * SROWS * MTOK;       // [16 parts][16 rows]
-    float* ss_s = scale_s + 256;                          // [SS_AHEAD][16 rows]
-    if (g.ss_in) {
-        const int chunks = (g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD) * 4;      // pieces of 16 bytes
-        const uint32_t ss_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ss_s;
-        for (int c0 = wave * 64; c0 < chunks; c0 += THREADS) {
-            const int c = c0 + lane;
-            const void* src = c < chunks ? (const void*)((const char*)g.ss_in + (size_t)c * 16) : (const void*)xr_zero_chunk;
-            lds_dma16(src, __builtin_amdgcn_readfirstlane(ss_lds + (uint32_t)c0 * 16));
-        }
-    }
-
-    const uint4 zero = make_uint4(0, 0, 0, 0);
-    for (int k0 = kbeg; k0 < kend; k0 += STEP * U) {
-        uint4 wreg[U][NWT][RT], areg[U][MT];
+    float part_ss[16];
+    const bool scales = g.ss_in != nullptr && tid < 256;
+    auto fetch_ss = [&](int p0) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = k0 + u * STEP + odd * 32 + lq * 8;
-            const bool k_ok = k < kend;
-            const int ks = k_ok ? k : 0;             // a column that exists; the value is dropped
-            const size_t wo = k_ok ? (size_t)(k0 / STEP + u) * step_stride + lane_off : (size_t)dead_off;
+        for (int i = 0; i < 16; ++i) part_ss[i] = p0 + i * 16 < g.n_ss ? g.ss_in[(p0 + i * 16) * 16 + (tid & 15)] : 0.f;
+    };
+    if (scales) fetch_ss(tid >> 4);
+    auto sum_ss = [&]() {
+        if (!scales) return;
+        float s = 0.f;
+        for (int p0 = tid >> 4;;) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s += part_ss[i];
+            if ((p0 += 256) >= g.n_ss) break;
+            fetch_ss(p0);
+        }
+        scale_s[tid] = s;
+    };
+
+    if constexpr (WHOLE) {
+        // K is whole steps: a ring of U steps' loads, each on its way again as soon as its products are made, with bases that the wave shares and a
+        // fixed offset a lane.  Nothing is masked: a lane whose weight row or token does not exist reads one that does, and its
+        // results are not used; a step past the wave's last is that one once more, and not multiplied.
+        const int s0 = kbeg / STEP, s1 = kend / STEP;
+        const char* const a0 = (const char*)g.a;
+        const uint32_t a_lane = (uint32_t)(((l16 < g.M ? l16 : 0) * g.lda + odd * 32 + lq * 8) * 2);
+        const char* w0[NWT][RT];
+        uint32_t w_lane[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const int n0 = n_base + r * 16 < g.N ? n_base + r * 16 : 0;
+            const int row = n0 + l16 < g.N ? l16 : 0;
+            w_lane[r] = g.w_packed ? (uint32_t)lane_off * 2 : (uint32_t)((row * g.K + lane_off) * 2);
+#pragma unroll
+            for (int t = 0; t < NWT; ++t)
+                w0[t][r] = (const char*)(g.w + (g.w_packed ? ((size_t)(t ? g.N / 16 : 0) + n0 / 16) * kblocks * 512 : (size_t)(t ? g.N + n0 : n0) * g.K));
+        }
+        uint4 wreg[U][NWT][RT], areg[U];
+        auto load = [&](int u, int s) {
+            const size_t at = (size_t)(s < s1 ? s : s1 - 1);
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int t = 0; t < NWT; ++t)
-                    wreg[u][t][r] = keep_if(k_ok && w_ok[r], NT ? ldg16_stream(wp[t][r] + wo) : ldg16(wp[t][r] + wo));
+                for (int t = 0; t < NWT; ++t) {
+                    const bf16_t* p = (const bf16_t*)(w0[t][r] + at * (step_stride * 2) + w_lane[r]);
+                    wreg[u][t][r] = NT ? ldg16_stream(p) : ldg16(p);
+                }
+            areg[u] = ldg16((const bf16_t*)(a0 + at * (STEP * 2) + a_lane));
+        };
+        auto use = [&](int u) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i) areg[u][i] = keep_if(k_ok && a_ok[i], ldg16(ap[i] + ks));
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int t = 0; t < NWT; ++t) {
+                    f32x4& sum = acc[PAIRS == 2 ? u & 1 : t][r][0];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), as_bf16x8(areg[u]), sum, 0, 0, 0);
+                }
+        };
+        if (s0 < s1) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) load(u, s0 + u);
+            __builtin_amdgcn_sched_barrier(0);
+            sum_ss();
+            int s = s0;
+            for (; s + U < s1; s += U) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    use(u);
+                    load(u, s + U + u);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (s + u < s1) use(u);
+        } else {
+            sum_ss();
         }
-        __builtin_amdgcn_sched_barrier(0);      // every load of the batch is issued before the first use
+    } else {
+        for (int k0 = kbeg; k0 < kend; k0 += STEP * U) {
+            uint4 wreg[U][NWT][RT], areg[U][MT];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                const bf16x8 af = as_bf16x8(areg[u][i]);
+            for (int u = 0; u < U; ++u) {
+                const int k = k0 + u * STEP + odd * 32 + lq * 8;
+                const bool k_ok = k < kend;
+                const int ks = k_ok ? k : 0;             // a column that exists; the value is dropped
+                const size_t wo = k_ok ? (size_t)(k0 / STEP + u) * step_stride + lane_off : (size_t)dead_off;
 #pragma unroll
                 for (int r = 0; r < RT; ++r)
 #pragma unroll
-                    for (int t = 0; t < NWT; ++t) {
-                        f32x4& sum = acc[PAIRS == 2 ? u & 1 : t][r][i];
-                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), af, sum, 0, 0, 0);
-                    }
+                    for (int t = 0; t < NWT; ++t)
+                        wreg[u][t][r] = keep_if(k_ok && w_ok[r], NT ? ldg16_stream(wp[t][r] + wo) : ldg16(wp[t][r] + wo));
+#pragma unroll
+                for (int i = 0; i < MT; ++i) areg[u][i] = keep_if(k_ok && a_ok[i], ldg16(ap[i] + ks));
             }
+            __builtin_amdgcn_sched_barrier(0);      // every load of the batch is issued before the first use
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    const bf16x8 af = as_bf16x8(areg[u][i]);
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int t = 0; t < NWT; ++t) {
+                            f32x4& sum = acc[PAIRS == 2 ? u & 1 : t][r][i];
+                            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), af, sum, 0, 0, 0);
+                        }
+                }
+        }
+        sum_ss();
     }
 
     // acc[t][r][i][e]: weight row r*16 + 4*(lane/16) + e of the workgroup's ROWS, token i*16 + lane%16
@@ -1303,21 +1375,6 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                 for (int e = 0; e < 4; ++e)
                     red[((wave * NWT + t) * SROWS + r * 16 + lq * 4 + e) * MTOK + i * 16 + (lane & 15)] =
                         PAIRS == 2 ? acc[0][r][i][e] + acc[NSUM - 1][r][i][e] : acc[t][r][i][e];
-    // the rows' scales, from the partial sums the producer of `a` left: thread (part, tok) of the
-    // first 256 sums every 16th partial, each thread of the last loop sums the 16 parts of its
-    // row; the order is the same in every instance of this kernel, so a row's scale does not
-    // depend on the batch
-    if (g.ss_in) {
-        wait_vmcnt<0>();
-        __syncthreads();                                  // every wave's copies have landed
-        if (tid < 256) {
-            float s = 0.f;
-            const int n_lds = g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD;
-            for (int p = tid >> 4; p < n_lds; p += 16) s += ss_s[p * 16 + (tid & 15)];
-            for (int p = (tid >> 4) + SS_AHEAD; p < g.n_ss; p += 16) s += g.ss_in[p * 16 + (tid & 15)];
-            scale_s[tid] = s;
-        }
-    }
     __syncthreads();
     for (int q = tid; q < ROWS * MTOK; q += THREADS) {
         int col = q % ROWS, tok = q / ROWS;          // consecutive threads write consecutive columns
@@ -1434,13 +1491,13 @@ static int launch_tile_variant(int variant, const GemmArgs& g, hipStream_t strea
 // returns the number of workgroups, or an error (< 0)
 static inline int rc_of(int launched) { return launched < 0 ? launched : XR_OK; }
 
-template <int MT, int RT, int KSW, int U, bool SW, bool NT = false, int PAIRS = 0>
+template <int MT, int RT, int KSW, int U, bool SW, bool NT = false, int PAIRS = 0, bool WHOLE = false>
 static int launch_skinny(const GemmArgs& g, hipStream_t stream) {
     constexpr int NWT = SW ? 2 : 1;
-    size_t smem = (size_t)KSW * NWT * RT * 16 * MT * 16 * 4 + 256 * 4 + 256 * 64;    // the sums of the waves, 256 partial scales, 256 rows of partial sums
+    size_t smem = (size_t)KSW * NWT * RT * 16 * MT * 16 * 4 + 256 * 4;    // the sums of the waves, 256 partial scales
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS, WHOLE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) {
             (void)hipGetLastError();             // or the next launch's check would report this refusal
@@ -1451,7 +1508,7 @@ static int launch_skinny(const GemmArgs& g, hipStream_t stream) {
     }
     constexpr int rows = PAIRS == 1 ? 8 : 16 * RT;
     unsigned blocks = (unsigned)((g.N + rows - 1) / rows);
-    k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS><<<blocks, 64 * KSW, smem, stream>>>(g);
+    k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS, WHOLE><<<blocks, 64 * KSW, smem, stream>>>(g);
     XR_CHECK_LAUNCH("gemm_skinny");
     return (int)blocks;
 }
@@ -1757,21 +1814,40 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
     if (variant == 1) {
         XR_REQUIRE(M <= 64, "gemm: the skinny kernel takes at most 64 rows, got %d", M);
         if (M <= 16) {
-            // measured on MI355X with packed weights at M = 1, 8 and 16 (waves per workgroup, loads
-            // per batch): the output head, q/k/v, the down product, the output product.  The weights
-            // are read once, with loads marked as streaming: that alone gave 3-9% on every one of
-            // them (the head of the 8B shape at one row: 1.05 GB in 149 us, 7.1 TB/s).
+            // (waves a workgroup, loads a batch or ring.)  The weights are read once, with loads marked as streaming: that alone gave
+            // 3-9% on the head, q/k/v, the output and the down product (the head of the 8B shape at one row: 1.05 GB in 149 us, 7.1 TB/s).
             int blocks;
             // Up to 2,048 weight rows, 2,048 columns on: workgroups of 8 weight rows (one for every compute unit at 2,048).  us without and
             // with at 1 and 8 rows: 2048 x 8192 11.3, 11.5 and 8.3, 9.2; 2048 x 10752 15.5, 15.1 and 10.8, 12.4; 2048 x 2048 4.7, 5.2 and 4.2, 4.7; 1024 x
             // 4096 6.1, 7.0 and 4.8, 5.8.  Not so 3072 x 2048 (5.0, 5.4 and 5.1, 6.3), 2560 x 6912 (10.9, 11.2 and 11.4, 14.7) and 1024 x 1024 (3.6 and
             // 3.7).  (Rotated results are made from 16 columns.)
             const bool pairs = !sw && !rope && N <= 2048 && K >= 2048;
-            if (sw) blocks = launch_skinny<1, 1, 8, 8, true, true>(g, stream);
-            else if (pairs) blocks = M <= 8 ? launch_skinny<1, 1, 8, 4, false, true, 1>(g, stream) : launch_skinny<1, 1, 8, 4, false, true, 2>(g, stream);
-            else if (N >= 65536) blocks = M <= 8 ? launch_skinny<1, 1, 8, 8, false, true>(g, stream) : launch_skinny<1, 2, 4, 8, false, true>(g, stream);
-            else if (N > 4096 && K <= 8192) blocks = K > 4096 ? launch_skinny<1, 1, 4, 8, false, true>(g, stream) : launch_skinny<1, 1, 4, 4, false, true>(g, stream);
-            else blocks = launch_skinny<1, 1, 8, 4, false, true>(g, stream);
+            if (pairs) {
+                // (9 to 16 rows without the ring: 2048 x 8192 12.1 us, 12.5 with it; 2048 x 10752 15.8 and 16.8)
+                blocks = M > 8          ? launch_skinny<1, 1, 8, 4, false, true, 2>(g, stream)
+                         : K % 64 == 0  ? launch_skinny<1, 1, 8, 4, false, true, 1, true>(g, stream)
+                                        : launch_skinny<1, 1, 8, 4, false, true, 1>(g, stream);
+            } else if (K % 32 == 0) {
+                // Whole steps.  Measured in recorded decode steps, us, batches (below) and ring: gated 14336 x 4096 at 1 and 8 rows 39.4, 41.3 and 38.6,
+                // 40.0, 8192 x 2048 at one 13.4 and 12.5, 11008 x 4096 at 3 31.6 and 29.8 (four waves and a ring of 8: 39.6, 40.2; 13.4; 30.4).  Plain, four waves
+                // and a ring of 8 from 4,096 weight rows on: 4096 x 4096 8.6 and 8.3, 4096 x 11008 17.8 and 16.7, 4096 x 21504 27.2 and 26.7, 10752 x 2048 at 8
+                // rows 11.5 and 10.6, 12352 x 4096 21.8 and 20.0, 16384 x 4096 23.8 and 22.6, 21504 x 4096 30.8 and 29.8, 32000 x 4096 42.6 and 40.4;
+                // no gain, and no more than 1% lost, 6144 x 4096 and 4096 x 14336.  Fewer weight rows than that leave compute units idle, and eight waves
+                // help the others: 3072 x 2048 5.9, with four 6.4, with eight 5.8.  From 65,536 weight rows on eight waves and a ring of 8 (128256 x 2048 at one row 82 with
+                // four in a loop of its own, 75 and 77.5 in a step), and from 9 rows on two groups of weight rows a wave (at 16 rows 117 with one, 89).
+                blocks = sw            ? launch_skinny<1, 1, 8, 4, true, true, 0, true>(g, stream)
+                         : N >= 65536  ? (M > 8 ? launch_skinny<1, 2, 4, 8, false, true, 0, true>(g, stream) : launch_skinny<1, 1, 8, 8, false, true, 0, true>(g, stream))
+                         : N >= 4096   ? launch_skinny<1, 1, 4, 8, false, true, 0, true>(g, stream)
+                                       : launch_skinny<1, 1, 8, 4, false, true, 0, true>(g, stream);
+            } else if (sw) {
+                blocks = launch_skinny<1, 1, 8, 8, true, true>(g, stream);
+            } else if (N >= 65536) {
+                blocks = M <= 8 ? launch_skinny<1, 1, 8, 8, false, true>(g, stream) : launch_skinny<1, 2, 4, 8, false, true>(g, stream);
+            } else if (N > 4096 && K <= 8192) {
+                blocks = K > 4096 ? launch_skinny<1, 1, 4, 8, false, true>(g, stream) : launch_skinny<1, 1, 4, 4, false, true>(g, stream);
+            } else {
+                blocks = launch_skinny<1, 1, 8, 4, false, true>(g, stream);
+            }
             if (blocks < 0) return blocks;
             if (norm) norm->ss_out_rows = pairs ? (N + 7) / 8 : (N + 15) / 16;
             return XR_OK;
