@@ -102,12 +102,15 @@ __global__ __launch_bounds__(64) void k_attention_ref(
 // The same for 32-bit operands with the two products on the matrix cores (v_mfma_f32_16x16x4_f32: 32-bit operands, products
 // and sums).  A workgroup of four waves takes 32 rows (token x head of the group, token major) of one request and key/value
 // head and walks the keys they see in tiles of 64: keys and values through LDS, wave w the scores of keys 16 w .. 16 w + 15,
-// a softmax row a wave at a time, then wave w every fourth 16 channels of the output.  An MFMA step takes one
+// the softmax eight lanes a row, then wave w every fourth 16 channels of the output.  An MFMA step takes one
 // column from each quarter of the wave; a lane reads the four columns of its quarter at once and feeds four steps.
 // Keys that no row of the workgroup sees are never read (their pages may be gone) and count as zeros.  A tile whose values are not
 // all finite is added key by key, so that such a value shows in the rows that see it and in no other.
 // One wave a (token, head) walked the keys lane by lane, every lane a row of its own: 401 tokens, 32 heads of 64 took
-// 900 us and now 89, a decoded token of a tiny model 12 and now 7.
+// 900 us and with this kernel 90, a decoded token of a tiny model 12 and 7.  Bound by the chain of a tile's steps in the workgroups that see
+// most keys: with a softmax row a wave at a time (eight rows one after another, each with twelve exchanges) and every tile's keys read
+// when the tile before was done, 90 us; all rows' softmax at once and the next tile fetched meanwhile 60; its pieces' places by a product
+// instead of divisions, and the row blocks that see most keys first 55; the pages looked up a step ahead 48.
 #define AF_ROWS 32
 #define AF_KEYS 64
 #define AF_MAX_D 128
@@ -134,14 +137,17 @@ static inline size_t af_lds_bytes(int D, int Dv) {
     return sizeof(float) * ((size_t)(AF_ROWS + AF_KEYS) * af_ld(D) + (size_t)((Dv + 15) & ~15) * AF_LD_S + AF_ROWS * AF_LD_S);
 }
 
+// PIECES: 16-byte pieces of a tile's keys, and of its values, a thread: heads of up to 16 PIECES channels, or (FULL) keys of so many exactly.
+template <int PIECES, bool FULL>
 __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
+    constexpr int CS = (PIECES + 3) / 4;                // 16 channels of the output a wave
     extern __shared__ __align__(16) float lds[];
     __shared__ int row_pos[AF_ROWS], row_lo[AF_ROWS];
     __shared__ float row_corr[AF_ROWS], row_l[AF_ROWS], row_m[AF_ROWS];
     __shared__ int odd_tile;                            // the last tile of keys with a value that is not finite
     const int b = blockIdx.z, kvh = blockIdx.y, G = a.H / a.Hk;
     const int t0 = a.cu_q[b], nq = a.cu_q[b + 1] - t0;
-    const int r0 = blockIdx.x * AF_ROWS;                // of the request's nq * G rows
+    const int r0 = (int)(gridDim.x - 1 - blockIdx.x) * AF_ROWS;     // of the request's nq * G rows; the last ones, which see most keys, first
     const int n_rows = nq * G - r0 < AF_ROWS ? nq * G - r0 : AF_ROWS;
     if (n_rows <= 0) return;
     const int D16 = (a.D + 15) & ~15, Dv16 = (a.Dv + 15) & ~15, ldd = D16 + 4;
@@ -172,54 +178,101 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
     // positions rise with the rows, and so do the first keys
     const int lo_min = row_lo[0], lo_max = row_lo[AF_ROWS - 1], hi = row_pos[AF_ROWS - 1] + 1;
     const int kept_max = a.keep < lo_max ? a.keep : lo_max;     // first keys that stay readable behind the window
-    f32x4 acc[2][AF_MAX_D / 64];
+    f32x4 acc[2][CS];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int c = 0; c < AF_MAX_D / 64; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < CS; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int l16 = lane & 15, quad = lane >> 4;
     const int tiles = n_rows > 16 ? 2 : 1;
 
-    for (int seg = kept_max > 0 ? 0 : 1; seg < 2; ++seg) {
+    // A tile's pieces are fetched into registers while the tile before is worked on, and its keys' pages are looked up before that: a piece's
+    // place is two reads, one behind the other.
+    // (i / (D16 / 4) for i up to 2,047 and D16 / 4 up to 32, as a product: the remainder's share of 2^16 stays below one)
+    const int ck = D16 / 4;
+    const uint32_t inv_ck = (65536u + (uint32_t)ck - 1u) / (uint32_t)ck;
+    float4 pk[PIECES], pv[PIECES];
+    int page_k[PIECES], page_v[PIECES];                     // -1: nothing is read
+    auto pages = [&](int seg, int k0) {
         const int from = seg ? lo_min : 0, to = seg ? hi : kept_max;
-        for (int k0 = from & ~(AF_KEYS - 1); k0 < to; k0 += AF_KEYS) {
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int i = u * 256 + tid, j = (int)(((uint32_t)i * inv_ck) >> 16), jv = i % (AF_KEYS / 4) * 4;
+            const bool k_in = i < AF_KEYS * ck && (i - j * ck) * 4 < a.D && k0 + j >= from && k0 + j < to;
+            const bool v_in = i / (AF_KEYS / 4) < a.Dv && k0 + jv + 3 >= from && k0 + jv < to;
+            page_k[u] = k_in ? bt[(k0 + j) >> a.page_shift] : -1;
+            page_v[u] = v_in ? bt[(k0 + jv) >> a.page_shift] : -1;      // (four keys of a channel lie in one page, side by side)
+        }
+    };
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int i = u * 256 + tid, j = (int)(((uint32_t)i * inv_ck) >> 16), jv = i % (AF_KEYS / 4) * 4;
+            pk[u] = pv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (page_k[u] >= 0)
+                pk[u] = *reinterpret_cast<const float4*>(a.kc + (((size_t)page_k[u] * a.Hk + kvh) * a.page_size + ((k0 + j) & a.page_mask)) * a.D + (i - j * ck) * 4);
+            if (page_v[u] >= 0)
+                pv[u] = *reinterpret_cast<const float4*>(a.vc + (((size_t)page_v[u] * a.Hk + kvh) * a.Dv + i / (AF_KEYS / 4)) * a.page_size + ((k0 + jv) & a.page_mask));
+        }
+    };
+    int seg = kept_max > 0 ? 0 : 1, k0 = (seg ? lo_min : 0) & ~(AF_KEYS - 1);
+    pages(seg, k0);
+    fetch(k0);
+    for (;;) {
+        const int from = seg ? lo_min : 0, to = seg ? hi : kept_max;
+        int seg_next = seg, k0_next = k0 + AF_KEYS;
+        if (k0_next >= to && seg == 0) { seg_next = 1; k0_next = lo_min & ~(AF_KEYS - 1); }
+        const bool more = k0_next < (seg_next ? hi : kept_max);
+        if (more) pages(seg_next, k0_next);
+        {
             __syncthreads();                            // the tile before has been read
-            for (int i = tid; i < AF_KEYS * D16 / 4; i += 256) {
-                const int j = i / (D16 / 4), d = (i - j * (D16 / 4)) * 4, key = k0 + j;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (key >= from && key < to && d < a.D)
-                    v = *reinterpret_cast<const float4*>(a.kc + (((size_t)bt[key >> a.page_shift] * a.Hk + kvh) * a.page_size + (key & a.page_mask)) * a.D + d);
-                *reinterpret_cast<float4*>(Kt + j * ldd + d) = v;
-            }
-            for (int i = tid; i < Dv16 * (AF_KEYS / 4); i += 256) {     // four keys of a channel lie in one page, side by side
-                const int d = i / (AF_KEYS / 4), j = (i - d * (AF_KEYS / 4)) * 4, key = k0 + j;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (d < a.Dv && key + 3 >= from && key < to) {
-                    v = *reinterpret_cast<const float4*>(a.vc + (((size_t)bt[key >> a.page_shift] * a.Hk + kvh) * a.Dv + d) * a.page_size + (key & a.page_mask));
-                    if (key < from) v.x = 0.f;
+#pragma unroll
+            for (int u = 0; u < PIECES; ++u) {
+                const int i = u * 256 + tid;
+                if (i < AF_KEYS * D16 / 4) {
+                    const int j = (int)(((uint32_t)i * inv_ck) >> 16), d = (i - j * ck) * 4;
+                    *reinterpret_cast<float4*>(Kt + j * ldd + d) = pk[u];
+                }
+                if (i < Dv16 * (AF_KEYS / 4)) {
+                    const int d = i / (AF_KEYS / 4), j = (i - d * (AF_KEYS / 4)) * 4, key = k0 + j;
+                    float4 v = pv[u];
+                    if (key < from || key >= to) v.x = 0.f;
                     if (key + 1 < from || key + 1 >= to) v.y = 0.f;
                     if (key + 2 < from || key + 2 >= to) v.z = 0.f;
-                    if (key + 3 >= to) v.w = 0.f;
+                    if (key + 3 < from || key + 3 >= to) v.w = 0.f;
                     const float n = 0.f * v.x + 0.f * v.y + 0.f * v.z + 0.f * v.w;      // (0, or no number where one of them is not finite)
                     if (n != n) odd_tile = 2 * k0 + seg;
+                    *reinterpret_cast<float4*>(Vt + d * AF_LD_S + j) = v;
                 }
-                *reinterpret_cast<float4*>(Vt + d * AF_LD_S + j) = v;
             }
             __syncthreads();
+            if (more) fetch(k0_next);
             {   // scores: a lane has key 16 wave + lane % 16 and rows 4 (lane / 16) + e of each 16
                 f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
                 const float* kp = Kt + (16 * wave + l16) * ldd + 4 * quad;
                 const float* qp = Q + l16 * ldd + 4 * quad;
-                for (int d = 0; d < D16; d += 16) {
+                auto step = [&](int d) {                // (the two sums in turn: a product waits for the one before it in its own sum)
                     const float4 fk = *reinterpret_cast<const float4*>(kp + d);
                     const float4 f0 = *reinterpret_cast<const float4*>(qp + d);
+                    const float4 f1 = *reinterpret_cast<const float4*>(qp + 16 * ldd + d);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fk.x)[x], s[0], 0, 0, 0);
-                    if (tiles > 1) {
-                        const float4 f1 = *reinterpret_cast<const float4*>(qp + 16 * ldd + d);
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fk.x)[x], s[1], 0, 0, 0);
+                    for (int x = 0; x < 4; ++x) {
+                        s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fk.x)[x], s[0], 0, 0, 0);
+                        s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fk.x)[x], s[1], 0, 0, 0);
                     }
+                };
+                if (tiles == 1) {
+                    for (int d = 0; d < D16; d += 16) {
+                        const float4 fk = *reinterpret_cast<const float4*>(kp + d);
+                        const float4 f0 = *reinterpret_cast<const float4*>(qp + d);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fk.x)[x], s[0], 0, 0, 0);
+                    }
+                } else if constexpr (FULL) {
+#pragma unroll
+                    for (int d = 0; d < 16 * PIECES; d += 16) step(d);
+                } else {
+                    for (int d = 0; d < D16; d += 16) step(d);
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
@@ -227,30 +280,49 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
                     for (int e = 0; e < 4; ++e) S[(16 * i + 4 * quad + e) * AF_LD_S + 16 * wave + l16] = s[i][e];
             }
             __syncthreads();
-            // softmax: rows wave, wave + 4, ...; a lane has one key
-            const int key = k0 + lane;
+            {   // softmax: eight lanes a row, all rows at a time; a lane has keys 4 j .. 4 j + 3 of either half of the tile
+                const int r = tid >> 3, j = tid & 7;
+                float* const row = S + r * AF_LD_S + 4 * j;
+                if (r < n_rows) {
+                    const int pos = row_pos[r], lo = row_lo[r];
+                    const float slope = a.slopes ? a.slopes[kvh * G + (r0 + r) % G] : 0.f;
+                    float v[8];
+                    bool valid[8];
 #pragma unroll
-            for (int x = 0; x < AF_ROWS / 4; ++x) {
-                const int r = wave + 4 * x;
-                if (r >= n_rows) { if (r < 16 * tiles) S[r * AF_LD_S + lane] = 0.f; continue; }
-                const int pos = row_pos[r], lo = row_lo[r];
-                const bool valid = key >= from && key < to && (seg ? key >= lo && key <= pos : key < a.keep && key < lo);
-                float v = -INFINITY;
-                if (valid) {
-                    v = S[r * AF_LD_S + lane] * a.scale;
-                    if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
-                    if (a.slopes) v -= a.slopes[kvh * G + (r0 + r) % G] * (float)(pos - key);
-                }
-                const float m = row_m[r];
-                const float mn = fmaxf(m, wave_max(v));
-                const float p = valid ? expf(v - mn) : 0.f;
-                const float sum = wave_sum(p);
-                S[r * AF_LD_S + lane] = p;
-                if (lane == 0) {
-                    const float corr = m == -INFINITY ? 0.f : expf(m - mn);
-                    row_corr[r] = corr;
-                    row_l[r] = row_l[r] * corr + sum;
-                    row_m[r] = mn;
+                    for (int x = 0; x < 8; ++x) {
+                        const int key = k0 + 4 * j + (x & 3) + (x >> 2) * (AF_KEYS / 2);
+                        valid[x] = key >= from && key < to && (seg ? key >= lo && key <= pos : key < a.keep && key < lo);
+                        float y = row[(x & 3) + (x >> 2) * (AF_KEYS / 2)] * a.scale;
+                        if (a.cap > 0.f) y = a.cap * tanhf(y / a.cap);
+                        if (a.slopes) y -= slope * (float)(pos - key);
+                        v[x] = valid[x] ? y : -INFINITY;
+                    }
+                    const float m = row_m[r];
+                    float mn = v[0];
+#pragma unroll
+                    for (int x = 1; x < 8; ++x) mn = fmaxf(mn, v[x]);
+#pragma unroll
+                    for (int o = 4; o > 0; o >>= 1) mn = fmaxf(mn, __shfl_xor(mn, o, 64));
+                    mn = fmaxf(m, mn);
+                    float sum = 0.f;
+#pragma unroll
+                    for (int x = 0; x < 8; ++x) {
+                        v[x] = valid[x] ? expf(v[x] - mn) : 0.f;
+                        sum += v[x];
+                    }
+#pragma unroll
+                    for (int o = 4; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+                    *reinterpret_cast<float4*>(row) = make_float4(v[0], v[1], v[2], v[3]);
+                    *reinterpret_cast<float4*>(row + AF_KEYS / 2) = make_float4(v[4], v[5], v[6], v[7]);
+                    if (j == 0) {
+                        const float corr = m == -INFINITY ? 0.f : expf(m - mn);
+                        row_corr[r] = corr;
+                        row_l[r] = row_l[r] * corr + sum;
+                        row_m[r] = mn;
+                    }
+                } else if (r < 16 * tiles) {
+                    *reinterpret_cast<float4*>(row) = make_float4(0.f, 0.f, 0.f, 0.f);
+                    *reinterpret_cast<float4*>(row + AF_KEYS / 2) = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
             }
             __syncthreads();
@@ -260,7 +332,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) corr[i][e] = row_corr[16 * i + 4 * quad + e];
 #pragma unroll
-            for (int c = 0; c < AF_MAX_D / 64; ++c) {
+            for (int c = 0; c < CS; ++c) {
                 const int d0 = 16 * (wave + 4 * c);
                 if (d0 >= Dv16) continue;
 #pragma unroll
@@ -281,20 +353,32 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
                 }
                 const float* vp = Vt + (d0 + l16) * AF_LD_S + 4 * quad;
                 const float* pp = S + l16 * AF_LD_S + 4 * quad;
+                if (tiles == 1) {
 #pragma unroll
-                for (int k = 0; k < AF_KEYS; k += 16) {
-                    const float4 fv = *reinterpret_cast<const float4*>(vp + k);
-                    const float4 f0 = *reinterpret_cast<const float4*>(pp + k);
+                    for (int k = 0; k < AF_KEYS; k += 16) {
+                        const float4 fv = *reinterpret_cast<const float4*>(vp + k);
+                        const float4 f0 = *reinterpret_cast<const float4*>(pp + k);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fv.x)[x], acc[0][c], 0, 0, 0);
-                    if (tiles > 1) {
+                        for (int x = 0; x < 4; ++x) acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fv.x)[x], acc[0][c], 0, 0, 0);
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < AF_KEYS; k += 16) {
+                        const float4 fv = *reinterpret_cast<const float4*>(vp + k);
+                        const float4 f0 = *reinterpret_cast<const float4*>(pp + k);
                         const float4 f1 = *reinterpret_cast<const float4*>(pp + 16 * AF_LD_S + k);
 #pragma unroll
-                        for (int x = 0; x < 4; ++x) acc[1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fv.x)[x], acc[1][c], 0, 0, 0);
+                        for (int x = 0; x < 4; ++x) {
+                            acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f0.x)[x], (&fv.x)[x], acc[0][c], 0, 0, 0);
+                            acc[1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32((&f1.x)[x], (&fv.x)[x], acc[1][c], 0, 0, 0);
+                        }
                     }
                 }
             }
         }
+        if (!more) break;
+        seg = seg_next;
+        k0 = k0_next;
     }
     __syncthreads();
     // a lane has channel lane % 16 of its 16 and rows 4 (lane / 16) + e
@@ -313,7 +397,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
             }
             const float f = a.gate ? a.out_scale / (1.0f + expf(-a.gate[(size_t)t * a.ld_gate + h])) : a.out_scale;
 #pragma unroll
-            for (int c = 0; c < AF_MAX_D / 64; ++c) {
+            for (int c = 0; c < CS; ++c) {
                 const int d = 16 * (wave + 4 * c) + l16;
                 if (d < a.Dv) a.out[(size_t)t * a.ld_out + (size_t)h * a.Dv + d] = acc[i][c][e] * corr / l * f;
             }
@@ -339,16 +423,23 @@ extern "C" int xr_attention_f32(float* out, const float* q, const float* k_cache
     AttnF32 a{out, q, k_cache, v_cache, positions, cu_q, block_table, slopes, sinks, gate, table_stride, H, Hk, D, Dv, shift,
               page_size - 1, page_size, window, chunk, keep, ld_gate, ld_out, scale, cap, out_scale};
     const size_t bytes = af_lds_bytes(D, Dv);
-    if (bytes > 65536) {
-        // (the largest there is, whatever this call needs: smaller heads of another thread would take it back)
-        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)af_lds_bytes(AF_MAX_D, AF_MAX_D));
-        if (e != hipSuccess) (void)hipGetLastError();
-        XR_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
-    }
     dim3 grid((unsigned)(((long long)max_q * (H / Hk) + AF_ROWS - 1) / AF_ROWS), Hk, B);
-    k_attention_f32<<<grid, 256, bytes, stream>>>(a);
-    XR_CHECK_LAUNCH("attention_f32");
-    return XR_OK;
+    auto run = [&](auto kernel) {
+        if (bytes > 65536) {
+            // (the largest there is, whatever this call needs: smaller heads of another thread would take it back)
+            const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)af_lds_bytes(AF_MAX_D, AF_MAX_D));
+            if (e != hipSuccess) (void)hipGetLastError();
+            XR_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+        }
+        kernel<<<grid, 256, bytes, stream>>>(a);
+        XR_CHECK_LAUNCH("attention_f32");
+        return XR_OK;
+    };
+    const int widest = D > Dv ? D : Dv;
+    const int keys = (D + 15) / 16;
+    if (widest <= 16) return run(k_attention_f32<1, true>);
+    if (widest <= 64) return keys == 4 ? run(k_attention_f32<4, true>) : run(k_attention_f32<4, false>);
+    return keys == 8 ? run(k_attention_f32<8, true>) : run(k_attention_f32<8, false>);
 }
 
 extern "C" int xr_attention_ref(void* out, const void* q, const void* k_cache, const void* v_cache,
