@@ -26,6 +26,7 @@ from .batch import ATTN_MIN_RANGE, ATTN_STREAM_SLOTS, ATTN_TILE, AttentionPlan, 
 
 BUCKETS = (1, 2, 4, 8, 16, 32, 64, 128, 256, 512)
 SPLITS = (1, 2, 4, 8, 16, 32)
+ONE_RANGE_TILES = 16
 
 
 def bucket_for(n: int) -> Optional[int]:
@@ -36,7 +37,14 @@ def bucket_for(n: int) -> Optional[int]:
 
 
 def splits_for(batch_cap: int, max_tiles: int, n_kv_heads: int) -> int:
-    """Key ranges per request: one round of workgroups, and no range shorter than it pays."""
+    """Key ranges per request: one round of workgroups, and no range shorter than it pays.
+
+    Below ``ONE_RANGE_TILES`` one range, and no kernel that merges ranges: recorded steps with 8 key/value heads and 330 cached
+    tokens, two ranges and one: 1B class 765 us and 723 (4 requests 783 and 737), 8B shape 905 and 888 (16 requests 1,096 and 1,069); from
+    16 tiles on ranges gain (700 tokens 771 and 767, 1,000 tokens 767 and 799).  Measured with 8 workgroups and more; fewer are cut up
+    as before."""
+    if max_tiles < ONE_RANGE_TILES and batch_cap * n_kv_heads >= 8:
+        return 1
     want = max(1, min(ATTN_STREAM_SLOTS // (batch_cap * n_kv_heads), max_tiles // ATTN_MIN_RANGE))
     best = 1
     for s in SPLITS:
