@@ -58,6 +58,7 @@ struct RopeFuse {
     bf16_t* k_cache;
     bf16_t* v_cache;
     const float2* cs;          // [M][rot/2] (cosine, sine) of each row's angles, times mscale: set where the tile kernel rotates
+    const float2* table;       // the same, or null, where the kernel that adds K ranges up rotates
 };
 
 struct GemmArgs {
@@ -1011,6 +1012,10 @@ __global__ __launch_bounds__(256) void k_gemm_finish(GemmArgs g) {
 // RMSNorm or a layer norm: a workgroup takes a whole row, so it can also sum the squares of the updated row
 // (threads, then waves, in a fixed order) and write the normed row, times the norm's weight,
 // to xg.  N is a multiple of 4.
+// Bound by its chain of trips to memory, two of them: the ranges' sums beside the old row and the norm's weight, and the results' way out.  R: a
+// thread's groups of 4 columns, which stay in registers (rows of up to 4096 R); 0: longer rows, which are written and read again.  (All rows
+// written and read again, the weight fetched behind the row's sum: 64 rows of 4,096 in 8 ranges 5.7 us, 137 6.6, so 5.2 and 6.3.)
+template <int R>
 __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
     __shared__ float wave_sq[16];
     __shared__ float rstd_s, mean_s;
@@ -1018,8 +1023,15 @@ __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
     const size_t step = (size_t)g.M * g.N;
     float* xrow = g.post_x ? g.post_x + (size_t)m * g.post_ld : (float*)g.out + (size_t)m * g.ldo;
     const float keep = g.post_x ? g.post_alpha : 1.0f;
-    float sq = 0.f;
-    for (int n = tid * 4; n < g.N; n += 1024 * 4) {
+    constexpr int RR = R ? R : 1;
+    float4 rx[RR];
+    float rw[RR][4];
+    auto weight = [&](int n, float (&w)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = g.norm_w_bf16 ? bf16_to_f32(((const bf16_t*)g.norm_w)[n + i]) : ((const float*)g.norm_w)[n + i];
+    };
+    // the updated columns n .. n + 3, from their old values `x`
+    auto updated = [&](int n, float4 x) {
         const float* p = g.partial + (size_t)m * g.N + n;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int s0 = 0; s0 < g.splits; s0 += 8) {          // eight ranges' loads on their way at a time, summed in order
@@ -1031,10 +1043,45 @@ __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
             for (int i = 0; i < 8; ++i) { v.x += part[i].x; v.y += part[i].y; v.z += part[i].z; v.w += part[i].w; }
         }
         if (g.bias) { v.x += g.bias[n]; v.y += g.bias[n + 1]; v.z += g.bias[n + 2]; v.w += g.bias[n + 3]; }
-        float4 x = *reinterpret_cast<const float4*>(xrow + n);
-        x.x = fmaf(keep, x.x, v.x); x.y = fmaf(keep, x.y, v.y); x.z = fmaf(keep, x.z, v.z); x.w = fmaf(keep, x.w, v.w);
-        *reinterpret_cast<float4*>(xrow + n) = x;
-        sq += g.norm_centred ? x.x + x.y + x.z + x.w : x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+        return make_float4(fmaf(keep, x.x, v.x), fmaf(keep, x.y, v.y), fmaf(keep, x.z, v.z), fmaf(keep, x.w, v.w));
+    };
+    auto first_sum = [&](const float4& x) { return g.norm_centred ? x.x + x.y + x.z + x.w : x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; };
+    // f(r, n, x): the thread's columns n .. n + 3 of the updated row, its r-th
+    auto each = [&](auto f) {
+        if constexpr (R > 0) {
+#pragma unroll
+            for (int r = 0; r < RR; ++r) {
+                const int n = (r * 1024 + tid) * 4;
+                if (n < g.N) f(r, n, rx[r]);
+            }
+        } else {
+            for (int n = tid * 4; n < g.N; n += 1024 * 4) f(0, n, *reinterpret_cast<const float4*>(xrow + n));     // what this thread wrote
+        }
+    };
+    float sq = 0.f;
+    if constexpr (R > 0) {
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+            const int n = (r * 1024 + tid) * 4;
+            if (n < g.N) {
+                rx[r] = *reinterpret_cast<const float4*>(xrow + n);
+                weight(n, rw[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+            const int n = (r * 1024 + tid) * 4;
+            if (n >= g.N) continue;
+            rx[r] = updated(n, rx[r]);
+            if (!g.post_x) *reinterpret_cast<float4*>(xrow + n) = rx[r];
+            sq += first_sum(rx[r]);
+        }
+    } else {
+        for (int n = tid * 4; n < g.N; n += 1024 * 4) {
+            const float4 x = updated(n, *reinterpret_cast<const float4*>(xrow + n));
+            *reinterpret_cast<float4*>(xrow + n) = x;
+            sq += first_sum(x);
+        }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
@@ -1050,11 +1097,10 @@ __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
         __syncthreads();
         mean = mean_s;
         sq = 0.f;
-        for (int n = tid * 4; n < g.N; n += 1024 * 4) {
-            const float4 x = *reinterpret_cast<const float4*>(xrow + n);     // what this thread wrote above
+        each([&](int, int, const float4& x) {
             const float a = x.x - mean, b = x.y - mean, c = x.z - mean, d = x.w - mean;
             sq += a * a + b * b + c * c + d * d;
-        }
+        });
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
         if ((tid & 63) == 0) wave_sq[tid >> 6] = sq;
@@ -1067,15 +1113,98 @@ __global__ __launch_bounds__(1024) void k_gemm_finish_norm(GemmArgs g) {
     }
     __syncthreads();
     const float rstd = rstd_s;
-    for (int n = tid * 4; n < g.N; n += 1024 * 4) {
-        const float4 x = *reinterpret_cast<const float4*>(xrow + n);     // what this thread wrote above
+    each([&](int r, int n, const float4& x) {
         float w[4];
+        if constexpr (R > 0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            w[i] = g.norm_w_bf16 ? bf16_to_f32(((const bf16_t*)g.norm_w)[n + i]) : ((const float*)g.norm_w)[n + i];
+            for (int i = 0; i < 4; ++i) w[i] = rw[r][i];
+        } else {
+            weight(n, w);
+        }
         const float4 y = make_float4((x.x - mean) * rstd * w[0], (x.y - mean) * rstd * w[1], (x.z - mean) * rstd * w[2], (x.w - mean) * rstd * w[3]);
         if (g.post_x) *reinterpret_cast<float4*>(xrow + n) = y;
         *reinterpret_cast<uint2*>(g.xg + (size_t)m * g.N + n) = make_uint2(pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w));
+    });
+}
+
+// What k_gemm_finish does for a product that is rotated and cached, four columns a thread: 16-byte reads of the ranges' sums, queries and
+// keys stored four channels at a time, and the cosines and sines from the step's table where there is one (two calls of each a number
+// were half of the kernel's time: 137 rows of 6,144 in 6 ranges 8.0 us one column a thread, so 6.2; 64 rows 6.7 and 6.6; a prompt of 450 tokens, both kernels, 2,525 us and 2,440).  The columns of a pair, 8 apart in
+// paired order, are two lanes apart.
+__global__ __launch_bounds__(256) void k_gemm_finish_rope(GemmArgs g) {
+    const RopeFuse& rp = g.rope;
+    const uint32_t n4 = (uint32_t)g.N / 4, idx = blockIdx.x * 256 + threadIdx.x;
+    const bool ok = idx < (uint32_t)g.M * n4;
+    const int m = ok ? (int)(idx / n4) : 0, col = ok ? (int)(idx - (uint32_t)m * n4) * 4 : 0;
+    const int Q = rp.H * rp.D, KV = rp.Hk * rp.D, half = rp.rot >> 1;
+    const int sec = col < Q ? 0 : col < Q + KV ? 1 : 2;
+    const int rel = col - (sec == 0 ? 0 : sec == 1 ? Q : Q + KV), hs = rel / rp.D, c = rel - hs * rp.D;
+    const int pos = rp.positions[m];
+    const bool turns = sec < 2 && c < rp.rot;
+    const int hi = (c >> 3) & 1, j0 = (c >> 4) * 8 + (c & 7);       // (paired order)
+    float2 f[4];
+    if (turns)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = rp.interleaved ? (c + e) >> 1 : j0 + e;
+            if (rp.interleaved && c + e >= rp.rot) continue;
+            if (rp.table) {
+                f[e] = rp.table[(size_t)m * half + j];
+            } else {
+                const float ang = (float)pos * rp.inv_freq[j];
+                f[e] = make_float2(cosf(ang) * rp.mscale, sinf(ang) * rp.mscale);
+            }
+        }
+    PageRef pr{0, 0};
+    if (sec > 0) pr = page_of(rp.block_table, rp.table_stride, rp.req_of_token[m], pos, rp.page_shift, rp.page_mask);
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* p = g.partial + (size_t)m * g.N + col;
+    const size_t step = (size_t)g.M * g.N;
+    for (int s0 = 0; s0 < g.splits; s0 += 8) {
+        float4 part[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            part[i] = s0 + i < g.splits ? *reinterpret_cast<const float4*>(p + (size_t)(s0 + i) * step) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { v[0] += part[i].x; v[1] += part[i].y; v[2] += part[i].z; v[3] += part[i].w; }
+    }
+    if (g.bias)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += g.bias[col + e];
+    float o[4], other[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        o[e] = v[e];
+        other[e] = __shfl_xor(v[e], 2);
+    }
+    int d0 = c;
+    if (turns) {
+        if (rp.interleaved) {
+#pragma unroll
+            for (int e = 0; e < 4; e += 2)
+                if (c + e < rp.rot) {
+                    o[e] = v[e] * f[e].x - v[e + 1] * f[e].y;
+                    o[e + 1] = v[e] * f[e + 1].y + v[e + 1] * f[e + 1].x;
+                }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x0 = hi ? other[e] : v[e], x1 = hi ? v[e] : other[e];
+                o[e] = hi ? x0 * f[e].y + x1 * f[e].x : x0 * f[e].x - x1 * f[e].y;
+            }
+            d0 = j0 + hi * half;
+        }
+    }
+    if (!ok) return;
+    const uint2 w = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    if (sec == 0) {
+        *reinterpret_cast<uint2*>(rp.q_out + ((size_t)m * rp.H + hs) * rp.D + d0) = w;
+    } else if (sec == 1) {
+        *reinterpret_cast<uint2*>(rp.k_cache + (((size_t)pr.page * rp.Hk + hs) * rp.page_size + pr.off) * rp.D + d0) = w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            rp.v_cache[(((size_t)pr.page * rp.Hk + hs) * rp.D + c + e) * rp.page_size + pr.off] = (bf16_t)(e & 1 ? (e < 2 ? w.x : w.y) >> 16 : e < 2 ? w.x : w.y);
     }
 }
 
@@ -1162,8 +1291,14 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
         k_gemm_tile_async<BM, BN, WM_, WN_, ST, PIPE, BK><<<groups, 64 * WM_ * WN_, smem, stream>>>(g);
     XR_CHECK_LAUNCH("gemm_tile_async");
     if (g.norm_whole) {
-        k_gemm_finish_norm<<<(unsigned)g.M, 1024, 0, stream>>>(g);
+        if (g.N <= 4096) k_gemm_finish_norm<1><<<(unsigned)g.M, 1024, 0, stream>>>(g);
+        else if (g.N <= 8192) k_gemm_finish_norm<2><<<(unsigned)g.M, 1024, 0, stream>>>(g);
+        else k_gemm_finish_norm<0><<<(unsigned)g.M, 1024, 0, stream>>>(g);
         XR_CHECK_LAUNCH("gemm_finish_norm");
+    } else if (g.rope.q_out && (g.splits > 1 || g.raw) && g.N % 16 == 0 && g.rope.D % 4 == 0 && (size_t)g.M * g.N < (1ull << 31) &&
+               (((uintptr_t)g.rope.q_out | (uintptr_t)g.rope.k_cache) % 8) == 0 && (uintptr_t)g.partial % 16 == 0) {
+        k_gemm_finish_rope<<<(unsigned)(((size_t)g.M * (g.N / 4) + 255) / 256), 256, 0, stream>>>(g);
+        XR_CHECK_LAUNCH("gemm_finish_rope");
     } else if (g.splits > 1 || g.raw) {
         size_t n = (size_t)g.M * g.N;
         k_gemm_finish<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(g);
@@ -1618,7 +1753,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             }
         }
     }
-    g.rope.q_out = nullptr; g.rope.cs = nullptr;
+    g.rope.q_out = nullptr; g.rope.cs = g.rope.table = nullptr;
     // many rows: the tile kernel rotates and caches its own result, with the rows' cosines and
     // sines from a table that a small kernel writes into the workspace first; K is then not split
     // from XR_ROPE_TILE_ROWS rows on; below, the kernel that adds up the K ranges rotates and caches
@@ -1651,6 +1786,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         g.rope.mscale = rope->mscale; g.rope.page_shift = shift < 0 ? 0 : shift; g.rope.page_mask = rope->page_size - 1;
         g.rope.page_size = rope->page_size;
         g.rope.q_out = (bf16_t*)rope->q_out; g.rope.k_cache = (bf16_t*)rope->k_cache; g.rope.v_cache = (bf16_t*)rope->v_cache;
+        if (!rope_direct) g.rope.table = (const float2*)rope->cs_table;
         if (rope_direct && rope->cs_table) {
             g.rope.cs = (const float2*)rope->cs_table;      // made once for the step, for every layer with this rotation
         } else if (rope_direct) {

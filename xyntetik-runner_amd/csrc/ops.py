@@ -791,7 +791,8 @@ class Ops:
 
     def project_rope_kv_write(self, h, w, bias, k_cache, v_cache, positions, req_of_token, block_table,
                               inv_freq, H: int, Hk: int, D: int, rot: int, interleaved: bool, mscale: float,
-                              page_size: int, paired: bool = False, cs_table=None, variant: int = 0) -> torch.Tensor:
+                              page_size: int, paired: bool = False, cs_table=None, variant: int = 0,
+                              finish_table=None) -> torch.Tensor:
         """``[q | k | v] = h @ w^T (+ bias)``, queries and keys rotated, keys and values written
         to their pages; returns the rotated queries ``[T, H*D]`` in the compute dtype.
 
@@ -802,7 +803,8 @@ class Ops:
         512 the tile kernel (with the rows' cosines and sines from a table made first), which
         saves a kernel; in float32, and where the kernels' conditions on sizes do not hold, the
         product and ``rope_kv_write`` run one after the other.  ``cs_table``: a callable that returns the
-        step's ``rope_table`` (asked for only where the tile kernel rotates).  ``variant``: a tile kernel
+        step's ``rope_table`` (asked for only where the tile kernel rotates); ``finish_table``: the same for 17 to 511 rows,
+        where the kernel that adds the ranges up makes its own without one.  ``variant``: a tile kernel
         by number instead of the library's choice (tests; from 512 rows on)."""
         rows = h.data if isinstance(h, (UnscaledRows, UnnormedRows)) else h
         wt = w.data if isinstance(w, PackedWeight) else w
@@ -827,7 +829,8 @@ class Ops:
             rp.inv_freq, rp.H, rp.Hk, rp.D, rp.rot = _ptr(inv_freq), H, Hk, D, rot
             rp.interleaved, rp.mscale, rp.page_size = 1 if interleaved else 0, float(mscale), page_size
             rp.q_out, rp.k_cache, rp.v_cache = q.data_ptr(), _ptr(k_cache) if Hk else None, _ptr(v_cache) if Hk else None
-            table = cs_table() if (cs_table is not None and T >= self.ROPE_TILE_ROWS and rot > 0) else None
+            ask = cs_table if T >= self.ROPE_TILE_ROWS else finish_table if T > UnscaledRows.MAX_ROWS else None
+            table = ask() if (ask is not None and rot > 0) else None
             rp.cs_table = _ptr(table)
             self.lib.check(self.lib.xr_gemm_bf16(None, rows.data_ptr(), wt.data_ptr(), _ptr(bias), T, w.shape[0],
                                                  rows.shape[1], rows.stride(0), w.shape[0], XR_F32, 0, 0, 0.0, variant,

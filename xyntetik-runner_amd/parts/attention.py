@@ -303,11 +303,12 @@ class PagedAttention(Mixer):
                                         rot.inv_freq if rot else None, H, Hk, D, rot.rotary_dim if rot else 0,
                                         rot.interleaved if rot else False, rot.mscale if rot else 1.0, cache.page_size, rt.dtype)
         elif (self.position is None or rot is not None) and writes == (not self.kv_shared) and self.qk_transform is None:
+            step_table = (lambda: self._step_table(ctx, rot)) if rot else None
             q = ops.project_rope_kv_write(
                 h, self.w_in, self.b_in, cache.k if writes else None, cache.v if writes else None, ctx.positions,
                 ctx.req_of_token, table, rot.inv_freq if rot else None, H, Hk if writes else 0, D,
                 rot.rotary_dim if rot else 0, rot.interleaved if rot else False, rot.mscale if rot else 1.0,
-                cache.page_size, paired=self.paired, cs_table=(lambda: self._step_table(ctx, rot)) if rot else None)
+                cache.page_size, paired=self.paired, cs_table=step_table, finish_table=step_table)
         else:
             # a transform or a position encoding of its own works on the 32-bit queries and keys before
             # they are cached; or the keys and values this layer computes are another layer's to store
