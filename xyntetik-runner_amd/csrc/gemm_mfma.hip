@@ -281,121 +281,198 @@ __global__ __launch_bounds__(256) void k_rope_table(float2* cs, const int* posit
     cs[q] = make_float2(cosf(ang) * mscale, sinf(ang) * mscale);
 }
 
-// The tile kernel's way of doing what rope_store does: NT side-by-side 32x32 accumulator tiles
-// of the [query heads | key heads | value heads] product go through the wave's LDS area, and a
-// lane then has 4 consecutive columns of a row and, 8 columns away (paired order) or beside
-// them (interleaved pairs), their partners.  Queries and keys leave rotated, 4 channels a
-// store; values, cached transposed, leave 8 positions of a channel at a time where the rows
-// bring an aligned group of 8 positions of one request, else one by one.
-template <int NT>
-__device__ inline void rope_tiles(float* stage, const f32x16 (&t)[NT], const RopeFuse& rp,
-                                  int m_base, int M, int col_base, int N, int lane) {
-    constexpr int SW = 32 * NT, LD = SW + 4, CPR = SW / 4, RPI = 64 / CPR;
+// f(integral_constant<int, I>) for I = FROM .. TO-1, each call with its index a constant
+template <int FROM, int TO, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (FROM < TO) {
+        f(std::integral_constant<int, FROM>{});
+        static_for<FROM + 1, TO>(f);
+    }
+}
+
+// The tile kernel's way of doing what rope_store does, a workgroup's whole part of the [query heads | key heads | value heads] product:
+// NT side-by-side 32x32 accumulator tiles of a wave at a time go through its LDS area, and a lane then has 16 consecutive columns of a
+// row, 8 pairs in either order: a cosine and sine is read once, and an address made once, for all of them.  (With 4 columns a
+// lane, and their partners read beside them, arithmetic and LDS reads were the most of it.)  Queries and keys leave rotated, 8
+// channels a store; values, cached transposed, leave 8 positions of a channel at a time where 8 rows are
+// an aligned group of one request's positions (whatever row they begin at), else one by one.
+// With a workgroup to a compute unit nothing hides a trip to memory here, and one counter serves loads and stores: after stores that lanes may skip,
+// a load is waited for together with all of them.  So what the tiles need is fetched before the first store: the rows'
+// places in the cache, handed over between lanes, and the rows' cosines and sines, copied to LDS, all of the workgroup's where they fit beside the areas, else 32
+// rows of each wave at a time (rotary widths that fit neither way are read from memory).  Rotating products
+// cost, over plain ones in the same tiles, us: 1524 x 12288 x 4096 in 192x192 14, with 4 columns a lane and no table 35; 2048 x 6144 x 4096 in 128x256 12
+// and 35, in 256x192 12 and 14; 600 x 6144 x 4096 in 128x128 5 and 8.  (The table and early places alone gave nothing, nor did fetching one
+// step ahead.)
+template <int BM, int WARPS_M, int WARPS_N, int TM, int TN, int NT, int LDS_BYTES>
+__device__ __forceinline__ void rope_out(float* lds, const f32x16 (&acc)[TM][TN], const GemmArgs& g, int m0, int n0, int wave, int lane) {
+    constexpr int SW = 32 * NT, LD = SW + 4, CPR = SW / 16, RPI = 64 / CPR, ITS = 32 / RPI, WAVES = WARPS_M * WARPS_N, THREADS = WAVES * 64;
+    constexpr int ROOM = LDS_BYTES - WAVES * 32 * LD * 4;
+    static_assert(TN % NT == 0 && ROOM > 0, "the output areas leave no room");
+    const RopeFuse& rp = g.rope;
+    const int Q = rp.H * rp.D, KV = rp.Hk * rp.D, half = rp.rot >> 1, M = g.M, N = g.N;
     const int lr = lane & 31, lg = lane >> 5;
+    const int wave_m = wave / WARPS_N * TM * 32, m_wave = m0 + wave_m, n_wave = n0 + wave % WARPS_N * TN * 32;
+    float* const stage = lds + wave * 32 * LD;
+    float2* const tab = reinterpret_cast<float2*>(lds + WAVES * 32 * LD);
+    const int pitch = half + 2;                              // of the table's rows, in pairs: 16 bytes apart in the banks
+    const bool turns = half > 0 && n0 < Q + KV;
+    const bool whole = turns && (size_t)BM * pitch * 8 <= (size_t)ROOM, parts = turns && !whole && (size_t)WARPS_M * 32 * pitch * 8 <= (size_t)ROOM;
+    // rows [m, m + rows) of the cosines and sines, to the table's row `to` on: 32 threads a row
+    auto copy = [&](int m, int rows, int to) __attribute__((always_inline)) {
+        constexpr int RPT = THREADS / 32;
+        const int tid = wave * 64 + lane, n = m + rows < M ? rows : M - m;
+        if (half % 2 == 0 && (uintptr_t)rp.cs % 16 == 0) {
+            for (int u = tid & 31; u < half >> 1; u += 32)
+                for (int r0 = tid >> 5; r0 < n; r0 += RPT * 8) {
+                    float4 v[8];
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+                    for (int k = 0; k < 8; ++k)
+                        v[k] = reinterpret_cast<const float4*>(rp.cs + (size_t)(m + (r0 + k * RPT < n ? r0 + k * RPT : n - 1)) * half)[u];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) stage[((e / 4) * 8 + lg * 4 + (e % 4)) * LD + n * 32 + lr] = t[n][e];
-    const int Q = rp.H * rp.D, KV = rp.Hk * rp.D, half = rp.rot >> 1;
-    // values: the tiles hold columns of one section only where sections begin at multiples of 32 * NT;
-    // so every (8 rows, column) or (row, 4 columns) item asks for its own section
-    const int ch = lane % CPR, col = col_base + ch * 4;
-    if (col < Q + KV && col < N) {
-        const int sec = col < Q ? 0 : 1;
-        const int rel = col - (sec ? Q : 0);
-        const int hs = rel / rp.D, c = rel - hs * rp.D;
-        constexpr int ITS = 32 / RPI;
-        const int hi = (c >> 3) & 1, j0 = (c >> 4) * 8 + (c & 7);           // (paired order)
-        // what the rows' stores need from memory first (cosines and sines, the keys' places), then
-        // the arithmetic and the stores, four rows of the lane at a time (all eight are more
-        // registers than the eight-wave 256x256 kernel has): a load behind a store waits for that
-        // store, since they may be the same memory for all the compiler knows, and one trip to
-        // memory after the other was most of this function's time
-        constexpr int HB = ITS < 4 ? ITS : 4;
-        static_assert(ITS % HB == 0, "the lane's rows come in fours");
-#pragma unroll
-        for (int it0 = 0; it0 < ITS; it0 += HB) {
-        float2 f[HB][4];
-        size_t kdst[HB];
-#pragma unroll
-        for (int it = it0; it < it0 + HB; ++it) {
-            const int m = m_base + it * RPI + lane / CPR;
-            if (m >= M) continue;
-            if (c < rp.rot) {
-                const float2* cs = rp.cs + (size_t)m * half;
-                if (rp.interleaved) {
-#pragma unroll
-                    for (int e = 0; e < 4; e += 2)
-                        if (c + e < rp.rot) f[it - it0][e] = cs[(c + e) >> 1];
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) f[it - it0][e] = cs[j0 + e];
+                    for (int k = 0; k < 8; ++k)
+                        if (r0 + k * RPT < n) reinterpret_cast<float4*>(tab + (to + r0 + k * RPT) * pitch)[u] = v[k];
                 }
-            }
-            if (sec == 1) {
-                const PageRef pr = page_of(rp.block_table, rp.table_stride, rp.req_of_token[m], rp.positions[m], rp.page_shift, rp.page_mask);
-                kdst[it - it0] = (((size_t)pr.page * rp.Hk + hs) * rp.page_size + pr.off) * rp.D;
-            }
+        } else {
+            for (int u = tid & 31; u < half; u += 32)
+                for (int r = tid >> 5; r < n; r += RPT) tab[(to + r) * pitch + u] = rp.cs[(size_t)(m + r) * half + u];
         }
+    };
+    // lane l has the place of row l of the wave's first 64 rows, of its next 64, ..
+    int page[(TM + 1) / 2], pos[(TM + 1) / 2], req[(TM + 1) / 2];
+    const bool caches = KV > 0 && n_wave + TN * 32 > Q;
 #pragma unroll
-        for (int it = it0; it < it0 + HB; ++it) {
-            const int row = it * RPI + lane / CPR, m = m_base + row;
-            if (m >= M) continue;
-            const float4 x = *reinterpret_cast<const float4*>(stage + row * LD + ch * 4);
-            float o[4] = {x.x, x.y, x.z, x.w};
-            int d0 = c;
-            if (c < rp.rot) {
-                if (rp.interleaved) {
+    for (int s = 0; s < (TM + 1) / 2; ++s) {
+        page[s] = pos[s] = req[s] = 0;
+        if (caches) {
+            const int m = m_wave + s * 64 + lane < M ? m_wave + s * 64 + lane : M - 1;
+            pos[s] = rp.positions[m];
+            req[s] = rp.req_of_token[m];
+            page[s] = page_of(rp.block_table, rp.table_stride, req[s], pos[s], rp.page_shift, rp.page_mask).page;
+        }
+    }
+    float bias[TN];
 #pragma unroll
-                    for (int e = 0; e < 4; e += 2)
-                        if (c + e < rp.rot) {
-                            const float x0 = o[e], x1 = o[e + 1];
-                            o[e] = x0 * f[it - it0][e].x - x1 * f[it - it0][e].y;
-                            o[e + 1] = x0 * f[it - it0][e].y + x1 * f[it - it0][e].x;
+    for (int j = 0; j < TN; ++j) bias[j] = g.bias && n_wave + j * 32 + lr < N ? g.bias[n_wave + j * 32 + lr] : 0.f;
+    // the 16 columns of this lane in each of its tiles: which head's, and where in the head
+    int head[TN / NT], chan[TN / NT];
+#pragma unroll
+    for (int j = 0; j < TN / NT; ++j) {
+        const int col = n_wave + j * SW + lane % CPR * 16, rel = col < Q ? col : col - Q;
+        head[j] = rel / rp.D;
+        chan[j] = rel - head[j] * rp.D;
+    }
+    if (whole) {
+        copy(m0, BM, 0);
+        __syncthreads();
+    }
+    static_for<0, TM * (TN / NT)>([&](auto idx) {
+        constexpr int i = decltype(idx)::value / (TN / NT), j = decltype(idx)::value % (TN / NT) * NT;
+        const int col_base = n_wave + j * 32;
+        if (j == 0 && parts) {
+            if (i > 0) __syncthreads();
+#pragma unroll
+            for (int w = 0; w < WARPS_M; ++w) copy(m0 + (w * TM + i) * 32, 32, w * 32);
+            __syncthreads();
+        }
+        const int tab_row = whole ? wave_m + i * 32 : wave / WARPS_N * 32;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)                         // (a wave's LDS accesses are served in order)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) stage[((e / 4) * 8 + lg * 4 + (e % 4)) * LD + n * 32 + lr] = acc[i][j + n][e] + bias[j + n];
+        const int col = col_base + lane % CPR * 16, hs = head[j / NT], c = chan[j / NT];
+        const bool mine = col < Q + KV && col < N, key = col >= Q, turned = mine && c < rp.rot, paired = turned && !rp.interleaved;
+        if (col_base < Q + KV)
+#pragma unroll
+            for (int it = 0; it < ITS; ++it) {
+                const int row = it * RPI + lane / CPR, m = m_wave + i * 32 + row, from = (i & 1) * 32 + row;
+                const int pg = caches ? __shfl(page[i / 2], from) : 0;       // (exchanges between all lanes, whatever their columns)
+                const int of = caches ? __shfl(pos[i / 2], from) & rp.page_mask : 0;
+                float x[16], f[16];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float4 v = *reinterpret_cast<const float4*>(stage + row * LD + lane % CPR * 16 + k * 4);
+                    x[k * 4] = v.x; x[k * 4 + 1] = v.y; x[k * 4 + 2] = v.z; x[k * 4 + 3] = v.w;
+                }
+                if (turned) {
+                    // pairs c / 2 .. + 7 in either order; of a head's last rotated pairs there may be fewer (interleaved)
+                    const int left = (rp.rot - c) >> 1;
+                    if (whole || parts) {
+                        const float2* t = tab + (tab_row + row) * pitch + (c >> 1);
+                        if (half % 8 == 0) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                const float4 v = *reinterpret_cast<const float4*>(t + k * 2);
+                                f[k * 4] = v.x; f[k * 4 + 1] = v.y; f[k * 4 + 2] = v.z; f[k * 4 + 3] = v.w;
+                            }
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) {
+                                const float2 v = t[k < left ? k : left - 1];
+                                f[k * 2] = v.x; f[k * 2 + 1] = v.y;
+                            }
                         }
-                } else {
-                    const float4 y = *reinterpret_cast<const float4*>(stage + row * LD + (ch ^ 2) * 4);
-                    const float pv[4] = {y.x, y.y, y.z, y.w};
+                    } else {
+                        const float2* t = rp.cs + (size_t)(m < M ? m : M - 1) * half + (c >> 1);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float x0 = hi ? pv[e] : o[e], x1 = hi ? o[e] : pv[e];
-                        o[e] = hi ? x0 * f[it - it0][e].y + x1 * f[it - it0][e].x : x0 * f[it - it0][e].x - x1 * f[it - it0][e].y;
+                        for (int k = 0; k < 8; ++k) {
+                            const float2 v = t[k < left ? k : left - 1];
+                            f[k * 2] = v.x; f[k * 2 + 1] = v.y;
+                        }
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) asm volatile("" : "+v"(f[k]));      // (waited for here, so that the other way does not wait)
                     }
-                    d0 = j0 + hi * half;
-                }
-            }
-            const uint2 w = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-            if (sec == 0) *reinterpret_cast<uint2*>(rp.q_out + ((size_t)m * rp.H + hs) * rp.D + d0) = w;
-            else *reinterpret_cast<uint2*>(rp.k_cache + kdst[it - it0] + d0) = w;
-        }
-        }
-    }
-    if (col_base + SW > Q + KV && KV > 0) {
-        // value columns: items are (group of 8 rows, column)
-        for (int q = lane; q < 4 * SW; q += 64) {
-            const int grp = q / SW, cc = q - grp * SW, vcol = col_base + cc;
-            const int m8 = m_base + grp * 8;
-            if (vcol < Q + KV || vcol >= N || m8 >= M) continue;
-            const int rel = vcol - Q - KV, hs = rel / rp.D, d = rel - hs * rp.D;
-            const int pos = rp.positions[m8], req = rp.req_of_token[m8];
-            const bool whole = rp.page_size >= 8 && (pos & 7) == 0 && m8 + 7 < M && rp.req_of_token[m8 + 7] == req &&
-                               rp.positions[m8 + 7] == pos + 7;
-            if (whole) {
-                const PageRef pr = page_of(rp.block_table, rp.table_stride, req, pos, rp.page_shift, rp.page_mask);
-                float v[8];
+                    if (rp.interleaved) {
 #pragma unroll
-                for (int r = 0; r < 8; ++r) v[r] = stage[(grp * 8 + r) * LD + cc];
-                *reinterpret_cast<uint4*>(rp.v_cache + (((size_t)pr.page * rp.Hk + hs) * rp.D + d) * rp.page_size + pr.off) =
-                    make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-            } else {
-                for (int r = 0; r < 8 && m8 + r < M; ++r) {
-                    const int p = rp.positions[m8 + r];
-                    const PageRef pr = page_of(rp.block_table, rp.table_stride, rp.req_of_token[m8 + r], p, rp.page_shift, rp.page_mask);
-                    rp.v_cache[(((size_t)pr.page * rp.Hk + hs) * rp.D + d) * rp.page_size + pr.off] = f32_to_bf16(stage[(grp * 8 + r) * LD + cc]);
+                        for (int k = 0; k < 8; ++k) {
+                            const float x0 = x[k * 2], x1 = x[k * 2 + 1];
+                            x[k * 2] = k < left ? x0 * f[k * 2] - x1 * f[k * 2 + 1] : x0;
+                            x[k * 2 + 1] = k < left ? x0 * f[k * 2 + 1] + x1 * f[k * 2] : x1;
+                        }
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const float x0 = x[k], x1 = x[8 + k];
+                            x[k] = x0 * f[k * 2] - x1 * f[k * 2 + 1];
+                            x[8 + k] = x0 * f[k * 2 + 1] + x1 * f[k * 2];
+                        }
+                    }
+                }
+                // (products of two 32-bit numbers: a page's place, and a row's)
+                bf16_t* at = key ? rp.k_cache + (uint64_t)(uint32_t)pg * (uint32_t)(KV * rp.page_size) + (uint32_t)((hs * rp.page_size + of) * rp.D)
+                                 : rp.q_out + (uint64_t)(uint32_t)m * (uint32_t)Q + (uint32_t)(hs * rp.D);
+                const int d0 = paired ? c >> 1 : c, d1 = paired ? d0 + half : c + 8;
+                if (mine && m < M) {
+                    *reinterpret_cast<uint4*>(at + d0) = make_uint4(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]), pack_bf16x2(x[6], x[7]));
+                    *reinterpret_cast<uint4*>(at + d1) = make_uint4(pack_bf16x2(x[8], x[9]), pack_bf16x2(x[10], x[11]), pack_bf16x2(x[12], x[13]), pack_bf16x2(x[14], x[15]));
+                }
+            }
+        if (KV > 0 && col_base + SW > Q + KV) {
+            // value columns: items are (8 rows, column), the first of them ending where the first row's request has an aligned position
+            const int first = -(__shfl(pos[i / 2], (i & 1) * 32) & 7);
+            for (int r0 = first; r0 < 32; r0 += 2 * 8 / NT) {
+                const int r8 = r0 + (NT == 1 ? lane / SW * 8 : 0), cc = lane % SW, vcol = col_base + cc;
+                const int lo = r8 > 0 ? r8 : 0, up = r8 + 7 < 31 ? r8 + 7 : 31, m_lo = m_wave + i * 32 + lo, m_up = m_wave + i * 32 + up;
+                const int p0 = __shfl(pos[i / 2], (i & 1) * 32 + (lo & 31)), p7 = __shfl(pos[i / 2], (i & 1) * 32 + up);
+                const int q0 = __shfl(req[i / 2], (i & 1) * 32 + (lo & 31)), q7 = __shfl(req[i / 2], (i & 1) * 32 + up);
+                const int pg = __shfl(page[i / 2], (i & 1) * 32 + (lo & 31));
+                if (vcol < Q + KV || vcol >= N || lo > 31 || m_lo >= M) continue;
+                const int rel_v = vcol - Q - KV, hv = rel_v / rp.D, d = rel_v - hv * rp.D;
+                if (rp.page_size >= 8 && up - lo == 7 && (p0 & 7) == 0 && m_up < M && q7 == q0 && p7 == p0 + 7) {
+                    float v[8];
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) v[r] = stage[(lo + r) * LD + cc];
+                    *reinterpret_cast<uint4*>(rp.v_cache + (((size_t)pg * rp.Hk + hv) * rp.D + d) * rp.page_size + (p0 & rp.page_mask)) =
+                        make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+                } else {
+                    for (int r = lo; r <= up && m_wave + i * 32 + r < M; ++r) {
+                        const int m = m_wave + i * 32 + r;
+                        const PageRef pr = page_of(rp.block_table, rp.table_stride, rp.req_of_token[m], rp.positions[m], rp.page_shift, rp.page_mask);
+                        rp.v_cache[(((size_t)pr.page * rp.Hk + hv) * rp.D + d) * rp.page_size + pr.off] = f32_to_bf16(stage[r * LD + cc]);
+                    }
                 }
             }
         }
-    }
+    });
 }
 
 // ------------------------------------------------------------------------------ tile kernel
@@ -441,15 +518,6 @@ __device__ inline int w_row_of(int r, int bx, int N, int epi, int& out_col) {
 template <int CH> __device__ inline int swz(int r) {
     static_assert(CH == 8 || CH == 4, "rows of 8 or of 4 chunks");
     return CH == 8 ? (r >> 1) & 7 : (r >> 2) & 3;
-}
-
-// f(integral_constant<int, I>) for I = FROM .. TO-1, each call with its index a constant
-template <int FROM, int TO, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (FROM < TO) {
-        f(std::integral_constant<int, FROM>{});
-        static_for<FROM + 1, TO>(f);
-    }
 }
 
 // waits until at most `slices` slices of LOADS copies each are still on their way (a number the
@@ -917,11 +985,17 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
             }
         return;
     }
-    if (g.vec_out || rotate) {
+    if (rotate) {
+        constexpr int LDS_BYTES = STAGES * BUF * 16;         // (two tiles at a time where 64 pairs of 32 rows of each wave fit beside them)
+        constexpr int NTR = NTP == 2 && WAVES * STAGE_FLOATS * 4 + WARPS_M * 32 * (64 + 2) * 8 <= LDS_BYTES ? 2 : 1;
+        rope_out<BM, WARPS_M, WARPS_N, TM, TN, NTR, LDS_BYTES>(reinterpret_cast<float*>(lds), acc, g, m0, bx * BN, wave, lane);
+        return;
+    }
+    if (g.vec_out) {
         // (tile by tile through a recursion of templates: a loop that the compiler declines to unroll,
         // as it does one with 16 rotations in it, would index the accumulators at run time, and
         // they would live in memory)
-        const bool adding = !rotate && g.epi == EPI_ACCUM;
+        const bool adding = g.epi == EPI_ACCUM;
         float4 old[2][4 * NTP];                     // what the tiles of this round and of the next are added to
         if (adding) load_old<NTP>(old[0], g.out, g.ldo, m0 + wm0, g.M, bx * BN + wn0, g.N, lane);
         static_for<0, TM * (TN / NTP)>([&](auto idx) {
@@ -937,11 +1011,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const int item, uin
 #pragma unroll
                 for (int e = 0; e < 16; ++e) t[n][e] = acc[i][j + n][e] + b;
             }
-            if (rotate)
-                rope_tiles<NTP>(stage, t, g.rope, m0 + wm0 + i * 32, g.M, bx * BN + wn0 + j * 32, g.N, lane);
-            else
-                write_tiles<NTP>(stage, t, g.out, g.ldo, g.epi == EPI_ACCUM ? 1 : (g.out_bf16 ? 2 : 0) + (g.act == XR_POST_RELU2 && g.epi == EPI_STORE ? 4 : 0),
-                                 m0 + wm0 + i * 32, g.M, bx * BN + wn0 + j * 32, g.N, lane, adding ? old[decltype(idx)::value & 1] : nullptr);
+            write_tiles<NTP>(stage, t, g.out, g.ldo, g.epi == EPI_ACCUM ? 1 : (g.out_bf16 ? 2 : 0) + (g.act == XR_POST_RELU2 && g.epi == EPI_STORE ? 4 : 0),
+                             m0 + wm0 + i * 32, g.M, bx * BN + wn0 + j * 32, g.N, lane, adding ? old[decltype(idx)::value & 1] : nullptr);
         });
         return;
     }
@@ -1859,7 +1930,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // rows, 1 to 16 ranges; plain, gated, added up, added up and normed; weights from memory, and from the caches where they are small):
             // the tile and ranges chosen are 0.9% slower on average than the best of all eight tiles (1.2% for products left out of a fit); with
             // numbers fitted to fewer and wider products, without `round`, `else_rate` and 256x192 tiles, it was 3.0%, at worst 47%.  Rotating
-            // ones: 350 products of fifteen shapes, 512 to 4,096 rows, 0.1% (0.2%); fitted to three shapes it was 6.3%, at worst 73%.
+            // ones: 153 products of nine shapes, 512 to 4,096 rows, 0.4% (0.6%), at worst 11% (2,048 weight rows of 1,536 columns); with the numbers
+            // that fitted the rotation of 4 columns a lane 2.4%, at worst 17%.
             // Of the tiles that were left out none brings 0.2% on average:
             // 192x256, 256x192 and 128x192 with four waves, 320x192, 320x128, 96x256, and a fifth or sixth slice in flight.
             // (Rotating products in 256x256, 256x192 and 256x128 tiles: the eight-wave kernels.)
@@ -1869,14 +1941,14 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                                   {27, 192, 192, 3, true, 1.048, 1.048, 6.25e-6, 3.40e-6, 2.75e12}, {12, 256, 128, 3, false, 0.953, 0.835, 4.07e-6, 3.37e-6, 5.82e12},
                                   {29, 160, 256, 3, true, 1.103, 1.103, 4.48e-6, 4.32e-6, 10.10e12}, {16, 128, 256, 3, true, 0.924, 0.924, 5.22e-6, 3.17e-6, 11.30e12},
                                   {28, 192, 128, 3, true, 0.862, 0.862, 1.64e-6, 4.30e-6, 8.12e12}, {17, 128, 128, 4, false, 0.623, 0.449, 2.96e-6, 2.32e-6, 8.13e12}};
-            const Cand turning[] = {{14, 256, 256, 0, false, 0.929, 0.929, 3.33e-6, 16.3e-6, 6.04e12}, {26, 256, 192, 0, false, 0.743, 0.743, 1.31e-6, 2.95e-6, 12.1e12},
-                                    {27, 192, 192, 3, true, 0.934, 0.934, 0.56e-6, 20.7e-6, 15.6e12},  {12, 256, 128, 0, false, 0.715, 0.715, 1.24e-6, 2.64e-6, 2.65e12},
-                                    {29, 160, 256, 3, true, 0.927, 0.927, 1.97e-6, 15.8e-6, 5.75e12},  {16, 128, 256, 3, true, 0.849, 0.849, 1.80e-6, 18.1e-6, 7.27e12},
-                                    {28, 192, 128, 3, true, 0.855, 0.855, 2.01e-6, 14.3e-6, 9.94e12},  {17, 128, 128, 0, false, 0.661, 0.661, 3.23e-6, 6.19e-6, 8.21e12}};
+            const Cand turning[] = {{14, 256, 256, 0, false, 0.926, 0.926, 5.08e-6, 15.4e-6, 6.04e12}, {26, 256, 192, 0, false, 0.843, 0.843, 6.15e-6, 12.1e-6, 12.1e12},
+                                    {27, 192, 192, 3, true, 1.030, 1.030, 3.02e-6, 16.8e-6, 15.6e12},  {12, 256, 128, 0, false, 0.836, 0.836, 3.30e-6, 11.8e-6, 2.65e12},
+                                    {29, 160, 256, 3, true, 1.010, 1.010, 4.46e-6, 13.3e-6, 5.75e12},  {16, 128, 256, 3, true, 0.953, 0.953, 3.90e-6, 10.8e-6, 7.27e12},
+                                    {28, 192, 128, 3, true, 0.895, 0.895, 4.16e-6, 11.3e-6, 9.94e12},  {17, 128, 128, 0, false, 0.772, 0.772, 4.26e-6, 6.60e-6, 8.21e12}};
             constexpr int n_cands = sizeof(plain) / sizeof(Cand);
             static_assert(sizeof(turning) == sizeof(plain), "as many tiles");
             const Cand* cands = rope_direct ? turning : plain;
-            const double emptier = rope_direct ? 0.034 : 0.082;
+            const double emptier = rope_direct ? 0.526 : 0.082;
             auto width = [&](const Cand& c) { return sw ? c.bn / 2 : c.bn; };
             auto written = [&](const Cand& c, int ranges) {
                 int r = ranges;
