@@ -15,3 +15,30 @@ pytestmark = pytest.mark.gpu
                                                  (2, 1, 64, 6, True, 16), (2, 2, 96, 16, False, 32), (2, 1, 64, 0, False, 16)])
 def test_tables_and_row_groups(ops, variant, H, Hk, D, rot, inter, ps):      # noqa: F811
     check_projection_with_rotation_and_cache_write(ops, "bfloat16", H, Hk, D, rot, inter, ps, [3, 0, 7], [257, 11, 250], D == 96, 256, variant=variant)
+
+
+def test_keys_that_are_not_16_byte_aligned(ops):      # noqa: F811
+    """Tiles store 8 channels at a time; a cache that begins 8 bytes later takes the product and the rotation's own kernel."""
+    import torch
+    from test_kernels_gpu import DEV, FakeCtx, scatter_pages
+    torch.manual_seed(5)
+    H, Hk, D, ps, T = 2, 1, 64, 16, 520
+    tables, n_pages = scatter_pages([T], ps, 2)
+    ctx = FakeCtx([0], [T], tables, ps)
+    h = torch.randn(T, 256, device=DEV).bfloat16()
+    w = ops.pack_weight((torch.randn((H + 2 * Hk) * D, 256, device=DEV) * 0.1).bfloat16())
+    inv = (10000.0 ** (-torch.arange(D // 2, dtype=torch.float64) * 2 / D)).float().to(DEV)
+    results = []
+    for shift, fuse in ((0, False), (4, True)):
+        size = n_pages * Hk * ps * D
+        kc = torch.full((size + 8,), 7.0, device=DEV, dtype=torch.bfloat16)[shift:shift + size].view(n_pages, Hk, ps, D)
+        vc = torch.full((n_pages, Hk, D, ps), 7.0, device=DEV, dtype=torch.bfloat16)
+        assert kc.data_ptr() % 16 == 2 * shift
+        ops.fuse_rope = fuse
+        try:
+            q = ops.project_rope_kv_write(h, w, None, kc, vc, ctx.positions, ctx.req_of_token, ctx.block_table(0), inv, H, Hk, D, D, False, 1.0, ps,
+                                          paired=True)
+        finally:
+            ops.fuse_rope = True
+        results.append((q, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*results))

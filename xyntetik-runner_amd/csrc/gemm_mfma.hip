@@ -1835,7 +1835,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         if (rope_direct) {
             XR_REQUIRE(rope->cs_table || (workspace && (size_t)M * (rope->rot / 2 + 1) * sizeof(float2) <= workspace_bytes),
                        "gemm: rotation after a product of %d rows needs a workspace for its table", M);
-            XR_REQUIRE(((uintptr_t)rope->q_out % 8) == 0 && ((uintptr_t)rope->k_cache % 8) == 0 && ((uintptr_t)rope->v_cache % 16) == 0,
+            XR_REQUIRE(((uintptr_t)rope->q_out % 16) == 0 && ((uintptr_t)rope->k_cache % 16) == 0 && ((uintptr_t)rope->v_cache % 16) == 0,
                        "gemm: queries and caches must be 16-byte aligned");
         } else if (M > 16) {
             XR_REQUIRE(workspace && (size_t)M * N * 4 <= workspace_bytes, "gemm: rotation after a product of %d rows needs a workspace", M);

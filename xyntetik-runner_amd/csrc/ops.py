@@ -815,6 +815,7 @@ class Ops:
         if (self.fuse_rope and (T <= self.FINISH_ROWS or T >= self.ROPE_TILE_ROWS) and self._mfma_ok(rows, wt) and D % 16 == 0
                 and (T * w.shape[0] * 4 if T <= self.FINISH_ROWS else T * (rot // 2 + 1) * 8) <= self.GEMM_WORKSPACE_BYTES
                 and (Hk == 0 or (k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16))
+                and (T < self.ROPE_TILE_ROWS or Hk == 0 or k_cache.data_ptr() % 16 == 0)       # (tiles store 8 channels at a time)
                 and (rot == 0 or interleaved or (paired and rot % 16 == 0))):
             self._dev(rows, wt, bias, k_cache, v_cache, positions, req_of_token, block_table, inv_freq)
             self._contig(wt, "projection weight")
