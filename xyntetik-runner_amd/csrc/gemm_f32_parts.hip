@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
     fold();
 
     // Results that are not finite, or so small that parts may have fallen out of bfloat16's range (a number's last part below 2^-126 is lost, so
-    // 2^-126 times the other operands: nothing beside 2^-60), are made again from 32-bit products, a wave's 32 x 32 at a time: an infinity
+    // 2^-126 times the other operands: nothing beside 2^-60 while those are below 2^40), are made again from 32-bit products, a wave's 32 x 32 at a time: an infinity
     // stays one, whatever it meets, and an overflow happens where it did.  (Where every tile is made again, a product takes three times as long.)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -298,16 +298,17 @@ static int launch_parts(void* out, const float* a, const float* w, const float* 
     const long long items = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN) * ranges;
     XR_REQUIRE(items < (1ll << 28), "gemm: %lld tiles", items);
     const unsigned blocks = 8 * (unsigned)((items + 7) / 8);
-    auto run = [&](auto kernel, auto finish, auto* to) {
-        static bool attr_set = false;
-        if (!attr_set) {
+    // `which`: the kernel's number (that adds to its output and that stores it are of one type, and so share this function's statics)
+    auto run = [&](auto kernel, auto finish, auto* to, int which) {
+        static bool attr_set[3] = {};
+        if (!attr_set[which]) {
             const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
             if (e != hipSuccess) {
                 (void)hipGetLastError();             // or the next launch's check would report this refusal
                 xr_set_error("gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
                 return XR_LAUNCH;
             }
-            attr_set = true;
+            attr_set[which] = true;
         }
         kernel<<<blocks, 64 * GM * GN, smem, stream>>>(to, a, w, bias, M, N, K, lda, ldo, ranges, per, partial);
         XR_CHECK_LAUNCH("gemm_f32_parts");
@@ -317,9 +318,9 @@ static int launch_parts(void* out, const float* a, const float* w, const float* 
         }
         return XR_OK;
     };
-    if (out_dtype == XR_BF16) return run(k_gemm_f32_parts<bf16_t, false, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<bf16_t, false>, (bf16_t*)out);
-    if (accumulate) return run(k_gemm_f32_parts<float, true, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<float, true>, (float*)out);
-    return run(k_gemm_f32_parts<float, false, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<float, false>, (float*)out);
+    if (out_dtype == XR_BF16) return run(k_gemm_f32_parts<bf16_t, false, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<bf16_t, false>, (bf16_t*)out, 0);
+    if (accumulate) return run(k_gemm_f32_parts<float, true, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<float, true>, (float*)out, 1);
+    return run(k_gemm_f32_parts<float, false, GM, GN, TM, TN, MW, PF>, k_gemm_f32_ranges<float, false>, (float*)out, 2);
 }
 
 #define XR_PARTS_TILES 4
