@@ -87,6 +87,26 @@ def test_numbers_at_the_ends_of_the_range(tile, ranges):
     assert ((got.double() - want.double()).abs()[fin] <= (80 * U * size + K * 2.0 ** -149)[fin]).all()     # (a product below 2^-126 rounds to 2^-149)
 
 
+@pytest.mark.parametrize("ranges", [1, 3])
+@pytest.mark.parametrize("tile", range(TILES))
+def test_a_result_depends_on_its_own_row_and_column(tile, ranges):
+    """What is no ordinary number in some rows and weight rows (an infinity, a NaN, an overflow, tiny numbers, zeros) changes no bit elsewhere."""
+    import torch
+    M, N, K = 140, 150, 576
+    ops, a, w, _, _ = operands(M, N, K)
+    want = ops.linear(a, w, variant=plan(tile, ranges))
+    odd, odd_w = a.clone(), w.as_subclass(torch.Tensor).clone()
+    odd[0, 5], odd[37, 70], odd[70, 300], odd[139, K - 1] = float("inf"), float("nan"), 3.4e38, float("-inf")
+    odd[64] *= 1e-30
+    odd[100] = 0.0
+    odd_w[3, 9], odd_w[149, 0] = float("inf"), float("nan")
+    odd_w[90] *= 1e-30
+    got = ops.linear(odd, odd_w.as_subclass(type(w)), variant=plan(tile, ranges))
+    rows = [m for m in range(M) if m not in (0, 37, 64, 70, 100, 139)]
+    cols = [n for n in range(N) if n not in (3, 90, 149)]
+    assert torch.equal(got[rows][:, cols], want[rows][:, cols])
+
+
 def test_products_that_stay_with_the_32_bit_instructions():
     import torch
     from xyntetik_runner_amd.csrc.ops import F32Weight, load_ops

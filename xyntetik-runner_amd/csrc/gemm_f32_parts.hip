@@ -195,19 +195,20 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
 
     // Results that are not finite, or so small that parts may have fallen out of bfloat16's range (a number's last part below 2^-126 is lost, so
     // 2^-126 times the other operands: nothing beside 2^-60 while those are below 2^40), are made again from 32-bit products, a wave's 32 x 32 at a time: an infinity
-    // stays one, whatever it meets, and an overflow happens where it did.  (Where every tile is made again, a product takes three times as long.)
+    // stays one, whatever it meets, and an overflow happens where it did.  The others of the 32 x 32 stay as they are: a result depends on its own row
+    // and column alone.  (Where every tile is made again, a product takes three times as long.)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int n = n0 + wn + 32 * j + row, mb = m0 + wm + 32 * i + 4 * (lane >> 5);
-            bool bad = false;
+            uint32_t bad = 0;                               // a bit for each of the lane's 16
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const float v = fabsf(tot[i][j][e] + low[i][j][e]);
-                bad = bad || (mb + 8 * (e >> 2) + (e & 3) < M && !((v >= 0x1p-60f && v <= 3.402823466e38f) || v == 0.f));
+                if (n < N && mb + 8 * (e >> 2) + (e & 3) < M && !((v >= 0x1p-60f && v <= 3.402823466e38f) || v == 0.f)) bad |= 1u << e;
             }
-            if (__any(bad && n < N)) {
+            if (__any(bad != 0)) {
                 const float* const x = a + (size_t)min(m0 + wm + 32 * i + row, M - 1) * lda + 4 * (lane >> 5);
                 const float* const y = w + (size_t)min(n, N - 1) * K + 4 * (lane >> 5);
                 f32x16 acc{}, t{}, lost{};
@@ -226,9 +227,11 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
                             acc[e] = 0.f;
                         }
                 }
-                tot[i][j] = t;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) low[i][j][e] = -lost[e];
+                for (int e = 0; e < 16; ++e) {
+                    tot[i][j][e] = bad >> e & 1 ? t[e] : tot[i][j][e];
+                    low[i][j][e] = bad >> e & 1 ? -lost[e] : low[i][j][e];
+                }
             }
         }
     // a lane has column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a tile
