@@ -107,6 +107,32 @@ def test_a_result_depends_on_its_own_row_and_column(tile, ranges):
     assert torch.equal(got[rows][:, cols], want[rows][:, cols])
 
 
+@pytest.mark.parametrize("ranges", [1, 3])
+@pytest.mark.parametrize("tile", range(TILES))
+def test_tiny_numbers_that_meet_large_ones(tile, ranges):
+    """Numbers whose parts are below bfloat16's range count where the others are large: every bit of them, as with 32-bit products."""
+    import torch
+    M, N, K = 140, 150, 576
+    ops, a, w, _, _ = operands(M, N, K)
+    a, w = a.clone(), w.as_subclass(torch.Tensor).clone()
+    a[20:23] *= torch.tensor([1e-36, 1e-34, 1e-30], device=a.device)[:, None]
+    a[23, : K // 2], a[23, K // 2:] = a[23, : K // 2] * 1e-37, 0.0          # tiny ones alone, in some ranges nothing else
+    a[24], a[25] = 2.0 ** -140, 0.0
+    w[100:104] *= torch.tensor([1e35, 1e30, 1e20, 1e8], device=a.device)[:, None]
+    w[104], w[105] = w[104] * 1e-35, 0.0
+    a[40:42] *= 1e33
+    w = w.as_subclass(type(ops.pack_weight(w)))
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got, usual = (ops.linear(a, w, variant=v) for v in (plan(tile, ranges), 40))
+    # (as for ordinary numbers; a product below 2^-126 rounds to 2^-149; rows of numbers below 2^-126 are what 32-bit instructions make of them)
+    bound = 40 * U * size + K * 2.0 ** -149
+    fits = size < 1e38
+    fits[24] = False
+    assert ((got.double() - want).abs() <= bound)[fits].all() and torch.equal(got.isfinite() | fits, usual.isfinite() | fits)
+    assert torch.equal(got[24] == 0, usual[24] == 0) and ((got[24] - usual[24]).double().abs() <= bound[24]).all()
+    assert (got[25] == 0).all() and (got[:, 105] == 0).all()
+
+
 def test_products_that_stay_with_the_32_bit_instructions():
     import torch
     from xyntetik_runner_amd.csrc.ops import F32Weight, load_ops

@@ -47,6 +47,11 @@ __device__ inline void parts_of(float x, float y, uint32_t (&p)[3]) {
     }
 }
 
+// The largest of a >= 0 and of x and y without their signs: NaN if one of them is (one v_maximum3_f32).
+__device__ inline float larger(float a, float x, float y) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, fabsf(x)), fabsf(y));
+}
+
 // GM x GN waves, each TM x TN tiles of 32 x 32; MW: waves a SIMD there must be registers for.  ranges > 1: K is cut into ranges of range_slabs
 // slabs (an even number, as K / PK is), and a range's sum goes to `partial` [range][M][N] in two parts.  Item i of the grid runs on XCD i % 8,
 // and an XCD takes an eighth of the items, row tiles first, so that a weight tile comes from memory for one XCD.
@@ -56,8 +61,9 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
                                                      int range_slabs, float2* __restrict__ partial) {
     constexpr int WAVES = GM * GN, THREADS = 64 * WAVES, BM = GM * TM * 32, BN = GN * TN * 32, ROWS = BM + BN;
     static_assert(PF == 2 && PFOLD % PF == 0, "slabs come in pairs");
-    constexpr int UNITS = (ROWS * 2 * PCH + THREADS - 1) / THREADS; // pieces a thread moves of every slab
-    extern __shared__ __align__(16) uint4 lds[];            // [2 slabs][3 parts][ROWS][PCH], a row's pieces turned by a quarter of its number
+    static_assert(ROWS * 2 * PCH % THREADS == 0 && PCH == 4, "every thread has as many pieces, eight of them side by side a row's");
+    constexpr int UNITS = ROWS * 2 * PCH / THREADS; // pieces a thread moves of every slab
+    extern __shared__ __align__(16) uint4 lds[];            // [2 slabs][3 parts][ROWS][PCH], a row's pieces turned by a quarter of its number; [ROWS] numbers
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, items = tiles_m * tiles_n * ranges;
     const int item = (int)(blockIdx.x & 7) * ((items + 7) >> 3) + (int)(blockIdx.x >> 3);
@@ -67,16 +73,18 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
     const int slab0 = range * range_slabs, slabs = min(K / PK - slab0, range_slabs);
     auto turn = [](int r) { return (r >> 2) & (PCH - 1); };
 
-    // this thread's pieces: 4 numbers of a row (of the last row that exists where it does not: its results are not stored)
+    // this thread's pieces: 4 numbers of a row (of the last row that exists where it does not: its results are not stored), the same of every RU-th
+    constexpr int RU = THREADS / (2 * PCH);
+    static_assert(BM % RU == 0 && RU % 16 == 0, "a piece is the activations' or the weights' for all threads, and turned alike");
+    const int r0 = tid / (2 * PCH), c0 = tid % (2 * PCH), dst = (r0 * PCH + ((c0 >> 1) ^ turn(r0))) * 2 + (c0 & 1);
     const float* src[UNITS];
-    int dst[UNITS];
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
-        const int p = min(u * THREADS + tid, ROWS * 2 * PCH - 1), r = p / (2 * PCH), c = p % (2 * PCH);
-        src[u] = (r < BM ? a + (size_t)min(m0 + r, M - 1) * lda : w + (size_t)min(n0 + r - BM, N - 1) * K) + (size_t)slab0 * PK + c * 4;
-        dst[u] = (r * PCH + ((c >> 1) ^ turn(r))) * 2 + (c & 1);
+        const int r = u * RU + r0;
+        src[u] = (u * RU < BM ? a + (size_t)min(m0 + r, M - 1) * lda : w + (size_t)min(n0 + r - BM, N - 1) * K) + (size_t)slab0 * PK + c0 * 4;
     }
     float4 ahead[PF][UNITS];                                // the next slabs' pieces, on their way
+    float top[UNITS] = {};                                  // the largest number of this thread's pieces of a row so far, without its sign
     auto fetch = [&](int slot, int s) {
         const int at = min(s, slabs - 1) * PK;              // (past the end the last slab once more: it is not multiplied)
 #pragma unroll
@@ -90,8 +98,9 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
             uint32_t p[2][3];
             parts_of(x.x, x.y, p[0]);
             parts_of(x.z, x.w, p[1]);
+            top[u] = larger(larger(top[u], x.x, x.y), x.z, x.w);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) to[i * ROWS * PCH * 2 + dst[u]] = make_uint2(p[0][i], p[1][i]);
+            for (int i = 0; i < 3; ++i) to[i * ROWS * PCH * 2 + dst + u * RU * PCH * 2] = make_uint2(p[0][i], p[1][i]);
         }
     };
     auto meet = [&]() {                                     // LDS alone is waited for: the slabs on their way stay there
@@ -161,6 +170,8 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
             __builtin_amdgcn_sched_group_barrier(0x2, VA, 0);
             if (i >= MM - 3 * UNITS) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
         }
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) asm volatile("" : "+v"(top[u]));       // made here: left for later, the pieces would have to stay, too
         __builtin_amdgcn_sched_barrier(0);
         meet();
         __builtin_amdgcn_sched_barrier(0);
@@ -193,20 +204,44 @@ __global__ __launch_bounds__(64 * GM * GN, MW) void k_gemm_f32_parts(TO* __restr
     }
     fold();
 
-    // Results that are not finite, or so small that parts may have fallen out of bfloat16's range (a number's last part below 2^-126 is lost, so
-    // 2^-126 times the other operands: nothing beside 2^-60 while those are below 2^40), are made again from 32-bit products, a wave's 32 x 32 at a time: an infinity
-    // stays one, whatever it meets, and an overflow happens where it did.  The others of the 32 x 32 stay as they are: a result depends on its own row
-    // and column alone.  (Where every tile is made again, a product takes three times as long.)
+    // Results that are not finite, or so small that what parts have lost may count, are made again from 32-bit products, a wave's 32 x 32 at a time:
+    // an infinity stays one, whatever it meets, and an overflow happens where it did.  (The part of a number that is below 2^-126 is lost: over K columns
+    // up to K 2^-125 times the largest number of the row and of the weight row that meet, `most` here.  Where that is above 2^-27 of a result, or a result is
+    // below 2^-60 and products of parts may be too small for 32 bits, it is made again; a zero is one where one of the rows has nothing else.)  The others of
+    // the 32 x 32 stay as they are: a result depends on its own row and column alone.  (Where every tile is made again, a product takes three times as long.)
+    float* const tops = reinterpret_cast<float*>(lds + 2 * 3 * ROWS * PCH);
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        float t = top[u];
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) t = larger(t, __shfl_xor(t, o), 0.f);
+        if (c0 == 0) tops[u * RU + r0] = t;
+    }
+    meet();
+    const float lost_share = (float)(slabs * PK) * 0x1p-98f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int n = n0 + wn + 32 * j + row, mb = m0 + wm + 32 * i + 4 * (lane >> 5);
-            uint32_t bad = 0;                               // a bit for each of the lane's 16
+            const float top_w = tops[BM + wn + 32 * j + row];
+            float least = 1.f, largest = 0.f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const float v = fabsf(tot[i][j][e] + low[i][j][e]);
-                if (n < N && mb + 8 * (e >> 2) + (e & 3) < M && !((v >= 0x1p-60f && v <= 3.402823466e38f) || v == 0.f)) bad |= 1u << e;
+                least = __builtin_elementwise_minimum(least, v);
+                largest = larger(largest, v, 0.f);
+            }
+            const bool usual = least >= 0x1p-60f && largest <= 3.402823466e38f && lost_share * larger(top_w, tops[wm + 32 * i + row], 0.f) <= 0x1p-60f;
+            if (!__any(!usual)) continue;
+            uint32_t bad = 0;                               // a bit for each of the lane's 16
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float v = fabsf(tot[i][j][e] + low[i][j][e]), top_a = tops[wm + 32 * i + 4 * (lane >> 5) + 8 * (e >> 2) + (e & 3)];
+                const float most = larger(top_a, top_w, 0.f);
+                const bool fine = v <= 3.402823466e38f && ((v >= 0x1p-60f && v >= lost_share * most) || top_a == 0.f || top_w == 0.f);
+                if (n < N && mb + 8 * (e >> 2) + (e & 3) < M && !fine) bad |= 1u << e;
+                asm volatile("" : "+v"(bad));               // (a bit and not a mask of lanes each)
             }
             if (__any(bad != 0)) {
                 const float* const x = a + (size_t)min(m0 + wm + 32 * i + row, M - 1) * lda + 4 * (lane >> 5);
@@ -296,7 +331,7 @@ static int parts_range(int K, int& ranges) {
 template <int GM, int GN, int TM, int TN, int MW, int PF>
 static int launch_parts(void* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo, int out_dtype,
                         int accumulate, int ranges, float2* partial, hipStream_t stream) {
-    constexpr int BM = GM * TM * 32, BN = GN * TN * 32, smem = 2 * 3 * (BM + BN) * PK * 2;
+    constexpr int BM = GM * TM * 32, BN = GN * TN * 32, smem = 2 * 3 * (BM + BN) * PK * 2 + (BM + BN) * 4;
     const int per = parts_range(K, ranges);
     const long long items = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN) * ranges;
     XR_REQUIRE(items < (1ll << 28), "gemm: %lld tiles", items);
