@@ -30,7 +30,7 @@ def test_tiles_and_ranges(M, N, K):
     ops, a, w, bias, c = operands(M, N, K)
     want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
     # a run is 16 additions of 2^-24 of what has been added up so far (twice that, for what an instruction may round inside), the runs' sums lose
-    # a few 2^-24 more, the products left out 2^-26
+    # a few 2^-24 more, the products left out at most 2^-24 (of ordinary numbers together about 2^-26)
     bound = 40 * U * size
     whole = None
     for tile in range(TILES):
@@ -131,6 +131,20 @@ def test_tiny_numbers_that_meet_large_ones(tile, ranges):
     assert ((got.double() - want).abs() <= bound)[fits].all() and torch.equal(got.isfinite() | fits, usual.isfinite() | fits)
     assert torch.equal(got[24] == 0, usual[24] == 0) and ((got[24] - usual[24]).double().abs() <= bound[24]).all()
     assert (got[25] == 0).all() and (got[:, 105] == 0).all()
+
+
+# 1.00389862 has the parts 1, 2^-8 and -2^-17: of such a product the parts left out are 2^-24, all of one sign
+def test_products_whose_missing_parts_add_up():
+    import torch
+    M, N, K = 40, 200, 2048
+    ops, a, w, _, _ = operands(M, N, K)
+    x = 1 + 32704 * 2.0 ** -23
+    a.fill_(x), w.fill_(x)
+    for tile in range(TILES):
+        for ranges in (1, 4):
+            got = ops.linear(a, w, variant=plan(tile, ranges))
+            # 2^-24, and as much again for the runs' sums, whose losses are made up for, and the last rounding
+            assert ((got.double() / (K * x * x) - 1).abs() <= 2 * U).all()
 
 
 def test_products_that_stay_with_the_32_bit_instructions():

@@ -1,7 +1,8 @@
 // Matrix products of 32-bit operands, out[M,N] = a[M,K] * w[N,K]^T (+ bias), on the matrix cores' bfloat16 instructions, which do sixteen
 // products in the time the 32-bit ones (k_gemm_f32) do one.  Every number is three bfloat16 parts that add up to it exactly (8 bits a
 // part, rounded to nearest, each with its sign: 24 bits), and a product of two numbers the six largest of the nine products of
-// their parts; the three left out are below 2^-26 of it together.  Part 0 times part 0, which a bfloat16 instruction makes exactly
+// their parts; the three left out are 2^-24 of it at most together (x = y = 1.00389862, whose products all miss as much; 2^-27.4 in root mean
+// square of normal ones).  Part 0 times part 0, which a bfloat16 instruction makes exactly
 // and adds up in 32 bits, sixteen columns at a time, is summed in runs of PFOLD slabs and the runs' sums with what each addition loses; the
 // smaller products have a sum of their own over all of K, where 2^-8 of the size their rounding does not count.  That is fewer
 // roundings than a 32-bit instruction's, two columns at a time: root mean square error against 64 bits, in units of the result's, 401 x
