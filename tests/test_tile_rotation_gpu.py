@@ -42,3 +42,31 @@ def test_keys_that_are_not_16_byte_aligned(ops):      # noqa: F811
             ops.fuse_rope = True
         results.append((q, kc, vc))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_pages_of_more_than_32_bits_channels(ops):      # noqa: F811
+    """A page of 2^20 positions of 16 heads of 256: 2^32 channels."""
+    import torch
+    from test_kernels_gpu import DEV, FakeCtx
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("two pages of keys and of values are 32 GiB")
+    torch.manual_seed(6)
+    H, Hk, D, ps, T = 1, 16, 256, 1 << 20, 520
+    ctx = FakeCtx([3], [T], [[1]], ps)
+    h = torch.randn(T, 256, device=DEV).bfloat16()
+    w = ops.pack_weight((torch.randn((H + 2 * Hk) * D, 256, device=DEV) * 0.1).bfloat16())
+    inv = (10000.0 ** (-torch.arange(D // 2, dtype=torch.float64) * 2 / D)).float().to(DEV)
+    kc, vc = (torch.empty((2, Hk) + s, device=DEV, dtype=torch.bfloat16) for s in ((ps, D), (D, ps)))
+    results = []
+    for fuse in (False, True):
+        kc[:, :, :3 + T], vc[..., :3 + T] = 7.0, 7.0
+        ops.fuse_rope = fuse
+        try:
+            q = ops.project_rope_kv_write(h, w, None, kc, vc, ctx.positions, ctx.req_of_token, ctx.block_table(0), inv, H, Hk, D, D, False, 1.0, ps,
+                                          paired=True)
+        finally:
+            ops.fuse_rope = True
+        results.append([x.clone() for x in (q, kc[:, :, :3 + T], vc[..., :3 + T])])
+    for one, two in zip(*results):
+        # (the same product in tiles, both rounded to bfloat16)
+        assert ((one.double() - two.double()).abs() <= 2.0 ** -7 * one.double().abs() + 2.0 ** -9).all()

@@ -437,8 +437,8 @@ __device__ __forceinline__ void rope_out(float* lds, const f32x16 (&acc)[TM][TN]
                         }
                     }
                 }
-                // (products of two 32-bit numbers: a page's place, and a row's)
-                bf16_t* at = key ? rp.k_cache + (uint64_t)(uint32_t)pg * (uint32_t)(KV * rp.page_size) + (uint32_t)((hs * rp.page_size + of) * rp.D)
+                // (products of two 32-bit numbers; a page may have 2^32 channels and more, its size is a power of two)
+                bf16_t* at = key ? rp.k_cache + ((uint64_t)(uint32_t)pg * (uint32_t)KV << rp.page_shift) + (uint64_t)(uint32_t)((hs << rp.page_shift) + of) * (uint32_t)rp.D
                                  : rp.q_out + (uint64_t)(uint32_t)m * (uint32_t)Q + (uint32_t)(hs * rp.D);
                 const int d0 = paired ? c >> 1 : c, d1 = paired ? d0 + half : c + 8;
                 if (mine && m < M) {
