@@ -44,6 +44,24 @@ def test_product(M, N, K):
     assert torch.equal(ops.linear(many.contiguous(), packed, out_dtype=torch.float32)[:M], got)
 
 
+@pytest.mark.parametrize("N,K", [(40, 2048), (3000, 2048), (4112, 64)])
+def test_rows_that_are_far_apart(N, K):
+    """Rows that begin 2^28 numbers one behind the other: more bytes than 32 bits count."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    if torch.cuda.mem_get_info()[0] < 8 << 30:
+        pytest.skip("nine such rows are 4.5 GiB")
+    g = torch.Generator(device=dev)
+    g.manual_seed(N + K)
+    a, w = (torch.randn(s, generator=g, device=dev).bfloat16() for s in ((9, K), (N, K)))
+    far = torch.empty((8 * 2 ** 28 + K,), dtype=torch.bfloat16, device=dev).as_strided((9, K), (2 ** 28, 1))
+    far.copy_(a)
+    want, bound = a.double() @ w.double().T, (K + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    for M in (8, 9):
+        assert ((ops.linear(far[:M], ops.pack_weight(w), out_dtype=torch.float32).double() - want[:M]).abs() <= bound[:M]).all()
+
+
 @pytest.mark.parametrize("N,F,K", [(2048, 512, 2048), (2040, 8192, 2080), (24, 128256 // 16, 4096)])
 @pytest.mark.parametrize("M", [1, 8, 9])
 def test_the_norm_behind_it(M, N, F, K):

@@ -2030,12 +2030,13 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // 4096 6.1, 7.0 and 4.8, 5.8.  Not so 3072 x 2048 (5.0, 5.4 and 5.1, 6.3), 2560 x 6912 (10.9, 11.2 and 11.4, 14.7) and 1024 x 1024 (3.6 and
             // 3.7).  (Rotated results are made from 16 columns.)
             const bool pairs = !sw && !rope && N <= 2048 && K >= 2048;
+            const bool near = (size_t)16 * lda * 2 < (1ull << 32);      // the rings' offsets from the first row have 32 bits
             if (pairs) {
                 // (9 to 16 rows without the ring: 2048 x 8192 12.1 us, 12.5 with it; 2048 x 10752 15.8 and 16.8)
                 blocks = M > 8          ? launch_skinny<1, 1, 8, 4, false, true, 2>(g, stream)
-                         : K % 64 == 0  ? launch_skinny<1, 1, 8, 4, false, true, 1, true>(g, stream)
+                         : near && K % 64 == 0 ? launch_skinny<1, 1, 8, 4, false, true, 1, true>(g, stream)
                                         : launch_skinny<1, 1, 8, 4, false, true, 1>(g, stream);
-            } else if (K % 32 == 0) {
+            } else if (near && K % 32 == 0) {
                 // Whole steps.  Measured in recorded decode steps, us, batches (below) and ring: gated 14336 x 4096 at 1 and 8 rows 39.4, 41.3 and 38.6,
                 // 40.0, 8192 x 2048 at one 13.4 and 12.5, 11008 x 4096 at 3 31.6 and 29.8 (four waves and a ring of 8: 39.6, 40.2; 13.4; 30.4).  Plain, four waves
                 // and a ring of 8 from 4,096 weight rows on: 4096 x 4096 8.6 and 8.3, 4096 x 11008 17.8 and 16.7, 4096 x 21504 27.2 and 26.7, 10752 x 2048 at 8
