@@ -85,3 +85,27 @@ def test_the_norm_behind_it(M, N, F, K):
     rows, wt = h.data.double() * scale, ops.linear(torch.eye(N, device=dev).bfloat16(), w2, out_dtype=torch.float32).double() if N % 8 == 0 else None
     got = ops.linear(h, w2, out_dtype=torch.float32).double()
     assert ((got - rows @ wt).abs() <= (N + 8) * 2.0 ** -23 * (rows.abs() @ wt.abs())).all()
+
+
+def test_room_for_a_partial_sum_every_16_columns():
+    """Room for half as many partial sums of squares as workgroups of 8 weight rows make: the kernel that needs no more."""
+    import ctypes
+    import torch
+    from xyntetik_runner_amd.csrc.ops import XR_F32, _GemmNorm, _stream, load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    M, N, K = 3, 2048, 2048
+    g = torch.Generator(device=dev)
+    g.manual_seed(1)
+    a, w, x, nw = (torch.randn(s, generator=g, device=dev) for s in ((M, K), (N, K), (M, N), (N,)))
+    a, w = a.bfloat16(), w.bfloat16()
+    want, size = x.double() + a.double() @ w.double().T, x.double().abs() + a.double().abs() @ w.double().abs().T
+    xg, sums = torch.empty((M, N), dtype=torch.bfloat16, device=dev), torch.full((N // 8, 16), -1.0, device=dev)
+    then = _GemmNorm()
+    then.norm_w, then.xg, then.ss_out, then.ss_out_rows = nw.data_ptr(), xg.data_ptr(), sums.data_ptr(), N // 16
+    then.ss_inv_width, then.ss_eps = 1.0 / N, 1e-5
+    ops.lib.check(ops.lib.xr_gemm_bf16(x.data_ptr(), a.data_ptr(), w.data_ptr(), None, M, N, K, K, N, XR_F32, 1, 0, 0.0, 0, 0,
+                                       *ops._gemm_workspace(dev), ctypes.addressof(then), None, _stream()))
+    assert then.ss_out_rows == N // 16 and (sums[N // 16:] == -1).all()
+    assert ((x.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size).all() and torch.equal(xg, (x * nw).bfloat16())
+    d = x.double() ** 2
+    assert ((sums[:N // 16, :M].double().sum(0) - d.sum(1)).abs() <= (N + 2) * 2.0 ** -24 * d.sum(1)).all()

@@ -128,7 +128,7 @@ struct XrGemmNorm {
     int norm_w_bf16;
     void* xg;
     float* ss_out;
-    int ss_out_rows;   // in: partial rows that ss_out has room for; out: partial rows written
+    int ss_out_rows;   // in: partial rows that ss_out has room for, (N + 15) / 16 at least, (N + 7) / 8 for the fastest kernels; out: partial rows written
     int centred;       // the norm after the product is a layer norm (more than 16 rows, finished by k_gemm_finish_norm)
     void* post_x;      // or null: the rows [M, post_ld] that become the norm of post_alpha x themselves + the product (EPI_STORE)
     int post_ld;
@@ -1807,8 +1807,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
                            "gemm: rows that become a norm: more than 16, 16-byte aligned, %d apart", norm->post_ld);
                 g.post_x = (float*)norm->post_x; g.post_ld = norm->post_ld; g.post_alpha = norm->post_alpha;
             }
-            XR_REQUIRE(M > 16 || (norm->ss_out && norm->ss_out_rows >= (N + 7) / 8),
-                       "gemm: room for %d partial sums of squares, %d needed", norm->ss_out ? norm->ss_out_rows : 0, (N + 7) / 8);
+            XR_REQUIRE(M > 16 || (norm->ss_out && norm->ss_out_rows >= (N + 15) / 16),
+                       "gemm: room for %d partial sums of squares, %d needed", norm->ss_out ? norm->ss_out_rows : 0, (N + 15) / 16);
             XR_REQUIRE(!norm->centred || M > 16, "gemm: a layer norm after a product of %d rows: from 17 rows on", M);
             g.norm_centred = norm->centred ? 1 : 0;
             g.norm_w = norm->norm_w; g.norm_w_bf16 = norm->norm_w_bf16; g.xg = (bf16_t*)norm->xg; g.ss_out = norm->ss_out;
@@ -2028,8 +2028,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // Up to 2,048 weight rows, 2,048 columns on: workgroups of 8 weight rows (one for every compute unit at 2,048).  us without and
             // with at 1 and 8 rows: 2048 x 8192 11.3, 11.5 and 8.3, 9.2; 2048 x 10752 15.5, 15.1 and 10.8, 12.4; 2048 x 2048 4.7, 5.2 and 4.2, 4.7; 1024 x
             // 4096 6.1, 7.0 and 4.8, 5.8.  Not so 3072 x 2048 (5.0, 5.4 and 5.1, 6.3), 2560 x 6912 (10.9, 11.2 and 11.4, 14.7) and 1024 x 1024 (3.6 and
-            // 3.7).  (Rotated results are made from 16 columns.)
-            const bool pairs = !sw && !rope && N <= 2048 && K >= 2048;
+            // 3.7).  (Rotated results are made from 16 columns; twice as many partial sums of squares need room.)
+            const bool pairs = !sw && !rope && N <= 2048 && K >= 2048 && !(g.xg && norm->ss_out_rows < (N + 7) / 8);
             const bool near = (size_t)16 * lda * 2 < (1ull << 32);      // the rings' offsets from the first row have 32 bits
             if (pairs) {
                 // (9 to 16 rows without the ring: 2048 x 8192 12.1 us, 12.5 with it; 2048 x 10752 15.8 and 16.8)
