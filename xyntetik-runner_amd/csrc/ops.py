@@ -8,6 +8,7 @@ raw pointers and the current HIP stream to the entry point, and raises
 """
 from __future__ import annotations
 
+import copy
 import ctypes as C
 import threading
 from dataclasses import dataclass
@@ -163,9 +164,23 @@ class PackedWeight:
 
 class F32Weight(torch.Tensor):
     """A float32 weight matrix as it is, as one that a model keeps: its products of many rows may be made of bfloat16 parts
-    (``Ops.linear``).  Made by ``Ops.pack_weight``; what is computed from it is a plain tensor."""
+    (``Ops.linear``).  Made by ``Ops.pack_weight``; what is computed from it is a plain tensor, and so is what a file of it holds."""
 
     __torch_function__ = torch._C._disabled_torch_function_impl
+
+    def __copy__(self):
+        return self.as_subclass(torch.Tensor).as_subclass(F32Weight)
+
+    def __deepcopy__(self, memo):
+        if id(self) not in memo:
+            memo[id(self)] = copy.deepcopy(self.as_subclass(torch.Tensor), memo).as_subclass(F32Weight)
+        return memo[id(self)]
+
+    def __reduce_ex__(self, protocol):
+        return self.as_subclass(torch.Tensor).__reduce_ex__(protocol)
+
+    def detach(self):       # (a Parameter is made of what this returns, and has to be of one type with it)
+        return super().detach().as_subclass(F32Weight)
 
 
 class UnscaledRows:
