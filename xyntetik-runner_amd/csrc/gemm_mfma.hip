@@ -1457,7 +1457,7 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
     // instance of this kernel, so a row's scale does not depend on the batch.
     float* scale_s = red + KSW * NWT * SROWS * MTOK;       // [16 parts][16 rows]
     float part_ss[16];
-    const bool scales = g.ss_in != nullptr && tid < 256;
+    const bool scales = MT == 1 && g.ss_in != nullptr && tid < 256;      // (more than 16 rows have none)
     auto fetch_ss = [&](int p0) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) part_ss[i] = p0 + i * 16 < g.n_ss ? g.ss_in[(p0 + i * 16) * 16 + (tid & 15)] : 0.f;
