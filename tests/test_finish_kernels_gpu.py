@@ -76,3 +76,32 @@ def test_rotation(T, H, Hk, D, rot, inter, ps):
         assert torch.equal(one, two)
         # (the product's sums in another order, both rounded to bfloat16)
         assert ((one.double() - three.double()).abs() <= 2.0 ** -7 * three.double().abs() + 2.0 ** -9).all()
+
+
+@pytest.mark.parametrize("T", [17, 130, 511])
+@pytest.mark.parametrize("H,Hk,D,rot,inter", [(4, 2, 64, 64, False), (2, 1, 48, 32, False), (3, 1, 16, 6, True)])
+def test_keys_that_are_not_8_byte_aligned(T, H, Hk, D, rot, inter):
+    """The kernel that stores four channels at a time does not take them; one column a thread does, with the same sums."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, ps = load_ops(), 16
+    g = torch.Generator(device=DEV)
+    g.manual_seed(T + D)
+    tables, n_pages = scatter_pages([T + 3], ps, 2)
+    ctx = FakeCtx([3], [T], tables, ps)
+    h = torch.randn(T, 256, generator=g, device=DEV).bfloat16()
+    w = ops.pack_weight((torch.randn((H + 2 * Hk) * D, 256, generator=g, device=DEV) * 0.1).bfloat16())
+    inv = (10000.0 ** (-torch.arange(rot // 2, dtype=torch.float64) * 2 / rot)).float().to(DEV)
+    results = []
+    for shift in (0, 1):
+        size = n_pages * Hk * ps * D
+        kc = torch.full((size + 8,), 7.0, device=DEV, dtype=torch.bfloat16)[shift:shift + size].view(n_pages, Hk, ps, D)
+        vc = torch.full((n_pages, Hk, D, ps), 7.0, device=DEV, dtype=torch.bfloat16)
+        assert kc.data_ptr() % 8 == 2 * shift
+        q = ops.project_rope_kv_write(h, w, None, kc, vc, ctx.positions, ctx.req_of_token, ctx.block_table(0), inv, H, Hk, D, rot, inter, 1.0, ps,
+                                      paired=not inter, finish_table=lambda: ops.rope_table(ctx.positions, inv, 1.0))
+        results.append((q, kc, vc))
+    assert torch.equal(results[0][2], results[1][2])
+    for one, two in zip(*results):
+        # (a rotation's two products and their sum, in 32 bits in another order, then a bfloat16 rounding)
+        assert ((one.double() - two.double()).abs() <= 2.0 ** -8 * two.double().abs() + 2.0 ** -18).all()
