@@ -64,7 +64,8 @@ def test_rows_that_are_far_apart(N, K):
         assert ((ops.linear(far[:M], ops.pack_weight(w), out_dtype=torch.float32).double() - want[:M]).abs() <= bound[:M]).all()
 
 
-@pytest.mark.parametrize("N,F,K", [(2048, 512, 2048), (2040, 8192, 2080), (24, 128256 // 16, 4096)])
+# (what reads them: a ring, batches, and batches with more than 256 partial sums)
+@pytest.mark.parametrize("N,F,K", [(2048, 512, 2048), (2040, 8192, 2080), (24, 128256 // 16, 4096), (4104, 512, 512)])
 @pytest.mark.parametrize("M", [1, 8, 9])
 def test_the_norm_behind_it(M, N, F, K):
     """The product adds into a stream and leaves its weighted rows and the sums of their squares to the next product."""

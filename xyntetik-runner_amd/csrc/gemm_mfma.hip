@@ -1452,17 +1452,20 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[t][r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // The rows' scales, from the partial sums the producer of `a` left: thread (part, tok) of the first 256 sums every 16th partial (16 at a
-    // time on their way before the weights), each thread of the last loop sums the 16 parts of its row; the order is the same in every
-    // instance of this kernel, so a row's scale does not depend on the batch.
+    // The rows' scales, from the partial sums the producer of `a` left: thread (part, tok) of the first 256 sums every 16th partial, each thread of the
+    // last loop sums the 16 parts of its row; the order is the same in every instance of this kernel, so a row's scale does not depend on the
+    // batch.  Rings fetch 16 partials a thread before the weights and sum them while those are on their way.  Batches have their registers in use until
+    // the last product (16 more: gated 41072 x 776 31 us and 41, a workgroup a compute unit instead of two); there the first SS_AHEAD partials are copied to
+    // LDS meanwhile (a wave's copy moves 16 of them).
+    constexpr int SS_AHEAD = 256;
     float* scale_s = red + KSW * NWT * SROWS * MTOK;       // [16 parts][16 rows]
+    float* ss_s = scale_s + 256;                           // [SS_AHEAD][16 rows] (batches)
     float part_ss[16];
     const bool scales = MT == 1 && g.ss_in != nullptr && tid < 256;      // (more than 16 rows have none)
     auto fetch_ss = [&](int p0) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) part_ss[i] = p0 + i * 16 < g.n_ss ? g.ss_in[(p0 + i * 16) * 16 + (tid & 15)] : 0.f;
     };
-    if (scales) fetch_ss(tid >> 4);
     auto sum_ss = [&]() {
         if (!scales) return;
         float s = 0.f;
@@ -1474,6 +1477,17 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
         }
         scale_s[tid] = s;
     };
+    if constexpr (WHOLE) {
+        if (scales) fetch_ss(tid >> 4);
+    } else if (MT == 1 && g.ss_in) {
+        const int chunks = (g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD) * 4;      // pieces of 16 bytes
+        const uint32_t ss_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ss_s;
+        for (int c0 = wave * 64; c0 < chunks; c0 += THREADS) {
+            const int c = c0 + lane;
+            const void* src = c < chunks ? (const void*)((const char*)g.ss_in + (size_t)c * 16) : (const void*)xr_zero_chunk;
+            lds_dma16(src, __builtin_amdgcn_readfirstlane(ss_lds + (uint32_t)c0 * 16));
+        }
+    }
 
     if constexpr (WHOLE) {
         // K is whole steps: a ring of U steps' loads, each on its way again as soon as its products are made, with bases that the wave shares and a
@@ -1567,7 +1581,6 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                         }
                 }
         }
-        sum_ss();
     }
 
     // acc[t][r][i][e]: weight row r*16 + 4*(lane/16) + e of the workgroup's ROWS, token i*16 + lane%16
@@ -1581,6 +1594,19 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                 for (int e = 0; e < 4; ++e)
                     red[((wave * NWT + t) * SROWS + r * 16 + lq * 4 + e) * MTOK + i * 16 + (lane & 15)] =
                         PAIRS == 2 ? acc[0][r][i][e] + acc[NSUM - 1][r][i][e] : acc[t][r][i][e];
+    if constexpr (!WHOLE) {
+        if (MT == 1 && g.ss_in) {
+            wait_vmcnt<0>();
+            __syncthreads();                              // every wave's copies have landed
+            if (tid < 256) {
+                float s = 0.f;
+                const int n_lds = g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD;
+                for (int p = tid >> 4; p < n_lds; p += 16) s += ss_s[p * 16 + (tid & 15)];
+                for (int p = (tid >> 4) + SS_AHEAD; p < g.n_ss; p += 16) s += g.ss_in[p * 16 + (tid & 15)];
+                scale_s[tid] = s;
+            }
+        }
+    }
     __syncthreads();
     for (int q = tid; q < ROWS * MTOK; q += THREADS) {
         int col = q % ROWS, tok = q / ROWS;          // consecutive threads write consecutive columns
@@ -1700,7 +1726,7 @@ static inline int rc_of(int launched) { return launched < 0 ? launched : XR_OK; 
 template <int MT, int RT, int KSW, int U, bool SW, bool NT = false, int PAIRS = 0, bool WHOLE = false>
 static int launch_skinny(const GemmArgs& g, hipStream_t stream) {
     constexpr int NWT = SW ? 2 : 1;
-    size_t smem = (size_t)KSW * NWT * RT * 16 * MT * 16 * 4 + 256 * 4;    // the sums of the waves, 256 partial scales
+    size_t smem = (size_t)KSW * NWT * RT * 16 * MT * 16 * 4 + 256 * 4 + (WHOLE ? 0 : 256 * 64);    // the sums of the waves, 256 partial scales, 256 rows of partial sums
     static bool attr_set = false;
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)k_gemm_skinny<MT, RT, KSW, U, SW, NT, PAIRS, WHOLE>,
