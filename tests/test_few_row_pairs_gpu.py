@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 # of 8.  Rings: one step, fewer than waves, fewer than a ring, one past it, waves with different numbers of steps; fewer than 4,096 weight
 # rows, no multiple of 16, and more; 65,536 and more.  Batches (K no whole steps) beside them.
 @pytest.mark.parametrize("N,K", [(7, 2048), (2048, 2048), (2041, 2080), (2024, 2056), (40, 14336), (1000, 4104), (2048, 10752),
-                                 (40, 32), (3000, 288), (2060, 4128), (4100, 1056), (4112, 5152), (5000, 1064), (65552, 96), (65552, 2048)])
+                                 (40, 32), (3000, 288), (2060, 4128), (4100, 1056), (4112, 5152), (5000, 1064), (65552, 96), (65552, 2048),
+                                 (3000, 2080), (6000, 2048), (4100, 512), (4100, 544)])
 @pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
 def test_product(M, N, K):
     import torch

@@ -1393,7 +1393,7 @@ static int launch_tile_async(GemmArgs g, hipStream_t stream) {
 // WHOLE: K is whole steps.  Batches of U steps wait out a trip to memory each, and spend some 70 instructions on their addresses and on dropping
 // what does not exist; here the loads are a ring, with addresses that cost two instructions a step, and nothing is dropped.
 template <int MT, int RT, int KSW, int U, bool SWIGLU, bool NT, int PAIRS = 0, bool WHOLE = false>
-__global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
+__global__ __launch_bounds__(64 * KSW, WHOLE && RT == 1 ? 4 : 1) void k_gemm_skinny(GemmArgs g) {
     constexpr int NWT = SWIGLU ? 2 : 1;  // weight fragments per row group (gate and up)
     constexpr int MTOK = MT * 16, ROWS = PAIRS == 1 ? 8 : RT * 16, THREADS = 64 * KSW;
     constexpr int SROWS = RT * 16;
@@ -1493,7 +1493,7 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
         // K is whole steps: a ring of U steps' loads, each on its way again as soon as its products are made, with bases that the wave shares and a
         // fixed offset a lane.  Nothing is masked: a lane whose weight row or token does not exist reads one that does, and its
         // results are not used; a step past the wave's last is that one once more, and not multiplied.
-        const int s0 = kbeg / STEP, s1 = kend / STEP;
+        const int s0 = __builtin_amdgcn_readfirstlane(kbeg / STEP), s1 = __builtin_amdgcn_readfirstlane(kend / STEP);
         const char* const a0 = (const char*)g.a;
         const uint32_t a_lane = (uint32_t)(((l16 < g.M ? l16 : 0) * g.lda + odd * 32 + lq * 8) * 2);
         const char* w0[NWT][RT];
@@ -1509,7 +1509,8 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
         }
         uint4 wreg[U][NWT][RT], areg[U];
         auto load = [&](int u, int s) {
-            const size_t at = (size_t)(s < s1 ? s : s1 - 1);
+            asm("" : "+s"(s));                               // (a step's place is made in scalar registers, the lanes keep their offsets alone)
+            const size_t at = (size_t)(uint32_t)s;
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -1528,13 +1529,15 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                     sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wreg[u][t][r]), as_bf16x8(areg[u]), sum, 0, 0, 0);
                 }
         };
-        if (s0 < s1) {
+        // (Steps past the last one were loaded as that one once more: no branch, but 5 of 16 loads for nothing at 11 steps a wave, 6 of 8 at 2: 42784 x 256 17.5
+        // us at 16 rows, 38496 x 1408 20.7 at one.  The ring's own loop has none of them, nor has it branches, with which every load would be waited for at once.)
+        int s = s0;
+        auto ring = [&]() {
 #pragma unroll
-            for (int u = 0; u < U; ++u) load(u, s0 + u);
+            for (int u = 0; u < U; ++u) load(u, s + u);
             __builtin_amdgcn_sched_barrier(0);
             sum_ss();
-            int s = s0;
-            for (; s + U < s1; s += U) {
+            for (; s + 2 * U <= s1; s += U) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     __builtin_amdgcn_sched_barrier(0);
@@ -1543,11 +1546,29 @@ __global__ __launch_bounds__(64 * KSW) void k_gemm_skinny(GemmArgs g) {
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+        };
+        if (s1 > s0 && (s1 - s0) % U == 0) {
+            ring();
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (s + u < s1) use(u);
+            for (int u = 0; u < U; ++u) use(u);
+        } else if (s1 - s0 > U) {
+            ring();
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                use(u);
+                if (s + U + u < s1) load(u, s + U + u);
+            }
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u)
+                if (s + U + u < s1) use(u);
         } else {
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u)
+                if (s0 + u < s1) load(u, s0 + u);
             sum_ss();
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u)
+                if (s0 + u < s1) use(u);
         }
     } else {
         for (int k0 = kbeg; k0 < kend; k0 += STEP * U) {
@@ -2057,22 +2078,30 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // 3.7).  (Rotated results are made from 16 columns; twice as many partial sums of squares need room.)
             const bool pairs = !sw && !rope && N <= 2048 && K >= 2048 && !(g.xg && norm->ss_out_rows < (N + 7) / 8);
             const bool near = (size_t)16 * lda * 2 < (1ull << 32);      // the rings' offsets from the first row have 32 bits
+            // Rings or batches.  Plain products below 65,536 weight rows, us, batches and rings: the rings' longer beginning does not pay for up to 512 columns (52960 x
+            // 384 at 4 rows 9.0 and 9.8, x 576 14.0 and 11.5), nor between one and two workgroups a compute unit from 2,048 to 4,096 columns (5120 x 2560 at 8 rows 8.2
+            // and 8.6, 6144 x 4096 11.5 and 11.9; 6144 x 1024 5.2 and 5.2, x 5120 15.7 and 14.9; 12288 x 4096 18.6 and 18.1), and with eight waves nothing from 5 rows
+            // on but for few columns (3072 x 4096 at one row 6.7 and 6.4, at 8 7.5 and 7.8, x 1536 5.1 and 4.7).  1,020 products of 170 drawn shapes (256 to 131,072
+            // weight rows, 256 to 16,384 columns, 1 to 16 rows, a third gated) take 0.90 of what batches alone take; 4 of them 3 to 9% longer.
+            const bool four = N > 4096 || (N == 4096 && K >= 4096);     // waves of a ring (4096 x 4096 at 8 rows 8.1 us in eight, 7.8 in four; x 3968 8.3 and 9.0)
+            const bool ring = near && K % 32 == 0 && (sw || N >= 65536 || (four ? N == 4096 || (K > 512 && !(N <= 8192 && K >= 2048 && K <= 4096))
+                                                                                : M <= 4 || K <= 1536));
             if (pairs) {
                 // (9 to 16 rows without the ring: 2048 x 8192 12.1 us, 12.5 with it; 2048 x 10752 15.8 and 16.8)
                 blocks = M > 8          ? launch_skinny<1, 1, 8, 4, false, true, 2>(g, stream)
                          : near && K % 64 == 0 ? launch_skinny<1, 1, 8, 4, false, true, 1, true>(g, stream)
                                         : launch_skinny<1, 1, 8, 4, false, true, 1>(g, stream);
-            } else if (near && K % 32 == 0) {
+            } else if (ring) {
                 // Whole steps.  Measured in recorded decode steps, us, batches (below) and ring: gated 14336 x 4096 at 1 and 8 rows 39.4, 41.3 and 38.6,
                 // 40.0, 8192 x 2048 at one 13.4 and 12.5, 11008 x 4096 at 3 31.6 and 29.8 (four waves and a ring of 8: 39.6, 40.2; 13.4; 30.4).  Plain, four waves
                 // and a ring of 8 from 4,096 weight rows on: 4096 x 4096 8.6 and 8.3, 4096 x 11008 17.8 and 16.7, 4096 x 21504 27.2 and 26.7, 10752 x 2048 at 8
                 // rows 11.5 and 10.6, 12352 x 4096 21.8 and 20.0, 16384 x 4096 23.8 and 22.6, 21504 x 4096 30.8 and 29.8, 32000 x 4096 42.6 and 40.4;
-                // no gain, and no more than 1% lost, 6144 x 4096 and 4096 x 14336.  Fewer weight rows than that leave compute units idle, and eight waves
+                // no more than 1% lost, 4096 x 14336.  Fewer weight rows than that leave compute units idle, and eight waves
                 // help the others: 3072 x 2048 5.9, with four 6.4, with eight 5.8.  From 65,536 weight rows on eight waves and a ring of 8 (128256 x 2048 at one row 82 with
                 // four in a loop of its own, 75 and 77.5 in a step), and from 9 rows on two groups of weight rows a wave (at 16 rows 117 with one, 89).
                 blocks = sw            ? launch_skinny<1, 1, 8, 4, true, true, 0, true>(g, stream)
                          : N >= 65536  ? (M > 8 ? launch_skinny<1, 2, 4, 8, false, true, 0, true>(g, stream) : launch_skinny<1, 1, 8, 8, false, true, 0, true>(g, stream))
-                         : N >= 4096   ? launch_skinny<1, 1, 4, 8, false, true, 0, true>(g, stream)
+                         : four        ? launch_skinny<1, 1, 4, 8, false, true, 0, true>(g, stream)
                                        : launch_skinny<1, 1, 8, 4, false, true, 0, true>(g, stream);
             } else if (sw) {
                 blocks = launch_skinny<1, 1, 8, 8, true, true>(g, stream);
