@@ -1937,17 +1937,17 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         // rows from L2 for every 16 weight rows, as many bytes as the weights are, and takes longer for every row; tiles take as long for 9 as
         // for 16, and a round more where they are just over 256.  The lesser of two models in us: tiles pay for the launch, for each further round,
         // and K for the weights of a full round from memory, or for what a lone tile waits for its own; the skinny kernels (plain, plain from 65,536 weight rows
-        // on, gated) for the weights, or for their workgroups.  Fitted to 680 pairs (20,480 to 128,256 weight rows, K 256 to 8,192): 0.3% slower than
-        // the better one on average, at most 4.4% slower than the skinny kernel; tiles wherever there are 160 were up to 43% slower (9 rows of 512 to
-        // 40,960 11.1 us, in tiles 15.9; 16 rows of 4,096 to 32,000 63.0 and 45.2; 9 of 512 to 22,016 8.3 and 9.7).
+        // on, gated) for the weights, or for their workgroups.  Fitted to 1,000 pairs of the two that run today (16,384 to 131,072 weight rows, K 512 to 8,192; a third of them
+        // held back): 0.3% slower than the better one on average, at most 16%, and at most 14% slower than the skinny kernel (once; the next 8%); with the numbers
+        // that fitted batches 2.0% and 34% (gated 19392 x 576 9 rows 12.3 us, in tiles 16.5; 80064 x 4672 9 rows 115 and 129); tiles wherever there are 160 8.1%, skinny always 4.4%.
         const int wide_tiles = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), wide_rounds = (wide_tiles + 255) / 256;
         bool wide = M > 8 && M <= 16 && !norm && !rope && w_packed && wide_tiles >= 160 && takes_written_order(g, 1, K, 64, 128, 4, 64);
         if (wide) {
             const double last = 0.00925 * K * (wide_tiles - 256 * (wide_rounds - 1)) / 256, alone = 0.00526 * K, mb = 2e-6 * w_rows * K;
             const double tiles_us = 6.95 + (2.72 + 0.00925 * K) * (wide_rounds - 1) + (last > alone ? last : alone);
-            const double groups_us = sw ? 6.5 + 4.0e-4 * w_rows : N >= 65536 ? 5.8 + 2.48e-4 * w_rows : 0.0;
-            const double bytes_us = sw ? 3.0 + mb / 6.25 : N >= 65536 ? 3.0 + mb / 6.08 : 5.86 + mb / 6.31 * (1.0 + 0.0373 * (M - 9));
-            const double by_row = sw ? 1.0 + 0.0138 * (M - 9) : N >= 65536 ? 1.0 + 0.0104 * (M - 9) : 1.0;
+            const double groups_us = sw ? 2.56 + 2.45e-4 * w_rows : N >= 65536 ? 4.82 + 1.98e-4 * w_rows : 0.0;
+            const double bytes_us = sw ? 4.43 + mb / 6.53 : N >= 65536 ? 3.88 + mb / 6.72 : 5.86 + mb / 6.31 * (1.0 + 0.0373 * (M - 9));
+            const double by_row = sw ? 1.0 + 0.0094 * (M - 9) : N >= 65536 ? 1.0 + 0.0097 * (M - 9) : 1.0;
             wide = tiles_us < 0.985 * by_row * (bytes_us > groups_us ? bytes_us : groups_us);
         }
         if (M <= 16 && !wide) {
