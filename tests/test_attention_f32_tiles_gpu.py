@@ -42,3 +42,21 @@ def test_tiles(H, Hk, D, Dv, mask, ps):
                 bound = (16 * (D + 4) + len(seen) + 8) * 2.0 ** -24 * (w @ np.abs(v[seen, h // (H // Hk)])) + 1e-30
                 assert (np.abs(got[t, h] - w @ v[seen, h // (H // Hk)]) <= bound).all(), (p, h)
             t += 1
+
+
+@pytest.mark.parametrize("H,Hk,D", [(2, 2, 16), (2, 2, 32), (8, 2, 64)])
+def test_rows_beside_a_row(H, Hk, D):
+    """Four rows of a workgroup and fewer take their softmax with a wave each, more with eight lanes each: the same bits."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    g = torch.Generator()
+    g.manual_seed(D)
+    n, ps = 200, 16
+    tables, n_pages = scatter_pages([n], ps, 2)
+    q, k, v = torch.randn(n, H * D, generator=g), torch.randn(n, Hk, D, generator=g), torch.randn(n, Hk, D, generator=g)
+    kc, vc = fill_cache([k], [k], tables, n_pages, ps, torch.float32)[0], fill_cache([v], [v], tables, n_pages, ps, torch.float32)[1]
+    run = lambda a, b: ops.attention(q[a:b].to(DEV), kc, vc, FakeCtx([a], [b - a], tables, ps), 0, H, Hk, D, ps, 1 / math.sqrt(D))
+    whole = run(0, n)
+    for a, b in ((0, 1), (63, 64), (64, 66), (120, 124), (128, 133), (199, 200)):
+        assert torch.equal(run(a, b), whole[a:b]), (a, b)

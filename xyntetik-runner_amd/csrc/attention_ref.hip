@@ -110,7 +110,9 @@ __global__ __launch_bounds__(64) void k_attention_ref(
 // 900 us and with this kernel 90, a decoded token of a tiny model 12 and 7.  Bound by the chain of a tile's steps in the workgroups that see
 // most keys: with a softmax row a wave at a time (eight rows one after another, each with twelve exchanges) and every tile's keys read
 // when the tile before was done, 90 us; all rows' softmax at once and the next tile fetched meanwhile 60; its pieces' places by a product
-// instead of divisions, and the row blocks that see most keys first 55; the pages looked up a step ahead 48.
+// instead of divisions, and the row blocks that see most keys first 55; the pages looked up a step ahead 48.  Lone tokens with a wave a row (eight lanes
+// a row had made heads of 16 and 32 slower than before all this) and heads of up to 32 with two pieces a thread, 650 keys: heads of 16 30.2 us, 33.4 and 24.5, of 32 38.9, 43.1
+// and 30.7, of 64 (584 keys) 50.5, 45.3 and 36.8.
 #define AF_ROWS 32
 #define AF_KEYS 64
 #define AF_MAX_D 128
@@ -280,7 +282,32 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
                     for (int e = 0; e < 4; ++e) S[(16 * i + 4 * quad + e) * AF_LD_S + 16 * wave + l16] = s[i][e];
             }
             __syncthreads();
-            {   // softmax: eight lanes a row, all rows at a time; a lane has keys 4 j .. 4 j + 3 of either half of the tile
+            // softmax: eight lanes a row, all rows at a time; a lane has keys 4 j .. 4 j + 3 of either half of the tile.  Up to four rows a wave each, a key a lane:
+            // one exponential behind the other is what eight keys a lane wait for.  Either way a row's exponentials are added up in one order.
+            // (What rows that do not exist have in S is their own results' alone, which are not stored.)
+            if (n_rows <= 4) {
+                const int r = wave, key = k0 + lane;
+                if (r < n_rows) {
+                    const int pos = row_pos[r], lo = row_lo[r];
+                    const bool valid = key >= from && key < to && (seg ? key >= lo && key <= pos : key < a.keep && key < lo);
+                    float y = S[r * AF_LD_S + lane] * a.scale;
+                    if (a.cap > 0.f) y = a.cap * tanhf(y / a.cap);
+                    if (a.slopes) y -= a.slopes[kvh * G + (r0 + r) % G] * (float)(pos - key);
+                    y = valid ? y : -INFINITY;
+                    const float m = row_m[r], mn = fmaxf(m, wave_max(y));
+                    const float p = valid ? expf(y - mn) : 0.f;
+                    S[r * AF_LD_S + lane] = p;
+                    float sum = p;
+#pragma unroll
+                    for (int o : {1, 2, 32, 16, 8, 4}) sum += __shfl_xor(sum, o, 64);
+                    if (lane == 0) {
+                        const float corr = m == -INFINITY ? 0.f : expf(m - mn);
+                        row_corr[r] = corr;
+                        row_l[r] = row_l[r] * corr + sum;
+                        row_m[r] = mn;
+                    }
+                }
+            } else {
                 const int r = tid >> 3, j = tid & 7;
                 float* const row = S + r * AF_LD_S + 4 * j;
                 if (r < n_rows) {
@@ -304,12 +331,9 @@ __global__ __launch_bounds__(256) void k_attention_f32(AttnF32 a) {
 #pragma unroll
                     for (int o = 4; o > 0; o >>= 1) mn = fmaxf(mn, __shfl_xor(mn, o, 64));
                     mn = fmaxf(m, mn);
-                    float sum = 0.f;
 #pragma unroll
-                    for (int x = 0; x < 8; ++x) {
-                        v[x] = valid[x] ? expf(v[x] - mn) : 0.f;
-                        sum += v[x];
-                    }
+                    for (int x = 0; x < 8; ++x) v[x] = valid[x] ? expf(v[x] - mn) : 0.f;
+                    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 #pragma unroll
                     for (int o = 4; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
                     *reinterpret_cast<float4*>(row) = make_float4(v[0], v[1], v[2], v[3]);
@@ -438,6 +462,7 @@ extern "C" int xr_attention_f32(float* out, const float* q, const float* k_cache
     const int widest = D > Dv ? D : Dv;
     const int keys = (D + 15) / 16;
     if (widest <= 16) return run(k_attention_f32<1, true>);
+    if (widest <= 32) return keys == 2 ? run(k_attention_f32<2, true>) : run(k_attention_f32<2, false>);
     if (widest <= 64) return keys == 4 ? run(k_attention_f32<4, true>) : run(k_attention_f32<4, false>);
     return keys == 8 ? run(k_attention_f32<8, true>) : run(k_attention_f32<8, false>);
 }
