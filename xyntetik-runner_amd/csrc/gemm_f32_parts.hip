@@ -386,7 +386,8 @@ double xr_f32_tiles_us(int M, int N, int K);       // gemm_ref.hip: k_gemm_f32's
 
 // Whether a 32-bit product of more than 16 rows is faster in parts: 0, or 1 + its tile + XR_PARTS_TILES * (ranges - 1).  Taken where this model's
 // time is a tenth below the other kernel's (whose model leaves out 3 us of a launch): of the 245 timed products (M, N, K) 23% faster on average (24%
-// with the better of the two everywhere), five more than 3% slower (8% at most).  Few columns stay with k_gemm_f32: there is no gain.
+// with the better of the two everywhere), five more than 3% slower (8% at most); 183 drawn ones (64 to 60,000 weight rows) 31%, four
+// 3 to 5% slower.  Few columns stay with k_gemm_f32: there is no gain.
 extern "C" int xr_gemm_f32_parts_plan(int M, int N, int K) {
     if (M <= 16 || K < 512 || K % (2 * PK) != 0 || N < 1 || (long long)M * N > (1ll << 31)) return 0;
     static const int tried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};

@@ -1965,7 +1965,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // tiles takes its products' time, bm bn K x 0.36e-12 / rate (`else_rate` where the four-wave loop does not take the product: K no
             // whole slices), or that of its
             // weights from memory at `bytes` a second, whichever is longer; a last round that fills the chip by a share f does its products
-            // in 1 - e + e f of that, e 0.082 and rotating 0.034 (fewer tiles meet at L2, and the clock falls less); `launch` once and `round` for every round:
+            // in 1 - e + e f of that, e 0.082 and rotating 0.526 (fewer tiles meet at L2, and the clock falls less); `launch` once and `round` for every round:
             // the tile's results leave, 2.6 times as long where they are 32-bit, or are rotated (512 rows of a 512 to 22,016 product are 172 tiles of
             // 256x256, 28.9 us, or 230 of 256x192, 19.6; 2,048 rows of a rotating 768 to 2,304 one 108 tiles of 256x192 with eight waves, 28.3 us, or of
             // 192x192 with four, 47.5).  Adding ranges up moves (ranges x their width + 2 N) M 4 bytes
@@ -1978,7 +1978,8 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             // the tile and ranges chosen are 0.9% slower on average than the best of all eight tiles (1.2% for products left out of a fit); with
             // numbers fitted to fewer and wider products, without `round`, `else_rate` and 256x192 tiles, it was 3.0%, at worst 47%.  Rotating
             // ones: 153 products of nine shapes, 512 to 4,096 rows, 0.4% (0.6%), at worst 11% (2,048 weight rows of 1,536 columns); with the numbers
-            // that fitted the rotation of 4 columns a lane 2.4%, at worst 17%.
+            // that fitted the rotation of 4 columns a lane 2.4%, at worst 17%.  (Of 635 others, drawn from 500 columns on and of all head sizes, 1.1%, 9% of them more than 5%,
+            // nearly all below 1,000 columns, at worst 41%; numbers fitted to those gain 0.3% on average and lose more than 3% on 7% of them.)
             // Of the tiles that were left out none brings 0.2% on average:
             // 192x256, 256x192 and 128x192 with four waves, 320x192, 320x128, 96x256, and a fifth or sixth slice in flight.
             // (Rotating products in 256x256, 256x192 and 256x128 tiles: the eight-wave kernels.)
