@@ -1462,23 +1462,24 @@ __global__ __launch_bounds__(64 * KSW, WHOLE && RT == 1 ? 4 : 1) void k_gemm_ski
     float* ss_s = scale_s + 256;                           // [SS_AHEAD][16 rows] (batches)
     float part_ss[16];
     const bool scales = MT == 1 && g.ss_in != nullptr && tid < 256;      // (more than 16 rows have none)
-    auto fetch_ss = [&](int p0) {
+    auto fetch_ss = [&]() {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) part_ss[i] = p0 + i * 16 < g.n_ss ? g.ss_in[(p0 + i * 16) * 16 + (tid & 15)] : 0.f;
+        for (int i = 0; i < 16; ++i) {
+            const int p = (tid >> 4) + i * 16;
+            part_ss[i] = g.ss_in[(p < g.n_ss ? p : 0) * 16 + (tid & 15)];
+        }
     };
     auto sum_ss = [&]() {
         if (!scales) return;
         float s = 0.f;
-        for (int p0 = tid >> 4;;) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s += part_ss[i];
-            if ((p0 += 256) >= g.n_ss) break;
-            fetch_ss(p0);
-        }
+        for (int i = 0; i < 16; ++i) s += (tid >> 4) + i * 16 < g.n_ss ? part_ss[i] : 0.f;
+#pragma unroll 1
+        for (int p = (tid >> 4) + 256; p < g.n_ss; p += 16) s += g.ss_in[p * 16 + (tid & 15)];
         scale_s[tid] = s;
     };
     if constexpr (WHOLE) {
-        if (scales) fetch_ss(tid >> 4);
+        if (scales) fetch_ss();
     } else if (MT == 1 && g.ss_in) {
         const int chunks = (g.n_ss < SS_AHEAD ? g.n_ss : SS_AHEAD) * 4;      // pieces of 16 bytes
         const uint32_t ss_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ss_s;
