@@ -1939,7 +1939,7 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
         // for 16, and a round more where they are just over 256.  The lesser of two models in us: tiles pay for the launch, for each further round,
         // and K for the weights of a full round from memory, or for what a lone tile waits for its own; the skinny kernels (plain, plain from 65,536 weight rows
         // on, gated) for the weights, or for their workgroups.  Fitted to 1,000 pairs of the two that run today (16,384 to 131,072 weight rows, K 512 to 8,192; a third of them
-        // held back): 0.3% slower than the better one on average, at most 16%, and at most 14% slower than the skinny kernel (once; the next 8%); with the numbers
+        // held back; 440 more since the same): 0.3% slower than the better one on average, at most 16%, and at most 14% slower than the skinny kernel; with the numbers
         // that fitted batches 2.0% and 34% (gated 19392 x 576 9 rows 12.3 us, in tiles 16.5; 80064 x 4672 9 rows 115 and 129); tiles wherever there are 160 8.1%, skinny always 4.4%.
         const int wide_tiles = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), wide_rounds = (wide_tiles + 255) / 256;
         bool wide = M > 8 && M <= 16 && !norm && !rope && w_packed && wide_tiles >= 160 && takes_written_order(g, 1, K, 64, 128, 4, 64);
@@ -2081,10 +2081,10 @@ extern "C" int xr_gemm_bf16(void* out, const void* a, const void* w, const float
             const bool pairs = !sw && !rope && N <= 2048 && K >= 2048 && !(g.xg && norm->ss_out_rows < (N + 7) / 8);
             const bool near = (size_t)16 * lda * 2 < (1ull << 32);      // the rings' offsets from the first row have 32 bits
             // Rings or batches.  Plain products below 65,536 weight rows, us, batches and rings: the rings' longer beginning does not pay for up to 512 columns (52960 x
-            // 384 at 4 rows 9.0 and 9.8, x 576 14.0 and 11.5), nor between one and two workgroups a compute unit from 2,048 to 4,096 columns (5120 x 2560 at 8 rows 8.2
-            // and 8.6, 6144 x 4096 11.5 and 11.9; 6144 x 1024 5.2 and 5.2, x 5120 15.7 and 14.9; 12288 x 4096 18.6 and 18.1), and with eight waves nothing from 5 rows
-            // on but for few columns (3072 x 4096 at one row 6.7 and 6.4, at 8 7.5 and 7.8, x 1536 5.1 and 4.7).  1,020 products of 170 drawn shapes (256 to 131,072
-            // weight rows, 256 to 16,384 columns, 1 to 16 rows, a third gated) take 0.90 of what batches alone take; 4 of them 3 to 9% longer.
+            // 384 at one row 8.9 and 9.4, x 576 13.4 and 11.3), nor between one and two workgroups a compute unit from 2,048 to 4,096 columns (5120 x 2560 at 8 rows 8.2
+            // and 8.4, 6144 x 4096 11.5 and 11.6; 6144 x 1024 5.2 and 4.9, x 5120 15.7 and 14.6; 12288 x 4096 18.6 and 18.1), and with eight waves nothing from 5 rows
+            // on but for few columns (3072 x 4096 at one row 6.8 and 6.5, x 12288 at 8 16.7 and 17.9, x 1536 5.1 and 4.6).  1,020 products of 170 drawn shapes (256 to
+            // 131,072 weight rows, 256 to 16,384 columns, 1 to 16 rows, a third gated) take 0.89 of what batches alone take; none that are rings take longer by more than runs differ.
             const bool four = N > 4096 || (N == 4096 && K >= 4096);     // waves of a ring (4096 x 4096 at 8 rows 8.1 us in eight, 7.8 in four; x 3968 8.3 and 9.0)
             const bool ring = near && K % 32 == 0 && (sw || N >= 65536 || (four ? N == 4096 || (K > 512 && !(N <= 8192 && K >= 2048 && K <= 4096))
                                                                                 : M <= 4 || K <= 1536));
