@@ -1,0 +1,105 @@
+"""Attention of requests with up to 16 rows a key/value head: the work list on the CPU, the kernel against the plain formula."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from xyntetik_runner_amd.engine.batch import Chunked, FEW_MIN_RANGE, few_row_items, first_key
+
+
+@pytest.mark.parametrize("mask", [None, 40, Chunked(48)])
+@pytest.mark.parametrize("extra", [False, True])
+@pytest.mark.parametrize("room", [0, 1, 7, 64])
+def test_items_cover_every_key_once(mask, extra, room):
+    rng = np.random.default_rng(room + 2 * extra)
+    starts, lens = rng.integers(0, 700, 9), rng.integers(1, 4, 9)
+    starts[0] = 0
+    req, q0s = np.arange(9) + 3, np.cumsum(lens) - lens
+    items, extras, n_slots = few_row_items(req, starts, lens, q0s, mask, 9 + room, extra, first_slot=5)
+    paired = few_row_items(req, starts, lens, q0s, mask, 9 + room, extra, first_slot=5, pair_at=7)[0]
+    assert paired[:7].tolist() == items[:7].tolist() and sorted(paired.tolist()) == sorted(items.tolist())
+    assert paired[7:].tolist() == (items[7:][::-1] if 7 < len(items) <= 14 else items[7:]).tolist()
+    longest = {it[10]: -(-max(x[3] - x[2] for x in items.tolist() if x[10] == it[10]) // 32) for it in items.tolist()}
+    assert len(items) <= 9 + room and (np.diff([longest[i] for i in items[:, 10]]) <= 0).all()
+    taken = []
+    for i in range(9):
+        mine = sorted((it for it in items.tolist() if it[0] == req[i]), key=lambda it: it[2])
+        at = first_key(mask, int(starts[i])) // 32 * 32
+        for it in mine:
+            assert it[2] == at and it[3] > at and it[5:8] == [q0s[i], lens[i], starts[i]] and it[10] == i and it[11] == len(mine)
+            at = it[3]
+        assert at == starts[i] + lens[i]
+        slots = [it[4] for it in mine]
+        if len(mine) == 1 and not extra:
+            assert slots == [-1]
+        else:
+            assert slots == list(range(mine[0][8], mine[0][8] + len(mine))) and mine[0][9] == len(mine) + extra
+            taken += slots + ([int(extras[i, 2])] if extra else [])
+            if extra:
+                assert extras[i].tolist() == [req[i], 0, slots[-1] + 1, q0s[i], lens[i], starts[i], 0, 0]
+    assert sorted(taken) == list(range(5, 5 + n_slots))
+    if room == 64 and mask is None:
+        assert (items[:, 3] - items[:, 2]).max() <= 32 * max(FEW_MIN_RANGE, -(-int((-(-(starts + lens) // 32)).sum()) // room))
+
+
+CASES = [
+    # H, Hk, D, Dv, page, mask, starts, q_lens
+    (4, 1, 32, 32, 32, None, [0, 31, 32, 33], [1, 1, 1, 1]),
+    (8, 2, 128, 128, 64, None, [0, 63, 64, 127, 128, 129, 500, 1900], [1] * 8),
+    (8, 2, 64, 64, 64, None, [1000, 5, 191, 192, 193], [1, 4, 3, 2, 1]),         # 16, 12, 8 and 4 rows
+    (16, 1, 64, 32, 32, None, [300, 2], [1, 1]),                                  # 16 heads a group; values of another size
+    (5, 5, 128, 128, 128, 100, [0, 99, 100, 101, 700], [16, 9, 3, 1, 2]),        # a window
+    (6, 2, 256, 256, 32, None, [400, 2], [5, 1]),
+    (4, 2, 256, 192, 64, Chunked(64), [63, 64, 200], [2, 1, 3]),
+    (4, 2, 128, 128, 64, None, [5000], [1]),                                      # more than 64 pages
+    (3, 3, 96, 96, 32, 33, [3000, 40], [1, 1]),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("room", [1, 1024])
+@pytest.mark.parametrize("case", CASES)
+def test_few_rows_kernel(case, room, monkeypatch):
+    from test_kernels_gpu import DEV, FakeCtx, fill_cache, ref_attention, scatter_pages
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    from xyntetik_runner_amd.engine import batch
+    H, Hk, D, Dv, ps, mask, starts, q_lens = case
+    monkeypatch.setattr(batch, "FEW_SLOTS", room)
+    torch.manual_seed(D + len(starts))
+    lens = [s + n for s, n in zip(starts, q_lens)]
+    tables, n_pages = scatter_pages(lens, ps, D)
+    ctx = FakeCtx(starts, q_lens, tables, ps)
+    ctx.plans_few_rows, ctx._plans, ctx.device = True, {}, DEV
+    ctx.attention_plan = lambda *a, **k: batch.StepContext.attention_plan(ctx, *a, **k)
+    T = sum(q_lens)
+    q = torch.randn(T, H, D).bfloat16()
+    k_seq = [torch.randn(n, Hk, D).bfloat16() for n in lens]
+    v_seq = [torch.randn(n, Hk, Dv).bfloat16() for n in lens]
+    # (a size of its own for values: caches filled apart)
+    kc, _ = fill_cache(k_seq, [torch.zeros(n, Hk, D).bfloat16() for n in lens], tables, n_pages, ps, torch.bfloat16)
+    _, vc = fill_cache([torch.zeros(n, Hk, Dv).bfloat16() for n in lens], v_seq, tables, n_pages, ps, torch.bfloat16)
+    scale = 1 / math.sqrt(D)
+    window = mask if isinstance(mask, int) else None
+    chunk = mask.size if isinstance(mask, Chunked) else None
+    want = torch.empty(T, H, Dv, dtype=torch.float64)
+    r = 0
+    for b, n in enumerate(q_lens):
+        for i in range(n):
+            p = starts[b] + i
+            lo = first_key(mask, p)
+            for h in range(H):
+                g = h // (H // Hk)
+                s = (k_seq[b][lo:p + 1, g].double() @ q[r, h].double()) * scale
+                want[r, h] = torch.softmax(s, 0) @ v_seq[b][lo:p + 1, g].double()
+            r += 1
+    plan = ctx.attention_plan(0, H // Hk, mask, Hk, ps, few_rows=2 if D + Dv <= 256 else 1)
+    assert plan.n_few >= len(starts) and plan.n_items == plan.n_cta_items == plan.n_jobs == 0
+    for _ in range(3):          # (the counters are zero again after every launch)
+        got = load_ops().attention(q.to(DEV).reshape(T, H * D).contiguous(), kc, vc, ctx, 0, H, Hk, D, ps, scale, window, chunk=chunk, v_head_dim=Dv)
+        assert int(plan.counters.abs().sum()) == 0
+        got = got.cpu().reshape(T, H, Dv)
+        assert torch.isfinite(got.float()).all()
+        # probabilities and the result in bfloat16 (2^-9 each of a value) against the largest output
+        err = (got.double() - want).abs().amax() / want.abs().amax()
+        assert err < 1.2e-2, float(err)

@@ -62,13 +62,15 @@ struct AttnArgs {
     bf16_t* out;            // [T, H, HV], rows ld_out apart
     const int* items;       // [n_items, ITEM_INTS]; q0: the request's first row, start: its first position
     const int* cta_items;   // [n_cta_items, ITEM_INTS]: the same for 128-row blocks that a whole workgroup takes
+    const int* few_items;   // [n_few, FEW_INTS]: row blocks of up to 16 rows (k_attn_few), with where their parts lie
+    int* counters;          // [row blocks of few rows, Hk], all zero between launches
     const int* cu_q;        // [B + 1] first row (token) of each request in this step
     const int* starts;      // [B] position of each request's first token of this step
     const int* block_table; // [B, table_stride]
     int table_stride;
     float* part_o;          // [slots, Hk, ROWS, HV]
     float* part_ml;         // [slots, Hk, ROWS, 2]
-    int n_items, n_cta_items, H, Hk, page_shift, page_mask, page_size;
+    int n_items, n_cta_items, n_few, H, Hk, page_shift, page_mask, page_size;
     float scale;
     int window;             // > 0: a row at position p reads the keys from p - window + 1 on
     int chunk;              // > 0: it reads from p - p mod chunk on (its own chunk of positions, counted from 0)
@@ -1053,6 +1055,325 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void k_attn_stream(AttnArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------ few rows
+// Decoded tokens (and portions of a few tokens): a request's rows of one key/value head are 16 at most.  What bounds it is
+// how fast keys and values arrive, and for few requests the chain of dependent reads before the first of them does.  So
+// fragments go from memory to registers, not through LDS: a wave holds a step's tiles while it multiplies and the next step's are
+// on their way, two workgroups a compute unit (two waves of 230 registers a SIMD); products are 16x16x32, so 16 rows, not 32, are computed
+// for the few that there are; and key ranges of a row block find their whole themselves: every workgroup writes its
+// partial result past the caches, counts itself in, and the last to do so adds them up (no workgroup waits for another, and
+// no kernel of its own: the merge's took 4.8 us).
+//
+//     S^T[key, row] = K[key, :] . Q[row, :]        v_mfma_f32_16x16x32_bf16, two blocks of 16 keys
+//     O^T[d, row]  += V^T[d, key] * P^T[key, row]
+//
+// Row m of key block b stands for key 8 (m / 4) + 4 b + m % 4 of the tile: the 8 scores that a lane holds are the 8 keys that
+// the second product wants from it.  Keys are read once and whole (marked as streaming); a tile's values are half of a page's
+// 128-byte lines, whose other half another wave reads at about the same time (streaming too 75.8 us for 71.4).
+//
+// k_attn_stream with its merge and this, 8 key/value heads of 128 channels, 4 query heads each, in a recorded chain: 1 request of 1,900 keys
+// 11.5 us -> 8.6, of 8,000 21.6 -> 13.6, 8 of 1,000 to 2,000 20.6 -> 16.2, 64 of 950 to 1,900 75.7 -> 68.8 (5.4 TB/s), of 8,000 372 -> 342 (6.2 TB/s);
+// 32 key/value heads, 23 of 450 to 900 64.4 -> 51.1; heads of 64 channels, 1 of 700 8.8 -> 6.9.  Measured and left: eight waves a workgroup
+// (68.1 us for 64 requests, but 54.1 for the 23 of 32 heads), three workgroups a compute unit (spills: 152), both tiles of a page a step at 128 channels (one wave a SIMD: 27 us for 8 requests).
+#define FEW_ROWS 16
+#define FEW_INTS 12                   // an item's 8 numbers (slot -1: it covers all keys), then first slot, slots, counter, items of its row block
+constexpr bool FEW_OK = HD % 32 == 0;
+constexpr int FKD = FEW_OK ? HD / 32 : 1, FDB = HV / 16;
+constexpr int FEW_WAVES = 4;
+constexpr int FEW_SUBS = HD + HV <= 128 ? 2 : 1;              // tiles of 32 keys a step
+constexpr int FEW_STEP = 32 * FEW_SUBS;
+constexpr int FEW_PER_CU = HD + HV <= 256 ? 2 : 1;            // workgroups a compute unit has registers for (the plan's ``few_rows``)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+struct FewTile {
+    u32x4_t k[FEW_SUBS][2][FKD], v[FEW_SUBS][FDB];
+    int pg[FEW_SUBS];
+};
+
+__device__ __forceinline__ bf16x8 frag(u32x4_t v) {
+    union { u32x4_t u; bf16x8 b; } c;
+    c.u = v;
+    return c.b;
+}
+// a word past the caches of this XCD, to where the workgroups of the others read it
+__device__ __forceinline__ void store_agent(float* p, float x, float y) {
+    const unsigned long long v = (unsigned long long)__float_as_uint(x) | (unsigned long long)__float_as_uint(y) << 32;
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_agent(const float* p) {
+    const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+}
+
+template <int MODE, bool OK = FEW_OK>
+__global__ __launch_bounds__(64 * FEW_WAVES, FEW_PER_CU) void k_attn_few(AttnArgs a) {
+    if constexpr (OK) {
+    constexpr int MS = HV + 4;                                // floats between rows of the combining buffer
+    __shared__ float mo[FEW_WAVES * FEW_ROWS * MS];
+    __shared__ float mml[FEW_WAVES * FEW_ROWS * 2];
+    __shared__ int last_one;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int item_no = (int)(blockIdx.x / (unsigned)a.Hk);
+    const int kvh = (int)blockIdx.x - item_no * a.Hk;
+    const int* it = a.few_items + (size_t)item_no * FEW_INTS;
+    const int req = it[0], row0 = it[1], kbeg = it[2], kend = it[3], slot = it[4];
+    const int q0 = it[5], q_len = it[6], start = it[7];
+    if (kend <= kbeg) return;                                 // (an item that pads a recorded step's list)
+    const int G = a.H / a.Hk;
+    const int lr = lane & 15, quad = lane >> 4;
+    const int seq_len = start + q_len;
+    const int* bt = a.block_table + (size_t)req * a.table_stride;
+
+    int pages_base = kbeg >> a.page_shift;
+    int my_page;
+    auto look_up = [&]() {
+        const int pi = pages_base + lane;
+        const bool in = ((long)pi << a.page_shift) < seq_len;
+        my_page = bt[in ? pi : 0];
+        my_page = in ? my_page : -1;
+    };
+    look_up();
+
+    const int rho = row0 + lr;
+    const int tok = rho / G, hg = rho - tok * G;
+    const bool row_ok = tok < q_len;
+    const int t = q0 + tok, h = kvh * G + hg;
+    const int pos = start + tok;
+    auto first = [&](int p) { return a.chunk > 0 ? p - p % a.chunk : (a.window > 0 && p - a.window + 1 > 0) ? p - a.window + 1 : 0; };
+    const int lo = first(pos);
+    const int last_tok = (row0 + FEW_ROWS - 1) / G;
+    const int pos_min = start + row0 / G;
+    const int lo_max = first(start + (last_tok < q_len ? last_tok : q_len - 1));
+    const float sb = MODE == MODE_SLOPES ? a.slopes[row_ok ? h : 0] / a.scale : 0.f;
+    bf16x8 qf[FKD];
+    {
+        const bf16_t* qp = a.q + ((size_t)(row_ok ? t : q0) * a.H + (row_ok ? h : 0)) * HD + quad * 8;
+#pragma unroll
+        for (int kd = 0; kd < FKD; ++kd) qf[kd] = as_bf16x8(keep_if(row_ok, ldg16(qp + kd * 32)));
+    }
+    const uint32_t koff = (uint32_t)(((lr >> 2) * 8 + (lr & 3)) * HD + quad * 8);
+    const uint32_t voff = (uint32_t)(lr * a.page_size + quad * 8);
+
+    // the tiles of this wave's j-th step, which exist
+    auto load = [&](FewTile& x, int j) __attribute__((always_inline)) {
+        const int k0 = kbeg + (wave + j * FEW_WAVES) * FEW_STEP;
+        if (((k0 + FEW_STEP - 1) >> a.page_shift) - pages_base >= 64) {
+            pages_base = k0 >> a.page_shift;
+            look_up();
+        }
+#pragma unroll
+        for (int u = 0; u < FEW_SUBS; ++u) {
+            const int kt = k0 + 32 * u;
+            const int pg = __builtin_amdgcn_readlane(my_page, __builtin_amdgcn_readfirstlane((kt >> a.page_shift) - pages_base));
+            x.pg[u] = pg;
+            const size_t pb = (size_t)(pg < 0 ? 0 : pg) * a.Hk + kvh;
+            const int ko = kt & a.page_mask;
+            const bf16_t* kb = a.kc + (pb * a.page_size + ko) * HD;
+            const bf16_t* vb = a.vc + pb * HV * a.page_size + ko;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int kd = 0; kd < FKD; ++kd)
+                    x.k[u][b][kd] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(kb + (koff + (uint32_t)(b * 4 * HD + kd * 32))));
+#pragma unroll
+            for (int d = 0; d < FDB; ++d)
+                x.v[u][d] = *reinterpret_cast<const u32x4_t*>(vb + (voff + (uint32_t)(d * 16 * a.page_size)));
+        }
+    };
+
+    f32x4 o[FDB];
+#pragma unroll
+    for (int d = 0; d < FDB; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[d][e] = 0.f;
+    float m = -INFINITY, l = 0.f;      // m in units of log2
+    const float c2 = MODE == MODE_CAP ? 1.0f : a.scale * 1.44269504088896340736f;
+    const SoftCap cap(a.scale, a.cap);
+
+    auto compute = [&](FewTile& x, int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < FEW_SUBS; ++u) {
+            const int kt = kbeg + (wave + j * FEW_WAVES) * FEW_STEP + 32 * u;
+            if (FEW_SUBS > 1 && u > 0 && kt >= kend) break;
+            float s[8];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                f32x4 z;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) z[e] = MODE == MODE_SLOPES ? sb * (float)(kt + 8 * quad + 4 * b + e - pos) : 0.f;
+#pragma unroll
+                for (int kd = 0; kd < FKD; ++kd) z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(x.k[u][b][kd]), qf[kd], z, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[4 * b + e] = MODE == MODE_CAP ? cap.less(z[e], 0.f) : z[e];
+            }
+            const bool whole = kt + 32 <= kend && kt + 31 <= pos_min && kt >= lo_max;
+            if (!whole) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int key = kt + 8 * quad + e;
+                    const bool ok = row_ok && key <= pos && key >= lo && key < kend;
+                    s[e] = ok ? s[e] : -INFINITY;
+                }
+            }
+            if (kt + 32 > seq_len || x.pg[u] < 0) {        // the request's last tile: slots past its end hold old data
+                const int k8 = kt + 8 * quad, end = x.pg[u] < 0 ? 0 : seq_len;
+                u32x4_t mk;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    mk[e] = (k8 + 2 * e < end ? 0x0000FFFFu : 0u) | (k8 + 2 * e + 1 < end ? 0xFFFF0000u : 0u);
+#pragma unroll
+                for (int d = 0; d < FDB; ++d) x.v[u][d] &= mk;
+            }
+            float mt = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7]))) * c2;
+            // (the reference moves only where a maximum is more than 2^MAX_SLACK above it: no exchange between lanes otherwise)
+            if (__any(mt > m + MAX_SLACK)) {
+                mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+                mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+                const float mn = mt > m + MAX_SLACK ? mt : m;
+                const float corr = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+                m = mn;
+                l *= corr;
+#pragma unroll
+                for (int d = 0; d < FDB; ++d)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[d][e] *= corr;
+            }
+            const float mu = m == -INFINITY ? 0.f : m;
+            float p[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                p[e] = __builtin_amdgcn_exp2f(fmaf(s[e], c2, -mu));
+                l += p[e];
+            }
+            const bf16x8 pf = as_bf16x8(make_uint4(pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7])));
+#pragma unroll
+            for (int d = 0; d < FDB; ++d) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(x.v[u][d]), pf, o[d], 0, 0, 0);
+        }
+    };
+
+    const int n_steps = (kend - kbeg + FEW_STEP - 1) / FEW_STEP;
+    const int n = n_steps > wave ? (n_steps - wave + FEW_WAVES - 1) / FEW_WAVES : 0;
+    if (n > 0) {
+        FewTile x, y;
+        load(x, 0);
+        int j = 0;
+        for (; j + 2 < n; j += 2) {
+            load(y, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(x, j);
+            __builtin_amdgcn_sched_barrier(0);
+            load(x, j + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(y, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (j + 1 < n) {
+            load(y, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(x, j);
+            compute(y, j + 1);
+        } else {
+            compute(x, j);
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);                          // the row's sum from its four lanes
+
+    // ---- combine the waves: sum_w 2^(m_w - max) O_w over sum_w 2^(m_w - max) l_w
+    if (row_ok) {
+        float* dst = mo + (wave * FEW_ROWS + lr) * MS + quad * 4;
+#pragma unroll
+        for (int d = 0; d < FDB; ++d) *reinterpret_cast<float4*>(dst + d * 16) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]);
+        if (quad == 0) {
+            mml[(wave * FEW_ROWS + lr) * 2] = m;
+            mml[(wave * FEW_ROWS + lr) * 2 + 1] = l;
+        }
+    }
+    __syncthreads();
+    const int n_rows = q_len * G - row0 < FEW_ROWS ? q_len * G - row0 : FEW_ROWS;
+    for (int idx = tid; idx < n_rows * (HV / 2); idx += 64 * FEW_WAVES) {
+        const int r = idx / (HV / 2), d2 = (idx - r * (HV / 2)) * 2;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < FEW_WAVES; ++w) mx = fmaxf(mx, mml[(w * FEW_ROWS + r) * 2]);
+        float2 acc = make_float2(0.f, 0.f);
+        float lsum = 0.f;
+#pragma unroll
+        for (int w = 0; w < FEW_WAVES; ++w) {
+            const float mw = mml[(w * FEW_ROWS + r) * 2], lw = mml[(w * FEW_ROWS + r) * 2 + 1];
+            const float f = lw > 0.f ? __builtin_amdgcn_exp2f(mw - mx) : 0.f;
+            const float2 v = *reinterpret_cast<const float2*>(mo + (w * FEW_ROWS + r) * MS + d2);
+            acc.x += f * v.x; acc.y += f * v.y;
+            lsum += f * lw;
+        }
+        const int rr = row0 + r, tk = rr / G, hh = kvh * G + (rr - tk * G);
+        if (slot < 0) {
+            lsum = with_sink(a.sinks, hh, mx, lsum);
+            const float inv = (lsum > 0.f ? 1.0f / lsum : 0.f) * row_factor(a.gate, a.ld_gate, a.out_scale, q0 + tk, hh);
+            bf16_t* op = a.out + (size_t)(q0 + tk) * a.ld_out + hh * HV + d2;
+            *reinterpret_cast<uint32_t*>(op) = pack2(acc.x * inv, acc.y * inv);
+        } else {
+            const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+            store_agent(a.part_o + (((size_t)slot * a.Hk + kvh) * ROWS + r) * HV + d2, acc.x * inv, acc.y * inv);
+            if (d2 == 0) store_agent(a.part_ml + (((size_t)slot * a.Hk + kvh) * ROWS + r) * 2, mx, lsum);
+        }
+    }
+    if (slot < 0) return;
+
+    // ---- the last of a row block's workgroups adds the key ranges up.  Each has its partial result where all others read it
+    // (the wait is for this wave's own stores) before it counts itself in; the counter is zero again afterwards.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const int s0 = it[8], ns = it[9];
+    if (tid == 0) {
+        int* count = a.counters + (size_t)it[10] * a.Hk + kvh;
+        const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_one = before == it[11] - 1;
+        if (before == it[11] - 1) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last_one) return;
+    for (int idx = tid; idx < n_rows * (HV / 2); idx += 64 * FEW_WAVES) {
+        const int r = idx / (HV / 2), d2 = (idx - r * (HV / 2)) * 2;
+        const float* ml = a.part_ml + (((size_t)s0 * a.Hk + kvh) * ROWS + r) * 2;
+        const float* po = a.part_o + (((size_t)s0 * a.Hk + kvh) * ROWS + r) * HV + d2;
+        const size_t ml_step = (size_t)a.Hk * ROWS * 2, po_step = (size_t)a.Hk * ROWS * HV;
+        constexpr int U = 16;                            // slots whose loads are on their way together
+        float mx = -INFINITY, wsum = 0.f;
+        float2 acc = make_float2(0.f, 0.f);
+        for (int b = 0; b < ns; b += U) {
+            float2 mlv[U], pv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int sc = b + u < ns ? b + u : b;
+                mlv[u] = load_agent(ml + sc * ml_step);
+                pv[u] = load_agent(po + sc * po_step);
+            }
+            float cm = mx;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (b + u < ns) cm = fmaxf(cm, mlv[u].x);
+            const float resc = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - cm);
+            acc.x *= resc; acc.y *= resc;
+            wsum *= resc;
+            mx = cm;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float w = (b + u < ns && mlv[u].y > 0.f) ? mlv[u].y * __builtin_amdgcn_exp2f(mlv[u].x - mx) : 0.f;
+                acc.x += w * pv[u].x; acc.y += w * pv[u].y;
+                wsum += w;
+            }
+        }
+        const int rr = row0 + r, tk = rr / G, hh = kvh * G + (rr - tk * G);
+        wsum = with_sink(a.sinks, hh, mx, wsum);
+        const float inv = (wsum > 0.f ? 1.0f / wsum : 0.f) * row_factor(a.gate, a.ld_gate, a.out_scale, q0 + tk, hh);
+        bf16_t* op = a.out + (size_t)(q0 + tk) * a.ld_out + hh * HV + d2;
+        *reinterpret_cast<uint32_t*>(op) = pack2(acc.x * inv, acc.y * inv);
+    }
+    }
+}
+
 // One merge job: {req, row0, first_slot, n_slots, slot_stride, q0, q_len}.  Slot s holds the normalised output of
 // its keys with their maximum m_s (in units of log2) and sum l_s; the whole is
 // sum_s w_s O_s / sum_s w_s with w_s = l_s * 2^(m_s - max m).
@@ -1150,6 +1471,10 @@ static int launch_mode(const AttnArgs& a, const int* jobs, int n_jobs, const int
         k_attn_stream<MODE><<<dim3((unsigned)a.n_items * (unsigned)a.Hk), 64 * STREAM_WAVES, STREAM_LDS_BYTES, stream>>>(a);
         XR_CHECK_LAUNCH("attention_stream");
     }
+    if (a.n_few > 0) {
+        k_attn_few<MODE><<<dim3((unsigned)a.n_few * (unsigned)a.Hk), 64 * FEW_WAVES, 0, stream>>>(a);
+        XR_CHECK_LAUNCH("attention_few");
+    }
     if (n_jobs > 0) {
         MergeArgs mg;
         mg.jobs = jobs; mg.cu_q = cu_q; mg.part_o = a.part_o; mg.part_ml = a.part_ml; mg.out = a.out;
@@ -1164,7 +1489,8 @@ static int launch_mode(const AttnArgs& a, const int* jobs, int n_jobs, const int
 extern "C" int xr_attn_head_dim() { return HD; }
 
 extern "C" int xr_attention_mfma(void* out, const void* q, const void* k_cache, const void* v_cache,
-                                 const int* items, int n_items, int n_cta_items, const int* jobs, int n_jobs,
+                                 const int* items, int n_items, int n_cta_items, const int* few_items, int n_few, int* counters,
+                                 const int* jobs, int n_jobs,
                                  const int* cu_q,
                                  const int* starts, const int* block_table, int table_stride, float* part_o,
                                  float* part_ml, int H, int Hk, int D, int Dv, int page_size, float scale, int window,
@@ -1181,8 +1507,13 @@ extern "C" int xr_attention_mfma(void* out, const void* q, const void* k_cache, 
     XR_REQUIRE((long long)n_cta_items * Hk < (1LL << 31) && (long long)n_items * Hk < (1LL << 31), "attention: %d items of %d key/value heads are more workgroups than a launch takes", n_items + n_cta_items, Hk);
     XR_REQUIRE(n_cta_items == 0 || page_size >= 32, "attention: 128-row items need pages of at least 32 positions, got %d", page_size);
     XR_REQUIRE(n_jobs == 0 || (part_o && part_ml && jobs), "attention: split work without partial buffers");
-    if (n_items + n_cta_items == 0) return XR_OK;
+    XR_REQUIRE(n_few >= 0 && (long long)n_few * Hk < (1LL << 31), "attention: %d blocks of few rows of %d key/value heads", n_few, Hk);
+    XR_REQUIRE(n_few == 0 || (FEW_OK && page_size >= 32 && scale > 0.f && few_items && counters),
+               "attention: blocks of few rows need heads in steps of 32, pages of at least 32 positions, a positive scale and counters");
+    XR_REQUIRE(n_few == 0 || (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0, "attention: queries and cache must be 16-byte aligned");
+    if (n_items + n_cta_items + n_few == 0) return XR_OK;
     AttnArgs a;
+    a.few_items = few_items; a.n_few = n_few; a.counters = counters;
     a.q = (const bf16_t*)q; a.kc = (const bf16_t*)k_cache; a.vc = (const bf16_t*)v_cache; a.out = (bf16_t*)out;
     // the list begins with the items of the workgroup kernel
     a.cta_items = items; a.n_cta_items = n_cta_items; a.items = items + (size_t)n_cta_items * ITEM_INTS; a.cu_q = cu_q; a.starts = starts; a.block_table = block_table; a.table_stride = table_stride;

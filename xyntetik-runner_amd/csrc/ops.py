@@ -915,8 +915,7 @@ class Ops:
             extra = keep_first > 0
             lib = self.attention_lib(D, Dv)
             mask = Chunked(int(chunk)) if chunk else window
-            plan = (ctx.attention_plan(group, H // Hk, mask, Hk, page_size, extra_slot=True) if extra
-                    else ctx.attention_plan(group, H // Hk, mask, Hk, page_size))
+            plan = self._attention_plan(ctx, group, H, Hk, D, Dv, page_size, scale, mask, extra, q, k_cache, v_cache)
             part_o = part_ml = None
             if plan.n_slots:
                 part_o = torch.empty((plan.n_slots, Hk, 32, Dv), dtype=torch.float32, device=q.device)
@@ -929,7 +928,7 @@ class Ops:
                     float(softcap), dtype_code(q.dtype), _stream()))
             lib.check(lib.xr_attention_mfma(
                 out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), plan.items.data_ptr(),
-                plan.n_items, plan.n_cta_items, _ptr(plan.jobs), plan.n_jobs, ctx.cu_q.data_ptr(),
+                plan.n_items, plan.n_cta_items, _ptr(plan.few), plan.n_few, _ptr(plan.counters), _ptr(plan.jobs), plan.n_jobs, ctx.cu_q.data_ptr(),
                 ctx.starts_dev.data_ptr(), block_table.data_ptr(), block_table.stride(0), _ptr(part_o), _ptr(part_ml), H, Hk, D, Dv, page_size,
                 float(scale), int(window or 0), int(chunk or 0), _ptr(slopes), None if extra else _ptr(sinks),
                 float(softcap), *gating, _stream()))
@@ -948,6 +947,15 @@ class Ops:
             float(scale), int(window or 0), int(chunk or 0), int(keep_first), dtype_code(q.dtype), _ptr(slopes),
             _ptr(sinks), float(softcap), *gating, _stream()))
         return out
+
+    @staticmethod
+    def _attention_plan(ctx, group: int, H: int, Hk: int, D: int, Dv: int, page_size: int, scale: float, mask, extra: bool, q, k_cache, v_cache):
+        """The step's work list.  Requests of up to 16 rows a key/value head may go to the kernel for few rows where keys come in whole
+        products of 32 channels, a larger score is a larger product (a positive scale) and 16-byte loads are aligned."""
+        few = (getattr(ctx, "plans_few_rows", False) and D % 32 == 0 and scale > 0.0
+               and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) & 15)
+        more = {**({"extra_slot": True} if extra else {}), **({"few_rows": 2 if D + Dv <= 256 else 1} if few else {})}
+        return ctx.attention_plan(group, H // Hk, mask, Hk, page_size, **more)
 
     def attention_on_matrix_cores(self, dtype: torch.dtype, D: int, Dv: int, page_size: int = 64) -> bool:
         """Whether keys of ``D`` and values of ``Dv`` channels have matrix-core attention kernels."""
@@ -1033,7 +1041,7 @@ class Ops:
         if lib is None:
             unit = f"attn_d{D}" if D == Dv else f"attn_d{D}v{Dv}"
             path = _build.find_built(unit) or _build.build_unit(unit)
-            lib = _Lib(path, {"xr_attention_mfma": [_p, _p, _p, _p, _p, _i, _i, _p, _i, _p, _p, _p, _i, _p, _p,
+            lib = _Lib(path, {"xr_attention_mfma": [_p, _p, _p, _p, _p, _i, _i, _p, _i, _p, _p, _i, _p, _p, _p, _i, _p, _p,
                                                     _i, _i, _i, _i, _i, _f, _i, _i, _p, _p, _f, _p, _i, _f, _i, _p]})
             self._attn_libs[(D, Dv)] = lib
         return lib
@@ -1860,7 +1868,7 @@ class Ops:
             # The window's keys go to the matrix-core kernels, every row block leaving a partial
             # result; the block means leave theirs in a slot of their own; the kernels' merge adds them.
             lib = self.attention_lib(D)
-            plan = ctx.attention_plan(group, H // Hk, size, Hk, page_size, extra_slot=bool(P))
+            plan = self._attention_plan(ctx, group, H, Hk, D, D, page_size, scale, size, bool(P), q, k_cache, v_cache)
             part_o = part_ml = None
             if plan.n_slots:
                 part_o = torch.empty((plan.n_slots, Hk, 32, D), dtype=torch.float32, device=q.device)
@@ -1872,7 +1880,7 @@ class Ops:
                     int(P), dtype_code(q.dtype), _stream()))
             lib.check(lib.xr_attention_mfma(
                 out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), plan.items.data_ptr(),
-                plan.n_items, plan.n_cta_items, _ptr(plan.jobs), plan.n_jobs, ctx.cu_q.data_ptr(),
+                plan.n_items, plan.n_cta_items, _ptr(plan.few), plan.n_few, _ptr(plan.counters), _ptr(plan.jobs), plan.n_jobs, ctx.cu_q.data_ptr(),
                 ctx.starts_dev.data_ptr(), table.data_ptr(), table.stride(0), _ptr(part_o), _ptr(part_ml), H, Hk, D, D, page_size,
                 float(scale), int(size), 0, None, None, 0.0, None, 0, 1.0, out.stride(0), _stream()))
             return out

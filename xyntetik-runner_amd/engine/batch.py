@@ -43,6 +43,9 @@ class AttentionPlan:
     n_cta_items: int = 0
     extras: Optional[torch.Tensor] = None      # [n_extras, 8] (see ``plan_attention``, ``extra_slot``)
     n_extras: int = 0
+    few: Optional[torch.Tensor] = None         # [n_few, 12]: blocks of up to 16 rows (see ``few_row_items``)
+    n_few: int = 0
+    counters: Optional[torch.Tensor] = None    # [row blocks of few rows x key/value heads], zero between launches
 
 
 def first_key(mask, pos: int) -> int:
@@ -71,6 +74,12 @@ ATTN_CTA_MIN_ROWS = 64  # a request brings at least this many rows to be served 
 ATTN_STREAM_SLOTS = 256 # workgroups of the streaming kernel that run at a time (one a compute unit)
 ATTN_MIN_RANGE = 4      # tiles: the shortest key range worth a workgroup
 ATTN_CTA_FILL = 256     # 128-row items (times key/value heads) that give every compute unit one workgroup
+FEW_ROWS = 16           # rows of an item of the kernel for few rows (a request's tokens x heads-in-group, at most)
+FEW_PAGE = 32           # and the smallest page it takes
+FEW_INTS = 12           # numbers of such an item
+FEW_MIN_RANGE = 4       # tiles: its shortest key range (a tile a wave)
+FEW_SLOTS = 256         # workgroups of it that a step's requests are cut into: one a compute unit (twice as many cost the merge more than
+                        # they gain: 1 request of 8,000 keys 13.6 us -> 17.6, 16 of 330 10.7 -> 11.3, 32 of 1,000 to 2,000 with heads of 64 25.1 -> 26.2)
 
 
 def key_ranges(tiles: int, share: float) -> int:
@@ -85,10 +94,10 @@ def key_ranges(tiles: int, share: float) -> int:
 
 
 def plan_attention(starts, q_lens, group_size: int, window, n_kv_heads: int,
-                   page_size: int = 64, cta_tiles: Optional[int] = None, extra_slot: bool = False):
+                   page_size: int = 64, cta_tiles: Optional[int] = None, extra_slot: bool = False, skip=()):
     """Host side of ``AttentionPlan``: ``(cta_items, items, jobs, n_slots)`` as plain Python ints.
 
-    ``window``: None, a window's length, or a ``Chunked``.
+    ``window``: None, a window's length, or a ``Chunked``.  ``skip``: requests that are planned elsewhere.
 
     ``cta_tiles`` fixes the most tiles a 128-row item may cover (for measurements); by
     default it follows from how many such items the step has.
@@ -115,6 +124,8 @@ def plan_attention(starts, q_lens, group_size: int, window, n_kv_heads: int,
         return lo, hi, -(-(hi - lo) // ATTN_TILE)
 
     for b, (s, n) in enumerate(zip(starts, q_lens)):
+        if b in skip:
+            continue
         rows = n * group_size
         if rows >= ATTN_CTA_MIN_ROWS and page_size >= ATTN_TILE:
             for row0 in range(0, rows, ATTN_CTA_ROWS):
@@ -194,6 +205,68 @@ def plan_attention(starts, q_lens, group_size: int, window, n_kv_heads: int,
     return cta_items, items, jobs, slot
 
 
+def few_row_items(req, starts, lens, q0s, mask, room: int, extra_slot: bool, first_slot: int = 0, pair_at: int = 0):
+    """The work of the kernel for few rows: requests ``req`` of a step, each with one row block (its ``lens[i]`` tokens from row
+    ``q0s[i]`` and position ``starts[i]`` on), cut into at most ``room`` key ranges of about one length, so that a
+    long request takes as many workgroups as its keys are worth: ``(items [n, 12], extras [len(req), 8], slots)`` as int64 arrays.
+
+    An item: request, 0, first key, end key, partial slot (-1: all its keys), the request's first row, its tokens, its first
+    position, the row block's first slot, its slots, its counter and how many items it has.  With ``extra_slot`` a row block has
+    one slot more, its last, for a partial result of another kernel (``extras`` as ``plan_attention`` makes them).
+
+    The requests with the longest ranges come first, workgroups start in the items' order.  ``pair_at``: the items that give every compute unit one workgroup, where
+    it holds two at a time: if there are up to twice as many, all run at once, and the second half comes shortest first, so that
+    a unit has a long and a short one (64 requests of 950 to 1,900 keys 71.3 us -> 68.8, of 100 to 4,000 117.8 -> 96.8; 48 of 950 to 1,900 65.6 -> 57.8)."""
+    starts, lens = np.asarray(starts, dtype=np.int64), np.asarray(lens, dtype=np.int64)
+    n = len(starts)
+    hi = starts + lens
+    if mask:
+        lo = starts - starts % mask.size if isinstance(mask, Chunked) else np.maximum(0, starts - mask + 1)
+        lo = lo // ATTN_TILE * ATTN_TILE
+    else:
+        lo = 0
+    tiles = (hi - lo + (ATTN_TILE - 1)) // ATTN_TILE
+    # the shortest length c with at most ``room`` ranges: ceil(t / c) a request, which c >= total / (room - requests) has in any case
+    t = tiles.tolist()
+    longest = max(t)
+    if room > n:
+        total = sum(t)
+        most = max(FEW_MIN_RANGE, -(-total // (room - n)))
+        for c in range(max(FEW_MIN_RANGE, -(-total // room)), most, max(1, most // 32)):
+            if sum([-(-x // c) for x in t]) <= room:
+                most = c
+                break
+        longest = min(longest, most)
+    rec = np.zeros((n, FEW_INTS), dtype=np.int64)            # a request's items have this in common; 1: the keys of a range
+    rec[:, 0], rec[:, 2], rec[:, 3], rec[:, 5], rec[:, 6], rec[:, 7], rec[:, 10] = req, lo, hi, q0s, lens, starts, np.arange(n)
+    n_slots, extras = 0, rec[:0, :8]
+    if longest < max(t) or extra_slot:
+        parts = (tiles + (longest - 1)) // longest
+        per = (tiles + (parts - 1)) // parts
+        parts = (tiles + (per - 1)) // per
+        slots = parts + 1 if extra_slot else np.where(parts > 1, parts, 0)
+        end = np.cumsum(slots)
+        n_slots = int(end[-1])
+        rec[:, 1], rec[:, 8], rec[:, 9], rec[:, 11] = per * ATTN_TILE, first_slot + end - slots, slots, parts
+        if extra_slot:
+            extras = np.zeros((n, 8), dtype=np.int64)
+            extras[:, 0], extras[:, 2], extras[:, 3], extras[:, 4], extras[:, 5] = req, rec[:, 8] + parts, q0s, lens, starts
+        order = np.argsort(-per, kind="stable")
+        parts = parts[order]
+        items = np.repeat(rec[order], parts, axis=0)
+        k = np.arange(len(items)) - np.repeat(np.cumsum(parts) - parts, parts)
+        items[:, 2] += k * items[:, 1]
+        items[:, 3] = np.minimum(items[:, 3], items[:, 2] + items[:, 1])
+        items[:, 4] = np.where(items[:, 9] > 0, items[:, 8] + k, -1)
+        items[:, 1] = 0
+    else:
+        rec[:, 4], rec[:, 11] = -1, 1
+        items = rec[np.argsort(-tiles, kind="stable")]
+    if 0 < pair_at < len(items) <= 2 * pair_at:
+        items[pair_at:] = items[pair_at:][::-1].copy()
+    return items, extras, n_slots
+
+
 @dataclass
 class StepEntry:
     req_id: Hashable
@@ -203,6 +276,8 @@ class StepEntry:
 
 class StepContext:
     """Device views of one step's metadata, handed to every part."""
+
+    plans_few_rows = True       # its attention plans know the kernel for few rows
 
     def __init__(self, ops, device, entries: List[StepEntry], request_caches, n_groups: int, pad_to: int = 0):
         self.ops = ops
@@ -276,23 +351,40 @@ class StepContext:
         self.shared = {}        # what parts make once a step and share between layers (a rotation's table)
 
     def attention_plan(self, group: int, group_size: int, window, n_kv_heads: int,
-                       page_size: int = 64, extra_slot: bool = False) -> AttentionPlan:
-        """The MFMA attention work list, made once per step and shared by all layers that can."""
-        key = (group_size, window, n_kv_heads, page_size, extra_slot)
+                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0) -> AttentionPlan:
+        """The MFMA attention work list, made once per step and shared by all layers that can.  ``few_rows`` > 0:
+        requests of up to 16 rows a key/value head go to the kernel for few rows (where the page size allows), of which a compute unit
+        holds so many workgroups."""
+        key = (group_size, window, n_kv_heads, page_size, extra_slot, few_rows)
         plan = self._plans.get(key)
         if plan is None:
+            few = [b for b, n in enumerate(self.q_lens) if few_rows and page_size >= FEW_PAGE and n * group_size <= FEW_ROWS]
             planned = plan_attention(self.starts, self.q_lens, group_size, window, n_kv_heads, page_size,
-                                     extra_slot=extra_slot)
+                                     extra_slot=extra_slot, skip=frozenset(few))
             cta_items, items, jobs, n_slots = planned[:4]
-            extras = planned[4] if extra_slot else []
-            flat = ([v for it in cta_items + items for v in it] + [v for j in jobs for v in j]
-                    + [v for x in extras for v in x])
+            extras = [tuple(x) for x in planned[4]] if extra_slot else []
+            flat = [v for it in cta_items + items for v in it] + [v for j in jobs for v in j]
+            n_few = n_count = 0
+            if few:
+                q0s = np.concatenate([[0], np.cumsum(self.q_lens)])[few]
+                room = max(len(few), FEW_SLOTS // n_kv_heads)
+                few_items, few_extras, more = few_row_items(few, [self.starts[b] for b in few], [self.q_lens[b] for b in few], q0s,
+                                                            window, room, extra_slot, n_slots, ATTN_STREAM_SLOTS // n_kv_heads if few_rows == 2 else 0)
+                n_slots += more
+                n_few, n_count = len(few_items), len(few) * n_kv_heads
+                extras += few_extras.tolist()
+            flat += [v for x in extras for v in x]
+            if few:
+                flat += few_items.ravel().tolist() + [0] * n_count
             host = torch.tensor(flat, dtype=torch.int32).pin_memory()
             dev = host.to(self.device, non_blocking=True)
             nc, ni, nj = len(cta_items), len(items), len(jobs)
             nw = (nc + ni) * 8
-            plan = AttentionPlan(dev[:nw], ni, dev[nw:nw + nj * 7] if nj else None, nj, n_slots, nc,
-                                 dev[nw + nj * 7:] if extras else None, len(extras))
+            nx = nw + nj * 7
+            nf = nx + len(extras) * 8
+            plan = AttentionPlan(dev[:nw], ni, dev[nw:nx] if nj else None, nj, n_slots, nc,
+                                 dev[nx:nf] if extras else None, len(extras),
+                                 dev[nf:nf + n_few * FEW_INTS] if n_few else None, n_few, dev[nf + n_few * FEW_INTS:] if n_few else None)
             plan._host = host
             self._plans[key] = plan
         return plan

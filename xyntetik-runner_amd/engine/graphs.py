@@ -22,7 +22,8 @@ import numpy as np
 import torch
 
 from ..cache import NULL_PAGE
-from .batch import ATTN_MIN_RANGE, ATTN_STREAM_SLOTS, ATTN_TILE, AttentionPlan, Chunked, StepEntry, mask_reach
+from .batch import (ATTN_MIN_RANGE, ATTN_STREAM_SLOTS, ATTN_TILE, FEW_INTS, FEW_MIN_RANGE, FEW_PAGE, FEW_ROWS, FEW_SLOTS, AttentionPlan,
+                    Chunked, StepEntry, few_row_items, mask_reach)
 
 BUCKETS = (1, 2, 4, 8, 16, 32, 64, 128, 256, 512)
 SPLITS = (1, 2, 4, 8, 16, 32)
@@ -53,8 +54,16 @@ def splits_for(batch_cap: int, max_tiles: int, n_kv_heads: int) -> int:
     return best
 
 
+def few_row_splits(batch_cap: int, tiles: int, n_kv_heads: int) -> int:
+    """Key ranges a request that the kernel for few rows has room for: as many as fill its workgroups, and no more than ranges of
+    the shortest length (and one for what the requests' last ranges lack)."""
+    return max(1, min(FEW_SLOTS // (batch_cap * n_kv_heads), -(-tiles // FEW_MIN_RANGE) + 1))
+
+
 class StaticDecodeContext:
     """A ``StepContext`` for one token per request whose device arrays never move."""
+
+    plans_few_rows = True
 
     def __init__(self, ops, device, batch_cap: int, n_splits: int, table_widths: List[int],
                  windowed: Optional[List[bool]] = None, max_tiles: Optional[int] = None, *, null_slot: int):
@@ -78,10 +87,11 @@ class StaticDecodeContext:
         # [token_ids B][positions B][req_of_token B][cu_q B+1][seq_lens B][slots B][fresh B][starts B][want B]
         # [tables ...][plans ...]
         self._sizes = [B, B, B, B + 1, B, B, B, B, B] + [B * w for w in self.table_width]
-        self._plan_keys: List[Tuple[int, Optional[int], int, bool]] = []
-        self._plans: Dict[Tuple[int, Optional[int], int, bool], AttentionPlan] = {}
-        self._plan_off: Dict[Tuple[int, Optional[int], int, bool], int] = {}
-        self._plan_splits: Dict[Tuple[int, Optional[int], int, bool], int] = {}
+        # (group size, window, key/value heads, a slot more, workgroups of the kernel for few rows a compute unit holds: 0 another kernel)
+        self._plan_keys: List[Tuple[int, Optional[int], int, bool, int]] = []
+        self._plans: Dict[tuple, AttentionPlan] = {}
+        self._plan_off: Dict[tuple, int] = {}
+        self._plan_splits: Dict[tuple, int] = {}
         self._alloc()
         self.fresh_slots_host: List[int] = []
         self._copied = None
@@ -89,7 +99,8 @@ class StaticDecodeContext:
 
     def _alloc(self) -> None:
         B = self.B
-        n_plan = sum(B * self._plan_splits[k] * 8 + B * 7 + (B * 8 if k[3] else 0) for k in self._plan_keys)
+        n_plan = sum((B * self._plan_splits[k] * FEW_INTS + B * k[2] if k[4] else B * self._plan_splits[k] * 8 + B * 7) + (B * 8 if k[3] else 0)
+                     for k in self._plan_keys)
         offs = np.concatenate([[0], np.cumsum(self._sizes)]).astype(np.int64)
         total = int(offs[-1]) + n_plan
         self._offs = offs
@@ -110,6 +121,14 @@ class StaticDecodeContext:
         for k in self._plan_keys:
             S = self._plan_splits[k]
             self._plan_off[k] = base
+            if k[4]:
+                n_items, n_count, n_extra = B * S * FEW_INTS, B * k[2], B * 8 if k[3] else 0
+                few, counters = d[base:base + n_items], d[base + n_items:base + n_items + n_count]
+                extras = d[base + n_items + n_count:base + n_items + n_count + n_extra] if n_extra else None
+                self._plans[k] = AttentionPlan(few[:0], 0, None, 0, B * S + (B if n_extra else 0) if S > 1 or n_extra else 0, 0,
+                                               extras, B if n_extra else 0, few, B * S, counters)
+                base += n_items + n_count + n_extra
+                continue
             items = d[base:base + B * S * 8]
             jobs = d[base + B * S * 8:base + B * S * 8 + B * 7]
             if k[3]:        # a slot more a request, filled by another kernel: every request has a merge job
@@ -130,15 +149,19 @@ class StaticDecodeContext:
                            "ctx.slots (on the device), or sets capturable = False to be run eagerly")
 
     def attention_plan(self, group: int, group_size: int, window, n_kv_heads: int,
-                       page_size: int = 64, extra_slot: bool = False) -> AttentionPlan:
-        key = (group_size, window, n_kv_heads, bool(extra_slot))
+                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0) -> AttentionPlan:
+        few = few_rows if page_size >= FEW_PAGE and group_size <= FEW_ROWS else 0
+        key = (group_size, window, n_kv_heads, bool(extra_slot), few)
         if key not in self._plans:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("an attention plan was first asked for during graph capture")
             tiles = self.max_tiles
             if tiles is not None and window:
                 tiles = min(tiles, -(-mask_reach(window) // ATTN_TILE) + 1)
-            self._plan_splits[key] = self.S if tiles is None else min(self.S, splits_for(self.B, tiles, n_kv_heads))
+            if few:
+                self._plan_splits[key] = few_row_splits(self.B, tiles if tiles is not None else self.S * FEW_MIN_RANGE, n_kv_heads)
+            else:
+                self._plan_splits[key] = self.S if tiles is None else min(self.S, splits_for(self.B, tiles, n_kv_heads))
             self._plan_keys.append(key)
             self._alloc()
             self.fill(*self._last)
@@ -206,8 +229,19 @@ class StaticDecodeContext:
             self.token_ids[:n].copy_(token_source)
 
     def _fill_plan(self, h, base: int, key, starts) -> None:
-        group_size, window, _, extra = key
+        group_size, window, n_kv_heads, extra, few = key
         B, S = self.B, self._plan_splits[key]
+        if few:
+            got, extras, _ = few_row_items(np.arange(B), starts, np.ones(B, dtype=np.int64), np.arange(B), window, B * S, extra,
+                                           pair_at=ATTN_STREAM_SLOTS // n_kv_heads if few == 2 else 0)
+            items = h[base:base + B * S * FEW_INTS].reshape(B * S, FEW_INTS)
+            items[:len(got)] = got
+            items[len(got):, 2:4] = 0              # (no keys: nothing to do)
+            after = base + B * S * FEW_INTS
+            h[after:after + B * n_kv_heads] = 0
+            if extra:
+                h[after + B * n_kv_heads:after + B * n_kv_heads + B * 8] = extras.ravel()
+            return
         per_req = S + 1 if extra else S         # partial slots a request
         items = h[base:base + B * S * 8].reshape(B, S, 8)
         jobs = h[base + B * S * 8:base + B * S * 8 + B * 7].reshape(B, 7)
