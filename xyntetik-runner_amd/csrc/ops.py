@@ -92,7 +92,7 @@ _PROTOS = {
     "xr_head_rmsnorm": [_p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _f, _i, _p],
     "xr_moe_table_route": [_p, _p, _p, _p, _i, _i, _i, _i, _f, _p],
     "xr_sample": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p],
-    "xr_sample_split": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p, C.c_longlong, _i, _p],
+    "xr_sample_split": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p, C.c_longlong, _i, _i, _p],
     "xr_layernorm": [_p, _p, _p, _p, _i, _i, _i, _f, _i, _p],
     "xr_layernorm_conv": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _f, _i, _p],
     "xr_causal_conv": [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p],
@@ -1923,18 +1923,20 @@ class Ops:
         # again than they save.
         first = W * 32 * 2 * 4 if V >= 8192 else 0
         splits = max(1, min(8, 512 // max(1, W))) if first and top_k is not None else 0
-        ws = torch.empty((first + W * splits * _SAMPLE_BIN_BYTES,), dtype=torch.uint8, device=logits.device) if first else None
+        room = W * ((splits + 1) * _SAMPLE_BIN_BYTES + _SAMPLE_FOUND_BYTES) if splits else 0
+        ws = torch.empty((first + room,), dtype=torch.uint8, device=logits.device) if first else None
         part = ws.data_ptr() if first else None
         args = (out.data_ptr(), logits.data_ptr(), W, V, logits.stride(0), temp, top_k, top_p, min_p, repeat_penalty, draw, recent, n_recent,
                 recent_cap, _ptr(exempt), exempt.numel() if exempt is not None else 0, part)
         if splits:
-            self.lib.check(self.lib.xr_sample_split(*args, part + first, W * splits * _SAMPLE_BIN_BYTES, splits, _stream()))
+            self.lib.check(self.lib.xr_sample_split(*args, part + first, room, splits, splits, _stream()))
         else:
             self.lib.check(self.lib.xr_sample(*args, _stream()))
         return out
 
 
-_SAMPLE_BIN_BYTES = 2048 * 12       # a share of a row's histogram: mass and number of the candidates of every bin
+_SAMPLE_BIN_BYTES = 2048 * 12       # a share of a row's histogram, or their sum: mass and number of the candidates of every bin
+_SAMPLE_FOUND_BYTES = 2048 * 8 + 96 # candidates of a row's cuts, and what its workgroups tell each other
 _LOCK = threading.Lock()
 _OPS: Optional[Ops] = None
 
