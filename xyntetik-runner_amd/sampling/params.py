@@ -10,8 +10,10 @@ refused, and an absent seed is taken from the clock
 """
 from __future__ import annotations
 
+import struct
 import time
-from dataclasses import dataclass, field
+from array import array
+from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -66,9 +68,26 @@ class SamplerState:
             self.rng = params.seed & _MASK
         else:
             self.rng = (int(time.time()) ^ 0x9E3779B97F4A7C15) & _MASK or 1
-        self.recent: List[int] = [0] * RECENT_WINDOW
+        self.recent = array("i", [0]) * RECENT_WINDOW        # (32-bit words: a batch's windows are copied, not converted)
         self.n_recent = 0
         self.head = 0
+
+    @property
+    def params(self) -> SamplingParams:
+        return self._params
+
+    @params.setter
+    def params(self, p: SamplingParams) -> None:
+        self._params = p
+        # the options as the kernels read them: temperature (0: greedy), top-p, min-p, repeat penalty, top-k
+        floats = 0.0 if p.greedy else p.temperature, p.top_p, p.min_p, p.repeat_penalty
+        top_k = min(p.top_k, 0x7FFFFFFF)
+        try:
+            self.words = struct.pack("=4fi", *floats, top_k)
+        except OverflowError:                   # (beyond 32 bits: infinite)
+            self.words = np.array(floats, dtype=np.float32).tobytes() + struct.pack("=i", top_k)
+        self.greedy = p.greedy
+        self.penalised = not p.greedy and p.repeat_penalty != 1.0
 
     def draw(self) -> float:
         """The next uniform number in [0, 1): the top 24 bits of the next state."""
@@ -84,20 +103,31 @@ class SamplerState:
             self.n_recent += 1
 
 
-def draws(states: Sequence[SamplerState], greedy: Sequence[bool]) -> List[float]:
-    """``draw()`` of every state that samples, 0 for the greedy ones.  The generators of a larger batch step side by side in
-    64-bit words (for 64 rows 15 us instead of 60)."""
-    live = [s for s, g in zip(states, greedy) if not g]
-    if len(live) < 8 or len(set(map(id, live))) < len(live):        # (a state given twice draws twice)
-        return [0.0 if g else s.draw() for s, g in zip(states, greedy)]
-    x = np.array([s.rng for s in live], dtype=np.uint64)
+def _draw_together(states: Sequence[SamplerState]) -> np.ndarray:
+    """``draw()`` of every state, each of them given once: their generators step side by side in 64-bit words."""
+    x = np.array([s.rng for s in states], dtype=np.uint64)
     x ^= x << _SHIFTS[0]
     x ^= x >> _SHIFTS[1]
     x ^= x << _SHIFTS[2]
-    for s, v in zip(live, x.tolist()):
+    for s, v in zip(states, x.tolist()):
         s.rng = v
-    values = ((x >> _SHIFTS[3]) / 16777216.0).tolist()
+    return (x >> _SHIFTS[3]) / 16777216.0
+
+
+def draw_values(states: Sequence[SamplerState], greedy: Sequence[bool]) -> Sequence[float]:
+    """``draws`` as whatever sequence it is made as."""
+    live = states if not any(greedy) else [s for s, g in zip(states, greedy) if not g]
+    if len(live) < 8 or len(set(map(id, live))) < len(live):        # (a state given twice draws twice)
+        return [0.0 if g else s.draw() for s, g in zip(states, greedy)]
+    values = _draw_together(live)
     if len(live) == len(states):
         return values
-    rest = iter(values)
+    rest = iter(values.tolist())
     return [0.0 if g else next(rest) for g in greedy]
+
+
+def draws(states: Sequence[SamplerState], greedy: Sequence[bool]) -> List[float]:
+    """``draw()`` of every state that samples, 0 for the greedy ones.  The generators of a larger batch step side by side (for 64 rows
+    15 us instead of 60)."""
+    values = draw_values(states, greedy)
+    return values if isinstance(values, list) else values.tolist()

@@ -6,12 +6,13 @@ depend on its own seed only, not on what else is in the batch.
 """
 from __future__ import annotations
 
+from array import array
 from typing import List, Optional, Sequence
 
 import numpy as np
 import torch
 
-from .params import RECENT_WINDOW, SamplerState, draws
+from .params import RECENT_WINDOW, SamplerState, draw_values
 
 
 class Sampler:
@@ -35,28 +36,21 @@ class Sampler:
         """The same without waiting for the result: token ids ``[W]`` int32 on the device."""
         W = logits.shape[0]
         assert W == len(states) and W > 0
-        params = [s.params for s in states]
-        temps = [p.temperature for p in params]
-        greedy = [not (t > 0.0) for t in temps]
-        penalties = [p.repeat_penalty for p in params]
-        # floats: temp, top_p, min_p, rp, draw ; ints: top_k, n_recent ; window
-        need_window = any(x != 1.0 and not g for x, g in zip(penalties, greedy))
+        greedy = [s.greedy for s in states]
+        # floats: temp, top_p, min_p, rp, draw ; ints: top_k, n_recent ; window.  (Every state keeps its options as words: a batch of 64 is
+        # one join and one transposed copy, 25 us less than a list and its conversion an option, and 64 windows 6 us instead of 200.)
+        need_window = any([s.penalised for s in states])
         nf = 5 * W
         ni = 2 * W + (W * RECENT_WINDOW if need_window else 0)
         host = torch.empty((nf + ni,), dtype=torch.int32, pin_memory=True)
         h = host.numpy()
-        hf, hi = h[:nf].view(np.float32).reshape(5, W), h[nf:]
-        hf[0] = temps if not any(greedy) else [0.0 if g else t for t, g in zip(temps, greedy)]
-        hf[1] = [p.top_p for p in params]
-        hf[2] = [p.min_p for p in params]
-        hf[3] = penalties
-        hf[4] = draws(states, greedy)
-        hi[:W] = [p.top_k for p in params]
-        hi[W:2 * W] = [s.n_recent for s in states]
+        options = h[:7 * W].reshape(7, W)
+        words = np.frombuffer(b"".join([s.words for s in states]), dtype=np.int32).reshape(W, 5).T
+        options[:4], options[5] = words[:4], words[4]
+        options[4].view(np.float32)[:] = draw_values(states, greedy)
+        options[6] = [s.n_recent for s in states] if need_window else 0
         if need_window:
-            win = hi[2 * W:].reshape(W, RECENT_WINDOW)
-            for r, s in enumerate(states):
-                win[r, :] = s.recent
+            h[7 * W:] = np.frombuffer(b"".join([s.recent if type(s.recent) is array else array("i", s.recent) for s in states]), dtype=np.int32)
         dev = host.to(self.device, non_blocking=True)
         if all(greedy):
             temp, _, _, _, draw = dev[:nf].view(torch.float32).view(5, W).unbind(0)
