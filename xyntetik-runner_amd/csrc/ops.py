@@ -91,6 +91,8 @@ _PROTOS = {
     "xr_token_shift": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_head_rmsnorm": [_p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _f, _i, _p],
     "xr_moe_table_route": [_p, _p, _p, _p, _i, _i, _i, _i, _f, _p],
+    "xr_conv_qkv_store": [_p, _p, _p, _p, _i, _p, _p, _p, _i, _p, _p] + [_i] * 8 + [_p],
+    "xr_recurrence_step": [_p] * 15 + [_i] * 11 + [_f] * 4 + [_i, _i, _p],
     "xr_sample": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p],
     "xr_sample_split": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p, C.c_longlong, _i, _i, _p],
     "xr_layernorm": [_p, _p, _p, _p, _i, _i, _i, _f, _i, _p],
@@ -1586,6 +1588,52 @@ class Ops:
                                                  float(q_scale), float(unit_eps), _stream()))
 
     @staticmethod
+    def recurrence_step_applies(ctx, T: int, D: int, Dv: int) -> bool:
+        """Whether a recurrence's rows of this step can go through ``recurrence_step``: one row a request, heads of 33 to 128 by up to 128."""
+        return ctx.max_q_len == 1 and T == ctx.B and T < 65536 and 32 < D <= 128 and 0 < Dv <= 128
+
+    def recurrence_step(self, kind: str, q, k, v, state: torch.Tensor, ctx, H: int, G: int, D: int, Dv: int, out_gate, w_norm, eps: float,
+                        out_dtype: torch.dtype, gate_activation: str = "silu", decay=None, inv_freq=None, rot: int = 0, beta=None, gate=None,
+                        a_log=None, dt_bias=None, q_scale: float = 1.0, k_scale: float = 1.0, unit_eps: float = 0.0) -> torch.Tensor:
+        """A step of one row a request (``recurrence_step_applies``) from the input product's 32-bit rows to what the output product reads, in
+        one kernel and with the state brought up to date: "retention": ``rotate_rows_`` of q and k (``inv_freq``, ``rot``; then the scales), "delta":
+        ``delta_prepare_`` (``beta`` and ``gate`` as the product made them); ``linear_recurrence``; ``gated_rmsnorm`` per head."""
+        self._dev(q, k, v, state, out_gate, w_norm, decay, inv_freq, beta, gate, a_log, dt_bias)
+        T = q.shape[0]
+        f32 = [t for t in (q, k, v, out_gate, beta, gate) if t is not None]
+        if any(t.dtype != torch.float32 or t.stride(1) != 1 for t in f32) or len({t.stride(0) for t in (q, k, v)}) != 1:
+            raise KernelError("recurrence_step: the rows must be float32 views, q, k and v with one row stride")
+        if (tuple(q.shape) != (T, G * D) or tuple(k.shape) != (T, G * D) or tuple(v.shape) != (T, H * Dv) or tuple(out_gate.shape) != (T, H * Dv)
+                or not self.recurrence_step_applies(ctx, T, D, Dv)):
+            raise KernelError("recurrence_step: view widths do not fit the heads, or not one row a request")
+        rows, lanes = C.c_int(), C.c_int()
+        self.lib.dll.xr_recurrence_state_dims(int(D), C.byref(rows), C.byref(lanes))
+        if lanes.value != 16 or (H, rows.value, Dv, 16) != self.recurrence_state_shape(H, D, Dv):
+            raise KernelError("recurrence_step: the library lays its state out differently from recurrence_state_shape")
+        if state.dtype != torch.float32 or tuple(state.shape[1:]) != self.recurrence_state_shape(H, D, Dv) or not state.is_contiguous():
+            raise KernelError(f"recurrence_step: state must be float32 [slots, {self.recurrence_state_shape(H, D, Dv)}]")
+        if w_norm is not None and (w_norm.dtype != torch.float32 or w_norm.numel() not in (Dv, H * Dv) or not w_norm.is_contiguous()):
+            raise KernelError(f"recurrence_step: the norm's weight must be float32 [{Dv}] or [{H * Dv}]")
+        if gate_activation not in NORM_GATES:
+            raise KernelError(f"recurrence_step: gate activation {gate_activation!r} (known: {sorted(NORM_GATES)})")
+        if kind == "delta":
+            if (beta is None or gate is None or tuple(beta.shape) != (T, H) or tuple(gate.shape) != (T, H) or beta.stride(0) != gate.stride(0)
+                    or any(t is None or t.dtype != torch.float32 or t.numel() != H or not t.is_contiguous() for t in (a_log, dt_bias))):
+                raise KernelError(f"recurrence_step: the delta rule needs beta and gate [T, {H}] with one row stride, A_log and dt_bias [{H}]")
+        elif kind != "retention" or decay is None or decay.dtype != torch.float32 or decay.numel() != H:
+            raise KernelError(f"recurrence_step: retention needs float32 decay [{H}]; {kind!r}")
+        if rot and (inv_freq is None or inv_freq.dtype != torch.float32 or inv_freq.numel() != rot // 2):
+            raise KernelError(f"recurrence_step: {rot // 2} 32-bit frequencies are needed")
+        out = torch.empty((T, H * Dv), dtype=out_dtype, device=q.device)
+        self.lib.check(self.lib.xr_recurrence_step(
+            out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), state.data_ptr(), ctx.slots.data_ptr(), ctx.positions.data_ptr(),
+            _ptr(inv_freq) if rot else None, _ptr(decay), _ptr(beta), _ptr(gate), _ptr(a_log), _ptr(dt_bias), out_gate.data_ptr(), _ptr(w_norm),
+            T, H, G, D, Dv, q.stride(0), beta.stride(0) if beta is not None else 0, out_gate.stride(0), int(rot),
+            1 if (w_norm is not None and H > 1 and w_norm.numel() == H * Dv) else 0, NORM_GATES[gate_activation], float(q_scale), float(k_scale),
+            float(unit_eps), float(eps), 1 if kind == "delta" else 0, dtype_code(out_dtype), _stream()))
+        return out
+
+    @staticmethod
     def recurrence_state_shape(H: int, D: int, Dv: int):
         """The per-request state of ``linear_recurrence``: S[R j + r][c] of head h at ``[h, j, c, r]``,
         R = the lanes that share a column in the kernel (16 for key sizes above 32, else 4; the
@@ -1836,6 +1884,29 @@ class Ops:
                                              ctx.positions.data_ptr(), ctx.req_of_token.data_ptr(), table.data_ptr(),
                                              table.stride(0), T, H, Hk if writes else 0, D, Dv, page_size,
                                              dtype_code(out_dtype), _stream()))
+        return q_out
+
+    def conv_qkv_store(self, u, w, state, k_cache, v_cache, ctx, group: int, H: int, Hk: int, D: int, Dv: int, page_size: int,
+                       out_dtype: torch.dtype) -> torch.Tensor:
+        """``causal_conv`` of the input product's rows ``u [B, H * D + Hk * (D + Dv)]`` without activation, then ``qkv_store`` (``Hk`` 0: this
+        layer stores no keys), in one kernel for a step of one row a request; ``state`` is brought up to date."""
+        self._dev(u, w, state, k_cache, v_cache)
+        T, Cn = u.shape
+        if u.dtype != torch.float32 or u.stride(1) != 1 or Cn != H * D + Hk * (D + Dv) or ctx.max_q_len != 1 or T != ctx.B:
+            raise KernelError("conv_qkv_store: float32 rows of queries, keys and values are needed, one a request")
+        if w.dtype != torch.float32 or w.dim() != 2 or w.shape[0] != Cn or not w.is_contiguous() or w.shape[1] < 2:
+            raise KernelError(f"conv_qkv_store: the convolution's weight must be float32 [{Cn}, taps]")
+        taps = w.shape[1]
+        if state is None or state.dtype != torch.float32 or tuple(state.shape[1:]) != (taps - 1, Cn) or not state.is_contiguous():
+            raise KernelError(f"conv_qkv_store: state must be float32 [slots, {taps - 1}, {Cn}]")
+        if Hk and (k_cache.dtype != out_dtype or tuple(k_cache.shape[1:]) != (Hk, page_size, D) or tuple(v_cache.shape[1:]) != (Hk, Dv, page_size)):
+            raise KernelError("conv_qkv_store: the cache does not fit the heads")
+        table = ctx.block_table(group)
+        q_out = torch.empty((T, H * D), dtype=out_dtype, device=u.device)
+        self.lib.check(self.lib.xr_conv_qkv_store(
+            q_out.data_ptr(), _ptr(k_cache) if Hk else None, _ptr(v_cache) if Hk else None, u.data_ptr(), u.stride(0), w.data_ptr(), state.data_ptr(),
+            ctx.slots.data_ptr(), taps, ctx.positions.data_ptr(), table.data_ptr(), table.stride(0), T, H, Hk, D, Dv, page_size,
+            dtype_code(out_dtype), _stream()))
         return q_out
 
     def pool_blocks(self, pk, pv, k_cache, v_cache, ctx, group: int, pool_group: int, Hk: int, D: int, Dv: int, P: int,

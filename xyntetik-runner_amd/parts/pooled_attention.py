@@ -100,9 +100,13 @@ class PooledWindowAttention(Mixer):
         if writes == self.kv_shared:
             raise ValueError("pooled attention: a layer stores its keys and values exactly when it projects them")
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
-        y = ops.causal_conv(proj, self.w_conv, cache.states.get("mixer.conv"), ctx, torch.float32) if self.conv_taps else proj
-        q = ops.qkv_store(y[:, :Q], y[:, Q:Q + K] if writes else None, y[:, Q + K:] if writes else None,
-                          cache.k, cache.v, ctx, cache.group, H, G, D, Dv, cache.page_size, self.rt.dtype)
+        if self.conv_taps > 1 and ctx.max_q_len == 1 and proj.shape[0] == ctx.B and ctx.B < 65536:
+            q = ops.conv_qkv_store(proj, self.w_conv, cache.states.get("mixer.conv"), cache.k if writes else None, cache.v if writes else None,
+                                   ctx, cache.group, H, G if writes else 0, D, Dv, cache.page_size, self.rt.dtype)
+        else:
+            y = ops.causal_conv(proj, self.w_conv, cache.states.get("mixer.conv"), ctx, torch.float32) if self.conv_taps else proj
+            q = ops.qkv_store(y[:, :Q], y[:, Q:Q + K] if writes else None, y[:, Q + K:] if writes else None,
+                              cache.k, cache.v, ctx, cache.group, H, G, D, Dv, cache.page_size, self.rt.dtype)
         if P and cache.pool_owns:
             ops.pool_blocks(cache.pool_k, cache.pool_v, cache.k, cache.v, ctx, cache.group, cache.pool_group, G, D, Dv, P,
                             cache.page_size)

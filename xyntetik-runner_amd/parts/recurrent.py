@@ -127,6 +127,10 @@ class Retention(Mixer):
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
         q, k, v, gate = proj[:, :QK], proj[:, QK:2 * QK], proj[:, 2 * QK:2 * QK + V], proj[:, 2 * QK + V:]
         rot = self.position.rotary() if self.position is not None else None
+        if self.qkv_activation is None and self.norm_over == "head" and ops.recurrence_step_applies(ctx, h.shape[0], D, Dv):
+            return ops.recurrence_step("retention", q, k, v, cache.state, ctx, H, H, D, Dv, gate, self.w_norm, self.eps, self.rt.dtype,
+                                       self.gate_activation, decay=self.decay, inv_freq=rot.inv_freq if rot is not None else None,
+                                       rot=rot.rotary_dim if rot is not None else 0, k_scale=self.key_scale)
         # a short portion's recurrence applies the activation as it reads (a kernel less in a decode step); a portion in
         # chunks, whose rows are read again for every 16 columns of the state, takes rows that passed it before (32 heads
         # of 128, portions of 200 and 1,023 rows: 41 and 109 us with the activation's own kernel, 49 and 142 without)
@@ -334,6 +338,10 @@ class GatedDelta(Mixer):
             o = ops.linear_recurrence("delta_channel", q, k, v, cache.states["mixer.S"], ctx, H, G, D, Dv, beta=b, gate=w)
         else:
             a = proj[:, at + H:]
+            if ops.recurrence_step_applies(ctx, h.shape[0], D, Dv):
+                return ops.recurrence_step("delta", q, k, v, cache.states["mixer.S"], ctx, H, G, D, Dv, gate, self.w_norm, self.eps, self.rt.dtype,
+                                           self.gate_activation, beta=b, gate=a, a_log=self.a_log, dt_bias=self.dt_bias,
+                                           q_scale=D ** -0.5, unit_eps=self.UNIT_EPS)
             ops.delta_prepare_(q, k, b, a, self.a_log, self.dt_bias, G, H, D, D ** -0.5, self.UNIT_EPS)
             o = ops.linear_recurrence("delta", q, k, v, cache.states["mixer.S"], ctx, H, G, D, Dv, beta=b, gate=a)
         return ops.gated_rmsnorm(o, gate, self.w_norm, H, Dv, self.eps, self.rt.dtype, gate_activation=self.gate_activation)
