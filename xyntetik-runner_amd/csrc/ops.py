@@ -91,6 +91,7 @@ _PROTOS = {
     "xr_token_shift": [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
     "xr_head_rmsnorm": [_p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _f, _i, _p],
     "xr_moe_table_route": [_p, _p, _p, _p, _i, _i, _i, _i, _f, _p],
+    "xr_layernorm_conv_rows": [_p] * 7 + [_i] * 5 + [_f, _i, _p],
     "xr_conv_qkv_store": [_p, _p, _p, _p, _i, _p, _p, _p, _i, _p, _p] + [_i] * 8 + [_p],
     "xr_recurrence_step": [_p] * 15 + [_i] * 11 + [_f] * 4 + [_i, _i, _p],
     "xr_sample": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p],
@@ -1194,6 +1195,28 @@ class Ops:
         self.lib.check(self.lib.xr_layernorm_conv(out.data_ptr(), x.data_ptr(), _ptr(w), conv_w.data_ptr(), _ptr(state),
                                                   ctx.slots.data_ptr(), R, E, x.stride(0), taps, float(eps),
                                                   dtype_code(out_dtype), _stream()))
+        return out
+
+    def layernorm_conv_rows(self, x: torch.Tensor, w: Optional[torch.Tensor], eps: float, conv_w: torch.Tensor,
+                            state: Optional[torch.Tensor], ctx, out_dtype: torch.dtype) -> Optional[torch.Tensor]:
+        """``layernorm_conv`` for steps in which requests bring several rows; None where its kernel does not take the sizes
+        (2 to 4 taps, a width in fours up to 4,096, 16-byte aligned rows)."""
+        self._dev(x, w, conv_w, state)
+        T, E = x.shape
+        taps = conv_w.shape[1] if conv_w.dim() == 2 else 0
+        if (not 2 <= taps <= 4 or E % 4 or E > 4096 or x.dtype != torch.float32 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16
+                or (w is not None and w.data_ptr() % 16) or state is None or state.data_ptr() % 16 or conv_w.data_ptr() % 16):
+            return None
+        if w is not None and (w.dtype != torch.float32 or w.numel() != E or not w.is_contiguous()):
+            raise KernelError(f"layernorm_conv: the norm's weight must be float32 [{E}]")
+        if conv_w.dtype != torch.float32 or conv_w.shape[0] != E or not conv_w.is_contiguous():
+            raise KernelError(f"layernorm_conv: the convolution's weight must be float32 [{E}, taps]")
+        if state.dtype != torch.float32 or tuple(state.shape[1:]) != (taps - 1, E) or not state.is_contiguous():
+            raise KernelError(f"layernorm_conv state must be float32 [slots, {taps - 1}, {E}]")
+        out = torch.empty((T, E), dtype=out_dtype, device=x.device)
+        self.lib.check(self.lib.xr_layernorm_conv_rows(out.data_ptr(), x.data_ptr(), _ptr(w), conv_w.data_ptr(), state.data_ptr(),
+                                                       ctx.cu_q.data_ptr(), ctx.slots.data_ptr(), T, ctx.B, E, x.stride(0), taps, float(eps),
+                                                       dtype_code(out_dtype), _stream()))
         return out
 
     def polynorm(self, z: torch.Tensor, coef: torch.Tensor, eps: float, out_dtype: torch.dtype) -> torch.Tensor:

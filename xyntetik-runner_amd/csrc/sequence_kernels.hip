@@ -23,6 +23,8 @@ template <int NW> __device__ inline float block_sum(float v, float* part) {
     return t;
 }
 #define FEW_ROWS 128
+__device__ inline void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+__device__ inline void st4(bf16_t* p, float4 v) { *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)); }
 
 template <typename TO, int NW>
 __global__ __launch_bounds__(64 * NW) void k_layernorm(TO* __restrict__ out, const float* __restrict__ x,
@@ -154,9 +156,9 @@ extern "C" int xr_layernorm(void* out, const float* x, const float* w, const int
 // ---------------------------------------------------------------- short causal convolution over time
 // y_t[c] = sum_j w[c][j] * u_(t - taps + 1 + j)[c]  (+ bias[c]) (+ u_t[c] with `residual`), then the activation.
 // Inputs before a portion's first row come from the request's state row, which holds its last
-// taps - 1 inputs, oldest first, and is zero for a request that begins.  The state is rewritten by
-// a second kernel once every row has been read; in a step where every request brings one row
-// (`fuse`) a row's own thread is the only one that reads its request's state and rewrites it itself.
+// taps - 1 inputs, oldest first, and is zero for a request that begins.  Who reads a request's state rewrites it: in a
+// step where every request brings one row (`fuse`) a row's own thread, else the threads of the request's first rows
+// (k_causal_conv_rows); a kernel of its own (k_conv_state) only where taps are so many that several workgroups read it.
 #define CONV_MAX_TAPS 16
 #define XR_CONV_NONE 0
 #define XR_CONV_SILU 1
@@ -188,42 +190,61 @@ __global__ __launch_bounds__(256) void k_causal_conv(TO* __restrict__ out, const
     st<TO>(out, (size_t)t * ld_out + c, acc);
 }
 
-// Many rows: a thread takes CONV_ROWS consecutive rows of its channel.  What a row needs before its
-// first input (its request, the request's first row and state row) are three loads that wait for
-// each other; with a row a thread a workgroup spent most of its life on them (2,048 rows of 2,048
-// channels: 26 us), here the rows' chains run side by side.  (Four channels a thread with 16-byte
-// loads was slower still: 34 us.)
+// A step's rows in blocks of R, none of which holds rows of two requests: block `blk` is block k of request b.  At most
+// (T + B (R - 1)) / R blocks; false for those past the last.  (Every lane of a wave takes part; requests without rows have no block.)
+template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu_q, int B, int blk, int& b, int& k) {
+    if (B == 1) {                                       // (no search: the chain of loads and exchanges takes a workgroup over a microsecond)
+        b = 0, k = blk;
+        return blk * R < cu_q[1] - cu_q[0];
+    }
+    const int lane = threadIdx.x & 63;
+    for (int b0 = 0; b0 < B; b0 += 64) {
+        const int n = b0 + lane < B ? cu_q[b0 + lane + 1] - cu_q[b0 + lane] : 0, own = (n + R - 1) / R;
+        int upto = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += t;
+        }
+        const int total = __shfl(upto, 63, 64);
+        if (blk < total) {
+            const int at = __ffsll((unsigned long long)__ballot(upto > blk)) - 1;
+            b = __builtin_amdgcn_readfirstlane(b0 + at);
+            k = __builtin_amdgcn_readfirstlane(blk - __shfl(upto - own, at, 64));
+            return true;
+        }
+        blk -= total;
+    }
+    return false;
+}
+
+// Steps of several rows a request: a thread takes up to CONV_ROWS consecutive rows of its channel, all of one request, so that
+// every input is read once; what a row needs before its first input (its request, the request's first row and state row) are loads
+// that wait for each other, once a block and not once a row.  The first block of a request is the only one that reads its state (up to
+// CONV_ROWS + 1 taps), and writes it anew.  Bound by memory and, for few rows, by that chain.  (Four channels a thread with 16-byte loads was slower:
+// 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 26.7 us, and k_conv_state's 4.7 behind it are saved.
 #define CONV_ROWS 8
 template <typename TU, typename TO>
 __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, const TU* __restrict__ u,
-                                                          const float* __restrict__ w, const float* __restrict__ bias,
-                                                          const TU* __restrict__ state,
-                                                          const int* __restrict__ cu_q, const int* __restrict__ slots,
-                                                          const int* __restrict__ req_of_token, int T, int C, int taps,
-                                                          int ld_u, int ld_out, int residual, int act) {
-    const int t0 = blockIdx.y * CONV_ROWS;
+                                                          const float* __restrict__ w, const float* __restrict__ bias, TU* state,
+                                                          const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int C,
+                                                          int taps, int ld_u, int ld_out, int residual, int act) {
+    int b, k;
+    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
-    int row0[CONV_ROWS], slot[CONV_ROWS];
-#pragma unroll
-    for (int r = 0; r < CONV_ROWS; ++r) {
-        const int b = req_of_token[t0 + r < T ? t0 + r : T - 1];
-        row0[r] = cu_q[b];
-        slot[r] = slots[b];
-    }
+    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
+    TU* const srow = state + (size_t)slots[b] * (taps - 1) * C;
     float wt[CONV_MAX_TAPS];
 #pragma unroll
     for (int j = 0; j < CONV_MAX_TAPS; ++j) wt[j] = j < taps ? w[(size_t)c * taps + j] : 0.f;
     const float bc = bias ? bias[c] : 0.f;
-    if (taps <= 4 && t0 + CONV_ROWS <= T && row0[0] == row0[CONV_ROWS - 1]) {
-        // all rows of one request (the usual case): every input is read once, the rows share them in registers
-        const int i0 = t0 - row0[0];
-        const TU* srow = state + (size_t)slot[0] * (taps - 1) * C;
+    if (taps <= 4 && i0 + CONV_ROWS <= n) {
         float v[CONV_ROWS + 3];
 #pragma unroll
-        for (int k = 0; k < CONV_ROWS + 3; ++k) {
-            const int s = i0 + k - 3;               // (taps below 4 leave the first of them unread)
-            v[k] = k < 4 - taps ? 0.f : s >= 0 ? ld<TU>(u, (size_t)(row0[0] + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
+        for (int m = 0; m < CONV_ROWS + 3; ++m) {
+            const int s = i0 + m - 3;               // (taps below 4 leave the first of them unread)
+            v[m] = m < 4 - taps ? 0.f : s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
         }
 #pragma unroll
         for (int r = 0; r < CONV_ROWS; ++r) {
@@ -235,28 +256,39 @@ __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, 
             acc += bc;
             if (residual) acc += v[r + 3];
             if (act == XR_CONV_SILU) acc = acc / (1.0f + expf(-acc));
-            st<TO>(out, (size_t)(t0 + r) * ld_out + c, acc);
+            st<TO>(out, (size_t)(row0 + i0 + r) * ld_out + c, acc);
         }
-        return;
+    } else {
+#pragma unroll
+        for (int r = 0; r < CONV_ROWS; ++r) {
+            const int i = i0 + r;
+            if (i >= n) break;
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < CONV_MAX_TAPS; ++j) {
+                if (j >= taps) break;
+                const int s = i - (taps - 1) + j;
+                const float val = s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
+                acc = fmaf(wt[j], val, acc);
+            }
+            acc += bc;
+            if (residual) acc += ld<TU>(u, (size_t)(row0 + i) * ld_u + c);
+            if (act == XR_CONV_SILU) acc = acc / (1.0f + expf(-acc));
+            st<TO>(out, (size_t)(row0 + i) * ld_out + c, acc);
+        }
+    }
+    if (k > 0 || taps < 2 || taps - 1 > CONV_ROWS) return;
+    TU keep[CONV_ROWS];
+#pragma unroll
+    for (int m = 0; m < CONV_ROWS; ++m) {
+        if (m >= taps - 1) break;
+        const int s = n - (taps - 1) + m;
+        keep[m] = s >= 0 ? u[(size_t)(row0 + s) * ld_u + c] : srow[(size_t)(m + n) * C + c];
     }
 #pragma unroll
-    for (int r = 0; r < CONV_ROWS; ++r) {
-        const int t = t0 + r;
-        if (t >= T) break;
-        const int i = t - row0[r];
-        const TU* srow = state + (size_t)slot[r] * (taps - 1) * C;
-        float acc = 0.f;
-#pragma unroll
-        for (int j = 0; j < CONV_MAX_TAPS; ++j) {
-            if (j >= taps) break;
-            const int s = i - (taps - 1) + j;
-            const float val = s >= 0 ? ld<TU>(u, (size_t)(row0[r] + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
-            acc = fmaf(wt[j], val, acc);
-        }
-        acc += bc;
-        if (residual) acc += ld<TU>(u, (size_t)t * ld_u + c);
-        if (act == XR_CONV_SILU) acc = acc / (1.0f + expf(-acc));
-        st<TO>(out, (size_t)t * ld_out + c, acc);
+    for (int m = 0; m < CONV_ROWS; ++m) {
+        if (m >= taps - 1) break;
+        srow[(size_t)m * C + c] = keep[m];
     }
 }
 
@@ -296,18 +328,20 @@ extern "C" int xr_causal_conv(void* out, const void* u, const float* w, const fl
     XR_REQUIRE(!one_row_each || T == B, "causal_conv: %d rows of %d requests are not one row each", T, B);
     if (T == 0 || B == 0) return XR_OK;
     const int fuse = one_row_each && taps > 1 ? 1 : 0;
-    dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, B);
-    dim3 rgrid((C + 255) / 256, (T + CONV_ROWS - 1) / CONV_ROWS);
+    const long long blocks = ((long long)T + (long long)B * (CONV_ROWS - 1)) / CONV_ROWS;
+    XR_REQUIRE(one_row_each ? T <= 65535 : blocks <= 65535 && B <= 65535, "causal_conv: %d rows of %d requests", T, B);
+    dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, B), rgrid((C + 255) / 256, (unsigned)blocks);
 #define CC(TU, TO)                                                                                                   \
     do {                                                                                                             \
-        if (T >= 8 * CONV_ROWS && !fuse)                                                                             \
-            k_causal_conv_rows<TU, TO><<<rgrid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (const TU*)state, cu_q,  \
-                                                                  slots, req_of_token, T, C, taps, ld_u, ld_out,     \
-                                                                  residual, act);                                    \
-        else                                                                                                         \
-        k_causal_conv<TU, TO><<<grid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots,           \
-                                                        req_of_token, C, taps, ld_u, ld_out, residual, act, fuse);    \
-        if (taps > 1 && !fuse) k_conv_state<TU><<<sgrid, 256, 0, stream>>>((TU*)state, (const TU*)u, cu_q, slots, C, taps, ld_u); \
+        if (one_row_each) {                                                                                          \
+            k_causal_conv<TU, TO><<<grid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots, \
+                                                            req_of_token, C, taps, ld_u, ld_out, residual, act, fuse); \
+            break;                                                                                                   \
+        }                                                                                                            \
+        k_causal_conv_rows<TU, TO><<<rgrid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots, B, C, taps, \
+                                                              ld_u, ld_out, residual, act);                          \
+        if (taps - 1 > CONV_ROWS)                                                                                    \
+            k_conv_state<TU><<<sgrid, 256, 0, stream>>>((TU*)state, (const TU*)u, cu_q, slots, C, taps, ld_u);       \
     } while (0)
     if (u_dtype == XR_F32 && out_dtype == XR_F32) CC(float, float);
     else if (u_dtype == XR_F32 && out_dtype == XR_BF16) CC(float, bf16_t);
@@ -488,6 +522,149 @@ extern "C" int xr_layernorm_conv(void* out, const float* x, const float* w, cons
     return XR_OK;
 }
 
+// Layer norm and the convolution behind it (2 to 4 taps) for steps of several rows a request: a workgroup takes LNC_ROWS rows of one request and the
+// three before them, a thread 4 channels of all eight, which stay in its registers from the one read through both sums to the convolution: the
+// normed rows never go to memory.  A request's first workgroup alone reads the carried inputs; with no rows before its own it takes the portion's last three
+// in their place, which become the new ones.  Neighbouring workgroups, which share three rows, run on one XCD.  Bound by memory: a row comes 8 / LNC_ROWS
+// times, from L2 all but once, and goes once; and by a workgroup's two sums, one behind the other.  2,048 rows of 4,096 24.1 us, where k_layernorm_rows, k_causal_conv_rows and
+// k_conv_state took 13.2 + 18.2 + 4.7; 700 rows of 2,048 9.4 (5.1 + 6.5 + 3.3).  A wave a row for the sums and every row read again for the convolution: 40.8.
+// (Up to 4,096 channels: with 8 a thread the registers do not suffice.)
+#define LNC_ROWS 5
+#define LNC_HELD (LNC_ROWS + 3)
+
+// The workgroup's sums of eight numbers a thread, the lane % 8-th of them in a lane: halves of the numbers change lanes, so that ten
+// exchanges serve all eight.  (Whoever made its eight means and deviations in every thread would spend more on them than on its rows.)
+template <int NW> __device__ inline float sums_of_8(float (&s)[8], float (*part)[16]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int w = 4, bit = 32; w > 0; w >>= 1, bit >>= 1) {
+        const bool up = lane & bit;
+#pragma unroll
+        for (int i = 0; i < w; ++i) {
+            const float keep = up ? s[i + w] : s[i], send = up ? s[i] : s[i + w];
+            s[i] = keep + __shfl_xor(send, bit, 64);
+        }
+    }
+    float t = s[0];
+    t += __shfl_xor(t, 4, 64);
+    t += __shfl_xor(t, 2, 64);
+    t += __shfl_xor(t, 1, 64);
+    __syncthreads();
+    if ((lane & 7) == 0) part[lane >> 3][wave] = t;
+    __syncthreads();
+    float u = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w += 4) {
+        const float4 p = *reinterpret_cast<const float4*>(&part[lane & 7][w]);
+        u += (p.x + p.y) + (p.z + p.w);
+    }
+    return u;
+}
+__device__ inline float of_lane(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+__device__ inline float4 pick(bool first, float4 a, float4 b) {
+    return make_float4(first ? a.x : b.x, first ? a.y : b.y, first ? a.z : b.z, first ? a.w : b.w);
+}
+
+template <typename TO, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restrict__ out, const float* __restrict__ x,
+                                                                 const float* __restrict__ w, const float* __restrict__ cw,
+                                                                 float* state, const int* __restrict__ cu_q,
+                                                                 const int* __restrict__ slots, int B, int E, int ldx, int taps, float eps) {
+#pragma clang fp contract(off)      // (a normed row is rounded before it is added, as where the norm's kernel stores it)
+    __shared__ __align__(16) float part[8][16];
+    int b, k;
+    const int share = (int)gridDim.x >> 3;              // (the grid is a multiple of 8: an XCD takes an eighth of the blocks, in order)
+    if (!rows_of_block<LNC_ROWS>(cu_q, B, ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3), b, k)) return;
+    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * LNC_ROWS;
+    const int c = threadIdx.x * 4;
+    float4 h[LNC_HELD];                                 // the rows; then without their mean, normed, as the convolution reads them
+#pragma unroll
+    for (int m = 0; m < LNC_HELD; ++m) {
+        const int i = k == 0 && m < 3 ? n - 3 + m : i0 - 3 + m;
+        h[m] = c < E && i >= 0 && i < n ? *reinterpret_cast<const float4*>(x + (size_t)(row0 + i) * ldx + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    const int cs = c < E ? c : 0;                       // (weights are on their way, too, before the first sum)
+    const float4 gw = w ? *reinterpret_cast<const float4*>(w + cs) : make_float4(1.f, 1.f, 1.f, 1.f);
+    float wt[4][4];                                 // channel, tap (the last is the row itself)
+    if (taps == 4) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const float4 t = *reinterpret_cast<const float4*>(cw + (size_t)(cs + d) * 4);
+            wt[d][0] = t.x; wt[d][1] = t.y; wt[d][2] = t.z; wt[d][3] = t.w;
+        }
+    } else {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) wt[d][j] = j + taps >= 4 ? cw[(size_t)(cs + d) * taps + j + taps - 4] : 0.f;
+    }
+    float s[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) s[m] = (h[m].x + h[m].y) + (h[m].z + h[m].w);
+    const float mean = sums_of_8<NW>(s, part) / (float)E;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        const float mu = of_lane(mean, m);
+        float4& d = h[m];
+        d.x -= mu; d.y -= mu; d.z -= mu; d.w -= mu;
+        s[m] = c < E ? fmaf(d.x, d.x, d.y * d.y) + fmaf(d.z, d.z, d.w * d.w) : 0.f;
+    }
+    const float rinv = 1.0f / sqrtf(sums_of_8<NW>(s, part) / (float)E + eps);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) s[m] = of_lane(rinv, m);        // (here, where all lanes are: below, rinv would be made in those that go on)
+    float* const srow = state + (size_t)slots[b] * (taps - 1) * E;
+    if (c >= E) return;
+#pragma unroll
+    for (int m = 0; m < LNC_HELD; ++m) h[m] = make_float4(h[m].x * s[m] * gw.x, h[m].y * s[m] * gw.y, h[m].z * s[m] * gw.z, h[m].w * s[m] * gw.w);
+    if (k == 0) {
+        // (rows -3 to -1 are carried inputs taps - 4 to taps - 2, if there are so many; new input m of 3 is row n - 3 + m, or an old one)
+        float4 old[3], last[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            old[m] = m + taps >= 4 ? *reinterpret_cast<const float4*>(srow + (size_t)(m + taps - 4) * E + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) last[m] = pick(n >= 3 - m, h[m], pick(m + n == 1, old[1], old[2]));      // (n < 3 - m, n >= 1: m + n is 1 or 2)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) h[m] = old[m];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            if (m + taps >= 4) *reinterpret_cast<float4*>(srow + (size_t)(m + taps - 4) * E + c) = last[m];
+    }
+#pragma unroll
+    for (int r = 0; r < LNC_ROWS; ++r) {
+        float y[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            auto at = [&](int m) { return d == 0 ? h[m].x : d == 1 ? h[m].y : d == 2 ? h[m].z : h[m].w; };
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j + taps >= 4) acc = fmaf(wt[d][j], at(r + j), acc);
+            y[d] = acc + at(r + 3);
+        }
+        if (i0 + r < n) st4(out + (size_t)(row0 + i0 + r) * E + c, make_float4(y[0], y[1], y[2], y[3]));
+    }
+}
+
+// Row b's request brings rows cu_q[b] .. cu_q[b + 1] - 1 of the T; its carried inputs are row slots[b] of state [., taps - 1, E].
+extern "C" int xr_layernorm_conv_rows(void* out, const float* x, const float* w, const float* cw, float* state, const int* cu_q, const int* slots,
+                                      int T, int B, int E, int ldx, int taps, float eps, int out_dtype, hipStream_t stream) {
+    XR_REQUIRE(T >= 0 && B >= 0 && E > 0 && E % 4 == 0 && E <= 4096 && ldx >= E && ldx % 4 == 0, "layernorm_conv: bad sizes T=%d B=%d E=%d ldx=%d", T, B, E, ldx);
+    XR_REQUIRE(taps >= 2 && taps <= 4 && x && cw && state && cu_q && slots && out, "layernorm_conv: %d taps (2 to 4), or an operand is missing", taps);
+    XR_REQUIRE((((uintptr_t)out | (uintptr_t)x | (uintptr_t)w | (uintptr_t)state | (uintptr_t)cw) & 15) == 0, "layernorm_conv: operands must be 16-byte aligned");
+    XR_REQUIRE(out_dtype == XR_F32 || out_dtype == XR_BF16, "layernorm_conv: bad dtype %d", out_dtype);
+    if (T == 0 || B == 0) return XR_OK;
+    const unsigned blocks = (unsigned)(((long long)T + (long long)B * (LNC_ROWS - 1)) / LNC_ROWS + 7) / 8 * 8;
+#define LNC(TO, NW) k_layernorm_conv_rows<TO, NW><<<blocks, 64 * NW, 0, stream>>>((TO*)out, x, w, cw, state, cu_q, slots, B, E, ldx, taps, eps)
+#define LNCS(TO) do { if (E <= 2048) LNC(TO, 8); else LNC(TO, 16); } while (0)
+    if (out_dtype == XR_F32) LNCS(float);
+    else LNCS(bf16_t);
+#undef LNCS
+#undef LNC
+    XR_CHECK_LAUNCH("layernorm_conv_rows");
+    return XR_OK;
+}
+
 // ---------------------------------------------------------------- PolyNorm
 // y = a N(z) + b N(z^2) + c N(z^3) + e, powers element by element, N(v) = v / sqrt(mean(v^2) + eps)
 // over the row.  One workgroup a row: the three sums in one pass, the result in a second.
@@ -523,8 +700,6 @@ __device__ inline float4 ld4(const bf16_t* p) {
     const uint2 u = *reinterpret_cast<const uint2*>(p);
     return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
 }
-__device__ inline void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
-__device__ inline void st4(bf16_t* p, float4 v) { *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)); }
 
 template <typename TZ, typename TO, int NW, int N4>
 __global__ __launch_bounds__(64 * NW) void k_polynorm_v4(TO* __restrict__ out, const TZ* __restrict__ z, const float* __restrict__ coef,
