@@ -19,10 +19,11 @@
 // columns of the state (columns never meet), the state in LDS: three to five small products a chunk.  Rows past a portion's
 // end are zeros with beta 0 and no decay.  L is formed and subtracted in 64 bits; a decay of nothing counts as exp(-100).  A portion
 // that comes to something not finite, or has a negative decay, runs again token by token, a workgroup its 16 columns.
-// Bound by the chain of chunks, a chunk (5.7 us of the delta rule, 4.1 of retention) by five barriers, the trips to LDS between
-// them and, a third of it, its products.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 182 us and k_chunk_mats 74 for the
-// delta rule, 130 and 34 for retention (k_chunk_mats 57 and 24 with q . k in 32 bits); token by token (k_recurrence) 634, and
-// retention in two passes over chunks of 256 side by side 520.
+// Bound by the chain of chunks, a chunk 4.5 us of the delta rule, 3.0 of retention: 1.7 and 1.1 of them the products of a SIMD's two waves, the rest the
+// trips to LDS between them and how fast a compute unit gets 100 KB a chunk from L2.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 143 us and k_chunk_mats 79 for the
+// delta rule, 95 and 39 for retention (k_chunk_mats 57 and 24 with q . k in 32 bits); with four waves that staged every operand in LDS, at
+// barriers that waited for the next chunk's loads too, and a branch a number for the activation 189 and 138; 700 tokens, 16 heads 47 and 34 (67 and 51);
+// token by token (k_recurrence) 634, and retention in two passes over chunks of 256 side by side 520.
 #include "common.h"
 
 typedef float rc_f32x4 __attribute__((ext_vector_type(4)));
@@ -46,13 +47,14 @@ struct ChunkArgs {
     const int* cu_q;
     const int* slots;
     const int* reqs;            // the portions that run so: (request, place of its first chunk) of each
-    int H, G, Dv, ld, ld_g, ld_b, act;
+    int H, G, Dv, ld, ld_g, ld_b;
     float q_scale, k_scale;
 };
 
-__device__ inline float rc_act(float x, int act, float scale) { return (act ? x / (1.0f + expf(-x)) : x) * scale; }
-__device__ inline float4 rc_act4(float4 x, int act, float scale) {
-    return make_float4(rc_act(x.x, act, scale), rc_act(x.y, act, scale), rc_act(x.z, act, scale), rc_act(x.w, act, scale));
+// (ACT: SiLU first.  Decided at run time, it was a branch for every number: a third of the chunks' time.)
+template <bool ACT> __device__ inline float rc_act(float x, float scale) { return (ACT ? x / (1.0f + expf(-x)) : x) * scale; }
+template <bool ACT> __device__ inline float4 rc_act4(float4 x, float scale) {
+    return make_float4(rc_act<ACT>(x.x, scale), rc_act<ACT>(x.y, scale), rc_act<ACT>(x.z, scale), rc_act<ACT>(x.w, scale));
 }
 __device__ inline float4 rc_ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ inline void rc_st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
@@ -72,19 +74,27 @@ __device__ inline rc_f64x4 rc_mfma4(float4 a, float4 b, rc_f64x4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.w, (double)b.w, c, 0, 0, 0);
 }
 
-// 16 rows (a lane's at `rows`) times 16 columns of the state: four chains of products side by side, every operand read before them
+// 16 rows (a lane's pieces of its row in registers) times 16 columns of the state: four chains of products side by side
 template <int J>
-__device__ inline rc_f32x4 times_state(const float* rows, const float* state) {
-    float4 x[J], y[J];
+__device__ inline rc_f32x4 times_state(const float4 (&x)[J], const float* state) {
+    float4 y[J];
 #pragma unroll
-    for (int j = 0; j < J; ++j) { x[j] = rc_ld4(rows + 16 * j); y[j] = rc_ld4(state + j * RC_C * 20); }
+    for (int j = 0; j < J; ++j) y[j] = rc_ld4(state + j * RC_C * 20);
+    __builtin_amdgcn_sched_barrier(0);                  // (every operand is read before them, not two at a time)
     rc_f32x4 s[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int j = 0; j < J; ++j) s[j & 3] = rc_mfma4(x[j], y[j], s[j & 3]);
     return (s[0] + s[1]) + (s[2] + s[3]);
 }
+// a barrier for what lies in LDS: loads on their way to registers stay there
+__device__ inline void rc_meet() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ inline float4 rc_mul4(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
 
-template <int D, bool DELTA>
+template <int D, bool DELTA, bool ACT>
 __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
     constexpr int LD = D + 4;
     extern __shared__ __align__(16) float lds[];
@@ -108,8 +118,8 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
         float4 fq = make_float4(0.f, 0.f, 0.f, 0.f), fk = fq;
         if (r < rows) {
             const size_t at = (size_t)(row0 + r) * a.ld + (size_t)kvh * D + c;
-            fq = rc_act4(rc_ld4(a.q + at), a.act, a.q_scale);
-            fk = rc_act4(rc_ld4(a.k + at), a.act, a.k_scale);
+            fq = rc_act4<ACT>(rc_ld4(a.q + at), a.q_scale);
+            fk = rc_act4<ACT>(rc_ld4(a.k + at), a.k_scale);
         }
         rc_st4(Q + r * LD + c, fq);
         rc_st4(K + r * LD + c, fk);
@@ -201,18 +211,15 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
     }
 }
 
-template <int D, bool DELTA>
-__global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
-    constexpr int LD = D + 4, J = D / 16, NQ = RC_L * D / 1024, NM = RC_L * RC_L / 1024, MATS = DELTA ? 2 : 1;
-    extern __shared__ __align__(16) float lds[];
-    float* Q = lds;                                     // [64][LD]
-    float* K = Q + RC_L * LD;
-    float* P = K + RC_L * LD;                           // [64][RC_LDM]
-    float* T = P + RC_L * RC_LDM;                       // (delta) [64][RC_LDM]
-    __shared__ __align__(16) float S[J][RC_C][20];      // the state's columns, 16 rows side by side
-    __shared__ __align__(16) float U[RC_C][RC_LDM], W[RC_C][RC_LDM];     // by column: u_i; (delta) the right side; u_i exp(L_63 - L_i)
-    __shared__ float V[RC_L][RC_C + 1];
-    __shared__ float vec[RC_VEC];
+// Waves 0 to 3 carry the state on, waves 4 to 7 read it out: wave w and wave 7 - w have the same 16 rows of a chunk, so that a SIMD's two
+// waves, w and w + 4, have as many blocks of T and P together as any other's.  Whatever is used by one wave alone (rows of Q and K, the
+// triangles P and T, K once more by columns) goes from memory to its registers as the instructions want it, asked for as soon as
+// the chunk before has used its own; through LDS go the state, the right side and U.
+template <int D, bool DELTA, bool ACT>
+__global__ __launch_bounds__(512) void k_chunk_run(ChunkArgs a) {
+    constexpr int LD = D + 4, J = D / 16, JP = (J + 3) / 4, MATS = DELTA ? 2 : 1, BUFS = DELTA ? 1 : 2;
+    __shared__ __align__(16) float S[BUFS][J][RC_C][20];    // the state's columns, 16 rows side by side (retention: this chunk's and the next one's)
+    __shared__ __align__(16) float R[DELTA ? RC_C : 1][RC_LDM], U[DELTA ? RC_C : 1][RC_LDM], W[DELTA ? RC_C : 1][RC_LDM];   // by column: right side, u_i, u_i exp(L_63 - L_i)
     __shared__ int odd;                                 // something came out that is not finite
     // Workgroup i runs on XCD i % 8: the column workgroups of a head, which read the same rows and matrices, go to one XCD
     // (where the heads come in eights), so that its L2 serves all but the first of them.
@@ -221,149 +228,248 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
     const int h = eights ? (id >> 3) / shares * 8 + (id & 7) : id / shares, c0 = (eights ? (id >> 3) % shares : id % shares) * RC_C;
     const int row_b = a.cu_q[b], n = a.cu_q[b + 1] - row_b;
     if (n <= 0) return;
-    const int kvh = h / (a.H / a.G);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
-    const int place0 = a.reqs[2 * blockIdx.y + 1];
+    const int kvh = h / (a.H / a.G), chunks = (n + RC_L - 1) / RC_L;
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w16 = wave < 4 ? wave : 7 - wave;
+    const int i0 = 16 * w16 + 4 * quad;                 // this lane's rows of a product whose rows are the chunk's
+    const size_t place0 = (size_t)a.reqs[2 * blockIdx.y + 1] * a.H + h;
     float* st = a.state + (((size_t)a.slots[b] * a.H + h) * J * a.Dv + c0) * 16;
-    for (int i = tid; i < J * RC_C * 4; i += 256) {
+    for (int i = tid; i < J * RC_C * 4; i += 512) {
         const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
-        rc_st4(&S[j][c][r], rc_ld4(st + ((size_t)j * a.Dv + c) * 16 + r));
+        rc_st4(&S[0][j][c][r], rc_ld4(st + ((size_t)j * a.Dv + c) * 16 + r));
     }
-    // a chunk's operands come into registers while the chunk before it is worked on
-    float4 rq[NQ], rk[NQ], rm[MATS * NM], rv;
-    float rvec = 0.f;
-    auto fetch = [&](int chunk) {
-        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
-        const size_t place = (size_t)(place0 + chunk) * a.H + h;
-#pragma unroll
-        for (int e = 0; e < NQ; ++e) {
-            const int i = tid + e * 256, r = i / (D / 4), c = i % (D / 4) * 4;
-            const size_t at = (size_t)(row0 + (r < rows ? r : 0)) * a.ld + (size_t)kvh * D + c;
-            rq[e] = rc_ld4(a.q + at);
-            rk[e] = rc_ld4(a.k + at);
-            if (r >= rows) rq[e] = rk[e] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        const float* mats = a.mats + place * MATS * RC_L * RC_L;
-#pragma unroll
-        for (int e = 0; e < MATS * NM; ++e) {
-            const int i = tid + e * 256, r = i / (RC_L / 4) % RC_L, c = i % (RC_L / 4) * 4;
-            rm[e] = c / 16 <= r / 16 ? rc_ld4(mats + (size_t)i * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        const int r = tid / 4, c = tid % 4 * 4;
-        rv = rc_ld4(a.v + (size_t)(row0 + (r < rows ? r : 0)) * a.ld + (size_t)h * a.Dv + c0 + c);
-        if (r >= rows) rv = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (tid < RC_VEC) rvec = a.vecs[place * RC_VEC + tid];
-    };
-    auto stage = [&]() {                                // the fetched chunk to LDS
-#pragma unroll
-        for (int e = 0; e < NQ; ++e) {
-            const int i = tid + e * 256, r = i / (D / 4), c = i % (D / 4) * 4;
-            rc_st4(Q + r * LD + c, rc_act4(rq[e], a.act, a.q_scale));
-            rc_st4(K + r * LD + c, rc_act4(rk[e], a.act, a.k_scale));
-        }
-#pragma unroll
-        for (int e = 0; e < MATS * NM; ++e) {
-            const int i = tid + e * 256, r = i / (RC_L / 4), c = i % (RC_L / 4) * 4;
-            rc_st4(P + r * RC_LDM + c, rm[e]);          // (T lies behind P)
-        }
-        {
-            const int r = tid / 4, c = tid % 4 * 4;
-            const float4 x = rc_act4(rv, a.act, 1.f);
-            V[r][c] = x.x; V[r][c + 1] = x.y; V[r][c + 2] = x.z; V[r][c + 3] = x.w;
-        }
-        if (tid < RC_VEC) vec[tid] = rvec;
-    };
     if (tid == 0) odd = 0;
-    float none = 0.f;                                   // 0, or no number once a read-out was not finite
-    fetch(0);
-    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
-        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
-        __syncthreads();                                // the chunk before has been read, the state is written
-        stage();
-        __syncthreads();
-        if ((chunk + 1) * RC_L < n) fetch(chunk + 1);
-        const int i0 = 16 * wave + 4 * quad;            // this lane's rows of a product whose rows are the chunk's
-        rc_f32x4 u;
-        if (DELTA) {
-            const rc_f32x4 x = times_state<J>(K + (16 * wave + l16) * LD + 4 * quad, &S[0][l16][4 * quad]);       // K S0
-            float r[4];
+    __syncthreads();
+
+    // Where a chunk's operands lie: a base that all lanes share, which moves from chunk to chunk in scalar registers, and a lane's bytes from there.  A
+    // row past the portion's end is read from its last row, and dropped where it is used.
+    const uint32_t ldb = (uint32_t)a.ld * 4u;
+    auto rows_at = [&](const float* x, int chunk) { return reinterpret_cast<const char*>(x + (size_t)(row_b + chunk * RC_L) * a.ld); };
+    auto vec_at = [&](int chunk) { return a.vecs + (place0 + (size_t)chunk * a.H) * RC_VEC; };
+    auto mats_at = [&](int chunk) { return a.mats + (place0 + (size_t)chunk * a.H) * MATS * RC_L * RC_L; };
+    auto row_pieces = [&](float4 (&x)[J], const float* base, int chunk) {
+        const char* p = rows_at(base, chunk);
+        const uint32_t off = (uint32_t)min(16 * w16 + l16, n - 1 - chunk * RC_L) * ldb + (uint32_t)(kvh * D + 4 * quad) * 4u;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] = vec[2 * RC_L + i0 + e] * (V[i0 + e][l16] - vec[i0 + e] * x[e]);
-            rc_st4(&W[l16][i0], make_float4(r[0], r[1], r[2], r[3]));
-            __syncthreads();
-            u = rc_f32x4{0.f, 0.f, 0.f, 0.f};
-            for (int m = 0; m <= wave; ++m) u = rc_mfma4(rc_ld4(T + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&W[l16][16 * m + 4 * quad]), u);
-            __syncthreads();                            // W is read, and written again below
+        for (int j = 0; j < J; ++j) x[j] = *reinterpret_cast<const float4*>(p + off + 64 * j);
+    };
+    const uint32_t tri_off = (uint32_t)((16 * w16 + l16) * RC_L + 4 * quad);
+    auto triangle = [&](float4 (&x)[4], const float* mat) {      // (all four blocks, used or not: how many loads are on their way has to be known)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = rc_ld4(mat + tri_off + 16 * m);
+    };
+    // rows 16 m + 4 quad .. of a column (i: 4 m and which of the four rows)
+    auto columns = [&](auto& x, const float* base, int chunk, uint32_t col, auto put) {
+        const char* p = rows_at(base, chunk);
+        const uint32_t off = (uint32_t)(4 * quad) * ldb + col;
+        if (n - chunk * RC_L >= RC_L) {
+#pragma unroll
+            for (int i = 0; i < RC_L / 4; ++i) put(x, i, p + (size_t)((uint32_t)(i / 4 * 16 + i % 4) * ldb), off);
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) u[e] = V[i0 + e][l16];
+            for (int i = 0; i < RC_L / 4; ++i) put(x, i, p, (uint32_t)min(i / 4 * 16 + 4 * quad + i % 4, n - 1 - chunk * RC_L) * ldb + col);
         }
-        rc_st4(&U[l16][i0], make_float4(u[0], u[1], u[2], u[3]));
-        rc_st4(&W[l16][i0], make_float4(u[0] * vec[RC_L + i0], u[1] * vec[RC_L + i0 + 1], u[2] * vec[RC_L + i0 + 2], u[3] * vec[RC_L + i0 + 3]));
-        rc_f32x4 o = times_state<J>(Q + (16 * wave + l16) * LD + 4 * quad, &S[0][l16][4 * quad]);         // Q S0
+    };
+    auto put_one = [](float4& x, int e, const char* p, uint32_t off) { (e == 0 ? x.x : e == 1 ? x.y : e == 2 ? x.z : x.w) = *reinterpret_cast<const float*>(p + off); };
+    auto v_columns = [&](float4 (&x)[4], int chunk) {
+        columns(x, a.v, chunk, (uint32_t)(h * a.Dv + c0 + l16) * 4u, [&](float4 (&y)[4], int i, const char* p, uint32_t off) { put_one(y[i / 4], i % 4, p, off); });
+    };
+    // what is used of it: the activation's, times the scale, and nothing past the end
+    auto used_row = [&](float4 (&x)[J], float scale, int chunk) {
+        if (ACT || scale != 1.f) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] *= vec[i0 + e];
-        __syncthreads();                                // U and W are there, and the state of the chunk's start is read
-        rc_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int j = 0; j < J; ++j) x[j] = rc_act4<ACT>(x[j], scale);
+        }
+        if (n - chunk * RC_L < RC_L) {
+            const bool in = 16 * w16 + l16 < n - chunk * RC_L;
 #pragma unroll
-        for (int m = 0; m < RC_L / 16; ++m)
-            if (m <= wave) p[m & 1] = rc_mfma4(rc_ld4(P + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&U[l16][16 * m + 4 * quad]), p[m & 1]);
-        o += p[0] + p[1];
+            for (int j = 0; j < J; ++j) x[j] = make_float4(in ? x[j].x : 0.f, in ? x[j].y : 0.f, in ? x[j].z : 0.f, in ? x[j].w : 0.f);
+        }
+    };
+    auto used_columns = [&](float4 (&x)[4], float scale, int chunk) {      // rows 16 m + 4 quad ..
+        if (ACT || scale != 1.f) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (i0 + e < rows) a.out[((size_t)(row0 + i0 + e) * a.H + h) * a.Dv + c0 + l16] = o[e];
-        none += 0.f * o[0] + 0.f * o[1] + 0.f * o[2] + 0.f * o[3];
-        const float all = vec[RC_L - 1];                // exp(L_63)
-        for (int j = wave; j < J; j += 4) {             // 16 rows of the state: its own decayed, and K^T W
-            const float4 s0 = rc_ld4(&S[j][l16][4 * quad]);
-            rc_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int m = 0; m < 4; ++m) x[m] = rc_act4<ACT>(x[m], scale);
+        }
+        if (n - chunk * RC_L < RC_L) {
 #pragma unroll
-            for (int m = 0; m < RC_L / 16; ++m) {
-                const float* kp = K + (16 * m + 4 * quad) * LD + 16 * j + l16;
-                s[m & 1] = rc_mfma4(make_float4(kp[0], kp[LD], kp[2 * LD], kp[3 * LD]), rc_ld4(&W[l16][16 * m + 4 * quad]), s[m & 1]);
+            for (int m = 0; m < 4; ++m) {
+                const int rows = n - chunk * RC_L - 16 * m - 4 * quad;
+                x[m] = make_float4(rows > 0 ? x[m].x : 0.f, rows > 1 ? x[m].y : 0.f, rows > 2 ? x[m].z : 0.f, rows > 3 ? x[m].w : 0.f);
             }
-            const rc_f32x4 t = s[0] + s[1];
-            rc_st4(&S[j][l16][4 * quad], make_float4(fmaf(s0.x, all, t[0]), fmaf(s0.y, all, t[1]), fmaf(s0.z, all, t[2]), fmaf(s0.w, all, t[3])));
         }
-    }
-    __syncthreads();
-    for (int i = tid; i < J * RC_C * 4; i += 256) {
-        const float4 x = rc_ld4(&S[i / (RC_C * 4)][i / 4 % RC_C][i % 4 * 4]);
-        none += 0.f * x.x + 0.f * x.y + 0.f * x.z + 0.f * x.w;
+    };
+
+    float none = 0.f;                                   // 0, or no number once a read-out or the state was not finite
+    auto has = [&](int t) { return J % 4 == 0 || wave + 4 * t < J; };
+    float4 own[JP];                                     // waves 0 to 3: rows 16 j + 4 quad .. of column l16 of the state, j = wave, wave + 4
+    if (wave < 4) {
+        float4 kr[J], kc[JP][4], tri[4], v[4], grow[4], beta, fall;
+        float all = 0.f;
+        auto load_columns = [&](int chunk) {
+            columns(kc, a.k, chunk, (uint32_t)(kvh * D + 16 * wave + l16) * 4u, [&](float4 (&y)[JP][4], int i, const char* p, uint32_t off) {
+#pragma unroll
+                for (int t = 0; t < JP; ++t)
+                    if (has(t)) put_one(y[t][i / 4], i % 4, p, off + 256 * t);
+            });
+        };
+        // (delta: this lane's rows of V, beta, exp(L) and exp(L_63 - L); retention: V and exp(L_63 - L) of all rows, as an operand of its product)
+        auto load_rest = [&](int chunk) {
+            const float* vec = vec_at(chunk);
+            all = vec[RC_L - 1];
+            if (DELTA) {
+                const char* p = rows_at(a.v, chunk);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) put_one(v[0], e, p, (uint32_t)min(i0 + e, n - 1 - chunk * RC_L) * ldb + (uint32_t)(h * a.Dv + c0 + l16) * 4u);
+                grow[0] = rc_ld4(vec + RC_L + i0);
+                fall = rc_ld4(vec + i0);
+                beta = rc_ld4(vec + 2 * RC_L + i0);
+            } else {
+                v_columns(v, chunk);
+#pragma unroll
+                for (int m = 0; m < 4; ++m) grow[m] = rc_ld4(vec + RC_L + 16 * m + 4 * quad);
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < JP; ++t)
+            if (has(t)) own[t] = rc_ld4(st + ((size_t)(wave + 4 * t) * a.Dv + l16) * 16 + 4 * quad);
+        if (DELTA) {
+            row_pieces(kr, a.k, 0);
+            triangle(tri, mats_at(0) + RC_L * RC_L);
+        }
+        load_rest(0);
+        load_columns(0);
+        for (int chunk = 0; chunk < chunks; ++chunk) {
+            const int next = chunk + 1 < chunks ? chunk + 1 : chunk;
+            const float all_now = all;
+            float4 w[4];
+            if (DELTA) {
+                used_row(kr, a.k_scale, chunk);
+                const rc_f32x4 x = times_state<J>(kr, &S[0][0][l16][4 * quad]);          // K S0
+                row_pieces(kr, a.k, next);
+                const float4 vv = rc_act4<ACT>(v[0], 1.f);     // (past the end beta is 0)
+                rc_st4(&R[l16][i0], make_float4(beta.x * (vv.x - fall.x * x[0]), beta.y * (vv.y - fall.y * x[1]),
+                                                beta.z * (vv.z - fall.z * x[2]), beta.w * (vv.w - fall.w * x[3])));
+                rc_meet();
+                rc_f32x4 u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    if (m <= w16) u = rc_mfma4(tri[m], rc_ld4(&R[l16][16 * m + 4 * quad]), u);
+                triangle(tri, mats_at(next) + RC_L * RC_L);
+                const float4 uu = make_float4(u[0], u[1], u[2], u[3]);
+                rc_st4(&U[l16][i0], uu);
+                rc_st4(&W[l16][i0], rc_mul4(uu, grow[0]));
+                load_rest(next);
+                rc_meet();                              // U and W are there, and the state of the chunk's start is read
+#pragma unroll
+                for (int m = 0; m < 4; ++m) w[m] = rc_ld4(&W[l16][16 * m + 4 * quad]);
+            } else {
+                used_columns(v, 1.f, chunk);
+#pragma unroll
+                for (int m = 0; m < 4; ++m) w[m] = rc_mul4(v[m], grow[m]);
+                load_rest(next);
+            }
+#pragma unroll
+            for (int t = 0; t < JP; ++t) {              // 16 rows of the state: its own decayed, and K^T W
+                if (!has(t)) break;
+                rc_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                used_columns(kc[t], a.k_scale, chunk);
+#pragma unroll
+                for (int m = 0; m < 4; ++m) s[m & 1] = rc_mfma4(kc[t][m], w[m], s[m & 1]);
+                const rc_f32x4 x = s[0] + s[1];
+                own[t] = make_float4(fmaf(own[t].x, all_now, x[0]), fmaf(own[t].y, all_now, x[1]), fmaf(own[t].z, all_now, x[2]), fmaf(own[t].w, all_now, x[3]));
+                rc_st4(&S[DELTA ? 0 : (chunk + 1) & 1][wave + 4 * t][l16][4 * quad], own[t]);
+            }
+            load_columns(next);
+            rc_meet();                                  // the state is written, and U read
+        }
+#pragma unroll
+        for (int t = 0; t < JP; ++t)
+            if (has(t)) none += 0.f * own[t].x + 0.f * own[t].y + 0.f * own[t].z + 0.f * own[t].w;
+    } else {
+        float4 q[J], tri[4], v[4], fall;
+        row_pieces(q, a.q, 0);
+        fall = rc_ld4(vec_at(0) + i0);
+        triangle(tri, mats_at(0));
+        if (!DELTA) v_columns(v, 0);
+        for (int chunk = 0; chunk < chunks; ++chunk) {
+            const int next = chunk + 1 < chunks ? chunk + 1 : chunk, row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
+            used_row(q, a.q_scale, chunk);
+            rc_f32x4 o = times_state<J>(q, &S[DELTA ? 0 : chunk & 1][0][l16][4 * quad]);          // Q S0
+            row_pieces(q, a.q, next);
+            o[0] *= fall.x; o[1] *= fall.y; o[2] *= fall.z; o[3] *= fall.w;
+            fall = rc_ld4(vec_at(next) + i0);
+            if (DELTA) {
+                rc_meet();
+                rc_meet();
+            }
+            rc_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            if (!DELTA) used_columns(v, 1.f, chunk);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                if (m <= w16) p[m & 1] = rc_mfma4(tri[m], DELTA ? rc_ld4(&U[l16][16 * m + 4 * quad]) : v[m], p[m & 1]);
+            triangle(tri, mats_at(next));
+            if (!DELTA) v_columns(v, next);
+            o += p[0] + p[1];
+            {
+                float* to = a.out + ((size_t)(row0 + 16 * w16) * a.H + h) * a.Dv + c0;
+                const uint32_t off = (uint32_t)(4 * quad * a.H * a.Dv + l16), row = (uint32_t)(a.H * a.Dv);
+                if (rows >= RC_L) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) *(to + (size_t)(e * row) + off) = o[e];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (i0 + e < rows) *(to + (size_t)(e * row) + off) = o[e];
+                }
+            }
+            none += 0.f * o[0] + 0.f * o[1] + 0.f * o[2] + 0.f * o[3];
+            rc_meet();
+        }
     }
     if (none != none) odd = 1;
     __syncthreads();
     if (!odd) {
-        for (int i = tid; i < J * RC_C * 4; i += 256) {
-            const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
-            rc_st4(st + ((size_t)j * a.Dv + c) * 16 + r, rc_ld4(&S[j][c][r]));
-        }
+        if (wave < 4)
+#pragma unroll
+            for (int t = 0; t < JP; ++t)
+                if (has(t)) rc_st4(st + ((size_t)(wave + 4 * t) * a.Dv + l16) * 16 + 4 * quad, own[t]);
         return;
     }
     // Not finite somewhere (a state that once is stays so): the portion again from its first state, token by token.  0 times an
     // infinity or a NaN is no 0, so that above it shows in rows before its own, too; and a negative decay has no logarithm.
-    const int c = tid >> 4, r = tid & 15;               // 16 lanes a column, rows r, r + 16, ..
+    extern __shared__ __align__(16) float lds[];
+    float* Q = lds;                                     // [64][LD]
+    float* K = Q + RC_L * LD;
+    float* V = K + RC_L * LD;                           // [64][17]
+    const int c = tid >> 4 & 15, r = tid & 15;          // waves 0 to 3: 16 lanes a column, rows r, r + 16, ..
     float s[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) s[j] = st[((size_t)j * a.Dv + c) * 16 + r];
-    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
+    __syncthreads();                                    // (all have read the state before some write it)
+    for (int chunk = 0; chunk < chunks; ++chunk) {
         const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L < RC_L ? n - chunk * RC_L : RC_L;
-        fetch(chunk);
+        for (int i = tid; i < rows * (D / 4); i += 512) {
+            const int y = i / (D / 4), x = i % (D / 4) * 4;
+            const size_t at = (size_t)(row0 + y) * a.ld + (size_t)kvh * D + x;
+            rc_st4(Q + y * LD + x, rc_act4<ACT>(rc_ld4(a.q + at), a.q_scale));
+            rc_st4(K + y * LD + x, rc_act4<ACT>(rc_ld4(a.k + at), a.k_scale));
+        }
+        for (int i = tid; i < rows * RC_C; i += 512)
+            V[i / RC_C * (RC_C + 1) + i % RC_C] = rc_act<ACT>(a.v[(size_t)(row0 + i / RC_C) * a.ld + (size_t)h * a.Dv + c0 + i % RC_C], 1.f);
         __syncthreads();
-        stage();
-        __syncthreads();
-        for (int i = 0; i < rows; ++i) {
+        for (int i = 0; i < rows && wave < 4; ++i) {
             const float g = DELTA ? a.gate[(size_t)(row0 + i) * a.ld_g + h] : a.decay[h];
             const float* k = K + i * LD + r;
             const float* q = Q + i * LD + r;
-            float u = V[i][c], o = 0.f;
+            float u = V[i * (RC_C + 1) + c], o = 0.f;
             if (DELTA) {
                 float d = 0.f;
 #pragma unroll
                 for (int j = 0; j < J; ++j) d = fmaf(s[j], k[16 * j], d);
 #pragma unroll
                 for (int m = 8; m > 0; m >>= 1) d += __shfl_xor(d, m, 64);
-                u = vec[2 * RC_L + i] * (u - g * d);
+                u = a.beta[(size_t)(row0 + i) * a.ld_b + h] * (u - g * d);
             }
 #pragma unroll
             for (int j = 0; j < J; ++j) {
@@ -374,15 +480,17 @@ __global__ __launch_bounds__(256) void k_chunk_run(ChunkArgs a) {
             for (int m = 8; m > 0; m >>= 1) o += __shfl_xor(o, m, 64);
             if (r == 0) a.out[((size_t)(row0 + i) * a.H + h) * a.Dv + c0 + c] = o;
         }
+        __syncthreads();
     }
+    if (wave < 4)
 #pragma unroll
-    for (int j = 0; j < J; ++j) st[((size_t)j * a.Dv + c) * 16 + r] = s[j];
+        for (int j = 0; j < J; ++j) st[((size_t)j * a.Dv + c) * 16 + r] = s[j];
 }
 
-template <int D, bool DELTA>
+template <int D, bool DELTA, bool ACT>
 static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t stream) {
-    const int one = 2 * RC_L * (D + 4) * 4, mats = one + (DELTA ? 2 : 0) * RC_L * RC_LDM * 4, run = one + (DELTA ? 2 : 1) * RC_L * RC_LDM * 4;
-    const void* kernels[2] = {(const void*)k_chunk_mats<D, DELTA>, (const void*)k_chunk_run<D, DELTA>};
+    const int one = 2 * RC_L * (D + 4) * 4, mats = one + (DELTA ? 2 : 0) * RC_L * RC_LDM * 4, run = one + RC_L * (RC_C + 1) * 4;
+    const void* kernels[2] = {(const void*)k_chunk_mats<D, DELTA, ACT>, (const void*)k_chunk_run<D, DELTA, ACT>};
     const int bytes[2] = {mats, run};
     for (int i = 0; i < 2; ++i)
         if (bytes[i] > 65536) {
@@ -390,9 +498,9 @@ static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t strea
             if (e != hipSuccess) (void)hipGetLastError();
             XR_REQUIRE(e == hipSuccess, "recurrence in chunks: %d bytes of LDS: %s", bytes[i], hipGetErrorString(e));
         }
-    k_chunk_mats<D, DELTA><<<dim3((max_q + RC_L - 1) / RC_L, a.H, B), 256, mats, stream>>>(a);
+    k_chunk_mats<D, DELTA, ACT><<<dim3((max_q + RC_L - 1) / RC_L, a.H, B), 256, mats, stream>>>(a);
     XR_CHECK_LAUNCH("chunk_mats");
-    k_chunk_run<D, DELTA><<<dim3(a.Dv / RC_C * a.H, B), 256, run, stream>>>(a);
+    k_chunk_run<D, DELTA, ACT><<<dim3(a.Dv / RC_C * a.H, B), 512, run, stream>>>(a);
     XR_CHECK_LAUNCH("chunk_run");
     return XR_OK;
 }
@@ -411,14 +519,17 @@ extern "C" int xr_recurrence_chunks(float* out, const float* q, const float* k, 
     XR_REQUIRE(ld % 4 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)state | (uintptr_t)scratch) & 15) == 0,
                "recurrence in chunks: rows that are not 16-byte aligned (%d apart)", ld);
     XR_REQUIRE(act == 0 || act == 1, "recurrence in chunks: activation %d of q, k and v (0: none, 1: SiLU)", act);
+    XR_REQUIRE((long long)ld * RC_L * 4 < (1ll << 32) && (long long)H * Dv * RC_L < (1ll << 31), "recurrence in chunks: rows %d apart", ld);
     XR_REQUIRE(n_reqs <= 65535 && H <= 65535, "recurrence in chunks: %d requests, %d heads", n_reqs, H);
     const long long mats = (long long)places * H * (delta ? 2 : 1) * RC_L * RC_L;
     XR_REQUIRE(scratch_floats >= mats + (long long)places * H * RC_VEC, "recurrence in chunks: a scratch of %lld floats for %d chunks", scratch_floats, places);
     if (n_reqs == 0 || max_q == 0) return XR_OK;
     ChunkArgs a{out, q, k, v, beta, gate, decay, state, scratch, scratch + mats, cu_q, slots, reqs,
-                H, G, Dv, ld, ld_g, ld_b, act, q_scale, k_scale};
-#define RC(DD) case DD: return delta ? launch_chunks<DD, true>(a, n_reqs, max_q, stream) : launch_chunks<DD, false>(a, n_reqs, max_q, stream)
+                H, G, Dv, ld, ld_g, ld_b, q_scale, k_scale};
+#define RCA(DD, ACT) (delta ? launch_chunks<DD, true, ACT>(a, n_reqs, max_q, stream) : launch_chunks<DD, false, ACT>(a, n_reqs, max_q, stream))
+#define RC(DD) case DD: return act ? RCA(DD, true) : RCA(DD, false)
     switch (D) { RC(48); RC(64); RC(80); RC(96); RC(112); RC(128); }
 #undef RC
+#undef RCA
     return XR_BAD_ARG;
 }
