@@ -159,6 +159,13 @@ extern "C" int xr_head_rmsnorm(float* q, float* k, int ld, const float* wq, cons
     return XR_OK;
 }
 
+__device__ inline void unpack8(uint4 w, float* f) {
+    f[0] = __uint_as_float(w.x << 16); f[1] = __uint_as_float(w.x & 0xffff0000u);
+    f[2] = __uint_as_float(w.y << 16); f[3] = __uint_as_float(w.y & 0xffff0000u);
+    f[4] = __uint_as_float(w.z << 16); f[5] = __uint_as_float(w.z & 0xffff0000u);
+    f[6] = __uint_as_float(w.w << 16); f[7] = __uint_as_float(w.w & 0xffff0000u);
+}
+
 // ---------------------------------------------------------------- the means of the blocks a step completes
 // Request b held starts[b] positions before the step and brings n = cu_q[b+1] - cu_q[b]: the
 // blocks starts[b] / P .. (starts[b] + n) / P - 1 are complete now.  One workgroup per
@@ -197,6 +204,51 @@ __global__ __launch_bounds__(256) void k_pool_blocks(T* __restrict__ pk, T* __re
     }
 }
 
+// Blocks of P positions that begin at multiples of 8, in pages that do: a key's channel is read 16 positions at a time, a value's 8
+// positions in one load, and a page is looked up once for 8 (the sums' order is the same).
+// 32 blocks of 64, 8 key/value heads of 128: 25.6 us -> 5.1, bound by two trips to memory; 700 tokens, 4 heads 22.3 -> 4.9.
+__global__ __launch_bounds__(256) void k_pool_blocks8(bf16_t* __restrict__ pk, bf16_t* __restrict__ pv, const bf16_t* __restrict__ kc,
+                                                      const bf16_t* __restrict__ vc, const int* __restrict__ starts,
+                                                      const int* __restrict__ cu_q, const int* __restrict__ block_table,
+                                                      int table_stride, const int* __restrict__ pool_table, int pool_stride,
+                                                      int Hk, int D, int Dv, int P, int page_shift, int page_mask, int page_size) {
+    const int b = blockIdx.z, h = blockIdx.y;
+    const int s = starts[b], n = cu_q[b + 1] - cu_q[b];
+    const int blk = s / P + blockIdx.x;
+    if (blk >= (s + n) / P) return;
+    const int* bt = block_table + (size_t)b * table_stride;
+    const int ppage = pool_table[(size_t)b * pool_stride + (blk >> page_shift)];
+    const int poff = blk & page_mask;
+    const float inv = 1.0f / (float)P;
+    for (int e = threadIdx.x; e < D + Dv; e += 256) {
+        float acc = 0.f;
+        if (e < D) {
+#pragma unroll 2
+            for (int j = 0; j < P; j += 8) {
+                const int pos = blk * P + j;
+                const bf16_t* at = kc + (((size_t)bt[pos >> page_shift] * Hk + h) * page_size + (pos & page_mask)) * D + e;
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = ld<bf16_t>(at, (size_t)i * D);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc += x[i];
+            }
+            st<bf16_t>(pk, (((size_t)ppage * Hk + h) * page_size + poff) * D + e, acc * inv);
+        } else {
+            const int d = e - D;
+#pragma unroll 4
+            for (int j = 0; j < P; j += 8) {
+                const int pos = blk * P + j;
+                float x[8];
+                unpack8(*reinterpret_cast<const uint4*>(vc + (((size_t)bt[pos >> page_shift] * Hk + h) * Dv + d) * page_size + (pos & page_mask)), x);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc += x[i];
+            }
+            st<bf16_t>(pv, (((size_t)ppage * Hk + h) * Dv + d) * page_size + poff, acc * inv);
+        }
+    }
+}
+
 extern "C" int xr_pool_blocks(void* pk, void* pv, const void* k_cache, const void* v_cache, const int* starts,
                               const int* cu_q, const int* block_table, int table_stride, const int* pool_table,
                               int pool_stride, int B, int max_new_blocks, int Hk, int D, int Dv, int P, int page_size,
@@ -210,6 +262,9 @@ extern "C" int xr_pool_blocks(void* pk, void* pv, const void* k_cache, const voi
         k_pool_blocks<float><<<grid, 256, 0, stream>>>((float*)pk, (float*)pv, (const float*)k_cache, (const float*)v_cache,
                                                       starts, cu_q, block_table, table_stride, pool_table, pool_stride, Hk,
                                                       D, Dv, P, shift, page_size - 1, page_size);
+    else if (dtype == XR_BF16 && P % 8 == 0 && page_size % 8 == 0 && ((uintptr_t)v_cache & 15) == 0)
+        k_pool_blocks8<<<grid, 256, 0, stream>>>((bf16_t*)pk, (bf16_t*)pv, (const bf16_t*)k_cache, (const bf16_t*)v_cache, starts, cu_q, block_table,
+                                                 table_stride, pool_table, pool_stride, Hk, D, Dv, P, shift, page_size - 1, page_size);
     else if (dtype == XR_BF16)
         k_pool_blocks<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)pk, (bf16_t*)pv, (const bf16_t*)k_cache,
                                                        (const bf16_t*)v_cache, starts, cu_q, block_table, table_stride,
@@ -237,12 +292,6 @@ struct PoolAttnArgs {
 // a time, and the values, which lie position by position inside a page, eight positions of a
 // channel at a time; tiles then begin on multiples of 8 (keys below `lo` in the first tile count as
 // absent), so a group of eight never leaves its page.
-__device__ inline void unpack8(uint4 w, float* f) {
-    f[0] = __uint_as_float(w.x << 16); f[1] = __uint_as_float(w.x & 0xffff0000u);
-    f[2] = __uint_as_float(w.y << 16); f[3] = __uint_as_float(w.y & 0xffff0000u);
-    f[4] = __uint_as_float(w.z << 16); f[5] = __uint_as_float(w.z & 0xffff0000u);
-    f[6] = __uint_as_float(w.w << 16); f[7] = __uint_as_float(w.w & 0xffff0000u);
-}
 
 template <typename T, bool VEC, int MAXD = AP_MAX_D>
 __device__ inline void attend_range(const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ bt, int lo,

@@ -92,6 +92,8 @@ _PROTOS = {
     "xr_head_rmsnorm": [_p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _f, _i, _p],
     "xr_moe_table_route": [_p, _p, _p, _p, _i, _i, _i, _i, _f, _p],
     "xr_layernorm_conv_rows": [_p] * 7 + [_i] * 5 + [_f, _i, _p],
+    "xr_conv_rows_store": [_p] * 4 + [_i] + [_p] * 4 + [_i, _p, _p] + [_i] * 9 + [_p],
+    "xr_rotate_pair": [_p] * 4 + [_i] * 5 + [_f, _f, _p],
     "xr_conv_qkv_store": [_p, _p, _p, _p, _i, _p, _p, _p, _i, _p, _p] + [_i] * 8 + [_p],
     "xr_recurrence_step": [_p] * 15 + [_i] * 11 + [_f] * 4 + [_i, _i, _p],
     "xr_sample": [_p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _p],
@@ -1197,6 +1199,17 @@ class Ops:
                                                   dtype_code(out_dtype), _stream()))
         return out
 
+    def rotate_pair_(self, q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, inv_freq: Optional[torch.Tensor], heads: int, D: int,
+                     rot: int, q_scale: float = 1.0, k_scale: float = 1.0) -> None:
+        """``rotate_rows_`` of two views with one row stride and as many heads, in one kernel."""
+        self._dev(q, k, positions, inv_freq)
+        if any(x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1 or tuple(x.shape) != (positions.numel(), heads * D) for x in (q, k)) or q.stride(0) != k.stride(0):
+            raise KernelError(f"rotate_pair_: float32 views [rows, {heads * D}] with unit column stride and one row stride are needed")
+        if rot and (inv_freq is None or inv_freq.numel() != rot // 2 or inv_freq.dtype != torch.float32):
+            raise KernelError(f"rotate_pair_: {rot // 2} 32-bit frequencies are needed")
+        self.lib.check(self.lib.xr_rotate_pair(q.data_ptr(), k.data_ptr(), positions.data_ptr(), _ptr(inv_freq), q.shape[0], heads, D, rot,
+                                               q.stride(0), float(q_scale), float(k_scale), _stream()))
+
     def layernorm_conv_rows(self, x: torch.Tensor, w: Optional[torch.Tensor], eps: float, conv_w: torch.Tensor,
                             state: Optional[torch.Tensor], ctx, out_dtype: torch.dtype) -> Optional[torch.Tensor]:
         """``layernorm_conv`` for steps in which requests bring several rows; None where its kernel does not take the sizes
@@ -1909,14 +1922,17 @@ class Ops:
                                              dtype_code(out_dtype), _stream()))
         return q_out
 
+    CONV_STORE_TAPS = 9         # taps whose carried inputs one block of a request's rows reads
+
     def conv_qkv_store(self, u, w, state, k_cache, v_cache, ctx, group: int, H: int, Hk: int, D: int, Dv: int, page_size: int,
                        out_dtype: torch.dtype) -> torch.Tensor:
-        """``causal_conv`` of the input product's rows ``u [B, H * D + Hk * (D + Dv)]`` without activation, then ``qkv_store`` (``Hk`` 0: this
-        layer stores no keys), in one kernel for a step of one row a request; ``state`` is brought up to date."""
+        """``causal_conv`` of the input product's rows ``u [T, H * D + Hk * (D + Dv)]`` without activation, then ``qkv_store`` (``Hk`` 0: this
+        layer stores no keys), in one kernel; ``state`` is brought up to date.  2 to 16 taps, 2 to 9 where requests bring several rows."""
         self._dev(u, w, state, k_cache, v_cache)
         T, Cn = u.shape
-        if u.dtype != torch.float32 or u.stride(1) != 1 or Cn != H * D + Hk * (D + Dv) or ctx.max_q_len != 1 or T != ctx.B:
-            raise KernelError("conv_qkv_store: float32 rows of queries, keys and values are needed, one a request")
+        one_each = ctx.max_q_len == 1 and T == ctx.B
+        if u.dtype != torch.float32 or u.stride(1) != 1 or Cn != H * D + Hk * (D + Dv):
+            raise KernelError("conv_qkv_store: float32 rows of queries, keys and values are needed")
         if w.dtype != torch.float32 or w.dim() != 2 or w.shape[0] != Cn or not w.is_contiguous() or w.shape[1] < 2:
             raise KernelError(f"conv_qkv_store: the convolution's weight must be float32 [{Cn}, taps]")
         taps = w.shape[1]
@@ -1926,10 +1942,15 @@ class Ops:
             raise KernelError("conv_qkv_store: the cache does not fit the heads")
         table = ctx.block_table(group)
         q_out = torch.empty((T, H * D), dtype=out_dtype, device=u.device)
-        self.lib.check(self.lib.xr_conv_qkv_store(
-            q_out.data_ptr(), _ptr(k_cache) if Hk else None, _ptr(v_cache) if Hk else None, u.data_ptr(), u.stride(0), w.data_ptr(), state.data_ptr(),
-            ctx.slots.data_ptr(), taps, ctx.positions.data_ptr(), table.data_ptr(), table.stride(0), T, H, Hk, D, Dv, page_size,
-            dtype_code(out_dtype), _stream()))
+        kc, vc = _ptr(k_cache) if Hk else None, _ptr(v_cache) if Hk else None
+        if one_each:
+            self.lib.check(self.lib.xr_conv_qkv_store(
+                q_out.data_ptr(), kc, vc, u.data_ptr(), u.stride(0), w.data_ptr(), state.data_ptr(), ctx.slots.data_ptr(), taps,
+                ctx.positions.data_ptr(), table.data_ptr(), table.stride(0), T, H, Hk, D, Dv, page_size, dtype_code(out_dtype), _stream()))
+        else:
+            self.lib.check(self.lib.xr_conv_rows_store(
+                q_out.data_ptr(), kc, vc, u.data_ptr(), u.stride(0), w.data_ptr(), state.data_ptr(), ctx.cu_q.data_ptr(), ctx.slots.data_ptr(), taps,
+                ctx.starts_dev.data_ptr(), table.data_ptr(), table.stride(0), T, ctx.B, H, Hk, D, Dv, page_size, dtype_code(out_dtype), _stream()))
         return q_out
 
     def pool_blocks(self, pk, pv, k_cache, v_cache, ctx, group: int, pool_group: int, Hk: int, D: int, Dv: int, P: int,
@@ -1962,6 +1983,10 @@ class Ops:
             # The window's keys go to the matrix-core kernels, every row block leaving a partial
             # result; the block means leave theirs in a slot of their own; the kernels' merge adds them.
             lib = self.attention_lib(D)
+            # a step whose last position sees no whole block behind its window has no means to read, and needs no slot and no merge
+            # for them (a prompt of 700 tokens, 16 heads of 128 over a window of 1,024: 17 us a layer)
+            if P and getattr(ctx, "knows_lengths", False) and ctx.max_seq_len - size < P:
+                P = 0
             plan = self._attention_plan(ctx, group, H, Hk, D, D, page_size, scale, size, bool(P), q, k_cache, v_cache)
             part_o = part_ml = None
             if plan.n_slots:

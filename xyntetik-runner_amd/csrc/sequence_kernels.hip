@@ -224,21 +224,15 @@ template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu
 // CONV_ROWS + 1 taps), and writes it anew.  Bound by memory and, for few rows, by that chain.  (Four channels a thread with 16-byte loads was slower:
 // 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 26.7 us, and k_conv_state's 4.7 behind it are saved.
 #define CONV_ROWS 8
-template <typename TU, typename TO>
-__global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, const TU* __restrict__ u,
-                                                          const float* __restrict__ w, const float* __restrict__ bias, TU* state,
-                                                          const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int C,
-                                                          int taps, int ld_u, int ld_out, int residual, int act) {
-    int b, k;
-    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= C) return;
-    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
-    TU* const srow = state + (size_t)slots[b] * (taps - 1) * C;
+// Rows i0 to i0 + CONV_ROWS - 1 of channel c of request b (those that exist; the others' results mean nothing), before the activation; in the
+// request's first block also its new carried inputs.
+template <typename TU>
+__device__ __forceinline__ void conv_rows(float (&y)[CONV_ROWS], const TU* __restrict__ u, const float* __restrict__ w, float bias, TU* state, int row0,
+                                          int n, int i0, int slot, int c, int C, int taps, int ld_u, int residual) {
+    TU* const srow = state + (size_t)slot * (taps - 1) * C;
     float wt[CONV_MAX_TAPS];
 #pragma unroll
     for (int j = 0; j < CONV_MAX_TAPS; ++j) wt[j] = j < taps ? w[(size_t)c * taps + j] : 0.f;
-    const float bc = bias ? bias[c] : 0.f;
     if (taps <= 4 && i0 + CONV_ROWS <= n) {
         float v[CONV_ROWS + 3];
 #pragma unroll
@@ -253,31 +247,30 @@ __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, 
             for (int j = 0; j < 4; ++j)
                 if (j < taps) acc = fmaf(wt[j], taps == 4 ? v[r + j] : taps == 3 ? v[r + j + 1 < CONV_ROWS + 3 ? r + j + 1 : 0]
                                                 : taps == 2 ? v[r + j + 2 < CONV_ROWS + 3 ? r + j + 2 : 0] : v[r + 3], acc);
-            acc += bc;
+            acc += bias;
             if (residual) acc += v[r + 3];
-            if (act == XR_CONV_SILU) acc = acc / (1.0f + expf(-acc));
-            st<TO>(out, (size_t)(row0 + i0 + r) * ld_out + c, acc);
+            y[r] = acc;
         }
     } else {
 #pragma unroll
         for (int r = 0; r < CONV_ROWS; ++r) {
             const int i = i0 + r;
-            if (i >= n) break;
             float acc = 0.f;
+            if (i < n) {
 #pragma unroll
-            for (int j = 0; j < CONV_MAX_TAPS; ++j) {
-                if (j >= taps) break;
-                const int s = i - (taps - 1) + j;
-                const float val = s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
-                acc = fmaf(wt[j], val, acc);
+                for (int j = 0; j < CONV_MAX_TAPS; ++j) {
+                    if (j >= taps) break;
+                    const int s = i - (taps - 1) + j;
+                    const float val = s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
+                    acc = fmaf(wt[j], val, acc);
+                }
+                acc += bias;
+                if (residual) acc += ld<TU>(u, (size_t)(row0 + i) * ld_u + c);
             }
-            acc += bc;
-            if (residual) acc += ld<TU>(u, (size_t)(row0 + i) * ld_u + c);
-            if (act == XR_CONV_SILU) acc = acc / (1.0f + expf(-acc));
-            st<TO>(out, (size_t)(row0 + i) * ld_out + c, acc);
+            y[r] = acc;
         }
     }
-    if (k > 0 || taps < 2 || taps - 1 > CONV_ROWS) return;
+    if (i0 > 0 || taps < 2 || taps - 1 > CONV_ROWS) return;
     TU keep[CONV_ROWS];
 #pragma unroll
     for (int m = 0; m < CONV_ROWS; ++m) {
@@ -290,6 +283,95 @@ __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, 
         if (m >= taps - 1) break;
         srow[(size_t)m * C + c] = keep[m];
     }
+}
+
+template <typename TU, typename TO>
+__global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, const TU* __restrict__ u,
+                                                          const float* __restrict__ w, const float* __restrict__ bias, TU* state,
+                                                          const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int C,
+                                                          int taps, int ld_u, int ld_out, int residual, int act) {
+    int b, k;
+    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= C) return;
+    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
+    float y[CONV_ROWS];
+    conv_rows<TU>(y, u, w, bias ? bias[c] : 0.f, state, row0, n, i0, slots[b], c, C, taps, ld_u, residual);
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r) {
+        if (i0 + r >= n) break;
+        st<TO>(out, (size_t)(row0 + i0 + r) * ld_out + c, act == XR_CONV_SILU ? y[r] / (1.0f + expf(-y[r])) : y[r]);
+    }
+}
+
+// The convolution of a mixer's queries, keys and values (no bias, no activation) with the store behind it: queries go to q_out, keys and values to the cache pages
+// of their positions (K [page][kv head][place][D], V [page][kv head][Dv][place]; Hk 0: none).  A thread's rows of a value are places side by side, one store where they are
+// whole and aligned (store8), where a kernel of its own stored 2 bytes a lane 128 apart.  2,048 rows, 6,144 and 4,096 channels:
+// 20.9 us on average, as two kernels 21.3 + 17.0; 700 rows of half the width 8.3 (6.5 + 7.9).
+__device__ inline void store8(float* p, const float (&y)[CONV_ROWS]) {
+    reinterpret_cast<float4*>(p)[0] = make_float4(y[0], y[1], y[2], y[3]);
+    reinterpret_cast<float4*>(p)[1] = make_float4(y[4], y[5], y[6], y[7]);
+}
+__device__ inline void store8(bf16_t* p, const float (&y)[CONV_ROWS]) {
+    *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]), pack_bf16x2(y[6], y[7]));
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_conv_rows_store(T* __restrict__ q_out, T* __restrict__ kc, T* __restrict__ vc, const float* __restrict__ u, int ld,
+                                                         const float* __restrict__ w, float* state, const int* __restrict__ cu_q,
+                                                         const int* __restrict__ slots, int taps, const int* __restrict__ starts,
+                                                         const int* __restrict__ block_table, int table_stride, int B, int Q, int Hk, int D, int Dv,
+                                                         int page_shift, int page_mask, int page_size) {
+    int b, k;
+    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
+    const int C = Q + Hk * (D + Dv), c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= C) return;
+    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
+    float y[CONV_ROWS];
+    conv_rows<float>(y, u, w, 0.f, state, row0, n, i0, slots[b], c, C, taps, ld, 0);
+    if (c < Q) {
+#pragma unroll
+        for (int r = 0; r < CONV_ROWS; ++r)
+            if (i0 + r < n) st<T>(q_out, (size_t)(row0 + i0 + r) * Q + c, y[r]);
+        return;
+    }
+    const int pos = starts[b] + i0;
+    const int* bt = block_table + (size_t)b * table_stride;
+    const bool key = c - Q < Hk * D;
+    const int i = key ? c - Q : c - Q - Hk * D, size = key ? D : Dv, h = i / size, d = i - h * size;
+    if (!key && i0 + CONV_ROWS <= n && pos % CONV_ROWS == 0 && page_size % CONV_ROWS == 0) {
+        store8(vc + (((size_t)bt[pos >> page_shift] * Hk + h) * Dv + d) * page_size + (pos & page_mask), y);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r) {
+        if (i0 + r >= n) break;
+        const int page = bt[(pos + r) >> page_shift], off = (pos + r) & page_mask;
+        if (key) st<T>(kc, (((size_t)page * Hk + h) * page_size + off) * D + d, y[r]);
+        else st<T>(vc, (((size_t)page * Hk + h) * Dv + d) * page_size + off, y[r]);
+    }
+}
+
+extern "C" int xr_conv_rows_store(void* q_out, void* k_cache, void* v_cache, const float* u, int ld, const float* w, float* state, const int* cu_q,
+                                  const int* slots, int taps, const int* starts, const int* block_table, int table_stride, int T, int B, int H,
+                                  int Hk, int D, int Dv, int page_size, int dtype, hipStream_t stream) {
+    XR_REQUIRE(T >= 0 && B >= 0 && H > 0 && Hk >= 0 && D > 0 && Dv > 0 && taps > 1 && taps - 1 <= CONV_ROWS, "conv_rows_store: bad sizes T=%d B=%d H=%d Hk=%d D=%d Dv=%d taps=%d",
+               T, B, H, Hk, D, Dv, taps);
+    const int C = H * D + Hk * (D + Dv), shift = ilog2_exact(page_size);
+    XR_REQUIRE(shift >= 0 && ld >= C, "conv_rows_store: page size %d, rows %d apart for %d channels", page_size, ld, C);
+    XR_REQUIRE(q_out && u && w && state && cu_q && slots && starts && (Hk == 0 || (k_cache && v_cache && block_table)), "conv_rows_store: null operand");
+    XR_REQUIRE(Hk == 0 || ((uintptr_t)v_cache & 15) == 0, "conv_rows_store: values that are not 16-byte aligned");
+    const long long blocks = ((long long)T + (long long)B * (CONV_ROWS - 1)) / CONV_ROWS;
+    XR_REQUIRE(blocks <= 65535, "conv_rows_store: %d rows of %d requests", T, B);
+    XR_REQUIRE(dtype == XR_F32 || dtype == XR_BF16, "conv_rows_store: bad dtype %d", dtype);
+    if (T == 0 || B == 0) return XR_OK;
+    const dim3 grid((C + 255) / 256, (unsigned)blocks);
+#define CRS(T_) k_conv_rows_store<T_><<<grid, 256, 0, stream>>>((T_*)q_out, (T_*)k_cache, (T_*)v_cache, u, ld, w, state, cu_q, slots, taps, starts, block_table, \
+                                                               table_stride, B, H * D, Hk, D, Dv, shift, page_size - 1, page_size)
+    if (dtype == XR_F32) CRS(float);
+    else CRS(bf16_t);
+#undef CRS
+    XR_CHECK_LAUNCH("conv_rows_store");
+    return XR_OK;
 }
 
 template <typename TU>
@@ -802,6 +884,51 @@ extern "C" int xr_rotate_rows(float* x, const int* positions, const float* inv_f
     if (T == 0 || (rot == 0 && scale == 1.0f)) return XR_OK;
     k_rotate_rows<<<dim3(T, heads), 64, 0, stream>>>(x, positions, inv_freq, D, rot, ld, scale);
     XR_CHECK_LAUNCH("rotate_rows");
+    return XR_OK;
+}
+
+// Queries and keys of a token with the same number of heads in one launch, a workgroup a token: angles are made once a token, not once a head.  2,048 tokens,
+// 32 heads of 128: 26.1 us, as two launches of k_rotate_rows 42; 100 tokens and fewer cost a launch less.
+__global__ __launch_bounds__(256) void k_rotate_pair(float* __restrict__ x, float* __restrict__ y, const int* __restrict__ positions,
+                                                     const float* __restrict__ inv_freq, int heads, int D, int half, int ld, float scale_x, float scale_y) {
+    extern __shared__ float2 turn[];                    // [half]
+    const int t = blockIdx.x;
+    const float pos = (float)positions[t];
+    for (int j = threadIdx.x; j < half; j += 256) {
+        const float a = pos * inv_freq[j];
+        turn[j] = make_float2(cosf(a), sinf(a));
+    }
+    __syncthreads();
+    for (int which = 0; which < 2; ++which) {
+        float* row = (which ? y : x) + (size_t)t * ld;
+        const float scale = which ? scale_y : scale_x;
+        for (int i = threadIdx.x; i < heads * half; i += 256) {
+            const int h = i / half, j = i - h * half;
+            const float c = turn[j].x, s = turn[j].y;
+            float* at = row + (size_t)h * D + j;
+            const float u = at[0], v = at[half];
+            at[0] = (u * c - v * s) * scale;
+            at[half] = (v * c + u * s) * scale;
+        }
+        const int rest = D - 2 * half;
+        if (scale != 1.0f && rest > 0)
+            for (int i = threadIdx.x; i < heads * rest; i += 256) row[(size_t)(i / rest) * D + 2 * half + i % rest] *= scale;
+    }
+}
+
+extern "C" int xr_rotate_pair(float* x, float* y, const int* positions, const float* inv_freq, int T, int heads, int D, int rot, int ld, float scale_x,
+                              float scale_y, hipStream_t stream) {
+    XR_REQUIRE(T >= 0 && heads > 0 && D > 0 && ld >= heads * D, "rotate_pair: bad sizes T=%d heads=%d D=%d ld=%d", T, heads, D, ld);
+    XR_REQUIRE(rot >= 0 && rot <= D && rot % 2 == 0 && rot <= 4096, "rotate_pair: rotary width %d does not fit head size %d", rot, D);
+    XR_REQUIRE(x && y && positions && (rot == 0 || inv_freq), "rotate_pair: null operand");
+    if (T == 0) return XR_OK;
+    const int half = rot / 2;
+    if (half == 0) {
+        const int a = xr_rotate_rows(x, positions, inv_freq, T, heads, D, rot, ld, scale_x, stream);
+        return a != XR_OK ? a : xr_rotate_rows(y, positions, inv_freq, T, heads, D, rot, ld, scale_y, stream);
+    }
+    k_rotate_pair<<<T, 256, half * sizeof(float2), stream>>>(x, y, positions, inv_freq, heads, D, half, ld, scale_x, scale_y);
+    XR_CHECK_LAUNCH("rotate_pair");
     return XR_OK;
 }
 

@@ -278,6 +278,7 @@ class StepContext:
     """Device views of one step's metadata, handed to every part."""
 
     plans_few_rows = True       # its attention plans know the kernel for few rows
+    knows_lengths = True        # ``max_seq_len`` is this step's (a recorded step's lengths change from replay to replay)
 
     def __init__(self, ops, device, entries: List[StepEntry], request_caches, n_groups: int, pad_to: int = 0):
         self.ops = ops

@@ -100,7 +100,8 @@ class PooledWindowAttention(Mixer):
         if writes == self.kv_shared:
             raise ValueError("pooled attention: a layer stores its keys and values exactly when it projects them")
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
-        if self.conv_taps > 1 and ctx.max_q_len == 1 and proj.shape[0] == ctx.B and ctx.B < 65536:
+        one_each = ctx.max_q_len == 1 and proj.shape[0] == ctx.B
+        if self.conv_taps > 1 and ctx.B < 65536 and (one_each or self.conv_taps <= ops.CONV_STORE_TAPS):
             q = ops.conv_qkv_store(proj, self.w_conv, cache.states.get("mixer.conv"), cache.k if writes else None, cache.v if writes else None,
                                    ctx, cache.group, H, G if writes else 0, D, Dv, cache.page_size, self.rt.dtype)
         else:

@@ -139,9 +139,7 @@ class Retention(Mixer):
         if self.qkv_activation is not None and fused_act is None:
             ops.act_rows_(proj[:, :2 * QK + V], self.qkv_activation)
         if rot is not None:
-            ops.rotate_rows_(q, ctx.positions, rot.inv_freq, H, D, rot.rotary_dim, 1.0)
-        if rot is not None:
-            ops.rotate_rows_(k, ctx.positions, rot.inv_freq, H, D, rot.rotary_dim, self.key_scale)
+            ops.rotate_pair_(q, k, ctx.positions, rot.inv_freq, H, D, rot.rotary_dim, 1.0, self.key_scale)
         # (without a rotation the keys' scale is applied as the recurrence fetches them: a kernel less)
         o = ops.linear_recurrence("retention", q, k, v, cache.state, ctx, H, H, D, Dv, decay=self.decay, activation=fused_act,
                                   k_scale=self.key_scale if rot is None else 1.0)
