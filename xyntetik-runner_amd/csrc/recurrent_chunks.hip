@@ -20,8 +20,8 @@
 // end are zeros with beta 0 and no decay.  L is formed and subtracted in 64 bits; a decay of nothing counts as exp(-100).  A portion
 // that comes to something not finite, or has a negative decay, runs again token by token, a workgroup its 16 columns.
 // Bound by the chain of chunks, a chunk 4.5 us of the delta rule, 3.0 of retention: 1.7 and 1.1 of them the products of a SIMD's two waves, the rest the
-// trips to LDS between them and how fast a compute unit gets 100 KB a chunk from L2.  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 143 us and k_chunk_mats 79 for the
-// delta rule, 95 and 39 for retention (k_chunk_mats 57 and 24 with q . k in 32 bits); with four waves that staged every operand in LDS, at
+// barriers and trips to LDS between them (neither K's columns from LDS instead of memory nor rows asked for two chunks ahead made it faster).  2,048 tokens, 32 heads of 128 x 128: k_chunk_run 143 us and k_chunk_mats 70 for the
+// delta rule, 95 and 37 for retention (k_chunk_mats 77 and 39 with a row of blocks a wave, one to four of them; 57 and 24 of these with q . k in 32 bits); with four waves that staged every operand in LDS, at
 // barriers that waited for the next chunk's loads too, and a branch a number for the activation 189 and 138; 700 tokens, 16 heads 47 and 34 (67 and 51);
 // token by token (k_recurrence) 634, and retention in two passes over chunks of 256 side by side 520.
 #include "common.h"
@@ -147,7 +147,8 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
         vec[2 * RC_L + tid] = bt;
     }
     __syncthreads();
-    for (int ct = 0; ct <= wave; ++ct) {                // rows 16 wave .., columns 16 ct ..
+    for (int blk = wave; blk < 10; blk += 4) {          // the triangle's ten blocks, two or three a wave: rows 16 rt .., columns 16 ct ..
+        const int rt = blk < 1 ? 0 : blk < 3 ? 1 : blk < 6 ? 2 : 3, ct = blk - rt * (rt + 1) / 2;
         // q . k in 64 bits, k . k in four chains of 32: with one chain of 128 sums each the errors of the results were twice those
         // of the recurrence token by token, and with these they are as large or smaller (retention's half)
         rc_f64x4 s = {0.0, 0.0, 0.0, 0.0};
@@ -155,17 +156,17 @@ __global__ __launch_bounds__(256) void k_chunk_mats(ChunkArgs a) {
 #pragma unroll
         for (int d = 0; d < D; d += 16) {
             const float4 fb = rc_ld4(K + (16 * ct + l16) * LD + d + 4 * quad);
-            s = rc_mfma4(rc_ld4(Q + (16 * wave + l16) * LD + d + 4 * quad), fb, s);
-            if (DELTA) t[d / 16 & 3] = rc_mfma4(rc_ld4(K + (16 * wave + l16) * LD + d + 4 * quad), fb, t[d / 16 & 3]);
+            s = rc_mfma4(rc_ld4(Q + (16 * rt + l16) * LD + d + 4 * quad), fb, s);
+            if (DELTA) t[d / 16 & 3] = rc_mfma4(rc_ld4(K + (16 * rt + l16) * LD + d + 4 * quad), fb, t[d / 16 & 3]);
         }
         const rc_f32x4 kk = (t[0] + t[1]) + (t[2] + t[3]);
         const int j = 16 * ct + l16;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int i = 16 * wave + 4 * e + quad;
+            const int i = 16 * rt + 4 * e + quad;
             mats[i * RC_L + j] = j <= i ? (float)(s[e] * expf((float)(L[i] - L[j]))) : 0.f;
             if (DELTA) {
-                const int r = 16 * wave + 4 * quad + e;
+                const int r = 16 * rt + 4 * quad + e;
                 A[r * RC_LDM + j] = j < r ? beta[r] * expf((float)(L[r] - L[j])) * kk[e] : 0.f;
             }
         }
