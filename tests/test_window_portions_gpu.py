@@ -107,3 +107,20 @@ def test_steps_that_no_mean_reaches(longest, G):
     # probabilities in bfloat16 (2^-9 of each) and the result's rounding
     for other in (with_slot, plain):
         assert float((got.double() - other.double()).abs().max()) <= 2.0 ** -6 * float(plain.abs().max())
+
+
+@pytest.mark.parametrize("T,H,Dv", [(1, 1, 128), (3, 3, 128), (37, 5, 128), (8, 4, 132), (129, 3, 256)])
+@pytest.mark.parametrize("gate_first", [False, True])
+def test_gated_norm_of_two_heads_a_wave(T, H, Dv, gate_first):
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    rng = np.random.default_rng(T + Dv)
+    o, gate, w = dev(rng.normal(size=(T, H * Dv))), dev(rng.normal(size=(T, H * Dv + 4)))[:, :H * Dv], dev(rng.normal(size=Dv))
+    got = ops.gated_rmsnorm(o, gate, w, H, Dv, 1e-5, torch.bfloat16, gate_first=gate_first)
+    x, g = o.double().view(T, H, Dv), gate.double().reshape(T, H, Dv)
+    g = g * torch.sigmoid(g)
+    x = x * g if gate_first else x
+    want = x / torch.sqrt((x * x).mean(dim=2, keepdim=True) + 1e-5) * w.double() * (1 if gate_first else g)
+    # half an ulp of bfloat16, and 32-bit arithmetic's 1e-6
+    assert bool(((got.double().view(T, H, Dv) - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6 * float(want.abs().max())).all())
