@@ -651,6 +651,8 @@ __device__ __forceinline__ void plan_cuts(const SampleArgs& a, int r, const Opti
         if (last >= edge) {
             add(edge, last < past ? last : past);
             least = least < up_to(edge) ? least : up_to(edge);
+            const u64 whole = mass[last < past ? last : past];      // (what lies behind the cut's bins goes: min-p alone, 20 rows of 128,256 logits 62 us a pick with all
+            most = most < whole ? most : whole;                      // that mass left to the draw, whose run of bins then held more than the list takes)
         }
     }
     const double draw = (double)opt.draw;
