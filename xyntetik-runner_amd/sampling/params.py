@@ -81,7 +81,7 @@ class SamplerState:
         self._params = p
         # the options as the kernels read them: temperature (0: greedy), top-p, min-p, repeat penalty, top-k
         floats = 0.0 if p.greedy else p.temperature, p.top_p, p.min_p, p.repeat_penalty
-        top_k = min(p.top_k, 0x7FFFFFFF)
+        top_k = int(min(p.top_k, 0x7FFFFFFF)) if p.top_k == p.top_k else 0       # (any number's whole part; what is no number cuts nothing)
         try:
             self.words = struct.pack("=4fi", *floats, top_k)
         except OverflowError:                   # (beyond 32 bits: infinite)
