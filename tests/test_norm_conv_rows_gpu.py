@@ -91,3 +91,46 @@ def test_convolution_of_portions(dtypes, taps):
             if taps > 1:
                 assert np.array_equal(state[torch.tensor(slots, device=DEV)].double().cpu().numpy(), carried)
             at = [a + n for a, n in zip(at, lens)]
+
+
+def test_more_blocks_than_a_grid_has_rows():
+    """Rows in blocks of eight, each of one request, are up to (T + 7 B) / 8: with 21,000 requests of 1 to 40 rows more than 65,535, as with
+    600,000 rows of one; the store behind the convolution counts them alike."""
+    import torch
+    from types import SimpleNamespace
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    C, taps, ps = 4, 4, 64
+    rng = np.random.default_rng(5)
+    for lens in (rng.integers(1, 41, 21000), np.array([600_000]), np.array([524_281, 3])):
+        B, T = len(lens), int(lens.sum())
+        assert T + 7 * B > 8 * 65535
+        i32 = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)
+        cu = np.concatenate([[0], np.cumsum(lens)])
+        req = np.repeat(np.arange(B), lens)
+        pages = -(-lens // ps)
+        table = np.full((B, pages.max()), -1)
+        for b, a in enumerate(np.cumsum(pages) - pages):
+            table[b, :pages[b]] = np.arange(a, a + pages[b])
+        table = i32(table)
+        place = i32(np.arange(T) - cu[req])
+        ctx = SimpleNamespace(cu_q=i32(cu), slots=i32(np.arange(B)[::-1].copy()), req_of_token=i32(req), starts_dev=i32(np.zeros(B)), positions=place,
+                              block_table=lambda g: table, B=B, max_q_len=int(lens.max()))
+        u, w = dev(rng.normal(size=(T, C))), dev(rng.normal(size=(C, taps)))
+        before = dev(rng.normal(size=(B, taps - 1, C)))
+        states = [before.clone(), before.clone()]
+        got = ops.causal_conv(u, w, states[0], ctx, torch.float32)
+        # rows and carried inputs of all requests one behind the other
+        r = torch.tensor(req, device=DEV)
+        own = ctx.slots.long()[r]
+        want = torch.zeros((T, C), dtype=torch.float64, device=DEV)
+        for j in range(taps):
+            s = place.long() - (taps - 1) + j
+            x = torch.where((s >= 0)[:, None], u[(torch.arange(T, device=DEV) - (taps - 1) + j).clamp(min=0)], before[own, (taps - 1 + s).clamp(max=taps - 2)])
+            want += x.double() * w[:, j].double()
+        assert float((got.double() - want).abs().max()) < 1e-5 * float(want.abs().max())         # (32-bit sums of four products)
+        kc, vc = (torch.zeros((int(pages.sum()), 1, *shape), device=DEV) for shape in ((ps, 1), (1, ps)))
+        q = ops.conv_qkv_store(u, w, states[1], kc, vc, ctx, 0, 2, 1, 1, 1, ps, torch.float32)
+        assert torch.equal(q, got[:, :2]) and torch.equal(states[0], states[1])
+        page, off = table[r, place.long() // ps].long(), place.long() % ps
+        assert torch.equal(kc[page, 0, off, 0], got[:, 2]) and torch.equal(vc[page, 0, 0, off], got[:, 3])

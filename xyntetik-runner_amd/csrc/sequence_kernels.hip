@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, 
                                                           const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int C,
                                                           int taps, int ld_u, int ld_out, int residual, int act) {
     int b, k;
-    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
+    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), b, k)) return;
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
     const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
@@ -302,6 +302,14 @@ __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, 
         if (i0 + r >= n) break;
         st<TO>(out, (size_t)(row0 + i0 + r) * ld_out + c, act == XR_CONV_SILU ? y[r] / (1.0f + expf(-y[r])) : y[r]);
     }
+}
+
+// The blocks of a step's rows over y and z of a grid, however many they are.
+static bool conv_rows_grid(int C, int T, int B, dim3& grid) {
+    const long long blocks = ((long long)T + (long long)B * (CONV_ROWS - 1)) / CONV_ROWS, z = (blocks + 65534) / 65535;
+    if (blocks > 1 << 27) return false;
+    grid = dim3((C + 255) / 256, (unsigned)((blocks + z - 1) / z), (unsigned)z);
+    return true;
 }
 
 // The convolution of a mixer's queries, keys and values (no bias, no activation) with the store behind it: queries go to q_out, keys and values to the cache pages
@@ -322,7 +330,7 @@ __global__ __launch_bounds__(256) void k_conv_rows_store(T* __restrict__ q_out, 
                                                          const int* __restrict__ block_table, int table_stride, int B, int Q, int Hk, int D, int Dv,
                                                          int page_shift, int page_mask, int page_size) {
     int b, k;
-    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)blockIdx.y, b, k)) return;
+    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), b, k)) return;
     const int C = Q + Hk * (D + Dv), c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
     const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
@@ -360,11 +368,10 @@ extern "C" int xr_conv_rows_store(void* q_out, void* k_cache, void* v_cache, con
     XR_REQUIRE(shift >= 0 && ld >= C, "conv_rows_store: page size %d, rows %d apart for %d channels", page_size, ld, C);
     XR_REQUIRE(q_out && u && w && state && cu_q && slots && starts && (Hk == 0 || (k_cache && v_cache && block_table)), "conv_rows_store: null operand");
     XR_REQUIRE(Hk == 0 || ((uintptr_t)v_cache & 15) == 0, "conv_rows_store: values that are not 16-byte aligned");
-    const long long blocks = ((long long)T + (long long)B * (CONV_ROWS - 1)) / CONV_ROWS;
-    XR_REQUIRE(blocks <= 65535, "conv_rows_store: %d rows of %d requests", T, B);
     XR_REQUIRE(dtype == XR_F32 || dtype == XR_BF16, "conv_rows_store: bad dtype %d", dtype);
     if (T == 0 || B == 0) return XR_OK;
-    const dim3 grid((C + 255) / 256, (unsigned)blocks);
+    dim3 grid;
+    XR_REQUIRE(conv_rows_grid(C, T, B, grid), "conv_rows_store: %d rows of %d requests", T, B);
 #define CRS(T_) k_conv_rows_store<T_><<<grid, 256, 0, stream>>>((T_*)q_out, (T_*)k_cache, (T_*)v_cache, u, ld, w, state, cu_q, slots, taps, starts, block_table, \
                                                                table_stride, B, H * D, Hk, D, Dv, shift, page_size - 1, page_size)
     if (dtype == XR_F32) CRS(float);
@@ -410,9 +417,8 @@ extern "C" int xr_causal_conv(void* out, const void* u, const float* w, const fl
     XR_REQUIRE(!one_row_each || T == B, "causal_conv: %d rows of %d requests are not one row each", T, B);
     if (T == 0 || B == 0) return XR_OK;
     const int fuse = one_row_each && taps > 1 ? 1 : 0;
-    const long long blocks = ((long long)T + (long long)B * (CONV_ROWS - 1)) / CONV_ROWS;
-    XR_REQUIRE(one_row_each ? T <= 65535 : blocks <= 65535 && B <= 65535, "causal_conv: %d rows of %d requests", T, B);
-    dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, B), rgrid((C + 255) / 256, (unsigned)blocks);
+    dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, B), rgrid;
+    XR_REQUIRE(one_row_each ? T <= 65535 : conv_rows_grid(C, T, B, rgrid) && (taps - 1 <= CONV_ROWS || B <= 65535), "causal_conv: %d rows of %d requests", T, B);
 #define CC(TU, TO)                                                                                                   \
     do {                                                                                                             \
         if (one_row_each) {                                                                                          \
