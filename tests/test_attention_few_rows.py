@@ -103,3 +103,82 @@ def test_few_rows_kernel(case, room, monkeypatch):
         # probabilities and the result in bfloat16 (2^-9 each of a value) against the largest output
         err = (got.double() - want).abs().amax() / want.abs().amax()
         assert err < 1.2e-2, float(err)
+
+
+# What a softmax or a row may have beside its keys; every one of them is in both of the kernel's write-outs.
+EXTRAS = {
+    "sinks": dict(sinks=True),
+    "slopes": dict(slopes=True),
+    "slopes in a window, sinks": dict(slopes=True, sinks=True, window=100),
+    "cap": dict(cap=1.3),
+    "cap and sinks in chunks": dict(cap=1.3, sinks=True, chunk=64),
+    "gate": dict(gate=True, scale_out=0.75),
+    "gate and sinks in a window": dict(gate=True, scale_out=1.5, sinks=True, window=70),
+    "kept keys": dict(window=70, keep=5),
+    "kept keys, sinks, slopes, gate": dict(window=40, keep=70, sinks=True, slopes=True, gate=True, scale_out=0.5),
+    "kept keys, cap and sinks": dict(window=100, keep=3, sinks=True, cap=1.3),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("room", [1, 1024])
+@pytest.mark.parametrize("shape", [(8, 2, 64, 64), (4, 1, 128, 64), (5, 5, 32, 32), (2, 1, 256, 128)])
+@pytest.mark.parametrize("what", EXTRAS)
+def test_few_rows_kernel_with(what, shape, room, monkeypatch):
+    """Sinks, distance slopes, a soft cap, gates and kept first keys, one workgroup a request and many; pages that a window has given back are gone."""
+    from test_kernels_gpu import DEV, FakeCtx, fill_cache, scatter_pages
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    from xyntetik_runner_amd.engine import batch
+    opt = dict(dict(sinks=False, slopes=False, window=None, chunk=None, keep=0, cap=0.0, gate=False, scale_out=1.0), **EXTRAS[what])
+    H, Hk, D, ps = shape
+    window, chunk, keep = opt["window"], opt["chunk"], opt["keep"]
+    mask = Chunked(chunk) if chunk else window
+    monkeypatch.setattr(batch, "FEW_SLOTS", room)
+    rng = np.random.default_rng(len(what) * 100 + H + D)
+    starts, q_lens = [0, 37, 129, 300, 1500, 64], [1, 2, 1, 2, 1, 1]
+    lens = [s + n for s, n in zip(starts, q_lens)]
+    tables, n_pages = scatter_pages(lens, ps, D)
+    ctx = FakeCtx(starts, q_lens, tables, ps)
+    ctx.plans_few_rows, ctx._plans, ctx.device = True, {}, DEV
+    ctx.attention_plan = lambda *a, **k: batch.StepContext.attention_plan(ctx, *a, **k)
+    bf = lambda a: torch.tensor(a).bfloat16()
+    qs = [bf(rng.normal(size=(n, H, D)) * 2) for n in q_lens]
+    ks, vs = ([bf(rng.normal(size=(n, Hk, D))) for n in lens] for _ in range(2))
+    kc, vc = fill_cache(ks, vs, tables, n_pages, ps, torch.bfloat16)
+    if mask:
+        tab = ctx._table.cpu()
+        for b, s in enumerate(starts):
+            tab[b, -(-keep // ps):max(-(-keep // ps), first_key(mask, s) // ps)] = -1
+        ctx._table = tab.to(DEV)
+    T, scale = sum(q_lens), 1.1 / math.sqrt(D)
+    sinks = rng.normal(size=H) * 2
+    sinks[0], sinks[-1] = 30.0, -30.0           # one that outweighs every key, one that none feels
+    slopes, gate = 2.0 ** -np.linspace(2, 7, H), rng.normal(size=(T, H + 2))
+    dev = lambda a: torch.tensor(a, dtype=torch.float32, device=DEV)
+    want, r = np.empty((T, H, D)), 0
+    for b, n in enumerate(q_lens):
+        for i in range(n):
+            p = starts[b] + i
+            js = np.array(sorted(set(range(min(keep, p + 1))) | set(range(first_key(mask, p), p + 1))))
+            for h in range(H):
+                s = ks[b][js, h // (H // Hk)].double().numpy() @ qs[b][i, h].double().numpy() * scale
+                if opt["cap"]:
+                    s = opt["cap"] * np.tanh(s / opt["cap"])
+                if opt["slopes"]:
+                    s = s - np.float64(np.float32(slopes[h])) * (p - js)
+                top = max(s.max(), sinks[h]) if opt["sinks"] else s.max()
+                e = np.exp(s - top)
+                o = e / (e.sum() + (np.exp(sinks[h] - top) if opt["sinks"] else 0.0)) @ vs[b][js, h // (H // Hk)].double().numpy()
+                want[r, h] = o * (1 / (1 + np.exp(-gate[r, h])) if opt["gate"] else 1.0) * opt["scale_out"]
+            r += 1
+    q = torch.cat(qs).reshape(T, H * D).contiguous().to(DEV)
+    more = {**({"extra_slot": True} if keep else {}), "few_rows": 2 if 2 * D <= 256 else 1}
+    plan = ctx.attention_plan(0, H // Hk, mask, Hk, ps, **more)
+    assert plan.n_few >= len(starts) and plan.n_items == plan.n_cta_items == plan.n_jobs == 0
+    for _ in range(2):
+        got = load_ops().attention(q, kc, vc, ctx, 0, H, Hk, D, ps, scale, window, chunk=chunk, keep_first=keep, softcap=opt["cap"],
+                                   slopes=dev(slopes) if opt["slopes"] else None, sinks=dev(sinks) if opt["sinks"] else None,
+                                   gate=dev(gate)[:, :H] if opt["gate"] else None, out_scale=opt["scale_out"]).cpu().double().numpy().reshape(T, H, D)
+        assert len(ctx._plans) == 1 and int(plan.counters.abs().sum()) == 0 and np.isfinite(got).all()
+        # probabilities and the result in bfloat16 (2^-9 each of a value) against the largest output, as above
+        assert np.abs(got - want).max() < 1.2e-2 * np.abs(want).max()
