@@ -37,6 +37,26 @@ def test_convolution_of_portions_and_store(H, Hk, D, Dv, taps, ps, dtype):
         at = [a + n for a, n in zip(at, lens)]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("off", [1, 2, 4])
+def test_convolution_and_store_to_values_at_any_address(off, dtype):
+    """A value's eight places are stored one by one where the cache is not 16-byte aligned."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dt = load_ops(), getattr(torch, dtype)
+    H, Hk, D, ps, taps, lens = 2, 1, 8, 16, 4, [24, 9]
+    rng = np.random.default_rng(off)
+    C = (H + 2 * Hk) * D
+    u, w, tables = dev(rng.normal(size=(sum(lens), C))), dev(rng.normal(size=(C, taps))), tables_for(2, 2)
+    ctx = step_ctx([0, 0], lens, [1, 0], [tables])
+    got = []
+    for at in (0, off):
+        kc = torch.zeros((4, Hk, ps, D), dtype=dt, device=DEV)
+        vc = torch.zeros((4 * Hk * D * ps + at,), dtype=dt, device=DEV)[at:].view(4, Hk, D, ps)
+        got.append((ops.conv_qkv_store(u, w, torch.zeros((3, taps - 1, C), device=DEV), kc, vc, ctx, 0, H, Hk, D, D, ps, dt), kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][2].any())
+
+
 @pytest.mark.parametrize("heads,D,rot", [(1, 6, 4), (3, 64, 64), (32, 128, 96), (5, 130, 130), (2, 16, 0)])
 def test_queries_and_keys_turned_together(heads, D, rot):
     import torch

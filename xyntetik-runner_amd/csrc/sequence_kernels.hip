@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256) void k_conv_rows_store(T* __restrict__ q_out, 
                                                          const float* __restrict__ w, float* state, const int* __restrict__ cu_q,
                                                          const int* __restrict__ slots, int taps, const int* __restrict__ starts,
                                                          const int* __restrict__ block_table, int table_stride, int B, int Q, int Hk, int D, int Dv,
-                                                         int page_shift, int page_mask, int page_size) {
+                                                         int page_shift, int page_mask, int page_size, int wide) {
     int b, k;
     if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), b, k)) return;
     const int C = Q + Hk * (D + Dv), c = blockIdx.x * 256 + threadIdx.x;
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void k_conv_rows_store(T* __restrict__ q_out, 
     const int* bt = block_table + (size_t)b * table_stride;
     const bool key = c - Q < Hk * D;
     const int i = key ? c - Q : c - Q - Hk * D, size = key ? D : Dv, h = i / size, d = i - h * size;
-    if (!key && i0 + CONV_ROWS <= n && pos % CONV_ROWS == 0 && page_size % CONV_ROWS == 0) {
+    if (wide && !key && i0 + CONV_ROWS <= n && pos % CONV_ROWS == 0) {
         store8(vc + (((size_t)bt[pos >> page_shift] * Hk + h) * Dv + d) * page_size + (pos & page_mask), y);
         return;
     }
@@ -367,13 +367,13 @@ extern "C" int xr_conv_rows_store(void* q_out, void* k_cache, void* v_cache, con
     const int C = H * D + Hk * (D + Dv), shift = ilog2_exact(page_size);
     XR_REQUIRE(shift >= 0 && ld >= C, "conv_rows_store: page size %d, rows %d apart for %d channels", page_size, ld, C);
     XR_REQUIRE(q_out && u && w && state && cu_q && slots && starts && (Hk == 0 || (k_cache && v_cache && block_table)), "conv_rows_store: null operand");
-    XR_REQUIRE(Hk == 0 || ((uintptr_t)v_cache & 15) == 0, "conv_rows_store: values that are not 16-byte aligned");
     XR_REQUIRE(dtype == XR_F32 || dtype == XR_BF16, "conv_rows_store: bad dtype %d", dtype);
     if (T == 0 || B == 0) return XR_OK;
     dim3 grid;
     XR_REQUIRE(conv_rows_grid(C, T, B, grid), "conv_rows_store: %d rows of %d requests", T, B);
+    const int wide = page_size % CONV_ROWS == 0 && ((uintptr_t)v_cache & 15) == 0;      // (a value's eight places are 16 bytes or 32 behind one another)
 #define CRS(T_) k_conv_rows_store<T_><<<grid, 256, 0, stream>>>((T_*)q_out, (T_*)k_cache, (T_*)v_cache, u, ld, w, state, cu_q, slots, taps, starts, block_table, \
-                                                               table_stride, B, H * D, Hk, D, Dv, shift, page_size - 1, page_size)
+                                                               table_stride, B, H * D, Hk, D, Dv, shift, page_size - 1, page_size, wide)
     if (dtype == XR_F32) CRS(float);
     else CRS(bf16_t);
 #undef CRS
