@@ -190,27 +190,37 @@ __global__ __launch_bounds__(256) void k_causal_conv(TO* __restrict__ out, const
     st<TO>(out, (size_t)t * ld_out + c, acc);
 }
 
-// A step's rows in blocks of R, none of which holds rows of two requests: block `blk` is block k of request b.  At most
-// (T + B (R - 1)) / R blocks; false for those past the last.  (Every lane of a wave takes part; requests without rows have no block.)
-template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu_q, int B, int blk, int& b, int& k) {
-    if (B == 1) {                                       // (no search: the chain of loads and exchanges takes a workgroup over a microsecond)
-        b = 0, k = blk;
-        return blk * R < cu_q[1] - cu_q[0];
+// A lane's sum with another lane's number (DPP), where there is one.
+template <int CTRL, int ROWS> __device__ __forceinline__ int plus_lane(int v) { return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }
+
+// A step's rows in blocks of R, none of which holds rows of two requests: block `blk` is block k of request b, which has n rows from row0 on and
+// its carried inputs at `slot`.  At most (T + B (R - 1)) / R blocks; false for those past the last.  (Every lane of a wave takes part; requests without rows
+// have no block.  All a workgroup needs to know before its first row is one round of loads and a scan between lanes: with the request looked for by
+// shuffles, and what it has loaded again behind that, 8 requests of 7 rows took 1.1 us longer.)
+struct RowBlock { int b, k, row0, n, slot; };
+template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int blk, RowBlock& x) {
+    if (B == 1) {
+        x.b = 0; x.k = blk; x.row0 = cu_q[0]; x.n = cu_q[1] - x.row0; x.slot = slots[0];
+        return blk * R < x.n;
     }
     const int lane = threadIdx.x & 63;
     for (int b0 = 0; b0 < B; b0 += 64) {
-        const int n = b0 + lane < B ? cu_q[b0 + lane + 1] - cu_q[b0 + lane] : 0, own = (n + R - 1) / R;
-        int upto = own;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(upto, o, 64);
-            if (lane >= o) upto += t;
-        }
-        const int total = __shfl(upto, 63, 64);
+        const int b = b0 + lane < B ? b0 + lane : B - 1;
+        const int row0 = cu_q[b], n = b0 + lane < B ? cu_q[b + 1] - row0 : 0, slot = slots[b], own = (n + R - 1) / R;
+        int upto = plus_lane<0x111, 0xF>(own);          // shifts by 1, 2, 4 and 8 lanes inside a row of 16,
+        upto = plus_lane<0x112, 0xF>(upto);
+        upto = plus_lane<0x114, 0xF>(upto);
+        upto = plus_lane<0x118, 0xF>(upto);
+        upto = plus_lane<0x142, 0xA>(upto);             // the last lane of rows 0 and 2 to rows 1 and 3,
+        upto = plus_lane<0x143, 0xC>(upto);             // that of row 1 to rows 2 and 3
+        const int total = __builtin_amdgcn_readlane(upto, 63);
         if (blk < total) {
             const int at = __ffsll((unsigned long long)__ballot(upto > blk)) - 1;
-            b = __builtin_amdgcn_readfirstlane(b0 + at);
-            k = __builtin_amdgcn_readfirstlane(blk - __shfl(upto - own, at, 64));
+            x.b = b0 + at;
+            x.k = blk - __builtin_amdgcn_readlane(upto - own, at);
+            x.row0 = __builtin_amdgcn_readlane(row0, at);
+            x.n = __builtin_amdgcn_readlane(n, at);
+            x.slot = __builtin_amdgcn_readlane(slot, at);
             return true;
         }
         blk -= total;
@@ -222,85 +232,72 @@ template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu
 // every input is read once; what a row needs before its first input (its request, the request's first row and state row) are loads
 // that wait for each other, once a block and not once a row.  The first block of a request is the only one that reads its state (up to
 // CONV_ROWS + 1 taps), and writes it anew.  Bound by memory and, for few rows, by that chain.  (Four channels a thread with 16-byte loads was slower:
-// 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 26.7 us, and k_conv_state's 4.7 behind it are saved.
+// 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 26.6 us, and k_conv_state's 4.7 behind it are saved; 17 rows of 2,048
+// channels with 5 taps 4.2 (a row a thread and k_conv_state 4.9), 8 requests of 7 rows with 4 taps 4.2 (4.9), 200 rows of 8,192 with 9 taps 7.6 (18).
 #define CONV_ROWS 8
-// Rows i0 to i0 + CONV_ROWS - 1 of channel c of request b (those that exist; the others' results mean nothing), before the activation; in the
-// request's first block also its new carried inputs.
-template <typename TU>
-__device__ __forceinline__ void conv_rows(float (&y)[CONV_ROWS], const TU* __restrict__ u, const float* __restrict__ w, float bias, TU* state, int row0,
-                                          int n, int i0, int slot, int c, int C, int taps, int ld_u, int residual) {
-    TU* const srow = state + (size_t)slot * (taps - 1) * C;
-    float wt[CONV_MAX_TAPS];
+// Rows i0 to i0 + CONV_ROWS - 1 of channel c of a request (those that exist; the others' results mean nothing), before the activation; in the
+// request's first block also its new carried inputs.  All inputs of the rows are read before the first product, for up to TM taps and for rows that are fewer than a
+// block, too (input by input, a row after the other, 17 rows of 2,048 channels with 16 taps took 14.7 us, with 5 6.8).
+template <int TM, typename TU>
+__device__ __forceinline__ void conv_rows(float (&y)[CONV_ROWS], const TU* __restrict__ u, const float* __restrict__ w, float bias, TU* state, const RowBlock& x,
+                                          int i0, int c, int C, int taps, int ld_u, int residual) {
+    TU* const srow = state + (size_t)x.slot * (taps - 1) * C;
+    const TU* const col = u + (size_t)x.row0 * ld_u + c;
+    const int none = TM - taps;                     // places of the window that fewer taps leave unread
+    float wt[TM], v[CONV_ROWS + TM - 1];
 #pragma unroll
-    for (int j = 0; j < CONV_MAX_TAPS; ++j) wt[j] = j < taps ? w[(size_t)c * taps + j] : 0.f;
-    if (taps <= 4 && i0 + CONV_ROWS <= n) {
-        float v[CONV_ROWS + 3];
+    for (int j = 0; j < TM; ++j) wt[j] = j >= none ? w[(size_t)c * taps + j - none] : 0.f;
 #pragma unroll
-        for (int m = 0; m < CONV_ROWS + 3; ++m) {
-            const int s = i0 + m - 3;               // (taps below 4 leave the first of them unread)
-            v[m] = m < 4 - taps ? 0.f : s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
-        }
+    for (int m = 0; m < CONV_ROWS + TM - 1; ++m) {
+        const int s = i0 + m - (TM - 1);
+        v[m] = m < none ? 0.f : s >= 0 ? ld<TU>(col, (size_t)(s < x.n ? s : x.n - 1) * ld_u) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
+    }
+    const bool carries = i0 == 0 && taps > 1 && taps - 1 <= CONV_ROWS;
+    constexpr int KEEP = TM - 1 < CONV_ROWS ? TM - 1 : CONV_ROWS;
+    TU keep[KEEP];
+    if (carries) {
 #pragma unroll
-        for (int r = 0; r < CONV_ROWS; ++r) {
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (j < taps) acc = fmaf(wt[j], taps == 4 ? v[r + j] : taps == 3 ? v[r + j + 1 < CONV_ROWS + 3 ? r + j + 1 : 0]
-                                                : taps == 2 ? v[r + j + 2 < CONV_ROWS + 3 ? r + j + 2 : 0] : v[r + 3], acc);
-            acc += bias;
-            if (residual) acc += v[r + 3];
-            y[r] = acc;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < CONV_ROWS; ++r) {
-            const int i = i0 + r;
-            float acc = 0.f;
-            if (i < n) {
-#pragma unroll
-                for (int j = 0; j < CONV_MAX_TAPS; ++j) {
-                    if (j >= taps) break;
-                    const int s = i - (taps - 1) + j;
-                    const float val = s >= 0 ? ld<TU>(u, (size_t)(row0 + s) * ld_u + c) : ld<TU>(srow, (size_t)(taps - 1 + s) * C + c);
-                    acc = fmaf(wt[j], val, acc);
-                }
-                acc += bias;
-                if (residual) acc += ld<TU>(u, (size_t)(row0 + i) * ld_u + c);
-            }
-            y[r] = acc;
+        for (int m = 0; m < KEEP; ++m) {
+            const int s = x.n - (taps - 1) + m;
+            if (m < taps - 1) keep[m] = s >= 0 ? col[(size_t)s * ld_u] : srow[(size_t)(m + x.n) * C + c];
         }
     }
-    if (i0 > 0 || taps < 2 || taps - 1 > CONV_ROWS) return;
-    TU keep[CONV_ROWS];
 #pragma unroll
-    for (int m = 0; m < CONV_ROWS; ++m) {
-        if (m >= taps - 1) break;
-        const int s = n - (taps - 1) + m;
-        keep[m] = s >= 0 ? u[(size_t)(row0 + s) * ld_u + c] : srow[(size_t)(m + n) * C + c];
+    for (int r = 0; r < CONV_ROWS; ++r) y[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        if (j < none) continue;
+#pragma unroll
+        for (int r = 0; r < CONV_ROWS; ++r) y[r] = fmaf(wt[j], v[r + j], y[r]);
     }
 #pragma unroll
-    for (int m = 0; m < CONV_ROWS; ++m) {
-        if (m >= taps - 1) break;
-        srow[(size_t)m * C + c] = keep[m];
+    for (int r = 0; r < CONV_ROWS; ++r) {
+        y[r] += bias;
+        if (residual) y[r] += v[r + TM - 1];
+    }
+    if (carries) {
+#pragma unroll
+        for (int m = 0; m < KEEP; ++m)
+            if (m < taps - 1) srow[(size_t)m * C + c] = keep[m];
     }
 }
 
-template <typename TU, typename TO>
+template <int TM, typename TU, typename TO>
 __global__ __launch_bounds__(256) void k_causal_conv_rows(TO* __restrict__ out, const TU* __restrict__ u,
                                                           const float* __restrict__ w, const float* __restrict__ bias, TU* state,
                                                           const int* __restrict__ cu_q, const int* __restrict__ slots, int B, int C,
                                                           int taps, int ld_u, int ld_out, int residual, int act) {
-    int b, k;
-    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), b, k)) return;
+    RowBlock x;
+    if (!rows_of_block<CONV_ROWS>(cu_q, slots, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), x)) return;
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
-    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
+    const int i0 = x.k * CONV_ROWS;
     float y[CONV_ROWS];
-    conv_rows<TU>(y, u, w, bias ? bias[c] : 0.f, state, row0, n, i0, slots[b], c, C, taps, ld_u, residual);
+    conv_rows<TM, TU>(y, u, w, bias ? bias[c] : 0.f, state, x, i0, c, C, taps, ld_u, residual);
 #pragma unroll
     for (int r = 0; r < CONV_ROWS; ++r) {
-        if (i0 + r >= n) break;
-        st<TO>(out, (size_t)(row0 + i0 + r) * ld_out + c, act == XR_CONV_SILU ? y[r] / (1.0f + expf(-y[r])) : y[r]);
+        if (i0 + r >= x.n) break;
+        st<TO>(out, (size_t)(x.row0 + i0 + r) * ld_out + c, act == XR_CONV_SILU ? y[r] / (1.0f + expf(-y[r])) : y[r]);
     }
 }
 
@@ -323,27 +320,26 @@ __device__ inline void store8(float* p, const float (&y)[CONV_ROWS]) {
 __device__ inline void store8(bf16_t* p, const float (&y)[CONV_ROWS]) {
     *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]), pack_bf16x2(y[6], y[7]));
 }
-template <typename T>
+template <int TM, typename T>
 __global__ __launch_bounds__(256) void k_conv_rows_store(T* __restrict__ q_out, T* __restrict__ kc, T* __restrict__ vc, const float* __restrict__ u, int ld,
                                                          const float* __restrict__ w, float* state, const int* __restrict__ cu_q,
                                                          const int* __restrict__ slots, int taps, const int* __restrict__ starts,
                                                          const int* __restrict__ block_table, int table_stride, int B, int Q, int Hk, int D, int Dv,
                                                          int page_shift, int page_mask, int page_size, int wide) {
-    int b, k;
-    if (!rows_of_block<CONV_ROWS>(cu_q, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), b, k)) return;
+    RowBlock x;
+    if (!rows_of_block<CONV_ROWS>(cu_q, slots, B, (int)(blockIdx.z * gridDim.y + blockIdx.y), x)) return;
     const int C = Q + Hk * (D + Dv), c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
-    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * CONV_ROWS;
+    const int i0 = x.k * CONV_ROWS, n = x.n, pos = starts[x.b] + i0;
     float y[CONV_ROWS];
-    conv_rows<float>(y, u, w, 0.f, state, row0, n, i0, slots[b], c, C, taps, ld, 0);
+    conv_rows<TM, float>(y, u, w, 0.f, state, x, i0, c, C, taps, ld, 0);
     if (c < Q) {
 #pragma unroll
         for (int r = 0; r < CONV_ROWS; ++r)
-            if (i0 + r < n) st<T>(q_out, (size_t)(row0 + i0 + r) * Q + c, y[r]);
+            if (i0 + r < n) st<T>(q_out, (size_t)(x.row0 + i0 + r) * Q + c, y[r]);
         return;
     }
-    const int pos = starts[b] + i0;
-    const int* bt = block_table + (size_t)b * table_stride;
+    const int* bt = block_table + (size_t)x.b * table_stride;
     const bool key = c - Q < Hk * D;
     const int i = key ? c - Q : c - Q - Hk * D, size = key ? D : Dv, h = i / size, d = i - h * size;
     if (wide && !key && i0 + CONV_ROWS <= n && pos % CONV_ROWS == 0) {
@@ -372,7 +368,7 @@ extern "C" int xr_conv_rows_store(void* q_out, void* k_cache, void* v_cache, con
     dim3 grid;
     XR_REQUIRE(conv_rows_grid(C, T, B, grid), "conv_rows_store: %d rows of %d requests", T, B);
     const int wide = page_size % CONV_ROWS == 0 && ((uintptr_t)v_cache & 15) == 0;      // (a value's eight places are 16 bytes or 32 behind one another)
-#define CRS(T_) k_conv_rows_store<T_><<<grid, 256, 0, stream>>>((T_*)q_out, (T_*)k_cache, (T_*)v_cache, u, ld, w, state, cu_q, slots, taps, starts, block_table, \
+#define CRS(T_) (taps <= 4 ? k_conv_rows_store<4, T_> : k_conv_rows_store<CONV_ROWS + 1, T_>)<<<grid, 256, 0, stream>>>((T_*)q_out, (T_*)k_cache, (T_*)v_cache, u, ld, w, state, cu_q, slots, taps, starts, block_table, \
                                                                table_stride, B, H * D, Hk, D, Dv, shift, page_size - 1, page_size, wide)
     if (dtype == XR_F32) CRS(float);
     else CRS(bf16_t);
@@ -418,6 +414,9 @@ extern "C" int xr_causal_conv(void* out, const void* u, const float* w, const fl
     if (T == 0 || B == 0) return XR_OK;
     const int fuse = one_row_each && taps > 1 ? 1 : 0;
     dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, B), rgrid;
+    // Taps whose carried inputs a kernel of its own moves on: few rows go a row a thread, more of them side by side (17 rows of
+    // 2,048 channels, 16 taps 9.5 us and 8.1 a row a thread; 200 rows of 8,192 16.4 and more than 25)
+    const bool pair = taps - 1 > CONV_ROWS && T < 64;
     XR_REQUIRE(one_row_each ? T <= 65535 : conv_rows_grid(C, T, B, rgrid) && (taps - 1 <= CONV_ROWS || B <= 65535), "causal_conv: %d rows of %d requests", T, B);
 #define CC(TU, TO)                                                                                                   \
     do {                                                                                                             \
@@ -426,7 +425,11 @@ extern "C" int xr_causal_conv(void* out, const void* u, const float* w, const fl
                                                             req_of_token, C, taps, ld_u, ld_out, residual, act, fuse); \
             break;                                                                                                   \
         }                                                                                                            \
-        k_causal_conv_rows<TU, TO><<<rgrid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots, B, C, taps, \
+        if (pair) {                                                                                                  \
+            k_causal_conv<TU, TO><<<grid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots, \
+                                                            req_of_token, C, taps, ld_u, ld_out, residual, act, 0);  \
+        } else                                                                                                       \
+        (taps <= 4 ? k_causal_conv_rows<4, TU, TO> : taps <= CONV_ROWS + 1 ? k_causal_conv_rows<CONV_ROWS + 1, TU, TO> : k_causal_conv_rows<CONV_MAX_TAPS, TU, TO>)<<<rgrid, 256, 0, stream>>>((TO*)out, (const TU*)u, w, bias, (TU*)state, cu_q, slots, B, C, taps, \
                                                               ld_u, ld_out, residual, act);                          \
         if (taps - 1 > CONV_ROWS)                                                                                    \
             k_conv_state<TU><<<sgrid, 256, 0, stream>>>((TU*)state, (const TU*)u, cu_q, slots, C, taps, ld_u);       \
@@ -660,10 +663,10 @@ __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restri
                                                                  const int* __restrict__ slots, int B, int E, int ldx, int taps, float eps) {
 #pragma clang fp contract(off)      // (a normed row is rounded before it is added, as where the norm's kernel stores it)
     __shared__ __align__(16) float part[8][16];
-    int b, k;
+    RowBlock blk;
     const int share = (int)gridDim.x >> 3;              // (the grid is a multiple of 8: an XCD takes an eighth of the blocks, in order)
-    if (!rows_of_block<LNC_ROWS>(cu_q, B, ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3), b, k)) return;
-    const int row0 = cu_q[b], n = cu_q[b + 1] - row0, i0 = k * LNC_ROWS;
+    if (!rows_of_block<LNC_ROWS>(cu_q, slots, B, ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3), blk)) return;
+    const int row0 = blk.row0, n = blk.n, k = blk.k, i0 = k * LNC_ROWS;
     const int c = threadIdx.x * 4;
     float4 h[LNC_HELD];                                 // the rows; then without their mean, normed, as the convolution reads them
 #pragma unroll
@@ -700,7 +703,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restri
     const float rinv = 1.0f / sqrtf(sums_of_8<NW>(s, part) / (float)E + eps);
 #pragma unroll
     for (int m = 0; m < 8; ++m) s[m] = of_lane(rinv, m);        // (here, where all lanes are: below, rinv would be made in those that go on)
-    float* const srow = state + (size_t)slots[b] * (taps - 1) * E;
+    float* const srow = state + (size_t)blk.slot * (taps - 1) * E;
     if (c >= E) return;
 #pragma unroll
     for (int m = 0; m < LNC_HELD; ++m) h[m] = make_float4(h[m].x * s[m] * gw.x, h[m].y * s[m] * gw.y, h[m].z * s[m] * gw.z, h[m].w * s[m] * gw.w);
