@@ -792,7 +792,9 @@ __device__ inline float4 ld4(const bf16_t* p) {
     return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
 }
 
-template <typename TZ, typename TO, int NW, int N4>
+// AGAIN: squares and cubes are made again.  Kept from the sums, they take two registers more a value, and a compute unit then has room for one row of more
+// than 8,192 numbers instead of two or more; where it has one to work on anyway, making them again is the longer way.
+template <typename TZ, typename TO, int NW, int N4, bool AGAIN>
 __global__ __launch_bounds__(64 * NW) void k_polynorm_v4(TO* __restrict__ out, const TZ* __restrict__ z, const float* __restrict__ coef,
                                                          int F, int ld_z, float eps) {
     __shared__ float part[3][NW];
@@ -824,7 +826,7 @@ __global__ __launch_bounds__(64 * NW) void k_polynorm_v4(TO* __restrict__ out, c
     const float r1 = coef[0] / sqrtf(s2 * inv + eps), r2 = coef[1] / sqrtf(s4 * inv + eps), r3 = coef[2] / sqrtf(s6 * inv + eps), e = coef[3];
     auto value = [&](float x) { const float x2 = x * x; return x * r1 + x2 * r2 + x2 * x * r3 + e; };
     TO* o = out + (size_t)blockIdx.x * F;
-    // (squares and cubes are made again: kept from the sums, they took two registers more a value, and a compute unit had room for one row of 21,504 instead of two: 2,048 of them 54 us, 49)
+    if constexpr (AGAIN)
 #pragma unroll
     for (int u = 0; u < N4; ++u) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y), "+v"(v[u].z), "+v"(v[u].w));
 #pragma unroll
@@ -834,16 +836,22 @@ __global__ __launch_bounds__(64 * NW) void k_polynorm_v4(TO* __restrict__ out, c
     }
 }
 
+// More rows than compute units, each of more than 8,192 numbers, make their powers again (us without and with it, in bfloat16:
+// 257 rows of 10,752 7.4 and 6.2, of 21,504 9.6 and 8.0, 2,048 rows of them 30 and 22, 42 and 32; 64 rows of 16,384 4.8 and 5.1, 2,048 of 8,192 19.9 and 20.9)
+#define POLY_AGAIN_ROWS 256
 template <typename TZ, typename TO>
 static bool launch_polynorm_v4(TO* out, const TZ* z, const float* coef, int T, int F, int ld_z, float eps, hipStream_t stream) {
     if (F % 4 || ld_z % 4 || ((uintptr_t)z % 16) || ((uintptr_t)out % 16) || F > 16 * 64 * 4 * 8) return false;
-#define PV(NW, N4) k_polynorm_v4<TZ, TO, NW, N4><<<T, 64 * NW, 0, stream>>>(out, z, coef, F, ld_z, eps)
+    const bool again = T > POLY_AGAIN_ROWS;
+#define PV(NW, N4) k_polynorm_v4<TZ, TO, NW, N4, false><<<T, 64 * NW, 0, stream>>>(out, z, coef, F, ld_z, eps)
+#define PA(NW, N4) do { if (again) k_polynorm_v4<TZ, TO, NW, N4, true><<<T, 64 * NW, 0, stream>>>(out, z, coef, F, ld_z, eps); else PV(NW, N4); } while (0)
     // four waves a row where they hold it; 16 where rows are few (every lane's loads are a trip to memory) or long
     if (F <= 4 * 256 * 4 && !(T <= FEW_ROWS && F >= 1024)) PV(4, 4);
     else if (F <= 16 * 256 * 2) PV(16, 2);
-    else if (F <= 16 * 256 * 4) PV(16, 4);
-    else if (F <= 16 * 256 * 6) PV(16, 6);
-    else PV(16, 8);
+    else if (F <= 16 * 256 * 4) PA(16, 4);
+    else if (F <= 16 * 256 * 6) PA(16, 6);
+    else PA(16, 8);
+#undef PA
 #undef PV
     return true;
 }
