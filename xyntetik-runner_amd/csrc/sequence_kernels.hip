@@ -907,8 +907,10 @@ extern "C" int xr_rotate_rows(float* x, const int* positions, const float* inv_f
     return XR_OK;
 }
 
-// Queries and keys of a token with the same number of heads in one launch, a workgroup a token: angles are made once a token, not once a head.  2,048 tokens,
-// 32 heads of 128: 26.1 us, as two launches of k_rotate_rows 42; 100 tokens and fewer cost a launch less.
+// Queries and keys of a token with the same number of heads in one launch; angles are made once a workgroup, not once a head.  Bound by memory, and for few
+// tokens by a thread's chain of heads: so a token's 2 x heads heads are shared out to gridDim.y workgroups, which make its angles each.  2,048 tokens, 32 heads of
+// 128: 22 us, as two launches of k_rotate_rows 38; 8 tokens 2.8, as two launches 4.1, with one workgroup a token 5.4.
+#define ROT_PAIR_FILL 512
 __global__ __launch_bounds__(256) void k_rotate_pair(float* __restrict__ x, float* __restrict__ y, const int* __restrict__ positions,
                                                      const float* __restrict__ inv_freq, int heads, int D, int half, int ld, float scale_x, float scale_y) {
     extern __shared__ float2 turn[];                    // [half]
@@ -919,10 +921,13 @@ __global__ __launch_bounds__(256) void k_rotate_pair(float* __restrict__ x, floa
         turn[j] = make_float2(cosf(a), sinf(a));
     }
     __syncthreads();
+    const int share = (2 * heads + (int)gridDim.y - 1) / (int)gridDim.y, from = (int)blockIdx.y * share, to = min(from + share, 2 * heads);
+    const int rest = D - 2 * half;
     for (int which = 0; which < 2; ++which) {
-        float* row = (which ? y : x) + (size_t)t * ld;
+        const int lo = max(from - which * heads, 0), hi = min(to - which * heads, heads);       // this workgroup's heads of x, of y
+        float* row = (which ? y : x) + (size_t)t * ld + (size_t)lo * D;
         const float scale = which ? scale_y : scale_x;
-        for (int i = threadIdx.x; i < heads * half; i += 256) {
+        for (int i = threadIdx.x; i < (hi - lo) * half; i += 256) {
             const int h = i / half, j = i - h * half;
             const float c = turn[j].x, s = turn[j].y;
             float* at = row + (size_t)h * D + j;
@@ -930,9 +935,8 @@ __global__ __launch_bounds__(256) void k_rotate_pair(float* __restrict__ x, floa
             at[0] = (u * c - v * s) * scale;
             at[half] = (v * c + u * s) * scale;
         }
-        const int rest = D - 2 * half;
         if (scale != 1.0f && rest > 0)
-            for (int i = threadIdx.x; i < heads * rest; i += 256) row[(size_t)(i / rest) * D + 2 * half + i % rest] *= scale;
+            for (int i = threadIdx.x; i < (hi - lo) * rest; i += 256) row[(size_t)(i / rest) * D + 2 * half + i % rest] *= scale;
     }
 }
 
@@ -947,7 +951,11 @@ extern "C" int xr_rotate_pair(float* x, float* y, const int* positions, const fl
         const int a = xr_rotate_rows(x, positions, inv_freq, T, heads, D, rot, ld, scale_x, stream);
         return a != XR_OK ? a : xr_rotate_rows(y, positions, inv_freq, T, heads, D, rot, ld, scale_y, stream);
     }
-    k_rotate_pair<<<T, 256, half * sizeof(float2), stream>>>(x, y, positions, inv_freq, heads, D, half, ld, scale_x, scale_y);
+    // so many workgroups a token that a thread has one pair of each of two heads' rows, while all fit the compute units twice over
+    int shares = 1;
+    const long long most = (long long)heads * (half > D - 2 * half ? half : D - 2 * half);
+    while (2 * shares <= 2 * heads && 2LL * shares * T <= ROT_PAIR_FILL && most > 256LL * shares) shares *= 2;
+    k_rotate_pair<<<dim3(T, shares), 256, half * sizeof(float2), stream>>>(x, y, positions, inv_freq, heads, D, half, ld, scale_x, scale_y);
     XR_CHECK_LAUNCH("rotate_pair");
     return XR_OK;
 }
