@@ -617,8 +617,8 @@ extern "C" int xr_layernorm_conv(void* out, const float* x, const float* w, cons
 // three before them, a thread 4 channels of all eight, which stay in its registers from the one read through both sums to the convolution: the
 // normed rows never go to memory.  A request's first workgroup alone reads the carried inputs; with no rows before its own it takes the portion's last three
 // in their place, which become the new ones.  Neighbouring workgroups, which share three rows, run on one XCD.  Bound by memory: a row comes 8 / LNC_ROWS
-// times, from L2 all but once, and goes once; and by a workgroup's two sums, one behind the other.  2,048 rows of 4,096 24.1 us, where k_layernorm_rows, k_causal_conv_rows and
-// k_conv_state took 13.2 + 18.2 + 4.7; 700 rows of 2,048 9.4 (5.1 + 6.5 + 3.3).  A wave a row for the sums and every row read again for the convolution: 40.8.
+// times, from L2 all but once, and goes once; and by a workgroup's two sums, one behind the other.  2,048 rows of 4,096 23 us, where k_layernorm_rows, k_causal_conv_rows and
+// k_conv_state took 32; 700 rows of 2,048 6.9 (13.3), 33 rows of 4,096 9.3 (9.7; with loads that waited for one another 10.1, and weights of two taps loaded one by one 12.2).  A wave a row for the sums and every row read again for the convolution: 40.8.
 // (Up to 4,096 channels: with 8 a thread the registers do not suffice.)
 #define LNC_ROWS 5
 #define LNC_HELD (LNC_ROWS + 3)
@@ -656,11 +656,25 @@ __device__ inline float4 pick(bool first, float4 a, float4 b) {
     return make_float4(first ? a.x : b.x, first ? a.y : b.y, first ? a.z : b.z, first ? a.w : b.w);
 }
 
-template <typename TO, int NW>
+// The weights of four channels that lie behind one another, taps from the right, in as many 16-byte pieces as there are taps.
+template <int N> __device__ __forceinline__ void tap_weights(float (&wt)[4][4], const float* cw) {
+    float f[4 * N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float4 t = reinterpret_cast<const float4*>(cw)[i];
+        f[4 * i] = t.x; f[4 * i + 1] = t.y; f[4 * i + 2] = t.z; f[4 * i + 3] = t.w;
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wt[d][j] = j + N >= 4 ? f[d * N + j + N - 4] : 0.f;
+}
+
+template <typename TO, int NW, int TAPS>
 __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restrict__ out, const float* __restrict__ x,
                                                                  const float* __restrict__ w, const float* __restrict__ cw,
                                                                  float* state, const int* __restrict__ cu_q,
-                                                                 const int* __restrict__ slots, int B, int E, int ldx, int taps, float eps) {
+                                                                 const int* __restrict__ slots, int B, int E, int ldx, float eps) {
 #pragma clang fp contract(off)      // (a normed row is rounded before it is added, as where the norm's kernel stores it)
     __shared__ __align__(16) float part[8][16];
     RowBlock blk;
@@ -668,26 +682,21 @@ __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restri
     if (!rows_of_block<LNC_ROWS>(cu_q, slots, B, ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3), blk)) return;
     const int row0 = blk.row0, n = blk.n, k = blk.k, i0 = k * LNC_ROWS;
     const int c = threadIdx.x * 4;
+    const int cs = c < E ? c : 0;
     float4 h[LNC_HELD];                                 // the rows; then without their mean, normed, as the convolution reads them
+    auto row_of = [&](int m) { return k == 0 && m < 3 ? n - 3 + m : i0 - 3 + m; };
 #pragma unroll
-    for (int m = 0; m < LNC_HELD; ++m) {
-        const int i = k == 0 && m < 3 ? n - 3 + m : i0 - 3 + m;
-        h[m] = c < E && i >= 0 && i < n ? *reinterpret_cast<const float4*>(x + (size_t)(row0 + i) * ldx + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int m = 0; m < LNC_HELD; ++m) {                // (from some row and column in any case, so that no load waits for another)
+        const int i = row_of(m);
+        h[m] = *reinterpret_cast<const float4*>(x + (size_t)(row0 + (i < 0 ? 0 : i < n ? i : n - 1)) * ldx + cs);
     }
-    const int cs = c < E ? c : 0;                       // (weights are on their way, too, before the first sum)
     const float4 gw = w ? *reinterpret_cast<const float4*>(w + cs) : make_float4(1.f, 1.f, 1.f, 1.f);
     float wt[4][4];                                 // channel, tap (the last is the row itself)
-    if (taps == 4) {
+    tap_weights<TAPS>(wt, cw + (size_t)cs * TAPS);
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const float4 t = *reinterpret_cast<const float4*>(cw + (size_t)(cs + d) * 4);
-            wt[d][0] = t.x; wt[d][1] = t.y; wt[d][2] = t.z; wt[d][3] = t.w;
-        }
-    } else {
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) wt[d][j] = j + taps >= 4 ? cw[(size_t)(cs + d) * taps + j + taps - 4] : 0.f;
+    for (int m = 0; m < LNC_HELD; ++m) {
+        const bool in = c < E && row_of(m) >= 0 && row_of(m) < n;
+        h[m] = pick(in, h[m], make_float4(0.f, 0.f, 0.f, 0.f));
     }
     float s[8];
 #pragma unroll
@@ -703,23 +712,23 @@ __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restri
     const float rinv = 1.0f / sqrtf(sums_of_8<NW>(s, part) / (float)E + eps);
 #pragma unroll
     for (int m = 0; m < 8; ++m) s[m] = of_lane(rinv, m);        // (here, where all lanes are: below, rinv would be made in those that go on)
-    float* const srow = state + (size_t)blk.slot * (taps - 1) * E;
+    float* const srow = state + (size_t)blk.slot * (TAPS - 1) * E;
     if (c >= E) return;
 #pragma unroll
     for (int m = 0; m < LNC_HELD; ++m) h[m] = make_float4(h[m].x * s[m] * gw.x, h[m].y * s[m] * gw.y, h[m].z * s[m] * gw.z, h[m].w * s[m] * gw.w);
     if (k == 0) {
-        // (rows -3 to -1 are carried inputs taps - 4 to taps - 2, if there are so many; new input m of 3 is row n - 3 + m, or an old one)
+        // (rows -3 to -1 are carried inputs TAPS - 4 to TAPS - 2, if there are so many; new input m of 3 is row n - 3 + m, or an old one)
         float4 old[3], last[3];
 #pragma unroll
         for (int m = 0; m < 3; ++m)
-            old[m] = m + taps >= 4 ? *reinterpret_cast<const float4*>(srow + (size_t)(m + taps - 4) * E + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            old[m] = m + TAPS >= 4 ? *reinterpret_cast<const float4*>(srow + (size_t)(m + TAPS - 4) * E + c) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int m = 0; m < 3; ++m) last[m] = pick(n >= 3 - m, h[m], pick(m + n == 1, old[1], old[2]));      // (n < 3 - m, n >= 1: m + n is 1 or 2)
 #pragma unroll
         for (int m = 0; m < 3; ++m) h[m] = old[m];
 #pragma unroll
         for (int m = 0; m < 3; ++m)
-            if (m + taps >= 4) *reinterpret_cast<float4*>(srow + (size_t)(m + taps - 4) * E + c) = last[m];
+            if (m + TAPS >= 4) *reinterpret_cast<float4*>(srow + (size_t)(m + TAPS - 4) * E + c) = last[m];
     }
 #pragma unroll
     for (int r = 0; r < LNC_ROWS; ++r) {
@@ -730,7 +739,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_layernorm_conv_rows(TO* __restri
             float acc = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (j + taps >= 4) acc = fmaf(wt[d][j], at(r + j), acc);
+                if (j + TAPS >= 4) acc = fmaf(wt[d][j], at(r + j), acc);
             y[d] = acc + at(r + 3);
         }
         if (i0 + r < n) st4(out + (size_t)(row0 + i0 + r) * E + c, make_float4(y[0], y[1], y[2], y[3]));
@@ -746,7 +755,7 @@ extern "C" int xr_layernorm_conv_rows(void* out, const float* x, const float* w,
     XR_REQUIRE(out_dtype == XR_F32 || out_dtype == XR_BF16, "layernorm_conv: bad dtype %d", out_dtype);
     if (T == 0 || B == 0) return XR_OK;
     const unsigned blocks = (unsigned)(((long long)T + (long long)B * (LNC_ROWS - 1)) / LNC_ROWS + 7) / 8 * 8;
-#define LNC(TO, NW) k_layernorm_conv_rows<TO, NW><<<blocks, 64 * NW, 0, stream>>>((TO*)out, x, w, cw, state, cu_q, slots, B, E, ldx, taps, eps)
+#define LNC(TO, NW) (taps == 4 ? k_layernorm_conv_rows<TO, NW, 4> : taps == 3 ? k_layernorm_conv_rows<TO, NW, 3> : k_layernorm_conv_rows<TO, NW, 2>)<<<blocks, 64 * NW, 0, stream>>>((TO*)out, x, w, cw, state, cu_q, slots, B, E, ldx, eps)
 #define LNCS(TO) do { if (E <= 2048) LNC(TO, 8); else LNC(TO, 16); } while (0)
     if (out_dtype == XR_F32) LNCS(float);
     else LNCS(bf16_t);
