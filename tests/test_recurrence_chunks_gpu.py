@@ -151,3 +151,37 @@ def test_which_steps_read_rows_again():
     again = lambda kind, D, *q_lens: ops.recurrence_reads_rows_again(kind, step_ctx([0] * len(q_lens), list(q_lens), list(range(len(q_lens)))), 32, D, 128)
     assert again("retention", 128, 1, 200, 1) and again("retention", 128, 1023) and again("retention", 256, 1024)
     assert not again("retention", 128, 95) and not again("retention", 128, *[100] * 20) and not again("retention", 256, 1023)
+
+
+@pytest.mark.parametrize("kind,G,D", [("retention", 24, 48), ("retention", 24, 64), ("retention", 24, 80), ("delta", 12, 48)])
+@pytest.mark.parametrize("activation", [None, "silu"])
+def test_more_workgroups_than_compute_units(monkeypatch, kind, G, D, activation):
+    """Small heads of several portions at once, 288 workgroups, whose operands go through LDS; the last step's 144 and the 72 of a portion go straight to registers.
+    A decay below zero, and then an infinity in a value: those columns come out as token by token."""
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, H, Dv = load_ops(), 24, 48
+    rng = np.random.default_rng(D + G)
+    lens = [sum(n for _, n in p) for p in PORTIONS]
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    qs, ks = ([f32(S.unit(rng.normal(size=(n, G, D)))) for n in lens] for _ in range(2))
+    vs = [f32(rng.normal(size=(n, H, Dv))) for n in lens]
+    if kind == "delta":
+        if activation:
+            pytest.skip("the delta rule's activation is its convolution's")
+        extra = ([f32(S.sigmoid(rng.normal(size=(n, H)))) for n in lens], [f32(np.exp(-rng.exponential(0.1, size=(n, H)))) for n in lens])
+        want = [S.gated_delta_rule(np.repeat(q, 2, 1), np.repeat(k, 2, 1), v, b, g) for q, k, v, b, g in zip(qs, ks, vs, *extra)]
+    else:
+        extra = f32(np.resize([0.97, 1.0, 0.0, 0.5, -0.5], H))
+        act = S.silu if activation else (lambda x: x)
+        want = [S.retention(act(q), act(k) * 0.25, act(v), extra) for q, k, v in zip(qs, ks, vs)]
+    kw = dict(activation=activation, k_scale=0.25) if kind == "retention" else {}
+    chunks, plain = both(ops, monkeypatch, kind, qs, ks, vs, extra, H, G, D, Dv, PORTIONS, [2, 0, 4, 1], 5, **kw)
+    # as above: 2^-24 of each of some 330 updates of a state
+    assert error(chunks, want) < 5e-6, (error(chunks, want), error(plain, want))
+    assert error(chunks, want) < 2 * error(plain, want) + 2e-7, (error(chunks, want), error(plain, want))
+    vs[0][30, 3, 5] = np.inf
+    broken, plain = both(ops, monkeypatch, kind, qs, ks, vs, extra, H, G, D, Dv, PORTIONS, [2, 0, 4, 1], 5, **kw)
+    for b, p, c in zip(broken, plain, chunks):
+        assert np.array_equal(np.isfinite(b), np.isfinite(p))
+    assert np.array_equal(broken[0][:30], chunks[0][:30]) or error([broken[0][:30]], [chunks[0][:30]]) < 1e-6
+    assert not np.isfinite(broken[0][30:, 3, 5]).any() and np.isfinite(broken[1]).all()

@@ -488,10 +488,204 @@ __global__ __launch_bounds__(512) void k_chunk_run(ChunkArgs a) {
         for (int j = 0; j < J; ++j) st[((size_t)j * a.Dv + c) * 16 + r] = s[j];
 }
 
+#define RC_UNITS 256            // compute units
+template <int D, bool DELTA> constexpr bool RC_STAGED = D <= (DELTA ? 48 : 80);
+// The same with four waves a workgroup, which stage a chunk's operands in LDS and each do all of 16 rows: for small heads and more workgroups than compute
+// units.  Two of these run on a unit, whose products then wait for each other's trips to LDS; k_chunk_run has the registers for one of its own, and fetches K's columns number by
+// number: a shorter chain and more loads.  (It without fetching ahead, two a unit: no faster.)  Both, k_chunk_run and these, us with k_chunk_mats: retention, 8 portions of 1,024 rows,
+// 32 heads of 64 x 64 (1,024 workgroups) 200 and 165, 16 of 80 x 64 (512) 122 and 106, 4 of 512 rows, 16 heads of 48 x 96 (384) 48 and 38; the delta rule, of 48 x 96
+// 61.5 and 57.  Heads of 96 and more have no room for two; one workgroup a unit and fewer go faster with k_chunk_run (one portion of 2,048 rows, 32 heads of 64: 81, staged 107).
+template <int D, bool DELTA, bool ACT>
+__global__ __launch_bounds__(256) void k_chunk_run_staged(ChunkArgs a) {
+    constexpr int LD = D + 4, J = D / 16, NQ = RC_L * D / 1024, NM = RC_L * RC_L / 1024, MATS = DELTA ? 2 : 1;
+    extern __shared__ __align__(16) float lds[];
+    float* Q = lds;                                     // [64][LD]
+    float* K = Q + RC_L * LD;
+    float* P = K + RC_L * LD;                           // [64][RC_LDM]
+    float* T = P + RC_L * RC_LDM;                       // (delta) [64][RC_LDM]
+    __shared__ __align__(16) float S[J][RC_C][20];      // the state's columns, 16 rows side by side
+    __shared__ __align__(16) float U[RC_C][RC_LDM], W[RC_C][RC_LDM];     // by column: u_i; (delta) the right side; u_i exp(L_63 - L_i)
+    __shared__ float V[RC_L][RC_C + 1];
+    __shared__ float vec[RC_VEC];
+    __shared__ int odd;                                 // something came out that is not finite
+    // Workgroup i runs on XCD i % 8: the column workgroups of a head, which read the same rows and matrices, go to one XCD
+    // (where the heads come in eights), so that its L2 serves all but the first of them.
+    const int shares = a.Dv / RC_C, id = blockIdx.x, b = a.reqs[2 * blockIdx.y];
+    const bool eights = a.H % 8 == 0;
+    const int h = eights ? (id >> 3) / shares * 8 + (id & 7) : id / shares, c0 = (eights ? (id >> 3) % shares : id % shares) * RC_C;
+    const int row_b = a.cu_q[b], n = a.cu_q[b + 1] - row_b;
+    if (n <= 0) return;
+    const int kvh = h / (a.H / a.G);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
+    const int place0 = a.reqs[2 * blockIdx.y + 1];
+    float* st = a.state + (((size_t)a.slots[b] * a.H + h) * J * a.Dv + c0) * 16;
+    for (int i = tid; i < J * RC_C * 4; i += 256) {
+        const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
+        rc_st4(&S[j][c][r], rc_ld4(st + ((size_t)j * a.Dv + c) * 16 + r));
+    }
+    // a chunk's operands come into registers while the chunk before it is worked on
+    float4 rq[NQ], rk[NQ], rm[MATS * NM], rv;
+    float rvec = 0.f;
+    auto fetch = [&](int chunk) {
+        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
+        const size_t place = (size_t)(place0 + chunk) * a.H + h;
+#pragma unroll
+        for (int e = 0; e < NQ; ++e) {
+            const int i = tid + e * 256, r = i / (D / 4), c = i % (D / 4) * 4;
+            const size_t at = (size_t)(row0 + (r < rows ? r : 0)) * a.ld + (size_t)kvh * D + c;
+            rq[e] = rc_ld4(a.q + at);
+            rk[e] = rc_ld4(a.k + at);
+            if (r >= rows) rq[e] = rk[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const float* mats = a.mats + place * MATS * RC_L * RC_L;
+#pragma unroll
+        for (int e = 0; e < MATS * NM; ++e) {
+            const int i = tid + e * 256, r = i / (RC_L / 4) % RC_L, c = i % (RC_L / 4) * 4;
+            rm[e] = c / 16 <= r / 16 ? rc_ld4(mats + (size_t)i * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const int r = tid / 4, c = tid % 4 * 4;
+        rv = rc_ld4(a.v + (size_t)(row0 + (r < rows ? r : 0)) * a.ld + (size_t)h * a.Dv + c0 + c);
+        if (r >= rows) rv = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (tid < RC_VEC) rvec = a.vecs[place * RC_VEC + tid];
+    };
+    auto stage = [&]() {                                // the fetched chunk to LDS
+#pragma unroll
+        for (int e = 0; e < NQ; ++e) {
+            const int i = tid + e * 256, r = i / (D / 4), c = i % (D / 4) * 4;
+            rc_st4(Q + r * LD + c, rc_act4<ACT>(rq[e], a.q_scale));
+            rc_st4(K + r * LD + c, rc_act4<ACT>(rk[e], a.k_scale));
+        }
+#pragma unroll
+        for (int e = 0; e < MATS * NM; ++e) {
+            const int i = tid + e * 256, r = i / (RC_L / 4), c = i % (RC_L / 4) * 4;
+            rc_st4(P + r * RC_LDM + c, rm[e]);          // (T lies behind P)
+        }
+        {
+            const int r = tid / 4, c = tid % 4 * 4;
+            const float4 x = rc_act4<ACT>(rv, 1.f);
+            V[r][c] = x.x; V[r][c + 1] = x.y; V[r][c + 2] = x.z; V[r][c + 3] = x.w;
+        }
+        if (tid < RC_VEC) vec[tid] = rvec;
+    };
+    auto rows_times_state = [&](const float* rows, const float* state) {
+        float4 x[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) x[j] = rc_ld4(rows + (16 * wave + l16) * LD + 4 * quad + 16 * j);
+        return times_state<J>(x, state);
+    };
+    if (tid == 0) odd = 0;
+    float none = 0.f;                                   // 0, or no number once a read-out was not finite
+    fetch(0);
+    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
+        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L;
+        __syncthreads();                                // the chunk before has been read, the state is written
+        stage();
+        __syncthreads();
+        if ((chunk + 1) * RC_L < n) fetch(chunk + 1);
+        const int i0 = 16 * wave + 4 * quad;            // this lane's rows of a product whose rows are the chunk's
+        rc_f32x4 u;
+        if (DELTA) {
+            const rc_f32x4 x = rows_times_state(K, &S[0][l16][4 * quad]);       // K S0
+            float r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = vec[2 * RC_L + i0 + e] * (V[i0 + e][l16] - vec[i0 + e] * x[e]);
+            rc_st4(&W[l16][i0], make_float4(r[0], r[1], r[2], r[3]));
+            __syncthreads();
+            u = rc_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m <= wave; ++m) u = rc_mfma4(rc_ld4(T + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&W[l16][16 * m + 4 * quad]), u);
+            __syncthreads();                            // W is read, and written again below
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] = V[i0 + e][l16];
+        }
+        rc_st4(&U[l16][i0], make_float4(u[0], u[1], u[2], u[3]));
+        rc_st4(&W[l16][i0], make_float4(u[0] * vec[RC_L + i0], u[1] * vec[RC_L + i0 + 1], u[2] * vec[RC_L + i0 + 2], u[3] * vec[RC_L + i0 + 3]));
+        rc_f32x4 o = rows_times_state(Q, &S[0][l16][4 * quad]);         // Q S0
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] *= vec[i0 + e];
+        __syncthreads();                                // U and W are there, and the state of the chunk's start is read
+        rc_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int m = 0; m < RC_L / 16; ++m)
+            if (m <= wave) p[m & 1] = rc_mfma4(rc_ld4(P + (16 * wave + l16) * RC_LDM + 16 * m + 4 * quad), rc_ld4(&U[l16][16 * m + 4 * quad]), p[m & 1]);
+        o += p[0] + p[1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i0 + e < rows) a.out[((size_t)(row0 + i0 + e) * a.H + h) * a.Dv + c0 + l16] = o[e];
+        none += 0.f * o[0] + 0.f * o[1] + 0.f * o[2] + 0.f * o[3];
+        const float all = vec[RC_L - 1];                // exp(L_63)
+        for (int j = wave; j < J; j += 4) {             // 16 rows of the state: its own decayed, and K^T W
+            const float4 s0 = rc_ld4(&S[j][l16][4 * quad]);
+            rc_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int m = 0; m < RC_L / 16; ++m) {
+                const float* kp = K + (16 * m + 4 * quad) * LD + 16 * j + l16;
+                s[m & 1] = rc_mfma4(make_float4(kp[0], kp[LD], kp[2 * LD], kp[3 * LD]), rc_ld4(&W[l16][16 * m + 4 * quad]), s[m & 1]);
+            }
+            const rc_f32x4 t = s[0] + s[1];
+            rc_st4(&S[j][l16][4 * quad], make_float4(fmaf(s0.x, all, t[0]), fmaf(s0.y, all, t[1]), fmaf(s0.z, all, t[2]), fmaf(s0.w, all, t[3])));
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < J * RC_C * 4; i += 256) {
+        const float4 x = rc_ld4(&S[i / (RC_C * 4)][i / 4 % RC_C][i % 4 * 4]);
+        none += 0.f * x.x + 0.f * x.y + 0.f * x.z + 0.f * x.w;
+    }
+    if (none != none) odd = 1;
+    __syncthreads();
+    if (!odd) {
+        for (int i = tid; i < J * RC_C * 4; i += 256) {
+            const int j = i / (RC_C * 4), c = i / 4 % RC_C, r = i % 4 * 4;
+            rc_st4(st + ((size_t)j * a.Dv + c) * 16 + r, rc_ld4(&S[j][c][r]));
+        }
+        return;
+    }
+    // Not finite somewhere (a state that once is stays so): the portion again from its first state, token by token.  0 times an
+    // infinity or a NaN is no 0, so that above it shows in rows before its own, too; and a negative decay has no logarithm.
+    const int c = tid >> 4, r = tid & 15;               // 16 lanes a column, rows r, r + 16, ..
+    float s[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) s[j] = st[((size_t)j * a.Dv + c) * 16 + r];
+    for (int chunk = 0; chunk * RC_L < n; ++chunk) {
+        const int row0 = row_b + chunk * RC_L, rows = n - chunk * RC_L < RC_L ? n - chunk * RC_L : RC_L;
+        fetch(chunk);
+        __syncthreads();
+        stage();
+        __syncthreads();
+        for (int i = 0; i < rows; ++i) {
+            const float g = DELTA ? a.gate[(size_t)(row0 + i) * a.ld_g + h] : a.decay[h];
+            const float* k = K + i * LD + r;
+            const float* q = Q + i * LD + r;
+            float u = V[i][c], o = 0.f;
+            if (DELTA) {
+                float d = 0.f;
+#pragma unroll
+                for (int j = 0; j < J; ++j) d = fmaf(s[j], k[16 * j], d);
+#pragma unroll
+                for (int m = 8; m > 0; m >>= 1) d += __shfl_xor(d, m, 64);
+                u = vec[2 * RC_L + i] * (u - g * d);
+            }
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                s[j] = fmaf(g, s[j], k[16 * j] * u);
+                o = fmaf(s[j], q[16 * j], o);
+            }
+#pragma unroll
+            for (int m = 8; m > 0; m >>= 1) o += __shfl_xor(o, m, 64);
+            if (r == 0) a.out[((size_t)(row0 + i) * a.H + h) * a.Dv + c0 + c] = o;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) st[((size_t)j * a.Dv + c) * 16 + r] = s[j];
+}
+
 template <int D, bool DELTA, bool ACT>
 static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t stream) {
-    const int one = 2 * RC_L * (D + 4) * 4, mats = one + (DELTA ? 2 : 0) * RC_L * RC_LDM * 4, run = one + RC_L * (RC_C + 1) * 4;
-    const void* kernels[2] = {(const void*)k_chunk_mats<D, DELTA, ACT>, (const void*)k_chunk_run<D, DELTA, ACT>};
+    const int one = 2 * RC_L * (D + 4) * 4, mats = one + (DELTA ? 2 : 0) * RC_L * RC_LDM * 4, columns = a.Dv / RC_C * a.H;
+    const bool staged = RC_STAGED<D, DELTA> && (long long)columns * B > RC_UNITS;
+    const int run = one + (staged ? (DELTA ? 2 : 1) * RC_L * RC_LDM : RC_L * (RC_C + 1)) * 4;
+    const auto k_run = staged ? k_chunk_run_staged<RC_STAGED<D, DELTA> ? D : 48, DELTA, ACT> : k_chunk_run<D, DELTA, ACT>;
+    const void* kernels[2] = {(const void*)k_chunk_mats<D, DELTA, ACT>, (const void*)k_run};
     const int bytes[2] = {mats, run};
     for (int i = 0; i < 2; ++i)
         if (bytes[i] > 65536) {
@@ -501,7 +695,7 @@ static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t strea
         }
     k_chunk_mats<D, DELTA, ACT><<<dim3((max_q + RC_L - 1) / RC_L, a.H, B), 256, mats, stream>>>(a);
     XR_CHECK_LAUNCH("chunk_mats");
-    k_chunk_run<D, DELTA, ACT><<<dim3(a.Dv / RC_C * a.H, B), 512, run, stream>>>(a);
+    k_run<<<dim3(columns, B), staged ? 256 : 512, run, stream>>>(a);
     XR_CHECK_LAUNCH("chunk_run");
     return XR_OK;
 }
