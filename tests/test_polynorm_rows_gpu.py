@@ -28,3 +28,17 @@ def test_polynorm_rows(F, T):
     half = t.bfloat16()
     again = S.polynorm(half.double().cpu().numpy(), coef.double().cpu().numpy(), 1e-5)
     assert np.abs(ops.polynorm(half, coef, 1e-5, torch.bfloat16).double().cpu().numpy() - again).max() < np.abs(again).max() * 2.0 ** -8
+
+
+@pytest.mark.parametrize("F", [8192, 8196, 16388, 24580, 32768])
+def test_rows_on_either_side_of_one_a_compute_unit(F):
+    """More than 256 long rows make their powers again: the same numbers, to a rounding of a term."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops, dev = load_ops(), torch.device("cuda:0")
+    z = torch.randn((257, F), device=dev) * 2
+    coef = torch.tensor([0.7, -1.3, 0.45, 0.2], device=dev)
+    few, many = ops.polynorm(z[:256], coef, 1e-5, torch.float32), ops.polynorm(z, coef, 1e-5, torch.float32)
+    want = torch.tensor(S.polynorm(z.double().cpu().numpy(), coef.double().cpu().numpy(), 1e-5), device=dev)
+    bound = 2e-6 * float(want.abs().max())          # (as above)
+    assert float((many.double() - want).abs().max()) < bound and float((few.double() - want[:256]).abs().max()) < bound
