@@ -182,3 +182,29 @@ def test_few_rows_kernel_with(what, shape, room, monkeypatch):
         assert len(ctx._plans) == 1 and int(plan.counters.abs().sum()) == 0 and np.isfinite(got).all()
         # probabilities and the result in bfloat16 (2^-9 each of a value) against the largest output, as above
         assert np.abs(got - want).max() < 1.2e-2 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("B,n,heads", [(32, 17, 8), (32, 32, 8), (64, 33, 2), (1, 1, 8), (16, 9, 32), (4, 3, 1)])
+def test_padded_rows_leave_the_requests_their_ranges(B, n, heads):
+    """A recorded batch's list: the rows that pad it have an item each, the requests as many ranges together as fill the kernel's workgroups."""
+    from xyntetik_runner_amd.engine.batch import FEW_INTS, FEW_SLOTS
+    from xyntetik_runner_amd.engine.graphs import StaticDecodeContext, few_row_room
+    room = few_row_room(B, 125, heads)
+    ctx = object.__new__(StaticDecodeContext)
+    key = (4, None, heads, False, 2)
+    ctx.B, ctx._plan_splits = B, {key: room}
+    starts = np.zeros(B, dtype=np.int32)
+    starts[:n] = 3999 - np.arange(n) * 10
+    h = np.full(room * FEW_INTS + B * heads, -7, dtype=np.int32)
+    ctx._fill_plan(h, 0, key, starts, n)
+    items = h[:room * FEW_INTS].reshape(room, FEW_INTS)
+    live = items[items[:, 3] > items[:, 2]]
+    assert not h[room * FEW_INTS:].any() and (items[len(live):, 2:4] == 0).all()
+    ranges = [int((live[:, 0] == b).sum()) for b in range(B)]
+    assert ranges[n:] == [1] * (B - n) and n <= sum(ranges[:n]) <= max(n, FEW_SLOTS // heads)
+    if n < FEW_SLOTS // heads:
+        assert sum(ranges[:n]) > n          # (not all of them whole)
+    assert (live[:, 4] < room).all() and len(set(live[live[:, 4] >= 0, 4].tolist())) == int((live[:, 4] >= 0).sum())
+    for b in range(n):
+        mine = live[live[:, 0] == b]
+        assert mine[:, 2].min() == 0 and mine[:, 3].max() == starts[b] + 1 and (mine[:, 11] == len(mine)).all()

@@ -54,10 +54,10 @@ def splits_for(batch_cap: int, max_tiles: int, n_kv_heads: int) -> int:
     return best
 
 
-def few_row_splits(batch_cap: int, tiles: int, n_kv_heads: int) -> int:
-    """Key ranges a request that the kernel for few rows has room for: as many as fill its workgroups, and no more than ranges of
-    the shortest length (and one for what the requests' last ranges lack)."""
-    return max(1, min(FEW_SLOTS // (batch_cap * n_kv_heads), -(-tiles // FEW_MIN_RANGE) + 1))
+def few_row_room(batch_cap: int, tiles: int, n_kv_heads: int) -> int:
+    """Items that a recorded step keeps for the kernel for few rows: one a request, and as many key ranges as fill the kernel's workgroups beside the
+    rows that pad the batch (fewer than half of it, an item each), but no more than ranges of the shortest length (and one for what the requests' last ranges lack)."""
+    return max(batch_cap, min(FEW_SLOTS // n_kv_heads + batch_cap // 2, batch_cap * (-(-tiles // FEW_MIN_RANGE) + 1)))
 
 
 class StaticDecodeContext:
@@ -91,7 +91,7 @@ class StaticDecodeContext:
         self._plan_keys: List[Tuple[int, Optional[int], int, bool, int]] = []
         self._plans: Dict[tuple, AttentionPlan] = {}
         self._plan_off: Dict[tuple, int] = {}
-        self._plan_splits: Dict[tuple, int] = {}
+        self._plan_splits: Dict[tuple, int] = {}       # key ranges a request; the kernel for few rows: items of all together
         self._alloc()
         self.fresh_slots_host: List[int] = []
         self._copied = None
@@ -99,7 +99,7 @@ class StaticDecodeContext:
 
     def _alloc(self) -> None:
         B = self.B
-        n_plan = sum((B * self._plan_splits[k] * FEW_INTS + B * k[2] if k[4] else B * self._plan_splits[k] * 8 + B * 7) + (B * 8 if k[3] else 0)
+        n_plan = sum((self._plan_splits[k] * FEW_INTS + B * k[2] if k[4] else B * self._plan_splits[k] * 8 + B * 7) + (B * 8 if k[3] else 0)
                      for k in self._plan_keys)
         offs = np.concatenate([[0], np.cumsum(self._sizes)]).astype(np.int64)
         total = int(offs[-1]) + n_plan
@@ -122,11 +122,11 @@ class StaticDecodeContext:
             S = self._plan_splits[k]
             self._plan_off[k] = base
             if k[4]:
-                n_items, n_count, n_extra = B * S * FEW_INTS, B * k[2], B * 8 if k[3] else 0
+                n_items, n_count, n_extra = S * FEW_INTS, B * k[2], B * 8 if k[3] else 0
                 few, counters = d[base:base + n_items], d[base + n_items:base + n_items + n_count]
                 extras = d[base + n_items + n_count:base + n_items + n_count + n_extra] if n_extra else None
-                self._plans[k] = AttentionPlan(few[:0], 0, None, 0, B * S + (B if n_extra else 0) if S > 1 or n_extra else 0, 0,
-                                               extras, B if n_extra else 0, few, B * S, counters)
+                self._plans[k] = AttentionPlan(few[:0], 0, None, 0, S + (B if n_extra else 0) if S > B or n_extra else 0, 0,
+                                               extras, B if n_extra else 0, few, S, counters)
                 base += n_items + n_count + n_extra
                 continue
             items = d[base:base + B * S * 8]
@@ -159,7 +159,7 @@ class StaticDecodeContext:
             if tiles is not None and window:
                 tiles = min(tiles, -(-mask_reach(window) // ATTN_TILE) + 1)
             if few:
-                self._plan_splits[key] = few_row_splits(self.B, tiles if tiles is not None else self.S * FEW_MIN_RANGE, n_kv_heads)
+                self._plan_splits[key] = few_row_room(self.B, tiles if tiles is not None else self.S * FEW_MIN_RANGE, n_kv_heads)
             else:
                 self._plan_splits[key] = self.S if tiles is None else min(self.S, splits_for(self.B, tiles, n_kv_heads))
             self._plan_keys.append(key)
@@ -220,7 +220,7 @@ class StaticDecodeContext:
         self.seq_lens = [s + 1 for s in self.starts]
         self.max_seq_len = max(self.seq_lens)
         for key in self._plan_keys:
-            self._fill_plan(h, self._plan_off[key], key, starts)
+            self._fill_plan(h, self._plan_off[key], key, starts, n)
         self._dev.copy_(self._host, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
@@ -228,16 +228,17 @@ class StaticDecodeContext:
         if token_source is not None:
             self.token_ids[:n].copy_(token_source)
 
-    def _fill_plan(self, h, base: int, key, starts) -> None:
+    def _fill_plan(self, h, base: int, key, starts, n: int) -> None:
         group_size, window, n_kv_heads, extra, few = key
         B, S = self.B, self._plan_splits[key]
         if few:
-            got, extras, _ = few_row_items(np.arange(B), starts, np.ones(B, dtype=np.int64), np.arange(B), window, B * S, extra,
+            # (rows that pad the batch have an item each, and leave the requests all the workgroups)
+            got, extras, _ = few_row_items(np.arange(B), starts, np.ones(B, dtype=np.int64), np.arange(B), window, min(S, max(B, FEW_SLOTS // n_kv_heads + B - n)), extra,
                                            pair_at=ATTN_STREAM_SLOTS // n_kv_heads if few == 2 else 0)
-            items = h[base:base + B * S * FEW_INTS].reshape(B * S, FEW_INTS)
+            items = h[base:base + S * FEW_INTS].reshape(S, FEW_INTS)
             items[:len(got)] = got
             items[len(got):, 2:4] = 0              # (no keys: nothing to do)
-            after = base + B * S * FEW_INTS
+            after = base + S * FEW_INTS
             h[after:after + B * n_kv_heads] = 0
             if extra:
                 h[after + B * n_kv_heads:after + B * n_kv_heads + B * 8] = extras.ravel()
