@@ -172,7 +172,7 @@ def test_few_rows_kernel_with(what, shape, room, monkeypatch):
                 want[r, h] = o * (1 / (1 + np.exp(-gate[r, h])) if opt["gate"] else 1.0) * opt["scale_out"]
             r += 1
     q = torch.cat(qs).reshape(T, H * D).contiguous().to(DEV)
-    more = {**({"extra_slot": True} if keep else {}), "few_rows": 2 if 2 * D <= 256 else 1}
+    more = {**({"extra_slot": True} if keep else {}), "few_rows": 2 if 2 * D <= 256 else 1, "few_channels": 2 * D}
     plan = ctx.attention_plan(0, H // Hk, mask, Hk, ps, **more)
     assert plan.n_few >= len(starts) and plan.n_items == plan.n_cta_items == plan.n_jobs == 0
     for _ in range(2):
@@ -184,6 +184,15 @@ def test_few_rows_kernel_with(what, shape, room, monkeypatch):
         assert np.abs(got - want).max() < 1.2e-2 * np.abs(want).max()
 
 
+# (tiles, rows, channels of a key and a value): whole, ranges of 4 tiles and more, 16 ranges, 32
+@pytest.mark.parametrize("args,least", [((10, 4, 256), 10), ((11, 4, 256), 4), ((16, 16, 256), 16), ((17, 16, 256), 4), ((8, 1, 256), 8), ((9, 1, 256), 4),
+                                        ((15, 4, 128), 15), ((16, 4, 128), 4), ((125, 4, 256), 8), ((199, 4, 256), 13), ((200, 4, 256), 7), ((399, 16, 256), 25),
+                                        ((400, 16, 256), 13), ((250, 4, 128), 16), ((1, 1, 512), 1)])
+def test_shortest_ranges(args, least):
+    from xyntetik_runner_amd.engine.batch import few_row_least
+    assert few_row_least(*args) == least
+
+
 @pytest.mark.parametrize("B,n,heads", [(32, 17, 8), (32, 32, 8), (64, 33, 2), (1, 1, 8), (16, 9, 32), (4, 3, 1)])
 def test_padded_rows_leave_the_requests_their_ranges(B, n, heads):
     """A recorded batch's list: the rows that pad it have an item each, the requests as many ranges together as fill the kernel's workgroups."""
@@ -191,7 +200,7 @@ def test_padded_rows_leave_the_requests_their_ranges(B, n, heads):
     from xyntetik_runner_amd.engine.graphs import StaticDecodeContext, few_row_room
     room = few_row_room(B, 125, heads)
     ctx = object.__new__(StaticDecodeContext)
-    key = (4, None, heads, False, 2)
+    key = (4, None, heads, False, 2, 256)
     ctx.B, ctx._plan_splits = B, {key: room}
     starts = np.zeros(B, dtype=np.int32)
     starts[:n] = 3999 - np.arange(n) * 10

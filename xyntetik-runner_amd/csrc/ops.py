@@ -959,7 +959,7 @@ class Ops:
         products of 32 channels, a larger score is a larger product (a positive scale) and 16-byte loads are aligned."""
         few = (getattr(ctx, "plans_few_rows", False) and D % 32 == 0 and scale > 0.0
                and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) & 15)
-        more = {**({"extra_slot": True} if extra else {}), **({"few_rows": 2 if D + Dv <= 256 else 1} if few else {})}
+        more = {**({"extra_slot": True} if extra else {}), **({"few_rows": 2 if D + Dv <= 256 else 1, "few_channels": D + Dv} if few else {})}
         return ctx.attention_plan(group, H // Hk, mask, Hk, page_size, **more)
 
     def attention_on_matrix_cores(self, dtype: torch.dtype, D: int, Dv: int, page_size: int = 64) -> bool:

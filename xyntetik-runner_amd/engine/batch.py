@@ -13,6 +13,7 @@ src/cuda.c:4213-4236); an entry list covers both and their mixtures.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass, field
 from typing import Hashable, List, Optional, Sequence
 
@@ -205,14 +206,30 @@ def plan_attention(starts, q_lens, group_size: int, window, n_kv_heads: int,
     return cta_items, items, jobs, slot
 
 
-def few_row_items(req, starts, lens, q0s, mask, room: int, extra_slot: bool, first_slot: int = 0, pair_at: int = 0):
+def few_row_least(tiles: int, rows: int, channels: int = 256) -> int:
+    """Tiles of the shortest key range that pays where the longest request of a step has ``tiles`` tiles, ``rows`` rows a key/value head and ``channels`` of a
+    key and its value together.
+
+    The last workgroup of a row block adds the ranges up, 16 of them in a round of trips to memory, more rows in more rounds: some 3 us for 4 rows of 128 channels, 7 for 16,
+    in which a workgroup goes through 5 and 13 tiles of 256 channels (0.55 us each), through more of fewer.  A recorded layer of small products, whole and cut from 4 tiles
+    on: 8 tiles of 8 x 4 heads of 128 24.1 us and 25.9, of 1 x 16 23.6 and 29.4; 13 tiles 26.8 and 24.9, 26.0 and 28.9; of 64 22.5 and 22.6, 22.5 and 24.8; of 32 20.3 and 23.4.
+    Ranges beyond 16 begin a second round, which pays where each would be long: 125 tiles in 16 and in 31, 8 x 4 heads of 128 28.8 and 30.4, 1 x 16 31.2 and 35.1; 250 in 16, 32 and (1 x 16) 63 34.0
+    and 31.8, 35.5, 37.2 and 45; of 64 27.7 and 29.1, 28.0, 29.7 and 35.5."""
+    if tiles < (9 + rows // 2) * math.sqrt(256 / channels):
+        return tiles
+    most = 16 if tiles * channels < (51200 if rows <= 8 else 102400) else 32
+    return max(FEW_MIN_RANGE, -(-tiles // most))
+
+
+def few_row_items(req, starts, lens, q0s, mask, room: int, extra_slot: bool, first_slot: int = 0, pair_at: int = 0, least=None):
     """The work of the kernel for few rows: requests ``req`` of a step, each with one row block (its ``lens[i]`` tokens from row
     ``q0s[i]`` and position ``starts[i]`` on), cut into at most ``room`` key ranges of about one length, so that a
     long request takes as many workgroups as its keys are worth: ``(items [n, 12], extras [len(req), 8], slots)`` as int64 arrays.
 
     An item: request, 0, first key, end key, partial slot (-1: all its keys), the request's first row, its tokens, its first
     position, the row block's first slot, its slots, its counter and how many items it has.  With ``extra_slot`` a row block has
-    one slot more, its last, for a partial result of another kernel (``extras`` as ``plan_attention`` makes them).
+    one slot more, its last, for a partial result of another kernel (``extras`` as ``plan_attention`` makes them).  ``least``: the tiles of the
+    shortest range, from those of the longest request.
 
     The requests with the longest ranges come first, workgroups start in the items' order.  ``pair_at``: the items that give every compute unit one workgroup, where
     it holds two at a time: if there are up to twice as many, all run at once, and the second half comes shortest first, so that
@@ -231,8 +248,9 @@ def few_row_items(req, starts, lens, q0s, mask, room: int, extra_slot: bool, fir
     longest = max(t)
     if room > n:
         total = sum(t)
-        most = max(FEW_MIN_RANGE, -(-total // (room - n)))
-        for c in range(max(FEW_MIN_RANGE, -(-total // room)), most, max(1, most // 32)):
+        least = FEW_MIN_RANGE if least is None else max(1, least(longest))
+        most = max(least, -(-total // (room - n)))
+        for c in range(max(least, -(-total // room)), most, max(1, most // 32)):
             if sum([-(-x // c) for x in t]) <= room:
                 most = c
                 break
@@ -352,11 +370,11 @@ class StepContext:
         self.shared = {}        # what parts make once a step and share between layers (a rotation's table)
 
     def attention_plan(self, group: int, group_size: int, window, n_kv_heads: int,
-                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0) -> AttentionPlan:
+                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0, few_channels: int = 256) -> AttentionPlan:
         """The MFMA attention work list, made once per step and shared by all layers that can.  ``few_rows`` > 0:
         requests of up to 16 rows a key/value head go to the kernel for few rows (where the page size allows), of which a compute unit
-        holds so many workgroups."""
-        key = (group_size, window, n_kv_heads, page_size, extra_slot, few_rows)
+        holds so many workgroups; ``few_channels``: those of a key and its value together."""
+        key = (group_size, window, n_kv_heads, page_size, extra_slot, few_rows, few_channels)
         plan = self._plans.get(key)
         if plan is None:
             few = [b for b, n in enumerate(self.q_lens) if few_rows and page_size >= FEW_PAGE and n * group_size <= FEW_ROWS]
@@ -370,7 +388,8 @@ class StepContext:
                 q0s = np.concatenate([[0], np.cumsum(self.q_lens)])[few]
                 room = max(len(few), FEW_SLOTS // n_kv_heads)
                 few_items, few_extras, more = few_row_items(few, [self.starts[b] for b in few], [self.q_lens[b] for b in few], q0s,
-                                                            window, room, extra_slot, n_slots, ATTN_STREAM_SLOTS // n_kv_heads if few_rows == 2 else 0)
+                                                            window, room, extra_slot, n_slots, ATTN_STREAM_SLOTS // n_kv_heads if few_rows == 2 else 0,
+                                                            least=lambda t: few_row_least(t, group_size * max(self.q_lens[b] for b in few), few_channels))
                 n_slots += more
                 n_few, n_count = len(few_items), len(few) * n_kv_heads
                 extras += few_extras.tolist()

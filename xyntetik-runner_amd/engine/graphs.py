@@ -23,7 +23,7 @@ import torch
 
 from ..cache import NULL_PAGE
 from .batch import (ATTN_MIN_RANGE, ATTN_STREAM_SLOTS, ATTN_TILE, FEW_INTS, FEW_MIN_RANGE, FEW_PAGE, FEW_ROWS, FEW_SLOTS, AttentionPlan,
-                    Chunked, StepEntry, few_row_items, mask_reach)
+                    Chunked, StepEntry, few_row_items, few_row_least, mask_reach)
 
 BUCKETS = (1, 2, 4, 8, 16, 32, 64, 128, 256, 512)
 SPLITS = (1, 2, 4, 8, 16, 32)
@@ -87,8 +87,8 @@ class StaticDecodeContext:
         # [token_ids B][positions B][req_of_token B][cu_q B+1][seq_lens B][slots B][fresh B][starts B][want B]
         # [tables ...][plans ...]
         self._sizes = [B, B, B, B + 1, B, B, B, B, B] + [B * w for w in self.table_width]
-        # (group size, window, key/value heads, a slot more, workgroups of the kernel for few rows a compute unit holds: 0 another kernel)
-        self._plan_keys: List[Tuple[int, Optional[int], int, bool, int]] = []
+        # (group size, window, key/value heads, a slot more, workgroups of the kernel for few rows a compute unit holds: 0 another kernel; its channels)
+        self._plan_keys: List[Tuple[int, Optional[int], int, bool, int, int]] = []
         self._plans: Dict[tuple, AttentionPlan] = {}
         self._plan_off: Dict[tuple, int] = {}
         self._plan_splits: Dict[tuple, int] = {}       # key ranges a request; the kernel for few rows: items of all together
@@ -149,9 +149,9 @@ class StaticDecodeContext:
                            "ctx.slots (on the device), or sets capturable = False to be run eagerly")
 
     def attention_plan(self, group: int, group_size: int, window, n_kv_heads: int,
-                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0) -> AttentionPlan:
+                       page_size: int = 64, extra_slot: bool = False, few_rows: int = 0, few_channels: int = 256) -> AttentionPlan:
         few = few_rows if page_size >= FEW_PAGE and group_size <= FEW_ROWS else 0
-        key = (group_size, window, n_kv_heads, bool(extra_slot), few)
+        key = (group_size, window, n_kv_heads, bool(extra_slot), few, few_channels if few else 0)
         if key not in self._plans:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("an attention plan was first asked for during graph capture")
@@ -229,12 +229,12 @@ class StaticDecodeContext:
             self.token_ids[:n].copy_(token_source)
 
     def _fill_plan(self, h, base: int, key, starts, n: int) -> None:
-        group_size, window, n_kv_heads, extra, few = key
+        group_size, window, n_kv_heads, extra, few, few_channels = key
         B, S = self.B, self._plan_splits[key]
         if few:
             # (rows that pad the batch have an item each, and leave the requests all the workgroups)
             got, extras, _ = few_row_items(np.arange(B), starts, np.ones(B, dtype=np.int64), np.arange(B), window, min(S, max(B, FEW_SLOTS // n_kv_heads + B - n)), extra,
-                                           pair_at=ATTN_STREAM_SLOTS // n_kv_heads if few == 2 else 0)
+                                           pair_at=ATTN_STREAM_SLOTS // n_kv_heads if few == 2 else 0, least=lambda t: few_row_least(t, group_size, few_channels))
             items = h[base:base + S * FEW_INTS].reshape(S, FEW_INTS)
             items[:len(got)] = got
             items[len(got):, 2:4] = 0              # (no keys: nothing to do)
