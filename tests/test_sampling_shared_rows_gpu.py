@@ -76,3 +76,28 @@ def test_windows_of_a_batch(W):
     sampler = Sampler(load_ops(), torch.device(DEV))
     got = sampler.sample(torch.tensor(x, device=DEV), states)
     assert got == sampler.sample(torch.tensor(want_x, device=DEV), plain)
+
+
+# on either side of the lines between one workgroup a row, four of which the last picks, and eight that look for candidates; rows that are not 16-byte aligned
+@pytest.mark.parametrize("kind", ["plain", "equal", "steps", "ruled_out", "near", "far", "peaked", "nothing", "no_number"])
+@pytest.mark.parametrize("W,V,ld", [(2, 19996, 19996), (2, 20000, 20000), (64, 20004, 20008), (65, 20004, 20004), (3, 45996, 45996), (3, 46000, 46000), (2, 20001, 20003), (129, 46000, 46000)])
+def test_ways_to_share_a_row_pick_alike(kind, W, V, ld):
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    assert {ops._sample_shares(w, v, a) for w, v, a in ((2, 19996, True), (65, 20004, True), (129, 46000, True))} == {(0, 0)}
+    assert ops._sample_shares(64, 20004, True) == ops._sample_shares(3, 45996, True) == (4, 0)
+    assert ops._sample_shares(3, 46000, True) == ops._sample_shares(2, 20001, False) == (8, 8)
+    rng = np.random.default_rng(W * 31 + V + len(kind))
+    room = torch.zeros((W, ld), device=DEV)
+    room[:, :V] = torch.tensor(_rows(kind, W, V, rng), device=DEV)
+    logits = room[:, :V]
+    f = lambda v: torch.tensor(np.asarray(v, dtype=np.float32), device=DEV)
+    i = lambda v: torch.tensor(np.asarray(v, dtype=np.int32), device=DEV)
+    for turn in range(2):
+        temp, draw = f(rng.choice([0.0, 0.3, 0.8, 1.3, 2e-7, 3e7], W, p=[.1, .25, .3, .25, .05, .05])), f(rng.choice([0.0, 0.5, 1.0 - 2.0 ** -24, 0.123], W))
+        top_k, top_p, min_p = i(rng.choice([0, 1, 40, 2048, 2049, V], W)), f(rng.choice([1.0, 0.95, 0.0], W)), f(rng.choice([0.0, 0.05, 1.0], W) * turn)
+        got = ops.sample(logits, temp, draw, top_k=top_k, top_p=top_p, min_p=min_p).cpu().tolist()
+        out = torch.empty((W,), dtype=torch.int32, device=DEV)
+        ops.lib.check(ops.lib.xr_sample(out.data_ptr(), logits.data_ptr(), W, V, ld, temp.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), min_p.data_ptr(), None,
+                                        draw.data_ptr(), None, None, 0, None, 0, None, torch.cuda.current_stream().cuda_stream))
+        assert got == out.cpu().tolist(), (kind, W, V, turn)

@@ -2031,24 +2031,39 @@ class Ops:
         return self._sample(logits, exempt, o, o + 5 * step, o + step, o + 2 * step, o + 3 * step, o + 4 * step,
                             o + 7 * step if recent_cap else None, o + 6 * step if recent_cap else None, recent_cap)
 
+    @staticmethod
+    def _sample_shares(W: int, V: int, aligned: bool) -> tuple:
+        """(workgroups that share a sampled row's histogram, workgroups that look for its candidates; 0, 0: one workgroup a row; n, 0: the histogram's last
+        workgroup picks, reading the row again).  ``aligned``: rows are read 16 bytes at a time.
+
+        Sharing a row costs a kernel's boundary and what its workgroups tell each other.  Picks of 8 rows, us, one workgroup a row / 4 that leave it to the last / 8 and 8
+        with candidates: 8,192 logits top-k 40 16.1 / 17.6 / 24.0, min-p 17.2 / 18.3 / 22.0; 16,384 18.3 / 18.4 / 23.7 and 19.7 / 19.3 / 22.0; 32,000 22.1 / 20.0 / 24.1 and
+        24.0 / 21.6 / 22.8 (all cuts at once 29.8 / 28.6 / 27.1); 44,000 26.2 / 21.8 / 25.3 and 28.4 / 23.8 / 24.0; 65,536 and more: the last.  64 rows of 32,000 top-k 40 23.7 /
+        22.2 / 28.3, 200 rows 28.9 and, with 2 and 2, 41; 200 rows of 65,536 a fifth less than with 2 and 2, of 128,256 top-p 87.9 and 81.7.  Up to 512 workgroups of
+        1,024 threads, two a compute unit; more than 8 shares a row cost more to add up again than they save."""
+        if V < 20000 or (aligned and W > 64 and V < (44000 if W <= 128 else 66000)):
+            return 0, 0
+        if aligned and W <= 64 and V < 46000:
+            return 4, 0
+        n = max(1, min(8, 512 // max(1, W)))
+        return n, n
+
     def _sample(self, logits, exempt, temp, top_k, top_p, min_p, repeat_penalty, draw, recent, n_recent, recent_cap: int) -> torch.Tensor:
         if logits.dtype != torch.float32 or logits.dim() != 2 or logits.stride(1) != 1:
             raise KernelError("sample: logits must be float32 [rows, vocab]")
         W, V = logits.shape
         out = torch.empty((W,), dtype=torch.int32, device=logits.device)
         # room for the first pass (32 ranges a row) when a row is long enough to need one, and behind it for a sampled batch's
-        # histograms (a batch without any sampled row brings no options): a row's is shared out so that up to 512
-        # workgroups of 1,024 threads work on them, two a compute unit; more than 8 shares a row cost more to add up
-        # again than they save.
+        # histograms (a batch without any sampled row brings no options)
         first = W * 32 * 2 * 4 if V >= 8192 else 0
-        splits = max(1, min(8, 512 // max(1, W))) if first and top_k is not None else 0
+        splits, picks = self._sample_shares(W, V, logits.stride(0) % 4 == 0 and logits.data_ptr() % 16 == 0) if first and top_k is not None else (0, 0)
         room = W * ((splits + 1) * _SAMPLE_BIN_BYTES + _SAMPLE_FOUND_BYTES) if splits else 0
         ws = torch.empty((first + room,), dtype=torch.uint8, device=logits.device) if first else None
         part = ws.data_ptr() if first else None
         args = (out.data_ptr(), logits.data_ptr(), W, V, logits.stride(0), temp, top_k, top_p, min_p, repeat_penalty, draw, recent, n_recent,
                 recent_cap, _ptr(exempt), exempt.numel() if exempt is not None else 0, part)
         if splits:
-            self.lib.check(self.lib.xr_sample_split(*args, part + first, room, splits, splits, _stream()))
+            self.lib.check(self.lib.xr_sample_split(*args, part + first, room, splits, picks, _stream()))
         else:
             self.lib.check(self.lib.xr_sample(*args, _stream()))
         return out

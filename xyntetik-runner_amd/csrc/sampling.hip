@@ -676,79 +676,6 @@ __device__ __forceinline__ void plan_cuts(const SampleArgs& a, int r, const Opti
     }
 }
 
-// A share of a row's histogram (grid: rows x shares).  The last of the row's workgroups adds the shares up and leaves the sums of the
-// bins and the runs of bins to look into.
-__global__ __launch_bounds__(SM_THREADS, 8) void k_pick_hist(SampleArgs a) {
-    __shared__ u64 mass[SM_BINS];
-    __shared__ unsigned count[SM_BINS];
-    __shared__ u64 sh[SM_THREADS / 64];
-    __shared__ int shi[2];
-    __shared__ Bins shared_bins;
-    __shared__ Options options;
-    const int r = blockIdx.x, sp = blockIdx.y;
-    const float temp = a.temp[r];
-    if (!(temp > 0.f)) return;
-    const bool counts = a.top_k && a.top_k[r] > 0 && a.top_k[r] < a.V;
-    const int chunk = ((a.V + a.hist_splits - 1) / a.hist_splits + 3) & ~3;
-    const int lo = sp * chunk < a.V ? sp * chunk : a.V, hi = lo + chunk < a.V ? lo + chunk : a.V;
-    float* row = a.logits + (size_t)r * a.ld;
-    Bins bins;
-    auto prepare = [&] {
-        for (int i = threadIdx.x; i < SM_BINS; i += SM_THREADS) { mass[i] = 0; count[i] = 0; }
-        if (threadIdx.x < 64) {             // (by every wave, the divisions alone take a compute unit's 32 waves 1 us)
-            float mx, mn;
-            row_extent(a.part, r, mx, mn);
-            const Bins b = make_bins(mx, mn, temp);
-            if (threadIdx.x == 0) { shared_bins = b; options.load(a, r); }
-        }
-        __syncthreads();
-        bins = shared_bins;
-    };
-    // (an unusual row is left for the plain division; its loads are then for nothing)
-    bool unusual = false;
-    fill_hist<0, false>(row, lo, hi, temp, bins, counts, mass, count, [&] { prepare(); unusual = !bins.ordinary; }, unusual);
-    if (unusual && fabsf(bins.zmax) < INFINITY) fill_hist<0, true>(row, lo, hi, temp, bins, counts, mass, count, [] {}, false);
-    if (!(fabsf(bins.zmax) < INFINITY)) {           // (no histogram of such a row is read)
-        if (sp == 0 && threadIdx.x == 0) a.notes[r].n_cuts = -1;
-        return;
-    }
-    __syncthreads();
-    const size_t at = ((size_t)r * a.hist_splits + sp) * SM_BINS;
-    for (int i = threadIdx.x; i < SM_BINS; i += SM_THREADS) {
-        store_agent(a.hist_mass + at + i, mass[i]);
-        if (counts) store_agent(a.hist_count + at + i, count[i]);
-    }
-    if (!last_to_arrive(&a.notes[r].arrived[0], a.hist_splits, shi)) return;
-
-    const int b0 = 2 * threadIdx.x;
-    u64 m0 = 0, m1 = 0;
-    unsigned c0 = 0, c1 = 0;
-    for (int s0 = 0; s0 < a.hist_splits; s0 += 4) {      // (four shares' loads side by side)
-        u64 m[4][2];
-        unsigned c[4][2];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const size_t from = ((size_t)r * a.hist_splits + (s0 + u < a.hist_splits ? s0 + u : s0)) * SM_BINS + b0;
-            m[u][0] = load_agent(a.hist_mass + from);
-            m[u][1] = load_agent(a.hist_mass + from + 1);
-            c[u][0] = counts ? load_agent(a.hist_count + from) : 0;
-            c[u][1] = counts ? load_agent(a.hist_count + from + 1) : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (s0 + u < a.hist_splits) { m0 += m[u][0]; m1 += m[u][1]; c0 += c[u][0]; c1 += c[u][1]; }
-    }
-    scan_pairs(m0, m1, sh);
-    if (counts) scan_pairs(c0, c1, (unsigned*)sh);
-    mass[b0] = m0; mass[b0 + 1] = m1;
-    count[b0] = c0; count[b0 + 1] = c1;
-    const size_t to = (size_t)r * SM_BINS + b0;
-    *reinterpret_cast<ulonglong2*>(a.mass + to) = make_ulonglong2(m0, m1);
-    if (counts) *reinterpret_cast<uint2*>(a.count + to) = make_uint2(c0, c1);
-    __syncthreads();
-    if (threadIdx.x < 64) plan_cuts(a, r, options, bins, mass, count);
-}
-
 // The pick where a cut's bin does not fit the list: every boundary by a radix selection over the row.
 template <int U, int NT>
 __device__ __forceinline__ int sample_by_radix(const SampleArgs& a, int r, const float* row, float temp, float zmax, u64* hist, u64* sh, u64* sh2) {
@@ -879,6 +806,96 @@ __device__ __forceinline__ void pick_greedy(const SampleArgs& a, int r, const fl
             if (shf[w] > best || (shf[w] == best && shi[w] < bi)) { best = shf[w]; bi = shi[w]; }
         a.out[r] = bi == 0x7fffffff ? 0 : bi;
     }
+}
+
+// A share of a row's histogram (grid: rows x shares).  The last of the row's workgroups adds the shares up and leaves the sums of the
+// bins and the runs of bins to look into; or (PICK) it picks, reading the row again for every cut, which for a row that is not long is less than a kernel's
+// boundary and what the workgroups tell each other a second time.
+template <bool PICK>
+__global__ __launch_bounds__(SM_THREADS, 8) void k_pick_hist(SampleArgs a) {
+    __shared__ u64 mass[SM_BINS];
+    __shared__ unsigned count[SM_BINS];
+    __shared__ u64 sh[SM_THREADS / 64];
+    __shared__ int shi[2];
+    __shared__ Bins shared_bins;
+    __shared__ Options options;
+    const int r = blockIdx.x, sp = blockIdx.y;
+    const float temp = a.temp[r];
+    if (!(temp > 0.f)) {
+        if (PICK && sp == 0) pick_greedy(a, r, a.logits + (size_t)r * a.ld, (float*)sh, (int*)(sh + SM_THREADS / 128));
+        return;
+    }
+    const bool counts = a.top_k && a.top_k[r] > 0 && a.top_k[r] < a.V;
+    const int chunk = ((a.V + a.hist_splits - 1) / a.hist_splits + 3) & ~3;
+    const int lo = sp * chunk < a.V ? sp * chunk : a.V, hi = lo + chunk < a.V ? lo + chunk : a.V;
+    float* row = a.logits + (size_t)r * a.ld;
+    Bins bins;
+    auto prepare = [&] {
+        for (int i = threadIdx.x; i < SM_BINS; i += SM_THREADS) { mass[i] = 0; count[i] = 0; }
+        if (threadIdx.x < 64) {             // (by every wave, the divisions alone take a compute unit's 32 waves 1 us)
+            float mx, mn;
+            row_extent(a.part, r, mx, mn);
+            const Bins b = make_bins(mx, mn, temp);
+            if (threadIdx.x == 0) { shared_bins = b; options.load(a, r); }
+        }
+        __syncthreads();
+        bins = shared_bins;
+    };
+    // (an unusual row is left for the plain division; its loads are then for nothing)
+    bool unusual = false;
+    fill_hist<0, false>(row, lo, hi, temp, bins, counts, mass, count, [&] { prepare(); unusual = !bins.ordinary; }, unusual);
+    if (unusual && fabsf(bins.zmax) < INFINITY) fill_hist<0, true>(row, lo, hi, temp, bins, counts, mass, count, [] {}, false);
+    if (!(fabsf(bins.zmax) < INFINITY)) {           // (no histogram of such a row is read)
+        if (sp == 0 && threadIdx.x == 0) {
+            if (PICK) a.out[r] = 0;
+            else a.notes[r].n_cuts = -1;
+        }
+        return;
+    }
+    __syncthreads();
+    const size_t at = ((size_t)r * a.hist_splits + sp) * SM_BINS;
+    for (int i = threadIdx.x; i < SM_BINS; i += SM_THREADS) {
+        store_agent(a.hist_mass + at + i, mass[i]);
+        if (counts) store_agent(a.hist_count + at + i, count[i]);
+    }
+    if (!last_to_arrive(&a.notes[r].arrived[0], a.hist_splits, shi)) return;
+
+    const int b0 = 2 * threadIdx.x;
+    u64 m0 = 0, m1 = 0;
+    unsigned c0 = 0, c1 = 0;
+    for (int s0 = 0; s0 < a.hist_splits; s0 += 4) {      // (four shares' loads side by side)
+        u64 m[4][2];
+        unsigned c[4][2];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const size_t from = ((size_t)r * a.hist_splits + (s0 + u < a.hist_splits ? s0 + u : s0)) * SM_BINS + b0;
+            m[u][0] = load_agent(a.hist_mass + from);
+            m[u][1] = load_agent(a.hist_mass + from + 1);
+            c[u][0] = counts ? load_agent(a.hist_count + from) : 0;
+            c[u][1] = counts ? load_agent(a.hist_count + from + 1) : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (s0 + u < a.hist_splits) { m0 += m[u][0]; m1 += m[u][1]; c0 += c[u][0]; c1 += c[u][1]; }
+    }
+    scan_pairs(m0, m1, sh);
+    if (counts) scan_pairs(c0, c1, (unsigned*)sh);
+    mass[b0] = m0; mass[b0 + 1] = m1;
+    count[b0] = c0; count[b0 + 1] = c1;
+    if constexpr (PICK) {
+        __shared__ List list;
+        __shared__ u64 sh2[2];
+        __syncthreads();
+        int pick = sample_by_bins<4, SM_THREADS>(a, options, row, temp, bins, Found{nullptr, -1, nullptr}, mass, count, list, sh);
+        if (pick < 0) pick = sample_by_radix<4, SM_THREADS>(a, r, row, temp, bins.zmax, mass, sh, sh2);
+        if (threadIdx.x == 0) a.out[r] = pick;
+        return;
+    }
+    const size_t to = (size_t)r * SM_BINS + b0;
+    *reinterpret_cast<ulonglong2*>(a.mass + to) = make_ulonglong2(m0, m1);
+    if (counts) *reinterpret_cast<uint2*>(a.count + to) = make_uint2(c0, c1);
+    __syncthreads();
+    if (threadIdx.x < 64) plan_cuts(a, r, options, bins, mass, count);
 }
 
 // One workgroup a row: greedy rows, and sampled rows of short vocabularies and of callers that bring no work area.
@@ -1062,8 +1079,10 @@ static int sample_launch(int* out, float* logits, int W, int V, int ld, const fl
         XR_CHECK_LAUNCH("sample_extent");
     }
     if (a.notes) {
-        k_pick_hist<<<dim3(W, hist_splits), SM_THREADS, 0, stream>>>(a);
+        if (row_splits == 0) k_pick_hist<true><<<dim3(W, hist_splits), SM_THREADS, 0, stream>>>(a);
+        else k_pick_hist<false><<<dim3(W, hist_splits), SM_THREADS, 0, stream>>>(a);
         XR_CHECK_LAUNCH("sample_hist");
+        if (row_splits == 0) return XR_OK;
         k_pick_rows<<<dim3(W, row_splits), SM_THREADS, 0, stream>>>(a);
         XR_CHECK_LAUNCH("sample_rows");
         return XR_OK;
@@ -1082,7 +1101,7 @@ extern "C" int xr_sample(int* out, float* logits, int W, int V, int ld, const fl
 }
 
 // The same with a work area for the sampled rows: their histograms are shared out to `splits` workgroups a row, their candidates to
-// `row_splits`.  Its bytes a row:
+// `row_splits` (0: none, the histogram's last workgroup picks).  Its bytes a row:
 static long long sample_work_bytes(int splits) { return (long long)(splits + 1) * SM_BINS * 12 + SM_FOUND * 8 + (long long)sizeof(RowNotes); }
 
 extern "C" int xr_sample_split(int* out, float* logits, int W, int V, int ld, const float* temp, const int* top_k,
@@ -1090,7 +1109,7 @@ extern "C" int xr_sample_split(int* out, float* logits, int W, int V, int ld, co
                                const float* draw, const int* recent, const int* n_recent, int recent_cap,
                                const int* exempt, int n_exempt, float* greedy_ws, void* hist_ws, long long hist_bytes,
                                int splits, int row_splits, hipStream_t stream) {
-    XR_REQUIRE(greedy_ws && hist_ws && splits > 0 && splits <= 32 && row_splits > 0 && row_splits <= 64, "sample_split: no work area or %d and %d splits", splits, row_splits);
+    XR_REQUIRE(greedy_ws && hist_ws && splits > 0 && splits <= 32 && row_splits >= 0 && row_splits <= 64, "sample_split: no work area or %d and %d splits", splits, row_splits);
     XR_REQUIRE(((uintptr_t)hist_ws & 15) == 0 && hist_bytes >= W * sample_work_bytes(splits), "sample_split: a work area of %lld bytes for %d rows in %d parts",
                hist_bytes, W, splits);
     return sample_launch(out, logits, W, V, ld, temp, top_k, top_p, min_p, repeat_penalty, draw, recent, n_recent,
