@@ -24,3 +24,17 @@ def test_division_of_a_step(ops, kind, H):
 def test_scratch_is_bounded(ops, monkeypatch):
     monkeypatch.setattr(Ops, "CHUNKS_SCRATCH", 10 * Ops._chunk_floats("delta", 32))
     assert ops.chunked_rows("delta", [640], 32, 128) == 640 and ops.chunked_rows("delta", [641], 32, 128) is None
+
+
+# a workgroup a (request, head): on either side of how many of them are still the faster way, by the values' size
+@pytest.mark.parametrize("kind,Dv,most", [("retention", 16, 1024), ("delta", 16, 1024), ("retention", 17, 2048), ("delta", 17, 4096), ("retention", 64, 2048),
+                                          ("delta", 64, 4096), ("retention", 65, None), ("delta", 128, None)])
+def test_where_a_step_in_one_kernel_pays(kind, Dv, most):
+    from types import SimpleNamespace
+    from xyntetik_runner_amd.csrc.ops import Ops
+    pays = lambda B, H, **kw: Ops.recurrence_step_pays(kind, SimpleNamespace(max_q_len=kw.get("rows", 1), B=B), B, H, kw.get("D", 64), Dv)
+    assert pays(1, 1) and pays(8, 32) and not pays(8, 32, rows=2) and not pays(8, 32, D=32)
+    if most is None:
+        assert pays(512, 64)
+    else:
+        assert pays(most // 32, 32) and not pays(most // 32 + 1, 32)

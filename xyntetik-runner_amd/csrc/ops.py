@@ -1628,6 +1628,16 @@ class Ops:
         """Whether a recurrence's rows of this step can go through ``recurrence_step``: one row a request, heads of 33 to 128 by up to 128."""
         return ctx.max_q_len == 1 and T == ctx.B and T < 65536 and 32 < D <= 128 and 0 < Dv <= 128
 
+    @classmethod
+    def recurrence_step_pays(cls, kind: str, ctx, T: int, H: int, D: int, Dv: int) -> bool:
+        """Whether it applies and is the faster way.  A workgroup has 1,024 threads, of which Dv x 16 hold a piece of the state, and two of them run on a compute unit
+        at a time: many of them with few columns take longer than the kernels it stands for, which have no idle threads.  Its time over theirs, for 256, 1,024,
+        2,048, 4,096 and 8,192 (request, head) pairs: values of 16 channels (heads of 64) retention 0.46, 0.97, 1.37, 1.80, 2.4, the delta rule 0.57, 0.94, 1.23, 1.5,
+        1.9; of 32 (heads of 128) 0.45, 0.80, 1.0, 1.23, 1.4 and 0.54, 0.73, 0.85, 0.97, 1.05; of 64 (heads of 128) 0.45, 0.70, 0.95, 1.05, 1.2 and 0.53, 0.62, 0.78, 0.81,
+        0.86; of 128 0.46, 0.81, 0.89, 0.93, 0.97 and 0.51, 0.72, 0.80, 0.76, 0.94."""
+        most = 1024 if Dv <= 16 else (4096 if kind == "delta" else 2048) if Dv <= 64 else 1 << 30
+        return cls.recurrence_step_applies(ctx, T, D, Dv) and T * H <= most
+
     def recurrence_step(self, kind: str, q, k, v, state: torch.Tensor, ctx, H: int, G: int, D: int, Dv: int, out_gate, w_norm, eps: float,
                         out_dtype: torch.dtype, gate_activation: str = "silu", decay=None, inv_freq=None, rot: int = 0, beta=None, gate=None,
                         a_log=None, dt_bias=None, q_scale: float = 1.0, k_scale: float = 1.0, unit_eps: float = 0.0) -> torch.Tensor:

@@ -127,7 +127,7 @@ class Retention(Mixer):
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32)
         q, k, v, gate = proj[:, :QK], proj[:, QK:2 * QK], proj[:, 2 * QK:2 * QK + V], proj[:, 2 * QK + V:]
         rot = self.position.rotary() if self.position is not None else None
-        if self.qkv_activation is None and self.norm_over == "head" and ops.recurrence_step_applies(ctx, h.shape[0], D, Dv):
+        if self.qkv_activation is None and self.norm_over == "head" and ops.recurrence_step_pays("retention", ctx, h.shape[0], H, D, Dv):
             return ops.recurrence_step("retention", q, k, v, cache.state, ctx, H, H, D, Dv, gate, self.w_norm, self.eps, self.rt.dtype,
                                        self.gate_activation, decay=self.decay, inv_freq=rot.inv_freq if rot is not None else None,
                                        rot=rot.rotary_dim if rot is not None else 0, k_scale=self.key_scale)
@@ -336,7 +336,7 @@ class GatedDelta(Mixer):
             o = ops.linear_recurrence("delta_channel", q, k, v, cache.states["mixer.S"], ctx, H, G, D, Dv, beta=b, gate=w)
         else:
             a = proj[:, at + H:]
-            if ops.recurrence_step_applies(ctx, h.shape[0], D, Dv):
+            if ops.recurrence_step_pays("delta", ctx, h.shape[0], H, D, Dv):
                 return ops.recurrence_step("delta", q, k, v, cache.states["mixer.S"], ctx, H, G, D, Dv, gate, self.w_norm, self.eps, self.rt.dtype,
                                            self.gate_activation, beta=b, gate=a, a_log=self.a_log, dt_bias=self.dt_bias,
                                            q_scale=D ** -0.5, unit_eps=self.UNIT_EPS)
