@@ -27,3 +27,16 @@ def test_top_k_of_any_number(top_k, kept):
     for temperature in (0.8, 1e39):         # (the latter is beyond 32 bits)
         words = SamplerState(SamplingParams(temperature=temperature, top_k=top_k, top_p=0.5)).words
         assert struct.unpack("=4fi", words)[1:] == (0.5, 0.0, 1.0, kept)
+
+
+@pytest.mark.parametrize("n", [1, 8, 64])
+@pytest.mark.parametrize("every", [0, 3])
+def test_draws_as_the_kernels_get_them(n, every):
+    """What a batch stores into its options: the same 32-bit numbers, whether they come as a list or side by side."""
+    from xyntetik_runner_amd.sampling.params import SamplerState, SamplingParams, draw_values
+    mk = lambda: [SamplerState(SamplingParams(temperature=0.0 if every and i % every == 0 else 0.8, seed=i * 977 + 5)) for i in range(n)]
+    many, one = mk(), mk()
+    stored = np.empty(n, dtype=np.float32)
+    for _ in range(3):
+        stored[:] = draw_values(many, [s.greedy for s in many])
+        assert stored.tolist() == [0.0 if s.greedy else s.draw() for s in one]
