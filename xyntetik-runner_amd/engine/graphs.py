@@ -38,12 +38,12 @@ def bucket_for(n: int) -> Optional[int]:
 
 
 def splits_for(batch_cap: int, max_tiles: int, n_kv_heads: int) -> int:
-    """Key ranges per request: one round of workgroups, and no range shorter than it pays.
+    """Key ranges per request of the streaming kernel and its merge: one round of workgroups, and no range shorter than it pays; for all
+    plans of a step it is part of the key that its graph is kept by.
 
-    Below ``ONE_RANGE_TILES`` one range, and no kernel that merges ranges: recorded steps with 8 key/value heads and 330 cached
-    tokens, two ranges and one: 1B class 765 us and 723 (4 requests 783 and 737), 8B shape 905 and 888 (16 requests 1,096 and 1,069); from
-    16 tiles on ranges gain (700 tokens 771 and 767, 1,000 tokens 767 and 799).  Measured with 8 workgroups and more; fewer are cut up
-    as before."""
+    Below ``ONE_RANGE_TILES`` one range, and no kernel that merges ranges (more heads a key/value head than the kernel for few rows takes, heads that are not whole steps of
+    32 channels; measured with 8 key/value heads and 8 workgroups and more, when decoded tokens of all heads went this way: 330 cached tokens, two ranges and one, 1B class 765 us and 723, from 16 tiles on ranges
+    gain, 1,000 tokens 767 and 799); fewer workgroups are cut up."""
     if max_tiles < ONE_RANGE_TILES and batch_cap * n_kv_heads >= 8:
         return 1
     want = max(1, min(ATTN_STREAM_SLOTS // (batch_cap * n_kv_heads), max_tiles // ATTN_MIN_RANGE))
