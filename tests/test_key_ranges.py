@@ -14,6 +14,41 @@ def test_splits_for(args, ranges):
     assert splits_for(*args) == ranges
 
 
+@pytest.mark.parametrize("B,heads", [(1, 1), (1, 2), (1, 8), (1, 100), (4, 1), (8, 1), (8, 8), (16, 8), (32, 8), (64, 8), (512, 32)])
+@pytest.mark.parametrize("table_tiles", [7, 16, 64, 640, 5000])
+def test_longest_request_of_a_key(B, heads, table_tiles):
+    """What a graph keeps room for is what the longest request with its key would ask for, whatever it is recorded with."""
+    from xyntetik_runner_amd.engine.graphs import most_tiles
+    of = {}
+    for tiles in range(1, table_tiles + 1):
+        of.setdefault(splits_for(B, tiles, heads), []).append(tiles)
+    for ranges, tiles in of.items():
+        assert most_tiles(B, ranges, heads, table_tiles) == tiles[-1], (ranges, tiles[0], tiles[-1])
+
+
+@pytest.mark.gpu
+def test_results_do_not_hang_on_the_length_that_was_recorded(tmp_path):
+    """A request of 900 keys on the graph that one of 520 had recorded, and on its own: the same key ranges, so the same bits."""
+    from tiny import make_model, prompt_ids
+    from xyntetik_runner_amd.engine.batch import StepEntry
+    from xyntetik_runner_amd.engine.runner import ModelRunner
+    d = make_model("D", str(tmp_path))
+    toks = {n: prompt_ids(n + 3, 1000, n) for n in (520, 900)}
+
+    def decoded(lens):
+        runner = ModelRunner.from_folder(d, dtype="bfloat16", max_tokens=2048, page_size=64, max_requests=2)
+        for i, n in enumerate(lens):
+            runner.step([StepEntry(i, toks[n][:n], [])])
+            rows = [runner.step([StepEntry(i, [t], [0])]).cpu().numpy() for t in toks[n][n:]]
+        assert runner.graphs.captures == 1
+        (ctx, _, _), = runner.graphs.graphs.values()
+        return [p.n_few for p in ctx._plans.values()], np.stack(rows)
+
+    after, alone = decoded([520, 900]), decoded([900])
+    assert after[0] == alone[0] and min(alone[0]) >= 8
+    assert np.array_equal(after[1], alone[1])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_decoding_from_one_range_into_several(tmp_path, dtype):

@@ -54,9 +54,17 @@ def splits_for(batch_cap: int, max_tiles: int, n_kv_heads: int) -> int:
     return best
 
 
+def most_tiles(batch_cap: int, n_splits: int, n_kv_heads: int, table_tiles: int) -> int:
+    """Tiles of the longest request whose step has the same key as one with ``n_splits`` key ranges (``splits_for``) and block tables of ``table_tiles``."""
+    end = ONE_RANGE_TILES if n_splits == 1 and batch_cap * n_kv_heads >= 8 else 2 * n_splits * ATTN_MIN_RANGE      # the first with more, if there is one
+    return table_tiles if splits_for(batch_cap, end, n_kv_heads) == n_splits else min(end - 1, table_tiles)
+
+
 def few_row_room(batch_cap: int, tiles: int, n_kv_heads: int) -> int:
     """Items that a recorded step keeps for the kernel for few rows: one a request, and as many key ranges as fill the kernel's workgroups beside the
-    rows that pad the batch (fewer than half of it, an item each), but no more than ranges of the shortest length (and one for what the requests' last ranges lack)."""
+    rows that pad the batch (fewer than half of it, an item each), but no more than ranges of the shortest length (and one for what the requests' last ranges lack).
+    ``tiles``: those of the longest request that the graph will serve, not of the one it is recorded with: ranges and the last bits of a result then
+    do not hang on what ran before, and a request that grows gets as many as one that came long (items without keys return at once)."""
     return max(batch_cap, min(FEW_SLOTS // n_kv_heads + batch_cap // 2, batch_cap * (-(-tiles // FEW_MIN_RANGE) + 1)))
 
 
@@ -66,14 +74,15 @@ class StaticDecodeContext:
     plans_few_rows = True
 
     def __init__(self, ops, device, batch_cap: int, n_splits: int, table_widths: List[int],
-                 windowed: Optional[List[bool]] = None, max_tiles: Optional[int] = None, *, null_slot: int):
+                 windowed: Optional[List[bool]] = None, max_tiles: Optional[int] = None, *, null_slot: int,
+                 most: Optional[int] = None):
         """``n_splits``: the most key ranges a request is cut into; ``max_tiles``: the longest request's
-        tiles when the context is made.  Every attention plan (group size, window, key/value heads)
+        tiles when the context is made; ``most``: those of the longest it will serve (``most_tiles``).  Every attention plan (group size, window, key/value heads)
         gets a number of key ranges of its own from these: a windowed layer, or one with more
         key/value heads, needs fewer ranges to fill the chip than the bucket's longest request
         with the fewest heads."""
         self.ops, self.device = ops, device
-        self.max_tiles = max_tiles
+        self.max_tiles, self.most_tiles = max_tiles, most
         self.null_slot = null_slot          # the state row of the rows that pad the batch
         # groups whose requests give pages back while they live (their table rows are rewritten every step)
         self.windowed = list(windowed) if windowed is not None else [True] * len(table_widths)
@@ -155,7 +164,7 @@ class StaticDecodeContext:
         if key not in self._plans:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("an attention plan was first asked for during graph capture")
-            tiles = self.max_tiles
+            tiles = self.most_tiles if few else self.max_tiles
             if tiles is not None and window:
                 tiles = min(tiles, -(-mask_reach(window) // ATTN_TILE) + 1)
             if few:
@@ -332,7 +341,8 @@ class DecodeGraphs:
         # first time: run the step eagerly on the static context, then record it for later
         ctx = StaticDecodeContext(r.ops, r.device, cap, S, width,
                                   windowed=[g.spec.window is not None for g in r.manager.groups],
-                                  max_tiles=-(-max_len // ATTN_TILE), null_slot=r.storage.null_slot)
+                                  max_tiles=-(-max_len // ATTN_TILE), null_slot=r.storage.null_slot,
+                                  most=most_tiles(cap, S, self.kv_heads, w * r.page_size // ATTN_TILE))
         ctx.fill(entries, rcs, token_source)
         x = r.model.forward(ctx, r.storage.layers)
         out = r.model.logits(ctx, x, ctx.want_rows)
