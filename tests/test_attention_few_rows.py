@@ -105,6 +105,17 @@ def test_few_rows_kernel(case, room, monkeypatch):
         assert err < 1.2e-2, float(err)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hk,D,Dv", [(4, 1, 128, 128), (16, 1, 64, 32), (12, 1, 256, 192), (9, 1, 96, 96), (16, 1, 128, 128), (1, 1, 32, 32)])
+@pytest.mark.parametrize("least", [1, 3])
+def test_many_ranges_added_up(H, Hk, D, Dv, least, monkeypatch):
+    """A row block of 1 to 157 key ranges (16, 17, 64, 65 and 128 among them): the last workgroup weighs 64 of them a turn, for one row or sixteen."""
+    from xyntetik_runner_amd.engine import batch
+    monkeypatch.setattr(batch, "few_row_least", lambda tiles, *a: least)
+    starts = [31, 511, 543, 2047, 2079, 4095, 5000]
+    test_few_rows_kernel((H, Hk, D, Dv, 64, None, starts, [1] * len(starts)), 1024, monkeypatch)
+
+
 # What a softmax or a row may have beside its keys; every one of them is in both of the kernel's write-outs.
 EXTRAS = {
     "sinks": dict(sinks=True),
@@ -184,9 +195,9 @@ def test_few_rows_kernel_with(what, shape, room, monkeypatch):
         assert np.abs(got - want).max() < 1.2e-2 * np.abs(want).max()
 
 
-# (tiles, rows, channels of a key and a value): whole, ranges of 4 tiles and more, 16 ranges, 32
-@pytest.mark.parametrize("args,least", [((10, 4, 256), 10), ((11, 4, 256), 4), ((16, 16, 256), 16), ((17, 16, 256), 4), ((8, 1, 256), 8), ((9, 1, 256), 4),
-                                        ((15, 4, 128), 15), ((16, 4, 128), 4), ((125, 4, 256), 8), ((199, 4, 256), 13), ((200, 4, 256), 7), ((399, 16, 256), 25),
+# (tiles, rows, channels of a key and a value): whole, ranges of 3 tiles and more, 16 ranges, 32
+@pytest.mark.parametrize("args,least", [((10, 4, 256), 10), ((11, 4, 256), 3), ((13, 16, 256), 13), ((14, 16, 256), 3), ((9, 1, 256), 9), ((10, 1, 256), 3),
+                                        ((15, 4, 128), 15), ((16, 4, 128), 3), ((125, 4, 256), 8), ((199, 4, 256), 13), ((200, 4, 256), 7), ((399, 16, 256), 25),
                                         ((400, 16, 256), 13), ((250, 4, 128), 16), ((1, 1, 512), 1)])
 def test_shortest_ranges(args, least):
     from xyntetik_runner_amd.engine.batch import few_row_least

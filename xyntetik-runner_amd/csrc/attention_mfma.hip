@@ -1072,9 +1072,9 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void k_attn_stream(AttnArgs a) {
 // 128-byte lines, whose other half another wave reads at about the same time (streaming too 75.8 us for 71.4).
 //
 // k_attn_stream with its merge and this, 8 key/value heads of 128 channels, 4 query heads each, in a recorded chain: 1 request of 1,900 keys
-// 11.5 us -> 8.6, of 8,000 21.6 -> 13.6, 8 of 1,000 to 2,000 20.6 -> 16.2, 64 of 950 to 1,900 75.7 -> 68.8 (5.4 TB/s), of 8,000 372 -> 342 (6.2 TB/s);
-// 32 key/value heads, 23 of 450 to 900 64.4 -> 51.1; heads of 64 channels, 1 of 700 8.8 -> 6.9.  Measured and left: eight waves a workgroup
-// (68.1 us for 64 requests, but 54.1 for the 23 of 32 heads), three workgroups a compute unit (spills: 152), both tiles of a page a step at 128 channels (one wave a SIMD: 27 us for 8 requests).
+// 11.2 us -> 11.0 (4 key/value heads, 2,000 keys 11.7 -> 8.7), of 8,000 19.0 -> 13.7, 8 of 1,000 to 2,000 19.6 -> 15.0, 64 of 950 to 1,900 73.9 -> 57.6, of 8,000 369 -> 352;
+// 32 key/value heads, 23 of 450 to 900 48.7 -> 44.3; heads of 64 channels, 1 of 700 9.5 -> 6.7.  Measured and left: eight waves a workgroup
+// (68.1 us for 64 requests for then 68.8, but 54.1 for the 23 of 32 heads), three workgroups a compute unit (spills: 152), both tiles of a page a step at 128 channels (one wave a SIMD: 27 us for 8 requests).
 #define FEW_ROWS 16
 #define FEW_INTS 12                   // an item's 8 numbers (slot -1: it covers all keys), then first slot, slots, counter, items of its row block
 constexpr bool FEW_OK = HD % 32 == 0;
@@ -1083,6 +1083,8 @@ constexpr int FEW_WAVES = 4;
 constexpr int FEW_SUBS = HD + HV <= 128 ? 2 : 1;              // tiles of 32 keys a step
 constexpr int FEW_STEP = 32 * FEW_SUBS;
 constexpr int FEW_PER_CU = HD + HV <= 256 ? 2 : 1;            // workgroups a compute unit has registers for (the plan's ``few_rows``)
+constexpr int FEW_TURN = 64;                                  // key ranges that are weighed together
+constexpr int FEW_PAIRS = HV < 32 ? 1 : HV <= 128 ? HV / 32 : HV / 64;       // pairs of channels that a thread adds up together
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -1334,12 +1336,15 @@ __global__ __launch_bounds__(64 * FEW_WAVES, FEW_PER_CU) void k_attn_few(AttnArg
     }
     __syncthreads();
     if (!last_one) return;
-    for (int idx = tid; idx < n_rows * (HV / 2); idx += 64 * FEW_WAVES) {
-        const int r = idx / (HV / 2), d2 = (idx - r * (HV / 2)) * 2;
+    const int total = n_rows * (HV / 2);
+    const size_t ml_step = (size_t)a.Hk * ROWS * 2, po_step = (size_t)a.Hk * ROWS * HV;
+    if (total <= 64 * FEW_WAVES) {
+        // a pair of channels a thread, which weighs its row's ranges by itself, 16 at a time
+        if (tid >= total) return;
+        const int r = tid / (HV / 2), d2 = (tid - r * (HV / 2)) * 2;
         const float* ml = a.part_ml + (((size_t)s0 * a.Hk + kvh) * ROWS + r) * 2;
         const float* po = a.part_o + (((size_t)s0 * a.Hk + kvh) * ROWS + r) * HV + d2;
-        const size_t ml_step = (size_t)a.Hk * ROWS * 2, po_step = (size_t)a.Hk * ROWS * HV;
-        constexpr int U = 16;                            // slots whose loads are on their way together
+        constexpr int U = 16;
         float mx = -INFINITY, wsum = 0.f;
         float2 acc = make_float2(0.f, 0.f);
         for (int b = 0; b < ns; b += U) {
@@ -1350,6 +1355,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES, FEW_PER_CU) void k_attn_few(AttnArg
                 mlv[u] = load_agent(ml + sc * ml_step);
                 pv[u] = load_agent(po + sc * po_step);
             }
+            __builtin_amdgcn_sched_barrier(0);           // (or the first numbers are waited for one by one: 2 us)
             float cm = mx;
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -1370,6 +1376,108 @@ __global__ __launch_bounds__(64 * FEW_WAVES, FEW_PER_CU) void k_attn_few(AttnArg
         const float inv = (wsum > 0.f ? 1.0f / wsum : 0.f) * row_factor(a.gate, a.ld_gate, a.out_scale, q0 + tk, hh);
         bf16_t* op = a.out + (size_t)(q0 + tk) * a.ld_out + hh * HV + d2;
         *reinterpret_cast<uint32_t*>(op) = pack2(acc.x * inv, acc.y * inv);
+        return;
+    }
+    // More: 16 lanes a row weigh its ranges, 64 of them a turn, while a thread's pairs of channels are on their way, up to 64 loads.  (As above, a pair after
+    // the other, each with the weights anew: 6 trips for 16 rows of 192 channels.  A request of 500 keys, 16 heads over one of 256 x 192 21.6 us -> 13.3, of 128 x 128
+    // 11.3 -> 9.4, the streaming kernel and its merge 15.1 and 10.7; for 4 rows of 128 channels the way above is 0.6 us shorter.)
+    float* const weight = mo;                            // [FEW_ROWS][FEW_TURN]
+    float* const factor = mml;                           // [FEW_ROWS] what a turn's sums before it are multiplied by, then [FEW_ROWS] the results
+    const int wr = tid >> 4, wj = tid & 15;
+    const float* const ml = a.part_ml + (((size_t)s0 * a.Hk + kvh) * ROWS + (wr < n_rows ? wr : 0)) * 2;
+    const float* const po = a.part_o + ((size_t)s0 * a.Hk + kvh) * ROWS * HV;      // (a row block's rows lie one after the other)
+    constexpr int PB = FEW_PAIRS, U = 16;
+    for (int p0 = 0; p0 < total; p0 += PB * 64 * FEW_WAVES) {
+        float2 acc[PB];
+        int at[PB];
+#pragma unroll
+        for (int p = 0; p < PB; ++p) {
+            acc[p] = make_float2(0.f, 0.f);
+            at[p] = p0 + p * 64 * FEW_WAVES + tid < total ? p0 + p * 64 * FEW_WAVES + tid : 0;
+        }
+        float mx = -INFINITY, wsum = 0.f;
+        for (int g = 0; g < ns; g += FEW_TURN) {
+            const int n = ns - g < FEW_TURN ? ns - g : FEW_TURN;
+            const bool weigh = p0 == 0 || ns > FEW_TURN;
+            float2 mlv[FEW_TURN / 16], pv[PB][U];
+            if (weigh)
+#pragma unroll
+                for (int i = 0; i < FEW_TURN / 16; ++i)
+                    if (16 * i < n) mlv[i] = load_agent(ml + (g + (wj + 16 * i < n ? wj + 16 * i : 0)) * ml_step);
+            auto load = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+                for (int p = 0; p < PB; ++p)
+                    if (p0 + p * 64 * FEW_WAVES < total)
+#pragma unroll
+                        for (int e = 0; e < U; e += 8) {
+                            if (b + e < n) {
+#pragma unroll
+                                for (int u = e; u < e + 8; ++u) pv[p][u] = load_agent(po + (g + (b + u < n ? b + u : b)) * po_step + 2 * at[p]);
+                            } else {
+#pragma unroll
+                                for (int u = e; u < e + 8; ++u) pv[p][u] = make_float2(0.f, 0.f);
+                            }
+                        }
+            };
+            load(0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (weigh) {
+                float cm = mx, sum = 0.f;
+#pragma unroll
+                for (int i = 0; i < FEW_TURN / 16; ++i)
+                    if (wj + 16 * i < n) cm = fmaxf(cm, mlv[i].x);
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o, 64));
+                const float before = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - cm);
+                if (g > 0 || p0 > 0) __syncthreads();        // (the weights of the turn before are read)
+#pragma unroll
+                for (int i = 0; i < FEW_TURN / 16; ++i) {
+                    const float w = wj + 16 * i < n && mlv[i].y > 0.f ? mlv[i].y * __builtin_amdgcn_exp2f(mlv[i].x - cm) : 0.f;
+                    weight[wr * FEW_TURN + wj + 16 * i] = w;
+                    sum += w;
+                }
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o, 64);
+                wsum = wsum * before + sum;
+                mx = cm;
+                if (wj == 0) {
+                    factor[wr] = before;
+                    if (g + FEW_TURN >= ns && wr < n_rows) {
+                        const int rr = row0 + wr, tk = rr / G, hh = kvh * G + (rr - tk * G);
+                        const float all = with_sink(a.sinks, hh, mx, wsum);
+                        factor[FEW_ROWS + wr] = (all > 0.f ? 1.0f / all : 0.f) * row_factor(a.gate, a.ld_gate, a.out_scale, q0 + tk, hh);
+                    }
+                }
+                __syncthreads();
+            }
+            if (g > 0)
+#pragma unroll
+                for (int p = 0; p < PB; ++p) {
+                    const float f = factor[at[p] / (HV / 2)];
+                    acc[p].x *= f; acc[p].y *= f;
+                }
+            for (int b = 0; b < n; b += U) {
+                if (b > 0) load(b);
+#pragma unroll
+                for (int p = 0; p < PB; ++p)
+                    if (p0 + p * 64 * FEW_WAVES < total) {
+                        const float* const w = weight + at[p] / (HV / 2) * FEW_TURN + b;
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {         // (weights past the last range are 0)
+                            acc[p].x += w[u] * pv[p][u].x; acc[p].y += w[u] * pv[p][u].y;
+                        }
+                    }
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < PB; ++p) {
+            if (p0 + p * 64 * FEW_WAVES + tid >= total) continue;
+            const int r = at[p] / (HV / 2), d2 = (at[p] - r * (HV / 2)) * 2;
+            const int rr = row0 + r, tk = rr / G, hh = kvh * G + (rr - tk * G);
+            const float inv = factor[FEW_ROWS + r];
+            bf16_t* op = a.out + (size_t)(q0 + tk) * a.ld_out + hh * HV + d2;
+            *reinterpret_cast<uint32_t*>(op) = pack2(acc[p].x * inv, acc[p].y * inv);
+        }
     }
     }
 }

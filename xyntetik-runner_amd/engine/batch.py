@@ -78,9 +78,9 @@ ATTN_CTA_FILL = 256     # 128-row items (times key/value heads) that give every 
 FEW_ROWS = 16           # rows of an item of the kernel for few rows (a request's tokens x heads-in-group, at most)
 FEW_PAGE = 32           # and the smallest page it takes
 FEW_INTS = 12           # numbers of such an item
-FEW_MIN_RANGE = 4       # tiles: its shortest key range (a tile a wave)
-FEW_SLOTS = 256         # workgroups of it that a step's requests are cut into: one a compute unit (twice as many cost the merge more than
-                        # they gain: 1 request of 8,000 keys 13.6 us -> 17.6, 16 of 330 10.7 -> 11.3, 32 of 1,000 to 2,000 with heads of 64 25.1 -> 26.2)
+FEW_MIN_RANGE = 3       # tiles: its shortest key range
+FEW_SLOTS = 256         # workgroups of it that a step's requests are cut into: one a compute unit (twice as many cost more than they gain:
+                        # 8 requests of 1,000 to 2,000 keys 15.0 us -> 15.9, 16 of 330 9.4 -> 10.6, 32 of 1,000 to 2,000 with heads of 64 22.6 -> 23.3)
 
 
 def key_ranges(tiles: int, share: float) -> int:
@@ -210,12 +210,12 @@ def few_row_least(tiles: int, rows: int, channels: int = 256) -> int:
     """Tiles of the shortest key range that pays where the longest request of a step has ``tiles`` tiles, ``rows`` rows a key/value head and ``channels`` of a
     key and its value together.
 
-    The last workgroup of a row block adds the ranges up, 16 of them in a round of trips to memory, more rows in more rounds: some 3 us for 4 rows of 128 channels, 7 for 16,
-    in which a workgroup goes through 5 and 13 tiles of 256 channels (0.55 us each), through more of fewer.  A recorded layer of small products, whole and cut from 4 tiles
-    on: 8 tiles of 8 x 4 heads of 128 24.1 us and 25.9, of 1 x 16 23.6 and 29.4; 13 tiles 26.8 and 24.9, 26.0 and 28.9; of 64 22.5 and 22.6, 22.5 and 24.8; of 32 20.3 and 23.4.
-    Ranges beyond 16 begin a second round, which pays where each would be long: 125 tiles in 16 and in 31, 8 x 4 heads of 128 28.8 and 30.4, 1 x 16 31.2 and 35.1; 250 in 16, 32 and (1 x 16) 63 34.0
-    and 31.8, 35.5, 37.2 and 45; of 64 27.7 and 29.1, 28.0, 29.7 and 35.5."""
-    if tiles < (9 + rows // 2) * math.sqrt(256 / channels):
+    The last workgroup of a row block adds the ranges up, in a round of trips to memory for 16 of them (more where there are many rows of many channels, or more ranges): 2 to 3
+    us, in which a workgroup goes through 5 tiles of 256 channels, through more of fewer.  Whole and in 2, 4 and 8 ranges, us: 4 x 4 heads of 128, 9 tiles 7.4, 9.1, 8.1;
+    12 tiles 8.8, 9.1, 8.8; 16 tiles 10.3, 10.1, 8.8, 7.3; 4 x 16 heads, 12 tiles 9.9, 11.0, 10.2; 16 tiles 11.5, 11.8, 10.8, 9.2; 4 x 4 of 64, 16 tiles 6.9, 8.2, 7.5, 6.5.
+    16 ranges and 32: 125 tiles of 4 x 4 heads of 128 9.9 and 10.8, of 4 x 16 13.0 and 14.5; 250 tiles 13.4 and 12.2, 16.2 and 15.9; of 4 x 4 of 64 9.6 and 9.9.  Over 972 pairs of
+    heads, requests and tiles 1% to 3% over the best of nine numbers of ranges, none slower than the streaming kernel and its merge."""
+    if tiles < (10 + rows // 4) * math.sqrt(256 / channels):
         return tiles
     most = 16 if tiles * channels < (51200 if rows <= 8 else 102400) else 32
     return max(FEW_MIN_RANGE, -(-tiles // most))
