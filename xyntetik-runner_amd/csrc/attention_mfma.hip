@@ -1071,10 +1071,10 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void k_attn_stream(AttnArgs a) {
 // the second product wants from it.  Keys are read once and whole (marked as streaming); a tile's values are half of a page's
 // 128-byte lines, whose other half another wave reads at about the same time (streaming too 75.8 us for 71.4).
 //
-// k_attn_stream with its merge and this, 8 key/value heads of 128 channels, 4 query heads each, in a recorded chain: 1 request of 1,900 keys
-// 11.2 us -> 11.0 (4 key/value heads, 2,000 keys 11.7 -> 8.7), of 8,000 19.0 -> 13.7, 8 of 1,000 to 2,000 19.6 -> 15.0, 64 of 950 to 1,900 73.9 -> 57.6, of 8,000 369 -> 352;
-// 32 key/value heads, 23 of 450 to 900 48.7 -> 44.3; heads of 64 channels, 1 of 700 9.5 -> 6.7.  Measured and left: eight waves a workgroup
-// (68.1 us for 64 requests for then 68.8, but 54.1 for the 23 of 32 heads), three workgroups a compute unit (spills: 152), both tiles of a page a step at 128 channels (one wave a SIMD: 27 us for 8 requests).
+// k_attn_stream with its merge and this, 8 key/value heads of 128 channels, 4 query heads each, in a recorded chain over the same caches: 1 request of 2,000 keys
+// 11.6 us -> 9.2, of 8,000 18.5 -> 13.6, 8 of 1,000 to 2,000 19.1 -> 14.7, 64 of 950 to 1,900 73.9 -> 57.6 (in a model's step, behind its weights, 75.7 -> 70: 5.4 TB/s), of 8,000 370 -> 352 (6.0 TB/s);
+// 32 key/value heads, 23 of 450 to 900 49.1 -> 44.4; heads of 64 channels, 1 of 700 9.4 -> 6.7.  Measured and left: eight waves a workgroup
+// (1% less for 64 requests, 6% more for the 23 of 32 heads), three workgroups a compute unit (spills: 152), both tiles of a page a step at 128 channels (one wave a SIMD: 27 us for 8 requests).
 #define FEW_ROWS 16
 #define FEW_INTS 12                   // an item's 8 numbers (slot -1: it covers all keys), then first slot, slots, counter, items of its row block
 constexpr bool FEW_OK = HD % 32 == 0;
