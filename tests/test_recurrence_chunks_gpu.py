@@ -156,7 +156,7 @@ def test_which_steps_read_rows_again():
 @pytest.mark.parametrize("kind,G,D", [("retention", 24, 48), ("retention", 24, 64), ("retention", 24, 80), ("delta", 12, 48)])
 @pytest.mark.parametrize("activation", [None, "silu"])
 def test_more_workgroups_than_compute_units(monkeypatch, kind, G, D, activation):
-    """Small heads of several portions at once, 288 workgroups, whose operands go through LDS; the last step's 144 and the 72 of a portion go straight to registers.
+    """Small heads of several portions at once, 288 workgroups, whose operands go through LDS; without an activation the last step's 144 and the 72 of a portion go straight to registers.
     A decay below zero, and then an infinity in a value: those columns come out as token by token."""
     from xyntetik_runner_amd.csrc.ops import load_ops
     ops, H, Dv = load_ops(), 24, 48

@@ -494,7 +494,8 @@ template <int D, bool DELTA> constexpr bool RC_STAGED = D <= (DELTA ? 48 : 80);
 // units.  Two of these run on a unit, whose products then wait for each other's trips to LDS; k_chunk_run has the registers for one of its own, and fetches K's columns number by
 // number: a shorter chain and more loads.  (It without fetching ahead, two a unit: no faster.)  Both, k_chunk_run and these, us with k_chunk_mats: retention, 8 portions of 1,024 rows,
 // 32 heads of 64 x 64 (1,024 workgroups) 200 and 165, 16 of 80 x 64 (512) 122 and 106, 4 of 512 rows, 16 heads of 48 x 96 (384) 48 and 38; the delta rule, of 48 x 96
-// 61.5 and 57.  Heads of 96 and more have no room for two; one workgroup a unit and fewer go faster with k_chunk_run (one portion of 2,048 rows, 32 heads of 64: 81, staged 107).
+// 61.5 and 57.  Heads of 96 and more have no room for two; one workgroup a unit and fewer go faster with k_chunk_run (one portion of 2,048 rows, 32 heads of 64: 81, staged 107)
+// unless q, k and v are to pass an activation: every wave there makes the numbers it reads, K's once more by columns, here each is made once (2,048 rows, 8 heads of 48 x 96 140 us and 116, 32 of 64 163 and 151).
 template <int D, bool DELTA, bool ACT>
 __global__ __launch_bounds__(256) void k_chunk_run_staged(ChunkArgs a) {
     constexpr int LD = D + 4, J = D / 16, NQ = RC_L * D / 1024, NM = RC_L * RC_L / 1024, MATS = DELTA ? 2 : 1;
@@ -682,9 +683,10 @@ __global__ __launch_bounds__(256) void k_chunk_run_staged(ChunkArgs a) {
 template <int D, bool DELTA, bool ACT>
 static int launch_chunks(const ChunkArgs& a, int B, int max_q, hipStream_t stream) {
     const int one = 2 * RC_L * (D + 4) * 4, mats = one + (DELTA ? 2 : 0) * RC_L * RC_LDM * 4, columns = a.Dv / RC_C * a.H;
-    const bool staged = RC_STAGED<D, DELTA> && (long long)columns * B > RC_UNITS;
+    const bool staged = RC_STAGED<D, DELTA> && (ACT || (long long)columns * B > RC_UNITS);
+    constexpr bool always = RC_STAGED<D, DELTA> && ACT;
     const int run = one + (staged ? (DELTA ? 2 : 1) * RC_L * RC_LDM : RC_L * (RC_C + 1)) * 4;
-    const auto k_run = staged ? k_chunk_run_staged<RC_STAGED<D, DELTA> ? D : 48, DELTA, ACT> : k_chunk_run<D, DELTA, ACT>;
+    const auto k_run = staged ? k_chunk_run_staged<RC_STAGED<D, DELTA> ? D : 48, DELTA, ACT> : k_chunk_run<D, DELTA, ACT && !always>;
     const void* kernels[2] = {(const void*)k_chunk_mats<D, DELTA, ACT>, (const void*)k_run};
     const int bytes[2] = {mats, run};
     for (int i = 0; i < 2; ++i)
