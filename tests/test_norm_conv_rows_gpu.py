@@ -134,3 +134,32 @@ def test_more_blocks_than_a_grid_has_rows():
         assert torch.equal(q, got[:, :2]) and torch.equal(states[0], states[1])
         page, off = table[r, place.long() // ps].long(), place.long() % ps
         assert torch.equal(kc[page, 0, off, 0], got[:, 2]) and torch.equal(vc[page, 0, 0, off], got[:, 3])
+
+
+@pytest.mark.parametrize("taps", [4, 8, 12, 16])
+@pytest.mark.parametrize("C", [5, 256, 1030])
+def test_weights_in_pieces_and_number_by_number(taps, C):
+    """Weights at a multiple of 16 bytes are read in fours, others one by one: the same sums, so the same bits; and the formula."""
+    import torch
+    from xyntetik_runner_amd.csrc.ops import load_ops
+    ops = load_ops()
+    rng = np.random.default_rng(taps * 7 + C)
+    lens = [40, 1, 9, 23]                   # (73 rows: long convolutions of fewer than 64 go another way)
+    ctx = step_ctx([3] * 4, lens, [2, 0, 3, 1])
+    u, w = rng.normal(size=(ctx.T, C)).astype(np.float32), rng.normal(size=(C, taps)).astype(np.float32)
+    held = rng.normal(size=(5, taps - 1, C)).astype(np.float32)
+    room = torch.empty(C * taps + 1, device=DEV)
+    got = []
+    for shift in (0, 1):
+        wd = room[shift:shift + C * taps].view(C, taps).copy_(torch.tensor(w))
+        state = torch.tensor(held, device=DEV)
+        got.append((ops.causal_conv(torch.tensor(u, device=DEV), wd, state, ctx, torch.float32).cpu(), state.cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    r = 0
+    for n, slot in zip(lens, [2, 0, 3, 1]):
+        x = np.concatenate([held[slot], u[r:r + n]]).astype(np.float64)
+        want = sum(w[:, j].astype(np.float64) * x[j:j + n] for j in range(taps))
+        # 32-bit sums of up to 16 products
+        assert np.abs(got[0][0].numpy()[r:r + n] - want).max() < 16 * 2.0 ** -24 * (np.abs(w).astype(np.float64).sum(1) * np.abs(x).max()).max()
+        assert np.array_equal(got[0][1].numpy()[slot], x[n:].astype(np.float32))
+        r += n

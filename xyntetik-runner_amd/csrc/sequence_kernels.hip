@@ -232,7 +232,7 @@ template <int R> __device__ inline bool rows_of_block(const int* __restrict__ cu
 // every input is read once; what a row needs before its first input (its request, the request's first row and state row) are loads
 // that wait for each other, once a block and not once a row.  The first block of a request is the only one that reads its state (up to
 // CONV_ROWS + 1 taps), and writes it anew.  Bound by memory and, for few rows, by that chain.  (Four channels a thread with 16-byte loads was slower:
-// 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 26.6 us, and k_conv_state's 4.7 behind it are saved; 17 rows of 2,048
+// 34 us for 26 at 2,048 rows of 2,048 channels.)  2,048 rows of 8,192 channels 24.2 us, and k_conv_state's 4.7 behind it are saved; 17 rows of 2,048
 // channels with 5 taps 4.2 (a row a thread and k_conv_state 4.9), 8 requests of 7 rows with 4 taps 4.2 (4.9), 200 rows of 8,192 with 9 taps 7.6 (18).
 #define CONV_ROWS 8
 // Rows i0 to i0 + CONV_ROWS - 1 of channel c of a request (those that exist; the others' results mean nothing), before the activation; in the
@@ -245,8 +245,17 @@ __device__ __forceinline__ void conv_rows(float (&y)[CONV_ROWS], const TU* __res
     const TU* const col = u + (size_t)x.row0 * ld_u + c;
     const int none = TM - taps;                     // places of the window that fewer taps leave unread
     float wt[TM], v[CONV_ROWS + TM - 1];
+    // (a channel's weights in whole pieces: number by number the lanes' loads lie `taps` apart, 600 rows of 300 requests, 8,192 channels, 16 taps 128 us; so 83, 2,048 rows of one 79 and 41)
+    if (TM % 4 == 0 && taps % 4 == 0 && ((uintptr_t)w & 15) == 0) {
 #pragma unroll
-    for (int j = 0; j < TM; ++j) wt[j] = j >= none ? w[(size_t)c * taps + j - none] : 0.f;
+        for (int j = 0; j + 3 < TM; j += 4) {
+            const float4 f = j >= none ? *reinterpret_cast<const float4*>(w + (size_t)c * taps + j - none) : make_float4(0.f, 0.f, 0.f, 0.f);
+            wt[j] = f.x; wt[j + 1] = f.y; wt[j + 2] = f.z; wt[j + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < TM; ++j) wt[j] = j >= none ? w[(size_t)c * taps + j - none] : 0.f;
+    }
 #pragma unroll
     for (int m = 0; m < CONV_ROWS + TM - 1; ++m) {
         const int s = i0 + m - (TM - 1);
